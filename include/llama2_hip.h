@@ -42,7 +42,9 @@ enum { L2_WQ = 0, L2_WK = 1, L2_WV = 2, L2_WO = 3, L2_W1 = 4, L2_W2 = 5, L2_W3 =
 
 /* How l2_forward treats B > 1 (a prefill chunk). */
 enum {
-    L2_PREFILL_FP32 = 0, /* same fp32 kernels as decode, one pass per column: identical to B=1 */
+    L2_PREFILL_FP32 = 0, /* fp32 throughout: a few columns are the bits of B=1; larger batches run on the
+                          * matrix cores with every product exact and fp32 accumulation, so they differ
+                          * from B=1 by the order of the additions only (1e-6)                       */
     L2_PREFILL_MFMA = 1  /* dequant -> fp16 tiles -> MFMA, fp32 accumulate (tolerance 2e-3)    */
 };
 
@@ -156,7 +158,7 @@ int l2_qlinear_matvec(l2_qlinear *q, const float *x_host, int B, float *y_host);
  * y_dev f32[B][out] are DEVICE pointers; the gather and the matvec are enqueued on hip_stream (a
  * hipStream_t; NULL is the default stream) and the call returns without waiting.  It calls no hipMalloc,
  * hipFree or other allocating routine: the one intermediate (x in the layer's act-order) lives in a fixed
- * device array of L2_MATVEC_DEVICE_MAX_ELEMS floats (4 MiB) that each GPU holds until the process
+ * device array of L2_MATVEC_DEVICE_MAX_ELEMS floats (48 MiB with what a batch needs) that each GPU holds until the process
  * ends, so B * in must not exceed that count (L2_ERR_RANGE otherwise).  All calls on one GPU share the array:
  * calls that overlap in time on one GPU (two streams, two threads) race; serialise them.  y equals
  * l2_qlinear_matvec's bit for bit.  What a first launch does besides enqueueing (loading the code object on the

@@ -27,6 +27,7 @@ SOURCES = {
     "kernels_q4_stream.hip": [],
     # MFMA accumulators in VGPRs: the per-group fold reads and writes them with plain FMAs
     "kernels_q4_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "kernels_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1", "-ffp-contract=off"],
     # the block kernels keep the reference's rounded-multiply-then-add where they restate it
     "kernels_misc.hip": ["-ffp-contract=off"],
     "kernels_attn.hip": ["-ffp-contract=off"],

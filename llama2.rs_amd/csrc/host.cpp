@@ -268,6 +268,13 @@ extern "C" int l2_synth_image(const l2_dims *d, uint64_t seed, void *buf, size_t
 // ---------------------------------------------------------------------------
 // model
 
+// Scratch of the stand-alone operator on a batch: the activations as planes and the K slices' partial tiles.
+struct OperatorBufs {
+    void *planes = nullptr;
+    float *ws = nullptr;
+    size_t planes_bytes = 0, ws_floats = 0;
+};
+
 struct l2_model {
     l2_dims d{};
     l2_config cfg{};
@@ -293,28 +300,19 @@ struct l2_model {
     float *x = nullptr, *xq = nullptr, *xk = nullptr, *xv = nullptr, *qv = nullptr, *kv = nullptr,
           *vv = nullptr, *attg = nullptr, *x1 = nullptr, *x3 = nullptr, *hg = nullptr, *hd = nullptr,
           *logits = nullptr;
-    // extra scratch of the MFMA prefill path (cap_B_mfma columns): fp16 inputs, w1/w3 outputs, row scales
-    int cap_B_mfma = 0;
-    void *h16a = nullptr, *h16b = nullptr, *h16c = nullptr; // fp16 [B][max(dim, hidden)]
-    float *hb = nullptr, *hb2 = nullptr, *ssb = nullptr, *gemm_ws = nullptr;
-    size_t gemm_ws_floats = 0;
+    // Buffers of a batch through the matrix cores (kernels_gemm.hip).  l2_prefill_chunks runs consecutive passes of a
+    // prompt side by side, one layer apart, on lanes: lane 0 is the model's stream, every lane has buffers of its own.
+    struct ChunkBufs {
+        float *x = nullptr, *q = nullptr, *ss = nullptr, *ws = nullptr;
+        void *h[3] = {nullptr, nullptr, nullptr}; // activations of up to three consumers, as planes
+        size_t cap_B = 0, ws_floats = 0, h_bytes = 0;
+    };
     int32_t *dtok = nullptr, *dpos = nullptr;
     unsigned long long *amax = nullptr;
-    // l2_prefill_chunks: further streams, each with a set of chunk buffers of its own (consecutive chunks of a
-    // prompt run side by side, one layer apart), the whole prompt's ids and positions, one event per layer and lane.
-    // Lane 0 is the model's stream with its primary buffers; lanes 1.. use extra[lane - 1].
     static constexpr int kMaxLanes = 4; // the process has four hardware queues
     int n_lanes = 2;
     hipStream_t extra_stream[kMaxLanes - 1] = {nullptr, nullptr, nullptr};
-    struct ChunkBufs {
-        float *x = nullptr, *xq = nullptr, *xk = nullptr, *xv = nullptr, *qv = nullptr, *kv = nullptr, *vv = nullptr;
-        void *h16a = nullptr, *h16b = nullptr, *h16c = nullptr;
-        float *hb = nullptr, *hb2 = nullptr, *ssb = nullptr, *gemm_ws = nullptr;
-        size_t gemm_ws_floats = 0;
-        const int32_t *dtok = nullptr, *dpos = nullptr;
-    };
-    ChunkBufs extra[kMaxLanes - 1];
-    int cap_B_extra[kMaxLanes - 1] = {0, 0, 0};
+    ChunkBufs lane[kMaxLanes];
     int32_t *pf_tok = nullptr, *pf_pos = nullptr;
     int cap_pf = 0;
     std::vector<hipEvent_t> pf_ev[kMaxLanes];
@@ -332,6 +330,7 @@ struct l2_model {
     // scratch for the operator-level entry points
     float *op_x = nullptr, *op_xg = nullptr, *op_y = nullptr;
     size_t op_cap = 0;
+    OperatorBufs op_batch;
     // per-launch event timing, on only inside l2_decode_profile
     struct ProfRec { int cls; hipEvent_t e0, e1; };
     bool prof_on = false;
@@ -415,6 +414,7 @@ struct l2_qlinear {
     hipStream_t stream = nullptr;
     float *x = nullptr, *xg = nullptr, *y = nullptr;
     int cap_B = 0;
+    OperatorBufs batch;
 };
 
 extern "C" int l2_device_count(void) {
@@ -691,11 +691,10 @@ extern "C" void l2_model_close(l2_model *m) {
         if (es) (void)hipStreamSynchronize(es);
     void *ptrs[] = {m->dimage, m->dinv, m->rope_cos, m->rope_sin, m->dwn, m->attn_part, m->x, m->xq, m->xk,
                     m->xv, m->qv, m->kv, m->vv, m->attg, m->x1, m->x3, m->hg, m->hd, m->logits, m->dtok, m->dpos, m->dloop,
-                    m->amax, m->dprompt, m->dout_ids, m->op_x, m->op_xg, m->op_y, m->h16a, m->h16b, m->h16c,
-                    m->hb, m->hb2, m->ssb, m->gemm_ws};
+                    m->amax, m->dprompt, m->dout_ids, m->op_x, m->op_xg, m->op_y, m->op_batch.planes, m->op_batch.ws};
     for (void *p : ptrs) dfree(p);
-    for (auto &a : m->extra) {
-        void *bufs[] = {a.x, a.xq, a.xk, a.xv, a.qv, a.kv, a.vv, a.h16a, a.h16b, a.h16c, a.hb, a.hb2, a.ssb, a.gemm_ws};
+    for (auto &a : m->lane) {
+        void *bufs[] = {a.x, a.q, a.ss, a.ws, a.h[0], a.h[1], a.h[2]};
         for (void *p : bufs) dfree(p);
     }
     dfree(m->pf_tok);
@@ -739,6 +738,9 @@ extern "C" int l2_model_set_prefill_mode(l2_model *m, int mode) {
     const int G = m->d.group_size;
     if (mode == L2_PREFILL_MFMA && m->head_size != 128)
         return l2_fail(L2_ERR_ARG, "the MFMA prefill path is built for heads of 128 (this model: %d)", m->head_size);
+    auto q4_gemm_supports = [](int in, int out, int g) {
+        return in % 128 == 0 && out % 32 == 0 && in % g == 0 && (g < 64 || (in / g) % 2 == 0);
+    };
     if (mode == L2_PREFILL_MFMA && !(q4_gemm_supports(m->d.dim, m->d.dim, G) && q4_gemm_supports(m->d.hidden_dim, m->kv_dim, G) &&
                                      q4_gemm_supports(m->d.dim, m->d.hidden_dim, G)))
         return l2_fail(L2_ERR_ARG, "the MFMA prefill path needs dim and hidden_dim to be multiples of 128 (of 2 groups for "
@@ -747,7 +749,25 @@ extern "C" int l2_model_set_prefill_mode(l2_model *m, int mode) {
     return L2_OK;
 }
 
-static int ensure_batch_mfma(l2_model *m, int B);
+// When a batch of fp32 columns goes through the matrix cores (three exact bf16 planes): from four columns on, and from
+// where the arithmetic outweighs the launches around the product.  Anything less is columns of the vector-ALU matvec,
+// each the bits of a single one.  Measured on the operator, matvec against GEMM: 4096x4096 13.7 against 13.9 us at 4
+// columns, 22 against 14 at 8; 4096x1024 13.5 against 12.9 at 16; 1024x1024 13.0 against 13.9 at 48.
+static bool gemm_pays(int B, double weights) { return B >= 4 && B * weights >= 6e7; }
+// The same for the layers of a model (nine launches each instead of seven).
+static bool gemm_pays_layer(int B, double weights) { return B >= 8 && B * weights >= 6e8; }
+
+// What a batch of B columns of this model is computed with: 0 = the matvec kernels column by column, 1 or 3 = the GEMM
+// with that many planes of activations.
+static int batch_planes(const l2_model *m, int B) {
+    if (m->d.group_size == 0 || B < 2 || m->d.dim > kGemmMaxDim || m->d.hidden_dim > kGemmMaxHidden) return 0;
+    if (m->prefill_mode == L2_PREFILL_MFMA) return 1;
+    const double dim = m->d.dim, weights = dim * (2 * dim + 2.0 * m->kv_dim + 3.0 * m->d.hidden_dim);
+    return gemm_pays_layer(B, weights) ? 3 : 0;
+}
+
+// The same for the stand-alone operator.
+static int operator_planes(const DevQLinear &q, int B) { return gemm_pays(B, (double)q.in * q.out) ? 3 : 0; }
 
 // Nothing may be running on either of the model's streams when a buffer they use is freed.
 static int drain_streams(l2_model *m) {
@@ -930,19 +950,64 @@ static int check_qlinear_shape(int in, int out, int g) {
 }
 
 static int qlinear_scratch(l2_qlinear *q, int B);
-static int scratch_ptr(float **out);
+struct FixedScratch {
+    float *xg;
+    void *planes;
+    float *ws;
+};
+static int scratch_ptr(FixedScratch *out);
+
+// Workspace of a stand-alone batch: a launch takes several K slices only while all its blocks (at most 256 x 64 outputs
+// each) are resident at once, two per CU.
+static constexpr size_t kOperatorWsFloats = (size_t)512 * 256 * 64;
+
+// The operator on a batch through the matrix cores: gather + split into planes, GEMM, sum of the K slices.
+static int gemm_operator(const DevQLinear &q, const float *x, int B, float *y, int planes, void *xh, float *ws,
+                         size_t ws_floats, hipStream_t st) {
+    GemmInput in{};
+    in.out[0] = xh, in.g_index[0] = q.g_index, in.x = x, in.n = 1;
+    L2_TRY(gemm_input_launch(in, q.in, B, planes, st));
+    Q4Launch L = launch_of(q, B, 0.f);
+    L.m[0] = mat_of(q, nullptr, nullptr, y);
+    XhList X{{xh, nullptr, nullptr}};
+    return gemm_launch(L, X, nullptr, ws, ws_floats, planes, B, st);
+}
+
+static int operator_bufs(OperatorBufs &b, const DevQLinear &q, int B, int planes, hipStream_t st) {
+    Q4Launch L = launch_of(q, B, 0.f);
+    L.m[0] = mat_of(q, nullptr, nullptr, nullptr);
+    const int ks = gemm_shape(L, B, planes).slices;
+    const size_t pb = (size_t)B * planes * gemm_padded(q.in) * 2, wf = ks > 1 ? (size_t)ks * B * q.out : 0;
+    if (pb <= b.planes_bytes && wf <= b.ws_floats) return L2_OK;
+    L2_HIP(hipStreamSynchronize(st));
+    if (pb > b.planes_bytes) {
+        dfree(b.planes);
+        b.planes = nullptr, b.planes_bytes = 0;
+        char *p = nullptr;
+        L2_TRY(dalloc(&p, pb));
+        b.planes = p, b.planes_bytes = pb;
+    }
+    if (wf > b.ws_floats) {
+        dfree(b.ws);
+        b.ws = nullptr, b.ws_floats = 0;
+        L2_TRY(dalloc(&b.ws, wf));
+        b.ws_floats = wf;
+    }
+    return L2_OK;
+}
 
 // Everything a later launch of this layer's operator would otherwise do on first use, done once here and waited
 // for: the code object is loaded on this device, the kernel's dynamic-LDS limit is raised, the fixed scratch
 // array's address is resolved.  A call made under stream capture afterwards only enqueues kernels.
 static int qlinear_warm_up(l2_qlinear *q) {
     L2_TRY(qlinear_scratch(q, 1));
-    float *fixed = nullptr;
+    FixedScratch fixed{};
     L2_TRY(scratch_ptr(&fixed));
     L2_HIP(hipMemsetAsync(q->x, 0, (size_t)q->q.in * 4, q->stream));
     L2_TRY(q4_one_natural(q->q, q->x, q->xg, q->y, 1, q->stream));   // the form l2_qlinear_matvec runs
     L2_TRY(gather_launch(q->xg, q->x, q->q.g_index, q->q.in, 1, q->stream));
     L2_TRY(q4_one(q->q, q->xg, q->y, 1, q->stream));                 // the form l2_qlinear_matvec_device runs
+    L2_TRY(gemm_warm_up(q->q.group_size));                           // and what either runs for a batch
     L2_HIP(hipStreamSynchronize(q->stream));
     return L2_OK;
 }
@@ -998,6 +1063,8 @@ extern "C" void l2_qlinear_free(l2_qlinear *q) {
     dfree(q->x);
     dfree(q->xg);
     dfree(q->y);
+    dfree(q->batch.planes);
+    dfree(q->batch.ws);
     if (q->stream) (void)hipStreamDestroy(q->stream);
     delete q;
 }
@@ -1017,10 +1084,14 @@ static int qlinear_scratch(l2_qlinear *q, int B) {
 }
 
 // x (host, natural order) -> gather through g_index -> matvec -> y (host)
-static int matvec_host(const DevQLinear &q, float *dx, float *dxg, float *dy, const float *x_host, int B,
-                       float *y_host, hipStream_t st) {
+static int matvec_host(const DevQLinear &q, float *dx, float *dxg, float *dy, OperatorBufs &bufs, int planes,
+                       const float *x_host, int B, float *y_host, hipStream_t st) {
+    if (planes) L2_TRY(operator_bufs(bufs, q, B, planes, st));
     L2_HIP(hipMemcpyAsync(dx, x_host, (size_t)B * q.in * 4, hipMemcpyHostToDevice, st));
-    L2_TRY(q4_one_natural(q, dx, dxg, dy, B, st));
+    if (planes)
+        L2_TRY(gemm_operator(q, dx, B, dy, planes, bufs.planes, bufs.ws, bufs.ws_floats, st));
+    else
+        L2_TRY(q4_one_natural(q, dx, dxg, dy, B, st));
     L2_HIP(hipMemcpyAsync(y_host, dy, (size_t)B * q.out * 4, hipMemcpyDeviceToHost, st));
     L2_HIP(hipStreamSynchronize(st));
     return L2_OK;
@@ -1030,7 +1101,7 @@ extern "C" int l2_qlinear_matvec(l2_qlinear *q, const float *x_host, int B, floa
     if (!q || !x_host || !y_host) return l2_fail(L2_ERR_ARG, "null argument");
     if (B < 1 || B > 4096) return l2_fail(L2_ERR_RANGE, "batch %d (1..4096)", B);
     L2_TRY(qlinear_scratch(q, B));
-    return matvec_host(q->q, q->x, q->xg, q->y, x_host, B, y_host, q->stream);
+    return matvec_host(q->q, q->x, q->xg, q->y, q->batch, operator_planes(q->q, B), x_host, B, y_host, q->stream);
 }
 
 // ---- the same operator for callers that cannot allocate ---------------------------------------------
@@ -1040,23 +1111,27 @@ extern "C" int l2_qlinear_matvec(l2_qlinear *q, const float *x_host, int B, floa
 // the array, at its own address, until the process ends.
 static constexpr size_t kScratchFloats = L2_MATVEC_DEVICE_MAX_ELEMS; // 4 MiB
 static __device__ __align__(256) float scratch[kScratchFloats];
+// A batch: its activations as three 16-bit planes (rows padded to 64, so at most twice the elements) and partial tiles.
+static __device__ __align__(256) uint16_t scratch_planes[2 * 3 * kScratchFloats]; // 12 MiB
+static __device__ __align__(256) float scratch_ws[kOperatorWsFloats];             // 32 MiB
 
-// The array's address on the current device.  `scratch` by name is a host-side stand-in, not a device
+// The arrays' addresses on the current device.  `scratch` by name is a host-side stand-in, not a device
 // address; the address is asked for once per device, with that device current, and kept.
-static int scratch_ptr(float **out) {
+static int scratch_ptr(FixedScratch *out) {
     static constexpr int kMaxDevices = 64;
-    static float *ptrs[kMaxDevices] = {};
+    static FixedScratch ptrs[kMaxDevices] = {};
     static std::mutex mu;
     int dev = 0;
     L2_HIP(hipGetDevice(&dev));
     if (dev < 0 || dev >= kMaxDevices) return l2_fail(L2_ERR_HIP, "device %d: more devices than the scratch table holds", dev);
     std::lock_guard<std::mutex> lock(mu);
-    if (!ptrs[dev]) {
-        void *p = nullptr;
-        const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-        if (e != hipSuccess || !p)
-            return l2_fail(L2_ERR_HIP, "hipGetSymbolAddress(scratch) on device %d: %s", dev, hipGetErrorString(e));
-        ptrs[dev] = (float *)p;
+    if (!ptrs[dev].ws) {
+        void *p[3] = {nullptr, nullptr, nullptr};
+        L2_HIP(hipGetSymbolAddress(&p[0], HIP_SYMBOL(scratch)));
+        L2_HIP(hipGetSymbolAddress(&p[1], HIP_SYMBOL(scratch_planes)));
+        L2_HIP(hipGetSymbolAddress(&p[2], HIP_SYMBOL(scratch_ws)));
+        if (!p[0] || !p[1] || !p[2]) return l2_fail(L2_ERR_HIP, "hipGetSymbolAddress(scratch) on device %d", dev);
+        ptrs[dev] = {(float *)p[0], p[1], (float *)p[2]};
     }
     *out = ptrs[dev];
     return L2_OK;
@@ -1069,13 +1144,15 @@ extern "C" int l2_qlinear_matvec_device(l2_qlinear *q, const float *x_dev, int B
         return l2_fail(L2_ERR_RANGE, "B * in = %zu floats exceed the fixed scratch of %zu (no allocation is made here: "
                                      "use a smaller batch, or l2_qlinear_matvec)",
                        (size_t)B * (size_t)q->q.in, kScratchFloats);
-    float *xg = nullptr;
-    L2_TRY(scratch_ptr(&xg));
+    FixedScratch fixed{};
+    L2_TRY(scratch_ptr(&fixed));
     hipStream_t st = (hipStream_t)hip_stream;
-    // Every element of xg[0 .. B * in) is written by the gather before the matvec reads it: nothing of the
+    // Every element of the scratch that is read has been written before by the same call: nothing of the
     // previous call's contents is read, so nothing needs clearing.
-    L2_TRY(gather_launch(xg, x_dev, q->q.g_index, q->q.in, B, st));
-    L2_TRY(q4_one(q->q, xg, y_dev, B, st));
+    if (operator_planes(q->q, B))
+        return gemm_operator(q->q, x_dev, B, y_dev, 3, fixed.planes, fixed.ws, kOperatorWsFloats, st);
+    L2_TRY(gather_launch(fixed.xg, x_dev, q->q.g_index, q->q.in, B, st));
+    L2_TRY(q4_one(q->q, fixed.xg, y_dev, B, st));
     return L2_OK;
 }
 
@@ -1111,22 +1188,8 @@ extern "C" int l2_model_qmatvec(l2_model *m, int layer, int proj, const float *x
         L2_HIP(hipStreamSynchronize(st));
         return L2_OK;
     }
-    if (B > 1 && m->prefill_mode == L2_PREFILL_MFMA && q4_gemm_supports(q.in, q.out, q.group_size)) {
-        // the prefill form of the same operator: gather, round to fp16, dequant -> MFMA
-        hipStream_t st = m->stream;
-        L2_TRY(ensure_batch_mfma(m, B));
-        L2_HIP(hipMemcpyAsync(m->op_x, x_host, (size_t)B * q.in * 4, hipMemcpyHostToDevice, st));
-        L2_TRY(gather_launch(m->op_xg, m->op_x, q.g_index, q.in, B, st));
-        L2_TRY(prep_f16_launch(m->h16a, m->op_xg, nullptr, q.in, B, st));
-        Q4Launch Q = launch_of(q, B, 0.f);
-        Q.m[0] = mat_of(q, nullptr, nullptr, m->op_y);
-        XhList X{{m->h16a, nullptr, nullptr}};
-        L2_TRY(q4_gemm_launch(Q, X, nullptr, m->gemm_ws, m->gemm_ws_floats, st));
-        L2_HIP(hipMemcpyAsync(y_host, m->op_y, (size_t)B * q.out * 4, hipMemcpyDeviceToHost, st));
-        L2_HIP(hipStreamSynchronize(st));
-        return L2_OK;
-    }
-    return matvec_host(q, m->op_x, m->op_xg, m->op_y, x_host, B, y_host, m->stream);
+    const int planes = m->prefill_mode == L2_PREFILL_FP32 ? operator_planes(q, B) : batch_planes(m, B);
+    return matvec_host(q, m->op_x, m->op_xg, m->op_y, m->op_batch, planes, x_host, B, y_host, m->stream);
 }
 
 extern "C" int l2_model_classifier(l2_model *m, const float *x_host, float *y_host) {
@@ -1226,7 +1289,7 @@ static int forward_enqueue(l2_model *m, l2_state *s, int B, int max_pos, bool wa
         } else {
             LAUNCH(K_ROPE_KV, rope_kv_launch(m->qv, m->kv, m->vv, m->dpos, m->rope_cos, m->rope_sin, kc, vc, d.n_heads,
                                              d.n_kv_heads, m->head_size, B, st));
-            LAUNCH(K_ATTENTION, attention_launch(m->attg, nullptr, m->qv, kc, vc, m->dpos, wo.inv_index, d.n_heads,
+            LAUNCH(K_ATTENTION, attention_launch(m->attg, 0, m->qv, kc, vc, m->dpos, wo.inv_index, d.n_heads,
                                                  d.n_kv_heads, m->head_size, max_pos, B, st));
         }
         {   // wo (:260) + residual (:263-264); the new x also goes out in w1's and w3's order
@@ -1314,7 +1377,7 @@ static int forward_enqueue_dense(l2_model *m, l2_state *s, int B, int max_pos, b
         } else {
             LAUNCH(K_ROPE_KV, rope_kv_launch(m->qv, m->kv, m->vv, m->dpos, m->rope_cos, m->rope_sin, kc, vc, d.n_heads,
                                              d.n_kv_heads, m->head_size, B, st));
-            LAUNCH(K_ATTENTION, attention_launch(m->attg, nullptr, m->qv, kc, vc, m->dpos, nullptr, d.n_heads,
+            LAUNCH(K_ATTENTION, attention_launch(m->attg, 0, m->qv, kc, vc, m->dpos, nullptr, d.n_heads,
                                                  d.n_kv_heads, m->head_size, max_pos, B, st));
         }
         LAUNCH(K_Q4_WO, dense(m->q[L2_WO][l], m->attg, nullptr, m->x, m->x, nullptr));       // :260-264
@@ -1329,146 +1392,168 @@ static int forward_enqueue_dense(l2_model *m, l2_state *s, int B, int max_pos, b
     return L2_OK;
 }
 
-static int ensure_batch_mfma(l2_model *m, int B) {
-    if (B <= m->cap_B_mfma) return L2_OK;
-    L2_TRY(drain_streams(m));
-    void **bufs[] = {&m->h16a, &m->h16b, &m->h16c, (void **)&m->hb, (void **)&m->hb2, (void **)&m->ssb,
-                     (void **)&m->gemm_ws};
-    m->gemm_ws_floats = 0;
-    for (void **b : bufs) {
-        dfree(*b);
-        *b = nullptr;
+// Sizes of the four launches of a layer (q|k|v, wo, w1|w3, w2), for gemm_shape.
+static Q4Launch layer_launch(const l2_model *m, int i, int B) {
+    const l2_dims &d = m->d;
+    const int outs[4][3] = {{d.dim, m->kv_dim, m->kv_dim}, {d.dim, 0, 0}, {d.hidden_dim, d.hidden_dim, 0}, {d.dim, 0, 0}};
+    Q4Launch L{};
+    L.in = i == 3 ? d.hidden_dim : d.dim, L.group_size = d.group_size, L.batch = B;
+    for (int k = 0; k < 3 && outs[i][k]; k++) L.m[L.n_mats++].out = outs[i][k];
+    return L;
+}
+
+// Whether chunks of a and of b columns are cut into the same K slices in every launch of a layer.
+static bool cut_alike(const l2_model *m, int a, int b, int planes) {
+    for (int i = 0; i < 4 && a != b; i++) {
+        const Q4Launch L = layer_launch(m, i, a);
+        if (gemm_shape(L, a, planes).slices != gemm_shape(L, b, planes).slices) return false;
     }
-    m->cap_B_mfma = 0;
-    const size_t wide = (size_t)std::max(m->d.dim, m->d.hidden_dim);
-    uint16_t *p = nullptr;
-    L2_TRY(dalloc(&p, B * wide));
-    m->h16a = p;
-    L2_TRY(dalloc(&p, B * wide));
-    m->h16b = p;
-    L2_TRY(dalloc(&p, B * wide));
-    m->h16c = p;
-    L2_TRY(dalloc(&m->hb, B * (size_t)m->d.hidden_dim));
-    L2_TRY(dalloc(&m->hb2, B * (size_t)m->d.hidden_dim));
-    L2_TRY(dalloc(&m->ssb, (size_t)B));
-    // split-K partial tiles: up to 8 slices of the widest launch (w1|w3 or q|k|v)
-    m->gemm_ws_floats = (size_t)8 * B * std::max((size_t)2 * m->d.hidden_dim, (size_t)m->d.dim + 2 * m->kv_dim) / 2;
-    L2_TRY(dalloc(&m->gemm_ws, m->gemm_ws_floats));
-    m->cap_B_mfma = B;
+    return true;
+}
+
+// Buffers of one lane for passes of B columns cut as slice_batch columns are.
+static int ensure_lane(l2_model *m, int lane, int B, int slice_batch, int planes) {
+    l2_model::ChunkBufs &b = m->lane[lane];
+    const l2_dims &d = m->d;
+    const size_t wide = gemm_padded(std::max(d.dim, d.hidden_dim));
+    size_t ws = 0; // partial tiles of the widest launch
+    for (int i = 0; i < 4; i++) {
+        const Q4Launch L = layer_launch(m, i, B);
+        size_t rows = 0;
+        for (int k = 0; k < L.n_mats; k++) rows += L.m[k].out;
+        ws = std::max(ws, (size_t)gemm_shape(L, slice_batch, planes).slices * B * rows);
+    }
+    const size_t hb = (size_t)B * planes * wide * 2;
+    if ((size_t)B <= b.cap_B && ws <= b.ws_floats && hb <= b.h_bytes) return L2_OK;
+    L2_TRY(drain_streams(m));
+    if ((size_t)B > b.cap_B) {
+        float **f[3] = {&b.x, &b.q, &b.ss};
+        for (float **p : f) dfree(*p), *p = nullptr;
+        b.cap_B = 0;
+        L2_TRY(dalloc(&b.x, (size_t)B * d.dim));
+        L2_TRY(dalloc(&b.q, (size_t)B * d.dim));
+        L2_TRY(dalloc(&b.ss, (size_t)B));
+        b.cap_B = B;
+    }
+    if (ws > b.ws_floats) {
+        dfree(b.ws);
+        b.ws = nullptr, b.ws_floats = 0;
+        L2_TRY(dalloc(&b.ws, ws));
+        b.ws_floats = ws;
+    }
+    if (hb > b.h_bytes) {
+        for (void *&p : b.h) dfree(p), p = nullptr;
+        b.h_bytes = 0;
+        for (void *&p : b.h) {
+            char *c = nullptr;
+            L2_TRY(dalloc(&c, hb));
+            p = c;
+        }
+        b.h_bytes = hb;
+    }
     return L2_OK;
 }
 
-// A prefill chunk through the matrix cores: the same schedule as forward_enqueue,
-// with every QLinear as a dequant -> fp16 -> MFMA GEMM over the B tokens and the
-// element-wise steps as kernels of their own.  Logits are never produced here
-// (src/models.rs:288).
-static l2_model::ChunkBufs primary_bufs(const l2_model *m) {
-    l2_model::ChunkBufs b;
-    b.x = m->x, b.xq = m->xq, b.xk = m->xk, b.xv = m->xv, b.qv = m->qv, b.kv = m->kv, b.vv = m->vv;
-    b.h16a = m->h16a, b.h16b = m->h16b, b.h16c = m->h16c;
-    b.hb = m->hb, b.hb2 = m->hb2, b.ssb = m->ssb, b.gemm_ws = m->gemm_ws, b.gemm_ws_floats = m->gemm_ws_floats;
-    b.dtok = m->dtok, b.dpos = m->dpos;
-    return b;
-}
-
-// The chunk's buffers and stream are arguments: l2_prefill_chunks runs consecutive chunks on two streams.  What a
-// chunk needs from the ones before it is their cache rows of the same layer, so `before_attn[l]` (the event of the
-// chunk before) is waited for in front of the attention of layer l, behind the kernel that writes this chunk's own
-// rows of layer l, and `after_kv[l]` is recorded right there (either may be null).
-static int forward_enqueue_mfma(l2_model *m, l2_state *s, int B, int max_pos, const l2_model::ChunkBufs &b,
-                                hipStream_t st, const hipEvent_t *after_kv, const hipEvent_t *before_attn) {
+// A pass of B positions through the matrix cores: the same schedule as forward_enqueue, with every QLinear as a GEMM
+// over the B columns and what stands between two of them as one kernel.  Logits are never produced here
+// (src/models.rs:288).  The pass may be several of the caller's chunks (slice_batch columns each, see GemmShape).
+//
+// The buffers and the stream are the lane's.  What a pass needs from the ones before it is their cache rows of the same
+// layer, so `before_attn[l]` (the event of the pass before) is waited for in front of the attention of layer l, behind
+// the kernel that writes this pass's own rows of layer l, and `after_kv[l]` is recorded right there (either may be null).
+static int forward_enqueue_gemm(l2_model *m, l2_state *s, int B, int max_pos, const int32_t *dtok, const int32_t *dpos,
+                                int planes, int slice_batch, int lane, const hipEvent_t *after_kv,
+                                const hipEvent_t *before_attn) {
     L2_TRY(check_position(m, max_pos));
     const l2_dims &d = m->d;
     const int dim = d.dim, hid = d.hidden_dim, kvd = m->kv_dim, L = d.n_layers;
+    const l2_model::ChunkBufs &b = m->lane[lane];
+    hipStream_t st = lane ? m->extra_stream[lane - 1] : m->stream;
+    auto gemm = [&](Q4Launch &Q, const XhList &X, const float *ss, int *ks) {
+        return gemm_launch(Q, X, ss, b.ws, b.ws_floats, planes, slice_batch, st, ks);
+    };
+    // rms scale of the stream in b.x and the inputs of layer l's q, k and v; ks partial tiles are added first
+    auto attn_inputs = [&](int l, int ks) {
+        ResNormPrep R{};
+        R.ws = ks ? b.ws : nullptr, R.KS = ks ? ks : 1, R.B = B, R.out = dim, R.res = b.x, R.x = b.x, R.ss = b.ss, R.eps = m->rms_eps;
+        R.n = 3, R.wn = m->rms_att + (size_t)l * dim;
+        for (int c = 0; c < 3; c++) R.inv[c] = m->q[L2_WQ + c][l].inv_index, R.out_h[c] = b.h[c];
+        return gemm_residual_norm_launch(R, planes, st);
+    };
     {
         ScatterTargets t{};
-        t.n = 3;
-        t.inv[0] = m->q[L2_WQ][0].inv_index, t.inv[1] = m->q[L2_WK][0].inv_index, t.inv[2] = m->q[L2_WV][0].inv_index;
-        t.out[0] = b.xq, t.out[1] = b.xk, t.out[2] = b.xv;
-        L2_TRY(embed_launch(b.x, m->tok_emb, b.dtok, dim, B, t, nullptr, st));
-        // the first layer's inputs; every later layer gets them from the kernel that ends the layer before
-        L2_TRY(rms_scale_launch(b.ssb, b.x, m->rms_eps, dim, B, st));
-        PrepList P{};
-        P.n_mats = 3;
-        P.out[0] = b.h16a, P.x[0] = b.xq, P.wn[0] = m->dwn + 0 * (size_t)dim;
-        P.out[1] = b.h16b, P.x[1] = b.xk, P.wn[1] = m->dwn + 1 * (size_t)dim;
-        P.out[2] = b.h16c, P.x[2] = b.xv, P.wn[2] = m->dwn + 2 * (size_t)dim;
-        L2_TRY(prep_f16_multi_launch(P, dim, B, st));
+        L2_TRY(embed_launch(b.x, m->tok_emb, dtok, dim, B, t, nullptr, st));
+        L2_TRY(attn_inputs(0, 0));
     }
     for (int l = 0; l < L; l++) {
         const DevQLinear &wq = m->q[L2_WQ][l], &wk = m->q[L2_WK][l], &wv = m->q[L2_WV][l],
                          &wo = m->q[L2_WO][l], &w1 = m->q[L2_W1][l], &w2 = m->q[L2_W2][l],
                          &w3 = m->q[L2_W3][l];
-        RopeKvArgs R{};
-        {
-            Q4Launch Q = launch_of(wq, B, m->rms_eps);
-            Q.m[0] = mat_of(wq, nullptr, nullptr, b.qv);
-            Q.m[1] = mat_of(wk, nullptr, nullptr, b.kv);
-            Q.m[2] = mat_of(wv, nullptr, nullptr, b.vv);
-            Q.n_mats = 3;
-            XhList X{{b.h16a, b.h16b, b.h16c}};
-            // partial tiles; the kernel that adds them also applies the rms scale, RoPE and the cache write
-            L2_TRY(q4_gemm_launch(Q, X, b.ssb, b.gemm_ws, b.gemm_ws_floats, st, &R.KS));
-        }
         float *kc = s->kcache + (size_t)l * m->max_seq * kvd;
         float *vc = s->vcache + (size_t)l * m->max_seq * kvd;
-        R.ws = b.gemm_ws, R.B = B, R.ss = b.ssb, R.pos = b.dpos, R.cos_t = m->rope_cos, R.sin_t = m->rope_sin;
-        R.q = b.qv, R.kcache = kc, R.vcache = vc, R.n_heads = d.n_heads, R.n_kv_heads = d.n_kv_heads;
-        L2_TRY(gemm_rope_kv_launch(R, st));
-        // Wait first, record second: the event of this chunk then stands for its own rows of layer l AND, through
-        // the event it waited for, for those of every chunk before it, so that a chunk two or more lanes behind
+        {   // q, k, v: partial tiles; the kernel that adds them also applies the rms scale, RoPE and the cache write
+            Q4Launch Q = launch_of(wq, B, m->rms_eps);
+            Q.m[0] = mat_of(wq, nullptr, nullptr, nullptr);
+            Q.m[1] = mat_of(wk, nullptr, nullptr, nullptr);
+            Q.m[2] = mat_of(wv, nullptr, nullptr, nullptr);
+            Q.n_mats = 3;
+            RopeKvArgs R{};
+            L2_TRY(gemm(Q, XhList{{b.h[0], b.h[1], b.h[2]}}, nullptr, &R.KS));
+            R.ws = b.ws, R.B = B, R.ss = b.ss, R.pos = dpos, R.cos_t = m->rope_cos, R.sin_t = m->rope_sin;
+            R.q = b.q, R.kcache = kc, R.vcache = vc, R.n_heads = d.n_heads, R.n_kv_heads = d.n_kv_heads;
+            L2_TRY(gemm_rope_kv_launch(R, st));
+        }
+        // Wait first, record second: the event of this pass then stands for its own rows of layer l AND, through
+        // the event it waited for, for those of every pass before it, so that a pass two or more lanes behind
         // needs to wait for its direct predecessor only.
         if (before_attn) L2_HIP(hipStreamWaitEvent(st, before_attn[l], 0));
         if (after_kv) L2_HIP(hipEventRecord(after_kv[l], st));
-        L2_TRY(attention_launch(nullptr, b.h16a, b.qv, kc, vc, b.dpos, wo.inv_index, d.n_heads, d.n_kv_heads,
-                                m->head_size, max_pos, B, st));
-        {   // wo: partial tiles, then residual + rms scale + the fp16 inputs of w1 and w3 in one kernel
+        L2_TRY(attention_launch(b.h[0], planes, b.q, kc, vc, dpos, wo.inv_index, d.n_heads, d.n_kv_heads, m->head_size,
+                                max_pos, B, st));
+        {   // wo: partial tiles, then residual + rms scale + the inputs of w1 and w3 in one kernel
             Q4Launch Q = launch_of(wo, B, 0.f);
-            Q.m[0] = mat_of(wo, nullptr, nullptr, b.x);
-            XhList X{{b.h16a, nullptr, nullptr}};
+            Q.m[0] = mat_of(wo, nullptr, nullptr, nullptr);
             ResNormPrep R{};
-            L2_TRY(q4_gemm_launch(Q, X, nullptr, b.gemm_ws, b.gemm_ws_floats, st, &R.KS));
-            R.ws = b.gemm_ws, R.B = B, R.out = dim, R.res = b.x, R.x = b.x, R.ss = b.ssb, R.eps = m->rms_eps;
+            L2_TRY(gemm(Q, XhList{{b.h[0], nullptr, nullptr}}, nullptr, &R.KS));
+            R.ws = b.ws, R.B = B, R.out = dim, R.res = b.x, R.x = b.x, R.ss = b.ss, R.eps = m->rms_eps;
             R.n = 2, R.wn = m->rms_ffn + (size_t)l * dim;
-            R.inv[0] = w1.inv_index, R.out_h[0] = b.h16a;
-            R.inv[1] = w3.inv_index, R.out_h[1] = b.h16b;
-            L2_TRY(gemm_residual_norm_prep_launch(R, st));
+            R.inv[0] = w1.inv_index, R.out_h[0] = b.h[0];
+            R.inv[1] = w3.inv_index, R.out_h[1] = b.h[1];
+            L2_TRY(gemm_residual_norm_launch(R, planes, st));
         }
-        {
+        {   // w1 | w3, then the gate in w2's order
             Q4Launch Q = launch_of(w1, B, m->rms_eps);
-            Q.m[0] = mat_of(w1, nullptr, nullptr, b.hb);
-            Q.m[1] = mat_of(w3, nullptr, nullptr, b.hb2);
+            Q.m[0] = mat_of(w1, nullptr, nullptr, nullptr);
+            Q.m[1] = mat_of(w3, nullptr, nullptr, nullptr);
             Q.n_mats = 2;
-            XhList X{{b.h16a, b.h16b, nullptr}};
-            L2_TRY(q4_gemm_launch(Q, X, b.ssb, b.gemm_ws, b.gemm_ws_floats, st));
+            SiluArgs S{};
+            L2_TRY(gemm(Q, XhList{{b.h[0], b.h[1], nullptr}}, nullptr, &S.KS));
+            S.ws = b.ws, S.B = B, S.n = hid, S.ss = b.ss, S.inv = w2.inv_index, S.out_h = b.h[2];
+            L2_TRY(gemm_silu_launch(S, planes, st));
         }
-        L2_TRY(silu_scatter_launch(nullptr, b.h16a, b.hb, b.hb2, w2.inv_index, hid, B, st));
-        {
+        {   // w2; the kernel that adds its tiles hands the next layer its q, k and v inputs
             Q4Launch Q = launch_of(w2, B, 0.f);
             Q.m[0] = mat_of(w2, nullptr, nullptr, b.x);
-            XhList X{{b.h16a, nullptr, nullptr}};
-            if (l + 1 < L) { // the same kernel hands the next layer its q, k and v inputs
-                ResNormPrep R{};
-                L2_TRY(q4_gemm_launch(Q, X, nullptr, b.gemm_ws, b.gemm_ws_floats, st, &R.KS));
-                R.ws = b.gemm_ws, R.B = B, R.out = dim, R.res = b.x, R.x = b.x, R.ss = b.ssb, R.eps = m->rms_eps;
-                R.n = 3, R.wn = m->rms_att + (size_t)(l + 1) * dim;
-                R.inv[0] = m->q[L2_WQ][l + 1].inv_index, R.out_h[0] = b.h16a;
-                R.inv[1] = m->q[L2_WK][l + 1].inv_index, R.out_h[1] = b.h16b;
-                R.inv[2] = m->q[L2_WV][l + 1].inv_index, R.out_h[2] = b.h16c;
-                L2_TRY(gemm_residual_norm_prep_launch(R, st));
+            int ks = 0;
+            if (l + 1 < L) {
+                L2_TRY(gemm(Q, XhList{{b.h[2], nullptr, nullptr}}, nullptr, &ks));
+                L2_TRY(attn_inputs(l + 1, ks));
             } else {
                 Q.e.kind = Q4_EPI_RESIDUAL;
                 Q.e.res = b.x;
-                L2_TRY(q4_gemm_launch(Q, X, nullptr, b.gemm_ws, b.gemm_ws_floats, st));
+                L2_TRY(gemm(Q, XhList{{b.h[2], nullptr, nullptr}}, nullptr, nullptr));
             }
         }
     }
     return L2_OK;
 }
 
-static int forward_enqueue_mfma(l2_model *m, l2_state *s, int B, int max_pos) {
-    L2_TRY(ensure_batch_mfma(m, B));
-    return forward_enqueue_mfma(m, s, B, max_pos, primary_bufs(m), m->stream, nullptr, nullptr);
+// transformer<B> on the model's stream for B > 1 tokens and positions already in device memory.
+static int forward_batch(l2_model *m, l2_state *s, int B, int max_pos) {
+    const int planes = batch_planes(m, B);
+    if (!planes) return forward_enqueue(m, s, B, max_pos, false);
+    L2_TRY(ensure_lane(m, 0, B, B, planes));
+    return forward_enqueue_gemm(m, s, B, max_pos, m->dtok, m->dpos, planes, B, 0, nullptr, nullptr);
 }
 
 static int check_tokens(const l2_model *m, const int32_t *tokens, const int32_t *pos, int B, int *max_pos) {
@@ -1494,28 +1579,29 @@ extern "C" int l2_forward(l2_model *m, l2_state *s, const int32_t *tokens, const
     L2_TRY(ensure_batch(m, B));
     L2_HIP(hipMemcpyAsync(m->dtok, tokens, (size_t)B * 4, hipMemcpyHostToDevice, m->stream));
     L2_HIP(hipMemcpyAsync(m->dpos, pos, (size_t)B * 4, hipMemcpyHostToDevice, m->stream));
-    if (B > 1 && m->prefill_mode == L2_PREFILL_MFMA)
-        L2_TRY(forward_enqueue_mfma(m, s, B, max_pos));
+    if (B > 1)
+        L2_TRY(forward_batch(m, s, B, max_pos));
     else
-        L2_TRY(forward_enqueue(m, s, B, max_pos, B == 1));
+        L2_TRY(forward_enqueue(m, s, B, max_pos, true));
     if (B == 1 && logits_host)
         L2_HIP(hipMemcpyAsync(logits_host, m->logits, (size_t)m->d.vocab_size * 4, hipMemcpyDeviceToHost, m->stream));
     L2_HIP(hipStreamSynchronize(m->stream));
     return L2_OK;
 }
 
-// The second set of chunk buffers, the second stream and the per-layer events of l2_prefill_chunks.
-static int ensure_prefill_pipeline(l2_model *m, int B, int n) {
-    const int lanes = B > 0 ? m->n_lanes : 1;
+// The lanes of l2_prefill_chunks (streams, events, buffers) and room for the whole prompt's ids and positions.
+static int ensure_prefill_pipeline(l2_model *m, int lanes, int B, int slice_batch, int planes, int n) {
     for (int i = 0; i + 1 < lanes; i++)
         if (!m->extra_stream[i]) L2_HIP(hipStreamCreate(&m->extra_stream[i])); // default priority, as the model's own
     if (!m->pf_join) L2_HIP(hipEventCreateWithFlags(&m->pf_join, hipEventDisableTiming));
-    for (int i = 0; i < lanes; i++)
+    for (int i = 0; i < lanes; i++) {
         while ((int)m->pf_ev[i].size() < m->d.n_layers) {
             hipEvent_t e = nullptr;
             L2_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
             m->pf_ev[i].push_back(e);
         }
+        if (planes) L2_TRY(ensure_lane(m, i, B, slice_batch, planes));
+    }
     if (n > m->cap_pf) {
         L2_TRY(drain_streams(m));
         dfree(m->pf_tok), dfree(m->pf_pos);
@@ -1524,48 +1610,21 @@ static int ensure_prefill_pipeline(l2_model *m, int B, int n) {
         L2_TRY(dalloc(&m->pf_pos, (size_t)n));
         m->cap_pf = n;
     }
-    for (int i = 0; i + 1 < lanes; i++) {
-        if (B <= m->cap_B_extra[i]) continue;
-        L2_TRY(drain_streams(m));
-        l2_model::ChunkBufs &a = m->extra[i];
-        void **bufs[] = {(void **)&a.x, (void **)&a.xq, (void **)&a.xk, (void **)&a.xv, (void **)&a.qv, (void **)&a.kv,
-                         (void **)&a.vv, &a.h16a, &a.h16b, &a.h16c, (void **)&a.hb, (void **)&a.hb2, (void **)&a.ssb,
-                         (void **)&a.gemm_ws};
-        for (void **b : bufs) {
-            dfree(*b);
-            *b = nullptr;
-        }
-        m->cap_B_extra[i] = 0;
-        const size_t dim = m->d.dim, hid = m->d.hidden_dim, kvd = m->kv_dim, wide = std::max(dim, hid);
-        L2_TRY(dalloc(&a.x, B * dim));
-        L2_TRY(dalloc(&a.xq, B * dim));
-        L2_TRY(dalloc(&a.xk, B * dim));
-        L2_TRY(dalloc(&a.xv, B * dim));
-        L2_TRY(dalloc(&a.qv, B * dim));
-        L2_TRY(dalloc(&a.kv, B * kvd));
-        L2_TRY(dalloc(&a.vv, B * kvd));
-        uint16_t *h = nullptr;
-        L2_TRY(dalloc(&h, B * wide));
-        a.h16a = h;
-        L2_TRY(dalloc(&h, B * wide));
-        a.h16b = h;
-        L2_TRY(dalloc(&h, B * wide));
-        a.h16c = h;
-        L2_TRY(dalloc(&a.hb, B * hid));
-        L2_TRY(dalloc(&a.hb2, B * hid));
-        L2_TRY(dalloc(&a.ssb, (size_t)B));
-        a.gemm_ws_floats = (size_t)8 * B * std::max((size_t)2 * hid, dim + 2 * kvd) / 2;
-        L2_TRY(dalloc(&a.gemm_ws, a.gemm_ws_floats));
-        m->cap_B_extra[i] = B;
-    }
     return L2_OK;
 }
 
-// prefill<A> (src/inference.rs:16-40) for a whole prompt: tokens[i] at position pos0 + i, in chunks of `chunk`,
-// no logits.  With the matrix-core mode consecutive chunks run on n_lanes streams, each with buffers of its own:
-// a chunk needs from its predecessor only that chunk's cache rows of the same layer (an event per layer), so
-// every chunk follows one layer behind the one before it and its kernels fill the compute units that the
-// others' short launches leave idle.  The arithmetic of a chunk is that of l2_forward on the same chunk.
+// One pass over consecutive positions: whole chunks of the caller's that are cut into the same K slices.
+struct PrefillPass {
+    int first, n, slice_batch, planes;
+};
+static constexpr int kPassTokens = 512;
+
+// prefill<A> (src/inference.rs:16-40) for a whole prompt: tokens[i] at position pos0 + i, in chunks of `chunk`, no
+// logits.  Chunks that the GEMM cuts alike go through it together, up to kPassTokens at a time: a column's arithmetic
+// does not depend on the columns beside it, so every chunk is what l2_forward computes for it, bit for bit, and the
+// weights are read and dequantised once per pass.  Passes run on n_lanes streams, each with buffers of its own: a pass
+// needs from its predecessor only the cache rows of the same layer (an event per layer), so every pass follows one layer
+// behind the one before it and its kernels fill the compute units that the others' short launches leave idle.
 extern "C" int l2_prefill_chunks(l2_model *m, l2_state *s, const int32_t *tokens, int n, int pos0, int chunk) {
     if (!m || !s || !tokens) return l2_fail(L2_ERR_ARG, "null argument");
     if (s->m != m) return l2_fail(L2_ERR_ARG, "state belongs to another model");
@@ -1575,11 +1634,26 @@ extern "C" int l2_prefill_chunks(l2_model *m, l2_state *s, const int32_t *tokens
     for (int i = 0; i < n; i++)
         if (tokens[i] < 0 || tokens[i] >= m->d.vocab_size)
             return l2_fail(L2_ERR_RANGE, "token id %d outside 0..%d", tokens[i], m->d.vocab_size - 1);
-    const int Bmax = std::min(chunk, n);
-    L2_TRY(ensure_batch(m, Bmax));
-    const bool mfma = m->prefill_mode == L2_PREFILL_MFMA;
-    if (mfma) L2_TRY(ensure_batch_mfma(m, Bmax));
-    L2_TRY(ensure_prefill_pipeline(m, mfma ? Bmax : 0, n));
+    std::vector<PrefillPass> passes;
+    int rest = 0; // most columns of a chunk that the matvec kernels take
+    int widest = 0, cut = 0, planes = 0;
+    for (int c0 = 0; c0 < n; c0 += chunk) {
+        const int B = std::min(chunk, n - c0), p = batch_planes(m, B);
+        if (!p) rest = std::max(rest, B);
+        if (p && !passes.empty()) {
+            PrefillPass &last = passes.back();
+            if (last.planes == p && cut_alike(m, last.slice_batch, B, p) && last.n + B <= kPassTokens) {
+                last.n += B;
+                continue;
+            }
+        }
+        passes.push_back({c0, B, B, p});
+    }
+    const int lanes = passes.size() > 1 ? m->n_lanes : 1;
+    for (const PrefillPass &p : passes)
+        if (p.planes) widest = std::max(widest, p.n), cut = cut ? std::min(cut, p.slice_batch) : p.slice_batch, planes = p.planes;
+    L2_TRY(ensure_batch(m, std::max(rest, 1)));
+    L2_TRY(ensure_prefill_pipeline(m, lanes, widest, cut, planes, n));
     std::vector<int32_t> pos((size_t)n);
     for (int i = 0; i < n; i++) pos[(size_t)i] = pos0 + i;
     // synchronous copies: the host arrays are the caller's and this function's own
@@ -1588,7 +1662,6 @@ extern "C" int l2_prefill_chunks(l2_model *m, l2_state *s, const int32_t *tokens
     L2_HIP(hipMemcpy(m->pf_pos, pos.data(), (size_t)n * 4, hipMemcpyHostToDevice));
     // Everything that is enqueued on the two streams; a failure half-way returns through the caller below, which
     // first waits for what earlier chunks already have in flight on either stream.
-    const int lanes = mfma ? m->n_lanes : 1;
     // the model's stream waits for everything the other lanes have been given so far
     auto join_lanes = [&]() -> int {
         for (int i = 0; i + 1 < lanes; i++) {
@@ -1598,27 +1671,23 @@ extern "C" int l2_prefill_chunks(l2_model *m, l2_state *s, const int32_t *tokens
         return L2_OK;
     };
     auto enqueue_all = [&]() -> int {
-        int c = 0;
-        for (int c0 = 0; c0 < n; c0 += chunk, c++) {
-            const int B = std::min(chunk, n - c0);
-            const int max_pos = pos0 + c0 + B - 1;
-            if (mfma && B > 1) {
+        int c = 0; // GEMM passes so far
+        for (const PrefillPass &p : passes) {
+            const int max_pos = pos0 + p.first + p.n - 1;
+            if (p.planes) {
                 const int lane = c % lanes, before = (c + lanes - 1) % lanes;
-                l2_model::ChunkBufs b = lane ? m->extra[lane - 1] : primary_bufs(m);
-                b.dtok = m->pf_tok + c0, b.dpos = m->pf_pos + c0;
-                hipStream_t st = lane ? m->extra_stream[lane - 1] : m->stream;
-                L2_TRY(forward_enqueue_mfma(m, s, B, max_pos, b, st, m->pf_ev[lane].data(),
-                                            c > 0 ? m->pf_ev[before].data() : nullptr));
+                L2_TRY(forward_enqueue_gemm(m, s, p.n, max_pos, m->pf_tok + p.first, m->pf_pos + p.first, p.planes, p.slice_batch,
+                                            lane, passes.size() > 1 ? m->pf_ev[lane].data() : nullptr, c > 0 ? m->pf_ev[before].data() : nullptr));
+                c++;
             } else {
-                // one token left over, or the fp32 mode: the fp32 kernels on the model's stream, behind everything
-                if (c > 0 && mfma) L2_TRY(join_lanes());
-                L2_HIP(hipMemcpyAsync(m->dtok, m->pf_tok + c0, (size_t)B * 4, hipMemcpyDeviceToDevice, m->stream));
-                L2_HIP(hipMemcpyAsync(m->dpos, m->pf_pos + c0, (size_t)B * 4, hipMemcpyDeviceToDevice, m->stream));
-                L2_TRY(forward_enqueue(m, s, B, max_pos, false));
+                // few columns: the matvec kernels on the model's stream, behind everything
+                L2_TRY(join_lanes());
+                L2_HIP(hipMemcpyAsync(m->dtok, m->pf_tok + p.first, (size_t)p.n * 4, hipMemcpyDeviceToDevice, m->stream));
+                L2_HIP(hipMemcpyAsync(m->dpos, m->pf_pos + p.first, (size_t)p.n * 4, hipMemcpyDeviceToDevice, m->stream));
+                L2_TRY(forward_enqueue(m, s, p.n, max_pos, false));
             }
         }
-        if (mfma) L2_TRY(join_lanes());
-        return L2_OK;
+        return join_lanes();
     };
     const int rc = enqueue_all();
     if (rc != L2_OK) {
@@ -1761,6 +1830,17 @@ int l2_prefill_ladder_end(int n_prompt) {
     return pos;
 }
 
+// The rungs of the ladder one behind the other are one prompt: the tokens START, prompt[0], ... (:29-33) at the
+// positions before l2_prefill_ladder_end.  They go through in as few, evenly filled passes as kPassTokens allows.
+int l2_prefill_ladder(l2_model *m, l2_state *s, const int32_t *prompt, int n_prompt) {
+    const int n = l2_prefill_ladder_end(n_prompt);
+    if (n == 0) return L2_OK;
+    std::vector<int32_t> toks((size_t)n);
+    for (int i = 0; i < n; i++) toks[i] = i == 0 ? 1 : prompt[i - 1];
+    const int passes = (n + kPassTokens - 1) / kPassTokens;
+    return l2_prefill_chunks(m, s, toks.data(), n, 0, (n + passes - 1) / passes);
+}
+
 extern "C" int l2_generate_greedy(l2_model *m, l2_state *s, const int32_t *prompt, int n_prompt, int steps,
                                   int use_prefill, int32_t *out_ids, int *n_out, double *ms) {
     if (!m || !s || !out_ids || !n_out || (n_prompt > 0 && !prompt)) return l2_fail(L2_ERR_ARG, "null argument");
@@ -1776,7 +1856,7 @@ extern "C" int l2_generate_greedy(l2_model *m, l2_state *s, const int32_t *promp
         if (prompt[i] < 0 || prompt[i] >= m->d.vocab_size)
             return l2_fail(L2_ERR_RANGE, "prompt token %d outside 0..%d", prompt[i], m->d.vocab_size - 1);
     L2_TRY(l2_state_reset(s)); // RunState::new per call (:59)
-    L2_TRY(ensure_batch(m, use_prefill ? 64 : 1));
+    L2_TRY(ensure_batch(m, 1));
     L2_TRY(ensure_loop_buffers(m, std::max(n_prompt, 1), std::max(steps, 1)));
     if (n_prompt > 0)
         L2_HIP(hipMemcpyAsync(m->dprompt, prompt, (size_t)n_prompt * 4, hipMemcpyHostToDevice, m->stream));
@@ -1784,24 +1864,8 @@ extern "C" int l2_generate_greedy(l2_model *m, l2_state *s, const int32_t *promp
     const auto t0 = std::chrono::steady_clock::now(); // :72
     int pos = 0;
     if (use_prefill) { // :78-127
-        static const int ladder[6] = {64, 32, 16, 8, 4, 2};
-        std::vector<int32_t> toks(64), poss(64);
-        for (int A : ladder) {
-            while (pos + A < n_prompt) { // :24
-                for (int i = 0; i < A; i++) {
-                    toks[i] = pos == 0 ? 1 : prompt[pos - 1]; // START, :29-33
-                    poss[i] = pos;
-                    pos++;
-                }
-                L2_HIP(hipMemcpyAsync(m->dtok, toks.data(), (size_t)A * 4, hipMemcpyHostToDevice, m->stream));
-                L2_HIP(hipMemcpyAsync(m->dpos, poss.data(), (size_t)A * 4, hipMemcpyHostToDevice, m->stream));
-                if (m->prefill_mode == L2_PREFILL_MFMA)
-                    L2_TRY(forward_enqueue_mfma(m, s, A, pos - 1));
-                else
-                    L2_TRY(forward_enqueue(m, s, A, pos - 1, false));
-                L2_HIP(hipStreamSynchronize(m->stream)); // toks/poss are reused
-            }
-        }
+        pos = l2_prefill_ladder_end(n_prompt);
+        L2_TRY(l2_prefill_ladder(m, s, prompt, n_prompt));
     }
     const int32_t first = pos == 0 ? 1 : prompt[pos - 1]; // :128-132
     L2_TRY(set_i32_launch(m->dtok, first, m->dpos, pos, m->stream));

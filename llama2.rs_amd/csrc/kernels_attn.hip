@@ -658,8 +658,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_mfma_kernel(const AttnDeco
 // the K and V rows a block streams are shared by 8 score/value streams instead of being re-read per query.
 // Query j sees timesteps 0..pos[j] (causal within the chunk as well).
 template <int QG>
-__global__ __launch_bounds__(256) void attn_prefill_kernel(float *__restrict__ out, _Float16 *__restrict__ out_h,
-                                                            const float *__restrict__ q,
+__global__ __launch_bounds__(256) void attn_prefill_kernel(float *__restrict__ out, const float *__restrict__ q,
                                                             const float *__restrict__ kc, const float *__restrict__ vc,
                                                             const int32_t *__restrict__ pos,
                                                             const int32_t *__restrict__ scatter, int n_heads,
@@ -814,16 +813,12 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(float *__restrict__ o
         }
         const int i = (kvh * QG + j % QG) * HS + d;
         const int dst = scatter ? scatter[i] : i;
-        if (out_h) // straight into the fp16 pair-interleaved order the next GEMM reads
-            out_h[(size_t)qi * dim + h16_slot(dst)] = (_Float16)(num / den);
-        else
-            out[(size_t)qi * dim + dst] = num / den;
+        out[(size_t)qi * dim + dst] = num / den;
     }
 }
 
-// Chunk attention on the matrix cores, all in fp32 (v_mfma_f32_16x16x4_f32), for the prefill mode that hands fp16
-// activations to the next GEMM.  Same function as attn_prefill_kernel (src/models.rs:131-176, causal per query over
-// the cache rows 0..pos), in the layout of attn_decode_mfma_kernel: a block owns 16 columns of one kv head, column
+// Chunk attention on the matrix cores, all in fp32 (v_mfma_f32_16x16x4_f32): src/models.rs:131-176 with B > 1, causal per
+// query over the cache rows 0..pos (every row of the chunk is already written, q is rotated), in the layout of attn_decode_mfma_kernel: a block owns 16 columns of one kv head, column
 // n = (query ct*16/QG + n/QG, head kvh*QG + n%QG), its NWV waves take the tiles of 16 cache rows w, w + NWV, ...
 // and merge through LDS at the end.  With lane = (i = lane % 16, kb = lane / 16):
 //   S^T = K Q^T      A: lane (row i, kb) holds K[t][16 m + 4 kb + e] -- what a 16-byte load of the cache row leaves
@@ -835,9 +830,9 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(float *__restrict__ o
 // 128 tokens of a 32-head model are 256 blocks, one per compute unit.  (A form on 32 columns and tiles of 32 rows,
 // v_mfma_f32_32x32x2_f32 with K and V turned through LDS, had half the blocks and took 16 to 31 us per chunk of a
 // 512-token prompt where this one takes 11 to 19.)
-template <int QG, int NWV>
+template <int QG, int NWV, int NP>
 __global__ __launch_bounds__(NWV * 64, NWV == 4 ? 2 : 1)
-void attn_prefill_mfma16_kernel(_Float16 *__restrict__ out_h, const float *__restrict__ q, const float *__restrict__ kc,
+void attn_prefill_mfma16_kernel(void *__restrict__ out, const float *__restrict__ q, const float *__restrict__ kc,
                                 const float *__restrict__ vc, const int32_t *__restrict__ pos,
                                 const int32_t *__restrict__ scatter, int n_heads, int n_kv_heads, int B, int max_pos) {
     constexpr int NT = NWV * 64, TK = 16, HS = 128, HALF = 64, NC = 16, QPT = NC / QG;
@@ -967,11 +962,10 @@ void attn_prefill_mfma16_kernel(_Float16 *__restrict__ out_h, const float *__res
         comb[wave][li][HS + 1] = l;
     }
     __syncthreads();
-    // merge the waves; a thread owns 8 consecutive d of one column, so that what it stores is one 16-byte piece of
-    // the fp16 pair-interleaved row when the consumer's order keeps those 8 together, and 8 two-byte stores otherwise
-    constexpr int NP = NC * HS / NT; // outputs per thread
+    // merge the waves; the outputs go to their places in the consumer's order
+    constexpr int NOUT = NC * HS / NT; // outputs per thread
 #pragma unroll
-    for (int u = 0; u < NP; u++) {
+    for (int u = 0; u < NOUT; u++) {
         const int idx = tid + u * NT;
         const int j = idx >> 7, d = idx & 127;
         const int qi = ct * QPT + j / QG;
@@ -988,7 +982,19 @@ void attn_prefill_mfma16_kernel(_Float16 *__restrict__ out_h, const float *__res
         if (qi < B) {
             const int i = (kvh * QG + j % QG) * HS + d;
             const int dst = scatter ? scatter[i] : i;
-            out_h[(size_t)qi * dim + h16_slot(dst)] = (_Float16)(nu / de); // the order the next GEMM reads
+            const float v = nu / de;
+            if constexpr (NP == 1) {
+                reinterpret_cast<_Float16 *>(out)[(size_t)qi * dim + h16_slot(dst)] = (_Float16)v;
+            } else { // three bf16 numbers that add up to v exactly
+                uint16_t *o = reinterpret_cast<uint16_t *>(out) + (size_t)qi * NP * dim + b16_slot(dst);
+                float left = v;
+#pragma unroll
+                for (int p = 0; p < NP; p++) {
+                    const uint32_t bits = __builtin_bit_cast(uint32_t, left) & 0xFFFF0000u;
+                    o[(size_t)p * dim] = (uint16_t)(bits >> 16);
+                    left -= __builtin_bit_cast(float, bits);
+                }
+            }
         }
     }
 }
@@ -1081,32 +1087,29 @@ int attention_decode_launch(const AttnDecode &a, hipStream_t st) {
     return L2_OK;
 }
 
-int attention_launch(float *out, void *out_f16, const float *q, const float *kcache_l, const float *vcache_l,
-                     const int32_t *pos, const int32_t *scatter, int n_heads, int n_kv_heads,
-                     int head_size, int max_pos, int B, hipStream_t st) {
-    if (head_size != 128) return l2_fail(L2_ERR_ARG, "attention: head_size=%d (128 only)", head_size);
-    const int qg = n_heads / n_kv_heads;
-    if (qg != 1 && qg != 2 && qg != 4 && qg != 8)
-        return l2_fail(L2_ERR_ARG, "attention: %d query heads per kv head (1, 2, 4 or 8)", qg);
-    if (out_f16) { // the matrix-core form: 16 columns (queries x heads of the group) per block
-        dim3 grid(n_kv_heads, (B * qg + 15) / 16), block(256);
-        switch (qg) {
-            case 1: hipLaunchKernelGGL((attn_prefill_mfma16_kernel<1, 4>), grid, block, 0, st, (_Float16 *)out_f16, q, kcache_l, vcache_l, pos, scatter, n_heads, n_kv_heads, B, max_pos); break;
-            case 2: hipLaunchKernelGGL((attn_prefill_mfma16_kernel<2, 4>), grid, block, 0, st, (_Float16 *)out_f16, q, kcache_l, vcache_l, pos, scatter, n_heads, n_kv_heads, B, max_pos); break;
-            case 4: hipLaunchKernelGGL((attn_prefill_mfma16_kernel<4, 4>), grid, block, 0, st, (_Float16 *)out_f16, q, kcache_l, vcache_l, pos, scatter, n_heads, n_kv_heads, B, max_pos); break;
-            default: hipLaunchKernelGGL((attn_prefill_mfma16_kernel<8, 4>), grid, block, 0, st, (_Float16 *)out_f16, q, kcache_l, vcache_l, pos, scatter, n_heads, n_kv_heads, B, max_pos); break;
-        }
-        L2_HIP(hipGetLastError());
-        return L2_OK;
-    }
-    const int qpb = 8 / qg;
-    dim3 grid(n_kv_heads, (B + qpb - 1) / qpb), block(256);
-    switch (qg) {
-        case 1: hipLaunchKernelGGL(attn_prefill_kernel<1>, grid, block, 0, st, out, (_Float16 *)out_f16, q, kcache_l, vcache_l, pos, scatter, n_heads, n_kv_heads, B); break;
-        case 2: hipLaunchKernelGGL(attn_prefill_kernel<2>, grid, block, 0, st, out, (_Float16 *)out_f16, q, kcache_l, vcache_l, pos, scatter, n_heads, n_kv_heads, B); break;
-        case 4: hipLaunchKernelGGL(attn_prefill_kernel<4>, grid, block, 0, st, out, (_Float16 *)out_f16, q, kcache_l, vcache_l, pos, scatter, n_heads, n_kv_heads, B); break;
-        default: hipLaunchKernelGGL(attn_prefill_kernel<8>, grid, block, 0, st, out, (_Float16 *)out_f16, q, kcache_l, vcache_l, pos, scatter, n_heads, n_kv_heads, B); break;
+template <int QG>
+static int prefill_qg(void *out, int planes, const float *q, const float *kc, const float *vc, const int32_t *pos,
+                      const int32_t *scatter, int n_heads, int n_kv_heads, int max_pos, int B, hipStream_t st) {
+    const dim3 block(256), grid(n_kv_heads, (B * QG + 15) / 16); // 16 columns (queries x heads of the group) per block
+    switch (planes) {
+        case 0: hipLaunchKernelGGL(attn_prefill_kernel<QG>, dim3(n_kv_heads, (B * QG + 7) / 8), block, 0, st, (float *)out, q, kc, vc, pos, scatter, n_heads, n_kv_heads, B); break;
+        case 1: hipLaunchKernelGGL((attn_prefill_mfma16_kernel<QG, 4, 1>), grid, block, 0, st, out, q, kc, vc, pos, scatter, n_heads, n_kv_heads, B, max_pos); break;
+        case 3: hipLaunchKernelGGL((attn_prefill_mfma16_kernel<QG, 4, 3>), grid, block, 0, st, out, q, kc, vc, pos, scatter, n_heads, n_kv_heads, B, max_pos); break;
+        default: return l2_fail(L2_ERR_ARG, "attention: %d planes", planes);
     }
     L2_HIP(hipGetLastError());
     return L2_OK;
+}
+
+int attention_launch(void *out, int planes, const float *q, const float *kcache_l, const float *vcache_l,
+                     const int32_t *pos, const int32_t *scatter, int n_heads, int n_kv_heads,
+                     int head_size, int max_pos, int B, hipStream_t st) {
+    if (head_size != 128) return l2_fail(L2_ERR_ARG, "attention: head_size=%d (128 only)", head_size);
+    switch (n_heads / n_kv_heads) {
+        case 1: return prefill_qg<1>(out, planes, q, kcache_l, vcache_l, pos, scatter, n_heads, n_kv_heads, max_pos, B, st);
+        case 2: return prefill_qg<2>(out, planes, q, kcache_l, vcache_l, pos, scatter, n_heads, n_kv_heads, max_pos, B, st);
+        case 4: return prefill_qg<4>(out, planes, q, kcache_l, vcache_l, pos, scatter, n_heads, n_kv_heads, max_pos, B, st);
+        case 8: return prefill_qg<8>(out, planes, q, kcache_l, vcache_l, pos, scatter, n_heads, n_kv_heads, max_pos, B, st);
+    }
+    return l2_fail(L2_ERR_ARG, "attention: %d query heads per kv head (1, 2, 4 or 8)", n_heads / n_kv_heads);
 }

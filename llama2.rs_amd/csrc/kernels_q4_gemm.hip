@@ -6,16 +6,16 @@
 //
 // for a chunk of T tokens whose inputs the caller has already brought into this
 // layer's g_index order, multiplied by the norm weight where one applies, and
-// rounded to fp16 (prep_f16_kernel).  This is the one place in the token loop
+// rounded to fp16 (kernels_gemm.hip).  This is the one place in the token loop
 // that is a dense contraction, hence the one place that uses MFMA; the decode
 // matvec stays on the vector ALU in fp32.
 //
 // Tiling.  A block is 4 waves; a wave owns one tile of 32 output rows and all NB
 // blocks of 32 tokens (the dequantised weights are reused NB times), so a block
 // covers 128 rows x 32*NB tokens.  With only 128 tokens per chunk that leaves
-// few blocks, so K is also cut into KS slices across grid.z; each slice writes
-// its fp32 partial tile to a workspace and q4_gemm_reduce_kernel adds the
-// slices in a fixed order and runs the epilogue.  K advances
+// few blocks, so K is also cut into KS slices; each slice writes
+// its fp32 partial tile to a workspace and the consumer (or gemm_reduce_kernel) adds
+// the slices in a fixed order.  K advances
 // 64 at a time: lane (r = l%32, h = l/32) loads the 16 bytes qweight[o][K/8+4h ..
 // +4) of its row -- four packed words, each of which is exactly the 8 k-values
 // one MFMA step wants from this lane.  The X slice [tokens][64] is staged in LDS
@@ -102,7 +102,7 @@ constexpr int gemm_xp(int kstep) { return 128 / kstep; }
 
 template <int G, int NB, int KSTEP>
 __global__ __launch_bounds__(256, NB > 2 ? 2 : 1) void q4_gemm_kernel(const Q4Launch L, const XhList xh_list, const float *__restrict__ ss,
-                                                      float *__restrict__ ws, int KS, int partials) {
+                                                      float *__restrict__ ws, int KS, int t_tiles, int partials) {
     constexpr int PW = kGemmPW, XP = gemm_xp(KSTEP), WR = gemm_wr(KSTEP);
     static_assert(PW % WR == 0 && PW % XP == 0, "ring slots are indexed by the position in the unrolled body");
     constexpr int W = KSTEP / 64;        // sub-steps of 64 k per K step
@@ -116,7 +116,13 @@ __global__ __launch_bounds__(256, NB > 2 ? 2 : 1) void q4_gemm_kernel(const Q4La
     const int in = L.in;
     const int n_k = in / KSTEP; // K iterations
 
-    int rb = blockIdx.x;
+    // blocks are dealt round-robin over the 8 XCDs: see q4_tile_gemm_kernel
+    const int n_blocks = gridDim.x, per_xcd = n_blocks >> 3, over = n_blocks & 7, xcd = blockIdx.x & 7;
+    const int work = xcd * per_xcd + min(xcd, over) + (blockIdx.x >> 3);
+    int rb = work / t_tiles;
+    const int t0 = (work - rb * t_tiles) * TN;
+    const int row_blocks = n_blocks / (t_tiles * KS), ks = rb / row_blocks; // K slice
+    rb -= ks * row_blocks;
     int mi = 0;
     while (mi + 1 < L.n_mats && rb >= L.m[mi].row_blocks) {
         rb -= L.m[mi].row_blocks;
@@ -127,7 +133,6 @@ __global__ __launch_bounds__(256, NB > 2 ? 2 : 1) void q4_gemm_kernel(const Q4La
     const int n_out = M.out;
     const int groups = L.groups;
     const int B = L.batch;
-    const int t0 = blockIdx.y * TN;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int r = lane & 31, h = lane >> 5;
     const int C4 = in >> 5; // uint4 per weight row
@@ -146,7 +151,6 @@ __global__ __launch_bounds__(256, NB > 2 ? 2 : 1) void q4_gemm_kernel(const Q4La
         for (int i = 0; i < 16; i++) acc[nb][i] = 0.f;
     constexpr int KPG = G / KSTEP > 0 ? G / KSTEP : 1; // K iterations per group
     // this block's slice of K, in whole groups
-    const int ks = blockIdx.z;
     const int n_grp = n_k / KPG;
     // slices start on an even group: the scales are fetched as aligned pairs
     const int kit0 = ((int)((long)n_grp * ks / KS) & ~1) * KPG;
@@ -396,386 +400,72 @@ __global__ __launch_bounds__(256, NB > 2 ? 2 : 1) void q4_gemm_kernel(const Q4La
                 v.z += rr.z;
                 v.w += rr.w;
             }
-            if (E.kind != Q4_EPI_SCATTER_ONLY) *reinterpret_cast<float4 *>(M.y + row + o) = v;
-            const float vals[4] = {v.x, v.y, v.z, v.w};
-            for (int c = 0; c < E.n_scatter; c++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) E.sc_out[c][row + E.sc_idx[c][o + e]] = vals[e];
+            *reinterpret_cast<float4 *>(M.y + row + o) = v;
         }
     }
-}
-
-// Adds the KS partial tiles of a split-K GEMM in slice order and runs the epilogue; a thread owns four
-// consecutive outputs of one token (every `out` is a multiple of 32).
-// grid: (ceil(sum_out / 1024), B); the matrices of the launch are laid end to end.
-__global__ __launch_bounds__(256) void q4_gemm_reduce_kernel(const Q4Launch L, const float *__restrict__ ss,
-                                                             const float *__restrict__ ws, int KS) {
-    const int t = blockIdx.y;
-    int o = (blockIdx.x * 256 + threadIdx.x) * 4;
-    int mi = 0;
-    size_t ws_base = 0;
-    const int B = L.batch;
-    while (mi + 1 < L.n_mats && o >= L.m[mi].out) {
-        o -= L.m[mi].out;
-        ws_base += (size_t)KS * B * L.m[mi].out;
-        mi++;
-    }
-    const Q4Mat &M = L.m[mi];
-    if (o >= M.out) return;
-    const float *p = ws + ws_base + (size_t)t * M.out + o;
-    const size_t slice = (size_t)B * M.out;
-    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int ks = 0; ks < KS; ks++) {
-        const float4 a = *reinterpret_cast<const float4 *>(p + ks * slice);
-        v.x += a.x, v.y += a.y, v.z += a.z, v.w += a.w;
-    }
-    if (ss) {
-        const float sc = ss[t];
-        v.x *= sc, v.y *= sc, v.z *= sc, v.w *= sc;
-    }
-    const Q4Epi &E = L.e;
-    const size_t row = (size_t)t * M.out;
-    if (E.kind == Q4_EPI_RESIDUAL) {
-        const float4 r = *reinterpret_cast<const float4 *>(E.res + row + o);
-        v.x += r.x, v.y += r.y, v.z += r.z, v.w += r.w;
-    }
-    if (E.kind != Q4_EPI_SCATTER_ONLY) *reinterpret_cast<float4 *>(M.y + row + o) = v;
-    const float vals[4] = {v.x, v.y, v.z, v.w};
-    for (int c = 0; c < E.n_scatter; c++) {
-        const int4 idx = *reinterpret_cast<const int4 *>(E.sc_idx[c] + o);
-        const int id[4] = {idx.x, idx.y, idx.z, idx.w};
-#pragma unroll
-        for (int e = 0; e < 4; e++) E.sc_out[c][row + id[e]] = vals[e];
-    }
-}
-
-// What follows a residual projection (wo, w2) of a chunk, in one kernel instead of three: add the KS partial
-// tiles in slice order and the residual (src/models.rs:263-264, 283-285), store the new residual stream,
-// take its rms scale (src/models.rs:55-60), and hand fp16 copies times the norm weight to up to three
-// consumers, each in its own act-order and in the pair-interleaved order the GEMM reads.
-// One block of 1024 threads per token, four outputs per thread and trip; every load of a trip (residual,
-// partial tiles, the consumers' indices, the norm weight) goes out before the first use.
-__global__ __launch_bounds__(1024) void gemm_residual_norm_prep_kernel(const ResNormPrep A) {
-    __shared__ float red[16];
-    extern __shared__ _Float16 perm_h[]; // [consumer][out]: the token's row in each consumer's order
-    const int t = blockIdx.x, tid = threadIdx.x;
-    const int n4 = A.out >> 2;
-    const size_t row = (size_t)t * A.out;
-    const size_t slice = (size_t)A.B * A.out;
-    float sq = 0.f;
-    for (int i4 = tid; i4 < n4; i4 += 1024) {
-        const float *p = A.ws + row + 4 * i4;
-        float4 v = *reinterpret_cast<const float4 *>(A.res + row + 4 * i4);
-        float4 part[8];
-#pragma unroll
-        for (int ks = 0; ks < 8; ks++) part[ks] = *reinterpret_cast<const float4 *>(p + min(ks, A.KS - 1) * slice);
-        int4 idx[3];
-#pragma unroll
-        for (int c = 0; c < 3; c++)
-            idx[c] = *reinterpret_cast<const int4 *>((c < A.n ? A.inv[c] : A.inv[0]) + 4 * i4);
-        const float4 g = *reinterpret_cast<const float4 *>(A.wn + 4 * i4); // one norm weight for all consumers
-        float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-        for (int ks = 0; ks < 8; ks++)
-            if (ks < A.KS) a.x += part[ks].x, a.y += part[ks].y, a.z += part[ks].z, a.w += part[ks].w;
-        v.x += a.x, v.y += a.y, v.z += a.z, v.w += a.w;
-        *reinterpret_cast<float4 *>(A.x + row + 4 * i4) = v;
-        sq = fmaf(v.x, v.x, sq), sq = fmaf(v.y, v.y, sq), sq = fmaf(v.z, v.z, sq), sq = fmaf(v.w, v.w, sq);
-        const _Float16 vals[4] = {(_Float16)(v.x * g.x), (_Float16)(v.y * g.y), (_Float16)(v.z * g.z), (_Float16)(v.w * g.w)};
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-            if (c >= A.n) continue;
-            const int id[4] = {idx[c].x, idx[c].y, idx[c].z, idx[c].w};
-            // the permutation happens in LDS: the global stores below are whole 16-byte pieces
-#pragma unroll
-            for (int e = 0; e < 4; e++) perm_h[c * A.out + h16_slot(id[e])] = vals[e];
-        }
-    }
-    for (int off = 32; off > 0; off >>= 1) sq += __shfl_xor(sq, off);
-    if ((tid & 63) == 0) red[tid >> 6] = sq;
-    __syncthreads();
-    if (tid == 0) {
-        float s = 0.f;
-        for (int w = 0; w < 16; w++) s += red[w];
-        s /= (float)A.out;
-        s += A.eps;
-        A.ss[t] = 1.0f / sqrtf(s);
-    }
-    const int n8 = A.out >> 3;
-    for (int i = tid; i < A.n * n8; i += 1024) {
-        const int c = i / n8, j8 = i - c * n8;
-        reinterpret_cast<uint4 *>(reinterpret_cast<_Float16 *>(A.out_h[c]) + row)[j8] =
-            reinterpret_cast<const uint4 *>(perm_h + (size_t)c * A.out)[j8];
-    }
-}
-
-// What follows the q|k|v projection of a chunk, in one kernel instead of two: add the KS partial tiles of
-// the three matrices in slice order, apply the token's rms scale, rotate q and k (src/models.rs:100-129: the
-// second half of a head uses the first half's ROTATED value), write q back and k and v into the cache rows
-// of the tokens' positions (:236-249).  One block per token; thread -> (head, i < 64).
-__global__ __launch_bounds__(1024) void gemm_rope_kv_kernel(const RopeKvArgs A) {
-    constexpr int HS = 128, HALF = 64;
-    const int b = blockIdx.x;
-    const int dim = A.n_heads * HS, kv_dim = A.n_kv_heads * HS;
-    const int p = A.pos[b];
-    const float ss = A.ss[b];
-    const float *ct = A.cos_t + (size_t)p * HALF, *st = A.sin_t + (size_t)p * HALF;
-    const float *wq = A.ws + (size_t)b * dim;
-    const float *wk = A.ws + (size_t)A.KS * A.B * dim + (size_t)b * kv_dim;
-    const float *wv = wk + (size_t)A.KS * A.B * kv_dim;
-    const size_t sq = (size_t)A.B * dim, sk = (size_t)A.B * kv_dim;
-    float *kc = A.kcache + (size_t)p * kv_dim, *vc = A.vcache + (size_t)p * kv_dim;
-    for (int idx = threadIdx.x; idx < A.n_heads * HALF; idx += 1024) {
-        const int h = idx >> 6, i = idx & 63;
-        const float c = ct[i], s = st[i];
-        float qa = 0.f, qb = 0.f, ka = 0.f, kb = 0.f;
-        const bool has_k = h < A.n_kv_heads;
-        for (int ks = 0; ks < A.KS; ks++) {
-            qa += wq[ks * sq + h * HS + i];
-            qb += wq[ks * sq + h * HS + i + HALF];
-            if (has_k) {
-                ka += wk[ks * sk + h * HS + i];
-                kb += wk[ks * sk + h * HS + i + HALF];
-            }
-        }
-        qa *= ss, qb *= ss;
-        const float first = qa * c - qb * s;
-        A.q[(size_t)b * dim + h * HS + i] = first;
-        A.q[(size_t)b * dim + h * HS + i + HALF] = qb * c + first * s;
-        if (has_k) {
-            ka *= ss, kb *= ss;
-            const float kf = ka * c - kb * s;
-            kc[h * HS + i] = kf;
-            kc[h * HS + i + HALF] = kb * c + kf * s;
-        }
-    }
-    for (int i = threadIdx.x; i < kv_dim; i += 1024) {
-        float v = 0.f;
-        for (int ks = 0; ks < A.KS; ks++) v += wv[ks * sk + i];
-        vc[i] = v * ss;
-    }
-}
-
-// fp32 [B][n] (already in the consumer's g_index order) -> fp16 [B][n], times the
-// norm weight if given, with the (0,4,1,5,2,6,3,7) interleave inside every 8.
-__global__ void prep_f16_kernel(const PrepList P, int n) {
-    _Float16 *out = reinterpret_cast<_Float16 *>(P.out[blockIdx.z]);
-    const float *x = P.x[blockIdx.z];
-    const float *wn = P.wn[blockIdx.z];
-    const int b = blockIdx.y;
-    const int j8 = blockIdx.x * blockDim.x + threadIdx.x; // group of 8
-    if (j8 * 8 >= n) return;
-    const float4 a = reinterpret_cast<const float4 *>(x + (size_t)b * n)[j8 * 2];
-    const float4 c = reinterpret_cast<const float4 *>(x + (size_t)b * n)[j8 * 2 + 1];
-    float v[8] = {a.x, a.y, a.z, a.w, c.x, c.y, c.z, c.w};
-    if (wn) {
-        const float4 g0 = reinterpret_cast<const float4 *>(wn)[j8 * 2];
-        const float4 g1 = reinterpret_cast<const float4 *>(wn)[j8 * 2 + 1];
-        const float g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
-#pragma unroll
-        for (int i = 0; i < 8; i++) v[i] *= g[i];
-    }
-    A8 o;
-    o.p[0] = h2{(_Float16)v[0], (_Float16)v[4]};
-    o.p[1] = h2{(_Float16)v[1], (_Float16)v[5]};
-    o.p[2] = h2{(_Float16)v[2], (_Float16)v[6]};
-    o.p[3] = h2{(_Float16)v[3], (_Float16)v[7]};
-    reinterpret_cast<uint4 *>(out + (size_t)b * n)[j8] = make_uint4(o.u[0], o.u[1], o.u[2], o.u[3]);
-}
-
-// ss[b] = 1 / sqrt(mean(x[b]^2) + eps)   (src/models.rs:55-60)
-__global__ __launch_bounds__(256) void rms_scale_kernel(float *ss, const float *x, float eps, int dim) {
-    __shared__ float red[4];
-    const int b = blockIdx.x;
-    float s = 0.f;
-    for (int i = threadIdx.x; i < dim; i += 256) {
-        const float v = x[(size_t)b * dim + i];
-        s = fmaf(v, v, s);
-    }
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float t = red[0] + red[1] + red[2] + red[3];
-        t /= (float)dim;
-        t += eps;
-        ss[b] = 1.0f / sqrtf(t);
-    }
-}
-
-// silu gate (src/models.rs:92-98) for a chunk: out[b][scatter[i]] = silu(a[b][i]) * c[b][i]
-__global__ void silu_scatter_kernel(float *out, const float *a, const float *c, const int32_t *scatter, int n) {
-    const int b = blockIdx.y;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    float s = a[(size_t)b * n + i];
-    s = s * (1.0f / (1.0f + expf(-s)));
-    s = s * c[(size_t)b * n + i];
-    out[(size_t)b * n + (scatter ? scatter[i] : i)] = s;
-}
-
-// The same gate handing fp16 to the next GEMM: one block per token permutes the token's row in LDS (the
-// consumer's act-order, pair-interleaved), so that the global stores are whole 16-byte pieces.
-__global__ __launch_bounds__(1024) void silu_scatter_f16_kernel(_Float16 *__restrict__ out_h, const float *__restrict__ a,
-                                                                const float *__restrict__ c,
-                                                                const int32_t *__restrict__ scatter, int n) {
-    extern __shared__ _Float16 perm_row[]; // [n]
-    const size_t row = (size_t)blockIdx.x * n;
-    const int tid = threadIdx.x;
-    for (int i4 = tid; i4 < (n >> 2); i4 += 1024) {
-        const float4 x = *reinterpret_cast<const float4 *>(a + row + 4 * i4);
-        const float4 y = *reinterpret_cast<const float4 *>(c + row + 4 * i4);
-        const int4 id = *reinterpret_cast<const int4 *>(scatter + 4 * i4);
-        const float xs[4] = {x.x, x.y, x.z, x.w}, ys[4] = {y.x, y.y, y.z, y.w};
-        const int ids[4] = {id.x, id.y, id.z, id.w};
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            float s = xs[e];
-            s = s * (1.0f / (1.0f + expf(-s)));
-            perm_row[h16_slot(ids[e])] = (_Float16)(s * ys[e]);
-        }
-    }
-    __syncthreads();
-    for (int j8 = tid; j8 < (n >> 3); j8 += 1024)
-        reinterpret_cast<uint4 *>(out_h + row)[j8] = reinterpret_cast<const uint4 *>(perm_row)[j8];
 }
 
 template <int G>
-int launch_gemm_g(Q4Launch &L, const XhList &xh, const float *ss, float *ws, size_t ws_floats, hipStream_t st,
-                  int *ks_out) {
-    int total = 0;
-    long rows = 0;
-    for (int i = 0; i < L.n_mats; i++) {
-        L.m[i].row_blocks = (L.m[i].out + 127) / 128;
-        total += L.m[i].row_blocks;
-        rows += L.m[i].out;
-    }
-    const int B = L.batch;
-    // Up to 255 tokens a wave takes 64 of them: with 128 a chunk of 128 tokens is too few blocks for the chip
-    // (w1|w3 of 7B: 172 blocks on 256 CUs; the launches of a 128-token chunk are 7 % slower that way).  From
-    // 256 tokens on a wave takes 128 (within 256 registers: two blocks per CU): every weight is dequantised
-    // once per 128 tokens instead of twice, and there are blocks enough whatever the tile (w1|w3 of 7B at 512
-    // tokens: 115 against 129 us).
-    const int NB = (G >= 64 && B >= 256) ? 4 : B > 32 ? 2 : 1;
-    const int TN = 32 * NB;
-    const int t_tiles = (B + TN - 1) / TN;
-    // K slices: as many as keep the grid within one round of 2 blocks per CU, whole groups per slice, at most 4.
-    // (Up to 8 fill the chip when a launch runs alone, but every slice is a partial tile that the consumer reads
-    // back, and with two chunks of a prompt in flight the other chunk's kernels take the free slots: at most 4
-    // measured 34.4 k against 32.7 k tok/s on the 7B prompt, 19.9 k against 19.5 k on 13B, no change on 70B, and
-    // 25.1 k against 24.6 k with a single chunk in flight.)
+int launch_gemm_g(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, int partials, hipStream_t st) {
     // K step: 128 where a group is at least that long (half the block barriers per k), else 64
     constexpr int KSTEP = G >= 128 ? 128 : 64;
-    const int n_grp = (L.in / KSTEP) / (G / KSTEP > 0 ? G / KSTEP : 1);
-    int KS = (2 * cu_count()) / (total * t_tiles); // all blocks resident at once: two per CU
-    if (KS > 4) KS = 4;
-    if (KS > n_grp / 2) KS = n_grp / 2; // slices start on even groups
-    if (KS < 1) KS = 1;
-    while (KS > 1 && (size_t)KS * B * rows > ws_floats) KS--;
-    dim3 grid(total, t_tiles, KS), block(256);
+    for (int i = 0; i < L.n_mats; i++) L.m[i].row_blocks = (L.m[i].out + 127) / 128;
+    const int TN = s.tokens, t_tiles = (L.batch + TN - 1) / TN;
+    const dim3 grid(s.row_blocks * t_tiles * s.slices), block(256);
     // the activation buffers, or the four output staging tiles of the epilogue (32 x 36 floats per wave)
     const size_t lds = std::max((size_t)2 * TN * (KSTEP + kXPad) * sizeof(_Float16), (size_t)4 * 32 * 36 * sizeof(float));
-    switch (NB) {
-        case 1: hipLaunchKernelGGL((q4_gemm_kernel<G, 1, KSTEP>), grid, block, lds, st, L, xh, ss, ws, KS, ks_out != nullptr); break;
-        case 2: hipLaunchKernelGGL((q4_gemm_kernel<G, 2, KSTEP>), grid, block, lds, st, L, xh, ss, ws, KS, ks_out != nullptr); break;
-        case 4:
+    switch (TN) {
+        case 32: hipLaunchKernelGGL((q4_gemm_kernel<G, 1, KSTEP>), grid, block, lds, st, L, xh, ss, ws, s.slices, t_tiles, partials); break;
+        case 64: hipLaunchKernelGGL((q4_gemm_kernel<G, 2, KSTEP>), grid, block, lds, st, L, xh, ss, ws, s.slices, t_tiles, partials); break;
+        case 128:
             if constexpr (G >= 64) {
                 static LdsLimit limit(48 * 1024);
                 L2_TRY(limit.ensure(reinterpret_cast<const void *>(q4_gemm_kernel<G, 4, KSTEP>), lds));
-                hipLaunchKernelGGL((q4_gemm_kernel<G, 4, KSTEP>), grid, block, lds, st, L, xh, ss, ws, KS, ks_out != nullptr);
+                hipLaunchKernelGGL((q4_gemm_kernel<G, 4, KSTEP>), grid, block, lds, st, L, xh, ss, ws, s.slices, t_tiles, partials);
                 break;
             }
             [[fallthrough]];
         default: return l2_fail(L2_ERR_ARG, "q4 gemm: token tile");
     }
     L2_HIP(hipGetLastError());
-    if (ks_out) { // the caller's own kernel adds the partial tiles
-        *ks_out = KS;
-        return L2_OK;
-    }
-    if (KS > 1) {
-        hipLaunchKernelGGL(q4_gemm_reduce_kernel, dim3((unsigned)((rows + 1023) / 1024), B), dim3(256), 0, st, L, ss, ws, KS);
-        L2_HIP(hipGetLastError());
-    }
     return L2_OK;
 }
 
 } // namespace
 
-int q4_gemm_launch(Q4Launch &L, const XhList &xh_list_dev, const float *ss, float *ws, size_t ws_floats,
-                   hipStream_t st, int *ks_out) {
-    if (L.n_mats < 1 || L.n_mats > 3) return l2_fail(L2_ERR_ARG, "q4 gemm: n_mats=%d", L.n_mats);
-    if (L.in % 128 != 0 || L.in % L.group_size != 0) return l2_fail(L2_ERR_ARG, "q4 gemm: in=%d must be a multiple of 128", L.in);
+GemmShape gemm_shape_f16(const Q4Launch &L, int slice_batch) {
+    GemmShape s{};
+    const int B = L.batch, G = L.group_size;
+    s.rows = 128;
+    for (int i = 0; i < L.n_mats; i++) s.row_blocks += (L.m[i].out + 127) / 128;
+    // Up to 255 tokens a wave takes 64 of them: with 128 a chunk of 128 tokens is too few blocks for the chip
+    // (w1|w3 of 7B: 172 blocks on 256 CUs; the launches of a 128-token chunk are 7 % slower that way).  From
+    // 256 tokens on a wave takes 128 (within 256 registers: two blocks per CU): every weight is dequantised
+    // once per 128 tokens instead of twice, and there are blocks enough whatever the tile (w1|w3 of 7B at 512
+    // tokens: 115 against 129 us).
+    auto tile = [&](int n) { return G >= 64 && n >= 256 ? 128 : n > 32 ? 64 : 32; };
+    s.tokens = tile(B);
+    // K slices: as many as keep the grid within one round of 2 blocks per CU, whole groups per slice, at most 4.
+    // (Up to 8 fill the chip when a launch runs alone, but every slice is a partial tile that the consumer reads
+    // back: 34.4 k against 32.7 k tok/s on the 7B prompt, 19.9 k against 19.5 k on 13B, no change on 70B.)
+    const int kstep = G >= 128 ? 128 : 64;
+    const int n_grp = (L.in / kstep) / (G / kstep > 0 ? G / kstep : 1);
+    const int t_tiles = (slice_batch + tile(slice_batch) - 1) / tile(slice_batch);
+    // slices start on even groups
+    s.slices = std::max(1, std::min({2 * cu_count() / (s.row_blocks * t_tiles), 4, n_grp / 2}));
+    return s;
+}
+
+int gemm_launch_f16(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, int partials, hipStream_t st) {
+    if (L.in % 128 != 0) return l2_fail(L2_ERR_ARG, "q4 gemm: in=%d must be a multiple of 128", L.in);
     if (L.group_size >= 64 && (L.in / L.group_size) % 2 != 0)
         return l2_fail(L2_ERR_ARG, "q4 gemm: in=%d is an odd number of groups of %d", L.in, L.group_size);
     for (int i = 0; i < L.n_mats; i++)
         if (L.m[i].out % 32 != 0) return l2_fail(L2_ERR_ARG, "q4 gemm: out=%d must be a multiple of 32", L.m[i].out);
-    if (L.pair) return l2_fail(L2_ERR_ARG, "q4 gemm: pair launches are not supported");
     switch (L.group_size) {
-        case 32: return launch_gemm_g<32>(L, xh_list_dev, ss, ws, ws_floats, st, ks_out);
-        case 64: return launch_gemm_g<64>(L, xh_list_dev, ss, ws, ws_floats, st, ks_out);
-        case 128: return launch_gemm_g<128>(L, xh_list_dev, ss, ws, ws_floats, st, ks_out);
+        case 32: return launch_gemm_g<32>(L, xh, ss, ws, s, partials, st);
+        case 64: return launch_gemm_g<64>(L, xh, ss, ws, s, partials, st);
+        case 128: return launch_gemm_g<128>(L, xh, ss, ws, s, partials, st);
     }
     return l2_fail(L2_ERR_ARG, "q4 gemm: group size %d", L.group_size);
-}
-
-bool q4_gemm_supports(int in, int out, int group_size) {
-    if (in % 128 != 0 || out % 32 != 0 || group_size <= 0 || in % group_size != 0) return false;
-    // groups of 64 and 128: the group scales are fetched as aligned pairs
-    return group_size < 64 || (in / group_size) % 2 == 0;
-}
-
-int prep_f16_multi_launch(const PrepList &P, int n, int B, hipStream_t st) {
-    if (n % 8 || P.n_mats < 1 || P.n_mats > 3) return l2_fail(L2_ERR_ARG, "prep: n=%d, %d vectors", n, P.n_mats);
-    hipLaunchKernelGGL(prep_f16_kernel, dim3((n / 8 + 255) / 256, B, P.n_mats), dim3(256), 0, st, P, n);
-    L2_HIP(hipGetLastError());
-    return L2_OK;
-}
-
-int prep_f16_launch(void *out_f16, const float *x, const float *wn, int n, int B, hipStream_t st) {
-    PrepList P{};
-    P.out[0] = out_f16, P.x[0] = x, P.wn[0] = wn, P.n_mats = 1;
-    return prep_f16_multi_launch(P, n, B, st);
-}
-
-int rms_scale_launch(float *ss, const float *x, float eps, int dim, int B, hipStream_t st) {
-    hipLaunchKernelGGL(rms_scale_kernel, dim3(B), dim3(256), 0, st, ss, x, eps, dim);
-    L2_HIP(hipGetLastError());
-    return L2_OK;
-}
-
-int silu_scatter_launch(float *out, void *out_f16, const float *a, const float *c, const int32_t *scatter, int n,
-                        int B, hipStream_t st) {
-    if (out_f16) {
-        if (!scatter || n % 8 || (size_t)n * 2 > 60 * 1024)
-            return l2_fail(L2_ERR_ARG, "silu gate (fp16): n=%d needs a permutation and at most 60 KB of LDS", n);
-        static LdsLimit limit(48 * 1024);
-        L2_TRY(limit.ensure(reinterpret_cast<const void *>(silu_scatter_f16_kernel), (size_t)n * 2));
-        hipLaunchKernelGGL(silu_scatter_f16_kernel, dim3(B), dim3(1024), (size_t)n * 2, st, (_Float16 *)out_f16, a, c, scatter, n);
-    } else {
-        hipLaunchKernelGGL(silu_scatter_kernel, dim3((n + 255) / 256, B), dim3(256), 0, st, out, a, c, scatter, n);
-    }
-    L2_HIP(hipGetLastError());
-    return L2_OK;
-}
-
-int gemm_residual_norm_prep_launch(const ResNormPrep &A, hipStream_t st) {
-    if (A.KS < 1 || A.KS > 8 || A.out % 4 || A.n < 0 || A.n > 3)
-        return l2_fail(L2_ERR_ARG, "residual epilogue: %d slices, %d outputs, %d consumers", A.KS, A.out, A.n);
-    if (A.n == 0) return l2_fail(L2_ERR_ARG, "residual epilogue: no consumer");
-    const size_t lds = (size_t)A.n * A.out * sizeof(_Float16);
-    if (A.out % 8 || lds > 60 * 1024) return l2_fail(L2_ERR_ARG, "residual epilogue: %d outputs x %d consumers", A.out, A.n);
-    static LdsLimit limit(48 * 1024);
-    L2_TRY(limit.ensure(reinterpret_cast<const void *>(gemm_residual_norm_prep_kernel), lds));
-    hipLaunchKernelGGL(gemm_residual_norm_prep_kernel, dim3(A.B), dim3(1024), lds, st, A);
-    L2_HIP(hipGetLastError());
-    return L2_OK;
-}
-
-int gemm_rope_kv_launch(const RopeKvArgs &A, hipStream_t st) {
-    if (A.KS < 1 || A.KS > 8 || A.B < 1 || A.n_heads < A.n_kv_heads)
-        return l2_fail(L2_ERR_ARG, "q|k|v epilogue: %d slices, %d tokens", A.KS, A.B);
-    hipLaunchKernelGGL(gemm_rope_kv_kernel, dim3(A.B), dim3(1024), 0, st, A);
-    L2_HIP(hipGetLastError());
-    return L2_OK;
 }

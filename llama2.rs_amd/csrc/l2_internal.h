@@ -72,6 +72,8 @@ struct LdsLimit {
 
 // Position at which the prefill ladder 64/32/16/8/4/2 (src/inference.rs:78-127) leaves off.
 int l2_prefill_ladder_end(int n_prompt);
+// What the ladder computes: the cache rows of the positions before that.
+int l2_prefill_ladder(l2_model *m, l2_state *s, const int32_t *prompt, int n_prompt);
 
 // ---- device views ---------------------------------------------------------
 
@@ -165,21 +167,43 @@ bool q4_stream_supports(const Q4Launch &L);
 // matrix, no rmsnorm, the default fp32 streaming form, rows of at most four waves); otherwise the caller gathers.
 bool q4_gathers_in_kernel(const Q4Launch &L);
 
-// ---- prefill chunks through the matrix cores ---------------------------------
+// ---- batches through the matrix cores (kernels_gemm.hip) -----------------------
+// `planes` is 1 (activations rounded to fp16) or 3 (fp32 activations as three exact bf16 planes).  The activations of
+// a GEMM are [B][planes][gemm_padded(in)] 16-bit values in the layer's g_index order, zero beyond `in`.
+constexpr int kMaxGemmSlices = 16;
+constexpr int kGemmMaxDim = 16384, kGemmMaxHidden = 38912; // a row of floats in LDS
+__host__ __device__ inline int gemm_padded(int in) { return (in + 63) / 64 * 64; }
 
 struct XhList {
-    const void *p[3]; // per matrix of the launch: fp16 [B][in], g_index order, pair-interleaved (prep_f16_launch)
+    const void *p[3]; // activations per matrix of the launch
 };
-// Y = X W^T for a chunk of L.batch tokens; ss (per token, may be null) scales the rows of Y.
-// Epilogues as in the matvec (no pair launches).  ws: workspace of ws_floats floats for split-K partial
-// tiles (the launcher uses as many K slices as fit).
-// ks_out given: the kernel leaves its K slices as partial tiles [KS][B][out] in ws (also when KS is 1), no
-// reduction is launched, and *ks_out says how many there are.
-int q4_gemm_launch(Q4Launch &L, const XhList &xh, const float *ss, float *ws, size_t ws_floats, hipStream_t st,
-                   int *ks_out = nullptr);
+// How a launch is cut.  The results depend on `slices` alone, and that on slice_batch, the number of columns the
+// caller's chunk has: a pass over several chunks then gives what the chunks one by one would have given.
+struct GemmShape {
+    int rows, tokens, row_blocks, slices;
+};
+GemmShape gemm_shape(const Q4Launch &L, int slice_batch, int planes);
+GemmShape gemm_shape_f16(const Q4Launch &L, int slice_batch);
+// Y = X W^T for L.batch columns; ss (per column, may be null) scales them.  Epilogues: store, residual add.  ws:
+// workspace for the K slices' partial tiles.  ks_out given: the kernel leaves its slices as partial tiles [KS][B][out]
+// in ws (also when there is one), no reduction is launched, and *ks_out says how many there are.
+int gemm_launch(Q4Launch &L, const XhList &xh, const float *ss, float *ws, size_t ws_floats, int planes, int slice_batch,
+                hipStream_t st, int *ks_out = nullptr);
+int gemm_launch_f16(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, int partials, hipStream_t st);
+// What a first launch for this group size does besides enqueueing (for callers under graph capture).
+int gemm_warm_up(int group_size);
+
+struct GemmInput {
+    void *out[3];
+    const int32_t *g_index[3];
+    const float *x;  // [B][n], natural order
+    const float *wn; // [n] norm weight in natural order, or null
+    int n;           // consumers (1..3)
+};
+int gemm_input_launch(const GemmInput &A, int n, int B, int planes, hipStream_t st);
 
 struct ResNormPrep {
-    const float *ws;   // partial tiles [KS][B][out] of one matrix
+    const float *ws;   // partial tiles [KS][B][out] of one matrix, or null: the stream is already complete
     int KS, B, out;
     const float *res;  // [B][out] residual stream in
     float *x;          // [B][out] residual stream out (may be res)
@@ -188,9 +212,18 @@ struct ResNormPrep {
     int n;             // consumers (1..3)
     const int32_t *inv[3]; // inverse act-order permutation of each consumer
     const float *wn;       // [out] norm weight of the consumers' rmsnorm, in the order of the residual stream
-    void *out_h[3];        // [B][out] fp16, pair-interleaved, in each consumer's order
+    void *out_h[3];        // the consumers' activations
 };
-int gemm_residual_norm_prep_launch(const ResNormPrep &A, hipStream_t st);
+int gemm_residual_norm_launch(const ResNormPrep &A, int planes, hipStream_t st);
+
+struct SiluArgs {
+    const float *ws; // partial tiles of w1 and w3 laid end to end: [KS][B][n] each
+    int KS, B, n;
+    const float *ss; // [B] rms scale of the layer's input
+    const int32_t *inv; // inverse act-order permutation of w2
+    void *out_h;
+};
+int gemm_silu_launch(const SiluArgs &A, int planes, hipStream_t st);
 
 struct RopeKvArgs {
     const float *ws;   // partial tiles of q, k, v laid end to end: [KS][B][dim], [KS][B][kv_dim], [KS][B][kv_dim]
@@ -203,22 +236,12 @@ struct RopeKvArgs {
     int n_heads, n_kv_heads; // head size 128
 };
 int gemm_rope_kv_launch(const RopeKvArgs &A, hipStream_t st);
-bool q4_gemm_supports(int in, int out, int group_size);
-// out_f16[b][j'] = fp16(x[b][j] * (wn ? wn[j] : 1)), j' = j with the order (0,4,1,5,2,6,3,7) inside every 8.
-int prep_f16_launch(void *out_f16, const float *x, const float *wn, int n, int B, hipStream_t st);
-// The same for up to three vectors of one length in one launch (q|k|v, w1|w3 inputs).
-struct PrepList {
-    void *out[3];
-    const float *x[3];
-    const float *wn[3];
-    int n_mats;
-};
-int prep_f16_multi_launch(const PrepList &P, int n, int B, hipStream_t st);
-int rms_scale_launch(float *ss, const float *x, float eps, int dim, int B, hipStream_t st);
-// out[b][scatter[i]] = silu(a[b][i]) * c[b][i]; with out_f16 set the result goes there instead, as fp16 in
-// the pair-interleaved order the GEMM reads (no separate conversion pass).
-int silu_scatter_launch(float *out, void *out_f16, const float *a, const float *c, const int32_t *scatter, int n,
-                        int B, hipStream_t st);
+
+// Slot of element j of a vector in the order of a GEMM's bf16 planes: (0,2,4,6,1,3,5,7) inside every 8.
+__host__ __device__ inline int b16_slot(int j) {
+    const int e = j & 7;
+    return (j & ~7) | ((e >> 1) + 4 * (e & 1));
+}
 // Slot of element j of a vector in the fp16 pair-interleaved order: (0,4,1,5,2,6,3,7) inside every 8.
 __host__ __device__ inline int h16_slot(int j) {
     const int e = j & 7;
@@ -240,8 +263,9 @@ int gather_launch(float *out, const float *x, const int32_t *g_index, int n, int
 int rope_kv_launch(float *q, const float *k, const float *v, const int32_t *pos, const float *cos_t,
                    const float *sin_t, float *kcache_l, float *vcache_l, int n_heads, int n_kv_heads,
                    int head_size, int B, hipStream_t st);
-// Batched attention over an already written cache: out[b][scatter[i]] for query b at pos[b].
-int attention_launch(float *out, void *out_f16, const float *q, const float *kcache_l, const float *vcache_l,
+// Batched attention over an already written cache: out[b][scatter[i]] for query b at pos[b]; fp32 (planes 0), or the
+// 16-bit planes that a GEMM over `dim` inputs reads (1 or 3).
+int attention_launch(void *out, int planes, const float *q, const float *kcache_l, const float *vcache_l,
                      const int32_t *pos, const int32_t *scatter, int n_heads, int n_kv_heads,
                      int head_size, int max_pos, int B, hipStream_t st);
 

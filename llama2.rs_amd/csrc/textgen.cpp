@@ -280,16 +280,12 @@ extern "C" int l2_generate(l2_model *m, l2_state *s, const l2_tokenizer *t, cons
         L2_TRY(l2_state_reset(s));
         int pos = 0;
         if (prefill) { // :16-44, :78-127
-            std::vector<int32_t> toks(64), poss(64);
-            for (int A = 64; A >= 2; A /= 2)
-                while (pos + A < n_prompt) {
-                    for (int i = 0; i < A; i++) {
-                        toks[i] = pos == 0 ? 1 : prompt32[pos - 1];
-                        poss[i] = pos++;
-                        L2_TRY(emit(toks[i], toks[i], false)); // :37-40
-                    }
-                    L2_TRY(l2_forward(m, s, toks.data(), poss.data(), A, nullptr));
-                }
+            const int end = l2_prefill_ladder_end(n_prompt);
+            for (; pos < end; pos++) {
+                const int tok = pos == 0 ? 1 : prompt32[pos - 1];
+                L2_TRY(emit(tok, tok, false)); // :37-40
+            }
+            L2_TRY(l2_prefill_ladder(m, s, prompt32.data(), n_prompt));
         }
         int32_t token = pos == 0 ? 1 : prompt32[pos - 1];
         L2_TRY(emit(token, token, false)); // :134-137

@@ -165,7 +165,7 @@ class Model:
         check(lib().l2_state_reset(self.state))
 
     def set_prefill_mode(self, mode: int):
-        """_lib.PREFILL_FP32 (default, identical to B=1) or _lib.PREFILL_MFMA (fp16 tiles, 2e-3)."""
+        """_lib.PREFILL_FP32 (default, fp32 throughout) or _lib.PREFILL_MFMA (fp16 tiles, 2e-3)."""
         check(lib().l2_model_set_prefill_mode(self.h, mode))
 
     def set_step_graph(self, on: bool):

@@ -1,0 +1,60 @@
+"""Batches in fp32 through the matrix cores (three exact bf16 planes of the activations): the operator at the edges of
+its tiles against fp64, and whole prompts against the CPU oracle."""
+import numpy as np
+import pytest
+
+from llama2_rs import checkpoint as ck
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from llama2_rs import ops as o, _lib
+    assert _lib.lib().l2_device_count() >= 1, "no HIP device: the GPU tests cannot run"
+    return o
+
+
+def nrel(got, want):
+    want = np.asarray(want, np.float64)
+    scale = np.maximum(np.abs(want), np.sqrt(np.mean(want ** 2)) + 1e-30)
+    return float(np.max(np.abs(np.asarray(got, np.float64) - want) / scale))
+
+
+# rows: a last row block of 8 rows, of 128 and a whole one; inputs: half a K step at the end, an odd number of groups;
+# columns: both sides of the token tiles of 32 and 64, one and several K slices
+@pytest.mark.parametrize("n_in,n_out,G,batches", [
+    (4128, 4104, 32, (4, 31, 32, 33, 64, 65)), (4160, 4232, 64, (8, 130)), (4224, 8320, 128, (5, 61, 300)),
+    (13824, 1160, 128, (16,)), (1056, 29000, 32, (40,))])
+def test_batch_operator_vs_fp64(ops, n_in, n_out, G, batches):
+    rng = np.random.default_rng(n_in)
+    qw, qz, sc, gi = ck.synth_qlinear(rng, n_in, n_out, G, act_order=True)
+    W = ck.dequant_bin(qw, qz, sc, gi, G).astype(np.float64)
+    q = ops.QLinear(qw, qz, sc, gi, G)
+    for B in batches:
+        # columns of very different size, so that no column leans on another's range
+        x = (rng.standard_normal((B, n_in)) * 10.0 ** rng.uniform(-6, 6, (B, 1))).astype(np.float32)
+        want = x.astype(np.float64) @ W.T
+        got = q.matvec(x)
+        for b in range(B):
+            assert nrel(got[b], want[b]) < 1e-5, (B, b)
+        np.testing.assert_array_equal(q.matvec(x), got)
+    q.close()
+
+
+@pytest.mark.parametrize("kv,hidden,G,n", [(8, 2816, 32, 70), (4, 2848, 32, 64), (2, 2816, 64, 131), (1, 2816, 128, 97)])
+def test_fp32_prompt_vs_oracle(ops, oracle, kv, hidden, G, n):
+    dims = ck.Dims(dim=1024, hidden_dim=hidden, n_layers=2, n_heads=8, n_kv_heads=kv, vocab_size=300, seq_len=160, group_size=G)
+    img = ck.synth_weights_image(dims, seed=3)
+    m, o = ops.Model(img, dims), oracle.Model(img, dims)
+    toks = np.random.default_rng(n).integers(0, dims.vocab_size, size=n).astype(np.int32)
+    m.prefill_chunks(toks, 0, n)
+    o.new_state()
+    o.transformer(toks, np.arange(n, dtype=np.int32))
+    ko, vo = o.kv_cache()
+    for l in range(dims.n_layers):
+        k, v = m.read_kv(l, 0, n)
+        assert nrel(k, ko[l, :n]) < 1e-4 and nrel(v, vo[l, :n]) < 1e-4
+    assert nrel(m.forward([7], [n]), o.transformer([7], [n])) < 1e-4
+    m.close()
+    o.close()
