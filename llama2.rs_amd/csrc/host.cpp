@@ -760,10 +760,11 @@ static bool gemm_pays_layer(int B, double weights) { return B >= 8 && B * weight
 // What a batch of B columns of this model is computed with: 0 = the matvec kernels column by column, 1 or 3 = the GEMM
 // with that many planes of activations.
 static int batch_planes(const l2_model *m, int B) {
-    if (m->d.group_size == 0 || B < 2 || m->d.dim > kGemmMaxDim || m->d.hidden_dim > kGemmMaxHidden) return 0;
-    if (m->prefill_mode == L2_PREFILL_MFMA) return 1;
+    if (B < 2 || m->d.dim > kGemmMaxDim || m->d.hidden_dim > kGemmMaxHidden) return 0;
+    if (m->prefill_mode == L2_PREFILL_MFMA) return 1; // quantised models only
     const double dim = m->d.dim, weights = dim * (2 * dim + 2.0 * m->kv_dim + 3.0 * m->d.hidden_dim);
-    return gemm_pays_layer(B, weights) ? 3 : 0;
+    if (!gemm_pays_layer(B, weights)) return 0;
+    return m->d.group_size == 0 ? kDensePlanes : 3;
 }
 
 // The same for the stand-alone operator.
@@ -900,7 +901,7 @@ extern "C" int l2_state_fill_synthetic(l2_state *s, int pos0, int npos, uint64_t
 
 static Q4Mat mat_of(const DevQLinear &q, const float *x, const float *wn, float *y) {
     Q4Mat M{};
-    M.qweight = q.qweight;
+    M.qweight = q.dense ? reinterpret_cast<const uint4 *>(q.dense) : q.qweight;
     M.qzeros = q.qzeros;
     M.scales = q.scales;
     M.x = x;
@@ -1181,9 +1182,16 @@ extern "C" int l2_model_qmatvec(l2_model *m, int layer, int proj, const float *x
     if (q.dense) { // Linear::matvec<B> (src/model.rs:22-31)
         hipStream_t st = m->stream;
         L2_HIP(hipMemcpyAsync(m->op_x, x_host, (size_t)B * q.in * 4, hipMemcpyHostToDevice, st));
-        DenseArgs a{};
-        a.y = m->op_y, a.w = q.dense, a.x = m->op_x, a.in = q.in, a.out = q.out, a.batch = B;
-        L2_TRY(dense_launch(a, st));
+        if (operator_planes(q, B) && q.in == gemm_padded(q.in)) {
+            L2_TRY(operator_bufs(m->op_batch, q, B, kDensePlanes, st));
+            Q4Launch L = launch_of(q, B, 0.f);
+            L.m[0] = mat_of(q, nullptr, nullptr, m->op_y);
+            L2_TRY(gemm_launch(L, XhList{{m->op_x, nullptr, nullptr}}, nullptr, m->op_batch.ws, m->op_batch.ws_floats, kDensePlanes, B, st));
+        } else {
+            DenseArgs a{};
+            a.y = m->op_y, a.w = q.dense, a.x = m->op_x, a.in = q.in, a.out = q.out, a.batch = B;
+            L2_TRY(dense_launch(a, st));
+        }
         L2_HIP(hipMemcpyAsync(y_host, m->op_y, (size_t)B * q.out * 4, hipMemcpyDeviceToHost, st));
         L2_HIP(hipStreamSynchronize(st));
         return L2_OK;
@@ -1468,6 +1476,7 @@ static int forward_enqueue_gemm(l2_model *m, l2_state *s, int B, int max_pos, co
     const l2_dims &d = m->d;
     const int dim = d.dim, hid = d.hidden_dim, kvd = m->kv_dim, L = d.n_layers;
     const l2_model::ChunkBufs &b = m->lane[lane];
+    const bool dense = d.group_size == 0;
     hipStream_t st = lane ? m->extra_stream[lane - 1] : m->stream;
     auto gemm = [&](Q4Launch &Q, const XhList &X, const float *ss, int *ks) {
         return gemm_launch(Q, X, ss, b.ws, b.ws_floats, planes, slice_batch, st, ks);
@@ -1478,6 +1487,7 @@ static int forward_enqueue_gemm(l2_model *m, l2_state *s, int B, int max_pos, co
         R.ws = ks ? b.ws : nullptr, R.KS = ks ? ks : 1, R.B = B, R.out = dim, R.res = b.x, R.x = b.x, R.ss = b.ss, R.eps = m->rms_eps;
         R.n = 3, R.wn = m->rms_att + (size_t)l * dim;
         for (int c = 0; c < 3; c++) R.inv[c] = m->q[L2_WQ + c][l].inv_index, R.out_h[c] = b.h[c];
+        if (dense) R.n = 1; // no act-order: one input serves q, k and v
         return gemm_residual_norm_launch(R, planes, st);
     };
     {
@@ -1498,7 +1508,7 @@ static int forward_enqueue_gemm(l2_model *m, l2_state *s, int B, int max_pos, co
             Q.m[2] = mat_of(wv, nullptr, nullptr, nullptr);
             Q.n_mats = 3;
             RopeKvArgs R{};
-            L2_TRY(gemm(Q, XhList{{b.h[0], b.h[1], b.h[2]}}, nullptr, &R.KS));
+            L2_TRY(gemm(Q, dense ? XhList{{b.h[0], b.h[0], b.h[0]}} : XhList{{b.h[0], b.h[1], b.h[2]}}, nullptr, &R.KS));
             R.ws = b.ws, R.B = B, R.ss = b.ss, R.pos = dpos, R.cos_t = m->rope_cos, R.sin_t = m->rope_sin;
             R.q = b.q, R.kcache = kc, R.vcache = vc, R.n_heads = d.n_heads, R.n_kv_heads = d.n_kv_heads;
             L2_TRY(gemm_rope_kv_launch(R, st));
@@ -1516,7 +1526,7 @@ static int forward_enqueue_gemm(l2_model *m, l2_state *s, int B, int max_pos, co
             ResNormPrep R{};
             L2_TRY(gemm(Q, XhList{{b.h[0], nullptr, nullptr}}, nullptr, &R.KS));
             R.ws = b.ws, R.B = B, R.out = dim, R.res = b.x, R.x = b.x, R.ss = b.ss, R.eps = m->rms_eps;
-            R.n = 2, R.wn = m->rms_ffn + (size_t)l * dim;
+            R.n = dense ? 1 : 2, R.wn = m->rms_ffn + (size_t)l * dim;
             R.inv[0] = w1.inv_index, R.out_h[0] = b.h[0];
             R.inv[1] = w3.inv_index, R.out_h[1] = b.h[1];
             L2_TRY(gemm_residual_norm_launch(R, planes, st));
@@ -1527,7 +1537,7 @@ static int forward_enqueue_gemm(l2_model *m, l2_state *s, int B, int max_pos, co
             Q.m[1] = mat_of(w3, nullptr, nullptr, nullptr);
             Q.n_mats = 2;
             SiluArgs S{};
-            L2_TRY(gemm(Q, XhList{{b.h[0], b.h[1], nullptr}}, nullptr, &S.KS));
+            L2_TRY(gemm(Q, XhList{{b.h[0], dense ? b.h[0] : b.h[1], nullptr}}, nullptr, &S.KS));
             S.ws = b.ws, S.B = B, S.n = hid, S.ss = b.ss, S.inv = w2.inv_index, S.out_h = b.h[2];
             L2_TRY(gemm_silu_launch(S, planes, st));
         }

@@ -72,7 +72,10 @@ struct Piece {
 template <int NP>
 __device__ __forceinline__ Piece<NP> make_piece(const float (&v)[8]) {
     Piece<NP> r;
-    if constexpr (NP == 1) {
+    if constexpr (NP == kDensePlanes) {
+        r.q[0] = __builtin_bit_cast(uint4, make_float4(v[0], v[1], v[2], v[3]));
+        r.q[1] = __builtin_bit_cast(uint4, make_float4(v[4], v[5], v[6], v[7]));
+    } else if constexpr (NP == 1) {
         Frag f;
         f.p[0] = h2{(_Float16)v[0], (_Float16)v[4]};
         f.p[1] = h2{(_Float16)v[1], (_Float16)v[5]};
@@ -98,12 +101,12 @@ __device__ __forceinline__ Piece<NP> make_piece(const float (&v)[8]) {
     return r;
 }
 
-// Plane p of token t: [t][p][in_p], in_p = the row padded to whole K steps.
+// Plane p of token t: [t][p][in_p], in_p = the row padded to whole K steps (fp32: [t][in_p]).
 template <int NP>
 __device__ __forceinline__ void store_piece(void *out, size_t t, int in_p, int j8, const Piece<NP> &r) {
     uint4 *dst = reinterpret_cast<uint4 *>(reinterpret_cast<uint16_t *>(out) + t * NP * in_p);
 #pragma unroll
-    for (int p = 0; p < NP; p++) dst[p * (in_p >> 3) + j8] = r.q[p];
+    for (int p = 0; p < NP; p++) dst[NP == kDensePlanes ? 2 * j8 + p : p * (in_p >> 3) + j8] = r.q[p];
 }
 
 // x[b][g_index[j]] * wn[g_index[j]] -> planes: the gather of src/gptq.rs:110-114 and the norm weight of
@@ -132,6 +135,24 @@ __global__ __launch_bounds__(256) void gemm_input_kernel(const GemmInput A, int 
 }
 
 // ---- the GEMM ----------------------------------------------------------------------------------------------------
+
+// Four consecutive outputs of column t: a partial tile of this K slice, or the result through the launch's epilogue.
+__device__ __forceinline__ void finish4(const Q4Launch &L, int mi, const float *ss, float *ws, int KS, int ks, int partials,
+                                        int t, int o, float4 v) {
+    const int n_out = L.m[mi].out;
+    if (KS > 1 || partials) {
+        *reinterpret_cast<float4 *>(ws + ((size_t)ks * L.batch + t) * n_out + o) = v;
+        return;
+    }
+    const float sc = ss ? ss[t] : 1.0f;
+    v.x *= sc, v.y *= sc, v.z *= sc, v.w *= sc;
+    const size_t at = (size_t)t * n_out + o;
+    if (L.e.kind == Q4_EPI_RESIDUAL) {
+        const float4 rr = *reinterpret_cast<const float4 *>(L.e.res + at);
+        v.x += rr.x, v.y += rr.y, v.z += rr.z, v.w += rr.w;
+    }
+    *reinterpret_cast<float4 *>(L.m[mi].y + at) = v;
+}
 
 constexpr int kRowHalves = 72; // halves per staged token row: 64 k + 8 (16-byte reads of 32 lanes stay conflict-free)
 
@@ -365,19 +386,127 @@ __global__ __launch_bounds__(256, 2) void q4_tile_gemm_kernel(const Q4Launch L, 
                 const int tt = pass * 8 + tl;
                 float4 v = *reinterpret_cast<const float4 *>(&tile[tt * kTRow + oc]);
                 const int t = t0 + nb * 32 + tt, o = obase + mt * 32 + oc;
-                if (t >= B || o >= n_out) continue;
-                if (KS > 1 || partials) {
-                    *reinterpret_cast<float4 *>(ws + ws_base + ((size_t)ks * B + t) * n_out + o) = v;
-                    continue;
-                }
-                const float sc = ss ? ss[t] : 1.0f;
-                v.x *= sc, v.y *= sc, v.z *= sc, v.w *= sc;
-                const size_t at = (size_t)t * n_out + o;
-                if (L.e.kind == Q4_EPI_RESIDUAL) {
-                    const float4 rr = *reinterpret_cast<const float4 *>(L.e.res + at);
-                    v.x += rr.x, v.y += rr.y, v.z += rr.z, v.w += rr.w;
-                }
-                *reinterpret_cast<float4 *>(L.m[mi].y + at) = v;
+                if (t < B && o < n_out) finish4(L, mi, ss, ws + ws_base, KS, ks, partials, t, o, v);
+            }
+        }
+}
+
+// Linear::matvec<B> of the model without quantisation (src/model.rs:22-31) for a batch: fp32 weights, fp32 activations,
+// fp32 products and sums (v_mfma_f32_32x32x2_f32, 157 TFLOP/s on this chip; it is what bounds the kernel, the loads hide
+// behind it).  The matvec kernel once per column read the weights once per column: two layers of 7B's widths, 99 columns
+// 16 -> 1 ms.
+//
+// A block is four waves of MT x NB tiles of 32 rows x 32 columns, side by side over the rows.  Lane (r = l % 32,
+// h = l / 32) loads inputs 16 h .. 16 h + 15 of every 32 of its row, 16 bytes at a time; step e of float4 i multiplies
+// inputs 4 i + e and 16 + 4 i + e.  The activations' 32 inputs per column pass through LDS, double-buffered.
+template <int MT, int NB>
+__global__ __launch_bounds__(256, 2) void dense_gemm_kernel(const Q4Launch L, const XhList xl, int in_p,
+                                                            const float *__restrict__ ss, float *__restrict__ ws, int KS,
+                                                            int t_tiles, int partials) {
+    constexpr int TN = 32 * NB, RW = 32 * MT, RB = 4 * RW, kRow = 36; // floats per staged column: 32 + 4
+    __shared__ __align__(16) float xs[4608]; // [2][TN][kRow], and the four output tiles of the epilogue
+    static_assert(2 * TN * kRow <= 4608 && 4 * 32 * 36 <= 4608, "LDS");
+    const int n_blocks = gridDim.x, per_xcd = n_blocks >> 3, over = n_blocks & 7, xcd = blockIdx.x & 7;
+    const int work = xcd * per_xcd + min(xcd, over) + (blockIdx.x >> 3); // as in q4_tile_gemm_kernel
+    int rb = work / t_tiles, mi = 0;
+    const int t0 = (work - rb * t_tiles) * TN;
+    const int row_blocks = n_blocks / (t_tiles * KS), ks = rb / row_blocks;
+    rb -= ks * row_blocks;
+    while (mi + 1 < L.n_mats && rb >= L.m[mi].row_blocks) {
+        rb -= L.m[mi].row_blocks;
+        mi++;
+    }
+    const void *__restrict__ const xh = xl.p[mi];
+    const void *__restrict__ const w = L.m[mi].qweight;
+    asm volatile("" ::"s"(xh), "s"(w));
+    const int n_out = L.m[mi].out, in = L.in, B = L.batch;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 31, h = lane >> 5;
+    const int n_unit = in / 32;
+    const int it0 = (int)((long)n_unit * ks / KS), it1 = (int)((long)n_unit * (ks + 1) / KS);
+    const int obase = rb * RB + wave * RW;
+    uint32_t wrow[MT], xoff[NB];
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) wrow[mt] = ((uint32_t)min(obase + mt * 32 + r, n_out - 1) * (uint32_t)in + 16 * h) * 4u;
+#pragma unroll
+    for (int p = 0; p < NB; p++) xoff[p] = ((uint32_t)min(t0 + p * 32 + (tid >> 3), B - 1) * (uint32_t)in_p + (tid & 7) * 4) * 4u;
+    struct WStage {
+        float4 w[MT][4];
+    };
+    auto fetch_w = [&](int it, WStage &d) __attribute__((always_inline)) {
+        const uint32_t c = (uint32_t)min(it, it1 - 1) * 128u;
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) d.w[mt][i] = ld_at<float4>(w, wrow[mt] + c + 16u * i);
+    };
+    float4 xr[NB];
+    auto fetch_x = [&](int it) __attribute__((always_inline)) {
+#pragma unroll
+        for (int p = 0; p < NB; p++) xr[p] = ld_at<float4>(xh, xoff[p] + (uint32_t)min(it, it1 - 1) * 128u);
+    };
+    auto store_x = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int p = 0; p < NB; p++) *reinterpret_cast<float4 *>(xs + (buf * TN + p * 32 + (tid >> 3)) * kRow + (tid & 7) * 4) = xr[p];
+    };
+    f16v acc[MT][NB];
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+        for (int nb = 0; nb < NB; nb++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[mt][nb][i] = 0.f;
+    WStage wr[2];
+    fetch_x(it0);
+    fetch_w(it0, wr[0]);
+    store_x(0);
+    __syncthreads();
+    auto k_step = [&](const int it, const int u) __attribute__((always_inline)) {
+        fetch_x(it + 1);
+        fetch_w(it + 1, wr[u ^ 1]);
+        __builtin_amdgcn_sched_barrier(0); // requested before this step's arithmetic, not behind it
+        const float *xb = xs + u * TN * kRow;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            float4 b[NB];
+#pragma unroll
+            for (int nb = 0; nb < NB; nb++) b[nb] = *reinterpret_cast<const float4 *>(xb + (nb * 32 + r) * kRow + 16 * h + 4 * i);
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+#pragma unroll
+                for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+                    for (int nb = 0; nb < NB; nb++)
+                        acc[mt][nb] = __builtin_amdgcn_mfma_f32_32x32x2f32((&wr[u].w[mt][i].x)[e], (&b[nb].x)[e], acc[mt][nb], 0, 0, 0);
+        }
+        store_x(u ^ 1);
+        __syncthreads();
+    };
+    int it = it0;
+    for (; it + 1 < it1; it += 2) {
+        k_step(it, 0);
+        k_step(it + 1, 1);
+    }
+    if (it < it1) k_step(it, 0);
+
+    size_t ws_base = 0;
+    for (int i = 0; i < mi; i++) ws_base += (size_t)KS * B * L.m[i].out;
+    float *tile = xs + wave * 32 * 36;
+    const int tl = lane >> 3, oc = (lane & 7) * 4;
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+        for (int nb = 0; nb < NB; nb++) {
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                *reinterpret_cast<float4 *>(&tile[r * 36 + q * 8 + h * 4]) =
+                    make_float4(acc[mt][nb][4 * q], acc[mt][nb][4 * q + 1], acc[mt][nb][4 * q + 2], acc[mt][nb][4 * q + 3]);
+#pragma unroll
+            for (int pass = 0; pass < 4; pass++) {
+                const int tt = pass * 8 + tl;
+                float4 v = *reinterpret_cast<const float4 *>(&tile[tt * 36 + oc]);
+                const int t = t0 + nb * 32 + tt, o = obase + mt * 32 + oc;
+                if (t < B && o < n_out) finish4(L, mi, ss, ws + ws_base, KS, ks, partials, t, o, v);
             }
         }
 }
@@ -465,7 +594,7 @@ __global__ __launch_bounds__(1024) void gemm_residual_norm_kernel(const ResNormP
         for (int k = 0; k < kTrips; k++) {
             const int i4 = tid + k * 1024;
             if (i4 >= n4) continue;
-            const int4 id = *reinterpret_cast<const int4 *>(A.inv[c] + 4 * i4);
+            const int4 id = A.inv[c] ? *reinterpret_cast<const int4 *>(A.inv[c] + 4 * i4) : make_int4(4 * i4, 4 * i4 + 1, 4 * i4 + 2, 4 * i4 + 3);
             perm[id.x] = v[k].x, perm[id.y] = v[k].y, perm[id.z] = v[k].z, perm[id.w] = v[k].w;
         }
         __syncthreads();
@@ -543,7 +672,7 @@ __global__ __launch_bounds__(1024) void gemm_silu_kernel(const SiluArgs A) {
     const size_t slice = (size_t)A.B * n, row = (size_t)t * n;
     const float ss = A.ss[t];
     for (int i4 = tid; i4 < (n >> 2); i4 += 1024) {
-        const int4 id = *reinterpret_cast<const int4 *>(A.inv + 4 * i4);
+        const int4 id = A.inv ? *reinterpret_cast<const int4 *>(A.inv + 4 * i4) : make_int4(4 * i4, 4 * i4 + 1, 4 * i4 + 2, 4 * i4 + 3);
         const float4 a = sum_slices(A.ws + row + 4 * i4, slice, A.KS);
         const float4 c = sum_slices(A.ws + A.KS * slice + row + 4 * i4, slice, A.KS);
         const float as[4] = {a.x, a.y, a.z, a.w}, cs[4] = {c.x, c.y, c.z, c.w};
@@ -590,7 +719,6 @@ int ready_group() {
     size_t lds = 0;
     L2_TRY((ready_tile<G, 1, 1>(&lds)));
     L2_TRY((ready_tile<G, 1, 2>(&lds)));
-    L2_TRY((ready_tile<G, 2, 1>(&lds)));
     L2_TRY((ready_tile<G, 2, 2>(&lds)));
     return L2_OK;
 }
@@ -598,10 +726,8 @@ int ready_group() {
 template <int G>
 int launch_group(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, int partials, hipStream_t st) {
     for (int i = 0; i < L.n_mats; i++) L.m[i].row_blocks = (L.m[i].out + s.rows - 1) / s.rows;
-    if (s.rows == 256) {
-        if (s.tokens == 64) return launch_tile<G, 2, 2>(L, xh, ss, ws, s.slices, partials, s.row_blocks, st);
-        return launch_tile<G, 2, 1>(L, xh, ss, ws, s.slices, partials, s.row_blocks, st);
-    }
+    if (s.rows == 256)
+        return launch_tile<G, 2, 2>(L, xh, ss, ws, s.slices, partials, s.row_blocks, st);
     if (s.tokens == 64) return launch_tile<G, 1, 2>(L, xh, ss, ws, s.slices, partials, s.row_blocks, st);
     return launch_tile<G, 1, 1>(L, xh, ss, ws, s.slices, partials, s.row_blocks, st);
 }
@@ -613,6 +739,17 @@ int launch_fp32(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const
         case 128: return launch_group<128>(L, xh, ss, ws, s, partials, st);
     }
     return l2_fail(L2_ERR_ARG, "q4 gemm: group size %d", L.group_size);
+}
+
+int launch_dense(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, int partials, hipStream_t st) {
+    for (int i = 0; i < L.n_mats; i++) L.m[i].row_blocks = (L.m[i].out + s.rows - 1) / s.rows;
+    const int t_tiles = (L.batch + s.tokens - 1) / s.tokens, in_p = gemm_padded(L.in);
+    const dim3 grid(s.row_blocks * t_tiles * s.slices), block(256);
+    if (s.rows == 256 && s.tokens == 64) hipLaunchKernelGGL((dense_gemm_kernel<2, 2>), grid, block, 0, st, L, xh, in_p, ss, ws, s.slices, t_tiles, partials);
+    else if (s.tokens == 64) hipLaunchKernelGGL((dense_gemm_kernel<1, 2>), grid, block, 0, st, L, xh, in_p, ss, ws, s.slices, t_tiles, partials);
+    else hipLaunchKernelGGL((dense_gemm_kernel<1, 1>), grid, block, 0, st, L, xh, in_p, ss, ws, s.slices, t_tiles, partials);
+    L2_HIP(hipGetLastError());
+    return L2_OK;
 }
 
 } // namespace
@@ -627,7 +764,7 @@ GemmShape gemm_shape(const Q4Launch &L, int slice_batch, int planes) {
     if (planes == 1) return gemm_shape_f16(L, slice_batch);
     GemmShape s{};
     const int B = L.batch;
-    const int kstep = L.group_size > 64 ? L.group_size : 64, units = (gemm_padded(L.in) + kstep - 1) / kstep;
+    const int kstep = planes == kDensePlanes ? 32 : L.group_size > 64 ? L.group_size : 64, units = (gemm_padded(L.in) + kstep - 1) / kstep;
     auto slices = [&](int slots, int blocks, int most) { return std::max(1, std::min({slots / blocks, most, units / 2})); };
     // K slices: as many as keep the grid within one round of resident blocks.  Up to 32 columns the registers and the
     // LDS hold four blocks per CU of 128 rows, and the partial tiles are small; beyond, two of 256 rows.
@@ -647,11 +784,11 @@ GemmShape gemm_shape(const Q4Launch &L, int slice_batch, int planes) {
 int gemm_launch(Q4Launch &L, const XhList &xh, const float *ss, float *ws, size_t ws_floats, int planes, int slice_batch,
                 hipStream_t st, int *ks_out) {
     if (L.n_mats < 1 || L.n_mats > 3 || L.pair) return l2_fail(L2_ERR_ARG, "q4 gemm: n_mats=%d pair=%d", L.n_mats, L.pair);
-    if (L.in % 32 || L.in % L.group_size || L.batch < 1) return l2_fail(L2_ERR_ARG, "q4 gemm: in=%d batch=%d", L.in, L.batch);
+    if (L.in % 32 || (planes != kDensePlanes && L.in % L.group_size) || L.batch < 1) return l2_fail(L2_ERR_ARG, "q4 gemm: in=%d batch=%d", L.in, L.batch);
     if (L.e.kind == Q4_EPI_SCATTER_ONLY || L.e.n_scatter) return l2_fail(L2_ERR_ARG, "q4 gemm: no scatter epilogue");
     long rows = 0;
     for (int i = 0; i < L.n_mats; i++) {
-        if (L.m[i].out < 8 || L.m[i].out % 8 || (size_t)L.m[i].out * (L.in / 8) * 4 >= ((size_t)1 << 32))
+        if (L.m[i].out < 8 || L.m[i].out % 8 || (size_t)L.m[i].out * (planes == kDensePlanes ? L.in : L.in / 8) * 4 >= ((size_t)1 << 32))
             return l2_fail(L2_ERR_ARG, "q4 gemm: out=%d in=%d", L.m[i].out, L.in);
         rows += L.m[i].out;
     }
@@ -660,6 +797,8 @@ int gemm_launch(Q4Launch &L, const XhList &xh, const float *ss, float *ws, size_
         return l2_fail(L2_ERR_ARG, "q4 gemm: %d slices of %d x %ld in a workspace of %zu", s.slices, L.batch, rows, ws_floats);
     if (planes == 1)
         L2_TRY(gemm_launch_f16(L, xh, ss, ws, s, ks_out != nullptr, st));
+    else if (planes == kDensePlanes)
+        L2_TRY(launch_dense(L, xh, ss, ws, s, ks_out != nullptr, st));
     else
         L2_TRY(launch_fp32(L, xh, ss, ws, s, ks_out != nullptr, st));
     if (ks_out) {
@@ -708,7 +847,7 @@ int gemm_residual_norm_launch(const ResNormPrep &A, int planes, hipStream_t st) 
     if (A.KS < 1 || A.KS > kMaxGemmSlices || A.out % 32 || A.out > kGemmMaxDim || A.n < 1 || A.n > 3)
         return l2_fail(L2_ERR_ARG, "residual epilogue: %d slices, %d outputs, %d consumers", A.KS, A.out, A.n);
     static_assert(kGemmMaxDim <= kTrips * 4096, "a thread keeps its part of the row in registers");
-    return planes == 1 ? residual_norm<1>(A, st) : residual_norm<3>(A, st);
+    return planes == 1 ? residual_norm<1>(A, st) : planes == kDensePlanes ? residual_norm<kDensePlanes>(A, st) : residual_norm<3>(A, st);
 }
 
 int gemm_rope_kv_launch(const RopeKvArgs &A, hipStream_t st) {
@@ -732,5 +871,5 @@ static int silu(const SiluArgs &A, hipStream_t st) {
 int gemm_silu_launch(const SiluArgs &A, int planes, hipStream_t st) {
     if (A.KS < 1 || A.KS > kMaxGemmSlices || A.n % 32 || A.n > kGemmMaxHidden)
         return l2_fail(L2_ERR_ARG, "silu gate: %d slices, n=%d", A.KS, A.n);
-    return planes == 1 ? silu<1>(A, st) : silu<3>(A, st);
+    return planes == 1 ? silu<1>(A, st) : planes == kDensePlanes ? silu<kDensePlanes>(A, st) : silu<3>(A, st);
 }

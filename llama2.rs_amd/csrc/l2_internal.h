@@ -169,7 +169,9 @@ bool q4_gathers_in_kernel(const Q4Launch &L);
 
 // ---- batches through the matrix cores (kernels_gemm.hip) -----------------------
 // `planes` is 1 (activations rounded to fp16) or 3 (fp32 activations as three exact bf16 planes).  The activations of
-// a GEMM are [B][planes][gemm_padded(in)] 16-bit values in the layer's g_index order, zero beyond `in`.
+// a GEMM are [B][planes][gemm_padded(in)] 16-bit values in the layer's g_index order, zero beyond `in`.  The model
+// without quantisation has fp32 activations as they are, [B][gemm_padded(in)] floats: as much room as two planes.
+constexpr int kDensePlanes = 2;
 constexpr int kMaxGemmSlices = 16;
 constexpr int kGemmMaxDim = 16384, kGemmMaxHidden = 38912; // a row of floats in LDS
 __host__ __device__ inline int gemm_padded(int in) { return (in + 63) / 64 * 64; }
@@ -210,7 +212,7 @@ struct ResNormPrep {
     float *ss;         // [B] rms scale of the new residual stream
     float eps;
     int n;             // consumers (1..3)
-    const int32_t *inv[3]; // inverse act-order permutation of each consumer
+    const int32_t *inv[3]; // inverse act-order permutation of each consumer (null: none)
     const float *wn;       // [out] norm weight of the consumers' rmsnorm, in the order of the residual stream
     void *out_h[3];        // the consumers' activations
 };
@@ -220,7 +222,7 @@ struct SiluArgs {
     const float *ws; // partial tiles of w1 and w3 laid end to end: [KS][B][n] each
     int KS, B, n;
     const float *ss; // [B] rms scale of the layer's input
-    const int32_t *inv; // inverse act-order permutation of w2
+    const int32_t *inv; // inverse act-order permutation of w2 (null: none)
     void *out_h;
 };
 int gemm_silu_launch(const SiluArgs &A, int planes, hipStream_t st);
@@ -264,7 +266,7 @@ int rope_kv_launch(float *q, const float *k, const float *v, const int32_t *pos,
                    const float *sin_t, float *kcache_l, float *vcache_l, int n_heads, int n_kv_heads,
                    int head_size, int B, hipStream_t st);
 // Batched attention over an already written cache: out[b][scatter[i]] for query b at pos[b]; fp32 (planes 0), or the
-// 16-bit planes that a GEMM over `dim` inputs reads (1 or 3).
+// planes that a GEMM over `dim` inputs reads.
 int attention_launch(void *out, int planes, const float *q, const float *kcache_l, const float *vcache_l,
                      const int32_t *pos, const int32_t *scatter, int n_heads, int n_kv_heads,
                      int head_size, int max_pos, int B, hipStream_t st);

@@ -42,7 +42,8 @@ def test_batch_operator_vs_fp64(ops, n_in, n_out, G, batches):
     q.close()
 
 
-@pytest.mark.parametrize("kv,hidden,G,n", [(8, 2816, 32, 70), (4, 2848, 32, 64), (2, 2816, 64, 131), (1, 2816, 128, 97)])
+@pytest.mark.parametrize("kv,hidden,G,n", [(8, 2816, 32, 70), (4, 2848, 32, 64), (2, 2816, 64, 131), (1, 2816, 128, 97),
+                                             (2, 2816, 0, 66), (8, 2848, 0, 135)])
 def test_fp32_prompt_vs_oracle(ops, oracle, kv, hidden, G, n):
     dims = ck.Dims(dim=1024, hidden_dim=hidden, n_layers=2, n_heads=8, n_kv_heads=kv, vocab_size=300, seq_len=160, group_size=G)
     img = ck.synth_weights_image(dims, seed=3)
@@ -56,5 +57,10 @@ def test_fp32_prompt_vs_oracle(ops, oracle, kv, hidden, G, n):
         k, v = m.read_kv(l, 0, n)
         assert nrel(k, ko[l, :n]) < 1e-4 and nrel(v, vo[l, :n]) < 1e-4
     assert nrel(m.forward([7], [n]), o.transformer([7], [n])) < 1e-4
+    if G == 0:  # the dense operator on a batch, at a ragged number of columns
+        from llama2_rs import _lib
+        import tests.test_oracle_loop as tol
+        x = np.random.default_rng(1).standard_normal((33, 1024)).astype(np.float32)
+        assert nrel(m.qmatvec(1, _lib.W1, x), x.astype(np.float64) @ tol._split_image(img, dims)["w1"][1].T.astype(np.float64)) < 1e-5
     m.close()
     o.close()
