@@ -308,12 +308,23 @@ struct l2_model {
         size_t cap_B = 0, ws_floats = 0, h_bytes = 0;
     };
     int32_t *dtok = nullptr, *dpos = nullptr;
+    // Running maxima (value, index) of the classifier: step n of a loop folds into slot n % 2, so that the embedding
+    // kernel of step n + 1 can read one slot while it clears the other.
     unsigned long long *amax = nullptr;
+    // Pinned host memory that kernels read and write directly: a completion flag, logits, token ids, ids and positions
+    // on their way in.  The calls on one model are serialised and each waits for its work, so it is free between calls.
+    struct HostStage {
+        char *base = nullptr;
+        volatile uint32_t *flag = nullptr;
+        uint32_t seq = 0;
+        float *logits = nullptr;
+        int32_t *ids = nullptr, *in = nullptr; // [max_seq] out; [2 * max(max_seq, 4096)] in
+    } hs;
     static constexpr int kMaxLanes = 4; // the process has four hardware queues
     int n_lanes = 2;
     hipStream_t extra_stream[kMaxLanes - 1] = {nullptr, nullptr, nullptr};
     ChunkBufs lane[kMaxLanes];
-    int32_t *pf_tok = nullptr, *pf_pos = nullptr;
+    int32_t *pf_ids = nullptr; // ids, then positions, of a batch or prompt
     int cap_pf = 0;
     std::vector<hipEvent_t> pf_ev[kMaxLanes];
     hipEvent_t pf_join = nullptr;
@@ -403,6 +414,7 @@ struct l2_state {
     l2_model *m = nullptr;
     float *kcache = nullptr, *vcache = nullptr; // [L][max_seq][kv_dim]
     size_t elems = 0;
+    int rows = 0; // rows [0, rows) of every layer may have been written since the last reset; the others are zero
     std::map<int, StepGraph> steps; // captured decode step per upper bound of the position
 };
 
@@ -627,7 +639,19 @@ static int model_build(const char *weights, size_t nbytes, const l2_dims *dims, 
         M_HIP(hipMemcpy(m->rope_cos, c.data(), c.size() * 4, hipMemcpyHostToDevice));
         M_HIP(hipMemcpy(m->rope_sin, s.data(), s.size() * 4, hipMemcpyHostToDevice));
     }
-    M_TRY(dalloc(&m->amax, 1));
+    M_TRY(dalloc(&m->amax, 2));
+    {
+        const size_t logits = 256, ids = logits + ((size_t)dims->vocab_size * 4 + 255) / 256 * 256,
+                     in = ids + ((size_t)max_seq * 4 + 255) / 256 * 256, end = in + (size_t)std::max(max_seq, 4096) * 8;
+        void *p = nullptr;
+        M_HIP(hipHostMalloc(&p, end, hipHostMallocCoherent));
+        m->hs.base = (char *)p;
+        m->hs.flag = (volatile uint32_t *)m->hs.base;
+        *m->hs.flag = 0;
+        m->hs.logits = (float *)(m->hs.base + logits);
+        m->hs.ids = (int32_t *)(m->hs.base + ids);
+        m->hs.in = (int32_t *)(m->hs.base + in);
+    }
     M_HIP(hipDeviceSynchronize());
 #undef M_HIP
 #undef M_TRY
@@ -697,11 +721,11 @@ extern "C" void l2_model_close(l2_model *m) {
         void *bufs[] = {a.x, a.q, a.ss, a.ws, a.h[0], a.h[1], a.h[2]};
         for (void *p : bufs) dfree(p);
     }
-    dfree(m->pf_tok);
-    dfree(m->pf_pos);
+    dfree(m->pf_ids);
     for (auto &v : m->pf_ev)
         for (hipEvent_t e : v) (void)hipEventDestroy(e);
     if (m->pf_join) (void)hipEventDestroy(m->pf_join);
+    if (m->hs.base) (void)hipHostFree(m->hs.base);
     for (hipStream_t es : m->extra_stream)
         if (es) (void)hipStreamDestroy(es);
     if (m->stream) (void)hipStreamDestroy(m->stream);
@@ -816,6 +840,17 @@ static int ensure_batch(l2_model *m, int B) {
     return L2_OK;
 }
 
+// Device room for the ids and the positions of n tokens.
+static int ensure_ids(l2_model *m, int n) {
+    if (n <= m->cap_pf) return L2_OK;
+    L2_TRY(drain_streams(m));
+    dfree(m->pf_ids);
+    m->pf_ids = nullptr, m->cap_pf = 0;
+    L2_TRY(dalloc(&m->pf_ids, (size_t)n * 2));
+    m->cap_pf = n;
+    return L2_OK;
+}
+
 // ---------------------------------------------------------------------------
 // state
 
@@ -830,6 +865,7 @@ extern "C" int l2_state_new(l2_model *m, l2_state **out) {
         l2_state_free(s);
         return rc;
     }
+    s->rows = m->max_seq; // nothing is known of fresh memory
     rc = l2_state_reset(s);
     if (rc != L2_OK) {
         l2_state_free(s);
@@ -848,10 +884,17 @@ extern "C" void l2_state_free(l2_state *s) {
     delete s;
 }
 
+// Zeroes what has been written since the last reset, on the model's stream.
+static int state_clear(l2_state *s) {
+    const l2_model *m = s->m;
+    L2_TRY(clear_rows_launch(s->kcache, s->vcache, m->d.n_layers, (size_t)m->max_seq * m->kv_dim, (size_t)s->rows * m->kv_dim, m->stream));
+    s->rows = 0;
+    return L2_OK;
+}
+
 extern "C" int l2_state_reset(l2_state *s) {
     if (!s) return l2_fail(L2_ERR_ARG, "null state");
-    L2_HIP(hipMemsetAsync(s->kcache, 0, s->elems * 4, s->m->stream));
-    L2_HIP(hipMemsetAsync(s->vcache, 0, s->elems * 4, s->m->stream));
+    L2_TRY(state_clear(s));
     L2_HIP(hipStreamSynchronize(s->m->stream));
     return L2_OK;
 }
@@ -875,6 +918,7 @@ extern "C" int l2_state_write_kv(l2_state *s, int layer, int pos0, int npos, con
     if (layer < 0 || layer >= m->d.n_layers || pos0 < 0 || npos < 0 || pos0 + npos > m->max_seq)
         return l2_fail(L2_ERR_RANGE, "write_kv: layer %d, positions [%d,%d)", layer, pos0, pos0 + npos);
     const size_t off = ((size_t)layer * m->max_seq + pos0) * m->kv_dim;
+    s->rows = std::max(s->rows, pos0 + npos);
     L2_HIP(hipStreamSynchronize(m->stream));
     L2_HIP(hipMemcpy(s->kcache + off, k_host, (size_t)npos * m->kv_dim * 4, hipMemcpyHostToDevice));
     L2_HIP(hipMemcpy(s->vcache + off, v_host, (size_t)npos * m->kv_dim * 4, hipMemcpyHostToDevice));
@@ -886,6 +930,7 @@ extern "C" int l2_state_fill_synthetic(l2_state *s, int pos0, int npos, uint64_t
     const l2_model *m = s->m;
     if (pos0 < 0 || npos < 0 || pos0 + npos > m->max_seq)
         return l2_fail(L2_ERR_RANGE, "fill: positions [%d,%d)", pos0, pos0 + npos);
+    s->rows = std::max(s->rows, pos0 + npos);
     for (int l = 0; l < m->d.n_layers; l++) {
         const size_t off = ((size_t)l * m->max_seq + pos0) * m->kv_dim;
         const size_t n = (size_t)npos * m->kv_dim;
@@ -1234,8 +1279,8 @@ static void attn_split_policy(int n_t, int n_kv_heads, int *ts_out, int *n_split
     *n_splits_out = (n_t + ts - 1) / ts;
 }
 
-// Enqueue one forward pass for the B tokens / positions already in m->dtok /
-// m->dpos.  max_pos is the largest position among them (sizes the attention
+// Enqueue one forward pass for the B tokens of `src` at the positions dpos (device; B == 1 takes its position from
+// max_pos).  max_pos is the largest position among them (sizes the attention
 // scratch).  With want_logits the classifier and the running argmax follow.
 //
 // Five launches per layer when B == 1: q|k|v with the attention rmsnorm in
@@ -1243,7 +1288,13 @@ static void attn_split_policy(int n_t, int n_kv_heads, int *ts_out, int *n_split
 // residual add behind; w1|w3 with the ffn rmsnorm in front and the SiLU gate
 // behind; w2 with the residual add behind.  Every producer writes its result
 // in the input order (g_index) of whoever reads it next.
-static int forward_enqueue_dense(l2_model *m, l2_state *s, int B, int max_pos, bool want_logits);
+struct ForwardIn {
+    TokenSource src;
+    const int32_t *dpos = nullptr;
+    float *logits = nullptr;             // B == 1: where the logits go, or null
+    unsigned long long *amax = nullptr;  // and their running maximum
+};
+static int forward_enqueue_dense(l2_model *m, l2_state *s, int B, int max_pos, const ForwardIn &in);
 
 static int check_position(const l2_model *m, int max_pos) {
     // No kernel clamps a position: the RoPE table and the cache end at max_seq (the reference panics on its
@@ -1253,9 +1304,21 @@ static int check_position(const l2_model *m, int max_pos) {
     return L2_OK;
 }
 
-static int forward_enqueue(l2_model *m, l2_state *s, int B, int max_pos, bool want_logits) {
+// Waits for everything on the model's stream: a last, tiny kernel stores the call's number in pinned host memory
+// (and, with `amax`, the index of that running maximum in *id), and the host watches it there.  hipStreamSynchronize
+// takes 4.5 us longer to notice the same; it is the way out where the number does not come (a failed launch), and
+// reports why.
+static int wait_host(l2_model *m, const unsigned long long *amax, int32_t *id) {
+    const uint32_t seq = ++m->hs.seq;
+    L2_TRY(finish_launch(amax, id, const_cast<uint32_t *>(m->hs.flag), seq, m->stream));
+    if (!watch_flag(m->hs.flag, seq)) L2_HIP(hipStreamSynchronize(m->stream));
+    return L2_OK;
+}
+
+static int forward_enqueue(l2_model *m, l2_state *s, int B, int max_pos, const ForwardIn &in) {
     L2_TRY(check_position(m, max_pos));
-    if (m->d.group_size == 0) return forward_enqueue_dense(m, s, B, max_pos, want_logits);
+    s->rows = std::max(s->rows, max_pos + 1);
+    if (m->d.group_size == 0) return forward_enqueue_dense(m, s, B, max_pos, in);
     const l2_dims &d = m->d;
     const int dim = d.dim, hid = d.hidden_dim, kvd = m->kv_dim, L = d.n_layers;
     hipStream_t st = m->stream;
@@ -1264,7 +1327,7 @@ static int forward_enqueue(l2_model *m, l2_state *s, int B, int max_pos, bool wa
         t.n = 3;
         t.inv[0] = m->q[L2_WQ][0].inv_index, t.inv[1] = m->q[L2_WK][0].inv_index, t.inv[2] = m->q[L2_WV][0].inv_index;
         t.out[0] = m->xq, t.out[1] = m->xk, t.out[2] = m->xv;
-        LAUNCH(K_EMBED, embed_launch(m->x, m->tok_emb, m->dtok, dim, B, t, m->amax, st));
+        LAUNCH(K_EMBED, embed_launch(m->x, m->tok_emb, in.src, dim, B, t, in.amax, st));
     }
     for (int l = 0; l < L; l++) {
         const DevQLinear &wq = m->q[L2_WQ][l], &wk = m->q[L2_WK][l], &wv = m->q[L2_WV][l],
@@ -1297,9 +1360,9 @@ static int forward_enqueue(l2_model *m, l2_state *s, int B, int max_pos, bool wa
                 return l2_fail(L2_ERR_RANGE, "attention: position %d needs %d splits", max_pos, a.n_splits);
             LAUNCH(K_ATTENTION, attention_decode_launch(a, st));
         } else {
-            LAUNCH(K_ROPE_KV, rope_kv_launch(m->qv, m->kv, m->vv, m->dpos, m->rope_cos, m->rope_sin, kc, vc, d.n_heads,
+            LAUNCH(K_ROPE_KV, rope_kv_launch(m->qv, m->kv, m->vv, in.dpos, m->rope_cos, m->rope_sin, kc, vc, d.n_heads,
                                              d.n_kv_heads, m->head_size, B, st));
-            LAUNCH(K_ATTENTION, attention_launch(m->attg, 0, m->qv, kc, vc, m->dpos, wo.inv_index, d.n_heads,
+            LAUNCH(K_ATTENTION, attention_launch(m->attg, 0, m->qv, kc, vc, in.dpos, wo.inv_index, d.n_heads,
                                                  d.n_kv_heads, m->head_size, max_pos, B, st));
         }
         {   // wo (:260) + residual (:263-264); the new x also goes out in w1's and w3's order
@@ -1338,22 +1401,22 @@ static int forward_enqueue(l2_model *m, l2_state *s, int B, int max_pos, bool wa
         }
         (void)hid;
     }
-    if (want_logits) // final rmsnorm + classifier (:288-297, B == 1 only) + running argmax
-        LAUNCH(K_CLASSIFIER, dense_matvec_launch(m->logits, m->wcls, m->x, m->rms_final, m->rms_eps, dim,
-                                                 d.vocab_size, m->amax, st));
+    if (in.logits) // final rmsnorm + classifier (:288-297, B == 1 only) + running argmax
+        LAUNCH(K_CLASSIFIER, dense_matvec_launch(in.logits, m->wcls, m->x, m->rms_final, m->rms_eps, dim,
+                                                 d.vocab_size, in.amax, st));
     return L2_OK;
 }
 
 // The same schedule for the model without quantisation (TransformerWeights, src/model.rs:36-67):
 // every projection is a dense matvec with its rmsnorm in front (q, k, v, w1, w3), the SiLU gate behind
 // (w3) or the residual add behind (wo, w2).  No act-order, so nothing is scattered.
-static int forward_enqueue_dense(l2_model *m, l2_state *s, int B, int max_pos, bool want_logits) {
+static int forward_enqueue_dense(l2_model *m, l2_state *s, int B, int max_pos, const ForwardIn &in) {
     const l2_dims &d = m->d;
     const int dim = d.dim, hid = d.hidden_dim, kvd = m->kv_dim, L = d.n_layers;
     hipStream_t st = m->stream;
     {
         ScatterTargets t{};
-        LAUNCH(K_EMBED, embed_launch(m->x, m->tok_emb, m->dtok, dim, B, t, m->amax, st));
+        LAUNCH(K_EMBED, embed_launch(m->x, m->tok_emb, in.src, dim, B, t, in.amax, st));
     }
     auto dense = [&](const DevQLinear &w, const float *x, const float *wn, float *y, const float *res,
                      const float *gate) {
@@ -1385,9 +1448,9 @@ static int forward_enqueue_dense(l2_model *m, l2_state *s, int B, int max_pos, b
                 return l2_fail(L2_ERR_RANGE, "attention: position %d needs %d splits", max_pos, a.n_splits);
             LAUNCH(K_ATTENTION, attention_decode_launch(a, st));
         } else {
-            LAUNCH(K_ROPE_KV, rope_kv_launch(m->qv, m->kv, m->vv, m->dpos, m->rope_cos, m->rope_sin, kc, vc, d.n_heads,
+            LAUNCH(K_ROPE_KV, rope_kv_launch(m->qv, m->kv, m->vv, in.dpos, m->rope_cos, m->rope_sin, kc, vc, d.n_heads,
                                              d.n_kv_heads, m->head_size, B, st));
-            LAUNCH(K_ATTENTION, attention_launch(m->attg, 0, m->qv, kc, vc, m->dpos, nullptr, d.n_heads,
+            LAUNCH(K_ATTENTION, attention_launch(m->attg, 0, m->qv, kc, vc, in.dpos, nullptr, d.n_heads,
                                                  d.n_kv_heads, m->head_size, max_pos, B, st));
         }
         LAUNCH(K_Q4_WO, dense(m->q[L2_WO][l], m->attg, nullptr, m->x, m->x, nullptr));       // :260-264
@@ -1396,9 +1459,9 @@ static int forward_enqueue_dense(l2_model *m, l2_state *s, int B, int max_pos, b
         LAUNCH(K_Q4_W2, dense(m->q[L2_W2][l], m->hg, nullptr, m->x, m->x, nullptr));          // :279-285
         (void)hid;
     }
-    if (want_logits)
-        LAUNCH(K_CLASSIFIER, dense_matvec_launch(m->logits, m->wcls, m->x, m->rms_final, m->rms_eps, dim,
-                                                 d.vocab_size, m->amax, st));
+    if (in.logits)
+        LAUNCH(K_CLASSIFIER, dense_matvec_launch(in.logits, m->wcls, m->x, m->rms_final, m->rms_eps, dim,
+                                                 d.vocab_size, in.amax, st));
     return L2_OK;
 }
 
@@ -1475,6 +1538,7 @@ static int forward_enqueue_gemm(l2_model *m, l2_state *s, int B, int max_pos, co
                                 int planes, int slice_batch, int lane, const hipEvent_t *after_kv,
                                 const hipEvent_t *before_attn) {
     L2_TRY(check_position(m, max_pos));
+    s->rows = std::max(s->rows, max_pos + 1);
     const l2_dims &d = m->d;
     const int dim = d.dim, hid = d.hidden_dim, kvd = m->kv_dim, L = d.n_layers;
     const l2_model::ChunkBufs &b = m->lane[lane];
@@ -1494,7 +1558,9 @@ static int forward_enqueue_gemm(l2_model *m, l2_state *s, int B, int max_pos, co
     };
     {
         ScatterTargets t{};
-        L2_TRY(embed_launch(b.x, m->tok_emb, dtok, dim, B, t, nullptr, st));
+        TokenSource src;
+        src.tokens = dtok;
+        L2_TRY(embed_launch(b.x, m->tok_emb, src, dim, B, t, nullptr, st));
         L2_TRY(attn_inputs(0, 0));
     }
     for (int l = 0; l < L; l++) {
@@ -1561,11 +1627,15 @@ static int forward_enqueue_gemm(l2_model *m, l2_state *s, int B, int max_pos, co
 }
 
 // transformer<B> on the model's stream for B > 1 tokens and positions already in device memory.
-static int forward_batch(l2_model *m, l2_state *s, int B, int max_pos) {
+static int forward_batch(l2_model *m, l2_state *s, int B, int max_pos, const int32_t *dtok, const int32_t *dpos) {
     const int planes = batch_planes(m, B);
-    if (!planes) return forward_enqueue(m, s, B, max_pos, false);
+    if (!planes) {
+        ForwardIn in;
+        in.src.tokens = dtok, in.dpos = dpos;
+        return forward_enqueue(m, s, B, max_pos, in);
+    }
     L2_TRY(ensure_lane(m, 0, B, B, planes));
-    return forward_enqueue_gemm(m, s, B, max_pos, m->dtok, m->dpos, planes, B, 0, nullptr, nullptr);
+    return forward_enqueue_gemm(m, s, B, max_pos, dtok, dpos, planes, B, 0, nullptr, nullptr);
 }
 
 static int check_tokens(const l2_model *m, const int32_t *tokens, const int32_t *pos, int B, int *max_pos) {
@@ -1589,20 +1659,25 @@ extern "C" int l2_forward(l2_model *m, l2_state *s, const int32_t *tokens, const
     int max_pos = 0;
     L2_TRY(check_tokens(m, tokens, pos, B, &max_pos));
     L2_TRY(ensure_batch(m, B));
-    L2_HIP(hipMemcpyAsync(m->dtok, tokens, (size_t)B * 4, hipMemcpyHostToDevice, m->stream));
-    L2_HIP(hipMemcpyAsync(m->dpos, pos, (size_t)B * 4, hipMemcpyHostToDevice, m->stream));
-    if (B > 1)
-        L2_TRY(forward_batch(m, s, B, max_pos));
-    else
-        L2_TRY(forward_enqueue(m, s, B, max_pos, true));
-    if (B == 1 && logits_host)
-        L2_HIP(hipMemcpyAsync(logits_host, m->logits, (size_t)m->d.vocab_size * 4, hipMemcpyDeviceToHost, m->stream));
-    L2_HIP(hipStreamSynchronize(m->stream));
+    if (B > 1) {
+        L2_TRY(ensure_ids(m, B));
+        memcpy(m->hs.in, tokens, (size_t)B * 4);
+        memcpy(m->hs.in + B, pos, (size_t)B * 4);
+        L2_HIP(hipMemcpyAsync(m->pf_ids, m->hs.in, (size_t)B * 8, hipMemcpyHostToDevice, m->stream));
+        L2_TRY(forward_batch(m, s, B, max_pos, m->pf_ids, m->pf_ids + B));
+        return wait_host(m, nullptr, nullptr);
+    }
+    ForwardIn in;
+    in.src.token = tokens[0];
+    in.logits = logits_host ? m->hs.logits : m->logits, in.amax = m->amax;
+    L2_TRY(forward_enqueue(m, s, 1, max_pos, in));
+    L2_TRY(wait_host(m, nullptr, nullptr));
+    if (logits_host) memcpy(logits_host, m->hs.logits, (size_t)m->d.vocab_size * 4);
     return L2_OK;
 }
 
-// The lanes of l2_prefill_chunks (streams, events, buffers) and room for the whole prompt's ids and positions.
-static int ensure_prefill_pipeline(l2_model *m, int lanes, int B, int slice_batch, int planes, int n) {
+// The lanes of l2_prefill_chunks: streams, events, buffers.
+static int ensure_prefill_pipeline(l2_model *m, int lanes, int B, int slice_batch, int planes) {
     for (int i = 0; i + 1 < lanes; i++)
         if (!m->extra_stream[i]) L2_HIP(hipStreamCreate(&m->extra_stream[i])); // default priority, as the model's own
     if (!m->pf_join) L2_HIP(hipEventCreateWithFlags(&m->pf_join, hipEventDisableTiming));
@@ -1613,14 +1688,6 @@ static int ensure_prefill_pipeline(l2_model *m, int lanes, int B, int slice_batc
             m->pf_ev[i].push_back(e);
         }
         if (planes) L2_TRY(ensure_lane(m, i, B, slice_batch, planes));
-    }
-    if (n > m->cap_pf) {
-        L2_TRY(drain_streams(m));
-        dfree(m->pf_tok), dfree(m->pf_pos);
-        m->pf_tok = m->pf_pos = nullptr, m->cap_pf = 0;
-        L2_TRY(dalloc(&m->pf_tok, (size_t)n));
-        L2_TRY(dalloc(&m->pf_pos, (size_t)n));
-        m->cap_pf = n;
     }
     return L2_OK;
 }
@@ -1637,7 +1704,7 @@ static constexpr int kPassTokens = 512;
 // weights are read and dequantised once per pass.  Passes run on n_lanes streams, each with buffers of its own: a pass
 // needs from its predecessor only the cache rows of the same layer (an event per layer), so every pass follows one layer
 // behind the one before it and its kernels fill the compute units that the others' short launches leave idle.
-extern "C" int l2_prefill_chunks(l2_model *m, l2_state *s, const int32_t *tokens, int n, int pos0, int chunk) {
+static int prefill_chunks(l2_model *m, l2_state *s, const int32_t *tokens, int n, int pos0, int chunk, bool wait) {
     if (!m || !s || !tokens) return l2_fail(L2_ERR_ARG, "null argument");
     if (s->m != m) return l2_fail(L2_ERR_ARG, "state belongs to another model");
     if (n < 1 || chunk < 1 || chunk > 4096) return l2_fail(L2_ERR_RANGE, "%d tokens in chunks of %d (1..4096)", n, chunk);
@@ -1665,13 +1732,16 @@ extern "C" int l2_prefill_chunks(l2_model *m, l2_state *s, const int32_t *tokens
     for (const PrefillPass &p : passes)
         if (p.planes) widest = std::max(widest, p.n), cut = cut ? std::min(cut, p.slice_batch) : p.slice_batch, planes = p.planes;
     L2_TRY(ensure_batch(m, std::max(rest, 1)));
-    L2_TRY(ensure_prefill_pipeline(m, lanes, widest, cut, planes, n));
-    std::vector<int32_t> pos((size_t)n);
-    for (int i = 0; i < n; i++) pos[(size_t)i] = pos0 + i;
-    // synchronous copies: the host arrays are the caller's and this function's own
-    L2_HIP(hipStreamSynchronize(m->stream));
-    L2_HIP(hipMemcpy(m->pf_tok, tokens, (size_t)n * 4, hipMemcpyHostToDevice));
-    L2_HIP(hipMemcpy(m->pf_pos, pos.data(), (size_t)n * 4, hipMemcpyHostToDevice));
+    L2_TRY(ensure_prefill_pipeline(m, lanes, widest, cut, planes));
+    L2_TRY(ensure_ids(m, n));
+    memcpy(m->hs.in, tokens, (size_t)n * 4);
+    for (int i = 0; i < n; i++) m->hs.in[n + i] = pos0 + i;
+    const int32_t *dtok = m->pf_ids, *dpos = m->pf_ids + n;
+    L2_HIP(hipMemcpyAsync(m->pf_ids, m->hs.in, (size_t)n * 8, hipMemcpyHostToDevice, m->stream));
+    if (lanes > 1) { // the other lanes start behind what the model's stream has been given so far
+        L2_HIP(hipEventRecord(m->pf_join, m->stream));
+        for (int i = 0; i + 1 < lanes; i++) L2_HIP(hipStreamWaitEvent(m->extra_stream[i], m->pf_join, 0));
+    }
     // Everything that is enqueued on the two streams; a failure half-way returns through the caller below, which
     // first waits for what earlier chunks already have in flight on either stream.
     // the model's stream waits for everything the other lanes have been given so far
@@ -1688,15 +1758,15 @@ extern "C" int l2_prefill_chunks(l2_model *m, l2_state *s, const int32_t *tokens
             const int max_pos = pos0 + p.first + p.n - 1;
             if (p.planes) {
                 const int lane = c % lanes, before = (c + lanes - 1) % lanes;
-                L2_TRY(forward_enqueue_gemm(m, s, p.n, max_pos, m->pf_tok + p.first, m->pf_pos + p.first, p.planes, p.slice_batch,
+                L2_TRY(forward_enqueue_gemm(m, s, p.n, max_pos, dtok + p.first, dpos + p.first, p.planes, p.slice_batch,
                                             lane, passes.size() > 1 ? m->pf_ev[lane].data() : nullptr, c > 0 ? m->pf_ev[before].data() : nullptr));
                 c++;
             } else {
                 // few columns: the matvec kernels on the model's stream, behind everything
                 L2_TRY(join_lanes());
-                L2_HIP(hipMemcpyAsync(m->dtok, m->pf_tok + p.first, (size_t)p.n * 4, hipMemcpyDeviceToDevice, m->stream));
-                L2_HIP(hipMemcpyAsync(m->dpos, m->pf_pos + p.first, (size_t)p.n * 4, hipMemcpyDeviceToDevice, m->stream));
-                L2_TRY(forward_enqueue(m, s, p.n, max_pos, false));
+                ForwardIn in;
+                in.src.tokens = dtok + p.first, in.dpos = dpos + p.first;
+                L2_TRY(forward_enqueue(m, s, p.n, max_pos, in));
             }
         }
         return join_lanes();
@@ -1714,13 +1784,15 @@ extern "C" int l2_prefill_chunks(l2_model *m, l2_state *s, const int32_t *tokens
         memcpy(g_err, keep, sizeof keep);
         return rc;
     }
-    L2_HIP(hipStreamSynchronize(m->stream));
-    return L2_OK;
+    return wait ? wait_host(m, nullptr, nullptr) : L2_OK;
 }
 
-static int ensure_loop_buffers(l2_model *m, int n_prompt, int n_out);
-static int loop_begin(l2_model *m, int n_prompt, int pos0);
-static int loop_step(l2_model *m, l2_state *s, int pos, int n_prompt, int pos0);
+extern "C" int l2_prefill_chunks(l2_model *m, l2_state *s, const int32_t *tokens, int n, int pos0, int chunk) {
+    return prefill_chunks(m, s, tokens, n, pos0, chunk, true);
+}
+
+static int steps_enqueue(l2_model *m, l2_state *s, int32_t first, int pos0, int n, const int32_t *prompt, int n_prompt);
+static int steps_collect(l2_model *m, int pos0, int n, const int32_t *prompt, int n_prompt, int32_t *ids);
 
 extern "C" int l2_decode_greedy(l2_model *m, l2_state *s, int32_t token, int32_t pos, int32_t *next) {
     if (!m || !s || !next) return l2_fail(L2_ERR_ARG, "null argument");
@@ -1728,15 +1800,8 @@ extern "C" int l2_decode_greedy(l2_model *m, l2_state *s, int32_t token, int32_t
     int max_pos = 0;
     L2_TRY(check_tokens(m, &token, &pos, 1, &max_pos));
     L2_TRY(ensure_batch(m, 1));
-    L2_TRY(ensure_loop_buffers(m, 1, 1));
-    L2_TRY(set_i32_launch(m->dtok, token, m->dpos, pos, m->stream));
-    L2_TRY(loop_begin(m, 0, pos));
-    L2_TRY(loop_step(m, s, pos, 0, pos)); // the argmax stays in m->amax; the hand-over it also does is harmless
-    unsigned long long key = 0;
-    L2_HIP(hipMemcpyAsync(&key, m->amax, 8, hipMemcpyDeviceToHost, m->stream));
-    L2_HIP(hipStreamSynchronize(m->stream));
-    *next = (int32_t)(key & 0xFFFFFFFFull);
-    return L2_OK;
+    L2_TRY(steps_enqueue(m, s, token, pos, 1, nullptr, 0));
+    return steps_collect(m, pos, 1, nullptr, 0, next);
 }
 
 static int ensure_loop_buffers(l2_model *m, int n_prompt, int n_out) {
@@ -1761,17 +1826,6 @@ static int ensure_loop_buffers(l2_model *m, int n_prompt, int n_out) {
     return L2_OK;
 }
 
-// The B=1 loop body with everything on the device: forward from m->dtok at
-// m->dpos (== pos, which the host tracks only to size the attention scratch),
-// then next = prompt[pos] if still inside the prompt else argmax
-// (src/inference.rs:146-162), stored to out_ids[pos - pos0], fed back as the
-// token, and the device position advanced.
-static int loop_step_eager(l2_model *m, l2_state *s, int pos, int n_prompt, int pos0) {
-    L2_TRY(forward_enqueue(m, s, 1, pos, true));
-    LAUNCH(K_NEXT_TOKEN, next_token_launch(m->amax, m->dprompt, n_prompt, m->dpos, m->dout_ids, pos0, m->dtok, m->stream));
-    return L2_OK;
-}
-
 static void step_graph_drop(StepGraph &g) {
     if (g.exec) (void)hipGraphExecDestroy(g.exec);
     if (g.graph) (void)hipGraphDestroy(g.graph);
@@ -1790,7 +1844,11 @@ static int step_graph_get(l2_model *m, l2_state *s, int upper, hipGraphExec_t *o
     step_graph_drop(g);
     L2_HIP(hipStreamBeginCapture(m->stream, hipStreamCaptureModeRelaxed));
     m->capturing = true;
-    int rc = forward_enqueue(m, s, 1, upper - 1, true);
+    ForwardIn in;
+    in.src.tokens = m->dtok, in.logits = m->logits, in.amax = m->amax;
+    const int rows = s->rows; // capturing writes nothing
+    int rc = forward_enqueue(m, s, 1, upper - 1, in);
+    s->rows = rows;
     if (rc == L2_OK)
         rc = next_token_launch(m->amax, m->dprompt, 0, m->dpos, m->dout_ids, 0, m->dtok, m->stream, m->dloop);
     m->capturing = false;
@@ -1820,17 +1878,59 @@ static int step_bucket(const l2_model *m, int pos) {
     return (int)upper;
 }
 
-// One step of a loop whose {n_prompt, pos0} are already in m->dloop (loop_begin).
-static int loop_step(l2_model *m, l2_state *s, int pos, int n_prompt, int pos0) {
-    if (!m->use_graph || m->prof_on) return loop_step_eager(m, s, pos, n_prompt, pos0);
-    hipGraphExec_t exec = nullptr;
-    L2_TRY(step_graph_get(m, s, step_bucket(m, pos), &exec));
-    L2_HIP(hipGraphLaunch(exec, m->stream));
+// The B = 1 loop (src/inference.rs:141-162) with everything on the device: n steps from token `first` at position pos0,
+// each one's next token being prompt[pos] while that is inside the prompt, else the argmax.
+//
+// Launched: the embedding kernel of a step takes the step before's argmax itself and records it (in pinned host memory),
+// so a step is its layers' launches, one in front and the classifier.  Forced tokens travel as kernel arguments.
+// As graphs: see step_graph_get.
+static int steps_enqueue(l2_model *m, l2_state *s, int32_t first, int pos0, int n, const int32_t *prompt, int n_prompt) {
+    if (m->use_graph && !m->prof_on) {
+        L2_TRY(ensure_loop_buffers(m, std::max(n_prompt, 1), std::max(n, 1)));
+        if (n_prompt > 0) {
+            L2_HIP(hipStreamSynchronize(m->stream)); // a prefill before may still be reading its ids there
+            memcpy(m->hs.in, prompt, (size_t)std::min(n_prompt, m->max_seq) * 4);
+            L2_HIP(hipMemcpyAsync(m->dprompt, m->hs.in, (size_t)std::min(n_prompt, m->max_seq) * 4, hipMemcpyHostToDevice, m->stream));
+        }
+        L2_TRY(set_i32_launch(m->dtok, first, m->dpos, pos0, m->stream));
+        L2_TRY(set_i32_launch(m->dloop, n_prompt, m->dloop + 1, pos0, m->stream));
+        for (int pos = pos0; pos < pos0 + n; pos++) {
+            L2_TRY(check_position(m, pos));
+            hipGraphExec_t exec = nullptr;
+            L2_TRY(step_graph_get(m, s, step_bucket(m, pos), &exec));
+            s->rows = std::max(s->rows, pos + 1);
+            L2_HIP(hipGraphLaunch(exec, m->stream));
+        }
+        return L2_OK;
+    }
+    ForwardIn in;
+    in.src.token = first, in.logits = m->logits;
+    for (int i = 0; i < n; i++) {
+        const int pos = pos0 + i;
+        in.amax = m->amax + (i & 1);
+        L2_TRY(forward_enqueue(m, s, 1, pos, in));
+        in.src = TokenSource{};
+        if (pos < n_prompt)
+            in.src.token = prompt[pos];
+        else
+            in.src.prev = in.amax, in.src.record = m->hs.ids + i;
+    }
     return L2_OK;
 }
 
-static int loop_begin(l2_model *m, int n_prompt, int pos0) {
-    return set_i32_launch(m->dloop, n_prompt, m->dloop + 1, pos0, m->stream);
+// Waits for the steps above and hands out every one's next token.
+static int steps_collect(l2_model *m, int pos0, int n, const int32_t *prompt, int n_prompt, int32_t *ids) {
+    if (n == 0) return wait_host(m, nullptr, nullptr);
+    if (m->use_graph && !m->prof_on) {
+        L2_HIP(hipMemcpyAsync(m->hs.ids, m->dout_ids, (size_t)n * 4, hipMemcpyDeviceToHost, m->stream));
+        L2_TRY(wait_host(m, nullptr, nullptr));
+    } else {
+        const bool forced = pos0 + n - 1 < n_prompt;
+        L2_TRY(wait_host(m, forced ? nullptr : m->amax + ((n - 1) & 1), m->hs.ids + n - 1));
+        for (int i = 0; i < n && pos0 + i < n_prompt; i++) m->hs.ids[i] = prompt[pos0 + i];
+    }
+    if (ids) memcpy(ids, m->hs.ids, (size_t)n * 4);
+    return L2_OK;
 }
 
 // Position at which prefill<64>, <32>, ... <2> (src/inference.rs:78-127) leave off for a prompt of n_prompt
@@ -1850,7 +1950,7 @@ int l2_prefill_ladder(l2_model *m, l2_state *s, const int32_t *prompt, int n_pro
     std::vector<int32_t> toks((size_t)n);
     for (int i = 0; i < n; i++) toks[i] = i == 0 ? 1 : prompt[i - 1];
     const int passes = (n + kPassTokens - 1) / kPassTokens;
-    return l2_prefill_chunks(m, s, toks.data(), n, 0, (n + passes - 1) / passes);
+    return prefill_chunks(m, s, toks.data(), n, 0, (n + passes - 1) / passes, false);
 }
 
 extern "C" int l2_generate_greedy(l2_model *m, l2_state *s, const int32_t *prompt, int n_prompt, int steps,
@@ -1867,12 +1967,8 @@ extern "C" int l2_generate_greedy(l2_model *m, l2_state *s, const int32_t *promp
     for (int i = 0; i < n_prompt; i++)
         if (prompt[i] < 0 || prompt[i] >= m->d.vocab_size)
             return l2_fail(L2_ERR_RANGE, "prompt token %d outside 0..%d", prompt[i], m->d.vocab_size - 1);
-    L2_TRY(l2_state_reset(s)); // RunState::new per call (:59)
+    L2_TRY(state_clear(s)); // RunState::new per call (:59)
     L2_TRY(ensure_batch(m, 1));
-    L2_TRY(ensure_loop_buffers(m, std::max(n_prompt, 1), std::max(steps, 1)));
-    if (n_prompt > 0)
-        L2_HIP(hipMemcpyAsync(m->dprompt, prompt, (size_t)n_prompt * 4, hipMemcpyHostToDevice, m->stream));
-    L2_HIP(hipStreamSynchronize(m->stream));
     const auto t0 = std::chrono::steady_clock::now(); // :72
     int pos = 0;
     if (use_prefill) { // :78-127
@@ -1880,18 +1976,11 @@ extern "C" int l2_generate_greedy(l2_model *m, l2_state *s, const int32_t *promp
         L2_TRY(l2_prefill_ladder(m, s, prompt, n_prompt));
     }
     const int32_t first = pos == 0 ? 1 : prompt[pos - 1]; // :128-132
-    L2_TRY(set_i32_launch(m->dtok, first, m->dpos, pos, m->stream));
-    const int pos0 = pos;
-    L2_TRY(loop_begin(m, n_prompt, pos0));
-    int n = 0;
-    while (pos < steps) { // :141
-        L2_TRY(loop_step(m, s, pos, n_prompt, pos0));
-        n++;
-        pos++;
-    }
-    L2_HIP(hipStreamSynchronize(m->stream));
+    const int n = std::max(steps - pos, 0); // :141
+    if (n > 0 && pos + n > m->max_seq) return l2_fail(L2_ERR_RANGE, "position %d outside 0..%d", pos + n - 1, m->max_seq - 1);
+    L2_TRY(steps_enqueue(m, s, first, pos, n, prompt, n_prompt));
+    L2_TRY(steps_collect(m, pos, n, prompt, n_prompt, out_ids));
     const auto t1 = std::chrono::steady_clock::now(); // :192
-    if (n > 0) L2_HIP(hipMemcpy(out_ids, m->dout_ids, (size_t)n * 4, hipMemcpyDeviceToHost));
     *n_out = n;
     if (ms) *ms = std::chrono::duration<double, std::milli>(t1 - t0).count();
     return L2_OK;
@@ -1998,10 +2087,8 @@ extern "C" int l2_decode_bench(l2_model *m, l2_state *s, int32_t token, int32_t 
     if (pos < 0 || pos + n_tokens > m->max_seq) return l2_fail(L2_ERR_RANGE, "positions [%d,%d) exceed the cache", pos, pos + n_tokens);
     if (token < 0 || token >= m->d.vocab_size) return l2_fail(L2_ERR_RANGE, "token %d", token);
     L2_TRY(ensure_batch(m, 1));
-    L2_TRY(ensure_loop_buffers(m, 1, n_tokens));
-    L2_TRY(set_i32_launch(m->dtok, token, m->dpos, pos, m->stream));
-    L2_TRY(loop_begin(m, 0, pos));
     if (m->use_graph) { // capture (if need be) outside the timed region
+        L2_TRY(ensure_loop_buffers(m, 1, n_tokens));
         hipGraphExec_t exec = nullptr;
         for (int b = step_bucket(m, pos);; b = step_bucket(m, b)) {
             L2_TRY(step_graph_get(m, s, b, &exec));
@@ -2013,14 +2100,13 @@ extern "C" int l2_decode_bench(l2_model *m, l2_state *s, int32_t token, int32_t 
     L2_HIP(hipEventCreate(&e1));
     L2_HIP(hipStreamSynchronize(m->stream));
     L2_HIP(hipEventRecord(e0, m->stream));
-    for (int i = 0; i < n_tokens; i++) L2_TRY(loop_step(m, s, pos + i, 0, pos));
+    L2_TRY(steps_enqueue(m, s, token, pos, n_tokens, nullptr, 0));
     L2_HIP(hipEventRecord(e1, m->stream));
     L2_HIP(hipEventSynchronize(e1));
     L2_HIP(hipEventElapsedTime(ms_total, e0, e1));
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    if (out_ids) L2_HIP(hipMemcpy(out_ids, m->dout_ids, (size_t)n_tokens * 4, hipMemcpyDeviceToHost));
-    return L2_OK;
+    return steps_collect(m, pos, n_tokens, nullptr, 0, out_ids);
 }
 
 // Which kernel each q4 launch class of this model's decode step runs: "class=kernel;..." with the kernel's
@@ -2122,14 +2208,10 @@ extern "C" int l2_decode_profile(l2_model *m, l2_state *s, int32_t token, int32_
     if (pos < 0 || pos + n_tokens > m->max_seq) return l2_fail(L2_ERR_RANGE, "positions [%d,%d) exceed the cache", pos, pos + n_tokens);
     if (token < 0 || token >= m->d.vocab_size) return l2_fail(L2_ERR_RANGE, "token %d", token);
     L2_TRY(ensure_batch(m, 1));
-    L2_TRY(ensure_loop_buffers(m, 1, n_tokens));
-    L2_TRY(set_i32_launch(m->dtok, token, m->dpos, pos, m->stream));
-    L2_TRY(loop_begin(m, 0, pos));
     L2_HIP(hipStreamSynchronize(m->stream));
     m->prof.clear();
     m->prof_on = true;
-    int rc = L2_OK;
-    for (int i = 0; i < n_tokens && rc == L2_OK; i++) rc = loop_step(m, s, pos + i, 0, pos);
+    int rc = steps_enqueue(m, s, token, pos, n_tokens, nullptr, 0);
     m->prof_on = false;
     hipError_t e = hipStreamSynchronize(m->stream);
     for (int c = 0; c < K_NCLASS; c++) {

@@ -10,6 +10,8 @@
 // element i of its result to slot inv[i] of the buffer the next QLinear reads,
 // which is that layer's x[g_index[j]] gather (src/gptq.rs:110-114) done once
 // at the source instead of once per consumer block.
+#include <chrono>
+
 #include "l2_internal.h"
 
 namespace {
@@ -66,11 +68,18 @@ __device__ __forceinline__ float block_max(float v, float *red) {
 // x[b] = token_embedding_table[token[b]]  (src/models.rs:189-191), also written
 // in the input order of the first layer's q, k and v projections.  Starts a
 // forward pass, so it also clears the running argmax.
-__global__ void embed_kernel(float *x, const float *emb, const int32_t *tokens, int dim, ScatterTargets t,
+__global__ void embed_kernel(float *x, const float *emb, const TokenSource src_, int dim, ScatterTargets t,
                              unsigned long long *amax) {
     const int b = blockIdx.y;
-    const float *src = emb + (size_t)tokens[b] * dim;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    int32_t token = src_.token;
+    if (src_.tokens)
+        token = src_.tokens[b];
+    else if (src_.prev) { // src/inference.rs:160-162, 185-189: the argmax of the step before is this step's token
+        token = (int32_t)(src_.prev[0] & 0xFFFFFFFFull);
+        if (i == 0) src_.record[0] = token;
+    }
+    const float *src = emb + (size_t)token * dim;
     if (i < dim) {
         const float v = src[i];
         x[(size_t)b * dim + i] = v;
@@ -276,6 +285,20 @@ __global__ void next_token_kernel(const unsigned long long *amax, const int32_t 
     }
 }
 
+__global__ void finish_kernel(const unsigned long long *amax, int32_t *id, uint32_t *flag, uint32_t seq) {
+    if (threadIdx.x == 0) {
+        if (amax) id[0] = (int32_t)(amax[0] & 0xFFFFFFFFull);
+        __threadfence_system(); // what the call left in host memory is there before the number is
+        *reinterpret_cast<volatile uint32_t *>(flag) = seq;
+    }
+}
+
+__global__ void clear_rows_kernel(float4 *k, float4 *v, size_t stride4, size_t n4) {
+    float4 *p = (blockIdx.z ? v : k) + blockIdx.y * stride4;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (size_t)gridDim.x * blockDim.x)
+        p[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+}
+
 __global__ void set_i32_kernel(int32_t *p, int32_t a, int32_t *q, int32_t b) {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
         p[0] = a;
@@ -295,10 +318,39 @@ __global__ void fill_pattern_kernel(float *p, size_t n, uint64_t seed) {
 
 } // namespace
 
-int embed_launch(float *x, const float *emb, const int32_t *tokens, int dim, int B, const ScatterTargets &t,
+int embed_launch(float *x, const float *emb, const TokenSource &src, int dim, int B, const ScatterTargets &t,
                  unsigned long long *amax_key, hipStream_t st) {
     if (t.n < 0 || t.n > 3) return l2_fail(L2_ERR_ARG, "embed: %d targets", t.n);
-    hipLaunchKernelGGL(embed_kernel, dim3((dim + 255) / 256, B), dim3(256), 0, st, x, emb, tokens, dim, t, amax_key);
+    hipLaunchKernelGGL(embed_kernel, dim3((dim + 255) / 256, B), dim3(256), 0, st, x, emb, src, dim, t, amax_key);
+    L2_HIP(hipGetLastError());
+    return L2_OK;
+}
+
+int finish_launch(const unsigned long long *amax, int32_t *id, uint32_t *flag, uint32_t seq, hipStream_t st) {
+    hipLaunchKernelGGL(finish_kernel, dim3(1), dim3(64), 0, st, amax, id, flag, seq);
+    L2_HIP(hipGetLastError());
+    return L2_OK;
+}
+
+bool watch_flag(volatile uint32_t *flag, uint32_t seq) {
+    const auto give_up = std::chrono::steady_clock::now() + std::chrono::seconds(2);
+    for (;;) {
+        for (int i = 0; i < 1024; i++) {
+            if (*flag == seq) {
+                std::atomic_thread_fence(std::memory_order_acquire);
+                return true;
+            }
+            __builtin_ia32_pause();
+        }
+        if (std::chrono::steady_clock::now() > give_up) return false;
+    }
+}
+
+int clear_rows_launch(float *k, float *v, int layers, size_t stride, size_t n, hipStream_t st) {
+    if (n == 0) return L2_OK;
+    const size_t n4 = n / 4, per = (n4 + 255) / 256, most = (size_t)(8 * cu_count() / layers + 1);
+    hipLaunchKernelGGL(clear_rows_kernel, dim3((unsigned)(per < most ? per : most), layers, 2), dim3(256), 0, st,
+                       reinterpret_cast<float4 *>(k), reinterpret_cast<float4 *>(v), stride / 4, n4);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }

@@ -72,7 +72,7 @@ struct LdsLimit {
 
 // Position at which the prefill ladder 64/32/16/8/4/2 (src/inference.rs:78-127) leaves off.
 int l2_prefill_ladder_end(int n_prompt);
-// What the ladder computes: the cache rows of the positions before that.
+// What the ladder computes: the cache rows of the positions before that (enqueued, not waited for).
 int l2_prefill_ladder(l2_model *m, l2_state *s, const int32_t *prompt, int n_prompt);
 
 // ---- device views ---------------------------------------------------------
@@ -258,9 +258,23 @@ struct ScatterTargets {
     int n;
 };
 
-// x[b] = emb[tokens[b]], also delivered through t; clears the running argmax.
-int embed_launch(float *x, const float *emb, const int32_t *tokens, int dim, int B, const ScatterTargets &t,
+// Where the tokens of a forward pass come from: an array in device memory; one token given here; or, for a step of the
+// greedy loop, the running maximum of the step before, which is recorded as that step's result.
+struct TokenSource {
+    const int32_t *tokens = nullptr;
+    const unsigned long long *prev = nullptr;
+    int32_t *record = nullptr;
+    int32_t token = 0;
+};
+// x[b] = emb[token b], also delivered through t; clears the running argmax.
+int embed_launch(float *x, const float *emb, const TokenSource &src, int dim, int B, const ScatterTargets &t,
                  unsigned long long *amax_key, hipStream_t st);
+// The end of a call's work: with amax, *id = its index; then *flag = seq (both in pinned host memory).
+int finish_launch(const unsigned long long *amax, int32_t *id, uint32_t *flag, uint32_t seq, hipStream_t st);
+// The host's side: true once *flag is seq; false if that takes so long that something may be wrong.
+bool watch_flag(volatile uint32_t *flag, uint32_t seq);
+// k and v: the first n floats (a multiple of 4) of each of `layers` stretches of `stride` floats become zero.
+int clear_rows_launch(float *k, float *v, int layers, size_t stride, size_t n, hipStream_t st);
 int gather_launch(float *out, const float *x, const int32_t *g_index, int n, int B, hipStream_t st);
 int rope_kv_launch(float *q, const float *k, const float *v, const int32_t *pos, const float *cos_t,
                    const float *sin_t, float *kcache_l, float *vcache_l, int n_heads, int n_kv_heads,
