@@ -461,6 +461,57 @@ static void dfree(void *p) {
     if (p) (void)hipFree(p);
 }
 
+// Pinned host memory for the operator's calls on host arrays, shared by all handles: a call takes a slot for its time, so
+// calls of several threads run side by side.  At most kKept idle slots are kept, and none once the last handle is gone.
+struct HostSlot {
+    static constexpr size_t kBytes = (size_t)1 << 20; // each of x and y
+    char *base = nullptr;
+    volatile uint32_t *flag = nullptr;
+    uint32_t seq = 0;
+    float *x = nullptr, *y = nullptr;
+};
+static struct HostSlots {
+    static constexpr size_t kKept = 4;
+    std::mutex mu;
+    std::vector<HostSlot> idle;
+    int users = 0;
+
+    void add_user() {
+        std::lock_guard<std::mutex> lock(mu);
+        users++;
+    }
+    void drop_user() {
+        std::lock_guard<std::mutex> lock(mu);
+        if (--users > 0) return;
+        for (HostSlot &s : idle) (void)hipHostFree(s.base);
+        idle.clear();
+    }
+    int take(HostSlot *out) {
+        {
+            std::lock_guard<std::mutex> lock(mu);
+            if (!idle.empty()) {
+                *out = idle.back();
+                idle.pop_back();
+                return L2_OK;
+            }
+        }
+        void *p = nullptr;
+        L2_HIP(hipHostMalloc(&p, 2 * HostSlot::kBytes + 256, hipHostMallocCoherent | hipHostMallocPortable));
+        out->base = (char *)p;
+        out->x = (float *)p, out->y = (float *)(out->base + HostSlot::kBytes);
+        out->flag = (volatile uint32_t *)(out->base + 2 * HostSlot::kBytes);
+        *out->flag = 0;
+        return L2_OK;
+    }
+    void give(const HostSlot &s) {
+        std::lock_guard<std::mutex> lock(mu);
+        if (idle.size() < kKept && users > 0)
+            idle.push_back(s);
+        else
+            (void)hipHostFree(s.base);
+    }
+} host_slots;
+
 static void invert_perm(const int32_t *g, int n, int32_t *inv, bool *ok) {
     std::fill(inv, inv + n, -1);
     for (int j = 0; j < n; j++) {
@@ -491,6 +542,7 @@ static int model_build(const char *weights, size_t nbytes, const l2_dims *dims, 
     L2_TRY(require_device());
 
     l2_model *m = new l2_model();
+    host_slots.add_user();
     m->use_graph = getenv("L2_STEP_GRAPH") != nullptr; // also l2_model_set_step_graph
     if (const char *v = getenv("L2_PREFILL_LANES")) { // chunks of a prompt in flight at once (l2_prefill_chunks)
         const int n = atoi(v);
@@ -730,6 +782,7 @@ extern "C" void l2_model_close(l2_model *m) {
         if (es) (void)hipStreamDestroy(es);
     if (m->stream) (void)hipStreamDestroy(m->stream);
     delete m;
+    host_slots.drop_user();
 }
 
 extern "C" int l2_model_config(const l2_model *m, l2_config *out) {
@@ -1069,6 +1122,7 @@ extern "C" int l2_qlinear_create(const int32_t *qweight, const int32_t *qzeros, 
     invert_perm(g_index, in, inv.data(), &ok);
     if (!ok) return l2_fail(L2_ERR_FORMAT, "g_index is not a permutation of 0..%d", in - 1);
     l2_qlinear *q = new l2_qlinear();
+    host_slots.add_user();
     const size_t sizes[5] = {(size_t)out * (in / 8) * 4, (size_t)(out / 8) * groups * 4, (size_t)out * groups * 4,
                              (size_t)in * 4, (size_t)in * 4};
     const void *src[5] = {qweight, qzeros, scales, g_index, inv.data()};
@@ -1113,6 +1167,7 @@ extern "C" void l2_qlinear_free(l2_qlinear *q) {
     dfree(q->batch.ws);
     if (q->stream) (void)hipStreamDestroy(q->stream);
     delete q;
+    host_slots.drop_user();
 }
 
 static int qlinear_scratch(l2_qlinear *q, int B) {
@@ -1129,18 +1184,47 @@ static int qlinear_scratch(l2_qlinear *q, int B) {
     return L2_OK;
 }
 
-// x (host, natural order) -> gather through g_index -> matvec -> y (host)
+static constexpr size_t kCopyKernelBytes = 64 * 1024; // up to here a copy kernel is quicker than the copy engine
+
+static int operator_enqueue(const DevQLinear &q, const float *dx, float *dxg, float *y, const OperatorBufs &bufs, int planes,
+                            int B, hipStream_t st) {
+    if (!planes) return q4_one_natural(q, dx, dxg, y, B, st);
+    return gemm_operator(q, dx, B, y, planes, bufs.planes, bufs.ws, bufs.ws_floats, st);
+}
+
+// x (host, natural order) -> gather through g_index -> matvec -> y (host).  Through a slot of pinned memory where x and y
+// fit one: x is fetched from there, the last kernel writes y there, and the host watches for the end of the call.  One
+// 4096x4096 matvec 31.6 -> 17 us (pageable copies either way and hipStreamSynchronize before).
 static int matvec_host(const DevQLinear &q, float *dx, float *dxg, float *dy, OperatorBufs &bufs, int planes,
                        const float *x_host, int B, float *y_host, hipStream_t st) {
     if (planes) L2_TRY(operator_bufs(bufs, q, B, planes, st));
-    L2_HIP(hipMemcpyAsync(dx, x_host, (size_t)B * q.in * 4, hipMemcpyHostToDevice, st));
-    if (planes)
-        L2_TRY(gemm_operator(q, dx, B, dy, planes, bufs.planes, bufs.ws, bufs.ws_floats, st));
-    else
-        L2_TRY(q4_one_natural(q, dx, dxg, dy, B, st));
-    L2_HIP(hipMemcpyAsync(y_host, dy, (size_t)B * q.out * 4, hipMemcpyDeviceToHost, st));
-    L2_HIP(hipStreamSynchronize(st));
-    return L2_OK;
+    const size_t xb = (size_t)B * q.in * 4, yb = (size_t)B * q.out * 4;
+    if (xb > HostSlot::kBytes || yb > HostSlot::kBytes) {
+        L2_HIP(hipMemcpyAsync(dx, x_host, xb, hipMemcpyHostToDevice, st));
+        L2_TRY(operator_enqueue(q, dx, dxg, dy, bufs, planes, B, st));
+        L2_HIP(hipMemcpyAsync(y_host, dy, yb, hipMemcpyDeviceToHost, st));
+        L2_HIP(hipStreamSynchronize(st));
+        return L2_OK;
+    }
+    HostSlot slot;
+    L2_TRY(host_slots.take(&slot));
+    auto call = [&]() -> int {
+        memcpy(slot.x, x_host, xb);
+        if (xb <= kCopyKernelBytes)
+            L2_TRY(copy_launch(dx, slot.x, xb / 4, st));
+        else
+            L2_HIP(hipMemcpyAsync(dx, slot.x, xb, hipMemcpyHostToDevice, st));
+        L2_TRY(operator_enqueue(q, dx, dxg, slot.y, bufs, planes, B, st));
+        return finish_launch(nullptr, nullptr, const_cast<uint32_t *>(slot.flag), ++slot.seq, st);
+    };
+    int rc = call();
+    if (rc != L2_OK || !watch_flag(slot.flag, slot.seq)) {
+        const hipError_t e = hipStreamSynchronize(st);
+        if (rc == L2_OK && e != hipSuccess) rc = l2_fail(L2_ERR_HIP, "matvec: %s", hipGetErrorString(e));
+    }
+    if (rc == L2_OK) memcpy(y_host, slot.y, yb);
+    host_slots.give(slot);
+    return rc;
 }
 
 extern "C" int l2_qlinear_matvec(l2_qlinear *q, const float *x_host, int B, float *y_host) {

@@ -293,6 +293,11 @@ __global__ void finish_kernel(const unsigned long long *amax, int32_t *id, uint3
     }
 }
 
+__global__ void copy_kernel(float4 *dst, const float4 *src, int n4) {
+    const int i = blockIdx.x * 64 + threadIdx.x;
+    if (i < n4) dst[i] = src[i];
+}
+
 __global__ void clear_rows_kernel(float4 *k, float4 *v, size_t stride4, size_t n4) {
     float4 *p = (blockIdx.z ? v : k) + blockIdx.y * stride4;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (size_t)gridDim.x * blockDim.x)
@@ -344,6 +349,13 @@ bool watch_flag(volatile uint32_t *flag, uint32_t seq) {
         }
         if (std::chrono::steady_clock::now() > give_up) return false;
     }
+}
+
+int copy_launch(float *dst, const float *src, size_t n, hipStream_t st) {
+    const int n4 = (int)(n / 4); // inputs are multiples of 32 floats
+    hipLaunchKernelGGL(copy_kernel, dim3((n4 + 63) / 64), dim3(64), 0, st, reinterpret_cast<float4 *>(dst), reinterpret_cast<const float4 *>(src), n4);
+    L2_HIP(hipGetLastError());
+    return L2_OK;
 }
 
 int clear_rows_launch(float *k, float *v, int layers, size_t stride, size_t n, hipStream_t st) {

@@ -273,6 +273,8 @@ int embed_launch(float *x, const float *emb, const TokenSource &src, int dim, in
 int finish_launch(const unsigned long long *amax, int32_t *id, uint32_t *flag, uint32_t seq, hipStream_t st);
 // The host's side: true once *flag is seq; false if that takes so long that something may be wrong.
 bool watch_flag(volatile uint32_t *flag, uint32_t seq);
+// dst = src, n floats; for small pieces of pinned host memory.
+int copy_launch(float *dst, const float *src, size_t n, hipStream_t st);
 // k and v: the first n floats (a multiple of 4) of each of `layers` stretches of `stride` floats become zero.
 int clear_rows_launch(float *k, float *v, int layers, size_t stride, size_t n, hipStream_t st);
 int gather_launch(float *out, const float *x, const int32_t *g_index, int n, int B, hipStream_t st);
