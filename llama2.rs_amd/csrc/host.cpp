@@ -317,7 +317,8 @@ struct l2_model {
         char *base = nullptr;
         volatile uint32_t *flag = nullptr;
         uint32_t seq = 0;
-        float *logits = nullptr;
+        float *logits = nullptr;               // [vocab]: logits, or the sampler's weights
+        unsigned long long *redo = nullptr;    // one bit per vocabulary entry
         int32_t *ids = nullptr, *in = nullptr; // [max_seq] out; [2 * max(max_seq, 4096)] in
     } hs;
     static constexpr int kMaxLanes = 4; // the process has four hardware queues
@@ -693,7 +694,8 @@ static int model_build(const char *weights, size_t nbytes, const l2_dims *dims, 
     }
     M_TRY(dalloc(&m->amax, 2));
     {
-        const size_t logits = 256, ids = logits + ((size_t)dims->vocab_size * 4 + 255) / 256 * 256,
+        const size_t logits = 256, redo = logits + ((size_t)dims->vocab_size * 4 + 255) / 256 * 256,
+                     ids = redo + ((size_t)dims->vocab_size / 64 + 32) / 32 * 256,
                      in = ids + ((size_t)max_seq * 4 + 255) / 256 * 256, end = in + (size_t)std::max(max_seq, 4096) * 8;
         void *p = nullptr;
         M_HIP(hipHostMalloc(&p, end, hipHostMallocCoherent));
@@ -701,6 +703,7 @@ static int model_build(const char *weights, size_t nbytes, const l2_dims *dims, 
         m->hs.flag = (volatile uint32_t *)m->hs.base;
         *m->hs.flag = 0;
         m->hs.logits = (float *)(m->hs.base + logits);
+        m->hs.redo = (unsigned long long *)(m->hs.base + redo);
         m->hs.ids = (int32_t *)(m->hs.base + ids);
         m->hs.in = (int32_t *)(m->hs.base + in);
     }
@@ -1757,6 +1760,20 @@ extern "C" int l2_forward(l2_model *m, l2_state *s, const int32_t *tokens, const
     L2_TRY(forward_enqueue(m, s, 1, max_pos, in));
     L2_TRY(wait_host(m, nullptr, nullptr));
     if (logits_host) memcpy(logits_host, m->hs.logits, (size_t)m->d.vocab_size * 4);
+    return L2_OK;
+}
+
+int l2_forward_weights(l2_model *m, l2_state *s, int32_t token, int32_t pos, float temperature, SampleWeights *out) {
+    if (s->m != m) return l2_fail(L2_ERR_ARG, "state belongs to another model");
+    int max_pos = 0;
+    L2_TRY(check_tokens(m, &token, &pos, 1, &max_pos));
+    L2_TRY(ensure_batch(m, 1));
+    ForwardIn in;
+    in.src.token = token, in.logits = m->logits, in.amax = m->amax;
+    L2_TRY(forward_enqueue(m, s, 1, pos, in));
+    L2_TRY(sample_weights_launch(m->hs.logits, m->hs.redo, m->logits, m->d.vocab_size, temperature, m->amax, m->stream));
+    L2_TRY(wait_host(m, nullptr, nullptr));
+    *out = {m->hs.logits, m->hs.redo};
     return L2_OK;
 }
 

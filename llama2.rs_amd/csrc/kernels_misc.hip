@@ -285,6 +285,27 @@ __global__ void next_token_kernel(const unsigned long long *amax, const int32_t 
     }
 }
 
+__global__ __launch_bounds__(256) void sample_weights_kernel(float *w, unsigned long long *redo, const float *logits, int n,
+                                                            float temperature, const unsigned long long *amax) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    const uint32_t key = (uint32_t)(amax[0] >> 32); // amax_key's ordered float
+    const float top = __builtin_bit_cast(float, (key & 0x80000000u) ? key & 0x7FFFFFFFu : ~key);
+    bool again = false;
+    if (i < n) {
+        // src/inference.rs:166-168, src/models.rs:68-76; the maximum of the quotients is the quotient of the maximum
+        const float d = logits[i] / temperature - top / temperature;
+        const double e = exp((double)d);
+        const float f = (float)e;
+        // within 0.02 units in the last place of a boundary (an expf good to 0.502 may go either way within 0.002), or a
+        // subnormal result
+        const double ulp = (double)__builtin_bit_cast(float, (__builtin_bit_cast(uint32_t, f) & 0x7F800000u)) * 0x1p-23;
+        again = !(fabs(e - (double)f) <= 0.48 * ulp) && !(d < -110.0f);
+        w[i] = again ? d : f;
+    }
+    const unsigned long long mask = __ballot(again);
+    if ((threadIdx.x & 63) == 0 && i < n) redo[i >> 6] = mask;
+}
+
 __global__ void finish_kernel(const unsigned long long *amax, int32_t *id, uint32_t *flag, uint32_t seq) {
     if (threadIdx.x == 0) {
         if (amax) id[0] = (int32_t)(amax[0] & 0xFFFFFFFFull);
@@ -327,6 +348,13 @@ int embed_launch(float *x, const float *emb, const TokenSource &src, int dim, in
                  unsigned long long *amax_key, hipStream_t st) {
     if (t.n < 0 || t.n > 3) return l2_fail(L2_ERR_ARG, "embed: %d targets", t.n);
     hipLaunchKernelGGL(embed_kernel, dim3((dim + 255) / 256, B), dim3(256), 0, st, x, emb, src, dim, t, amax_key);
+    L2_HIP(hipGetLastError());
+    return L2_OK;
+}
+
+int sample_weights_launch(float *w, unsigned long long *redo, const float *logits, int n, float temperature,
+                          const unsigned long long *amax, hipStream_t st) {
+    hipLaunchKernelGGL(sample_weights_kernel, dim3((n + 255) / 256), dim3(256), 0, st, w, redo, logits, n, temperature, amax);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }

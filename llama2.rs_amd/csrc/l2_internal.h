@@ -75,6 +75,14 @@ int l2_prefill_ladder_end(int n_prompt);
 // What the ladder computes: the cache rows of the positions before that (enqueued, not waited for).
 int l2_prefill_ladder(l2_model *m, l2_state *s, const int32_t *prompt, int n_prompt);
 
+// One forward step for the sampler: the weights above of the logits at `pos`, in host memory that belongs to the model
+// and stands until its next call.
+struct SampleWeights {
+    float *w;
+    const unsigned long long *redo;
+};
+int l2_forward_weights(l2_model *m, l2_state *s, int32_t token, int32_t pos, float temperature, SampleWeights *out);
+
 // ---- device views ---------------------------------------------------------
 
 // One QLinear resident in device memory, `.bin` layout (src/gptq.rs:68-84),
@@ -269,6 +277,11 @@ struct TokenSource {
 // x[b] = emb[token b], also delivered through t; clears the running argmax.
 int embed_launch(float *x, const float *emb, const TokenSource &src, int dim, int B, const ScatterTargets &t,
                  unsigned long long *amax_key, hipStream_t st);
+// For sampling at `temperature` > 0 behind a classifier whose running maximum is amax: with d_i = logits[i] / temperature -
+// max_j(logits[j] / temperature), w[i] = expf(d_i), correctly rounded; where that lies so close to the boundary between
+// two floats that another faithful expf may round it the other way, w[i] = d_i and bit i of `redo` is set.
+int sample_weights_launch(float *w, unsigned long long *redo, const float *logits, int n, float temperature,
+                          const unsigned long long *amax, hipStream_t st);
 // The end of a call's work: with amax, *id = its index; then *flag = seq (both in pinned host memory).
 int finish_launch(const unsigned long long *amax, int32_t *id, uint32_t *flag, uint32_t seq, hipStream_t st);
 // The host's side: true once *flag is seq; false if that takes so long that something may be wrong.

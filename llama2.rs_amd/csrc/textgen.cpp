@@ -8,6 +8,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
 #include <chrono>
 #include <string>
 #include <unordered_map>
@@ -185,6 +186,82 @@ static void softmax_host(float *x, int n) {
     for (int i = 0; i < n; i++) x[i] /= sum;
 }
 
+// Both sums of the sampler, softmax's denominator (src/models.rs:75-78) and the CDF (src/util.rs:105-111), run over the
+// vocabulary one fp32 addition at a time, and their roundings decide the token: they have to be these roundings.  While
+// the sum c stays within one binade [2^k, 2^(k+1)), though, c is a multiple of u = 2^(k-23), and c + p rounds to
+// c + (p rounded to a multiple of u) unless p lies exactly between two: 64 terms can be rounded side by side and added in
+// any order.  A block that leaves the binade, has a term between two multiples, or (found) passes `x` goes one by one.
+// `term(i)` gives four terms from i on.  Returns n, or the first index at which the sum exceeds x.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+
+template <class Term>
+static int chain_add(const Term &term, int n, float x, float *sum) {
+    float c = 0.0f;
+    constexpr int kBlock = 64;
+    for (int i0 = 0; i0 < n; i0 += kBlock) {
+        if (i0 + kBlock <= n && c > 1e-30f && c < 1e30f) {
+            uint32_t bits;
+            memcpy(&bits, &c, 4);
+            bits &= 0x7F800000u;
+            float lo;
+            memcpy(&lo, &bits, 4); // 2^k
+            const f32x4 base = f32x4{lo, lo, lo, lo};
+            const float half_u = lo * 0x1p-24f;
+            f32x4 acc[4] = {};
+            i32x4 tie = i32x4{0, 0, 0, 0};
+#pragma clang loop unroll(full)
+            for (int i = 0; i < kBlock; i += 4) {
+                const f32x4 p = term(i0 + i);
+                const f32x4 t = (p + base) - base, d = p - t;
+                tie |= (d == f32x4{half_u, half_u, half_u, half_u}) | (d == f32x4{-half_u, -half_u, -half_u, -half_u});
+                acc[i / 4 & 3] += t;
+            }
+            const f32x4 a = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+            const float next = c + ((a[0] + a[1]) + (a[2] + a[3]));
+            if (next < 2.0f * lo && next <= x && !(tie[0] | tie[1] | tie[2] | tie[3])) {
+                c = next;
+                continue;
+            }
+        }
+        for (int i = i0; i < std::min(i0 + kBlock, n); i += 4) {
+            const f32x4 p = term(i);
+            for (int e = 0; e < 4 && i + e < n; e++) {
+                c += p[e];
+                if (x < c) {
+                    *sum = c;
+                    return i + e;
+                }
+            }
+        }
+    }
+    *sum = c;
+    return n;
+}
+
+// Random::sample on softmax(logits / temperature) (src/inference.rs:166-172), from the weights of l2_forward_weights.
+static int sample_weights(const SampleWeights &s, int n, l2_random *rng) {
+    float *w = s.w;
+    for (int g = 0; g < (n + 63) / 64; g++)
+        for (unsigned long long m = s.redo[g]; m; m &= m - 1) {
+            const int i = 64 * g + __builtin_ctzll(m);
+            w[i] = expf(w[i]);
+        }
+    const int n4 = n & ~3;
+    f32x4 tail = f32x4{0.f, 0.f, 0.f, 0.f}; // the last, incomplete four
+    for (int i = n4; i < n; i++) tail[i & 3] = w[i];
+    auto weight = [&](int i) {
+        f32x4 v = tail;
+        if (i < n4) memcpy(&v, w + i, 16);
+        return v;
+    };
+    float sum = 0.0f, cdf = 0.0f;
+    chain_add(weight, n, __builtin_inff(), &sum);
+    const float x = l2_random_f32(rng);
+    const int i = chain_add([&](int j) { return weight(j) / f32x4{sum, sum, sum, sum}; }, n, x, &cdf);
+    return std::min(i, n - 1);
+}
+
 // get_token (src/util.rs:116-123): after BOS, a leading space is stripped
 static const char *token_text(const l2_tokenizer *t, int token, int next, int *len) {
     const std::string &s = t->vocab[next];
@@ -289,7 +366,7 @@ extern "C" int l2_generate(l2_model *m, l2_state *s, const l2_tokenizer *t, cons
         }
         int32_t token = pos == 0 ? 1 : prompt32[pos - 1];
         L2_TRY(emit(token, token, false)); // :134-137
-        std::vector<float> logits(temperature != 0.0f ? (size_t)d.vocab_size : 0);
+        std::vector<float> logits(temperature != 0.0f && !(temperature > 0.0f) ? (size_t)d.vocab_size : 0);
         while (pos < steps) {
             const int32_t p32 = pos;
             int32_t next = 0;
@@ -297,10 +374,15 @@ extern "C" int l2_generate(l2_model *m, l2_state *s, const l2_tokenizer *t, cons
                 L2_TRY(l2_decode_greedy(m, s, token, p32, &next)); // :160-162, argmax on the device
                 if (pos < n_prompt) next = prompt32[pos];
             } else {
-                L2_TRY(l2_forward(m, s, &token, &p32, 1, logits.data()));
                 if (pos < n_prompt) {
+                    L2_TRY(l2_forward(m, s, &token, &p32, 1, nullptr));
                     next = prompt32[pos];
-                } else {
+                } else if (temperature > 0.0f) {
+                    SampleWeights w{};
+                    L2_TRY(l2_forward_weights(m, s, token, p32, temperature, &w));
+                    next = sample_weights(w, d.vocab_size, rng);
+                } else { // a negative temperature (or none) turns the distribution round: everything here
+                    L2_TRY(l2_forward(m, s, &token, &p32, 1, logits.data()));
                     for (int q = 0; q < d.vocab_size; q++) logits[q] /= temperature; // :166-168
                     softmax_host(logits.data(), d.vocab_size);
                     next = l2_random_sample(rng, logits.data(), d.vocab_size);
