@@ -64,3 +64,21 @@ def test_fp32_prompt_vs_oracle(ops, oracle, kv, hidden, G, n):
         assert nrel(m.qmatvec(1, _lib.W1, x), x.astype(np.float64) @ tol._split_image(img, dims)["w1"][1].T.astype(np.float64)) < 1e-5
     m.close()
     o.close()
+
+
+# fp16 prompts: the last tile of tokens in each of its widths, behind tiles of 128 tokens and of 64
+@pytest.mark.parametrize("G,batches", [(32, (65, 100)), (64, (65, 257, 300, 340, 370)), (128, (65, 272, 300, 340, 370))])
+def test_fp16_operator_last_tile(ops, G, batches):
+    from llama2_rs import _lib
+    dims = ck.Dims(dim=1024, hidden_dim=2816, n_layers=1, n_heads=8, n_kv_heads=2, vocab_size=300, seq_len=512, group_size=G)
+    m = ops.Model(ck.synth_weights_image(dims, seed=5), dims)
+    for B in batches:
+        x = np.random.default_rng(B).standard_normal((B, 1024)).astype(np.float32)
+        m.set_prefill_mode(_lib.PREFILL_FP32)
+        want = m.qmatvec(0, _lib.W1, x)
+        m.set_prefill_mode(_lib.PREFILL_MFMA)
+        got = m.qmatvec(0, _lib.W1, x)
+        assert not np.array_equal(got, want)
+        for b in range(B):
+            assert nrel(got[b], want[b]) < 2e-3, (B, b)
+    m.close()
