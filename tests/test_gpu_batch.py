@@ -82,3 +82,21 @@ def test_fp16_operator_last_tile(ops, G, batches):
         for b in range(B):
             assert nrel(got[b], want[b]) < 2e-3, (B, b)
     m.close()
+
+
+# prompt attention with two sets of columns per block (two blocks per compute unit and more), the last block with one
+# set, against passes too short for that form
+@pytest.mark.parametrize("n_heads,n_kv,n", [(32, 32, 505), (16, 2, 1021)])
+def test_prompt_attention_two_sets(ops, n_heads, n_kv, n):
+    dims = ck.Dims(dim=128 * n_heads, hidden_dim=256, n_layers=2, n_heads=n_heads, n_kv_heads=n_kv, vocab_size=64,
+                   seq_len=1056, group_size=64)
+    m = ops.Model(ck.synth_weights_image(dims, seed=9), dims)
+    toks = np.random.default_rng(n).integers(0, 64, size=n).astype(np.int32)
+    m.prefill_chunks(toks, 0, n)
+    k, v = m.read_kv(1, 0, n)
+    m.reset()
+    for p in range(0, n, 101):
+        m.prefill_chunks(toks[p:p + 101], p, 101)
+    k2, v2 = m.read_kv(1, 0, n)
+    assert nrel(k, k2) < 1e-5 and nrel(v, v2) < 1e-5
+    m.close()
