@@ -835,16 +835,30 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(float *__restrict__ o
 // tokens 8.6, 7.9.  (v_mfma_f32_16x16x4_f32 at its peak: 63 us for the first of these.)  (A form on 32 columns and tiles of 32 rows,
 // v_mfma_f32_32x32x2_f32 with K and V turned through LDS, had half the blocks and took 16 to 31 us per chunk of a
 // 512-token prompt where this one takes 11 to 19.)
+
+// Column tile of block row y of n.  The work of a tile grows with its position, and blocks are dealt over the compute
+// units in turn, `unit_rows` rows until every unit has one.  With up to two blocks per unit all are resident at once and
+// the launch is as long as the unit with the most work, so the longest tiles get a unit to themselves and the others go
+// in pairs of a long and a short one: 32 heads, 511 tokens 41.5 -> 37.1 us (against longest first, which pairs the longest
+// with the middle).  Larger grids (unit_rows = 0) are worked off as units become free, longest first; dealing three per
+// unit the same way gained nothing (299 tokens 27.0, 27.9).
+__device__ __forceinline__ int column_tile(int y, int n, int unit_rows) {
+    if (unit_rows == 0) return n - 1 - y;
+    const int second = n - unit_rows; // rows of second blocks
+    if (y >= unit_rows) return y - unit_rows;
+    return n - 1 - (y < second ? unit_rows - second + y : y - second);
+}
+
 template <int QG, int NWV, int NP, int CS>
 __global__ __launch_bounds__(NWV * 64, NWV == 4 ? 2 : 1)
 void attn_prefill_mfma16_kernel(void *__restrict__ out, const float *__restrict__ q, const float *__restrict__ kc,
                                 const float *__restrict__ vc, const int32_t *__restrict__ pos,
-                                const int32_t *__restrict__ scatter, int n_heads, int n_kv_heads, int B, int max_pos) {
+                                const int32_t *__restrict__ scatter, int n_heads, int n_kv_heads, int B, int max_pos,
+                                int unit_rows) {
     constexpr int NT = NWV * 64, TK = 16, HS = 128, HALF = 64, NC = 16, QPT = NC / QG;
     __shared__ __align__(16) float comb[NWV][NC][kCombRow];
     __shared__ float4 qs[CS > 1 ? CS : 1][CS > 1 ? 8 : 1][64]; // several sets: their B operands
-    // the last columns of a chunk see the most cache rows: their blocks are dispatched first
-    const int kvh = blockIdx.x, ct = (gridDim.y - 1 - blockIdx.y) * CS;
+    const int kvh = blockIdx.x, ct = column_tile(blockIdx.y, gridDim.y, unit_rows) * CS;
     const int dim = n_heads * HS, kv_dim = n_kv_heads * HS;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, kb = lane >> 4;
@@ -1135,11 +1149,13 @@ static int prefill_qg(void *out, int planes, const float *q, const float *kc, co
     const int sets = (B * QG + 15) / 16;
     const bool two = (long)n_kv_heads * ((sets + 1) / 2) >= 2 * cu_count();
     const dim3 block(256), grid(n_kv_heads, two ? (sets + 1) / 2 : sets);
+    const int cus = cu_count(), per_unit = cus / n_kv_heads, rows = (int)grid.y;
+    const int unit_rows = cus % n_kv_heads == 0 && rows > per_unit && rows <= 2 * per_unit ? per_unit : 0; // see column_tile
 #define L2_PREFILL_ATTN(NP)                                                                                              \
     if (two)                                                                                                             \
-        hipLaunchKernelGGL((attn_prefill_mfma16_kernel<QG, 4, NP, 2>), grid, block, 0, st, out, q, kc, vc, pos, scatter, n_heads, n_kv_heads, B, max_pos); \
+        hipLaunchKernelGGL((attn_prefill_mfma16_kernel<QG, 4, NP, 2>), grid, block, 0, st, out, q, kc, vc, pos, scatter, n_heads, n_kv_heads, B, max_pos, unit_rows); \
     else                                                                                                                 \
-        hipLaunchKernelGGL((attn_prefill_mfma16_kernel<QG, 4, NP, 1>), grid, block, 0, st, out, q, kc, vc, pos, scatter, n_heads, n_kv_heads, B, max_pos); \
+        hipLaunchKernelGGL((attn_prefill_mfma16_kernel<QG, 4, NP, 1>), grid, block, 0, st, out, q, kc, vc, pos, scatter, n_heads, n_kv_heads, B, max_pos, unit_rows); \
     break
     switch (planes) {
         case 0: hipLaunchKernelGGL(attn_prefill_kernel<QG>, dim3(n_kv_heads, (B * QG + 7) / 8), block, 0, st, (float *)out, q, kc, vc, pos, scatter, n_heads, n_kv_heads, B); break;

@@ -85,8 +85,8 @@ def test_fp16_operator_last_tile(ops, G, batches):
 
 
 # prompt attention with two sets of columns per block (two blocks per compute unit and more), the last block with one
-# set, against passes too short for that form
-@pytest.mark.parametrize("n_heads,n_kv,n", [(32, 32, 505), (16, 2, 1021)])
+# set, and grids of one to two blocks per unit, whose tiles go in pairs, against passes too short for either
+@pytest.mark.parametrize("n_heads,n_kv,n", [(32, 32, 505), (16, 2, 1021), (32, 32, 200), (32, 32, 250), (16, 16, 300)])
 def test_prompt_attention_two_sets(ops, n_heads, n_kv, n):
     dims = ck.Dims(dim=128 * n_heads, hidden_dim=256, n_layers=2, n_heads=n_heads, n_kv_heads=n_kv, vocab_size=64,
                    seq_len=1056, group_size=64)
