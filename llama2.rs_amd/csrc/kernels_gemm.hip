@@ -561,25 +561,38 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const Q4Launch L, cons
 // What follows a residual projection (wo, w2) of a chunk: add the partial tiles and the residual (src/models.rs:263-264,
 // 283-285), store the new residual stream, take its rms scale (:55-60), and hand the stream times the norm weight to up
 // to three consumers, each in its own act-order: permuted in LDS in fp32, so that the global stores are whole 16-byte
-// pieces.  One block per token; at most kTrips x 4096 outputs.
-constexpr int kTrips = 4;
-template <int NP>
-__global__ __launch_bounds__(1024) void gemm_residual_norm_kernel(const ResNormPrep A) {
+// pieces.  One block per token; at most kTrips x 4096 outputs.  What bounds it is a chain of latencies (loads, the block's
+// sum, LDS, stores), so the consumers' orders are requested at the start, every consumer has an LDS row of its own where
+// two blocks per CU fit, and the kernel is compiled per trips and slices: at 64 registers two blocks share a CU.
+// 4096 outputs, 511 tokens 16.5 -> 12.2 us, 298 tokens in several slices 16.6 -> 12.7; 8192 outputs, 776 tokens 35.0 -> 26.0.
+constexpr int kTrips = 4, kConsumers = 3;
+template <int NP, int TRIPS, int SL>
+__global__ __launch_bounds__(1024, TRIPS <= 2 && TRIPS * SL <= 8 ? 8 : 4) void gemm_residual_norm_kernel(const ResNormPrep A, int rows) {
     __shared__ float red[16];
-    extern __shared__ __align__(16) float perm[]; // [out]
+    extern __shared__ __align__(16) float perm[]; // [rows][out]
     const int t = blockIdx.x, tid = threadIdx.x, n4 = A.out >> 2, n8 = A.out >> 3;
     const int in_p = gemm_padded(A.out);
     const size_t row = (size_t)t * A.out, slice = (size_t)A.B * A.out;
     float sq = 0.f;
-    float4 v[kTrips];
+    float4 v[TRIPS];
+    int4 id[kConsumers][TRIPS]; // the consumers' orders: requested with the rest, not behind the barriers
 #pragma unroll
-    for (int k = 0; k < kTrips; k++) {
+    for (int k = 0; k < TRIPS; k++) {
+        const int i4 = min(tid + k * 1024, n4 - 1);
+#pragma unroll
+        for (int c = 0; c < kConsumers; c++) {
+            const int32_t *inv = A.inv[min(c, A.n - 1)];
+            id[c][k] = inv ? *reinterpret_cast<const int4 *>(inv + 4 * i4) : make_int4(4 * i4, 4 * i4 + 1, 4 * i4 + 2, 4 * i4 + 3);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < TRIPS; k++) {
         const int i4 = tid + k * 1024;
         if (i4 >= n4) continue;
         const float4 g = *reinterpret_cast<const float4 *>(A.wn + 4 * i4);
         float4 w = *reinterpret_cast<const float4 *>(A.res + row + 4 * i4);
         if (A.ws) {
-            const float4 a = sum_slices(A.ws + row + 4 * i4, slice, A.KS);
+            const float4 a = sum_slices_n<SL>(A.ws + row + 4 * i4, slice, A.KS);
             w.x += a.x, w.y += a.y, w.z += a.z, w.w += a.w;
             *reinterpret_cast<float4 *>(A.x + row + 4 * i4) = w;
         }
@@ -588,39 +601,47 @@ __global__ __launch_bounds__(1024) void gemm_residual_norm_kernel(const ResNormP
     }
     for (int off = 32; off > 0; off >>= 1) sq += __shfl_xor(sq, off);
     if ((tid & 63) == 0) red[tid >> 6] = sq;
-    for (int c = 0; c < A.n; c++) {
-        if (c > 0) __syncthreads(); // the consumer before has been read out
+    for (int c0 = 0; c0 < A.n; c0 += rows) { // as many consumers at a time as the LDS has rows for
+        if (c0 > 0) __syncthreads();         // the consumers before have been read out
 #pragma unroll
-        for (int k = 0; k < kTrips; k++) {
-            const int i4 = tid + k * 1024;
-            if (i4 >= n4) continue;
-            const int4 id = A.inv[c] ? *reinterpret_cast<const int4 *>(A.inv[c] + 4 * i4) : make_int4(4 * i4, 4 * i4 + 1, 4 * i4 + 2, 4 * i4 + 3);
-            perm[id.x] = v[k].x, perm[id.y] = v[k].y, perm[id.z] = v[k].z, perm[id.w] = v[k].w;
+        for (int c = 0; c < kConsumers; c++) {
+            if (c < c0 || c >= min(c0 + rows, A.n)) continue;
+            float *pc = perm + (size_t)(c - c0) * A.out;
+#pragma unroll
+            for (int k = 0; k < TRIPS; k++) {
+                if (tid + k * 1024 >= n4) continue;
+                pc[id[c][k].x] = v[k].x, pc[id[c][k].y] = v[k].y, pc[id[c][k].z] = v[k].z, pc[id[c][k].w] = v[k].w;
+            }
         }
         __syncthreads();
-        if (c == 0 && tid == 0) {
+        if (c0 == 0 && tid == 0) {
             float s = 0.f;
             for (int w = 0; w < 16; w++) s += red[w];
             s /= (float)A.out;
             s += A.eps;
             A.ss[t] = 1.0f / sqrtf(s);
         }
-        for (int j8 = tid; j8 < (in_p >> 3); j8 += 1024) {
-            float e[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-            if (j8 < n8) {
-                const float4 a = *reinterpret_cast<const float4 *>(&perm[8 * j8]), b = *reinterpret_cast<const float4 *>(&perm[8 * j8 + 4]);
-                e[0] = a.x, e[1] = a.y, e[2] = a.z, e[3] = a.w, e[4] = b.x, e[5] = b.y, e[6] = b.z, e[7] = b.w;
+        for (int c = c0; c < min(c0 + rows, A.n); c++) {
+            const float *pc = perm + (size_t)(c - c0) * A.out;
+            for (int j8 = tid; j8 < (in_p >> 3); j8 += 1024) {
+                float e[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+                if (j8 < n8) {
+                    const float4 a = *reinterpret_cast<const float4 *>(&pc[8 * j8]), b = *reinterpret_cast<const float4 *>(&pc[8 * j8 + 4]);
+                    e[0] = a.x, e[1] = a.y, e[2] = a.z, e[3] = a.w, e[4] = b.x, e[5] = b.y, e[6] = b.z, e[7] = b.w;
+                }
+                store_piece<NP>(A.out_h[c], t, in_p, j8, make_piece<NP>(e));
             }
-            store_piece<NP>(A.out_h[c], t, in_p, j8, make_piece<NP>(e));
         }
     }
 }
 
 // What follows the q|k|v projection of a chunk: add the partial tiles of the three matrices in slice order, apply the
 // token's rms scale, rotate q and k (src/models.rs:100-129: the second half of a head uses the first half's ROTATED
-// value), write q back and k and v into the cache rows of the tokens' positions (:236-249).  One block per token;
-// thread -> (head, i < 64).
-__global__ __launch_bounds__(1024) void gemm_rope_kv_kernel(const RopeKvArgs A) {
+// value), write q back and k and v into the cache rows of the tokens' positions (:236-249).  One block per token; a thread
+// takes four neighbouring pairs of a head, or four values of v.  Blocks of 512: at one slice the launch is bound by memory
+// (50 MB in 12.3 us for 511 tokens of 4096 + 2 x 4096; 14.6 with blocks of 256, eight to a token).
+template <int SL>
+__global__ __launch_bounds__(512) void gemm_rope_kv_kernel(const RopeKvArgs A) {
     constexpr int HS = 128, HALF = 64;
     const int b = blockIdx.x;
     const int dim = A.n_heads * HS, kv_dim = A.n_kv_heads * HS;
@@ -632,49 +653,43 @@ __global__ __launch_bounds__(1024) void gemm_rope_kv_kernel(const RopeKvArgs A) 
     const float *wv = wk + (size_t)A.KS * A.B * kv_dim;
     const size_t sq = (size_t)A.B * dim, sk = (size_t)A.B * kv_dim;
     float *kc = A.kcache + (size_t)p * kv_dim, *vc = A.vcache + (size_t)p * kv_dim;
-    for (int idx = threadIdx.x; idx < A.n_heads * HALF; idx += 1024) {
-        const int h = idx >> 6, i = idx & 63;
-        const float c = ct[i], s = st[i];
-        float qa = 0.f, qb = 0.f, ka = 0.f, kb = 0.f;
-        const bool has_k = h < A.n_kv_heads;
-        for (int ks = 0; ks < A.KS; ks++) {
-            qa += wq[ks * sq + h * HS + i];
-            qb += wq[ks * sq + h * HS + i + HALF];
-            if (has_k) {
-                ka += wk[ks * sk + h * HS + i];
-                kb += wk[ks * sk + h * HS + i + HALF];
-            }
+    const int nq = dim >> 3, nk = kv_dim >> 3, nv = kv_dim >> 2;
+    for (int idx = threadIdx.x; idx < nq + nk + nv; idx += 512) {
+        if (idx >= nq + nk) {
+            const int i = (idx - nq - nk) * 4;
+            const float4 v = sum_slices_n<SL>(wv + i, sk, A.KS);
+            *reinterpret_cast<float4 *>(vc + i) = make_float4(v.x * ss, v.y * ss, v.z * ss, v.w * ss);
+            continue;
         }
-        qa *= ss, qb *= ss;
-        const float first = qa * c - qb * s;
-        A.q[(size_t)b * dim + h * HS + i] = first;
-        A.q[(size_t)b * dim + h * HS + i + HALF] = qb * c + first * s;
-        if (has_k) {
-            ka *= ss, kb *= ss;
-            const float kf = ka * c - kb * s;
-            kc[h * HS + i] = kf;
-            kc[h * HS + i + HALF] = kb * c + kf * s;
-        }
-    }
-    for (int i = threadIdx.x; i < kv_dim; i += 1024) {
-        float v = 0.f;
-        for (int ks = 0; ks < A.KS; ks++) v += wv[ks * sk + i];
-        vc[i] = v * ss;
+        const bool is_q = idx < nq;
+        const int j = is_q ? idx : idx - nq, i = (j & 15) * 4, at = (j >> 4) * HS + i;
+        const float4 c = *reinterpret_cast<const float4 *>(ct + i), s = *reinterpret_cast<const float4 *>(st + i);
+        const float *src = (is_q ? wq : wk) + at;
+        const size_t slice = is_q ? sq : sk;
+        float4 x = sum_slices_n<SL>(src, slice, A.KS), y = sum_slices_n<SL>(src + HALF, slice, A.KS);
+        x.x *= ss, x.y *= ss, x.z *= ss, x.w *= ss;
+        y.x *= ss, y.y *= ss, y.z *= ss, y.w *= ss;
+        const float4 f = make_float4(x.x * c.x - y.x * s.x, x.y * c.y - y.y * s.y, x.z * c.z - y.z * s.z, x.w * c.w - y.w * s.w);
+        float *dst = (is_q ? A.q + (size_t)b * dim : kc) + at;
+        *reinterpret_cast<float4 *>(dst) = f;
+        *reinterpret_cast<float4 *>(dst + HALF) =
+            make_float4(y.x * c.x + f.x * s.x, y.y * c.y + f.y * s.y, y.z * c.z + f.z * s.z, y.w * c.w + f.w * s.w);
     }
 }
 
 // The SiLU gate (src/models.rs:92-98) behind w1|w3 of a chunk: add the partial tiles of both, apply the token's rms
-// scale, gate, and hand the row to w2 in its act-order (permuted in LDS).  One block per token.
-template <int NP>
-__global__ __launch_bounds__(1024) void gemm_silu_kernel(const SiluArgs A) {
+// scale, gate, and hand the row to w2 in its act-order (permuted in LDS).  One block per token; with few slices in 64
+// registers, two blocks per CU: 11008 values, 511 tokens 13.6 -> 11.4 us.
+template <int NP, int SL>
+__global__ __launch_bounds__(1024, SL <= 2 ? 8 : 4) void gemm_silu_kernel(const SiluArgs A) {
     extern __shared__ __align__(16) float perm[]; // [n]
     const int t = blockIdx.x, tid = threadIdx.x, n = A.n, in_p = gemm_padded(n);
     const size_t slice = (size_t)A.B * n, row = (size_t)t * n;
     const float ss = A.ss[t];
     for (int i4 = tid; i4 < (n >> 2); i4 += 1024) {
         const int4 id = A.inv ? *reinterpret_cast<const int4 *>(A.inv + 4 * i4) : make_int4(4 * i4, 4 * i4 + 1, 4 * i4 + 2, 4 * i4 + 3);
-        const float4 a = sum_slices(A.ws + row + 4 * i4, slice, A.KS);
-        const float4 c = sum_slices(A.ws + A.KS * slice + row + 4 * i4, slice, A.KS);
+        const float4 a = sum_slices_n<SL>(A.ws + row + 4 * i4, slice, A.KS);
+        const float4 c = sum_slices_n<SL>(A.ws + A.KS * slice + row + 4 * i4, slice, A.KS);
         const float as[4] = {a.x, a.y, a.z, a.w}, cs[4] = {c.x, c.y, c.z, c.w};
         const int ids[4] = {id.x, id.y, id.z, id.w};
 #pragma unroll
@@ -833,14 +848,24 @@ int gemm_input_launch(const GemmInput &A, int n, int B, int planes, hipStream_t 
     return L2_OK;
 }
 
-template <int NP>
+template <int NP, int TRIPS, int SL>
 static int residual_norm(const ResNormPrep &A, hipStream_t st) {
-    const size_t lds = (size_t)A.out * sizeof(float);
+    // every consumer a row of LDS where two blocks per CU (a token each) still fit
+    const int rows = std::max(1, std::min(A.n, (int)(76 * 1024 / (A.out * sizeof(float)))));
+    const size_t lds = (size_t)rows * A.out * sizeof(float);
     static LdsLimit limit(48 * 1024);
-    L2_TRY(limit.ensure(reinterpret_cast<const void *>(gemm_residual_norm_kernel<NP>), lds));
-    hipLaunchKernelGGL(gemm_residual_norm_kernel<NP>, dim3(A.B), dim3(1024), lds, st, A);
+    L2_TRY(limit.ensure(reinterpret_cast<const void *>(gemm_residual_norm_kernel<NP, TRIPS, SL>), lds));
+    hipLaunchKernelGGL((gemm_residual_norm_kernel<NP, TRIPS, SL>), dim3(A.B), dim3(1024), lds, st, A, rows);
     L2_HIP(hipGetLastError());
     return L2_OK;
+}
+template <int NP, int TRIPS>
+static int residual_norm(const ResNormPrep &A, hipStream_t st) {
+    return A.KS <= 2 ? residual_norm<NP, TRIPS, 2>(A, st) : A.KS <= 8 ? residual_norm<NP, TRIPS, 8>(A, st) : residual_norm<NP, TRIPS, kMaxGemmSlices>(A, st);
+}
+template <int NP>
+static int residual_norm(const ResNormPrep &A, hipStream_t st) {
+    return A.out <= 4096 ? residual_norm<NP, 1>(A, st) : A.out <= 8192 ? residual_norm<NP, 2>(A, st) : residual_norm<NP, kTrips>(A, st);
 }
 
 int gemm_residual_norm_launch(const ResNormPrep &A, int planes, hipStream_t st) {
@@ -853,19 +878,26 @@ int gemm_residual_norm_launch(const ResNormPrep &A, int planes, hipStream_t st) 
 int gemm_rope_kv_launch(const RopeKvArgs &A, hipStream_t st) {
     if (A.KS < 1 || A.KS > kMaxGemmSlices || A.B < 1 || A.n_heads < A.n_kv_heads)
         return l2_fail(L2_ERR_ARG, "q|k|v epilogue: %d slices, %d tokens", A.KS, A.B);
-    hipLaunchKernelGGL(gemm_rope_kv_kernel, dim3(A.B), dim3(1024), 0, st, A);
+    const dim3 grid(A.B), block(512);
+    if (A.KS <= 2) hipLaunchKernelGGL(gemm_rope_kv_kernel<2>, grid, block, 0, st, A);
+    else if (A.KS <= 8) hipLaunchKernelGGL(gemm_rope_kv_kernel<8>, grid, block, 0, st, A);
+    else hipLaunchKernelGGL(gemm_rope_kv_kernel<kMaxGemmSlices>, grid, block, 0, st, A);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }
 
-template <int NP>
+template <int NP, int SL>
 static int silu(const SiluArgs &A, hipStream_t st) {
     const size_t lds = (size_t)A.n * sizeof(float);
     static LdsLimit limit(48 * 1024);
-    L2_TRY(limit.ensure(reinterpret_cast<const void *>(gemm_silu_kernel<NP>), lds));
-    hipLaunchKernelGGL(gemm_silu_kernel<NP>, dim3(A.B), dim3(1024), lds, st, A);
+    L2_TRY(limit.ensure(reinterpret_cast<const void *>(gemm_silu_kernel<NP, SL>), lds));
+    hipLaunchKernelGGL((gemm_silu_kernel<NP, SL>), dim3(A.B), dim3(1024), lds, st, A);
     L2_HIP(hipGetLastError());
     return L2_OK;
+}
+template <int NP>
+static int silu(const SiluArgs &A, hipStream_t st) {
+    return A.KS <= 2 ? silu<NP, 2>(A, st) : A.KS <= 8 ? silu<NP, 8>(A, st) : silu<NP, kMaxGemmSlices>(A, st);
 }
 
 int gemm_silu_launch(const SiluArgs &A, int planes, hipStream_t st) {

@@ -100,3 +100,30 @@ def test_prompt_attention_two_sets(ops, n_heads, n_kv, n):
     k2, v2 = m.read_kv(1, 0, n)
     assert nrel(k, k2) < 1e-5 and nrel(v, v2) < 1e-5
     m.close()
+
+
+# the kernels between the products of a chunk: rows of one, two and four trips of the block (and a consumer's order per
+# LDS row, or in turns), few K slices and many, in each kind of plane, against single tokens.  fp16 inputs carry 2^-11 each:
+# through the five products in front of the second layer's cache rows some 1e-3, and 4.5 times that at the furthest of
+# some 10^6 values, with as much again for rows of small inputs
+@pytest.mark.parametrize("n_heads,n_kv,G", [(8, 8, 64), (40, 40, 64), (64, 8, 64), (72, 9, 64), (72, 9, 0)])
+def test_between_products(ops, n_heads, n_kv, G):
+    from llama2_rs import _lib
+    dims = ck.Dims(dim=128 * n_heads, hidden_dim=384, n_layers=2, n_heads=n_heads, n_kv_heads=n_kv, vocab_size=64,
+                   seq_len=320, group_size=G)
+    m = ops.Model(ck.synth_weights_image(dims, seed=4), dims)
+    toks = np.random.default_rng(1).integers(0, 64, size=260).astype(np.int32)
+    for n in (33, 70, 260):
+        m.reset()
+        for t in range(n):
+            m.forward([int(toks[t])], [t], want_logits=False)
+        want = m.read_kv(1, 0, n)
+        for mode, tol in ((_lib.PREFILL_FP32, 1e-4), (_lib.PREFILL_MFMA, 3e-2)):
+            if mode == _lib.PREFILL_MFMA and not G:
+                continue
+            m.reset()
+            m.set_prefill_mode(mode)
+            m.prefill_chunks(toks[:n], 0, n)
+            for got, ref in zip(m.read_kv(1, 0, n), want):
+                assert nrel(got, ref) < tol, (n, mode)
+    m.close()
