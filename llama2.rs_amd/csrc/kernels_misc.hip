@@ -152,18 +152,18 @@ __device__ __forceinline__ unsigned long long amax_key(float v, int idx) {
 // eps).  Epilogue, all optional: the SiLU gate out = silu(gate[o]) * out
 // (src/models.rs:92-98, gate = the w1 output when this is w3), the residual
 // add out = res[o] + out (:47-51), and the fold of (value, index) into a 64-bit
-// maximum, one atomic per wave.  blockIdx.y is the batch column.
+// maximum, one atomic per block.  blockIdx.y is the batch column.
 //
 // A wave takes R rows at a time and issues all R * KI loads of 16 bytes per
-// lane (32 in all) before the first FMA, every load unconditional: columns past
+// lane (32 in all, fewer where the rows would not reach every compute unit)
+// before the first FMA, the first tile's in front of the staging of x, every load unconditional: columns past
 // the end re-read the row's last 16 bytes against a zero of x, rows past the
 // end re-read the last row.  Inputs longer than 32 * 64 float4 take several
 // such passes over a row (R = 1) into the same accumulator.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-template <int KI> // float4 per lane, row and pass
+template <int KI, int R> // float4 per lane, row and pass; rows
 __global__ __launch_bounds__(256) void dense_matvec_kernel(const DenseArgs A) {
-    constexpr int R = 32 / KI >= 1 ? 32 / KI : 1;
     extern __shared__ float xs[]; // n_pass * KI * 64 float4, zero beyond in
     __shared__ float red[16];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -177,6 +177,26 @@ __global__ __launch_bounds__(256) void dense_matvec_kernel(const DenseArgs A) {
     const float *__restrict__ wn = A.wn;
     const float4 *__restrict__ w4 = reinterpret_cast<const float4 *>(A.w);
     const float4 *__restrict__ xs4 = reinterpret_cast<const float4 *>(xs);
+
+    const int waves_total = gridDim.x * 4;
+    const int o_first = (blockIdx.x * 4 + wave) * R;
+    float4 wv[R][KI];
+    auto load_tile = [&](int o, int pass) {
+#pragma unroll
+        for (int k = 0; k < R; k++) {
+            // 32-bit byte offsets from the one base (the launcher checks that the matrix stays below 4 GiB)
+            const uint32_t row = (uint32_t)min(o + k, out - 1) * ((uint32_t)n4 << 4);
+#pragma unroll
+            for (int i = 0; i < KI; i++) {
+                const uint32_t col = (uint32_t)min((pass * KI + i) * 64 + lane, n4 - 1) << 4;
+                // read once per token: non-temporal, so that the rows do not displace what is re-read
+                wv[k][i] = __builtin_bit_cast(float4, __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(
+                                                          reinterpret_cast<const char *>(w4) + (row + col))));
+            }
+        }
+    };
+    load_tile(o_first, 0); // on its way while x is staged
+    __builtin_amdgcn_sched_barrier(0);
 
     float ssq = 0.f;
     for (int base = 0; base < padded; base += 256) {
@@ -207,23 +227,6 @@ __global__ __launch_bounds__(256) void dense_matvec_kernel(const DenseArgs A) {
     }
     __syncthreads();
 
-    const int waves_total = gridDim.x * 4;
-    const int o_first = (blockIdx.x * 4 + wave) * R;
-    float4 wv[R][KI];
-    auto load_tile = [&](int o, int pass) {
-#pragma unroll
-        for (int k = 0; k < R; k++) {
-            // 32-bit byte offsets from the one base (the launcher checks that the matrix stays below 4 GiB)
-            const uint32_t row = (uint32_t)min(o + k, out - 1) * ((uint32_t)n4 << 4);
-#pragma unroll
-            for (int i = 0; i < KI; i++) {
-                const uint32_t col = (uint32_t)min((pass * KI + i) * 64 + lane, n4 - 1) << 4;
-                // read once per token: non-temporal, so that the rows do not displace what is re-read
-                wv[k][i] = __builtin_bit_cast(float4, __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(
-                                                          reinterpret_cast<const char *>(w4) + (row + col))));
-            }
-        }
-    };
     unsigned long long key = 0ull;
     float *__restrict__ y = A.y + bcol * out;
     const float *__restrict__ res = A.res ? A.res + bcol * out : nullptr;
@@ -232,10 +235,13 @@ __global__ __launch_bounds__(256) void dense_matvec_kernel(const DenseArgs A) {
         float a[R];
 #pragma unroll
         for (int k = 0; k < R; k++) a[k] = 0.f;
+        float gv[R], rv[R]; // requested here: behind the next tile's loads they would wait for all of those
+#pragma unroll
+        for (int k = 0; k < R; k++) {
+            gv[k] = gate ? gate[min(o + k, out - 1)] : 0.f;
+            rv[k] = res ? res[min(o + k, out - 1)] : 0.f;
+        }
         for (int pass = 0; pass < n_pass; pass++) {
-            __builtin_amdgcn_sched_barrier(0); // a pass's loads stay behind the pass before it: one set of registers
-            load_tile(o, pass);
-            __builtin_amdgcn_sched_barrier(0); // every load of the pass before its first FMA
 #pragma unroll
             for (int i = 0; i < KI; i++) {
                 const float4 xx = xs4[(pass * KI + i) * 64 + lane];
@@ -247,23 +253,33 @@ __global__ __launch_bounds__(256) void dense_matvec_kernel(const DenseArgs A) {
                     a[k] = fmaf(wv[k][i].w, xx.w, a[k]);
                 }
             }
+            __builtin_amdgcn_sched_barrier(0); // the next pass's loads stay behind this one: one set of registers
+            const bool same = pass + 1 < n_pass;
+            const int next = same ? o : o + waves_total * R;
+            if (next < out) load_tile(next, same ? pass + 1 : 0);
+            __builtin_amdgcn_sched_barrier(0); // in front of the sums below and of the next pass's FMAs
         }
 #pragma unroll
         for (int k = 0; k < R; k++) {
             float v = wave_sum(a[k]) * ss;
             if (lane == 0 && o + k < out) {
-                if (gate) {
-                    const float g = gate[o + k];
-                    v = (g * (1.0f / (1.0f + expf(-g)))) * v;
-                }
-                if (res) v = res[o + k] + v;
+                if (gate) v = (gv[k] * (1.0f / (1.0f + expf(-gv[k])))) * v;
+                if (res) v = rv[k] + v;
                 y[o + k] = v;
                 const unsigned long long kk = amax_key(v, o + k);
                 key = kk > key ? kk : key;
             }
         }
     }
-    if (lane == 0 && A.amax && key) atomicMax(A.amax, key);
+    if (A.amax) { // one atomic per block: all of them go to one address, some 6 ns each (7B 83.3 -> 81.5 us)
+        __shared__ unsigned long long keys[4];
+        if (lane == 0) keys[wave] = key;
+        __syncthreads();
+        if (tid == 0) {
+            key = max(max(keys[0], keys[1]), max(keys[2], keys[3]));
+            if (key) atomicMax(A.amax, key);
+        }
+    }
 }
 
 // Greedy hand-over (src/inference.rs:154-162, 185-189): next is the forced
@@ -418,10 +434,14 @@ int dense_launch(const DenseArgs &a0, hipStream_t st) {
     if (a.amax && a.batch != 1) return l2_fail(L2_ERR_ARG, "dense matvec: the running maximum takes one column");
     const int ki = (a.in / 4 + 63) / 64; // float4 per lane and row
     const int KI = ki <= 4 ? 4 : ki <= 8 ? 8 : ki <= 16 ? 16 : ki <= 20 ? 20 : 32;
-    const int R = 32 / KI >= 1 ? 32 / KI : 1;
+    int R = 32 / KI >= 1 ? 32 / KI : 1;
+    // One column of few rows: fewer rows per wave where whole tiles would leave compute units without a block
+    // (2000 rows of 1024: 63 blocks 9.9 us, 250 blocks 6.6).
+    const bool few = KI <= 16 && a.batch == 1 && (a.out + 4 * R - 1) / (4 * R) < cu_count();
+    if (few) R = KI == 4 ? 2 : 1;
     a.n_pass = (ki + KI - 1) / KI;
     // One column (the classifier of a decode step): one block per CU -- 7B 93 -> 85 us, 13B 112 -> 103, 70B 172 ->
-    // 161 against three per CU, which the registers would allow and which stays the rule for several columns.
+    // 161 (7B now 81.5) against three per CU, which the registers would allow and which stays the rule for several columns.
     // Fewer when the rows run out.
     const int per_cu = a.batch == 1 ? 1 : 3;
     int blocks = (per_cu * cu_count() + a.batch - 1) / a.batch;
@@ -432,14 +452,15 @@ int dense_launch(const DenseArgs &a0, hipStream_t st) {
     if (lds > 48 * 1024) { // only rows of more than one pass, which run with KI = 32
         if (KI != 32) return l2_fail(L2_ERR_ARG, "dense matvec: in=%d out=%d needs %zu B of LDS with %d loads per pass", a.in, a.out, lds, KI);
         static LdsLimit limit;
-        L2_TRY(limit.ensure(reinterpret_cast<const void *>(dense_matvec_kernel<32>), lds));
+        L2_TRY(limit.ensure(reinterpret_cast<const void *>(dense_matvec_kernel<32, 1>), lds));
     }
+    auto launch = [&](void (*kernel)(DenseArgs)) { hipLaunchKernelGGL(kernel, grid, block, lds, st, a); };
     switch (KI) {
-        case 4: hipLaunchKernelGGL(dense_matvec_kernel<4>, grid, block, lds, st, a); break;
-        case 8: hipLaunchKernelGGL(dense_matvec_kernel<8>, grid, block, lds, st, a); break;
-        case 16: hipLaunchKernelGGL(dense_matvec_kernel<16>, grid, block, lds, st, a); break;
-        case 20: hipLaunchKernelGGL(dense_matvec_kernel<20>, grid, block, lds, st, a); break;
-        default: hipLaunchKernelGGL(dense_matvec_kernel<32>, grid, block, lds, st, a); break;
+        case 4: launch(few ? dense_matvec_kernel<4, 2> : dense_matvec_kernel<4, 8>); break;
+        case 8: launch(few ? dense_matvec_kernel<8, 1> : dense_matvec_kernel<8, 4>); break;
+        case 16: launch(few ? dense_matvec_kernel<16, 1> : dense_matvec_kernel<16, 2>); break;
+        case 20: launch(dense_matvec_kernel<20, 1>); break;
+        default: launch(dense_matvec_kernel<32, 1>); break;
     }
     L2_HIP(hipGetLastError());
     return L2_OK;

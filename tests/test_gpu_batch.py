@@ -127,3 +127,23 @@ def test_between_products(ops, n_heads, n_kv, G):
             for got, ref in zip(m.read_kv(1, 0, n), want):
                 assert nrel(got, ref) < tol, (n, mode)
     m.close()
+
+
+# the classifier with whole tiles of rows per wave and with a quarter, at both sides of where the rule changes, the last
+# wave ragged; its running maximum against the logits
+@pytest.mark.parametrize("n_heads,vocab", [(8, 1), (8, 2001), (8, 8160), (8, 8163), (16, 4080), (16, 4083), (32, 2033), (32, 2049), (40, 1025)])
+def test_classifier_few_rows(ops, n_heads, vocab):
+    dim = 128 * n_heads
+    dims = ck.Dims(dim=dim, hidden_dim=256, n_layers=1, n_heads=n_heads, n_kv_heads=n_heads, vocab_size=vocab, seq_len=32,
+                   group_size=64)
+    img = ck.synth_weights_image(dims, seed=vocab)
+    m = ops.Model(img, dims)
+    W = img[-4 * vocab * dim:].view(np.float32).reshape(vocab, dim).astype(np.float64)
+    x = np.random.default_rng(2).standard_normal(dim).astype(np.float32)
+    want = W @ x.astype(np.float64)
+    # fp32 sums of at most 80 dim / 4096 roundings in a row, and the six of a wave's lanes
+    assert np.all(np.abs(m.classifier(x) - want) < 90 * 2.0 ** -24 * (np.abs(W) @ np.abs(x.astype(np.float64))))
+    for pos in range(6):
+        logits = m.forward([0], [pos])
+        assert m.decode_greedy(0, pos) == vocab - 1 - int(np.argmax(logits[::-1]))
+    m.close()
