@@ -834,8 +834,10 @@ extern "C" int l2_model_set_prefill_mode(l2_model *m, int mode) {
 // each the bits of a single one.  Measured on the operator, matvec against GEMM: 4096x4096 13.7 against 13.9 us at 4
 // columns, 22 against 14 at 8; 4096x1024 13.5 against 12.9 at 16; 1024x1024 13.0 against 13.9 at 48.
 static bool gemm_pays(int B, double weights) { return B >= 4 && B * weights >= 6e7; }
-// The same for the layers of a model (nine launches each instead of seven).
-static bool gemm_pays_layer(int B, double weights) { return B >= 8 && B * weights >= 6e8; }
+// The same for the layers of a model (nine launches each instead of seven).  Three layers of 1024 inputs, 2816 hidden units,
+// with the logits behind them, matvec against GEMM: 8 columns 228 against 256 us, 12 257 against 258, 16 284 against 260,
+// 32 394 against 270, 48 514 against 300.
+static bool gemm_pays_layer(int B, double weights) { return B >= 8 && B * weights >= 1.4e8; }
 
 // What a batch of B columns of this model is computed with: 0 = the matvec kernels column by column, 1 or 3 = the GEMM
 // with that many planes of activations.
