@@ -919,12 +919,12 @@ extern "C" int l2_state_new(l2_model *m, l2_state **out) {
     s->elems = (size_t)m->d.n_layers * m->max_seq * m->kv_dim;
     int rc = dalloc(&s->kcache, s->elems);
     if (rc == L2_OK) rc = dalloc(&s->vcache, s->elems);
-    if (rc == L2_OK) { // fresh memory is cleared whole (2 GB: 60 us quicker than row by row)
-        hipError_t e = hipMemsetAsync(s->kcache, 0, s->elems * 4, m->stream);
-        if (e == hipSuccess) e = hipMemsetAsync(s->vcache, 0, s->elems * 4, m->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
-        if (e != hipSuccess) rc = l2_fail(L2_ERR_HIP, "clearing a new state: %s", hipGetErrorString(e));
+    if (rc != L2_OK) {
+        l2_state_free(s);
+        return rc;
     }
+    s->rows = m->max_seq; // nothing is known of fresh memory
+    rc = l2_state_reset(s);
     if (rc != L2_OK) {
         l2_state_free(s);
         return rc;
