@@ -320,6 +320,7 @@ struct l2_model {
         float *logits = nullptr;               // [vocab]: logits, or the sampler's weights
         unsigned long long *redo = nullptr;    // one bit per vocabulary entry
         int32_t *ids = nullptr, *in = nullptr; // [max_seq] out; [2 * max(max_seq, 4096)] in
+        bool reading = false; // a copy from `in` may still be on its way: no call has waited since
     } hs;
     static constexpr int kMaxLanes = 4; // the process has four hardware queues
     int n_lanes = 2;
@@ -474,7 +475,8 @@ struct HostSlot {
 static struct HostSlots {
     static constexpr size_t kKept = 4;
     std::mutex mu;
-    std::vector<HostSlot> idle;
+    HostSlot idle[kKept];
+    size_t n_idle = 0;
     int users = 0;
 
     void add_user() {
@@ -484,15 +486,13 @@ static struct HostSlots {
     void drop_user() {
         std::lock_guard<std::mutex> lock(mu);
         if (--users > 0) return;
-        for (HostSlot &s : idle) (void)hipHostFree(s.base);
-        idle.clear();
+        while (n_idle > 0) (void)hipHostFree(idle[--n_idle].base);
     }
     int take(HostSlot *out) {
         {
             std::lock_guard<std::mutex> lock(mu);
-            if (!idle.empty()) {
-                *out = idle.back();
-                idle.pop_back();
+            if (n_idle > 0) {
+                *out = idle[--n_idle];
                 return L2_OK;
             }
         }
@@ -506,8 +506,8 @@ static struct HostSlots {
     }
     void give(const HostSlot &s) {
         std::lock_guard<std::mutex> lock(mu);
-        if (idle.size() < kKept && users > 0)
-            idle.push_back(s);
+        if (n_idle < kKept && users > 0)
+            idle[n_idle++] = s;
         else
             (void)hipHostFree(s.base);
     }
@@ -1401,6 +1401,15 @@ static int wait_host(l2_model *m, const unsigned long long *amax, int32_t *id) {
     const uint32_t seq = ++m->hs.seq;
     L2_TRY(finish_launch(amax, id, const_cast<uint32_t *>(m->hs.flag), seq, m->stream));
     if (!watch_flag(m->hs.flag, seq)) L2_HIP(hipStreamSynchronize(m->stream));
+    m->hs.reading = false;
+    return L2_OK;
+}
+
+// Before hs.in is written: a call that enqueued a prompt and left without waiting (an error behind it) may have its copy
+// from there in flight.
+static int claim_host_ids(l2_model *m) {
+    if (m->hs.reading) L2_HIP(hipStreamSynchronize(m->stream));
+    m->hs.reading = true;
     return L2_OK;
 }
 
@@ -1750,6 +1759,7 @@ extern "C" int l2_forward(l2_model *m, l2_state *s, const int32_t *tokens, const
     L2_TRY(ensure_batch(m, B));
     if (B > 1) {
         L2_TRY(ensure_ids(m, B));
+        L2_TRY(claim_host_ids(m));
         memcpy(m->hs.in, tokens, (size_t)B * 4);
         memcpy(m->hs.in + B, pos, (size_t)B * 4);
         L2_HIP(hipMemcpyAsync(m->pf_ids, m->hs.in, (size_t)B * 8, hipMemcpyHostToDevice, m->stream));
@@ -1837,6 +1847,7 @@ static int prefill_chunks(l2_model *m, l2_state *s, const int32_t *tokens, int n
     L2_TRY(ensure_batch(m, std::max(rest, 1)));
     L2_TRY(ensure_prefill_pipeline(m, lanes, widest, cut, planes));
     L2_TRY(ensure_ids(m, n));
+    L2_TRY(claim_host_ids(m));
     memcpy(m->hs.in, tokens, (size_t)n * 4);
     for (int i = 0; i < n; i++) m->hs.in[n + i] = pos0 + i;
     const int32_t *dtok = m->pf_ids, *dpos = m->pf_ids + n;
@@ -1991,7 +2002,7 @@ static int steps_enqueue(l2_model *m, l2_state *s, int32_t first, int pos0, int 
     if (m->use_graph && !m->prof_on) {
         L2_TRY(ensure_loop_buffers(m, std::max(n_prompt, 1), std::max(n, 1)));
         if (n_prompt > 0) {
-            L2_HIP(hipStreamSynchronize(m->stream)); // a prefill before may still be reading its ids there
+            L2_TRY(claim_host_ids(m)); // a prefill before may still be reading its ids there
             memcpy(m->hs.in, prompt, (size_t)std::min(n_prompt, m->max_seq) * 4);
             L2_HIP(hipMemcpyAsync(m->dprompt, m->hs.in, (size_t)std::min(n_prompt, m->max_seq) * 4, hipMemcpyHostToDevice, m->stream));
         }
@@ -2047,13 +2058,13 @@ int l2_prefill_ladder_end(int n_prompt) {
 
 // The rungs of the ladder one behind the other are one prompt: the tokens START, prompt[0], ... (:29-33) at the
 // positions before l2_prefill_ladder_end.  They go through in as few, evenly filled passes as kPassTokens allows.
-int l2_prefill_ladder(l2_model *m, l2_state *s, const int32_t *prompt, int n_prompt) {
+int l2_prefill_ladder(l2_model *m, l2_state *s, const int32_t *prompt, int n_prompt, bool wait) {
     const int n = l2_prefill_ladder_end(n_prompt);
     if (n == 0) return L2_OK;
     std::vector<int32_t> toks((size_t)n);
     for (int i = 0; i < n; i++) toks[i] = i == 0 ? 1 : prompt[i - 1];
     const int passes = (n + kPassTokens - 1) / kPassTokens;
-    return prefill_chunks(m, s, toks.data(), n, 0, (n + passes - 1) / passes, false);
+    return prefill_chunks(m, s, toks.data(), n, 0, (n + passes - 1) / passes, wait);
 }
 
 extern "C" int l2_generate_greedy(l2_model *m, l2_state *s, const int32_t *prompt, int n_prompt, int steps,
@@ -2076,7 +2087,7 @@ extern "C" int l2_generate_greedy(l2_model *m, l2_state *s, const int32_t *promp
     int pos = 0;
     if (use_prefill) { // :78-127
         pos = l2_prefill_ladder_end(n_prompt);
-        L2_TRY(l2_prefill_ladder(m, s, prompt, n_prompt));
+        L2_TRY(l2_prefill_ladder(m, s, prompt, n_prompt, false));
     }
     const int32_t first = pos == 0 ? 1 : prompt[pos - 1]; // :128-132
     const int n = std::max(steps - pos, 0); // :141

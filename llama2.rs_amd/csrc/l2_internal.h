@@ -72,8 +72,8 @@ struct LdsLimit {
 
 // Position at which the prefill ladder 64/32/16/8/4/2 (src/inference.rs:78-127) leaves off.
 int l2_prefill_ladder_end(int n_prompt);
-// What the ladder computes: the cache rows of the positions before that (enqueued, not waited for).
-int l2_prefill_ladder(l2_model *m, l2_state *s, const int32_t *prompt, int n_prompt);
+// What the ladder computes: the cache rows of the positions before that (enqueued; waited for with `wait`).
+int l2_prefill_ladder(l2_model *m, l2_state *s, const int32_t *prompt, int n_prompt, bool wait);
 
 // One forward step for the sampler: the weights above of the logits at `pos`, in host memory that belongs to the model
 // and stands until its next call.

@@ -362,7 +362,7 @@ extern "C" int l2_generate(l2_model *m, l2_state *s, const l2_tokenizer *t, cons
                 const int tok = pos == 0 ? 1 : prompt32[pos - 1];
                 L2_TRY(emit(tok, tok, false)); // :37-40
             }
-            L2_TRY(l2_prefill_ladder(m, s, prompt32.data(), n_prompt));
+            L2_TRY(l2_prefill_ladder(m, s, prompt32.data(), n_prompt, pos >= steps)); // no step waits for it behind the last
         }
         int32_t token = pos == 0 ? 1 : prompt32[pos - 1];
         L2_TRY(emit(token, token, false)); // :134-137

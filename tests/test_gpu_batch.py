@@ -147,3 +147,23 @@ def test_classifier_few_rows(ops, n_heads, vocab):
         logits = m.forward([0], [pos])
         assert m.decode_greedy(0, pos) == vocab - 1 - int(np.argmax(logits[::-1]))
     m.close()
+
+
+# a text whose prompt alone passes `steps`: the prompt's rows are there whatever the next call stages on the host
+def test_prompt_past_the_steps(ops):
+    import os
+    import types
+    import llama2_rs
+    dims = ck.Dims(dim=1024, hidden_dim=512, n_layers=2, n_heads=8, n_kv_heads=8, vocab_size=32000, seq_len=1024, group_size=64)
+    m = ops.Model(ck.synth_weights_image(dims, seed=6), dims)
+    tok = llama2_rs.Tokenizer(os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden", "tokenizer.bin"))
+    text = "the quick brown fox " * 100
+    rows = []
+    for follow in (False, True):
+        llama2_rs.generate(types.SimpleNamespace(_m=m), tok, text, 2, llama2_rs.Random(1), 0.8)
+        if follow:
+            m.prefill_chunks(np.full(400, 7, np.int32), 600, 64)
+        rows.append(m.read_kv(1, 0, 384))
+    for a, b in zip(*rows):
+        assert np.any(a[383]) and np.array_equal(a, b)
+    m.close()
