@@ -817,6 +817,19 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(float *__restrict__ o
     }
 }
 
+// Column tile of block row y of n.  The work of a tile grows with its position, and blocks are dealt over the compute
+// units in turn, `unit_rows` rows until every unit has one.  With up to two blocks per unit all are resident at once and
+// the launch is as long as the unit with the most work, so the longest tiles get a unit to themselves and the others go
+// in pairs of a long and a short one: 32 heads, 511 tokens 41.5 -> 37.1 us (against longest first, which pairs the longest
+// with the middle).  Larger grids (unit_rows = 0) are worked off as units become free, longest first; dealing three per
+// unit the same way gained nothing (299 tokens 27.0, 27.9).
+__device__ __forceinline__ int column_tile(int y, int n, int unit_rows) {
+    if (unit_rows == 0) return n - 1 - y;
+    const int second = n - unit_rows; // rows of second blocks
+    if (y >= unit_rows) return y - unit_rows;
+    return n - 1 - (y < second ? unit_rows - second + y : y - second);
+}
+
 // Chunk attention on the matrix cores, all in fp32 (v_mfma_f32_16x16x4_f32): src/models.rs:131-176 with B > 1, causal per
 // query over the cache rows 0..pos (every row of the chunk is already written, q is rotated), in the layout of attn_decode_mfma_kernel: a block owns 16 columns of one kv head, column
 // n = (query ct*16/QG + n/QG, head kvh*QG + n%QG), its NWV waves take the tiles of 16 cache rows w, w + NWV, ...
@@ -835,20 +848,6 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(float *__restrict__ o
 // tokens 8.6, 7.9.  (v_mfma_f32_16x16x4_f32 at its peak: 63 us for the first of these.)  (A form on 32 columns and tiles of 32 rows,
 // v_mfma_f32_32x32x2_f32 with K and V turned through LDS, had half the blocks and took 16 to 31 us per chunk of a
 // 512-token prompt where this one takes 11 to 19.)
-
-// Column tile of block row y of n.  The work of a tile grows with its position, and blocks are dealt over the compute
-// units in turn, `unit_rows` rows until every unit has one.  With up to two blocks per unit all are resident at once and
-// the launch is as long as the unit with the most work, so the longest tiles get a unit to themselves and the others go
-// in pairs of a long and a short one: 32 heads, 511 tokens 41.5 -> 37.1 us (against longest first, which pairs the longest
-// with the middle).  Larger grids (unit_rows = 0) are worked off as units become free, longest first; dealing three per
-// unit the same way gained nothing (299 tokens 27.0, 27.9).
-__device__ __forceinline__ int column_tile(int y, int n, int unit_rows) {
-    if (unit_rows == 0) return n - 1 - y;
-    const int second = n - unit_rows; // rows of second blocks
-    if (y >= unit_rows) return y - unit_rows;
-    return n - 1 - (y < second ? unit_rows - second + y : y - second);
-}
-
 template <int QG, int NWV, int NP, int CS>
 __global__ __launch_bounds__(NWV * 64, NWV == 4 ? 2 : 1)
 void attn_prefill_mfma16_kernel(void *__restrict__ out, const float *__restrict__ q, const float *__restrict__ kc,
