@@ -1046,6 +1046,12 @@ static int q4_one_natural(const DevQLinear &q, const float *x, float *xg_scratch
     return q4_one(q, xg_scratch, y, B, st);
 }
 
+// Whether n floats at a and m floats at b share any.
+static bool ranges_overlap(const float *a, size_t n, const float *b, size_t m) {
+    const uintptr_t a0 = (uintptr_t)a, b0 = (uintptr_t)b;
+    return a0 < b0 + m * sizeof(float) && b0 < a0 + n * sizeof(float);
+}
+
 static int check_qlinear_shape(int in, int out, int g) {
     if (g != 32 && g != 64 && g != 128) return l2_fail(L2_ERR_ARG, "group size %d (32, 64 or 128)", g);
     if (in <= 0 || out <= 0 || in % 32 || in % g || out % 8)
@@ -1287,8 +1293,9 @@ extern "C" int l2_qlinear_matvec_device(l2_qlinear *q, const float *x_dev, int B
     if (operator_planes(q->q, B))
         return gemm_operator(q->q, x_dev, B, y_dev, 3, fixed.planes, fixed.ws, kOperatorWsFloats, st);
     // One column: the kernel applies the permutation while it stages x (one launch where the host's launch rate is what
-    // counts: 9.7 -> 6.6 us per call at 8192x1024).  Several columns are gathered once, rather than by every block of every column.
-    if (B == 1) return q4_one_natural(q->q, x_dev, fixed.xg, y_dev, 1, st);
+    // counts: 9.7 -> 6.6 us per call at 8192x1024).  Its blocks read all of x while others write y already, so where y lies
+    // over x, x is gathered by a launch in front.  Several columns are gathered once, rather than by every block of every column.
+    if (B == 1 && !ranges_overlap(x_dev, q->q.in, y_dev, q->q.out)) return q4_one_natural(q->q, x_dev, fixed.xg, y_dev, 1, st);
     L2_TRY(gather_launch(fixed.xg, x_dev, q->q.g_index, q->q.in, B, st));
     return q4_one(q->q, fixed.xg, y_dev, B, st);
 }

@@ -1,0 +1,59 @@
+"""l2_qlinear_matvec_device on buffers as a caller may lay them out, against the same operator on host arrays."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from llama2_rs import checkpoint as ck
+from tests.test_zz_no_alloc import _Hip
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from llama2_rs import ops as o, _lib
+    assert _lib.lib().l2_device_count() >= 1, "no HIP device: the GPU tests cannot run"
+    return o
+
+
+# y over x: in place, shifted either way, sharing four elements, and touching without sharing any.  One column (which
+# takes one launch only where nothing is shared), a few (the matvec kernels) and a batch (the matrix cores).
+@pytest.mark.parametrize("n_in,n_out,G", [(1024, 1024, 32), (4096, 4096, 128), (8192, 1024, 64), (2816, 8448, 128)])
+@pytest.mark.parametrize("B", [1, 3, 24])
+def test_result_over_the_input(ops, n_in, n_out, G, B):
+    hip = _Hip()
+    rng = np.random.default_rng(n_in + B)
+    q = ops.QLinear(*ck.synth_qlinear(rng, n_in, n_out, G, act_order=True), G)
+    x = rng.standard_normal((B, n_in)).astype(np.float32)
+    want = q.matvec(x)
+    nx, ny = B * n_in, B * n_out
+    image = np.full(nx + 2 * ny, np.nan, np.float32)
+    image[ny:ny + nx] = x.reshape(-1)
+    for shift in (0, 4, -4, nx // 2, nx - 4, 4 - ny, nx, -ny):
+        buf = hip.upload(image)
+        q.matvec_device(buf + 4 * ny, B, buf + 4 * (ny + shift))
+        np.testing.assert_array_equal(hip.download(buf + 4 * (ny + shift), (B, n_out)), want, err_msg=f"shift {shift}")
+    q.close()
+    hip.close()
+
+
+# what one column enqueues (captured, not run): one kernel where x and y are apart, a gather in front where they meet
+def test_one_launch_only_apart(ops):
+    hip = _Hip()
+    rt = hip.rt
+    q = ops.QLinear(*ck.synth_qlinear(np.random.default_rng(2), 4096, 1024, 128, act_order=True), 128)
+    buf, stream = hip.empty(4 * (4096 + 2 * 1024)), C.c_void_p()
+    assert rt.hipStreamCreate(C.byref(stream)) == 0
+    for shift, nodes in ((0, 2), (-1024, 1), (-1020, 2), (2048, 2), (4092, 2), (4096, 1)):
+        graph, n = C.c_void_p(), C.c_size_t()
+        assert rt.hipStreamBeginCapture(stream, 0) == 0            # hipStreamCaptureModeGlobal
+        try:
+            q.matvec_device(buf + 4 * 1024, 1, buf + 4 * (1024 + shift), stream=stream.value)
+        finally:
+            assert rt.hipStreamEndCapture(stream, C.byref(graph)) == 0
+        assert rt.hipGraphGetNodes(graph, None, C.byref(n)) == 0 and n.value == nodes, shift
+        assert rt.hipGraphDestroy(graph) == 0
+    assert rt.hipStreamDestroy(stream) == 0
+    q.close()
+    hip.close()
