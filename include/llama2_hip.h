@@ -157,7 +157,8 @@ int l2_qlinear_matvec(l2_qlinear *q, const float *x_host, int B, float *y_host);
  * serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  x_dev f32[B][in] and
  * y_dev f32[B][out] are DEVICE pointers; the operator's kernels are enqueued on hip_stream (a
  * hipStream_t; NULL is the default stream) and the call returns without waiting.  y may lie over x, in part or
- * as a whole (compared by address: memory mapped at two addresses must not be given as both).  It calls no hipMalloc,
+ * as a whole (compared by address: memory mapped at two addresses must not be given as both).  Both are aligned
+ * as floats are; more is not asked for.  It calls no hipMalloc,
  * hipFree or other allocating routine: the one intermediate (x in the layer's act-order) lives in a fixed
  * device array of L2_MATVEC_DEVICE_MAX_ELEMS floats (48 MiB with what a batch needs) that each GPU holds until the process
  * ends, so B * in must not exceed that count (L2_ERR_RANGE otherwise).  All calls on one GPU share the array:

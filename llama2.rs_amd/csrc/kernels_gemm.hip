@@ -151,7 +151,7 @@ __device__ __forceinline__ void finish4(const Q4Launch &L, int mi, const float *
         const float4 rr = *reinterpret_cast<const float4 *>(L.e.res + at);
         v.x += rr.x, v.y += rr.y, v.z += rr.z, v.w += rr.w;
     }
-    *reinterpret_cast<float4 *>(L.m[mi].y + at) = v;
+    *reinterpret_cast<float4_any *>(L.m[mi].y + at) = float4_any{v.x, v.y, v.z, v.w};
 }
 
 constexpr int kRowHalves = 72; // halves per staged token row: 64 k + 8 (16-byte reads of 32 lanes stay conflict-free)
@@ -555,7 +555,7 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const Q4Launch L, cons
         const float4 r = *reinterpret_cast<const float4 *>(L.e.res + at);
         v.x += r.x, v.y += r.y, v.z += r.z, v.w += r.w;
     }
-    *reinterpret_cast<float4 *>(M.y + at) = v;
+    *reinterpret_cast<float4_any *>(M.y + at) = float4_any{v.x, v.y, v.z, v.w};
 }
 
 // What follows a residual projection (wo, w2) of a chunk: add the partial tiles and the residual (src/models.rs:263-264,

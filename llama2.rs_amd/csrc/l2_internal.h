@@ -29,6 +29,10 @@ inline int cu_count() {
     return n;
 }
 
+// Four floats at an address that a caller of the C ABI chose, aligned as a float is and no more.  gfx950 moves 16 bytes
+// at any multiple of four, so a load or store through this is the same one instruction as through float4.
+typedef float float4_any __attribute__((ext_vector_type(4), aligned(4)));
+
 // ---- error plumbing -------------------------------------------------------
 int l2_fail(int code, const char *fmt, ...) __attribute__((format(printf, 2, 3)));
 

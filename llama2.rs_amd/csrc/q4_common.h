@@ -69,14 +69,14 @@ struct StageRegs {
 template <int NW>
 __device__ __forceinline__ void stage_issue(const float *__restrict__ xin_f, const float *__restrict__ wn_f,
                                             int in, int base, int tid, StageRegs &r) {
-    const float4 *xin = reinterpret_cast<const float4 *>(xin_f);
+    const float4_any *xin = reinterpret_cast<const float4_any *>(xin_f); // may be a caller's (the gathering form)
     const float4 *wn = reinterpret_cast<const float4 *>(wn_f);
     const int n4 = in >> 2;
     constexpr int T = NW * 64;
 #pragma unroll
     for (int u = 0; u < kStageBatch; u++) {
         const int j4 = base + u * T + tid;
-        r.v[u] = j4 < n4 ? xin[j4] : make_float4(0.f, 0.f, 0.f, 0.f);
+        r.v[u] = j4 < n4 ? __builtin_bit_cast(float4, xin[j4]) : make_float4(0.f, 0.f, 0.f, 0.f);
         r.g[u] = (wn_f && j4 < n4) ? wn[j4] : make_float4(1.f, 1.f, 1.f, 1.f);
     }
 }

@@ -38,6 +38,28 @@ def test_result_over_the_input(ops, n_in, n_out, G, B):
     hip.close()
 
 
+# x and y at addresses that are multiples of four bytes and of nothing more, and nothing written beside y: one column, a
+# few, and batches in one K slice (17160 outputs) and in several
+@pytest.mark.parametrize("n_in,n_out,G,batches", [(1024, 264, 32, (1, 3, 250)), (4096, 4104, 128, (1, 3, 5, 40, 250)),
+                                                  (8192, 8192, 64, (1, 2, 100)), (1024, 17160, 32, (250,))])
+def test_any_float_address(ops, n_in, n_out, G, batches):
+    hip = _Hip()
+    rng = np.random.default_rng(n_in)
+    q = ops.QLinear(*ck.synth_qlinear(rng, n_in, n_out, G, act_order=True), G)
+    for B in batches:
+        x = rng.standard_normal((B, n_in)).astype(np.float32)
+        want = q.matvec(x)
+        for dx, dy in ((1, 0), (0, 1), (2, 3), (3, 2)):
+            px = hip.upload(np.concatenate([np.full(dx, np.nan, np.float32), x.reshape(-1)]))
+            py = hip.upload(np.full(dy + want.size + 4, 7.0, np.float32))
+            q.matvec_device(px + 4 * dx, B, py + 4 * dy)
+            got = hip.download(py, (dy + want.size + 4,))
+            np.testing.assert_array_equal(got[dy:dy + want.size].reshape(want.shape), want, err_msg=f"{B} {dx} {dy}")
+            assert np.all(got[:dy] == 7.0) and np.all(got[dy + want.size:] == 7.0)
+    q.close()
+    hip.close()
+
+
 # what one column enqueues (captured, not run): one kernel where x and y are apart, a gather in front where they meet
 def test_one_launch_only_apart(ops):
     hip = _Hip()
