@@ -396,14 +396,26 @@ __global__ __launch_bounds__(256, 2) void q4_tile_gemm_kernel(const Q4Launch L, 
 // behind it).  The matvec kernel once per column read the weights once per column: two layers of 7B's widths, 99 columns
 // 16 -> 1 ms.
 //
-// A block is four waves of MT x NB tiles of 32 rows x 32 columns, side by side over the rows.  Lane (r = l % 32,
-// h = l / 32) loads inputs 16 h .. 16 h + 15 of every 32 of its row, 16 bytes at a time; step e of float4 i multiplies
-// inputs 4 i + e and 16 + 4 i + e.  The activations' 32 inputs per column pass through LDS, double-buffered.
-template <int MT, int NB>
-__global__ __launch_bounds__(256, 2) void dense_gemm_kernel(const Q4Launch L, const XhList xl, int in_p,
+// A block is four waves of NB tiles of 32 rows x 32 columns, side by side over the rows.  Lane (r = l % 32, h = l / 32)
+// loads inputs 16 h .. 16 h + 15 of every 32 of its row, 16 bytes at a time; step e of float4 i multiplies inputs 4 i + e
+// and 16 + 4 i + e.  The activations' 32 inputs per column pass through LDS, double-buffered.
+//
+// Sums.  The matrix unit rounds once per product, and the error of a sum of n terms, each added to all before it, grows
+// with n.  The matvec adds 64 lanes' shares in a tree, so that in / 64 products follow each other; to be no further from
+// the exact sum than that, the products of a K step (of a part of it where the matvec's own chains are short) are summed
+// from zero, the steps of a run are added to each other, and the runs; the slices of K follow in a tree (sum_slices_n).
+// Runs of sqrt(steps / 2) and more make the two upper chains about equally long.  Relative rms error against fp64, normal
+// inputs, matvec / this / one accumulator for the whole slice: 1024 inputs, 61 columns 1.00e-7 / 9.1e-8 / 2.1e-7; 4096,
+// 128 columns 1.59e-7 / 1.27e-7 / 4.1e-7; 11008, 512 columns 2.44e-7 / 1.44e-7 / 9.4e-7.
+// The sums take the registers of a second row tile (which would reuse every LDS read twice: the matrix unit is slow enough
+// in fp32 for one).  Prompts, two row tiles and one accumulator / this: two layers of 7B's widths, 100 tokens 0.95-0.99 /
+// 0.98 ms, 512 tokens 3.60 / 3.41; four layers of 1024 inputs, 33 tokens 0.29 / 0.31; one of 70B's widths, 64 tokens
+// 1.09-1.13 / 1.12-1.17.
+template <int NB, int FOLDS> // FOLDS: sums from zero per K step
+__global__ __launch_bounds__(256, FOLDS == 4 ? 2 : 3) void dense_gemm_kernel(const Q4Launch L, const XhList xl, int in_p,
                                                             const float *__restrict__ ss, float *__restrict__ ws, int KS,
                                                             int t_tiles, int partials) {
-    constexpr int TN = 32 * NB, RW = 32 * MT, RB = 4 * RW, kRow = 36; // floats per staged column: 32 + 4
+    constexpr int TN = 32 * NB, RB = 128, kRow = 36; // floats per staged column: 32 + 4
     __shared__ __align__(16) float xs[4608]; // [2][TN][kRow], and the four output tiles of the epilogue
     static_assert(2 * TN * kRow <= 4608 && 4 * 32 * 36 <= 4608, "LDS");
     const int n_blocks = gridDim.x, per_xcd = n_blocks >> 3, over = n_blocks & 7, xcd = blockIdx.x & 7;
@@ -424,21 +436,18 @@ __global__ __launch_bounds__(256, 2) void dense_gemm_kernel(const Q4Launch L, co
     const int r = lane & 31, h = lane >> 5;
     const int n_unit = in / 32;
     const int it0 = (int)((long)n_unit * ks / KS), it1 = (int)((long)n_unit * (ks + 1) / KS);
-    const int obase = rb * RB + wave * RW;
-    uint32_t wrow[MT], xoff[NB];
-#pragma unroll
-    for (int mt = 0; mt < MT; mt++) wrow[mt] = ((uint32_t)min(obase + mt * 32 + r, n_out - 1) * (uint32_t)in + 16 * h) * 4u;
+    const int obase = rb * RB + wave * 32;
+    const uint32_t wrow = ((uint32_t)min(obase + r, n_out - 1) * (uint32_t)in + 16 * h) * 4u;
+    uint32_t xoff[NB];
 #pragma unroll
     for (int p = 0; p < NB; p++) xoff[p] = ((uint32_t)min(t0 + p * 32 + (tid >> 3), B - 1) * (uint32_t)in_p + (tid & 7) * 4) * 4u;
     struct WStage {
-        float4 w[MT][4];
+        float4 w[4];
     };
     auto fetch_w = [&](int it, WStage &d) __attribute__((always_inline)) {
         const uint32_t c = (uint32_t)min(it, it1 - 1) * 128u;
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) d.w[mt][i] = ld_at<float4>(w, wrow[mt] + c + 16u * i);
+        for (int i = 0; i < 4; i++) d.w[i] = ld_at<float4>(w, wrow + c + 16u * i);
     };
     float4 xr[NB];
     auto fetch_x = [&](int it) __attribute__((always_inline)) {
@@ -449,13 +458,11 @@ __global__ __launch_bounds__(256, 2) void dense_gemm_kernel(const Q4Launch L, co
 #pragma unroll
         for (int p = 0; p < NB; p++) *reinterpret_cast<float4 *>(xs + (buf * TN + p * 32 + (tid >> 3)) * kRow + (tid & 7) * 4) = xr[p];
     };
-    f16v acc[MT][NB];
+    f16v run[NB], acc[NB];
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-        for (int nb = 0; nb < NB; nb++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) acc[mt][nb][i] = 0.f;
+    for (int nb = 0; nb < NB; nb++) run[nb] = acc[nb] = f16v{};
+    int run_steps = 2; // K steps per run
+    while (2 * run_steps * run_steps < it1 - it0) run_steps *= 2;
     WStage wr[2];
     fetch_x(it0);
     fetch_w(it0, wr[0]);
@@ -466,64 +473,83 @@ __global__ __launch_bounds__(256, 2) void dense_gemm_kernel(const Q4Launch L, co
         fetch_w(it + 1, wr[u ^ 1]);
         __builtin_amdgcn_sched_barrier(0); // requested before this step's arithmetic, not behind it
         const float *xb = xs + u * TN * kRow;
+        f16v even[NB]; // of four sums, pairs are added first
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            float4 b[NB];
+        for (int f = 0; f < FOLDS; f++) {
+            constexpr int N = 4 / FOLDS;
+            f16v sum[NB];
 #pragma unroll
-            for (int nb = 0; nb < NB; nb++) b[nb] = *reinterpret_cast<const float4 *>(xb + (nb * 32 + r) * kRow + 16 * h + 4 * i);
+            for (int i = f * N; i < (f + 1) * N; i++) {
+                float4 b[NB];
 #pragma unroll
-            for (int e = 0; e < 4; e++)
+                for (int nb = 0; nb < NB; nb++) b[nb] = *reinterpret_cast<const float4 *>(xb + (nb * 32 + r) * kRow + 16 * h + 4 * i);
 #pragma unroll
-                for (int mt = 0; mt < MT; mt++)
+                for (int e = 0; e < 4; e++)
 #pragma unroll
                     for (int nb = 0; nb < NB; nb++)
-                        acc[mt][nb] = __builtin_amdgcn_mfma_f32_32x32x2f32((&wr[u].w[mt][i].x)[e], (&b[nb].x)[e], acc[mt][nb], 0, 0, 0);
+                        sum[nb] = __builtin_amdgcn_mfma_f32_32x32x2f32((&wr[u].w[i].x)[e], (&b[nb].x)[e],
+                                                                       i == f * N && e == 0 ? f16v{} : sum[nb], 0, 0, 0);
+            }
+#pragma unroll
+            for (int nb = 0; nb < NB; nb++) {
+                if (FOLDS < 4) run[nb] += sum[nb];
+                else if (f & 1) run[nb] += even[nb] + sum[nb];
+                else even[nb] = sum[nb];
+            }
         }
         store_x(u ^ 1);
         __syncthreads();
     };
     int it = it0;
-    for (; it + 1 < it1; it += 2) {
+    for (int end = it0 + run_steps; it + 1 < it1; it += 2) {
         k_step(it, 0);
         k_step(it + 1, 1);
+        if (it + 2 == end) {
+            end += run_steps;
+#pragma unroll
+            for (int nb = 0; nb < NB; nb++) acc[nb] += run[nb], run[nb] = f16v{};
+        }
     }
     if (it < it1) k_step(it, 0);
+#pragma unroll
+    for (int nb = 0; nb < NB; nb++) acc[nb] += run[nb];
 
     size_t ws_base = 0;
     for (int i = 0; i < mi; i++) ws_base += (size_t)KS * B * L.m[i].out;
     float *tile = xs + wave * 32 * 36;
     const int tl = lane >> 3, oc = (lane & 7) * 4;
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++)
+    for (int nb = 0; nb < NB; nb++) {
 #pragma unroll
-        for (int nb = 0; nb < NB; nb++) {
+        for (int q = 0; q < 4; q++)
+            *reinterpret_cast<float4 *>(&tile[r * 36 + q * 8 + h * 4]) =
+                make_float4(acc[nb][4 * q], acc[nb][4 * q + 1], acc[nb][4 * q + 2], acc[nb][4 * q + 3]);
 #pragma unroll
-            for (int q = 0; q < 4; q++)
-                *reinterpret_cast<float4 *>(&tile[r * 36 + q * 8 + h * 4]) =
-                    make_float4(acc[mt][nb][4 * q], acc[mt][nb][4 * q + 1], acc[mt][nb][4 * q + 2], acc[mt][nb][4 * q + 3]);
-#pragma unroll
-            for (int pass = 0; pass < 4; pass++) {
-                const int tt = pass * 8 + tl;
-                float4 v = *reinterpret_cast<const float4 *>(&tile[tt * 36 + oc]);
-                const int t = t0 + nb * 32 + tt, o = obase + mt * 32 + oc;
-                if (t < B && o < n_out) finish4(L, mi, ss, ws + ws_base, KS, ks, partials, t, o, v);
-            }
+        for (int pass = 0; pass < 4; pass++) {
+            const int tt = pass * 8 + tl;
+            float4 v = *reinterpret_cast<const float4 *>(&tile[tt * 36 + oc]);
+            const int t = t0 + nb * 32 + tt, o = obase + oc;
+            if (t < B && o < n_out) finish4(L, mi, ss, ws + ws_base, KS, ks, partials, t, o, v);
         }
+    }
 }
 
 // ---- what follows a GEMM -----------------------------------------------------------------------------------------
 
-// Sum of the K slices of four consecutive outputs, in slice order; every load goes out before the first add.
+// Sum of the K slices of four consecutive outputs, as a tree; every load goes out before the first add.
 template <int N>
 __device__ __forceinline__ float4 sum_slices_n(const float *p, size_t slice, int KS) {
     float4 part[N];
 #pragma unroll
     for (int k = 0; k < N; k++) part[k] = *reinterpret_cast<const float4 *>(p + min(k, KS - 1) * slice);
-    float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-    for (int k = 0; k < N; k++)
-        if (k < KS) a.x += part[k].x, a.y += part[k].y, a.z += part[k].z, a.w += part[k].w;
-    return a;
+    for (int k = 1; k < N; k++)
+        if (k >= KS) part[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int d = 1; d < N; d *= 2)
+#pragma unroll
+        for (int k = 0; k < N; k += 2 * d) part[k].x += part[k + d].x, part[k].y += part[k + d].y, part[k].z += part[k + d].z, part[k].w += part[k + d].w;
+    return part[0];
 }
 __device__ __forceinline__ float4 sum_slices(const float *p, size_t slice, int KS) {
     if (KS <= 2) return sum_slices_n<2>(p, slice, KS);
@@ -635,7 +661,7 @@ __global__ __launch_bounds__(1024, TRIPS <= 2 && TRIPS * SL <= 8 ? 8 : 4) void g
     }
 }
 
-// What follows the q|k|v projection of a chunk: add the partial tiles of the three matrices in slice order, apply the
+// What follows the q|k|v projection of a chunk: add the partial tiles of the three matrices, apply the
 // token's rms scale, rotate q and k (src/models.rs:100-129: the second half of a head uses the first half's ROTATED
 // value), write q back and k and v into the cache rows of the tokens' positions (:236-249).  One block per token; a thread
 // takes four neighbouring pairs of a head, or four values of v.  Blocks of 512: at one slice the launch is bound by memory
@@ -760,9 +786,14 @@ int launch_dense(Q4Launch &L, const XhList &xh, const float *ss, float *ws, cons
     for (int i = 0; i < L.n_mats; i++) L.m[i].row_blocks = (L.m[i].out + s.rows - 1) / s.rows;
     const int t_tiles = (L.batch + s.tokens - 1) / s.tokens, in_p = gemm_padded(L.in);
     const dim3 grid(s.row_blocks * t_tiles * s.slices), block(256);
-    if (s.rows == 256 && s.tokens == 64) hipLaunchKernelGGL((dense_gemm_kernel<2, 2>), grid, block, 0, st, L, xh, in_p, ss, ws, s.slices, t_tiles, partials);
-    else if (s.tokens == 64) hipLaunchKernelGGL((dense_gemm_kernel<1, 2>), grid, block, 0, st, L, xh, in_p, ss, ws, s.slices, t_tiles, partials);
-    else hipLaunchKernelGGL((dense_gemm_kernel<1, 1>), grid, block, 0, st, L, xh, in_p, ss, ws, s.slices, t_tiles, partials);
+    auto launch = [&](void (*kernel)(Q4Launch, XhList, int, const float *, float *, int, int, int)) {
+        hipLaunchKernelGGL(kernel, grid, block, 0, st, L, xh, in_p, ss, ws, s.slices, t_tiles, partials);
+    };
+    // products summed from zero: 32; 16 and 8 where the matvec's chains are so short that it would be nearer to the exact sum
+    // (1024 inputs: 16s 1.01e-7 in eight slices and 1.09e-7 in one against its 1.00e-7)
+    if (L.in >= 2560) launch(s.tokens == 64 ? dense_gemm_kernel<2, 1> : dense_gemm_kernel<1, 1>);
+    else if (L.in >= 2048) launch(s.tokens == 64 ? dense_gemm_kernel<2, 2> : dense_gemm_kernel<1, 2>);
+    else launch(s.tokens == 64 ? dense_gemm_kernel<2, 4> : dense_gemm_kernel<1, 4>);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }
@@ -782,16 +813,19 @@ GemmShape gemm_shape(const Q4Launch &L, int slice_batch, int planes) {
     const int kstep = planes == kDensePlanes ? 32 : L.group_size > 64 ? L.group_size : 64, units = (gemm_padded(L.in) + kstep - 1) / kstep;
     auto slices = [&](int slots, int blocks, int most) { return std::max(1, std::min({slots / blocks, most, units / 2})); };
     // K slices: as many as keep the grid within one round of resident blocks.  Up to 32 columns the registers and the
-    // LDS hold four blocks per CU of 128 rows, and the partial tiles are small; beyond, two of 256 rows.
+    // LDS hold four blocks per CU of 128 rows, and the partial tiles are small; beyond, two of 256 rows (fp32 weights: three
+    // of 128).
     const int rows32 = row_blocks(L, 128), rows64 = row_blocks(L, 256);
     if (slice_batch <= 32)
         s.slices = slices(4 * cu_count(), rows32, kMaxGemmSlices);
+    else if (planes == kDensePlanes)
+        s.slices = slices(3 * cu_count(), rows32 * ((slice_batch + 63) / 64), 8);
     else
         s.slices = slices(2 * cu_count(), rows64 * ((slice_batch + 63) / 64), 8);
     s.tokens = B <= 32 ? 32 : 64;
     // 256 rows reuse every 16 bytes read from the LDS twice; 128 where the blocks would not fill the chip
     const int tiles = (B + s.tokens - 1) / s.tokens;
-    s.rows = s.tokens == 32 || rows64 * tiles * s.slices < 3 * cu_count() / 2 ? 128 : 256;
+    s.rows = planes == kDensePlanes || s.tokens == 32 || rows64 * tiles * s.slices < 3 * cu_count() / 2 ? 128 : 256;
     s.row_blocks = s.rows == 128 ? rows32 : rows64;
     return s;
 }

@@ -66,6 +66,30 @@ def test_fp32_prompt_vs_oracle(ops, oracle, kv, hidden, G, n):
     o.close()
 
 
+def rms_error(got, want):
+    return float(np.sqrt(np.mean(((got - want) / np.sqrt(np.mean(want ** 2, axis=1, keepdims=True))) ** 2)))
+
+
+# fp32 weights: a batch is no further from the exact sums than its columns one by one.  Rows on both sides of where the
+# products summed from zero change (2048, 2560), one K slice (512 columns of 11008 outputs) and eight.  The rms over N > 2e4 values of
+# similar size has a standard error of 1 / sqrt(2 N) < 0.5 %, the two of a ratio 0.7 %; three of those
+@pytest.mark.parametrize("dim,hidden", [(1024, 11008), (1920, 2528), (2048, 2816)])
+def test_dense_batch_error(ops, dim, hidden):
+    from llama2_rs import _lib
+    import tests.test_oracle_loop as tol
+    dims = ck.Dims(dim=dim, hidden_dim=hidden, n_layers=1, n_heads=dim // 128, n_kv_heads=1, vocab_size=64, seq_len=32, group_size=0)
+    img = ops.synth_image(dims, 4)
+    m, rng = ops.Model(img, dims), np.random.default_rng(dim)
+    for name, proj in (("w1", _lib.W1), ("w2", _lib.W2)):
+        W = tol._split_image(img, dims)[name][0].astype(np.float64)
+        for B in (33, 128, 512):
+            x = rng.standard_normal((B, W.shape[1])).astype(np.float32)
+            want = x.astype(np.float64) @ W.T
+            one = np.stack([m.qmatvec(0, proj, x[b]) for b in range(24)])
+            assert rms_error(m.qmatvec(0, proj, x), want) < 1.02 * rms_error(one, want[:24]), (name, B)
+    m.close()
+
+
 # fp16 prompts: the last tile of tokens in each of its widths, behind tiles of 128 tokens and of 64
 @pytest.mark.parametrize("G,batches", [(32, (65, 100)), (64, (65, 257, 300, 340, 370)), (128, (65, 272, 300, 340, 370))])
 def test_fp16_operator_last_tile(ops, G, batches):
