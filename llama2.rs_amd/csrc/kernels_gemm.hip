@@ -6,9 +6,17 @@
 //
 // fp32 activations, exactly: x = b0 + b1 + b2 with three bf16 numbers of 8 significant bits each, obtained by cutting x
 // after its first, second and third byte of significand.  The weights are integers n - z1 of at most five bits, exact in
-// bf16.  Every product that enters the fp32 accumulator (v_mfma_f32_32x32x16_bf16) is therefore exact, and what is left
-// is one rounding per addition, as in the vector-ALU matvec (kernels_q4_stream.hip), in another order.  The fp32 group
-// scale is applied to the fp32 partial sum of each group.
+// bf16, and so is every product that enters the fp32 accumulator (v_mfma_f32_32x32x16_bf16).  What is left is the sums:
+//   - The matrix unit's sum of 16 products and the accumulator is not rounded to nearest; it comes out too small on
+//     average, whatever its sign.  Left alone that adds up over K (28672 inputs in groups of 32: mean error -1.7e-7 of
+//     the result's rms).  So every other group enters negated, weights and scale: the mean is below 1e-9.
+//   - Of the three planes of a step the smallest is added first.
+//   - The fp32 group scale is applied to the fp32 sum of each group, and these are added in runs of at most kRunGroups,
+//     the runs to each other, the slices of K in a tree: the error of a chain grows with its length.
+// Relative rms error against fp64 over 1024..28672 inputs, 8..512 columns, normal inputs: 0.49 to 0.95 of that of the
+// matvec (kernels_q4_stream.hip) in every group size; inputs all of one sign, where the matvec is better than elsewhere,
+// 0.42 to 1.36 (the largest at 4096 inputs in groups of 32, 512 columns).  One chain, largest plane first, no negation:
+// 0.60 to 1.91 and 0.59 to 2.30.
 //
 // Against the matvec kernels run once per column, which read and dequantise the weights for each of them: 4096x11008,
 // group 32, 61 columns 330 -> 46 us with everything around it; a 299-token prompt on 7B 230 -> 22 ms.
@@ -37,15 +45,15 @@ __device__ __forceinline__ T ld_at(const void *base, uint32_t byte_offset) {
     return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + byte_offset);
 }
 
-// bf16: (n - z1) 2^-9 in the order (0,2,4,6,1,3,5,7).  A nibble in the low half of a byte is n 2^-9 as an OCP E4M3
+// bf16: sign (n - z1) 2^-9 in the order (0,2,4,6,1,3,5,7).  A nibble in the low half of a byte is n 2^-9 as an OCP E4M3
 // number; two at a time become fp32, the zero point is subtracted there, and the upper halves of two results are the
 // bf16 pair (the integers have at most five bits: nothing is cut off).
 struct Dequant {
-    float z;
+    float sign, z; // sign: 1 or -1
     static constexpr float kUnit = 0.001953125f; // 2^-9: value of the integer 1
-    __device__ __forceinline__ explicit Dequant(int zn) : z((float)(zn + 1) * kUnit) {}
+    __device__ __forceinline__ Dequant(int zn, float sg) : sign(sg), z((float)(zn + 1) * (-kUnit * sg)) {}
     __device__ __forceinline__ uint32_t pair(v2f v) const {
-        return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, v.y - z), __builtin_bit_cast(uint32_t, v.x - z), 0x07060302u);
+        return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, fmaf(v.y, sign, z)), __builtin_bit_cast(uint32_t, fmaf(v.x, sign, z)), 0x07060302u);
     }
     __device__ __forceinline__ Frag operator()(uint32_t w) const {
         const uint32_t l = w & 0x0F0F0F0Fu, h = (w >> 4) & 0x0F0F0F0Fu;
@@ -257,14 +265,15 @@ __global__ __launch_bounds__(256, 2) void q4_tile_gemm_kernel(const Q4Launch L, 
                 *reinterpret_cast<uint4 *>(xs + ((size_t)(buf * NP + q) * TN + (idx >> 3)) * kRowHalves + (idx & 7) * 8) = d.v[q * NB + p];
             }
     };
-    // scales of the group(s) that start with K step it, one row per thread
+    // scales of the group(s) that start with K step it, one row per thread; negative for the groups that enter negated
+    auto negated = [](int slot, int g) __attribute__((always_inline)) { return (G < 64 ? g : slot) != 0; };
     auto fetch_s = [&](int it, float (&d)[GPS]) __attribute__((always_inline)) {
 #pragma unroll
         for (int g = 0; g < GPS; g++) d[g] = ld_at<float>(qs, srow + ((uint32_t)min(it * GPS / KPG + g, groups - 1) << 2));
     };
     auto store_s = [&](int slot, const float (&d)[GPS]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int g = 0; g < GPS; g++) gsc[slot][g][tid & (RB - 1)] = d[g] * (1.0f / Dequant::kUnit);
+        for (int g = 0; g < GPS; g++) gsc[slot][g][tid & (RB - 1)] = d[g] * (negated(slot, g) ? -1.0f / Dequant::kUnit : 1.0f / Dequant::kUnit);
     };
 
     f16v acc[MT][NB], accg[MT][NB];
@@ -326,16 +335,16 @@ __global__ __launch_bounds__(256, 2) void q4_tile_gemm_kernel(const Q4Launch L, 
                 for (int nb = 0; nb < NB; nb++)
                     b[q][nb].q = *reinterpret_cast<const uint4 *>(xb + ((size_t)q * TN + nb * 32 + r) * kRowHalves + piece * 8);
 #pragma unroll
-            for (int mt = 0; mt < MT; mt++) a[mt] = Dequant(zw[mt][G >= 64 ? 0 : s >> 1])(wd[mt][s]);
+            for (int mt = 0; mt < MT; mt++) a[mt] = Dequant(zw[mt][G >= 64 ? 0 : s >> 1], negated(gpar, s >> 1) ? -1.0f : 1.0f)(wd[mt][s]);
             const bool zero = first && (G >= 64 ? s == 0 : (s & 1) == 0);
 #pragma unroll
-            for (int q = 0; q < NP; q++)
+            for (int q = NP - 1; q >= 0; q--)
 #pragma unroll
                 for (int mt = 0; mt < MT; mt++)
 #pragma unroll
                     for (int nb = 0; nb < NB; nb++)
-                        accg[mt][nb] = Dequant::mfma(a[mt], b[q][nb], zero && q == 0 ? f16v{} : accg[mt][nb]);
-            if (G >= 64 ? (last && s == 3) : (s & 1) == 1) { // a group ends: its partial sum, scaled, joins the result
+                        accg[mt][nb] = Dequant::mfma(a[mt], b[q][nb], zero && q == NP - 1 ? f16v{} : accg[mt][nb]);
+            if (G >= 64 ? (last && s == 3) : (s & 1) == 1) { // a group ends: its partial sum, scaled, joins the run
                 const float *sc = gsc[gpar][G >= 64 ? 0 : s >> 1] + wave * RW;
 #pragma unroll
                 for (int mt = 0; mt < MT; mt++)
@@ -356,20 +365,52 @@ __global__ __launch_bounds__(256, 2) void q4_tile_gemm_kernel(const Q4Launch L, 
         store_x(u ^ 1, xr);
         __syncthreads();
     };
+    size_t ws_base = 0;
+    for (int i = 0; i < mi; i++) ws_base += (size_t)KS * B * L.m[i].out;
+    // Runs that have ended: their sum lies where the result goes, every lane's own elements.  (There are no registers for a
+    // third set of tiles.  What it costs is this traffic: 4096 -> 22016 outputs, 512 columns, group 32, 45 MB a time; a layer
+    // of 7B, 512 tokens, 0.88 -> 0.93 ms with runs of 64 groups, 0.98 with 32; 299 tokens, group 128 has one run.)
+    float *__restrict__ const sums = KS > 1 || partials ? ws + ws_base + (size_t)ks * B * n_out : L.m[mi].y;
+    auto each_sum = [&](auto &&f) __attribute__((always_inline)) {
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+            for (int nb = 0; nb < NB; nb++)
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const int t = t0 + nb * 32 + r, o = obase + mt * 32 + k * 8 + h * 4;
+                    if (t < B && o < n_out) f(*reinterpret_cast<float4_any *>(sums + (size_t)t * n_out + o), acc[mt][nb], 4 * k);
+                }
+    };
     const int n_it = it1 - it0;
     const int n_full = n_it / PW * PW;
-    for (int i = 0; i < n_full; i += PW) {
+    constexpr int kRunGroups = 64, kRunSteps = kRunGroups * KPG / GPS;
+    const int runs = (n_it + kRunSteps - 1) / kRunSteps, run_len = (n_it / runs + PW) / PW * PW;
+    int i = 0;
+    for (;;) { // whole rounds of PW steps, run by run
+        for (const int end = min(i + run_len, n_full); i < end; i += PW) {
 #pragma unroll
-        for (int u = 0; u < PW; u++) k_step(it0 + i + u, u);
+            for (int u = 0; u < PW; u++) k_step(it0 + i + u, u);
+        }
+        if (i >= n_full) break;
+        each_sum([&](float4_any &at, f16v &v, int k) __attribute__((always_inline)) {
+            float4_any c{v[k], v[k + 1], v[k + 2], v[k + 3]};
+            if (i > run_len) c += at;
+            at = c;
+            v[k] = v[k + 1] = v[k + 2] = v[k + 3] = 0.f;
+        });
     }
 #pragma unroll
     for (int u = 0; u < PW - 1; u++) // the rest straight-line: a loop left half-way copies ring registers, and waits
         if (n_full + u < n_it) k_step(it0 + n_full + u, u);
+    if (n_full > run_len)
+        each_sum([&](float4_any &at, f16v &v, int k) __attribute__((always_inline)) {
+            const float4_any c = at;
+            v[k] += c.x, v[k + 1] += c.y, v[k + 2] += c.z, v[k + 3] += c.w;
+        });
 
     // C layout: lane (column r = token, h), register i -> row (i / 4) * 8 + h * 4 + i % 4.  Turned through LDS (the
     // activation buffers are free now) so that a store writes 128 contiguous bytes per token.
-    size_t ws_base = 0;
-    for (int i = 0; i < mi; i++) ws_base += (size_t)KS * B * L.m[i].out;
     constexpr int kTRow = 36;
     float *tile = reinterpret_cast<float *>(xs) + wave * 32 * kTRow;
     const int tl = lane >> 3, oc = (lane & 7) * 4;
@@ -842,19 +883,21 @@ int gemm_launch(Q4Launch &L, const XhList &xh, const float *ss, float *ws, size_
         rows += L.m[i].out;
     }
     const GemmShape s = gemm_shape(L, slice_batch, planes);
-    if ((s.slices > 1 || ks_out) && (size_t)s.slices * L.batch * rows > ws_floats)
+    // the fp32 kernel keeps its runs' sums where the result goes, which is where the residual lies
+    const bool partials = ks_out || (planes == 3 && L.e.kind == Q4_EPI_RESIDUAL);
+    if ((s.slices > 1 || partials) && (size_t)s.slices * L.batch * rows > ws_floats)
         return l2_fail(L2_ERR_ARG, "q4 gemm: %d slices of %d x %ld in a workspace of %zu", s.slices, L.batch, rows, ws_floats);
     if (planes == 1)
-        L2_TRY(gemm_launch_f16(L, xh, ss, ws, s, ks_out != nullptr, st));
+        L2_TRY(gemm_launch_f16(L, xh, ss, ws, s, partials, st));
     else if (planes == kDensePlanes)
-        L2_TRY(launch_dense(L, xh, ss, ws, s, ks_out != nullptr, st));
+        L2_TRY(launch_dense(L, xh, ss, ws, s, partials, st));
     else
-        L2_TRY(launch_fp32(L, xh, ss, ws, s, ks_out != nullptr, st));
+        L2_TRY(launch_fp32(L, xh, ss, ws, s, partials, st));
     if (ks_out) {
         *ks_out = s.slices;
         return L2_OK;
     }
-    if (s.slices > 1) {
+    if (s.slices > 1 || partials) {
         hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)((rows + 1023) / 1024), L.batch), dim3(256), 0, st, L, ss, ws, s.slices);
         L2_HIP(hipGetLastError());
     }

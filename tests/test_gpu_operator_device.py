@@ -39,9 +39,9 @@ def test_result_over_the_input(ops, n_in, n_out, G, B):
 
 
 # x and y at addresses that are multiples of four bytes and of nothing more, and nothing written beside y: one column, a
-# few, and batches in one K slice (17160 outputs) and in several
+# few, and batches in one K slice (17160 outputs; 4128 inputs: in several runs of groups) and in several
 @pytest.mark.parametrize("n_in,n_out,G,batches", [(1024, 264, 32, (1, 3, 250)), (4096, 4104, 128, (1, 3, 5, 40, 250)),
-                                                  (8192, 8192, 64, (1, 2, 100)), (1024, 17160, 32, (250,))])
+                                                  (8192, 8192, 64, (1, 2, 100)), (1024, 17160, 32, (250,)), (4128, 17160, 32, (250,))])
 def test_any_float_address(ops, n_in, n_out, G, batches):
     hip = _Hip()
     rng = np.random.default_rng(n_in)
