@@ -44,8 +44,11 @@ enum { L2_WQ = 0, L2_WK = 1, L2_WV = 2, L2_WO = 3, L2_W1 = 4, L2_W2 = 5, L2_W3 =
 enum {
     L2_PREFILL_FP32 = 0, /* fp32 throughout: a few columns are the bits of B=1; larger batches run on the
                           * matrix cores with every product exact and fp32 accumulation, so they differ
-                          * from B=1 by the order of the additions only (1e-6)                       */
-    L2_PREFILL_MFMA = 1  /* dequant -> fp16 tiles -> MFMA, fp32 accumulate (tolerance 2e-3)    */
+                          * from B=1 by the rounding of the additions only (1e-6)                    */
+    L2_PREFILL_MFMA = 1, /* dequant -> fp16 tiles -> MFMA, fp32 accumulate (tolerance 2e-3)    */
+    L2_PREFILL_COLUMNS = 2 /* fp32 throughout, and every column of a projection is the bits of B=1
+                            * whatever the batch, as L2_PREFILL_FP32 has for a few columns: the
+                            * weights are read once per column                                  */
 };
 
 /* Run-time form of the reference's compile-time constants
@@ -152,6 +155,10 @@ void l2_qlinear_free(l2_qlinear *q);
  * overwritten, synchronous.  fp32 throughout (the CUDA path's fp16 rounding of
  * x and y is not reproduced; the CPU path is the parity target). */
 int l2_qlinear_matvec(l2_qlinear *q, const float *x_host, int B, float *y_host);
+
+/* L2_PREFILL_FP32 (the default) or L2_PREFILL_COLUMNS: how both entry points of this layer's operator treat
+ * B > 1. */
+int l2_qlinear_set_mode(l2_qlinear *q, int mode);
 
 /* The same operator for callers that cannot allocate device memory (code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  x_dev f32[B][in] and

@@ -428,6 +428,7 @@ struct l2_qlinear {
     hipStream_t stream = nullptr;
     float *x = nullptr, *xg = nullptr, *y = nullptr;
     int cap_B = 0;
+    int mode = L2_PREFILL_FP32;
     OperatorBufs batch;
 };
 
@@ -812,7 +813,7 @@ extern "C" int l2_model_set_step_graph(l2_model *m, int on) {
 
 extern "C" int l2_model_set_prefill_mode(l2_model *m, int mode) {
     if (!m) return l2_fail(L2_ERR_ARG, "null model");
-    if (mode != L2_PREFILL_FP32 && mode != L2_PREFILL_MFMA) return l2_fail(L2_ERR_ARG, "prefill mode %d", mode);
+    if (mode != L2_PREFILL_FP32 && mode != L2_PREFILL_MFMA && mode != L2_PREFILL_COLUMNS) return l2_fail(L2_ERR_ARG, "prefill mode %d", mode);
     if (mode == L2_PREFILL_MFMA && m->d.group_size == 0)
         return l2_fail(L2_ERR_ARG, "the MFMA prefill path is the quantised model's");
     const int G = m->d.group_size;
@@ -842,7 +843,7 @@ static bool gemm_pays_layer(int B, double weights) { return B >= 8 && B * weight
 // What a batch of B columns of this model is computed with: 0 = the matvec kernels column by column, 1 or 3 = the GEMM
 // with that many planes of activations.
 static int batch_planes(const l2_model *m, int B) {
-    if (B < 2 || m->d.dim > kGemmMaxDim || m->d.hidden_dim > kGemmMaxHidden) return 0;
+    if (B < 2 || m->prefill_mode == L2_PREFILL_COLUMNS || m->d.dim > kGemmMaxDim || m->d.hidden_dim > kGemmMaxHidden) return 0;
     if (m->prefill_mode == L2_PREFILL_MFMA) return 1; // quantised models only
     const double dim = m->d.dim, weights = dim * (2 * dim + 2.0 * m->kv_dim + 3.0 * m->d.hidden_dim);
     if (!gemm_pays_layer(B, weights)) return 0;
@@ -850,7 +851,9 @@ static int batch_planes(const l2_model *m, int B) {
 }
 
 // The same for the stand-alone operator.
-static int operator_planes(const DevQLinear &q, int B) { return gemm_pays(B, (double)q.in * q.out) ? 3 : 0; }
+static int operator_planes(const DevQLinear &q, int B, int mode) {
+    return mode != L2_PREFILL_COLUMNS && gemm_pays(B, (double)q.in * q.out) ? 3 : 0;
+}
 
 // Nothing may be running on either of the model's streams when a buffer they use is freed.
 static int drain_streams(l2_model *m) {
@@ -1181,6 +1184,13 @@ extern "C" void l2_qlinear_free(l2_qlinear *q) {
     host_slots.drop_user();
 }
 
+extern "C" int l2_qlinear_set_mode(l2_qlinear *q, int mode) {
+    if (!q) return l2_fail(L2_ERR_ARG, "null qlinear");
+    if (mode != L2_PREFILL_FP32 && mode != L2_PREFILL_COLUMNS) return l2_fail(L2_ERR_ARG, "operator mode %d", mode);
+    q->mode = mode;
+    return L2_OK;
+}
+
 static int qlinear_scratch(l2_qlinear *q, int B) {
     if (B <= q->cap_B) return L2_OK;
     dfree(q->x);
@@ -1242,7 +1252,7 @@ extern "C" int l2_qlinear_matvec(l2_qlinear *q, const float *x_host, int B, floa
     if (!q || !x_host || !y_host) return l2_fail(L2_ERR_ARG, "null argument");
     if (B < 1 || B > 4096) return l2_fail(L2_ERR_RANGE, "batch %d (1..4096)", B);
     L2_TRY(qlinear_scratch(q, B));
-    return matvec_host(q->q, q->x, q->xg, q->y, q->batch, operator_planes(q->q, B), x_host, B, y_host, q->stream);
+    return matvec_host(q->q, q->x, q->xg, q->y, q->batch, operator_planes(q->q, B, q->mode), x_host, B, y_host, q->stream);
 }
 
 // ---- the same operator for callers that cannot allocate ---------------------------------------------
@@ -1290,7 +1300,7 @@ extern "C" int l2_qlinear_matvec_device(l2_qlinear *q, const float *x_dev, int B
     hipStream_t st = (hipStream_t)hip_stream;
     // Every element of the scratch that is read has been written before by the same call: nothing of the
     // previous call's contents is read, so nothing needs clearing.
-    if (operator_planes(q->q, B))
+    if (operator_planes(q->q, B, q->mode))
         return gemm_operator(q->q, x_dev, B, y_dev, 3, fixed.planes, fixed.ws, kOperatorWsFloats, st);
     // One column: the kernel applies the permutation while it stages x (one launch where the host's launch rate is what
     // counts: 9.7 -> 6.6 us per call at 8192x1024).  Its blocks read all of x while others write y already, so where y lies
@@ -1325,7 +1335,7 @@ extern "C" int l2_model_qmatvec(l2_model *m, int layer, int proj, const float *x
     if (q.dense) { // Linear::matvec<B> (src/model.rs:22-31)
         hipStream_t st = m->stream;
         L2_HIP(hipMemcpyAsync(m->op_x, x_host, (size_t)B * q.in * 4, hipMemcpyHostToDevice, st));
-        if (operator_planes(q, B) && q.in == gemm_padded(q.in)) {
+        if (operator_planes(q, B, m->prefill_mode) && q.in == gemm_padded(q.in)) {
             L2_TRY(operator_bufs(m->op_batch, q, B, kDensePlanes, st));
             Q4Launch L = launch_of(q, B, 0.f);
             L.m[0] = mat_of(q, nullptr, nullptr, m->op_y);
@@ -1339,7 +1349,7 @@ extern "C" int l2_model_qmatvec(l2_model *m, int layer, int proj, const float *x
         L2_HIP(hipStreamSynchronize(st));
         return L2_OK;
     }
-    const int planes = m->prefill_mode == L2_PREFILL_FP32 ? operator_planes(q, B) : batch_planes(m, B);
+    const int planes = m->prefill_mode == L2_PREFILL_MFMA ? batch_planes(m, B) : operator_planes(q, B, m->prefill_mode);
     return matvec_host(q, m->op_x, m->op_xg, m->op_y, m->op_batch, planes, x_host, B, y_host, m->stream);
 }
 

@@ -17,7 +17,7 @@ L2_OK = 0
 ERR_NAMES = {-1: "L2_ERR_ARG", -2: "L2_ERR_IO", -3: "L2_ERR_FORMAT", -4: "L2_ERR_HIP", -5: "L2_ERR_RANGE"}
 
 WQ, WK, WV, WO, W1, W2, W3 = range(7)
-PREFILL_FP32, PREFILL_MFMA = 0, 1
+PREFILL_FP32, PREFILL_MFMA, PREFILL_COLUMNS = 0, 1, 2
 
 
 class L2Error(RuntimeError):
@@ -65,6 +65,7 @@ SIGNATURES = {
     "l2_state_fill_synthetic": (_I, [_VP, _I, _I, C.c_uint64]),
     "l2_qlinear_create": (_I, [_VP, _VP, _VP, _VP, _I, _I, _I, C.POINTER(_VP)]),
     "l2_qlinear_free": (None, [_VP]),
+    "l2_qlinear_set_mode": (_I, [_VP, _I]),
     "l2_qlinear_matvec": (_I, [_VP, _VP, _I, _VP]),
     "l2_qlinear_matvec_device": (_I, [_VP, _VP, _I, _VP, _VP]),
     "l2_model_q4_kernels": (_I, [_VP, C.c_char_p, _SZ]),

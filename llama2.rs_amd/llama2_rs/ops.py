@@ -75,6 +75,10 @@ class QLinear:
         check(lib().l2_qlinear_create(_p(qweight), _p(qzeros), _p(scales), _p(g_index), self.n_in,
                                       self.n_out, group_size, C.byref(self.h)))
 
+    def set_mode(self, mode: int):
+        """_lib.PREFILL_FP32 (default) or _lib.PREFILL_COLUMNS (every column of a batch the bits of a single one)."""
+        check(lib().l2_qlinear_set_mode(self.h, mode))
+
     def matvec(self, x) -> np.ndarray:
         """x [IN] or [B][IN] -> y [OUT] or [B][OUT]  (QLinear::matvec<B>)."""
         x = _f32(x)
@@ -165,7 +169,8 @@ class Model:
         check(lib().l2_state_reset(self.state))
 
     def set_prefill_mode(self, mode: int):
-        """_lib.PREFILL_FP32 (default, fp32 throughout) or _lib.PREFILL_MFMA (fp16 tiles, 2e-3)."""
+        """_lib.PREFILL_FP32 (default, fp32 throughout), _lib.PREFILL_MFMA (fp16 tiles, 2e-3) or _lib.PREFILL_COLUMNS
+        (fp32, every column of a projection the bits of a single one)."""
         check(lib().l2_model_set_prefill_mode(self.h, mode))
 
     def set_step_graph(self, on: bool):

@@ -65,6 +65,7 @@ int main(int argc, char **argv) {
     REQUIRE(l2_qlinear_matvec(nullptr, &f, 1, &f) != L2_OK);
     REQUIRE(l2_qlinear_matvec_device(nullptr, &f, 1, &f, nullptr) != L2_OK);
     REQUIRE(l2_model_set_prefill_mode(nullptr, 0) != L2_OK);
+    REQUIRE(l2_qlinear_set_mode(nullptr, 0) != L2_OK);
     REQUIRE(l2_model_max_seq(nullptr) == 0);
     l2_model_close(nullptr);
     l2_state_free(nullptr);

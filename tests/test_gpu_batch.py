@@ -111,6 +111,45 @@ def test_batch_error(ops, n_in, n_out, G):
     q.close()
 
 
+# batches that must be the bits of their columns: the operator by both entry points, a projection of a model (quantised
+# and not), and the rows that a prompt's first layer leaves, at sizes the default mode gives to the matrix cores
+def test_columns_mode(ops):
+    from llama2_rs import _lib
+    from tests.test_zz_no_alloc import _Hip
+    rng = np.random.default_rng(8)
+    q = ops.QLinear(*ck.synth_qlinear(rng, 4096, 1160, 32, act_order=True), 32)
+    x = rng.standard_normal((61, 4096)).astype(np.float32)
+    one = np.stack([q.matvec(c) for c in x])
+    assert not np.array_equal(q.matvec(x), one)
+    q.set_mode(_lib.PREFILL_COLUMNS)
+    np.testing.assert_array_equal(q.matvec(x), one)
+    hip = _Hip()
+    dx, dy = hip.upload(x), hip.empty(one.nbytes)
+    q.matvec_device(dx, 61, dy)
+    np.testing.assert_array_equal(hip.download(dy, one.shape), one)
+    with pytest.raises(_lib.L2Error):
+        q.set_mode(_lib.PREFILL_MFMA)
+    q.set_mode(_lib.PREFILL_FP32)
+    assert not np.array_equal(q.matvec(x), one)
+    q.close()
+    hip.close()
+    for G in (64, 0):
+        dims = ck.Dims(dim=1024, hidden_dim=2816, n_layers=1, n_heads=8, n_kv_heads=2, vocab_size=300, seq_len=128, group_size=G)
+        m = ops.Model(ck.synth_weights_image(dims, seed=5), dims)
+        x = rng.standard_normal((100, 1024)).astype(np.float32)
+        toks = rng.integers(0, 300, size=100).astype(np.int32)
+        for t in range(100):
+            m.forward([int(toks[t])], [t], want_logits=False)
+        rows, one = m.read_kv(0, 0, 100), np.stack([m.qmatvec(0, _lib.W1, c) for c in x])
+        for mode in (_lib.PREFILL_FP32, _lib.PREFILL_COLUMNS):
+            m.reset()
+            m.set_prefill_mode(mode)
+            m.prefill_chunks(toks, 0, 100)
+            same = [np.array_equal(a, b) for a, b in zip(m.read_kv(0, 0, 100), rows)] + [np.array_equal(m.qmatvec(0, _lib.W1, x), one)]
+            assert same == [mode == _lib.PREFILL_COLUMNS] * 3, (G, mode)
+        m.close()
+
+
 # fp16 prompts: the last tile of tokens in each of its widths, behind tiles of 128 tokens and of 64
 @pytest.mark.parametrize("G,batches", [(32, (65, 100)), (64, (65, 257, 300, 340, 370)), (128, (65, 272, 300, 340, 370))])
 def test_fp16_operator_last_tile(ops, G, batches):
