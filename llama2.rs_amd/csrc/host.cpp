@@ -311,12 +311,10 @@ struct l2_model {
     // Running maxima (value, index) of the classifier: step n of a loop folds into slot n % 2, so that the embedding
     // kernel of step n + 1 can read one slot while it clears the other.
     unsigned long long *amax = nullptr;
-    // Pinned host memory that kernels read and write directly: a completion flag, logits, token ids, ids and positions
-    // on their way in.  The calls on one model are serialised and each waits for its work, so it is free between calls.
+    // Pinned host memory that kernels read and write directly: logits, token ids, ids and positions on their way in.  The
+    // calls on one model are serialised and each waits for its work, so it is free between calls.
     struct HostStage {
         char *base = nullptr;
-        volatile uint32_t *flag = nullptr;
-        uint32_t seq = 0;
         float *logits = nullptr;               // [vocab]: logits, or the sampler's weights
         unsigned long long *redo = nullptr;    // one bit per vocabulary entry
         int32_t *ids = nullptr, *in = nullptr; // [max_seq] out; [2 * max(max_seq, 4096)] in
@@ -469,8 +467,6 @@ static void dfree(void *p) {
 struct HostSlot {
     static constexpr size_t kBytes = (size_t)1 << 20; // each of x and y
     char *base = nullptr;
-    volatile uint32_t *flag = nullptr;
-    uint32_t seq = 0;
     float *x = nullptr, *y = nullptr;
 };
 static struct HostSlots {
@@ -498,11 +494,9 @@ static struct HostSlots {
             }
         }
         void *p = nullptr;
-        L2_HIP(hipHostMalloc(&p, 2 * HostSlot::kBytes + 256, hipHostMallocCoherent | hipHostMallocPortable));
+        L2_HIP(hipHostMalloc(&p, 2 * HostSlot::kBytes, hipHostMallocCoherent | hipHostMallocPortable));
         out->base = (char *)p;
         out->x = (float *)p, out->y = (float *)(out->base + HostSlot::kBytes);
-        out->flag = (volatile uint32_t *)(out->base + 2 * HostSlot::kBytes);
-        *out->flag = 0;
         return L2_OK;
     }
     void give(const HostSlot &s) {
@@ -695,15 +689,13 @@ static int model_build(const char *weights, size_t nbytes, const l2_dims *dims, 
     }
     M_TRY(dalloc(&m->amax, 2));
     {
-        const size_t logits = 256, redo = logits + ((size_t)dims->vocab_size * 4 + 255) / 256 * 256,
+        const size_t redo = ((size_t)dims->vocab_size * 4 + 255) / 256 * 256,
                      ids = redo + ((size_t)dims->vocab_size / 64 + 32) / 32 * 256,
                      in = ids + ((size_t)max_seq * 4 + 255) / 256 * 256, end = in + (size_t)std::max(max_seq, 4096) * 8;
         void *p = nullptr;
         M_HIP(hipHostMalloc(&p, end, hipHostMallocCoherent));
         m->hs.base = (char *)p;
-        m->hs.flag = (volatile uint32_t *)m->hs.base;
-        *m->hs.flag = 0;
-        m->hs.logits = (float *)(m->hs.base + logits);
+        m->hs.logits = (float *)m->hs.base;
         m->hs.redo = (unsigned long long *)(m->hs.base + redo);
         m->hs.ids = (int32_t *)(m->hs.base + ids);
         m->hs.in = (int32_t *)(m->hs.base + in);
@@ -840,13 +832,16 @@ static bool gemm_pays(int B, double weights) { return B >= 4 && B * weights >= 6
 // 32 394 against 270, 48 514 against 300.
 static bool gemm_pays_layer(int B, double weights) { return B >= 8 && B * weights >= 1.4e8; }
 
+static double layer_weights(const l2_model *m) {
+    return (double)m->d.dim * (2.0 * m->d.dim + 2.0 * m->kv_dim + 3.0 * m->d.hidden_dim);
+}
+
 // What a batch of B columns of this model is computed with: 0 = the matvec kernels column by column, 1 or 3 = the GEMM
 // with that many planes of activations.
 static int batch_planes(const l2_model *m, int B) {
     if (B < 2 || m->prefill_mode == L2_PREFILL_COLUMNS || m->d.dim > kGemmMaxDim || m->d.hidden_dim > kGemmMaxHidden) return 0;
     if (m->prefill_mode == L2_PREFILL_MFMA) return 1; // quantised models only
-    const double dim = m->d.dim, weights = dim * (2 * dim + 2.0 * m->kv_dim + 3.0 * m->d.hidden_dim);
-    if (!gemm_pays_layer(B, weights)) return 0;
+    if (!gemm_pays_layer(B, layer_weights(m))) return 0;
     return m->d.group_size == 0 ? kDensePlanes : 3;
 }
 
@@ -1214,8 +1209,8 @@ static int operator_enqueue(const DevQLinear &q, const float *dx, float *dxg, fl
 }
 
 // x (host, natural order) -> gather through g_index -> matvec -> y (host).  Through a slot of pinned memory where x and y
-// fit one: x is fetched from there, the last kernel writes y there, and the host watches for the end of the call.  One
-// 4096x4096 matvec 31.6 -> 17 us (pageable copies either way and hipStreamSynchronize before).
+// fit one: x is fetched from there and the last kernel writes y there.  One 4096x4096 matvec 28-40 -> 19.6 us (pageable
+// copies either way before).
 static int matvec_host(const DevQLinear &q, float *dx, float *dxg, float *dy, OperatorBufs &bufs, int planes,
                        const float *x_host, int B, float *y_host, hipStream_t st) {
     if (planes) L2_TRY(operator_bufs(bufs, q, B, planes, st));
@@ -1235,14 +1230,11 @@ static int matvec_host(const DevQLinear &q, float *dx, float *dxg, float *dy, Op
             L2_TRY(copy_launch(dx, slot.x, xb / 4, st));
         else
             L2_HIP(hipMemcpyAsync(dx, slot.x, xb, hipMemcpyHostToDevice, st));
-        L2_TRY(operator_enqueue(q, dx, dxg, slot.y, bufs, planes, B, st));
-        return finish_launch(nullptr, nullptr, const_cast<uint32_t *>(slot.flag), ++slot.seq, st);
+        return operator_enqueue(q, dx, dxg, slot.y, bufs, planes, B, st);
     };
     int rc = call();
-    if (rc != L2_OK || !watch_flag(slot.flag, slot.seq)) {
-        const hipError_t e = hipStreamSynchronize(st);
-        if (rc == L2_OK && e != hipSuccess) rc = l2_fail(L2_ERR_HIP, "matvec: %s", hipGetErrorString(e));
-    }
+    const hipError_t e = hipStreamSynchronize(st);
+    if (rc == L2_OK && e != hipSuccess) rc = l2_fail(L2_ERR_HIP, "matvec: %s", hipGetErrorString(e));
     if (rc == L2_OK) memcpy(y_host, slot.y, yb);
     host_slots.give(slot);
     return rc;
@@ -1410,14 +1402,12 @@ static int check_position(const l2_model *m, int max_pos) {
     return L2_OK;
 }
 
-// Waits for everything on the model's stream: a last, tiny kernel stores the call's number in pinned host memory
-// (and, with `amax`, the index of that running maximum in *id), and the host watches it there.  hipStreamSynchronize
-// takes 4.5 us longer to notice the same; it is the way out where the number does not come (a failed launch), and
-// reports why.
+// Waits for everything on the model's stream; with `amax`, the index of that running maximum is in *id (pinned host
+// memory) then.  (A number that a last kernel stores in pinned memory is seen 4 to 13 us earlier than a synchronisation
+// returns, but what the runtime does at one is then left for the next call: l2_state_reset behind a pass 13 -> 44 us.)
 static int wait_host(l2_model *m, const unsigned long long *amax, int32_t *id) {
-    const uint32_t seq = ++m->hs.seq;
-    L2_TRY(finish_launch(amax, id, const_cast<uint32_t *>(m->hs.flag), seq, m->stream));
-    if (!watch_flag(m->hs.flag, seq)) L2_HIP(hipStreamSynchronize(m->stream));
+    if (amax) L2_TRY(index_launch(amax, id, m->stream));
+    L2_HIP(hipStreamSynchronize(m->stream));
     m->hs.reading = false;
     return L2_OK;
 }
@@ -2015,6 +2005,8 @@ static int step_bucket(const l2_model *m, int pos) {
 // Launched: the embedding kernel of a step takes the step before's argmax itself and records it (in pinned host memory),
 // so a step is its layers' launches, one in front and the classifier.  Forced tokens travel as kernel arguments.
 // As graphs: see step_graph_get.
+static constexpr int kAskLaunches = 128;
+static constexpr double kAskWeights = 5e7; // a layer of 7B has 2e8 and takes 40 us
 static int steps_enqueue(l2_model *m, l2_state *s, int32_t first, int pos0, int n, const int32_t *prompt, int n_prompt) {
     if (m->use_graph && !m->prof_on) {
         L2_TRY(ensure_loop_buffers(m, std::max(n_prompt, 1), std::max(n, 1)));
@@ -2034,12 +2026,19 @@ static int steps_enqueue(l2_model *m, l2_state *s, int32_t first, int pos0, int 
         }
         return L2_OK;
     }
+    // The runtime keeps a record of every launch until it is asked about the stream or has a thousand of them, and a loop of
+    // so many launches behind a synchronisation is slow to enqueue in most processes (three layers of 1024 inputs, 48 steps:
+    // 2.1 or 3.2 ms, 4.0 or 4.5 ms in all; 167 steps 14.0 or 14.5).  Asked about in between, the loop takes 4.04 and 14.1 ms in
+    // every process.  That pays where a launch is too short to hide the enqueueing (an ask costs the GPU 5 us); not shortly
+    // before the end, where the wait would meet it.
+    const int ask_steps = layer_weights(m) < kAskWeights ? std::max(1, kAskLaunches / (5 * m->d.n_layers + 2)) : n;
     ForwardIn in;
     in.src.token = first, in.logits = m->logits;
     for (int i = 0; i < n; i++) {
         const int pos = pos0 + i;
         in.amax = m->amax + (i & 1);
         L2_TRY(forward_enqueue(m, s, 1, pos, in));
+        if ((i + 1) % ask_steps == 0 && i + ask_steps < n && hipStreamQuery(m->stream) == hipErrorNotReady) (void)hipGetLastError();
         in.src = TokenSource{};
         if (pos < n_prompt)
             in.src.token = prompt[pos];

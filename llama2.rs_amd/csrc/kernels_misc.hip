@@ -10,8 +10,6 @@
 // element i of its result to slot inv[i] of the buffer the next QLinear reads,
 // which is that layer's x[g_index[j]] gather (src/gptq.rs:110-114) done once
 // at the source instead of once per consumer block.
-#include <chrono>
-
 #include "l2_internal.h"
 
 namespace {
@@ -322,12 +320,8 @@ __global__ __launch_bounds__(256) void sample_weights_kernel(float *w, unsigned 
     if ((threadIdx.x & 63) == 0 && i < n) redo[i >> 6] = mask;
 }
 
-__global__ void finish_kernel(const unsigned long long *amax, int32_t *id, uint32_t *flag, uint32_t seq) {
-    if (threadIdx.x == 0) {
-        if (amax) id[0] = (int32_t)(amax[0] & 0xFFFFFFFFull);
-        __threadfence_system(); // what the call left in host memory is there before the number is
-        *reinterpret_cast<volatile uint32_t *>(flag) = seq;
-    }
+__global__ void index_kernel(const unsigned long long *amax, int32_t *id) {
+    if (threadIdx.x == 0) id[0] = (int32_t)(amax[0] & 0xFFFFFFFFull);
 }
 
 __global__ void copy_kernel(float4 *dst, const float4 *src, int n4) {
@@ -375,24 +369,10 @@ int sample_weights_launch(float *w, unsigned long long *redo, const float *logit
     return L2_OK;
 }
 
-int finish_launch(const unsigned long long *amax, int32_t *id, uint32_t *flag, uint32_t seq, hipStream_t st) {
-    hipLaunchKernelGGL(finish_kernel, dim3(1), dim3(64), 0, st, amax, id, flag, seq);
+int index_launch(const unsigned long long *amax, int32_t *id, hipStream_t st) {
+    hipLaunchKernelGGL(index_kernel, dim3(1), dim3(64), 0, st, amax, id);
     L2_HIP(hipGetLastError());
     return L2_OK;
-}
-
-bool watch_flag(volatile uint32_t *flag, uint32_t seq) {
-    const auto give_up = std::chrono::steady_clock::now() + std::chrono::seconds(2);
-    for (;;) {
-        for (int i = 0; i < 1024; i++) {
-            if (*flag == seq) {
-                std::atomic_thread_fence(std::memory_order_acquire);
-                return true;
-            }
-            __builtin_ia32_pause();
-        }
-        if (std::chrono::steady_clock::now() > give_up) return false;
-    }
 }
 
 int copy_launch(float *dst, const float *src, size_t n, hipStream_t st) {

@@ -286,10 +286,8 @@ int embed_launch(float *x, const float *emb, const TokenSource &src, int dim, in
 // two floats that another faithful expf may round it the other way, w[i] = d_i and bit i of `redo` is set.
 int sample_weights_launch(float *w, unsigned long long *redo, const float *logits, int n, float temperature,
                           const unsigned long long *amax, hipStream_t st);
-// The end of a call's work: with amax, *id = its index; then *flag = seq (both in pinned host memory).
-int finish_launch(const unsigned long long *amax, int32_t *id, uint32_t *flag, uint32_t seq, hipStream_t st);
-// The host's side: true once *flag is seq; false if that takes so long that something may be wrong.
-bool watch_flag(volatile uint32_t *flag, uint32_t seq);
+// *id = the index of the running maximum.
+int index_launch(const unsigned long long *amax, int32_t *id, hipStream_t st);
 // dst = src, n floats; for small pieces of pinned host memory.
 int copy_launch(float *dst, const float *src, size_t n, hipStream_t st);
 // k and v: the first n floats (a multiple of 4) of each of `layers` stretches of `stride` floats become zero.
