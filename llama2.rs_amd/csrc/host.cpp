@@ -327,7 +327,7 @@ struct l2_model {
     int32_t *pf_ids = nullptr; // ids, then positions, of a batch or prompt
     int cap_pf = 0;
     std::vector<hipEvent_t> pf_ev[kMaxLanes];
-    hipEvent_t pf_join = nullptr;
+    hipEvent_t pf_join = nullptr, step_done = nullptr;
     int32_t *dprompt = nullptr, *dout_ids = nullptr;
     int cap_prompt = 0, cap_out = 0;
     // The decode step as a HIP graph (one per bucket of positions, kept in the state).  Off by default: a
@@ -773,6 +773,7 @@ extern "C" void l2_model_close(l2_model *m) {
     for (auto &v : m->pf_ev)
         for (hipEvent_t e : v) (void)hipEventDestroy(e);
     if (m->pf_join) (void)hipEventDestroy(m->pf_join);
+    if (m->step_done) (void)hipEventDestroy(m->step_done);
     if (m->hs.base) (void)hipHostFree(m->hs.base);
     for (hipStream_t es : m->extra_stream)
         if (es) (void)hipStreamDestroy(es);
@@ -1782,7 +1783,7 @@ extern "C" int l2_forward(l2_model *m, l2_state *s, const int32_t *tokens, const
     return L2_OK;
 }
 
-int l2_forward_weights(l2_model *m, l2_state *s, int32_t token, int32_t pos, float temperature, SampleWeights *out) {
+int l2_forward_weights(l2_model *m, l2_state *s, int32_t token, int32_t pos, float temperature, bool more, SampleWeights *out) {
     if (s->m != m) return l2_fail(L2_ERR_ARG, "state belongs to another model");
     int max_pos = 0;
     L2_TRY(check_tokens(m, &token, &pos, 1, &max_pos));
@@ -1791,7 +1792,13 @@ int l2_forward_weights(l2_model *m, l2_state *s, int32_t token, int32_t pos, flo
     in.src.token = token, in.logits = m->logits, in.amax = m->amax;
     L2_TRY(forward_enqueue(m, s, 1, pos, in));
     L2_TRY(sample_weights_launch(m->hs.logits, m->hs.redo, m->logits, m->d.vocab_size, temperature, m->amax, m->stream));
-    L2_TRY(wait_host(m, nullptr, nullptr));
+    if (more) { // an event is all that a step inside a call has to wait for (7B: 24 us less than for the stream)
+        if (!m->step_done) L2_HIP(hipEventCreateWithFlags(&m->step_done, hipEventDisableTiming));
+        L2_HIP(hipEventRecord(m->step_done, m->stream));
+        L2_HIP(hipEventSynchronize(m->step_done));
+    } else {
+        L2_TRY(wait_host(m, nullptr, nullptr));
+    }
     *out = {m->hs.logits, m->hs.redo};
     return L2_OK;
 }

@@ -80,12 +80,12 @@ int l2_prefill_ladder_end(int n_prompt);
 int l2_prefill_ladder(l2_model *m, l2_state *s, const int32_t *prompt, int n_prompt, bool wait);
 
 // One forward step for the sampler: the weights above of the logits at `pos`, in host memory that belongs to the model
-// and stands until its next call.
+// and stands until its next call.  more: another step of the caller's call follows (else the call's work is waited for).
 struct SampleWeights {
     float *w;
     const unsigned long long *redo;
 };
-int l2_forward_weights(l2_model *m, l2_state *s, int32_t token, int32_t pos, float temperature, SampleWeights *out);
+int l2_forward_weights(l2_model *m, l2_state *s, int32_t token, int32_t pos, float temperature, bool more, SampleWeights *out);
 
 // ---- device views ---------------------------------------------------------
 

@@ -379,7 +379,7 @@ extern "C" int l2_generate(l2_model *m, l2_state *s, const l2_tokenizer *t, cons
                     next = prompt32[pos];
                 } else if (temperature > 0.0f) {
                     SampleWeights w{};
-                    L2_TRY(l2_forward_weights(m, s, token, p32, temperature, &w));
+                    L2_TRY(l2_forward_weights(m, s, token, p32, temperature, pos + 1 < steps, &w));
                     next = sample_weights(w, d.vocab_size, rng);
                 } else { // a negative temperature (or none) turns the distribution round: everything here
                     L2_TRY(l2_forward(m, s, &token, &p32, 1, logits.data()));
