@@ -166,12 +166,12 @@ int l2_qlinear_set_mode(l2_qlinear *q, int mode);
  * hipStream_t; NULL is the default stream) and the call returns without waiting.  y may lie over x, in part or
  * as a whole (compared by address: memory mapped at two addresses must not be given as both).  Both are aligned
  * as floats are; more is not asked for.  It calls no hipMalloc,
- * hipFree or other allocating routine: the one intermediate (x in the layer's act-order) lives in a fixed
- * device array of L2_MATVEC_DEVICE_MAX_ELEMS floats (48 MiB with what a batch needs) that each GPU holds until the process
- * ends, so B * in must not exceed that count (L2_ERR_RANGE otherwise).  All calls on one GPU share the array:
- * calls that overlap in time on one GPU (two streams, two threads) race; serialise them.  y equals
+ * hipFree or other allocating routine: what it needs beyond x and y (x in the layer's
+ * act-order, or a batch's planes and partial tiles) lives in fixed device arrays, 48 MiB in all, that each GPU holds
+ * until the process ends, sized for B * in of up to L2_MATVEC_DEVICE_MAX_ELEMS floats (L2_ERR_RANGE beyond).  All calls
+ * on one GPU share the arrays: calls that overlap in time on one GPU (two streams, two threads) race; serialise them.  y equals
  * l2_qlinear_matvec's bit for bit.  What a first launch does besides enqueueing (loading the code object on the
- * device, raising the kernel's LDS limit, resolving the array's address) l2_qlinear_create has already done, with
+ * device, raising the kernel's LDS limit, resolving the arrays' addresses) l2_qlinear_create has already done, with
  * the device that is current at that time: a handle is used on the device it was created on, and every call
  * here, the first included, may be made while hip_stream is being captured into a graph.  Nothing it enqueues
  * is a memset node. */

@@ -1107,7 +1107,7 @@ static int operator_bufs(OperatorBufs &b, const DevQLinear &q, int B, int planes
 
 // Everything a later launch of this layer's operator would otherwise do on first use, done once here and waited
 // for: the code object is loaded on this device, the kernel's dynamic-LDS limit is raised, the fixed scratch
-// array's address is resolved.  A call made under stream capture afterwards only enqueues kernels.
+// arrays' addresses are resolved.  A call made under stream capture afterwards only enqueues kernels.
 static int qlinear_warm_up(l2_qlinear *q) {
     L2_TRY(qlinear_scratch(q, 1));
     FixedScratch fixed{};
@@ -1249,10 +1249,10 @@ extern "C" int l2_qlinear_matvec(l2_qlinear *q, const float *x_host, int B, floa
 }
 
 // ---- the same operator for callers that cannot allocate ---------------------------------------------
-// (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).  The one buffer
-// l2_qlinear_matvec needs beyond its input and output -- x gathered into the layer's act-order -- lives in a
-// fixed device array instead of a hipMalloc'ed one.  Every GPU the library runs on holds its own copy of
-// the array, at its own address, until the process ends.
+// (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).  What
+// l2_qlinear_matvec needs beyond its input and output lives in fixed device arrays instead of hipMalloc'ed ones.
+// Every GPU the library runs on holds its own copy of the arrays, at its own addresses, until the process ends.
+// A few columns: x gathered into the layer's act-order.
 static constexpr size_t kScratchFloats = L2_MATVEC_DEVICE_MAX_ELEMS; // 4 MiB
 static __device__ __align__(256) float scratch[kScratchFloats];
 // A batch: its activations as three 16-bit planes (rows padded to 64, so at most twice the elements) and partial tiles.

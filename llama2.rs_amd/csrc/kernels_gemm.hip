@@ -19,7 +19,7 @@
 // 0.60 to 1.91 and 0.59 to 2.30.
 //
 // Against the matvec kernels run once per column, which read and dequantise the weights for each of them: 4096x11008,
-// group 32, 61 columns 330 -> 46 us with everything around it; a 299-token prompt on 7B 230 -> 22 ms.
+// group 32, 61 columns 330 -> 40.4 us with everything around it; a 298-token prompt on 7B 230 -> 15.1 ms.
 #include <algorithm>
 
 #include "l2_internal.h"
@@ -855,7 +855,8 @@ GemmShape gemm_shape(const Q4Launch &L, int slice_batch, int planes) {
     auto slices = [&](int slots, int blocks, int most) { return std::max(1, std::min({slots / blocks, most, units / 2})); };
     // K slices: as many as keep the grid within one round of resident blocks.  Up to 32 columns the registers and the
     // LDS hold four blocks per CU of 128 rows, and the partial tiles are small; beyond, two of 256 rows (fp32 weights: three
-    // of 128).
+    // of 128).  Where the rows are cut in 128s all the same (below), the grid is twice what was counted and may take a
+    // second round: 11008 outputs, 61 columns are 688 blocks in 8 slices on 512 slots.
     const int rows32 = row_blocks(L, 128), rows64 = row_blocks(L, 256);
     if (slice_batch <= 32)
         s.slices = slices(4 * cu_count(), rows32, kMaxGemmSlices);
@@ -864,7 +865,7 @@ GemmShape gemm_shape(const Q4Launch &L, int slice_batch, int planes) {
     else
         s.slices = slices(2 * cu_count(), rows64 * ((slice_batch + 63) / 64), 8);
     s.tokens = B <= 32 ? 32 : 64;
-    // 256 rows reuse every 16 bytes read from the LDS twice; 128 where the blocks would not fill the chip
+    // 256 rows reuse every 16 bytes read from the LDS twice; 128 where such blocks would be fewer than three to two CUs
     const int tiles = (B + s.tokens - 1) / s.tokens;
     s.rows = planes == kDensePlanes || s.tokens == 32 || rows64 * tiles * s.slices < 3 * cu_count() / 2 ? 128 : 256;
     s.row_blocks = s.rows == 128 ? rows32 : rows64;

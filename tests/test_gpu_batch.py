@@ -213,7 +213,7 @@ def test_between_products(ops, n_heads, n_kv, G):
     m.close()
 
 
-# the classifier with whole tiles of rows per wave and with a quarter, at both sides of where the rule changes, the last
+# the classifier with whole tiles of rows per wave and with a quarter or half of them, at both sides of where the rule changes, the last
 # wave ragged; its running maximum against the logits
 @pytest.mark.parametrize("n_heads,vocab", [(8, 1), (8, 2001), (8, 8160), (8, 8163), (16, 4080), (16, 4083), (32, 2033), (32, 2049), (40, 1025)])
 def test_classifier_few_rows(ops, n_heads, vocab):
