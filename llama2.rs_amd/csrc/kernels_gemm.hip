@@ -370,7 +370,7 @@ __global__ __launch_bounds__(256, 2) void q4_tile_gemm_kernel(const Q4Launch L, 
     // Runs that have ended: their sum lies where the result goes, every lane's own elements.  (There are no registers for a
     // third set of tiles.  What it costs is this traffic: 4096 -> 22016 outputs, 512 columns, group 32, 45 MB a time; a layer
     // of 7B, 512 tokens, 0.88 -> 0.93 ms with runs of 64 groups, 0.98 with 32; 299 tokens, group 128 has one run.)
-    float *__restrict__ const sums = KS > 1 || partials ? ws + ws_base + (size_t)ks * B * n_out : L.m[mi].y;
+    float *const sums = KS > 1 || partials ? ws + ws_base + (size_t)ks * B * n_out : L.m[mi].y;
     auto each_sum = [&](auto &&f) __attribute__((always_inline)) {
 #pragma unroll
         for (int mt = 0; mt < MT; mt++)
