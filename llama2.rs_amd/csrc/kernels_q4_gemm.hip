@@ -1,26 +1,32 @@
 // Batched-prefill form of the GPTQ 4-bit linear layer for gfx950: dequantise
 // tiles of the packed weights to fp16 in registers and feed them to the matrix
-// cores (v_mfma_f32_32x32x16_f16), fp32 accumulate.
+// cores (v_mfma_f32_16x16x32_f16), fp32 accumulate.
 //
 //   Y[t][o] = sum_k W[o][k] * X[t][k],   W[o][k] = scales[o][k/G] * (nib(qweight[o],k) - z1[o][k/G])
 //
 // for a chunk of T tokens whose inputs the caller has already brought into this
 // layer's g_index order, multiplied by the norm weight where one applies, and
-// rounded to fp16 (kernels_gemm.hip).  This is the one place in the token loop
-// that is a dense contraction, hence the one place that uses MFMA; the decode
-// matvec stays on the vector ALU in fp32.
+// rounded to fp16 (kernels_gemm.hip).
 //
-// Tiling.  A block is 4 waves; a wave owns one tile of 32 output rows and all NB
-// blocks of 32 tokens (the dequantised weights are reused NB times), so a block
-// covers 128 rows x 32*NB tokens.  With only 128 tokens per chunk that leaves
-// few blocks, so K is also cut into KS slices; each slice writes
-// its fp32 partial tile to a workspace and the consumer (or gemm_reduce_kernel) adds
-// the slices in a fixed order.  K advances
-// 64 at a time: lane (r = l%32, h = l/32) loads the 16 bytes qweight[o][K/8+4h ..
-// +4) of its row -- four packed words, each of which is exactly the 8 k-values
-// one MFMA step wants from this lane.  The X slice [tokens][64] is staged in LDS
-// (rows padded to 72 halves so that 16-byte reads of 32 lanes are conflict-free),
-// double-buffered.
+// Tiling.  A wave owns 32 output rows and 32 NB tokens (its dequantised weights are reused for all of them); a block is 8 waves
+// side by side over the rows with NB = 4, one per CU, or 4 waves with NB <= 2, two or three per CU.  K may be cut into KS
+// slices; each writes its fp32 partial tile to a workspace and the consumer (or gemm_reduce_kernel) adds them in a fixed order.
+//
+// Memory.  Everything the K loop reads comes through LDS without touching a register (buffer_load ... lds): the activation
+// tiles [tokens][64 k], which the block shares, and, for each wave alone, the packed weights, scales and zero points of its
+// rows in units of 128 k.  Tiles are requested one unit ahead, weights two; the only waits are one vmcnt per kind and unit
+// and ONE block barrier per unit.  16-byte pieces of a token (a row of weights) lie in the tile permuted by its number, so
+// that the reads of 16 lanes meet 16 different banks; the lanes of the load permute their addresses accordingly.
+//
+// What bounds it, and what the layout of the loop answers (70B's w1|w3, 776 tokens: 928 -> 804 us; 7B's at 511: 116 -> 107):
+//   - A SIMD issues an instruction every 4 to 5 cycles from its two waves, and one wave alone gets half of that.  So the
+//     vector work (dequantisation of the next step, fold of the group before) stands evenly between the MFMAs of both halves
+//     of a step, operands are read from LDS four pairs of MFMAs ahead, and a wave's priority falls with its progress since
+//     the last barrier: with equal priorities the older wave of a SIMD ran ahead and waited 30 % of the time at the barrier
+//     (1862 cycles per step of 64 k; 1650 now, 1024 of them MFMAs).
+//   - Power.  With 70B's shapes the clock falls to 1.8 - 1.9 GHz; all-zero activations run the same code at 2.23 GHz.  The
+//     16x16x32 form needs less than 32x32x16 for the same products (a loop of nothing else: 1974 against 1655 TFLOP/s), and
+//     blocks of 256 rows read every activation tile half as often as blocks of 128.
 //
 // Dequant.  (w >> 4i) & 0x000F000F | 0x64006400 is the fp16 pair (1024+n_i,
 // 1024+n_{i+4}); subtracting 1024+z1 is exact.  The pairs come out as
@@ -28,8 +34,8 @@
 // inside every 8 consecutive k.  For G >= 64 the matrix cores see the exact
 // integers n - z1 and the fp32 scale is applied to the fp32 partial sum of each
 // group (one FMA per accumulator element and group), so the only rounding on
-// the weight side is none at all; for G = 32 a K step of 64 straddles two
-// groups, and the weights are multiplied by fp16(scale) before the MFMA.
+// the weight side is none at all; for G = 32 a step of 32 k would be a group,
+// and the weights are multiplied by fp16(scale) before the MFMA.
 #include "l2_internal.h"
 #include <algorithm>
 
@@ -37,9 +43,7 @@ namespace {
 
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef float f16v __attribute__((ext_vector_type(16)));
-
-constexpr int kXPad = 8; // halves of padding per staged token row (K step + 8: 16-byte reads stay conflict-free)
+typedef float f4v __attribute__((ext_vector_type(4)));
 
 union A8 {
     h8 v;
@@ -47,347 +51,293 @@ union A8 {
     uint32_t u[4];
 };
 
-// (x & mask) | magic in one instruction; the compiler splits it into v_and + v_or because both constants
-// would be literals.  mask lives in a VGPR, magic in an SGPR (one scalar operand per VALU instruction).
-__device__ __forceinline__ uint32_t and_or(uint32_t x, uint32_t mask_v, uint32_t magic_s) {
-    uint32_t r;
-    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "v"(mask_v), "s"(magic_s));
-    return r;
-}
-
-struct DequantConsts {
-    uint32_t mask_lo, mask_hi; // 0x000F000F, 0x00F000F0 (VGPRs)
-    uint32_t magic;            // 0x64006400: fp16 1024 in both halves (SGPR)
-    h2 neg_off;                // -(1024 + z1)
-    h2 neg_off16;              // -(64 + z1)
-    h2 sixteenth;              // 1/16
+// The constants of a lane's row and group, and the dequantisation of a packed word: 8 nibbles -> 8 fp16 values n - z1
+// (exact), times `scale` if SCALED, in the pair order (0,4,1,5,2,6,3,7).  Nibbles 0 and 4 (and 2, 6 after one shift by 8)
+// land in the low mantissa bits of the fp16 pair: 1024 + n.  Nibbles 1 and 5 (3, 7) are taken where they stand, four bits
+// higher: 1024 + 16 n, and one packed FMA with 1/16 brings them to 64 + n, both exact.  9 instructions per word.
+struct Dequant16 {
+    uint32_t mask_lo, mask_hi, magic; // 0x000F000F, 0x00F000F0, 0x64006400: opaque, so that and + or is one instruction
+    uint32_t c1024, c64;              // fp16 pairs -(1024 + 1), -(64 + 1)
+    h2 neg_off, neg_off16;            // -(1024 + z1), -(64 + z1)
+    __device__ __forceinline__ Dequant16() : mask_lo(0x000F000Fu), mask_hi(0x00F000F0u), magic(0x64006400u), c1024(0xE401E401u), c64(0xD410D410u) {
+        asm("" : "+v"(mask_lo), "+v"(mask_hi), "+s"(magic), "+v"(c1024), "+v"(c64));
+    }
+    // z1 = zn + 1 in the mantissas of 1024 (steps of 1) and 64 (steps of 1/16)
+    __device__ __forceinline__ void zero_point(uint32_t zn) {
+        neg_off = __builtin_bit_cast(h2, __umul24(zn, 0x10001u) + c1024);
+        neg_off16 = __builtin_bit_cast(h2, __umul24(zn, 0x100010u) + c64);
+    }
+    // pair i of a word; i = 2 and 3 of the word shifted by 8
+    template <bool SCALED>
+    __device__ __forceinline__ h2 pair(uint32_t w, int i, h2 scale) const {
+        const h2 sixteenth = h2{(_Float16)0.0625f, (_Float16)0.0625f};
+        const h2 v = i % 2 == 0 ? __builtin_bit_cast(h2, (w & mask_lo) | magic) + neg_off
+                                : __builtin_elementwise_fma(__builtin_bit_cast(h2, (w & mask_hi) | magic), sixteenth, neg_off16);
+        return SCALED ? v * scale : v;
+    }
 };
 
-// One packed word of 8 nibbles -> 8 fp16 values n - z1 (exact), times `scale` if SCALED, in the pair
-// order (0,4,1,5,2,6,3,7).  Nibbles 0 and 4 (and 2, 6 after one shift by 8) land in the low mantissa bits
-// of the fp16 pair: 1024 + n.  Nibbles 1 and 5 (3, 7) are taken where they stand, four bits higher:
-// 1024 + 16 n, and one packed FMA with 1/16 brings them to 64 + n, both exact.  9 instructions per word.
-template <bool SCALED>
-__device__ __forceinline__ h8 dequant8(uint32_t w, const DequantConsts &c, h2 scale) {
-    A8 a;
-    const uint32_t w8 = w >> 8;
-    h2 v0 = __builtin_bit_cast(h2, and_or(w, c.mask_lo, c.magic)) + c.neg_off;
-    h2 v1 = __builtin_elementwise_fma(__builtin_bit_cast(h2, and_or(w, c.mask_hi, c.magic)), c.sixteenth, c.neg_off16);
-    h2 v2 = __builtin_bit_cast(h2, and_or(w8, c.mask_lo, c.magic)) + c.neg_off;
-    h2 v3 = __builtin_elementwise_fma(__builtin_bit_cast(h2, and_or(w8, c.mask_hi, c.magic)), c.sixteenth, c.neg_off16);
-    a.p[0] = SCALED ? v0 * scale : v0;
-    a.p[1] = SCALED ? v1 * scale : v1;
-    a.p[2] = SCALED ? v2 * scale : v2;
-    a.p[3] = SCALED ? v3 * scale : v3;
-    return a.v;
-}
+constexpr int kStepRow = 128; // bytes of a token in an activation tile of 64 k
 
-template <class T>
-__device__ __forceinline__ T ld_at(const void *base, uint32_t byte_offset) {
-    return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + byte_offset);
-}
-
-// Software pipeline of the K loop.  The weights of a K step are loaded WR steps ahead, its activation
-// tile XP steps ahead, the scales and zero points of PW groups once per PW steps, all unconditionally
-// (steps past the end of the block's K slice re-read its last step), into rings of registers indexed
-// statically by the position in the loop body, which is unrolled PW times.  Loads return in order, so a
-// wait for the oldest ring slot leaves the younger ones in flight; within a step the activation tile is
-// requested before the weights, because the end of the step waits for it (it comes from the L2) and would
-// otherwise wait for the weights requested before it as well.  Shallow rings on purpose: at K steps of 128,
-// depths of 4 and 2 instead of 2 and 1 cost 34 more registers and were 3 % slower.
-constexpr int kGemmPW = 4;
-// ring depths in K steps: 256 k ahead for the weights, 128 k for the activation tile
-constexpr int gemm_wr(int kstep) { return 256 / kstep; }
-constexpr int gemm_xp(int kstep) { return 128 / kstep; }
-
+// LDS of a block of NW waves: four activation tiles, and for each wave three units of 128 k of its 32 rows' weights, scales
+// and zero points.
+template <int G, int NW>
 struct GemmLds {
-    float gsc[2][kGemmPW][128];   // fp32 scales of the block's 128 rows, PW groups at a time
-    int32_t zsc[2][kGemmPW][16]; // their packed zero points: one word per 8 rows and group
+    static constexpr int kScaleLoads = G == 32 ? 2 : 1; // of 64 words per unit
+    static constexpr int kWeights = 32 * 64, kScales = 256 * kScaleLoads;
+    static constexpr int kUnit = kWeights + 2 * kScales;
+    static constexpr size_t size(int tokens) { return (size_t)4 * tokens * kStepRow + (size_t)NW * 3 * kUnit; }
 };
 
-// 128 rows rb * 128.. of the matrices of a launch against the 32 NB tokens t0.., K slice ks of KS.
-template <int G, int NB, int KSTEP>
-__device__ __forceinline__ void q4_gemm_tile(const Q4Launch &L, const XhList &xh_list, const float *__restrict__ ss,
-                                             float *__restrict__ ws, int KS, int partials, int rb, int ks, int t0, GemmLds &S) {
-    constexpr int PW = kGemmPW, XP = gemm_xp(KSTEP), WR = gemm_wr(KSTEP);
-    static_assert(PW % WR == 0 && PW % XP == 0, "ring slots are indexed by the position in the unrolled body");
-    constexpr int W = KSTEP / 64;        // sub-steps of 64 k per K step
-    constexpr int kXRow = KSTEP + kXPad; // halves per staged token row
-    static_assert(KSTEP == 64 || G >= KSTEP, "a longer K step stays inside one group");
-    constexpr int TN = 32 * NB;
-    constexpr bool SA = G >= 64; // scale after the group's partial sum
-    extern __shared__ _Float16 xs[]; // [2][TN][kXRow]
-    auto &gsc = S.gsc;
-    auto &zsc = S.zsc;
-    const int in = L.in;
-    const int n_k = in / KSTEP; // K iterations
+typedef uint32_t u4v __attribute__((ext_vector_type(4)));
 
+// Memory as a buffer of `bytes` from `base` (both the same in every lane).
+__device__ __forceinline__ u4v buffer(const void *base, uint32_t bytes) {
+    const uint64_t p = reinterpret_cast<uint64_t>(base);
+    return u4v{(uint32_t)__builtin_amdgcn_readfirstlane((int)p), (uint32_t)__builtin_amdgcn_readfirstlane((int)(p >> 32)) & 0xFFFFu,
+               (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
+}
+
+// From memory into LDS past the registers: lane l's piece (16 or 4 bytes) at `off` + `soff` bytes of the buffer goes to
+// lds + size * l.  `at` shifts both by the same constant, so callers have it taken off `off`.  vmcnt counts them, and since the
+// compiler does not know of them, nothing else in the loop may load from memory.
+#define LDS_TO(lds) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" ::"s"(lds) : "memory")
+#define LDS_LOAD(n, at, buf, off, soff) \
+    asm volatile("buffer_load_dword" n " %0, %1, %2 offen offset:%3 lds" ::"v"(off), "s"(buf), "s"(soff), "n"(at) : "memory")
+
+// 32 NW rows rb * 32 NW.. of the matrices of a launch against the 32 NB tokens t0.., K slice ks of KS.
+template <int G, int NB, int NW>
+__device__ __forceinline__ void q4_gemm_tile(const Q4Launch &L, const XhList &xh_list, const float *__restrict__ ss,
+                                             float *__restrict__ ws, int KS, int partials, int rb, int ks, int t0) {
+    using S = GemmLds<G, NW>;
+    constexpr int TN = 32 * NB, kTile = TN * kStepRow;
+    constexpr bool SA = G >= 64; // scale after the group's partial sum
+    extern __shared__ __align__(16) char lds[];
     int mi = 0;
     while (mi + 1 < L.n_mats && rb >= L.m[mi].row_blocks) {
         rb -= L.m[mi].row_blocks;
         mi++;
     }
     const Q4Mat &M = L.m[mi];
-    const _Float16 *xh = reinterpret_cast<const _Float16 *>(xh_list.p[mi]); // [B][in] fp16, pair-interleaved
-    const int n_out = M.out;
-    const int groups = L.groups;
-    const int B = L.batch;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int r = lane & 31, h = lane >> 5;
-    const int C4 = in >> 5; // uint4 per weight row
+    const int n_out = M.out, groups = L.groups, B = L.batch, in = L.in;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, kg = lane >> 4;
+    const int obase = rb * (32 * NW) + wave * 32;
+    // this block's slice of K, in units of 128
+    const int n_units = in / 128;
+    const int u0 = (int)((long)n_units * ks / KS), u1 = (int)((long)n_units * (ks + 1) / KS);
 
-    const int o_lane = rb * 128 + wave * 32 + r;
-    const int orow = min(o_lane, n_out - 1);
-    // scale-after form: the thread fetches the scales of row `grow` for two of every PW groups
-    const int grow = min(rb * 128 + (tid & 127), n_out - 1);
-    const int ghalf = tid >> 7;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)lds;
+    const uint32_t wave_at = 4 * kTile + wave * 3 * S::kUnit; // of this wave's weights, scales and zero points
 
-    f16v acc[NB];  // running result
-    f16v accg[NB]; // partial sum of the current group (SA only): every K step starts it from zero
+    // Where a lane's pieces come from.  A wave's 1 KB pieces of an activation tile follow each other in the LDS (fewer pieces
+    // than waves: the last ones fetch the same), as do the parts of a unit: one base each, the rest in the instructions.
+    constexpr int XP = (NB * 4 + NW - 1) / NW;
+    constexpr int kBias = 4096;
+    const u4v xbuf = buffer(reinterpret_cast<const char *>(xh_list.p[mi]) - kBias, (uint32_t)((size_t)B * in * 2 + kBias));
+    const u4v wbuf = buffer(reinterpret_cast<const char *>(M.qweight) - kBias, (uint32_t)((size_t)n_out * (in >> 1) + kBias));
+    const u4v sbuf = buffer(reinterpret_cast<const char *>(M.scales) - kBias, (uint32_t)((size_t)n_out * groups * 4 + kBias));
+    const u4v zbuf = buffer(reinterpret_cast<const char *>(M.qzeros) - kBias, (uint32_t)((size_t)(n_out >> 3) * groups * 4 + kBias));
+    const int xfirst = min(wave * XP, NB * 4 - XP);
+    uint32_t xoff[XP], woff[2], soff, zoff;
 #pragma unroll
-    for (int nb = 0; nb < NB; nb++)
-#pragma unroll
-        for (int i = 0; i < 16; i++) acc[nb][i] = 0.f;
-    constexpr int KPG = G / KSTEP > 0 ? G / KSTEP : 1; // K iterations per group
-    // this block's slice of K, in whole groups
-    const int n_grp = n_k / KPG;
-    // slices start on an even group: the scales are fetched as aligned pairs
-    const int kit0 = ((int)((long)n_grp * ks / KS) & ~1) * KPG;
-    const int kit1 = ks + 1 == KS ? n_k : ((int)((long)n_grp * (ks + 1) / KS) & ~1) * KPG;
-    const int n_it = kit1 - kit0;
-
-    struct WStage {
-        uint4 w[W];
-        int32_t z;
-        float s;  // this lane's row, scaled form only
-    };
-    const void *qw_base = M.qweight;
-    const void *qz_base = M.qzeros;
-    const void *sc_base = M.scales;
-    auto fetch_w = [&](int kit, WStage &d) {
-        const int kc = min(kit, kit1 - 1);
-        const int g = (kc * KSTEP + 32 * h) / G;
-#pragma unroll
-        for (int sw = 0; sw < W; sw++)
-            d.w[sw] = ld_at<uint4>(qw_base, (uint32_t)(orow * C4 + kc * (2 * W) + 2 * sw + h) << 4);
-        if constexpr (SA) {
-            d.z = 0, d.s = 0.f; // scale-after form: zero points and scales travel by the block, PW groups at a time
-        } else {
-            d.z = ld_at<int32_t>(qz_base, (uint32_t)((orow >> 3) * groups + g) << 2);
-            d.s = ld_at<float>(sc_base, (uint32_t)(orow * groups + g) << 2);
-        }
-    };
-    // Scale-after form: one 8-byte load per thread and PW K steps (a K step is a group there) instead of
-    // one scattered 4-byte load per thread and step.  Block j of PW groups starts at group kit0 + PW * j;
-    // pairs past the row's last group re-read its last pair (their steps are never run).
-    static_assert(!SA || KPG == 1, "scale-after form: a K step is one group");
-    auto fetch_gs = [&](int j) {
-        const int ge = min(kit0 + PW * j + 2 * ghalf, groups - 2);
-        return ld_at<float2>(sc_base, (uint32_t)(grow * groups + ge) << 2);
-    };
-    auto store_gs = [&](int j, const float2 v) {
-        gsc[j & 1][2 * ghalf][tid & 127] = v.x;
-        gsc[j & 1][2 * ghalf + 1][tid & 127] = v.y;
-    };
-    // zero points of the same PW groups: 16 row groups x PW words per block; every wave fetches the same 64
-    // words (no load under a branch), lane -> (row group lane / 4, group lane % 4)
-    const int zrg = min(rb * 16 + (lane >> 2), (n_out - 1) >> 3);
-    auto fetch_zs = [&](int j) {
-        const int ge = min(kit0 + PW * j + (lane & 3), groups - 1);
-        return ld_at<int32_t>(qz_base, (uint32_t)(zrg * groups + ge) << 2);
-    };
-    auto store_zs = [&](int j, const int32_t v) { zsc[j & 1][lane & 3][lane >> 2] = v; };
-    // staging map: thread -> (token, 16-byte segment) x (TN*8/256) pieces
-    constexpr int SEGS = KSTEP / 8; // 16-byte segments per token and K step
-    constexpr int PIECES = TN * SEGS / 256;
-    struct XStage {
-        uint4 v[PIECES];
-    };
-    uint32_t xoff[PIECES]; // byte offset of this thread's pieces within a K step
-#pragma unroll
-    for (int p = 0; p < PIECES; p++) {
-        const int idx = p * 256 + tid;
-        const int t = idx / SEGS, seg = idx % SEGS;
-        xoff[p] = ((uint32_t)min(t0 + t, B - 1) * (uint32_t)in + seg * 8) * 2u;
+    for (int i = 0; i < XP; i++) { // activations: 8 tokens of 128 bytes, a token's 16-byte pieces permuted by its number
+        const int t = (xfirst + i) * 8 + (lane >> 3);
+        xoff[i] = (uint32_t)min(t0 + t, B - 1) * (uint32_t)in * 2u + (((lane & 7) ^ ((t >> 1) & 7)) << 4) + kBias - i * 1024;
     }
-    auto fetch_x = [&](int kit, XStage &d) {
-        const uint32_t kb = (uint32_t)min(kit, kit1 - 1) * (uint32_t)(KSTEP * 2);
 #pragma unroll
-        for (int p = 0; p < PIECES; p++) d.v[p] = ld_at<uint4>(xh, xoff[p] + kb);
+    for (int i = 0; i < 2; i++) { // weights: 16 rows of 64 bytes, permuted likewise
+        const int row = i * 16 + (lane >> 2);
+        woff[i] = (uint32_t)min(obase + row, n_out - 1) * (uint32_t)(in >> 1) + (((lane & 3) ^ ((row >> 2) & 3)) << 4) + kBias - i * 1024;
+    }
+    const int srow = min(obase + (lane & 31), n_out - 1), lane_group = G == 128 ? 0 : lane >> 5; // of two groups (G = 128: the same one again)
+    soff = ((uint32_t)(srow * groups) + lane_group) * 4u + kBias - S::kWeights;
+    zoff = ((uint32_t)((srow >> 3) * groups) + lane_group) * 4u + kBias - S::kWeights - S::kScales;
+    // ... and where it reads them
+    uint32_t xr[2]; // piece 2 kg + s of token r
+#pragma unroll
+    for (int s = 0; s < 2; s++) xr[s] = (uint32_t)r * kStepRow + (((2 * kg + s) ^ ((r >> 1) & 7)) << 4);
+    const uint32_t wr = wave_at + r * 64 + (((kg >> 1) ^ ((r >> 2) & 3)) << 4) + (kg & 1) * 8; // of a unit's first step; the second's: ^ 32
+    const uint32_t sr = wave_at + S::kWeights + kg * 16, zr = wave_at + S::kWeights + ((G == 32 ? (kg >> 1) * 32 : 0) + r) * 4;
+    const int zsh = 4 * (r & 7); // obase is a multiple of 8
+
+    const uint32_t x_last = (uint32_t)u1 * 256 - 128, w_last = (uint32_t)(u1 - 1) * 64; // requests past the slice's end take its last piece again
+    uint32_t x_at = (uint32_t)u0 * 256, w_at = (uint32_t)u0 * 64;                       // what is requested next
+    constexpr int WL = 2 + 2 * S::kScaleLoads;
+    auto fetch_x = [&](const int slot, const int i) __attribute__((always_inline)) { // piece i of XP
+        LDS_TO(lds0 + slot * kTile + xfirst * 1024);
+        LDS_LOAD("x4", i * 1024, xbuf, xoff[i], x_at);
+        if (i == XP - 1) x_at = min(x_at + 128, x_last);
     };
-    auto store_x = [&](int buf, const XStage &d) {
+    auto fetch_w = [&](const uint32_t unit, const int i) __attribute__((always_inline)) { // piece i of WL
+        const uint32_t s_at = G == 128 ? w_at >> 4 : G == 64 ? w_at >> 3 : w_at >> 2;
+        LDS_TO(lds0 + wave_at + unit);
+        if (i < 2) LDS_LOAD("x4", i * 1024, wbuf, woff[i], w_at);
+        else if (i == 2) LDS_LOAD("", S::kWeights, sbuf, soff, s_at);
+        else if (i == 3) LDS_LOAD("", S::kWeights + S::kScales, zbuf, zoff, s_at);
+        else if (i == 4) LDS_LOAD("", S::kWeights + 256, sbuf, soff - 256 + 8, s_at); // G = 32: the second step's groups
+        else LDS_LOAD("", S::kWeights + S::kScales + 256, zbuf, zoff - 256 + 8, s_at);
+        if (i == WL - 1) w_at = min(w_at + 64, w_last);
+    };
+
+    constexpr int NT = 2 * NB; // tiles of 16 tokens
+    f4v acc[NT][2], accg[NT][2]; // running result, two tiles of 16 rows; partial sums of the current group (SA)
 #pragma unroll
-        for (int p = 0; p < PIECES; p++) {
-            const int idx = p * 256 + tid;
-            const int t = idx / SEGS, seg = idx % SEGS;
-            *reinterpret_cast<uint4 *>(xs + ((size_t)buf * TN + t) * kXRow + seg * 8) = d.v[p];
+    for (int n = 0; n < NT; n++)
+#pragma unroll
+        for (int m = 0; m < 2; m++) acc[n][m] = accg[n][m] = f4v{0.f, 0.f, 0.f, 0.f};
+    f4v sv[2] = {}; // scales of the group that accg holds
+    auto fold = [&](int n, int m) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[n][m][e] = fmaf(sv[m][e], accg[n][m][e], acc[n][m][e]);
+        asm volatile("" : "+v"(acc[n][m])); // here, and not where the compiler would rather have it
+    };
+
+    Dequant16 dq[2];      // of the two rows of a lane
+    A8 aq[2][2][2];       // weights of this step and the next: [rows][k]
+    uint2 wd[2];          // packed weights of the next step,
+    int zw[2];            // their zero points
+    float sl[2] = {};     // and scales (G = 32)
+    h2 s16[2] = {};
+    h8 bq[8];             // activations of eight pairs of MFMAs
+    auto read_w = [&](const int par, uint32_t unit) __attribute__((always_inline)) {
+        const int gi = G == 128 ? 0 : G == 64 ? par * 128 : par * 256; // of the step's group
+#pragma unroll
+        for (int m = 0; m < 2; m++) {
+            wd[m] = *reinterpret_cast<const uint2 *>(lds + (wr ^ (par * 32)) + unit + m * 1024);
+            if (G != 128 || par == 0) zw[m] = *reinterpret_cast<const int *>(lds + zr + unit + S::kScales + gi + m * 64);
+            if (!SA) sl[m] = *reinterpret_cast<const float *>(lds + zr + unit + gi + m * 64);
         }
     };
+    auto constants = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int m = 0; m < 2; m++) {
+            dq[m].zero_point((zw[m] >> zsh) & 15);
+            if (!SA) s16[m] = h2{(_Float16)sl[m], (_Float16)sl[m]};
+        }
+    };
+    auto dequant = [&](const int to, const int i) __attribute__((always_inline)) { // piece i of 16
+        const int m = i >> 3, k = (i >> 2) & 1;
+        uint32_t &w = k ? wd[m].y : wd[m].x;
+        if (i % 4 == 2) w >>= 8;
+        aq[to][m][k].p[i % 4] = dq[m].template pair<!SA>(w, i % 4, s16[m]);
+    };
 
-    XStage xr[XP];
-    WStage wr[WR];
-    float2 gs2 = make_float2(0.f, 0.f);
-    int32_t zs2 = 0;
-    if constexpr (SA) gs2 = fetch_gs(0), zs2 = fetch_zs(0);
+    // A step of 64 k is 4 NB pairs of MFMAs (two tiles of 16 rows with one of 16 tokens, 32 k), the first half of the token
+    // tiles', then the others'.  Between them stands, evenly spread, what the vector unit has to do: the fold of the OTHER
+    // tiles' finished group, the next step's weights.
+    constexpr int T = 4 * NB, H = T / 2, N0 = NT / 2, AHEAD = 4;
+    auto n_of = [](int t) { return t / H * N0 + t % H % N0; };
+    auto k_of = [](int t) { return t % H / N0; };
+    auto read_x = [&](const int par, const int t, const int tile) __attribute__((always_inline)) {
+        bq[(par * T + t) % 8] = *reinterpret_cast<const h8 *>(lds + xr[k_of(t)] + tile + n_of(t) * 16 * kStepRow);
+    };
+    uint32_t unit = 0, unit1 = S::kUnit, unit2 = 2 * S::kUnit; // this unit's place, the next one's and the one's after it
+    // Step u of a round of four, which fixes the tiles' places.  Two steps (a unit) go between barriers; in the first of them
+    // the two tiles of the next unit are requested, in the places of the one before, and the weights of the one after it.
+    auto k_step = [&](const int u) __attribute__((always_inline)) {
+        const int par = u & 1, tile = u * kTile, tile1 = (u + 1) % 4 * kTile;
+        const bool first = G <= 64 || par == 0, last = G <= 64 || par == 1; // of its group
+        const int gi = G == 64 ? par * 128 : 0;
+        if (G != 128 || par == 1) constants(); // of the next step
 #pragma unroll
-    for (int j = 0; j < XP; j++) fetch_x(kit0 + j, xr[j]);
-#pragma unroll
-    for (int j = 0; j < WR; j++) fetch_w(kit0 + j, wr[j]);
-    __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0): the loop's waits then reflect its own order only
-    store_x(0, xr[0]);
-    if constexpr (SA) store_gs(0, gs2), store_zs(0, zs2);
-    __syncthreads();
-
-    // One K step; u = step % PW indexes the register rings (a compile-time constant where it is called).
-    auto k_step = [&](const int stepi, const int u) __attribute__((always_inline)) {
-        {
-            const int base = stepi - u;
-            const int kit = kit0 + stepi;
-            const int buf = u & 1; // PW is even: the parity of the step
-            // this step's weights -> registers of their own, then refill the slot
-            const int zword = SA ? zsc[(stepi / PW) & 1][u][(wave * 32 + r) >> 3] : wr[u % WR].z;
-            const int zn = (zword >> (4 * (orow & 7))) & 15;
-            DequantConsts dc;
-            dc.mask_lo = 0x000F000Fu, dc.mask_hi = 0x00F000F0u, dc.magic = 0x64006400u;
-            const _Float16 off = (_Float16)(-(1024.0f + (float)(zn + 1)));
-            const _Float16 off16 = (_Float16)(-(64.0f + (float)(zn + 1)));
-            dc.neg_off = h2{off, off};
-            dc.neg_off16 = h2{off16, off16};
-            dc.sixteenth = h2{(_Float16)0.0625f, (_Float16)0.0625f};
-            const _Float16 s1 = (_Float16)wr[u % WR].s;
-            const h2 s16 = h2{s1, s1};
-            uint32_t wd[W][4];
-#pragma unroll
-            for (int sw = 0; sw < W; sw++) {
-                wd[sw][0] = wr[u % WR].w[sw].x, wd[sw][1] = wr[u % WR].w[sw].y, wd[sw][2] = wr[u % WR].w[sw].z, wd[sw][3] = wr[u % WR].w[sw].w;
-                asm volatile("" : "+v"(wd[sw][0]), "+v"(wd[sw][1]), "+v"(wd[sw][2]), "+v"(wd[sw][3])::"memory");
+        for (int t = 0; t < T; t++) {
+            const int n = n_of(t), k = k_of(t);
+            if (par == 1 && t == T - AHEAD) {
+                // The next tiles: what this wave requested of them has landed, then what everybody has; and all reads of
+                // this unit's have come back, so that they may be overwritten.
+                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(WL) : "memory");
             }
-            // The ring slot stays in its own registers up to here (the copies above live elsewhere), so the
-            // refill can land in them: otherwise the copy takes the slot's registers over, the refill goes to
-            // fresh ones and is copied back at the loop's end, behind a wait for the load just issued.
+            const int behind = (par * T + t + AHEAD) % (2 * T); // MFMA pairs since the barrier
+            if (behind % (T / 2) == 0) asm volatile("s_setprio %0" ::"n"(3 - behind / (T / 2)));
+            if (t % 4 == 0) { // the next four pairs' activations, behind the arrival of these four's
+                __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0)
 #pragma unroll
-            for (int sw = 0; sw < W; sw++)
-                asm volatile("" : "+v"(wr[u % WR].w[sw].x), "+v"(wr[u % WR].w[sw].y), "+v"(wr[u % WR].w[sw].z), "+v"(wr[u % WR].w[sw].w));
-            if constexpr (!SA) asm volatile("" : "+v"(wr[u % WR].z));
+                for (int i = t + 4; i < t + 8; i++) read_x(i < T ? par : par ^ 1, i < T ? i : i - T, i < T ? tile : tile1);
+            }
+#pragma unroll
+            for (int m = 0; m < 2; m++) {
+                f4v &c = SA ? accg[n][m] : acc[n][m];
+                c = __builtin_amdgcn_mfma_f32_16x16x32_f16(aq[par][m][k].v, bq[(par * T + t) % 8], SA && first && k == 0 ? f4v{} : c, 0, 0, 0);
+            }
+            if (SA && (t < H ? first : last)) fold((t < H ? N0 : 0) + t % H / 2, t % 2);
+#pragma unroll
+            for (int i = t * 16 / T; i < (t + 1) * 16 / T; i++) dequant(par ^ 1, i);
+            // the scales of the group that ends with this step, once the folds above no longer need the one before's
+            if (SA && last && t >= H - 2 && t < H)
+                sv[t % 2] = *reinterpret_cast<const f4v *>(lds + sr + unit + gi + t % 2 * 64);
+            if (par == 0) {
+                // one request at a time: several in a row wait for the address unit
+                constexpr int NL = 2 * XP + WL;
+#pragma unroll
+                for (int i = t * NL / T; i < (t + 1) * NL / T; i++) {
+                    if (i < 2 * XP) fetch_x((u + 2 + i / XP) % 4, i % XP);
+                    else fetch_w(unit2, i - 2 * XP);
+                }
+            }
             __builtin_amdgcn_sched_barrier(0);
-            // The refills of this step (ring slot u of the weights, slot u % XP of the activations, once per
-            // round the next PW groups' scales and zero points) are issued one at a time between the MFMA
-            // steps below: a global load takes the wave hundreds of cycles to issue when the address unit is
-            // busy, and issued in one burst here those cycles stood in front of the first MFMA.
-            const int kc_w = min(kit + WR, kit1 - 1);
-            const uint32_t kb_x = (uint32_t)min(kit + XP, kit1 - 1) * (uint32_t)(KSTEP * 2);
-            constexpr int NL = W + 1 + PIECES + 1;
-            auto refill = [&](const int i) __attribute__((always_inline)) {
-                if (i < PIECES) { // the activations first: the end of the step waits for them, not for what follows
-                    xr[u % XP].v[i] = ld_at<uint4>(xh, xoff[i] + kb_x);
-                } else if (i < PIECES + W) {
-                    wr[u % WR].w[i - PIECES] =
-                        ld_at<uint4>(qw_base, (uint32_t)(orow * C4 + kc_w * (2 * W) + 2 * (i - PIECES) + h) << 4);
-                } else if (i == PIECES + W) {
-                    if constexpr (!SA) {
-                        const int g = (kc_w * KSTEP + 32 * h) / G;
-                        wr[u % WR].z = ld_at<int32_t>(qz_base, (uint32_t)((orow >> 3) * groups + g) << 2);
-                        wr[u % WR].s = ld_at<float>(sc_base, (uint32_t)(orow * groups + g) << 2);
-                    }
-                } else if (SA && u == 0) {
-                    gs2 = fetch_gs(base / PW + 1), zs2 = fetch_zs(base / PW + 1);
-                }
-            };
-            const _Float16 *xb = xs + (size_t)buf * TN * kXRow;
-            // W * 4 steps of 16 k.  The operands of step i + 1 (two LDS reads per token tile, the
-            // dequantised weights) are produced while the MFMAs of step i run: without this the
-            // LDS latency stands in front of every MFMA.
-            constexpr int NSTEP = W * 4;
-            h8 aq[2], bq[2][NB];
-            auto produce = [&](int step, int slot) {
-                const int sw = step >> 2, j = step & 3;
-#pragma unroll
-                for (int nb = 0; nb < NB; nb++)
-                    bq[slot][nb] = *reinterpret_cast<const h8 *>(xb + (size_t)(nb * 32 + r) * kXRow +
-                                                                 (sw * 8 + 4 * h + j) * 8);
-                aq[slot] = dequant8<!SA>(wd[sw][j], dc, s16);
-            };
-            produce(0, 0);
-            // The wave that has its MFMAs to issue goes first on its SIMD; the other wave there is in its fold, its
-            // tile store or at its barrier (q|k|v at 512 tokens 68 -> 64 us, the other launches 1-4 %).
-            __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-            for (int step = 0; step < NSTEP; step++) {
-#pragma unroll
-                for (int i = step * NL / NSTEP; i < (step + 1) * NL / NSTEP; i++) refill(i);
-                if (step + 1 < NSTEP) produce(step + 1, (step + 1) & 1);
-#pragma unroll
-                for (int nb = 0; nb < NB; nb++) {
-                    if (SA) // a K step is one group: its first MFMA starts from zero, so the fold below clears nothing
-                        accg[nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(aq[step & 1], bq[step & 1][nb],
-                                                                          step == 0 ? f16v{} : accg[nb], 0, 0, 0);
-                    else
-                        acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(aq[step & 1], bq[step & 1][nb], acc[nb], 0, 0, 0);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            __builtin_amdgcn_s_setprio(0);
-            if (SA && (u + 1) % KPG == 0) {
-                // end of a group: fold its partial sum into the result with the fp32 scale of each row
-                const int gb = (base / PW) & 1;
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const float4 sv = *reinterpret_cast<const float4 *>(&gsc[gb][u][wave * 32 + q * 8 + h * 4]);
-                    const float svv[4] = {sv.x, sv.y, sv.z, sv.w};
-#pragma unroll
-                    for (int nb = 0; nb < NB; nb++)
-#pragma unroll
-                        for (int e = 0; e < 4; e++)
-                            acc[nb][4 * q + e] = fmaf(svv[e], accg[nb][4 * q + e], acc[nb][4 * q + e]);
-                }
-                if (u == PW - 1) store_gs(base / PW + 1, gs2), store_zs(base / PW + 1, zs2); // fetched at the round's first step
-            }
-            // the next step's activation tile was fetched XP - 1 steps ago
-            store_x(buf ^ 1, xr[(u + 1) % XP]);
-            __syncthreads();
+        }
+        if (par == 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * XP + WL) : "memory"); // the next unit's weights
+        read_w(par, unit1); // of the step after the next: the same half of the next unit
+        if (par == 1) {
+            const uint32_t free = unit;
+            unit = unit1, unit1 = unit2, unit2 = free;
         }
     };
-    // Whole rounds of PW steps in the loop, the remaining steps straight-line after it: an exit from the
-    // middle of the unrolled body makes the compiler copy ring registers at the loop's end, and every copy
-    // waits for its load, which drains the prefetch once per round.
-    const int n_full = n_it / PW, n_rem = n_it - n_full * PW;
-    for (int bi = 0; bi < n_full; bi++) {
 #pragma unroll
-        for (int u = 0; u < PW; u++) k_step(bi * PW + u, u);
+    for (int i = 0; i < WL; i++) fetch_w(0, i);
+#pragma unroll
+    for (int i = 0; i < 2 * XP; i++) fetch_x(i / XP, i % XP);
+#pragma unroll
+    for (int i = 0; i < WL; i++) fetch_w(S::kUnit, i);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(WL) : "memory");
+    read_w(0, 0);
+    constants();
+#pragma unroll
+    for (int i = 0; i < 16; i++) dequant(0, i);
+    read_w(1, 0);
+#pragma unroll
+    for (int t = 0; t < 4; t++) read_x(0, t, 0);
+    int u = u0;
+    for (; u + 2 <= u1; u += 2) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) k_step(i);
     }
+    if (u < u1) k_step(0), k_step(1);
+    if (SA) {
 #pragma unroll
-    for (int u = 0; u < PW - 1; u++)
-        if (u < n_rem) k_step(n_full * PW + u, u);
+        for (int n = N0; n < NT; n++) fold(n, 0), fold(n, 1);
+    }
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory"); // the LDS is reused below
 
-    // C layout: lane (col n = l%32 -> token, h = l/32), register i -> row (i/4)*8 + h*4 + i%4.
-    // Stored as it stands, every store instruction would touch 64 separate 16-byte pieces; instead each
-    // wave turns its 32 rows x 32 tokens through LDS (the activation buffers are free now) so that a
-    // store instruction writes 8 tokens x 128 contiguous bytes.
+    // C layout: lane (column r = token, kg), register i -> row 4 kg + i.  Stored as it stands, every store instruction would
+    // touch 16 separate 64-byte pieces; instead each wave turns its 32 rows x 32 tokens through LDS (the activation buffers
+    // are free now) so that a store instruction writes 8 tokens x 128 contiguous bytes.
     const Q4Epi &E = L.e;
     // workspace of matrix mi starts after those of the matrices before it
     size_t ws_base = 0;
     for (int i = 0; i < mi; i++) ws_base += (size_t)KS * B * L.m[i].out;
-    const int obase = rb * 128 + wave * 32;
     constexpr int kTRow = 36; // floats per staged token row: 32 + 4 pad (16-byte reads of 8 lanes per token)
-    float *tile = reinterpret_cast<float *>(xs) + wave * 32 * kTRow; // 4.5 KB per wave
+    float *tile_o = reinterpret_cast<float *>(lds) + wave * 32 * kTRow; // 4.5 KB per wave
     const int tl = lane >> 3, oc = (lane & 7) * 4; // read-back map: token within a pass of 8, 4 rows
 #pragma unroll
     for (int nb = 0; nb < NB; nb++) {
 #pragma unroll
-        for (int q = 0; q < 4; q++)
-            *reinterpret_cast<float4 *>(&tile[r * kTRow + q * 8 + h * 4]) =
-                make_float4(acc[nb][4 * q + 0], acc[nb][4 * q + 1], acc[nb][4 * q + 2], acc[nb][4 * q + 3]);
+        for (int i = 0; i < 4; i++)
+            *reinterpret_cast<f4v *>(&tile_o[(i / 2 * 16 + r) * kTRow + i % 2 * 16 + kg * 4]) = acc[2 * nb + i / 2][i % 2];
         // the wave reads what the wave wrote: no block barrier, the LDS queue of a wave is in order
 #pragma unroll
         for (int pass = 0; pass < 4; pass++) {
             const int tt = pass * 8 + tl;
-            float4 v = *reinterpret_cast<const float4 *>(&tile[tt * kTRow + oc]);
+            float4 v = *reinterpret_cast<const float4 *>(&tile_o[tt * kTRow + oc]);
             const int t = t0 + nb * 32 + tt;
             const int o = obase + oc;
             if (t >= B || o >= n_out) continue;
             const size_t row = (size_t)t * n_out;
             if (KS > 1 || partials) { // partial tile of this K slice
-                *reinterpret_cast<float4 *>(ws + ws_base + ((size_t)ks * B + t) * n_out + o) = v;
+                float *at = ws + ws_base + ((size_t)ks * B + t) * n_out + o;
+                if (partials > 1) __builtin_nontemporal_store(f4v{v.x, v.y, v.z, v.w}, reinterpret_cast<f4v *>(at));
+                else *reinterpret_cast<float4 *>(at) = v;
                 continue;
             }
             const float scale_t = ss ? ss[t] : 1.0f;
@@ -404,78 +354,107 @@ __device__ __forceinline__ void q4_gemm_tile(const Q4Launch &L, const XhList &xh
     }
 }
 
-// A block takes 32 NB tokens.  The last tile of tokens takes 32, 64 or 96 where that is enough for those left: a tile costs
-// its whole width whatever is in it (70B prompt of 777 tokens, six tiles of 128 and one of 32 instead of seven of 128:
-// eight layers 18.2 -> 17.7 ms; what a narrow tile does not save is the dequantisation of its weights).
-template <int G, int NB, int KSTEP>
-__global__ __launch_bounds__(256, NB > 2 ? 2 : 1) void q4_gemm_kernel(const Q4Launch L, const XhList xh, const float *__restrict__ ss,
-                                                      float *__restrict__ ws, int KS, int t_tiles, int partials) {
-    __shared__ GemmLds S;
-    // blocks are dealt round-robin over the 8 XCDs: see q4_tile_gemm_kernel
-    const int n_blocks = gridDim.x, per_xcd = n_blocks >> 3, over = n_blocks & 7, xcd = blockIdx.x & 7;
-    const int work = xcd * per_xcd + min(xcd, over) + (blockIdx.x >> 3);
-    int rb = work / t_tiles;
-    const int t0 = (work - rb * t_tiles) * (32 * NB);
-    const int row_blocks = n_blocks / (t_tiles * KS), ks = rb / row_blocks; // K slice
-    rb -= ks * row_blocks;
-    if (NB > 1 && L.batch - t0 <= 32)
-        q4_gemm_tile<G, 1, KSTEP>(L, xh, ss, ws, KS, partials, rb, ks, t0, S);
-    else if (NB > 2 && L.batch - t0 <= 64)
-        q4_gemm_tile<G, NB < 2 ? NB : 2, KSTEP>(L, xh, ss, ws, KS, partials, rb, ks, t0, S);
-    else if (NB > 3 && L.batch - t0 <= 96)
-        q4_gemm_tile<G, NB < 3 ? NB : 3, KSTEP>(L, xh, ss, ws, KS, partials, rb, ks, t0, S);
+// One block per work item.  The first `whole` items are tiles of 32 NB tokens, K slice by K slice; the tiles of a last,
+// partly filled round of blocks follow in two halves; then the last tokens of every row block, where they need no more than
+// half a tile.  A tile costs its width in steps of 32 and the dequantisation of its weights (128, 64, 32 tokens of 70B's w1:
+// 119, 75, 62 us).
+template <int G, int NB, int NW>
+__global__ __launch_bounds__(64 * NW, NB > 2 ? 2 : 1) void q4_gemm_kernel(const Q4Launch L, const XhList xh, const float *__restrict__ ss,
+                                                      float *__restrict__ ws, int KS, int partials, int row_blocks, int t_full, int whole) {
+    // Blocks are dealt round-robin over the 8 XCDs, each with an L2 of its own: a contiguous range of items for each.
+    auto place = [](int b, int n) { const int per = n >> 3, over = n & 7, xcd = b & 7; return xcd * per + min(xcd, over) + (b >> 3); };
+    constexpr int TN = 32 * NB, CHUNK = 8;
+    const int tiles = row_blocks * t_full;
+    int item, half = -1, ks, rb, tt;
+    if ((int)blockIdx.x < whole) {
+        item = place(blockIdx.x, whole);
+    } else {
+        const int halves = 2 * (tiles * KS - whole);
+        item = place(blockIdx.x - whole, gridDim.x - whole);
+        if (item < halves) half = item & 1, item = whole + (item >> 1);
+        else item += tiles * KS - halves;
+    }
+    if (item < tiles * KS) { // 8 row blocks at a time, token tile by token tile: what runs on an XCD shares tiles and weights
+        ks = item / tiles, item -= ks * tiles;
+        const int c = item / (CHUNK * t_full), n = min(CHUNK, row_blocks - c * CHUNK);
+        item -= c * CHUNK * t_full;
+        tt = item / n, rb = c * CHUNK + item - tt * n;
+    } else {
+        item -= tiles * KS;
+        ks = item / row_blocks, rb = item - ks * row_blocks, tt = t_full;
+    }
+    const int t0 = tt * TN + (half > 0 ? TN / 2 : 0), n = half < 0 ? L.batch - t0 : min(L.batch - t0, TN / 2);
+    if (NB > 1 && n <= 32)
+        q4_gemm_tile<G, 1, NW>(L, xh, ss, ws, KS, partials, rb, ks, t0);
+    else if (NB > 2 && n <= 64)
+        q4_gemm_tile<G, NB < 2 ? NB : 2, NW>(L, xh, ss, ws, KS, partials, rb, ks, t0);
+    else if (NB > 3 && n <= 96)
+        q4_gemm_tile<G, NB < 3 ? NB : 3, NW>(L, xh, ss, ws, KS, partials, rb, ks, t0);
     else
-        q4_gemm_tile<G, NB, KSTEP>(L, xh, ss, ws, KS, partials, rb, ks, t0, S);
+        q4_gemm_tile<G, NB, NW>(L, xh, ss, ws, KS, partials, rb, ks, t0);
+}
+
+template <int G, int NB, int NW>
+int launch_gemm(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, int partials, hipStream_t st) {
+    constexpr int TN = 32 * NB;
+    int row_blocks = 0;
+    for (int i = 0; i < L.n_mats; i++) row_blocks += L.m[i].row_blocks = (L.m[i].out + 32 * NW - 1) / (32 * NW);
+    const int rest = L.batch % TN, t_full = L.batch / TN + (rest > TN / 2), narrow = rest > 0 && rest <= TN / 2;
+    const int tiles = row_blocks * t_full * s.slices;
+    int whole = tiles;
+    // halves where they and the narrow tiles fit one round: 7B's w1|w3, 511 tokens, 344 tiles on 256 CUs 123 -> 112 us; with
+    // 224 narrow tiles behind 64 left over (70B's, 776) they take 822 and whole tiles 804
+    if (NB == 4 && s.slices == 1 && 2 * (tiles % cu_count()) + narrow * row_blocks <= cu_count()) whole = tiles / cu_count() * cu_count();
+    // partial tiles past the caches where they would fill them: what a launch leaves dirty there is written back at its end
+    // (7B, 511 tokens: the four launches 13 us less per layer, their consumers 5 more; below 16 MB the other way round)
+    size_t bytes = 0;
+    for (int i = 0; i < L.n_mats; i++) bytes += (size_t)s.slices * L.batch * L.m[i].out * 4;
+    if (partials && bytes > ((size_t)16 << 20)) partials = 2;
+    const dim3 grid(whole + 2 * (tiles - whole) + narrow * row_blocks * s.slices), block(64 * NW);
+    // the tiles, or the output staging tiles of the epilogue (32 x 36 floats per wave)
+    const size_t lds = std::max(GemmLds<G, NW>::size(TN), (size_t)NW * 32 * 36 * sizeof(float));
+    static LdsLimit limit(48 * 1024);
+    L2_TRY(limit.ensure(reinterpret_cast<const void *>(q4_gemm_kernel<G, NB, NW>), lds));
+    hipLaunchKernelGGL((q4_gemm_kernel<G, NB, NW>), grid, block, lds, st, L, xh, ss, ws, s.slices, partials, row_blocks, t_full, whole);
+    L2_HIP(hipGetLastError());
+    return L2_OK;
 }
 
 template <int G>
 int launch_gemm_g(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, int partials, hipStream_t st) {
-    // K step: 128 where a group is at least that long (half the block barriers per k), else 64
-    constexpr int KSTEP = G >= 128 ? 128 : 64;
-    for (int i = 0; i < L.n_mats; i++) L.m[i].row_blocks = (L.m[i].out + 127) / 128;
-    const int TN = s.tokens, t_tiles = (L.batch + TN - 1) / TN;
-    const dim3 grid(s.row_blocks * t_tiles * s.slices), block(256);
-    // the activation buffers, or the four output staging tiles of the epilogue (32 x 36 floats per wave)
-    const size_t lds = std::max((size_t)2 * TN * (KSTEP + kXPad) * sizeof(_Float16), (size_t)4 * 32 * 36 * sizeof(float));
-    switch (TN) {
-        case 32: hipLaunchKernelGGL((q4_gemm_kernel<G, 1, KSTEP>), grid, block, lds, st, L, xh, ss, ws, s.slices, t_tiles, partials); break;
-        case 64: hipLaunchKernelGGL((q4_gemm_kernel<G, 2, KSTEP>), grid, block, lds, st, L, xh, ss, ws, s.slices, t_tiles, partials); break;
-        case 128:
-            if constexpr (G >= 64) {
-                static LdsLimit limit(48 * 1024);
-                L2_TRY(limit.ensure(reinterpret_cast<const void *>(q4_gemm_kernel<G, 4, KSTEP>), lds));
-                hipLaunchKernelGGL((q4_gemm_kernel<G, 4, KSTEP>), grid, block, lds, st, L, xh, ss, ws, s.slices, t_tiles, partials);
-                break;
-            }
-            [[fallthrough]];
-        default: return l2_fail(L2_ERR_ARG, "q4 gemm: token tile");
+    switch (s.tokens) {
+        case 32: return launch_gemm<G, 1, 4>(L, xh, ss, ws, s, partials, st);
+        case 64: return launch_gemm<G, 2, 4>(L, xh, ss, ws, s, partials, st);
+        case 128: return launch_gemm<G, 4, 8>(L, xh, ss, ws, s, partials, st);
     }
-    L2_HIP(hipGetLastError());
-    return L2_OK;
+    return l2_fail(L2_ERR_ARG, "q4 gemm: token tile");
 }
 
 } // namespace
 
 GemmShape gemm_shape_f16(const Q4Launch &L, int slice_batch) {
     GemmShape s{};
-    const int B = L.batch, G = L.group_size;
+    const int B = L.batch;
     s.rows = 128;
     for (int i = 0; i < L.n_mats; i++) s.row_blocks += (L.m[i].out + 127) / 128;
-    // Up to 255 tokens a wave takes 64 of them: with 128 a chunk of 128 tokens is too few blocks for the chip
-    // (w1|w3 of 7B: 172 blocks on 256 CUs; the launches of a 128-token chunk are 7 % slower that way).  From
-    // 256 tokens on a wave takes 128 (within 256 registers: two blocks per CU): every weight is dequantised
-    // once per 128 tokens instead of twice, and there are blocks enough whatever the tile (w1|w3 of 7B at 512
-    // tokens: 115 against 129 us).
-    auto tile = [&](int n) { return G >= 64 && n >= 256 ? 128 : n > 32 ? 64 : 32; };
-    s.tokens = tile(B);
-    // K slices: as many as keep the grid within one round of 2 blocks per CU, whole groups per slice, at most 4.
-    // (Up to 8 fill the chip when a launch runs alone, but every slice is a partial tile that the consumer reads
-    // back: 34.4 k against 32.7 k tok/s on the 7B prompt, 19.9 k against 19.5 k on 13B, no change on 70B.)
-    const int kstep = G >= 128 ? 128 : 64;
-    const int n_grp = (L.in / kstep) / (G / kstep > 0 ? G / kstep : 1);
+    // K slices: as many as keep the grid within one round of 2 blocks per CU, of two units or more, at most 4; chunks of up
+    // to 64 tokens, whose partial tiles are small, at most 8.  (More slices fill the chip when a launch runs alone, but every
+    // one is a partial tile that the consumer reads back.  8 for 4, 32 tokens: two layers of 7B, group 128, 226 -> 202 us, of
+    // 70B, group 64, 492 -> 450; 16: 210 and 456.)  They depend on the chunk and not on the pass: its bits must not.
+    auto tile = [](int n) { return n >= 192 ? 128 : n > 32 ? 64 : 32; };
     const int t_tiles = (slice_batch + tile(slice_batch) - 1) / tile(slice_batch);
-    // slices start on even groups
-    s.slices = std::max(1, std::min({2 * cu_count() / (s.row_blocks * t_tiles), 4, n_grp / 2}));
+    s.slices = std::max(1, std::min({2 * cu_count() / (s.row_blocks * t_tiles), slice_batch <= 64 ? 8 : 4, L.in / 256}));
+    // From 192 tokens on a block is 256 rows x 128 tokens, one per CU (every weight is dequantised once per 128 tokens instead
+    // of twice, every token tile read once per 256 rows), where that gives work to at least half the CUs; below, or for a small
+    // model, 128 rows x 64 tokens, two or three blocks per CU.  Two layers, 256 x 128 / 128 x 64, us: 7B, group 128, 192 tokens
+    // 401 / 395, 250 431 / 450, 511 669 / 768; 13B 192 507 / 521; 70B, group 64, 250 1314 / 1371; dim 1024, 511 233 / 217.
+    s.tokens = tile(B);
+    if (s.tokens == 128) {
+        int rows = 0;
+        for (int i = 0; i < L.n_mats; i++) rows += (L.m[i].out + 255) / 256;
+        if (rows * ((B + 127) / 128) * s.slices >= cu_count() / 2) s.rows = 256, s.row_blocks = rows;
+        else s.tokens = 64;
+    }
     return s;
 }
 

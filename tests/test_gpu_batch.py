@@ -168,6 +168,30 @@ def test_fp16_operator_last_tile(ops, G, batches):
     m.close()
 
 
+# fp16 prompts in blocks of 256 rows: token tiles of every width, tiles left over in halves, with and without narrow ones
+# behind them, one, two and three units of K, a last row block that is not full, rows of one matrix only
+@pytest.mark.parametrize("dim,hidden,G,batches", [
+    (256, 11008, 64, (890, 788, 800)), (256, 11136, 32, (257, 788)), (128, 22016, 64, (511,)), (384, 11008, 64, (520,)),
+    (512, 11264, 128, (890, 430, 224)), (1024, 2816, 32, (300, 511))])
+def test_fp16_operator_wide_blocks(ops, dim, hidden, G, batches):
+    from llama2_rs import _lib
+    dims = ck.Dims(dim=dim, hidden_dim=hidden, n_layers=1, n_heads=dim // 128, n_kv_heads=dim // 128, vocab_size=64, seq_len=1024,
+                   group_size=G)
+    m = ops.Model(ck.synth_weights_image(dims, seed=9), dims)
+    for B in batches:
+        # inputs that fp16 holds: with groups of 64 and 128 nothing is rounded but the fp32 sums.  With groups of 32 every weight
+        # is, twice to 2^-12 of itself at most: the sum's error is 4e-4 of its rms, and 4e-3 ten times that
+        x = np.random.default_rng(B).standard_normal((B, dim)).astype(np.float16).astype(np.float32)
+        m.set_prefill_mode(_lib.PREFILL_FP32)
+        want = m.qmatvec(0, _lib.W1, x)
+        m.set_prefill_mode(_lib.PREFILL_MFMA)
+        got = m.qmatvec(0, _lib.W1, x)
+        assert not np.array_equal(got, want)
+        for b in range(B):
+            assert nrel(got[b], want[b]) < (4e-3 if G == 32 else 2e-5), (B, b)
+    m.close()
+
+
 # prompt attention with two sets of columns per block (two blocks per compute unit and more), the last block with one
 # set, and grids of one to two blocks per unit, whose tiles go in pairs, against passes too short for either
 @pytest.mark.parametrize("n_heads,n_kv,n", [(32, 32, 505), (16, 2, 1021), (32, 32, 200), (32, 32, 250), (16, 16, 300)])
