@@ -6,23 +6,23 @@
 //
 // fp32 activations, exactly: x = b0 + b1 + b2 with three bf16 numbers of 8 significant bits each, obtained by cutting x
 // after its first, second and third byte of significand.  The weights are integers n - z1 of at most five bits, exact in
-// bf16, and so is every product that enters the fp32 accumulator (v_mfma_f32_32x32x16_bf16).  What is left is the sums:
-//   - The matrix unit's sum of 16 products and the accumulator is not rounded to nearest; it comes out too small on
-//     average, whatever its sign.  Left alone that adds up over K (28672 inputs in groups of 32: mean error -1.7e-7 of
-//     the result's rms).  So every other group enters negated, weights and scale: the mean is below 1e-9.
+// bf16, and so is every product that enters the fp32 accumulator (v_mfma_f32_16x16x32_bf16).  What is left is the sums:
+//   - The matrix unit's sum of products and accumulator is not rounded to nearest; it comes out too small on average, whatever
+//     its sign.  So every other group enters negated, weights and scale: the mean is below 1e-9.
 //   - Of the three planes of a step the smallest is added first.
-//   - The fp32 group scale is applied to the fp32 sum of each group, and these are added in runs of at most kRunGroups,
-//     the runs to each other, the slices of K in a tree: the error of a chain grows with its length.
-// Relative rms error against fp64 over 1024..28672 inputs, 8..512 columns, normal inputs: 0.49 to 0.95 of that of the
-// matvec (kernels_q4_stream.hip) in every group size; inputs all of one sign, where the matvec is better than elsewhere,
-// 0.42 to 1.36 (the largest at 4096 inputs in groups of 32, 512 columns).  One chain, largest plane first, no negation:
-// 0.60 to 1.91 and 0.59 to 2.30.
+//   - The fp32 group scale is applied to the fp32 sum of each group, and these are added in runs of 8 to 16 groups, the runs to
+//     each other, the slices of K in a tree: the error of a chain grows with its length.
+// Relative rms error against fp64 over 1024..28672 inputs, 8..512 columns, of that of the matvec (kernels_q4_stream.hip): normal
+// inputs 0.45 to 0.74, inputs all of one sign, where the matvec is better than elsewhere, 0.39 to 1.06 (1024 inputs, group 128).
 //
 // Against the matvec kernels run once per column, which read and dequantise the weights for each of them: 4096x11008,
-// group 32, 61 columns 330 -> 40.4 us with everything around it; a 298-token prompt on 7B 230 -> 15.1 ms.
+// group 32, 61 columns 330 -> 35.0 us with everything around it.  Against the form before this one (activations and weights
+// through registers, 32x32x16 tiles, two blocks of four waves per CU): that call 40.3 us; 16 columns of 13824x5120 33.7 -> 26.3;
+// two layers of 7B, group 128, 16, 64, 299 columns 280 / 365 / 967 -> 222 / 328 / 930; 70B, group 64, 16 and 299 763 / 3593 ->
+// 544 / 3350.
 #include <algorithm>
 
-#include "l2_internal.h"
+#include "gemm_lds.h"
 
 namespace {
 
@@ -45,27 +45,16 @@ __device__ __forceinline__ T ld_at(const void *base, uint32_t byte_offset) {
     return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + byte_offset);
 }
 
-// bf16: sign (n - z1) 2^-9 in the order (0,2,4,6,1,3,5,7).  A nibble in the low half of a byte is n 2^-9 as an OCP E4M3
-// number; two at a time become fp32, the zero point is subtracted there, and the upper halves of two results are the
-// bf16 pair (the integers have at most five bits: nothing is cut off).
+// bf16: sign (n - z1) in the order (0,2,4,6,1,3,5,7).  A nibble in the low half of a byte is n 2^-9 as an OCP E4M3 number; two
+// at a time become fp32, one FMA each makes sign (n - z1) of it, and the upper halves of two results are the bf16 pair (the
+// integers have at most five bits: nothing is cut off).
 struct Dequant {
-    float sign, z; // sign: 1 or -1
-    static constexpr float kUnit = 0.001953125f; // 2^-9: value of the integer 1
-    __device__ __forceinline__ Dequant(int zn, float sg) : sign(sg), z((float)(zn + 1) * (-kUnit * sg)) {}
-    __device__ __forceinline__ uint32_t pair(v2f v) const {
-        return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, fmaf(v.y, sign, z)), __builtin_bit_cast(uint32_t, fmaf(v.x, sign, z)), 0x07060302u);
-    }
-    __device__ __forceinline__ Frag operator()(uint32_t w) const {
-        const uint32_t l = w & 0x0F0F0F0Fu, h = (w >> 4) & 0x0F0F0F0Fu;
-        Frag f;
-        f.u[0] = pair(__builtin_amdgcn_cvt_pk_f32_fp8(l, false));
-        f.u[1] = pair(__builtin_amdgcn_cvt_pk_f32_fp8(l, true));
-        f.u[2] = pair(__builtin_amdgcn_cvt_pk_f32_fp8(h, false));
-        f.u[3] = pair(__builtin_amdgcn_cvt_pk_f32_fp8(h, true));
-        return f;
-    }
-    static __device__ __forceinline__ f16v mfma(const Frag &a, const Frag &b, f16v c) {
-        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.b, b.b, c, 0, 0, 0);
+    float unit, z; // +-2^9, -+z1
+    __device__ __forceinline__ void set(int zn, float sign) { unit = 512.0f * sign, z = (float)(zn + 1) * -sign; }
+    // pair i of a word; i = 2 and 3 of the word shifted by 4
+    __device__ __forceinline__ uint32_t pair(uint32_t masked, int i) const {
+        const v2f v = i % 2 == 0 ? __builtin_amdgcn_cvt_pk_f32_fp8(masked, false) : __builtin_amdgcn_cvt_pk_f32_fp8(masked, true);
+        return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, fmaf(v.y, unit, z)), __builtin_bit_cast(uint32_t, fmaf(v.x, unit, z)), 0x07060302u);
     }
 };
 
@@ -162,274 +151,304 @@ __device__ __forceinline__ void finish4(const Q4Launch &L, int mi, const float *
     *reinterpret_cast<float4_any *>(L.m[mi].y + at) = float4_any{v.x, v.y, v.z, v.w};
 }
 
-constexpr int kRowHalves = 72; // halves per staged token row: 64 k + 8 (16-byte reads of 32 lanes stay conflict-free)
+// LDS of a block of NW waves: three activation tiles of 64 k (three planes of 16 NT tokens), and for each wave three units of
+// 128 k of its 32 rows' weights, scales and zero points.
+template <int G, int NT, int NW>
+struct TileLds {
+    static constexpr int kPlane = 16 * NT * kStepRow, kTile = 3 * kPlane;
+    static constexpr int kGroupLoads = G == 32 ? 2 : 1; // of 64 scales (zero points) per unit
+    static constexpr int kWeights = 32 * 64, kScales = 256 * kGroupLoads;
+    static constexpr int kUnit = kWeights + 2 * kScales;
+    static constexpr size_t kSize = 3 * (size_t)kTile + (size_t)NW * 3 * kUnit;
+};
 
-// A block is four waves side by side over the output rows, each with MT x NB tiles of 32 rows x 32 tokens, all of them
-// on the same tokens: the activation tile (64 k) is staged in LDS once per block, double-buffered, and every 16 bytes a
-// lane reads from it feed MT MFMAs.  (The LDS gives a compute unit some 150 B/ns: with MT = 1 the reads of the tile
-// would hold the matrix pipes below 60 %.)  Weights are dequantised in registers, NB * NP times used.
+// A wave owns 32 rows x 16 NT tokens, in tiles of 16 x 16 (v_mfma_f32_16x16x32_bf16); a block is NW waves side by side over the
+// rows, on the same tokens.  What the K loop reads comes through LDS past the registers, as in the fp16 kernel
+// (kernels_q4_gemm.hip, which explains the layout and the waits): tiles of 64 k two steps ahead, weights two units.  One
+// barrier per step; a step is 6 NT pairs of MFMAs, with the dequantisation of the next one's weights and the folds of finished
+// groups spread between them: some 230 instructions for 64 tokens, which the two waves of a SIMD issue at one per 4.9 cycles
+// (2546 cycles per step of 7B's w1|w3 at 299 tokens, 1536 of them MFMAs).  Eight waves and 64 tokens take 133 KB of LDS, one
+// block per CU; four waves and 16 or 32 tokens, where weights are what is read, two or three.
 //
-// Lane (r = l % 32, h = l / 32) of a 32-row tile.  G >= 64: the lane loads inputs 32 h .. 32 h + 31 of every 64 of its
-// row, MFMA step s takes word s.  G = 32: an MFMA step must stay inside one group, so the lane loads both groups of the
-// 64 and step s takes word 2 (s % 2) + h of group s / 2.
-template <int G, int MT, int NB>
-__global__ __launch_bounds__(256, 2) void q4_tile_gemm_kernel(const Q4Launch L, const XhList xl, int in_p,
-                                                              const float *__restrict__ ss, float *__restrict__ ws, int KS,
-                                                              int t_tiles, int partials) {
-    constexpr int NP = 3, TN = 32 * NB, RW = 32 * MT, RB = 4 * RW;
+// Lane (r = l % 16, kg = l / 16).  G >= 64: the lane's words of a step are 2 kg and 2 kg + 1, MFMA k takes one each.  G = 32: an
+// MFMA must stay inside one group, so its words are kg and 4 + kg.
+template <int G, int NT, int NW>
+__device__ __forceinline__ void q4_tile(const Q4Launch &L, const XhList &xl, int in_p, const float *__restrict__ ss, float *__restrict__ ws,
+                                        int KS, int partials, int rb, int ks, int t0) {
+    using S = TileLds<G, NT, NW>;
+    constexpr int NP = 3, TN = 16 * NT, RB = 32 * NW;
     constexpr int KPG = G >= 64 ? G / 64 : 1; // K steps per group
     constexpr int GPS = G >= 64 ? 1 : 64 / G; // groups per K step
-    constexpr int WL = G >= 64 ? 1 : 2;       // 16-byte loads of weights per lane, row tile and K step
-    constexpr int PIECES = NP * NB;           // 16-byte pieces of the activation tile per thread
-    // K steps that weights are requested ahead (the activations: one): a step is 12 MT NB MFMAs, which cover the way
-    // from memory; more would cost the registers of the second block per CU.
-    constexpr int WR = 2, PW = 2;
-    extern __shared__ __align__(16) uint16_t xs[]; // [2][NP][TN][kRowHalves]
-    __shared__ float gsc[2][GPS][RB]; // scales of the group(s) of this K step and the next
-    // Blocks are dealt round-robin over the 8 XCDs, each with an L2 of its own.  An XCD gets a contiguous range of the
-    // work, all token tiles of a row block one behind the other: what runs on it at one time shares a few row blocks'
-    // weights and the tiles' activations.
-    const int n_blocks = gridDim.x, per_xcd = n_blocks >> 3, over = n_blocks & 7, xcd = blockIdx.x & 7;
-    const int work = xcd * per_xcd + min(xcd, over) + (blockIdx.x >> 3);
-    int rb = work / t_tiles, mi = 0;
-    const int t0 = (work - rb * t_tiles) * TN;
-    const int row_blocks = n_blocks / (t_tiles * KS), ks = rb / row_blocks;
-    rb -= ks * row_blocks;
+    extern __shared__ __align__(16) char lds[];
+    int mi = 0;
     while (mi + 1 < L.n_mats && rb >= L.m[mi].row_blocks) {
         rb -= L.m[mi].row_blocks;
         mi++;
     }
-    // in registers for good: the loop must not ask for kernel arguments again
-    const void *__restrict__ const xh = xl.p[mi];
-    const void *__restrict__ const qw = L.m[mi].qweight;
-    const void *__restrict__ const qz = L.m[mi].qzeros;
-    const void *__restrict__ const qs = L.m[mi].scales;
-    asm volatile("" ::"s"(xh), "s"(qw), "s"(qz), "s"(qs));
-    const int n_out = L.m[mi].out, groups = L.groups, B = L.batch, C4 = L.in >> 5;
+    const int n_out = L.m[mi].out, groups = L.groups, B = L.batch, in = L.in;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int r = lane & 31, h = lane >> 5;
+    const int r = lane & 15, kg = lane >> 4;
+    const int obase = rb * RB + wave * 32;
     // this block's slice of K, in whole groups and whole K steps
     const int n_unit = in_p / (64 * KPG);
-    const int it0 = (int)((long)n_unit * ks / KS) * KPG, it1 = (int)((long)n_unit * (ks + 1) / KS) * KPG;
+    const int it0 = (int)((long)n_unit * ks / KS) * KPG, it1 = (int)((long)n_unit * (ks + 1) / KS) * KPG, n_it = it1 - it0;
 
-    const int obase = rb * RB + wave * RW;
-    uint32_t wrow[MT], zrow[MT]; // byte offsets of the lane's rows
-    int zsh[MT];
+    const uint32_t lds0 = lds_offset(lds), wave_at = 3 * S::kTile + wave * 3 * S::kUnit;
+    const u4v xbuf = biased_buffer(xl.p[mi], (size_t)B * NP * in_p * 2), wbuf = biased_buffer(L.m[mi].qweight, (size_t)n_out * (in >> 1));
+    const u4v sbuf = biased_buffer(L.m[mi].scales, (size_t)n_out * groups * 4), zbuf = biased_buffer(L.m[mi].qzeros, (size_t)(n_out >> 3) * groups * 4);
+    constexpr int PIECES = NP * 2 * NT, XP = (PIECES + NW - 1) / NW; // 1 KB pieces of a tile: 8 tokens of a plane
+    static_assert(XP <= 4, "the instruction's own offset has 12 bits");
+    const int xfirst = min(wave * XP, PIECES - XP);
+    uint32_t xoff[XP], woff[2];
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) {
-        const int o = min(obase + mt * 32 + r, n_out - 1);
-        wrow[mt] = (uint32_t)(o * C4) << 4;
-        zrow[mt] = (uint32_t)((o >> 3) * groups) << 2;
-        zsh[mt] = 4 * (o & 7);
+    for (int i = 0; i < XP; i++) {
+        const int p = (xfirst + i) / (2 * NT), t = (xfirst + i) % (2 * NT) * 8 + (lane >> 3);
+        xoff[i] = ((uint32_t)min(t0 + t, B - 1) * NP + p) * (uint32_t)in_p * 2u + (((lane & 7) ^ ((t >> 1) & 7)) << 4) + kBias - i * 1024;
     }
-    const uint32_t srow = (uint32_t)(min(rb * RB + (tid & (RB - 1)), n_out - 1) * groups) << 2;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const int row = i * 16 + (lane >> 2);
+        woff[i] = (uint32_t)min(obase + row, n_out - 1) * (uint32_t)(in >> 1) + (((lane & 3) ^ ((row >> 2) & 3)) << 4) + kBias - i * 1024;
+    }
+    const int srow = min(obase + (lane & 31), n_out - 1), lane_group = G == 128 ? 0 : lane >> 5;
+    const uint32_t soff = (uint32_t)(srow * groups) * 4u + kBias - S::kWeights, zoff = (uint32_t)((srow >> 3) * groups) * 4u + kBias - S::kWeights - S::kScales;
+    uint32_t xr[2]; // where the lane reads a token's piece of MFMA k
+#pragma unroll
+    for (int k = 0; k < 2; k++) xr[k] = (uint32_t)r * kStepRow + (((G == 32 ? 4 * k + kg : 2 * kg + k) ^ ((r >> 1) & 7)) << 4);
+    // ... and its words of a unit's first step (the second's: ^ 32)
+    const int wsw = (r >> 2) & 3;
+    const uint32_t wr0 = wave_at + r * 64 + (G == 32 ? (wsw << 4) + kg * 4 : (((kg >> 1) ^ wsw) << 4) + (kg & 1) * 8);
+    const uint32_t sr = wave_at + S::kWeights + kg * 16, zr = wave_at + S::kWeights + S::kScales + r * 4;
+    const int zsh = 4 * (r & 7);
 
-    struct WStage {
-        uint4 w[MT][WL];
-        int32_t z[MT][GPS];
+    const uint32_t x_last = (uint32_t)(it1 - 1) * 128;
+    uint32_t x_at = (uint32_t)it0 * 128, w_at = (uint32_t)it0 * 32; // what is requested next (requests past the slice's end are never read)
+    auto fetch_x = [&](uint32_t tile, const int i) __attribute__((always_inline)) {
+        LDS_TO(lds0 + tile + xfirst * 1024);
+        LDS_LOAD("x4", i * 1024, xbuf, xoff[i], x_at);
+        if (i == XP - 1) x_at = min(x_at + 128, x_last);
     };
-    auto fetch_w = [&](int it, WStage &d) __attribute__((always_inline)) {
-        const int c = min(it, it1 - 1);
+    constexpr int WL = 2 + 2 * S::kGroupLoads;
+    auto fetch_w = [&](uint32_t unit, const int i) __attribute__((always_inline)) {
+        LDS_TO(lds0 + wave_at + unit);
+        if (i < 2) {
+            LDS_LOAD("x4", i * 1024, wbuf, woff[i], w_at);
+        } else { // in % 64 = 32: the last step's second group is the first one again (its inputs are zero)
+            const uint32_t g = min(w_at * 2 / G + lane_group + (i >= 4 ? 2 : 0), (uint32_t)groups - 1) * 4;
+            if (i == 2) LDS_LOAD("", S::kWeights, sbuf, soff + g, 0);
+            else if (i == 3) LDS_LOAD("", S::kWeights + S::kScales, zbuf, zoff + g, 0);
+            else if (i == 4) LDS_LOAD("", S::kWeights + 256, sbuf, soff - 256 + g, 0);
+            else LDS_LOAD("", S::kWeights + S::kScales + 256, zbuf, zoff - 256 + g, 0);
+        }
+        if (i == WL - 1) w_at += 64;
+    };
+
+    f4v top[NT][2], acc[NT][2], accg[NT][2]; // sums of the runs, of the current run, of the current group; two tiles of 16 rows
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++) {
+    for (int n = 0; n < NT; n++)
 #pragma unroll
-            for (int i = 0; i < WL; i++) // past the row's end (in % 64 = 32) the last chunk again: its inputs are zero
-                d.w[mt][i] = ld_at<uint4>(qw, wrow[mt] + ((uint32_t)min(2 * c + (WL == 1 ? h : i), C4 - 1) << 4));
+        for (int m = 0; m < 2; m++) top[n][m] = acc[n][m] = accg[n][m] = f4v{0.f, 0.f, 0.f, 0.f};
+    f4v sv[GPS][2]; // scales of the group(s) that accg holds
+#pragma unroll
+    for (int g = 0; g < GPS; g++) sv[g][0] = sv[g][1] = f4v{0.f, 0.f, 0.f, 0.f};
+    float sign = 1.0f; // G = 128: of this unit's group (every other group enters negated, weights and scale)
+    auto negated = [](int par, int k) { return G == 32 ? k == 1 : G == 64 && par == 1; };
+
+    Dequant dq[GPS][2];
+    Frag aq[2][2][2]; // weights of this step and the next: [rows][k]
+    uint32_t wd[2][2]; // packed weights of the next step
+    int zw[GPS][2];
+    Frag bq[4][NP];    // activations of four tiles of tokens
+    auto read_w = [&](const int par, uint32_t unit) __attribute__((always_inline)) {
+#pragma unroll
+        for (int m = 0; m < 2; m++) {
+            if constexpr (G == 32) {
+#pragma unroll
+                for (int k = 0; k < 2; k++) // piece 2 par + k of the row
+                    wd[m][k] = *reinterpret_cast<const uint32_t *>(lds + (wr0 ^ ((2 * par + k) * 16)) + unit + m * 1024);
+            } else {
+                const uint2 v = *reinterpret_cast<const uint2 *>(lds + (wr0 ^ (par * 32)) + unit + m * 1024);
+                wd[m][0] = v.x, wd[m][1] = v.y;
+            }
 #pragma unroll
             for (int g = 0; g < GPS; g++)
-                d.z[mt][g] = ld_at<int32_t>(qz, zrow[mt] + ((uint32_t)min(c * GPS / KPG + g, groups - 1) << 2));
+                if (G != 128 || par == 0)
+                    zw[g][m] = *reinterpret_cast<const int *>(lds + zr + unit + (G == 128 ? 0 : (par * GPS + g) * 128) + m * 64);
         }
     };
-    struct XStage {
-        uint4 v[PIECES];
+    auto constants = [&](const int par, float sg) __attribute__((always_inline)) { // of a step with this parity
+#pragma unroll
+        for (int g = 0; g < GPS; g++)
+#pragma unroll
+            for (int m = 0; m < 2; m++) dq[g][m].set((zw[g][m] >> zsh) & 15, G == 128 ? sg : negated(par, g) ? -1.0f : 1.0f);
     };
-    uint32_t xoff[NB];
-#pragma unroll
-    for (int p = 0; p < NB; p++) {
-        const int idx = p * 256 + tid;
-        xoff[p] = ((uint32_t)min(t0 + (idx >> 3), B - 1) * (uint32_t)(NP * in_p) + (idx & 7) * 8) * 2u;
-    }
-    auto fetch_x = [&](int it, XStage &d) __attribute__((always_inline)) {
-        const uint32_t kb = (uint32_t)min(it, it1 - 1) * 128u;
-#pragma unroll
-        for (int q = 0; q < NP; q++)
-#pragma unroll
-            for (int p = 0; p < NB; p++) d.v[q * NB + p] = ld_at<uint4>(xh, xoff[p] + kb + (uint32_t)(q * in_p) * 2u);
+    uint32_t masked = 0;
+    auto dequant = [&](const int to, const int i) __attribute__((always_inline)) { // piece i of 16
+        const int m = i >> 3, k = (i >> 2) & 1;
+        if (i % 4 == 0) masked = wd[m][k] & 0x0F0F0F0Fu;
+        if (i % 4 == 2) masked = (wd[m][k] >> 4) & 0x0F0F0F0Fu;
+        aq[to][m][k].u[i % 4] = dq[G == 32 ? k : 0][m].pair(masked, i % 4);
     };
-    auto store_x = [&](int buf, const XStage &d) __attribute__((always_inline)) {
+    // Tile t of a step: tokens n = t % NT, MFMA k = t / NT.  Its group, if it ended there, is folded LAG tiles later.
+    constexpr int T = 2 * NT, AHEAD = T < 3 ? T : 3, LAG = NT < 2 ? 1 : 2;
+    auto read_x = [&](const int par, const int t, uint32_t tile) __attribute__((always_inline)) {
 #pragma unroll
-        for (int q = 0; q < NP; q++)
+        for (int p = 0; p < NP; p++)
+            bq[(par * T + t) % 4][p].q = *reinterpret_cast<const uint4 *>(lds + xr[t / NT] + tile + p * S::kPlane + t % NT * 16 * kStepRow);
+    };
+    auto fold = [&](const int par, const int t) __attribute__((always_inline)) { // tile t of a step of this parity
+        const int n = t % NT, k = t / NT;
+        if (!(G == 32 || (k == 1 && (G == 64 || par == 1)))) return;
 #pragma unroll
-            for (int p = 0; p < NB; p++) {
-                const int idx = p * 256 + tid;
-                *reinterpret_cast<uint4 *>(xs + ((size_t)(buf * NP + q) * TN + (idx >> 3)) * kRowHalves + (idx & 7) * 8) = d.v[q * NB + p];
+        for (int m = 0; m < 2; m++) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float s = sv[G == 32 ? k : 0][m][e];
+                acc[n][m][e] = fmaf(negated(par, k) ? -s : s, accg[n][m][e], acc[n][m][e]);
             }
+            asm volatile("" : "+v"(acc[n][m])); // here, and not where the compiler would rather have it
+        }
     };
-    // scales of the group(s) that start with K step it, one row per thread; negative for the groups that enter negated
-    auto negated = [](int slot, int g) __attribute__((always_inline)) { return (G < 64 ? g : slot) != 0; };
-    auto fetch_s = [&](int it, float (&d)[GPS]) __attribute__((always_inline)) {
+    uint32_t tile = 0, tile1 = S::kTile, tile2 = 2 * S::kTile; // this step's tile, the next one's, the one after it
+    uint32_t unit = 0, unit1 = S::kUnit, unit2 = 2 * S::kUnit;
+    auto k_step = [&](const int par) __attribute__((always_inline)) {
+        if (G != 128 || par == 1) constants(par ^ 1, -sign); // of the next step
 #pragma unroll
-        for (int g = 0; g < GPS; g++) d[g] = ld_at<float>(qs, srow + ((uint32_t)min(it * GPS / KPG + g, groups - 1) << 2));
-    };
-    auto store_s = [&](int slot, const float (&d)[GPS]) __attribute__((always_inline)) {
+        for (int t = 0; t < T; t++) {
+            const int n = t % NT, k = t / NT;
+            if (t == T - AHEAD) {
+                // The next tile: what this wave requested of it has landed, then what everybody has; and all reads of this one
+                // have come back: its place is the next request's.
+                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(XP + (par == 1 ? WL : 0)) : "memory");
+            }
+            const int behind = (t + AHEAD) % T; // tiles since the barrier: the wave that is behind goes first
+            if (T >= 4 && behind % (T / 4) == 0) asm volatile("s_setprio %0" ::"n"(3 - behind * 4 / T));
+            read_x(t + AHEAD < T ? par : par ^ 1, (t + AHEAD) % T, t + AHEAD < T ? tile : tile1);
+            fold(t < LAG ? par ^ 1 : par, (t + T - LAG) % T);
+            const bool fresh = G == 32 || (k == 0 && (G == 64 || par == 0));
 #pragma unroll
-        for (int g = 0; g < GPS; g++) gsc[slot][g][tid & (RB - 1)] = d[g] * (negated(slot, g) ? -1.0f / Dequant::kUnit : 1.0f / Dequant::kUnit);
-    };
-
-    f16v acc[MT][NB], accg[MT][NB];
+            for (int p = NP - 1; p >= 0; p--)
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++)
+                for (int m = 0; m < 2; m++)
+                    accg[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(aq[par][m][k].b, bq[(par * T + t) % 4][p].b,
+                                                                         fresh && p == NP - 1 ? f4v{} : accg[n][m], 0, 0, 0);
 #pragma unroll
-        for (int nb = 0; nb < NB; nb++)
+            for (int i = t * 16 / T; i < (t + 1) * 16 / T; i++) dequant(par ^ 1, i);
+            if (G == 32 ? t % NT == 0 : (t == NT && (G == 64 || par == 1))) { // scales of the group that ends with these tiles
 #pragma unroll
-            for (int i = 0; i < 16; i++) acc[mt][nb][i] = 0.f;
-
-    WStage wr[WR];
-    XStage xr;
-    float sr[GPS];
-    fetch_s(it0, sr);
-    fetch_x(it0, xr);
-#pragma unroll
-    for (int j = 0; j < WR; j++) fetch_w(it0 + j, wr[j]);
-    store_s(0, sr);
-    store_x(0, xr);
-    __syncthreads();
-
-    // One K step; u = its number within a round of PW (slots of the rings and buffers, known where it is called).
-    auto k_step = [&](const int it, const int u) __attribute__((always_inline)) {
-        const int gpar = KPG == 2 ? ((it - it0) >> 1) & 1 : u; // buffer of this group's scales
-        const bool first = KPG == 1 || u == 0, last = KPG == 1 || u == 1;
-        fetch_x(it + 1, xr);
-        if (first) fetch_s(it + KPG, sr);
-        uint32_t wd[MT][4];
-        int zw[MT][GPS];
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++) {
-            if constexpr (WL == 1) {
-                wd[mt][0] = wr[u].w[mt][0].x, wd[mt][1] = wr[u].w[mt][0].y, wd[mt][2] = wr[u].w[mt][0].z, wd[mt][3] = wr[u].w[mt][0].w;
-            } else {
-#pragma unroll
-                for (int i = 0; i < 2; i++) {
-                    wd[mt][2 * i] = h ? wr[u].w[mt][i].y : wr[u].w[mt][i].x;
-                    wd[mt][2 * i + 1] = h ? wr[u].w[mt][i].w : wr[u].w[mt][i].z;
+                for (int m = 0; m < 2; m++) {
+                    sv[G == 32 ? k : 0][m] = *reinterpret_cast<const f4v *>(lds + sr + unit + (G == 128 ? 0 : (par * GPS + (G == 32 ? k : 0)) * 128) + m * 64);
+                    if (G == 128) sv[0][m] *= sign;
                 }
             }
+            // requests, one at a time: the weights two units ahead in front of the tile three steps ahead
+            if (t >= T - AHEAD) {
+                const int NL = XP + (par == 0 ? WL : 0), j = t - (T - AHEAD);
 #pragma unroll
-            for (int g = 0; g < GPS; g++) zw[mt][g] = (wr[u].z[mt][g] >> zsh[mt]) & 15;
-        }
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++) // the slot's registers are free from here on, and not before
-            asm volatile("" : "+v"(wd[mt][0]), "+v"(wd[mt][1]), "+v"(wd[mt][2]), "+v"(wd[mt][3])::"memory");
-        __builtin_amdgcn_sched_barrier(0);
-        fetch_w(it + WR, wr[u]);
-        __builtin_amdgcn_sched_barrier(0);
-        const uint16_t *xb = xs + (size_t)u * NP * TN * kRowHalves;
-        __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-        for (int s = 0; s < 4; s++) {
-            const int piece = G >= 64 ? 4 * h + s : (s >> 1) * 4 + (s & 1) * 2 + h;
-            Frag a[MT], b[NP][NB];
-#pragma unroll
-            for (int q = 0; q < NP; q++)
-#pragma unroll
-                for (int nb = 0; nb < NB; nb++)
-                    b[q][nb].q = *reinterpret_cast<const uint4 *>(xb + ((size_t)q * TN + nb * 32 + r) * kRowHalves + piece * 8);
-#pragma unroll
-            for (int mt = 0; mt < MT; mt++) a[mt] = Dequant(zw[mt][G >= 64 ? 0 : s >> 1], negated(gpar, s >> 1) ? -1.0f : 1.0f)(wd[mt][s]);
-            const bool zero = first && (G >= 64 ? s == 0 : (s & 1) == 0);
-#pragma unroll
-            for (int q = NP - 1; q >= 0; q--)
-#pragma unroll
-                for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-                    for (int nb = 0; nb < NB; nb++)
-                        accg[mt][nb] = Dequant::mfma(a[mt], b[q][nb], zero && q == NP - 1 ? f16v{} : accg[mt][nb]);
-            if (G >= 64 ? (last && s == 3) : (s & 1) == 1) { // a group ends: its partial sum, scaled, joins the run
-                const float *sc = gsc[gpar][G >= 64 ? 0 : s >> 1] + wave * RW;
-#pragma unroll
-                for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-                    for (int k = 0; k < 4; k++) {
-                        const float4 sv = *reinterpret_cast<const float4 *>(sc + mt * 32 + k * 8 + h * 4);
-                        const float svv[4] = {sv.x, sv.y, sv.z, sv.w};
-#pragma unroll
-                        for (int nb = 0; nb < NB; nb++)
-#pragma unroll
-                            for (int e = 0; e < 4; e++)
-                                acc[mt][nb][4 * k + e] = fmaf(svv[e], accg[mt][nb][4 * k + e], acc[mt][nb][4 * k + e]);
-                    }
-            }
-        }
-        __builtin_amdgcn_s_setprio(0);
-        if (last) store_s(gpar ^ 1, sr);
-        store_x(u ^ 1, xr);
-        __syncthreads();
-    };
-    size_t ws_base = 0;
-    for (int i = 0; i < mi; i++) ws_base += (size_t)KS * B * L.m[i].out;
-    // Runs that have ended: their sum lies where the result goes, every lane's own elements.  (There are no registers for a
-    // third set of tiles.  What it costs is this traffic: 4096 -> 22016 outputs, 512 columns, group 32, 45 MB a time; a layer
-    // of 7B, 512 tokens, 0.88 -> 0.93 ms with runs of 64 groups, 0.98 with 32; 299 tokens, group 128 has one run.)
-    float *const sums = KS > 1 || partials ? ws + ws_base + (size_t)ks * B * n_out : L.m[mi].y;
-    auto each_sum = [&](auto &&f) __attribute__((always_inline)) {
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-            for (int nb = 0; nb < NB; nb++)
-#pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    const int t = t0 + nb * 32 + r, o = obase + mt * 32 + k * 8 + h * 4;
-                    if (t < B && o < n_out) f(*reinterpret_cast<float4_any *>(sums + (size_t)t * n_out + o), acc[mt][nb], 4 * k);
+                for (int i = j * NL / AHEAD; i < (j + 1) * NL / AHEAD; i++) {
+                    if (par == 0 && i < WL) fetch_w(unit2, i);
+                    else fetch_x(tile, par == 0 ? i - WL : i);
                 }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        read_w(par, unit1); // of the step after the next: the same half of the next unit
+        const uint32_t free = tile;
+        tile = tile1, tile1 = tile2, tile2 = free;
+        if (par == 1) {
+            const uint32_t free_unit = unit;
+            unit = unit1, unit1 = unit2, unit2 = free_unit;
+            sign = -sign;
+        }
     };
-    const int n_it = it1 - it0;
-    const int n_full = n_it / PW * PW;
-    constexpr int kRunGroups = 64, kRunSteps = kRunGroups * KPG / GPS;
-    const int runs = (n_it + kRunSteps - 1) / kRunSteps, run_len = (n_it / runs + PW) / PW * PW;
+    auto requests = [&](const int tiles, const int units) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < WL; i++) fetch_w(units * S::kUnit, i);
+#pragma unroll
+        for (int i = 0; i < XP; i++) fetch_x(tiles * S::kTile, i);
+    };
+    requests(0, 0);
+    requests(1, 1);
+#pragma unroll
+    for (int i = 0; i < XP; i++) fetch_x(2 * S::kTile, i);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * XP + WL) : "memory");
+    read_w(0, 0);
+    constants(0, sign);
+#pragma unroll
+    for (int i = 0; i < 16; i++) dequant(0, i);
+    read_w(1, 0);
+#pragma unroll
+    for (int t = 0; t < AHEAD; t++) read_x(0, t, 0);
+
+    auto finish_folds = [&](const int par) __attribute__((always_inline)) { // those still due behind a step; they add nothing again
+#pragma unroll
+        for (int t = T - LAG; t < T; t++) fold(par, t), accg[t % NT][0] = accg[t % NT][1] = f4v{0.f, 0.f, 0.f, 0.f};
+    };
+    const int n_full = n_it / 2 * 2;
+    constexpr int kRunGroups = G == 32 ? 16 : G == 64 ? 10 : 8, kRunSteps = kRunGroups * KPG / GPS;
+    const int runs = (n_it + kRunSteps - 1) / kRunSteps, run_len = (n_it / runs + 2) / 2 * 2;
+    auto end_run = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int n = 0; n < NT; n++)
+#pragma unroll
+            for (int m = 0; m < 2; m++) top[n][m] += acc[n][m], acc[n][m] = f4v{0.f, 0.f, 0.f, 0.f};
+    };
     int i = 0;
-    for (;;) { // whole rounds of PW steps, run by run
-        for (const int end = min(i + run_len, n_full); i < end; i += PW) {
-#pragma unroll
-            for (int u = 0; u < PW; u++) k_step(it0 + i + u, u);
+    for (;;) { // whole units, run by run
+        for (const int end = min(i + run_len, n_full); i < end; i += 2) {
+            k_step(0);
+            k_step(1);
         }
         if (i >= n_full) break;
-        each_sum([&](float4_any &at, f16v &v, int k) __attribute__((always_inline)) {
-            float4_any c{v[k], v[k + 1], v[k + 2], v[k + 3]};
-            if (i > run_len) c += at;
-            at = c;
-            v[k] = v[k + 1] = v[k + 2] = v[k + 3] = 0.f;
-        });
+        finish_folds(1);
+        end_run();
     }
-#pragma unroll
-    for (int u = 0; u < PW - 1; u++) // the rest straight-line: a loop left half-way copies ring registers, and waits
-        if (n_full + u < n_it) k_step(it0 + n_full + u, u);
-    if (n_full > run_len)
-        each_sum([&](float4_any &at, f16v &v, int k) __attribute__((always_inline)) {
-            const float4_any c = at;
-            v[k] += c.x, v[k + 1] += c.y, v[k + 2] += c.z, v[k + 3] += c.w;
-        });
+    if (n_full < n_it) {
+        k_step(0);
+        finish_folds(0);
+    } else {
+        finish_folds(1);
+    }
+    end_run();
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory"); // the LDS is reused below
 
-    // C layout: lane (column r = token, h), register i -> row (i / 4) * 8 + h * 4 + i % 4.  Turned through LDS (the
-    // activation buffers are free now) so that a store writes 128 contiguous bytes per token.
-    constexpr int kTRow = 36;
-    float *tile = reinterpret_cast<float *>(xs) + wave * 32 * kTRow;
+    size_t ws_base = 0;
+    for (int i = 0; i < mi; i++) ws_base += (size_t)KS * B * L.m[i].out;
+    // C layout: lane (column r = token, kg), register e -> row 4 kg + e.  Turned through LDS so that a store writes 128
+    // contiguous bytes per token.
+    constexpr int kTRow = 36, PASS = TN < 32 ? TN : 32;
+    float *tile_o = reinterpret_cast<float *>(lds) + wave * 32 * kTRow;
     const int tl = lane >> 3, oc = (lane & 7) * 4;
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++)
+    for (int n0 = 0; n0 < NT; n0 += PASS / 16) {
 #pragma unroll
-        for (int nb = 0; nb < NB; nb++) {
+        for (int n = 0; n < PASS / 16; n++)
 #pragma unroll
-            for (int q = 0; q < 4; q++)
-                *reinterpret_cast<float4 *>(&tile[r * kTRow + q * 8 + h * 4]) =
-                    make_float4(acc[mt][nb][4 * q], acc[mt][nb][4 * q + 1], acc[mt][nb][4 * q + 2], acc[mt][nb][4 * q + 3]);
+            for (int m = 0; m < 2; m++) *reinterpret_cast<f4v *>(&tile_o[(n * 16 + r) * kTRow + m * 16 + kg * 4]) = top[n0 + n][m];
 #pragma unroll
-            for (int pass = 0; pass < 4; pass++) {
-                const int tt = pass * 8 + tl;
-                float4 v = *reinterpret_cast<const float4 *>(&tile[tt * kTRow + oc]);
-                const int t = t0 + nb * 32 + tt, o = obase + mt * 32 + oc;
-                if (t < B && o < n_out) finish4(L, mi, ss, ws + ws_base, KS, ks, partials, t, o, v);
-            }
+        for (int pass = 0; pass < PASS / 8; pass++) {
+            const int tt = pass * 8 + tl;
+            float4 v = *reinterpret_cast<const float4 *>(&tile_o[tt * kTRow + oc]);
+            const int t = t0 + n0 * 16 + tt, o = obase + oc;
+            if (t < B && o < n_out) finish4(L, mi, ss, ws + ws_base, KS, ks, partials, t, o, v);
         }
+    }
+}
+
+// The last tile of tokens takes 16 or 32 where that is enough.
+template <int G, int NT, int NW>
+__global__ __launch_bounds__(64 * NW, NT == 1 ? 3 : 2) void q4_tile_gemm_kernel(const Q4Launch L, const XhList xl, int in_p,
+                                                              const float *__restrict__ ss, float *__restrict__ ws, int KS,
+                                                              int t_tiles, int partials) {
+    // an XCD gets all token tiles of a row block one behind the other: what runs on it at one time shares weights and tiles
+    const int work = xcd_item(blockIdx.x, gridDim.x);
+    int rb = work / t_tiles;
+    const int t0 = (work - rb * t_tiles) * 16 * NT, n = L.batch - t0;
+    const int row_blocks = gridDim.x / (t_tiles * KS), ks = rb / row_blocks;
+    rb -= ks * row_blocks;
+    if (NT > 1 && n <= 16) q4_tile<G, 1, NW>(L, xl, in_p, ss, ws, KS, partials, rb, ks, t0);
+    else if (NT > 2 && n <= 32) q4_tile<G, NT < 2 ? NT : 2, NW>(L, xl, in_p, ss, ws, KS, partials, rb, ks, t0);
+    else q4_tile<G, NT, NW>(L, xl, in_p, ss, ws, KS, partials, rb, ks, t0);
 }
 
 // Linear::matvec<B> of the model without quantisation (src/model.rs:22-31) for a batch: fp32 weights, fp32 activations,
@@ -779,19 +798,19 @@ __global__ __launch_bounds__(1024, SL <= 2 ? 8 : 4) void gemm_silu_kernel(const 
 
 // ---- launchers ---------------------------------------------------------------------------------------------------
 
-template <int G, int MT, int NB>
+template <int G, int NT, int NW>
 int ready_tile(size_t *lds) {
-    *lds = std::max((size_t)2 * 3 * 32 * NB * kRowHalves * 2, (size_t)4 * 32 * 36 * sizeof(float));
+    *lds = std::max(TileLds<G, NT, NW>::kSize, (size_t)NW * 32 * 36 * sizeof(float));
     static LdsLimit limit; // per instantiation
-    return limit.ensure(reinterpret_cast<const void *>(q4_tile_gemm_kernel<G, MT, NB>), *lds);
+    return limit.ensure(reinterpret_cast<const void *>(q4_tile_gemm_kernel<G, NT, NW>), *lds);
 }
 
-template <int G, int MT, int NB>
+template <int G, int NT, int NW>
 int launch_tile(const Q4Launch &L, const XhList &xh, const float *ss, float *ws, int KS, int partials, int total, hipStream_t st) {
     size_t lds = 0;
-    L2_TRY((ready_tile<G, MT, NB>(&lds)));
-    const int t_tiles = (L.batch + 32 * NB - 1) / (32 * NB);
-    hipLaunchKernelGGL((q4_tile_gemm_kernel<G, MT, NB>), dim3(total * t_tiles * KS), dim3(256), lds, st, L, xh, gemm_padded(L.in), ss, ws, KS, t_tiles, partials);
+    L2_TRY((ready_tile<G, NT, NW>(&lds)));
+    const int t_tiles = (L.batch + 16 * NT - 1) / (16 * NT);
+    hipLaunchKernelGGL((q4_tile_gemm_kernel<G, NT, NW>), dim3(total * t_tiles * KS), dim3(64 * NW), lds, st, L, xh, gemm_padded(L.in), ss, ws, KS, t_tiles, partials);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }
@@ -799,19 +818,18 @@ int launch_tile(const Q4Launch &L, const XhList &xh, const float *ss, float *ws,
 template <int G>
 int ready_group() {
     size_t lds = 0;
-    L2_TRY((ready_tile<G, 1, 1>(&lds)));
-    L2_TRY((ready_tile<G, 1, 2>(&lds)));
-    L2_TRY((ready_tile<G, 2, 2>(&lds)));
+    L2_TRY((ready_tile<G, 1, 4>(&lds)));
+    L2_TRY((ready_tile<G, 2, 4>(&lds)));
+    L2_TRY((ready_tile<G, 4, 8>(&lds)));
     return L2_OK;
 }
 
 template <int G>
 int launch_group(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, int partials, hipStream_t st) {
     for (int i = 0; i < L.n_mats; i++) L.m[i].row_blocks = (L.m[i].out + s.rows - 1) / s.rows;
-    if (s.rows == 256)
-        return launch_tile<G, 2, 2>(L, xh, ss, ws, s.slices, partials, s.row_blocks, st);
-    if (s.tokens == 64) return launch_tile<G, 1, 2>(L, xh, ss, ws, s.slices, partials, s.row_blocks, st);
-    return launch_tile<G, 1, 1>(L, xh, ss, ws, s.slices, partials, s.row_blocks, st);
+    if (s.tokens == 64) return launch_tile<G, 4, 8>(L, xh, ss, ws, s.slices, partials, s.row_blocks, st);
+    if (s.tokens == 32) return launch_tile<G, 2, 4>(L, xh, ss, ws, s.slices, partials, s.row_blocks, st);
+    return launch_tile<G, 1, 4>(L, xh, ss, ws, s.slices, partials, s.row_blocks, st);
 }
 
 int launch_fp32(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, int partials, hipStream_t st) {
@@ -851,23 +869,38 @@ GemmShape gemm_shape(const Q4Launch &L, int slice_batch, int planes) {
     if (planes == 1) return gemm_shape_f16(L, slice_batch);
     GemmShape s{};
     const int B = L.batch;
-    const int kstep = planes == kDensePlanes ? 32 : L.group_size > 64 ? L.group_size : 64, units = (gemm_padded(L.in) + kstep - 1) / kstep;
-    auto slices = [&](int slots, int blocks, int most) { return std::max(1, std::min({slots / blocks, most, units / 2})); };
-    // K slices: as many as keep the grid within one round of resident blocks.  Up to 32 columns the registers and the
-    // LDS hold four blocks per CU of 128 rows, and the partial tiles are small; beyond, two of 256 rows (fp32 weights: three
-    // of 128).  Where the rows are cut in 128s all the same (below), the grid is twice what was counted and may take a
-    // second round: 11008 outputs, 61 columns are 688 blocks in 8 slices on 512 slots.
-    const int rows32 = row_blocks(L, 128), rows64 = row_blocks(L, 256);
-    if (slice_batch <= 32)
-        s.slices = slices(4 * cu_count(), rows32, kMaxGemmSlices);
-    else if (planes == kDensePlanes)
-        s.slices = slices(3 * cu_count(), rows32 * ((slice_batch + 63) / 64), 8);
-    else
-        s.slices = slices(2 * cu_count(), rows64 * ((slice_batch + 63) / 64), 8);
-    s.tokens = B <= 32 ? 32 : 64;
-    // 256 rows reuse every 16 bytes read from the LDS twice; 128 where such blocks would be fewer than three to two CUs
-    const int tiles = (B + s.tokens - 1) / s.tokens;
-    s.rows = planes == kDensePlanes || s.tokens == 32 || rows64 * tiles * s.slices < 3 * cu_count() / 2 ? 128 : 256;
+    // inputs per slice, at least: 64 (fp32 weights), 256, and from 4096 inputs on 512 (4096 -> 4096, group 128, 32 columns, 16 slices
+    // 19.4 us, 8 17.0; 1024 inputs, 4 slices or 2, a three-layer prompt of 32: 140 or 153)
+    const int shortest = planes == kDensePlanes ? 64 : L.in >= 4096 && L.group_size > 32 ? 512 : 256;
+    auto slices = [&](int slots, int blocks, int most) { return std::max(1, std::min({slots / blocks, most, gemm_padded(L.in) / shortest})); };
+    const int rows32 = row_blocks(L, 128), rows64 = row_blocks(L, 256), cus = cu_count();
+    if (planes == kDensePlanes) {
+        // as many K slices as keep the grid within one round of resident blocks, four per CU up to 32 columns, else three
+        s.slices = slice_batch <= 32 ? slices(4 * cus, rows32, kMaxGemmSlices) : slices(3 * cus, rows32 * ((slice_batch + 63) / 64), 8);
+        s.tokens = B <= 32 ? 32 : 64, s.rows = 128;
+    } else if (slice_batch <= 32) {
+        // two blocks of 128 rows per CU (13824 -> 5120, 16 columns, 12 slices: 26 us; with three or four per CU 28)
+        s.slices = slices(2 * cus, rows32, kMaxGemmSlices);
+    } else {
+        // One block of 256 rows x 64 columns per CU.  A block costs its share of K, the first and last microseconds (4.5 % of
+        // 4096 inputs) and, with several slices, its partial tile, written and read again (7.5 %): the slices, of those that
+        // take two rounds of blocks at most (what the operator's fixed workspace holds), for which that sum is the smallest.
+        const int blocks = rows64 * ((slice_batch + 63) / 64), most = std::min(slice_batch <= 64 ? kMaxGemmSlices : 8, L.in / shortest);
+        const float per = 4096.0f / L.in;
+        float best = 0.f;
+        for (int n = 1; n <= std::max(1, most) && (n == 1 || n * blocks <= 2 * cus); n++) {
+            const int rounds = (n * blocks + cus - 1) / cus;
+            const float cost = rounds * (1.0f / n + 0.045f * per) + (n > 1 ? 0.075f * per * n * blocks / cus : 0.f);
+            if (n == 1 || cost < best) best = cost, s.slices = n;
+        }
+    }
+    if (planes != kDensePlanes) {
+        // tiles of 32 columns and 128 rows too where wider blocks would leave half the CUs without one (six layers of 1024
+        // inputs, group 64, 64 columns: 404 -> 380 us)
+        const bool few = 2 * rows64 * ((B + 63) / 64) * s.slices <= cus;
+        s.tokens = B <= 16 ? 16 : B <= 32 || few ? 32 : 64;
+        s.rows = s.tokens == 64 ? 256 : 128;
+    }
     s.row_blocks = s.rows == 128 ? rows32 : rows64;
     return s;
 }
@@ -884,8 +917,7 @@ int gemm_launch(Q4Launch &L, const XhList &xh, const float *ss, float *ws, size_
         rows += L.m[i].out;
     }
     const GemmShape s = gemm_shape(L, slice_batch, planes);
-    // the fp32 kernel keeps its runs' sums where the result goes, which is where the residual lies
-    const bool partials = ks_out || (planes == 3 && L.e.kind == Q4_EPI_RESIDUAL);
+    const bool partials = ks_out;
     if ((s.slices > 1 || partials) && (size_t)s.slices * L.batch * rows > ws_floats)
         return l2_fail(L2_ERR_ARG, "q4 gemm: %d slices of %d x %ld in a workspace of %zu", s.slices, L.batch, rows, ws_floats);
     if (planes == 1)

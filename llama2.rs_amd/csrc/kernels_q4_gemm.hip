@@ -36,14 +36,13 @@
 // group (one FMA per accumulator element and group), so the only rounding on
 // the weight side is none at all; for G = 32 a step of 32 k would be a group,
 // and the weights are multiplied by fp16(scale) before the MFMA.
-#include "l2_internal.h"
+#include "gemm_lds.h"
 #include <algorithm>
 
 namespace {
 
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef float f4v __attribute__((ext_vector_type(4)));
 
 union A8 {
     h8 v;
@@ -77,8 +76,6 @@ struct Dequant16 {
     }
 };
 
-constexpr int kStepRow = 128; // bytes of a token in an activation tile of 64 k
-
 // LDS of a block of NW waves: four activation tiles, and for each wave three units of 128 k of its 32 rows' weights, scales
 // and zero points.
 template <int G, int NW>
@@ -88,22 +85,6 @@ struct GemmLds {
     static constexpr int kUnit = kWeights + 2 * kScales;
     static constexpr size_t size(int tokens) { return (size_t)4 * tokens * kStepRow + (size_t)NW * 3 * kUnit; }
 };
-
-typedef uint32_t u4v __attribute__((ext_vector_type(4)));
-
-// Memory as a buffer of `bytes` from `base` (both the same in every lane).
-__device__ __forceinline__ u4v buffer(const void *base, uint32_t bytes) {
-    const uint64_t p = reinterpret_cast<uint64_t>(base);
-    return u4v{(uint32_t)__builtin_amdgcn_readfirstlane((int)p), (uint32_t)__builtin_amdgcn_readfirstlane((int)(p >> 32)) & 0xFFFFu,
-               (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
-}
-
-// From memory into LDS past the registers: lane l's piece (16 or 4 bytes) at `off` + `soff` bytes of the buffer goes to
-// lds + size * l.  `at` shifts both by the same constant, so callers have it taken off `off`.  vmcnt counts them, and since the
-// compiler does not know of them, nothing else in the loop may load from memory.
-#define LDS_TO(lds) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" ::"s"(lds) : "memory")
-#define LDS_LOAD(n, at, buf, off, soff) \
-    asm volatile("buffer_load_dword" n " %0, %1, %2 offen offset:%3 lds" ::"v"(off), "s"(buf), "s"(soff), "n"(at) : "memory")
 
 // 32 NW rows rb * 32 NW.. of the matrices of a launch against the 32 NB tokens t0.., K slice ks of KS.
 template <int G, int NB, int NW>
@@ -127,17 +108,15 @@ __device__ __forceinline__ void q4_gemm_tile(const Q4Launch &L, const XhList &xh
     const int n_units = in / 128;
     const int u0 = (int)((long)n_units * ks / KS), u1 = (int)((long)n_units * (ks + 1) / KS);
 
-    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)lds;
+    const uint32_t lds0 = lds_offset(lds);
     const uint32_t wave_at = 4 * kTile + wave * 3 * S::kUnit; // of this wave's weights, scales and zero points
 
     // Where a lane's pieces come from.  A wave's 1 KB pieces of an activation tile follow each other in the LDS (fewer pieces
     // than waves: the last ones fetch the same), as do the parts of a unit: one base each, the rest in the instructions.
     constexpr int XP = (NB * 4 + NW - 1) / NW;
-    constexpr int kBias = 4096;
-    const u4v xbuf = buffer(reinterpret_cast<const char *>(xh_list.p[mi]) - kBias, (uint32_t)((size_t)B * in * 2 + kBias));
-    const u4v wbuf = buffer(reinterpret_cast<const char *>(M.qweight) - kBias, (uint32_t)((size_t)n_out * (in >> 1) + kBias));
-    const u4v sbuf = buffer(reinterpret_cast<const char *>(M.scales) - kBias, (uint32_t)((size_t)n_out * groups * 4 + kBias));
-    const u4v zbuf = buffer(reinterpret_cast<const char *>(M.qzeros) - kBias, (uint32_t)((size_t)(n_out >> 3) * groups * 4 + kBias));
+    static_assert(XP <= 4, "the instruction's own offset has 12 bits");
+    const u4v xbuf = biased_buffer(xh_list.p[mi], (size_t)B * in * 2), wbuf = biased_buffer(M.qweight, (size_t)n_out * (in >> 1));
+    const u4v sbuf = biased_buffer(M.scales, (size_t)n_out * groups * 4), zbuf = biased_buffer(M.qzeros, (size_t)(n_out >> 3) * groups * 4);
     const int xfirst = min(wave * XP, NB * 4 - XP);
     uint32_t xoff[XP], woff[2], soff, zoff;
 #pragma unroll
@@ -361,16 +340,14 @@ __device__ __forceinline__ void q4_gemm_tile(const Q4Launch &L, const XhList &xh
 template <int G, int NB, int NW>
 __global__ __launch_bounds__(64 * NW, NB > 2 ? 2 : 1) void q4_gemm_kernel(const Q4Launch L, const XhList xh, const float *__restrict__ ss,
                                                       float *__restrict__ ws, int KS, int partials, int row_blocks, int t_full, int whole) {
-    // Blocks are dealt round-robin over the 8 XCDs, each with an L2 of its own: a contiguous range of items for each.
-    auto place = [](int b, int n) { const int per = n >> 3, over = n & 7, xcd = b & 7; return xcd * per + min(xcd, over) + (b >> 3); };
     constexpr int TN = 32 * NB, CHUNK = 8;
     const int tiles = row_blocks * t_full;
     int item, half = -1, ks, rb, tt;
     if ((int)blockIdx.x < whole) {
-        item = place(blockIdx.x, whole);
+        item = xcd_item(blockIdx.x, whole);
     } else {
         const int halves = 2 * (tiles * KS - whole);
-        item = place(blockIdx.x - whole, gridDim.x - whole);
+        item = xcd_item(blockIdx.x - whole, gridDim.x - whole);
         if (item < halves) half = item & 1, item = whole + (item >> 1);
         else item += tiles * KS - halves;
     }

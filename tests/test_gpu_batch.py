@@ -42,6 +42,25 @@ def test_batch_operator_vs_fp64(ops, n_in, n_out, G, batches):
     q.close()
 
 
+# the tiles' other widths: 16, 32 and 64 columns as the only tile and as the last one of a wide block, few blocks (tiles of 32),
+# several runs of groups, a slice of one step
+@pytest.mark.parametrize("n_in,n_out,G,batches", [
+    (4224, 8320, 128, (16, 17, 84, 96, 144)), (1056, 520, 32, (16, 17, 40, 50)), (1088, 264, 64, (15, 33, 80)),
+    (28672, 1032, 64, (20, 36)), (2080, 24584, 32, (70, 86)), (64, 8200, 64, (60, 300)), (96, 8200, 32, (300,))])
+def test_batch_tiles_vs_fp64(ops, n_in, n_out, G, batches):
+    rng = np.random.default_rng(n_out)
+    qw, qz, sc, gi = ck.synth_qlinear(rng, n_in, n_out, G, act_order=True)
+    W = ck.dequant_bin(qw, qz, sc, gi, G).astype(np.float64)
+    q = ops.QLinear(qw, qz, sc, gi, G)
+    for B in batches:
+        x = rng.standard_normal((B, n_in)).astype(np.float32)
+        x[:, n_in // 2] *= 1e6  # one input far above the others
+        want, got = x.astype(np.float64) @ W.T, q.matvec(x)
+        for b in range(B):
+            assert nrel(got[b], want[b]) < 1e-5, (B, b)
+    q.close()
+
+
 @pytest.mark.parametrize("kv,hidden,G,n", [(8, 2816, 32, 70), (4, 2848, 32, 64), (2, 2816, 64, 131), (1, 2816, 128, 97),
                                              (2, 2816, 0, 66), (8, 2848, 0, 135)])
 def test_fp32_prompt_vs_oracle(ops, oracle, kv, hidden, G, n):
