@@ -174,6 +174,72 @@ __device__ __forceinline__ MatOps mat_ops(const Q4Mat &M) {
     return o;
 }
 
+// What a thread holds of a vector on its way to LDS, NX pieces of four floats.  NX * 64 * NW pieces cover the
+// longest vector of the kernel, so the staging has no loop, and past the vector's end a buffer load returns zeros,
+// so it has no branch per piece either.  That is for the length of the code: a launch of 5 to 13 us runs its
+// prologue once, from an instruction cache that does not hold it, and pays some 0.1 us per kilobyte.  With a guard
+// per piece and a loop for what a first batch had left, the kernels were 2 to 4 KB longer and a 7B token took
+// 1332 us, against 1301 in this form.
+template <int NX>
+struct XRegs {
+    float4 v[NX], g[NX];
+};
+
+__device__ __forceinline__ float4 ld_bounded(__amdgpu_buffer_rsrc_t r, int byte_offset) {
+    return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, byte_offset, 0, 0));
+}
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t bounded(const float *p, int n) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p), 0, n * 4, 0x00020000);
+}
+
+template <int NW, int NX>
+__device__ __forceinline__ void x_issue(const float *x, const float *wn, int in, int tid, XRegs<NX> &r) {
+    const __amdgpu_buffer_rsrc_t rx = bounded(x, in);
+#pragma unroll
+    for (int u = 0; u < NX; u++) r.v[u] = ld_bounded(rx, (u * NW * 64 + tid) * 16);
+    if (wn) {
+        const __amdgpu_buffer_rsrc_t rg = bounded(wn, in);
+#pragma unroll
+        for (int u = 0; u < NX; u++) r.g[u] = ld_bounded(rg, (u * NW * 64 + tid) * 16);
+    }
+}
+
+// The pieces into the padded chunks, with the sums of the chunks; returns the thread's share of sum(x^2).
+// All slots are written (zeros past the vector's end).
+template <int NWK, int NW, int NX>
+__device__ __forceinline__ float x_stage(bool norm, int tid, XRegs<NX> &r, float *xs, float *xsum) {
+    float ssq = 0.f;
+    if (norm) {
+#pragma unroll
+        for (int u = 0; u < NX; u++) {
+            float4 &v = r.v[u];
+            ssq = fmaf(v.x, v.x, ssq);
+            ssq = fmaf(v.y, v.y, ssq);
+            ssq = fmaf(v.z, v.z, ssq);
+            ssq = fmaf(v.w, v.w, ssq);
+            v.x *= r.g[u].x;
+            v.y *= r.g[u].y;
+            v.z *= r.g[u].z;
+            v.w *= r.g[u].w;
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < NX; u++) {
+        const int j4 = u * NW * 64 + tid;
+        const float4 v = r.v[u];
+        float s = (v.x + v.y) + (v.z + v.w);
+        s += dpp_xchg<0xB1>(s);  // the 8 lanes that hold one chunk add up its sum: lanes ^1
+        s += dpp_xchg<0x4E>(s);  // lanes ^2
+        s += dpp_xchg<0x141>(s); // 7 - lane within each 8: the other quad
+        if ((u + 1) * NW * 64 <= NWK * 512 || j4 < NWK * 512) {
+            *reinterpret_cast<float4 *>(&xs[(j4 >> 3) * kChunkPad + (j4 & 7) * 4]) = v;
+            xsum[j4 >> 3] = s; // the same value from all 8 lanes
+        }
+    }
+    return ssq;
+}
+
 struct RowData {
     uint4 w;
     float s;
@@ -237,7 +303,9 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const Q4Launch L
         }
     }
     const int C = in >> 5;
-    const int xstride = C * kChunkPad + C;
+    constexpr int NC = NWK * 64;                 // chunks the waves of a row cover
+    constexpr int xstride = NC * kChunkPad + NC; // floats of LDS per staged vector
+    constexpr int NX = (8 + S - 1) / S;          // pieces of x per thread
 
     const int b = blockIdx.y;
     const int tid = threadIdx.x;
@@ -282,14 +350,14 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const Q4Launch L
 
     // x first, then the first rows of the weights: loads return in order, and
     // the staging of x (a cache hit) must not queue behind rows that come from HBM.
-    StageRegs xr[DIRECT ? 1 : NM];
+    XRegs<NX> xr[DIRECT ? 1 : NM];
     float4 xd[DIRECT ? 8 : 1];
-    int4 gi[GATHER ? kStageBatch : 1];
-    if constexpr (GATHER) { // the first batch covers the whole vector (checked by the launcher)
+    int4 gi[GATHER ? NX : 1];
+    if constexpr (GATHER) {
         const int n4 = in >> 2;
         const int4 *g4 = reinterpret_cast<const int4 *>(mat[0].gidx);
 #pragma unroll
-        for (int u = 0; u < kStageBatch; u++) {
+        for (int u = 0; u < NX; u++) {
             const int j4 = u * (NW * 64) + tid;
             gi[u] = j4 < n4 ? g4[j4] : make_int4(0, 0, 0, 0);
         }
@@ -304,16 +372,40 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const Q4Launch L
     } else {
 #pragma unroll
         for (int q = 0; q < NM; q++)
-            stage_issue<NW>(mat[q].x + (size_t)b * in, mat[q].wn, in, 0, tid, xr[q]);
+            x_issue<NW, NX>(mat[q].x + (size_t)b * in, mat[q].wn, in, tid, xr[q]);
         // No wave of the block asks for weights before every wave has asked for its piece of x: a CU returns
         // loads in the order it received them, and a piece of x (a cache hit) requested behind another wave's
         // first rows (HBM) would hold up the staging of the whole block until those rows are in.
         if constexpr (NW > 1) __builtin_amdgcn_s_barrier();
     }
     __builtin_amdgcn_sched_barrier(0);
+    // The first half of the rows in flight now, the rest once x is staged: HBM has something to do meanwhile, and x,
+    // which has to cross the same memory pipe (another XCD wrote it), does not queue behind all of it.  Half
+    // was best: 7B token 1275 us, 1294 with all rows of the pair first and 1311 with none; 13B of 20 layers 1246,
+    // 1264 with all.
+    constexpr int PRE = (P + 1) / 2;
     RowData pipe[P][NM];
 #pragma unroll
-    for (int u = 0; u < P; u++) fetch(u, pipe[u]);
+    for (int u = 0; u < PRE; u++) fetch(u, pipe[u]);
+    // What the epilogues read besides the sums (residual, scatter indices): by the thread that finishes the row,
+    // once, before the first tile.  A load in each tile would be a wait in front of the tile's end, and as only the
+    // finishing wave would issue it, that wave's counts of younger rows would be inexact.  Thread t finishes row t
+    // of the block, and the row SPAN further on where a block has more rows than threads.  Operands that are absent
+    // are not read (a dummy in their place was a cold line: 7B token 1275 us with it, 1264 without).
+    constexpr int SPAN = NW * 64 / TR * TR;
+    const size_t out_base = (size_t)b * n_out;
+    const bool has_res = !PAIR && epi_kind == Q4_EPI_RESIDUAL;
+    int eo = row0 + tid;
+    float res_v = 0.f;
+    uint32_t sidx[3] = {0, 0, 0};
+    auto epi_fetch = [&]() __attribute__((always_inline)) {
+        if (eo < row1) {
+            if (has_res) res_v = res[out_base + eo];
+#pragma unroll
+            for (int t = 0; t < 3; t++)
+                if (t < n_scatter) sidx[t] = (uint32_t)sc_idx[t][eo];
+        }
+    };
     __builtin_amdgcn_sched_barrier(0);
 
     // this lane's slice of x, for good: 32 floats, or 24 digit words + step + sum of q
@@ -357,7 +449,7 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const Q4Launch L
             if constexpr (GATHER) {
                 const int n4 = in >> 2;
 #pragma unroll
-                for (int u = 0; u < kStageBatch; u++) {
+                for (int u = 0; u < NX; u++) {
                     const int j4 = u * (NW * 64) + tid;
                     if (j4 < n4) { // element 4 j4 + e of x is input gi[u].e of the sorted rows
                         xs[(gi[u].x >> 5) * kChunkPad + (gi[u].x & 31)] = xr[q].v[u].x;
@@ -367,8 +459,7 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const Q4Launch L
                     }
                 }
             } else {
-                p = stage_consume<NW>(M.wn != nullptr, in, 0, tid, xr[q], xs, xs + C * kChunkPad, 0.f);
-                p = stage_rest<NW>(M.x + (size_t)b * in, M.wn, in, xs, xs + C * kChunkPad, tid, p);
+                p = x_stage<NWK, NW, NX>(M.wn != nullptr, tid, xr[q], xs, xs + NC * kChunkPad);
             }
             if (q == 0) ssq = p;
         }
@@ -412,7 +503,7 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const Q4Launch L
                     for (int i = 0; i < 24; i++) xp[q][i] = 0;
                 }
             } else {
-                if (has_chunk) {
+                if (!GATHER || has_chunk) { // the staged form has zeros in the slots past the vector's end
                     const float4 *p = reinterpret_cast<const float4 *>(&xs[c * kChunkPad]);
 #pragma unroll
                     for (int i = 0; i < 8; i++) {
@@ -431,7 +522,7 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const Q4Launch L
                             s4[k] = (x[q][4 * k] + x[q][4 * k + 1]) + (x[q][4 * k + 2] + x[q][4 * k + 3]);
                         sx[q] = ((s4[0] + s4[1]) + (s4[2] + s4[3])) + ((s4[7] + s4[6]) + (s4[5] + s4[4]));
                     } else {
-                        sx[q] = xs[C * kChunkPad + c];
+                        sx[q] = xs[NC * kChunkPad + c];
                     }
                 } else {
 #pragma unroll
@@ -451,19 +542,18 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const Q4Launch L
     const int n_full = n_steps / P;
     const int n_rem = n_steps - n_full * P;
     int buf = 0;
-    // Enter the loop with no load outstanding (the primed rows arrived while x
-    // was staged). The compiler's wait counts inside the loop are then those of
-    // the steady state alone: vmcnt leaves the P - 1 younger rows in flight.
-    // Otherwise the issue order of the prologue leaks into the loop's waits.
-    __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0), expcnt and lgkmcnt untouched
-    const size_t out_base = (size_t)b * n_out;
-    float *__restrict__ const yout = mat[0].y;
-    // what the epilogue lanes prefetch; the scales (at least one word per row) stand in for absent operands
-    const bool has_res = !PAIR && epi_kind == Q4_EPI_RESIDUAL;
-    const float *__restrict__ res_p = has_res ? res + out_base : sc[0];
-    const int32_t *__restrict__ idx_p[3];
+    // The second half of the rows, and a wait for the first, which arrived while x was staged.  The compiler's wait
+    // counts inside the loop are then those of the steady state alone: vmcnt leaves the P - 1 younger rows in
+    // flight.  Otherwise the issue order of the prologue leaks into the loop's waits.
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int t = 0; t < 3; t++) idx_p[t] = t < n_scatter ? sc_idx[t] : reinterpret_cast<const int32_t *>(sc[0]);
+    for (int u = PRE; u < P; u++) fetch(u, pipe[u]);
+    __builtin_amdgcn_sched_barrier(0);
+    constexpr int YOUNGER = (P - PRE) * NM * 3;
+    static_assert(YOUNGER < 64, "vmcnt");
+    __builtin_amdgcn_s_waitcnt(0x0F70 | (YOUNGER & 15) | (YOUNGER >> 4) << 14); // expcnt and lgkmcnt untouched
+    epi_fetch();
+    float *__restrict__ const yout = mat[0].y;
 
     // one row (row pair) of this stream: dequantised dot product of the lane's chunk -> pr
     auto row_dot = [&](int o, const RowData(&d)[NM], float(&pr)[NM]) __attribute__((always_inline)) {
@@ -493,13 +583,13 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const Q4Launch L
         }
     };
     // one thread per row of the tile: fixed-order sum of the partials, then the epilogue
-    auto tile_finish = [&](int eo, float res_v, const uint32_t(&sidx)[3]) __attribute__((always_inline)) {
+    auto tile_finish = [&](int r) __attribute__((always_inline)) {
         float sum[NM];
 #pragma unroll
         for (int q = 0; q < NM; q++) {
             float a = 0.f;
 #pragma unroll
-            for (int k = 0; k < PW; k++) a += part[buf][tid][q][k];
+            for (int k = 0; k < PW; k++) a += part[buf][r][q][k];
             sum[q] = a;
         }
         float v = sum[0] * ss;
@@ -516,19 +606,8 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const Q4Launch L
             if (t < n_scatter) st_at(sc_out[t], ((uint32_t)out_base + sidx[t]) << 2, v); // 32-bit offset: nothing widens the loaded index
     };
 
+    int r = tid; // the thread's row within the tile, if 0 <= r < TR
     for (int tile = 0; tile < n_full; tile++) {
-        // The lanes that finish this tile's rows fetch what the epilogue reads
-        // (residual, scatter indices) now: by the time it is needed, P rows of
-        // younger loads stand behind it and the wait leaves those in flight.
-        const int eo = row0 + tile * TR + tid;
-        const bool epi = tid < TR && eo < row1;
-        float res_v = 0.f;
-        uint32_t sidx[3] = {0, 0, 0};
-        if (epi) { // no branch per operand: an unused one reads a valid dummy
-            res_v = res_p[eo];
-#pragma unroll
-            for (int t = 0; t < 3; t++) sidx[t] = (uint32_t)idx_p[t][eo];
-        }
 #pragma unroll
         for (int u = 0; u < P; u++) {
             const int i = tile * P + u;
@@ -547,19 +626,16 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const Q4Launch L
             row_fold(u, pr);
         }
         __syncthreads();
-        if (epi) tile_finish(eo, res_v, sidx);
+        if ((unsigned)r < (unsigned)TR && eo < row1) tile_finish(r);
         buf ^= 1;
+        r -= TR;
+        if ((tile + 1) % (SPAN / TR) == 0) { // a block of more rows than threads: the next SPAN of them
+            eo += SPAN;
+            r = tid;
+            epi_fetch();
+        }
     }
     if (n_rem > 0) { // the rows already in the pipe: no refill, nothing younger to leave in flight
-        const int eo = row0 + n_full * TR + tid;
-        const bool epi = tid < TR && eo < row1;
-        float res_v = 0.f;
-        uint32_t sidx[3] = {0, 0, 0};
-        if (epi) {
-            res_v = res_p[eo];
-#pragma unroll
-            for (int t = 0; t < 3; t++) sidx[t] = (uint32_t)idx_p[t][eo];
-        }
 #pragma unroll
         for (int u = 0; u < P - 1; u++) {
             if (u < n_rem) {
@@ -569,7 +645,7 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const Q4Launch L
             }
         }
         __syncthreads();
-        if (epi) tile_finish(eo, res_v, sidx);
+        if ((unsigned)r < (unsigned)TR && eo < row1) tile_finish(r);
     }
 }
 
@@ -601,8 +677,7 @@ static int plan_rows(const Q4Launch &L, int NW, int TR, size_t lds, bool pair, i
 
 // Wave-rows of arithmetic per CU for a candidate shape: what the choice between shapes minimises.
 static long plan_cost(const Q4Launch &L, int NWK, int S, int P, bool pair) {
-    const int C = L.in / 32;
-    const size_t lds = (size_t)(C * kChunkPad + C) * sizeof(float) * (pair ? 2 : 1);
+    const size_t lds = (size_t)NWK * 64 * (kChunkPad + 1) * sizeof(float) * (pair ? 2 : 1);
     const int NW = NWK * S, TR = P * S;
     int per_cu = 16 / NW;
     if (pair) per_cu = 1; // w1|w3: one block per CU measured faster than two (7B: 13.1 -> 12.4 us, 722 -> 733 tok/s)
@@ -618,11 +693,8 @@ template <int G, int NWK, int S, bool PAIR, int MODE, int P = (PAIR ? 2 : 4), bo
 int launch_s(Q4Launch &L, hipStream_t stream) {
     constexpr int NW = NWK * S;
     constexpr int TR = P * S;
-    const int C = L.in / 32;
     const size_t lds = MODE == 2 ? (size_t)NW * 64 * kChunkPad * sizeof(float)
-                                 : (size_t)(C * kChunkPad + C) * sizeof(float) * (PAIR ? 2 : 1);
-    if (GATHER && L.in > NW * 64 * 4 * kStageBatch)
-        return l2_fail(L2_ERR_ARG, "q4 matvec (gathering): in=%d is more than one staging batch of %d waves", L.in, NW);
+                                 : (size_t)NWK * 64 * (kChunkPad + 1) * sizeof(float) * (PAIR ? 2 : 1);
     if (lds + 8 * 1024 > 160 * 1024) return l2_fail(L2_ERR_ARG, "q4 matvec: in=%d needs %zu B of LDS", L.in, lds);
     int total = 0;
     const int rpb = plan_rows(L, NW, TR, lds, PAIR, &total);

@@ -63,6 +63,23 @@ def test_qmatvec_vs_oracle(ops, oracle, n_in, n_out, G, B):
     q.close()
 
 
+@pytest.mark.parametrize("n_in,n_out", [
+    (32, 8), (2048, 72), (2080, 72), (4064, 24), (6112, 24), (8160, 24),  # x gathered: one chunk, and ragged last waves
+    (8224, 24), (12288, 2056), (12256, 24), (16384, 24), (14368, 24),     # x staged for the block, 6 and 8 waves a row
+    (14336, 2056), (16416, 24),                                           # x by every wave for itself
+    (64, 270000),                                                         # a block of more rows than threads
+])
+def test_qmatvec_staging_edges(ops, oracle, n_in, n_out):
+    rng = np.random.default_rng(n_in + n_out)
+    qw, qz, sc, gi = ck.synth_qlinear(rng, n_in, n_out, 32, act_order=True)
+    x = rng.standard_normal(n_in).astype(np.float32)
+    q = ops.QLinear(qw, qz, sc, gi, 32)
+    got = q.matvec(x)
+    assert nrel(got, oracle.qmatvec(qw, qz, sc, gi, 32, x[None])[0]) < REL_FP32
+    np.testing.assert_array_equal(q.matvec(x), got)
+    q.close()
+
+
 _ALT_FORM_SNIPPET = r"""
 import sys, numpy as np
 sys.path.insert(0, sys.argv[1]); sys.path.insert(0, sys.argv[2])
