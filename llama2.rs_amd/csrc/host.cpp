@@ -1359,14 +1359,17 @@ extern "C" int l2_model_classifier(l2_model *m, const float *x_host, float *y_ho
 // ---------------------------------------------------------------------------
 // transformer<B>
 
-// How the timesteps of a decode step are cut across blocks: one block per kv head up to 256 timesteps,
-// beyond that one block per CU where the context allows it, at least 64 timesteps each.  (Two per CU, the
-// earlier rule, left some CUs with two blocks and the launch as long as those: 70B behind 4096 positions
-// 18.6 -> 16.5 us per layer, 13B behind 1000 positions 16.7 -> 15.3, 7B unchanged; half a block per CU is
-// slower everywhere.)
-static void attn_split_policy(int n_t, int n_kv_heads, int *ts_out, int *n_splits_out) {
-    if (n_t <= 256) {
-        *ts_out = 256;
+// How the timesteps of a decode step are cut across blocks: not at all in a short context (512 timesteps for one or
+// two query heads per kv head, where a head's dimensions are spread over blocks instead: 7B at 400 393 us per token
+// of 8 layers against 402 in splits, equal near 850; 13B at 400 575 against 585, equal near 700; 256 for more: four
+// heads, 2 kv heads, 3 layers 82.3 against 84.1 at 260, 87.7 against 84.6 at 400), beyond that one block per CU where
+// the context allows it, at least 64 timesteps each.  (Two per CU, the earlier rule, left some CUs with two blocks
+// and the launch as long as those: 70B behind 4096 positions 18.6 -> 16.5 us per layer, 13B behind 1000 positions
+// 16.7 -> 15.3, 7B unchanged; half a block per CU is slower everywhere.)
+static void attn_split_policy(int n_t, int n_heads, int n_kv_heads, int *ts_out, int *n_splits_out) {
+    const int whole = n_heads / n_kv_heads <= 2 ? 512 : 256;
+    if (n_t <= whole) {
+        *ts_out = whole;
         *n_splits_out = 1;
         return;
     }
@@ -1461,7 +1464,7 @@ static int forward_enqueue(l2_model *m, l2_state *s, int B, int max_pos, const F
             a.part = m->attn_part;
             a.n_heads = d.n_heads, a.n_kv_heads = d.n_kv_heads;
             a.max_splits = kMaxSplits;
-            attn_split_policy(max_pos + 1, d.n_kv_heads, &a.ts, &a.n_splits);
+            attn_split_policy(max_pos + 1, d.n_heads, d.n_kv_heads, &a.ts, &a.n_splits);
             if (a.n_splits > kMaxSplits)
                 return l2_fail(L2_ERR_RANGE, "attention: position %d needs %d splits", max_pos, a.n_splits);
             LAUNCH(K_ATTENTION, attention_decode_launch(a, st));
@@ -1549,7 +1552,7 @@ static int forward_enqueue_dense(l2_model *m, l2_state *s, int B, int max_pos, c
             a.part = m->attn_part;
             a.n_heads = d.n_heads, a.n_kv_heads = d.n_kv_heads;
             a.max_splits = kMaxSplits;
-            attn_split_policy(max_pos + 1, d.n_kv_heads, &a.ts, &a.n_splits);
+            attn_split_policy(max_pos + 1, d.n_heads, d.n_kv_heads, &a.ts, &a.n_splits);
             if (a.n_splits > kMaxSplits)
                 return l2_fail(L2_ERR_RANGE, "attention: position %d needs %d splits", max_pos, a.n_splits);
             LAUNCH(K_ATTENTION, attention_decode_launch(a, st));

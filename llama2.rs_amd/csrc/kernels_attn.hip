@@ -40,6 +40,22 @@ __device__ __forceinline__ void pin_args(const AttnDecode &A) {
                  "s"(A.ts), "s"(A.n_splits), "s"(A.max_splits));
 }
 
+// A lane's value and that of the lane 32 (16) away, in the same order for both lanes: one instruction that swaps
+// halves (rows) of two registers, in the vector ALU, where a shuffle goes through the LDS pipe.
+struct Both {
+    float lo, hi;
+};
+__device__ __forceinline__ Both both32(float v) {
+    const uint32_t b = __builtin_bit_cast(uint32_t, v);
+    const auto r = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+    return {__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1])};
+}
+__device__ __forceinline__ Both both16(float v) {
+    const uint32_t b = __builtin_bit_cast(uint32_t, v);
+    const auto r = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+    return {__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1])};
+}
+
 constexpr float kNoScore = -1e30f; // "no timestep yet": finite, so that differences never give NaN
 
 __device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
@@ -69,35 +85,51 @@ __device__ __forceinline__ float wave_max(float v) {
 constexpr int kCombRow = 128 + 4;
 static_assert(kCombRow * sizeof(float) % 16 == 0, "rows of the merge tiles are written with 16-byte stores");
 
-// Layout of a block: NWV waves x 4 rows of 16 lanes.  One row of lanes handles
-// one timestep at a time, each lane 8 of the 128 head dimensions; a block
-// covers 4 NWV timesteps per step and PD steps per tile, all of a tile's loads
-// being issued before its arithmetic.  NWV is 4 when the timesteps are cut
-// into splits; wider blocks were measured slower for the single block per kv
-// head of a short context (more waves to start and to merge).  All QG query heads of the kv head share
-// each K and V load (grouped-query attention, src/models.rs:142-145).
-template <int QG, int NWV>
+// Layout of a block: NWV waves x 4 rows of 16 lanes.  One row of lanes handles one timestep at a time, each lane 8
+// of the 128 head dimensions of the key; a block covers 4 NWV timesteps per step and PD steps per tile, all of a
+// tile's loads being issued before its arithmetic.  All QG query heads of the kv head share each K and V load
+// (grouped-query attention, src/models.rs:142-145).
+//
+// A short context (n_splits == 1) is one block per kv head and slice of 128 / DS output dimensions: every slice
+// computes all scores, and reads and sums only its part of the values, so nothing has to be merged across blocks.  A
+// single block per kv head leaves most CUs idle and is bound by what one CU can fetch (some 100 GB/s) and by the
+// merge of its rows; eight slices read 9/16 of the bytes each and merge an eighth.  7B (32 kv heads), per token of 32
+// layers, one block -> 8 slices: 1241 -> 1215 us at position 16, 1292 -> 1257 at 120; 13B (40 kv heads), 8 layers, 4
+// slices: 566 -> 561 at 190, where 8 (320 blocks) took 570.  4 waves up to one tile of timesteps (position 16: 1215 us
+// against 1227 with 8 waves), 8 beyond (190: 381 against 383 with 8 layers); four query heads have more to merge per
+// wave, there 4 waves are better up to two tiles (100: 76.4 against 77.2 us).  Four query heads through this kernel
+// instead of the matrix cores: 76.6 -> 72.7 us per token of 3 layers at 30, 88 -> 79 at 190; at eight the matrix cores
+// stay ahead (70B: 937 against 940-948 us at 60).
+// Longer contexts are cut into splits of timesteps (DS = 1, 4 waves) that attn_combine_kernel merges.
+template <int QG, int NWV, int DS>
 __global__ __launch_bounds__(NWV * 64) void attn_decode_kernel(const AttnDecode A) {
     constexpr int NT = NWV * 64, TSTEP = NWV * 4;
     constexpr int HS = 128, HALF = 64;
-    constexpr int PD = QG >= 8 ? 2 : 4; // steps in flight and per pass through the phases (4 at 8 heads: over 256 registers, one block per CU, slower)
+    constexpr int VD = HS / DS, VE = VD / 16; // head dimensions of the value that are this block's, and a lane's share
+#ifndef V_PD
+#define V_PD 4
+#endif
+    constexpr int PD = QG >= 8 ? 2 : NWV > 4 ? V_PD : 4; // steps in flight and per pass through the phases (4 at 8 heads: over 256 registers, one block per CU, slower)
     __shared__ float qs[QG * HS];
     __shared__ float kvnew[2][HS];
     // With 4 or 8 query heads per kv head the four 16-lane rows of every wave hand their partial results
     // over through (dynamic) LDS: merging them with cross-row shuffles first takes 10 shuffles per head and
     // step, 160 at 8 heads, a fifth of the kernel at long contexts.
-    constexpr bool kRowsInLds = QG >= 4;
+    constexpr bool kRowsInLds = QG * VE >= 32;
     constexpr int NR = kRowsInLds ? NWV * 4 : NWV; // partial results that meet in LDS
     __shared__ __align__(16) float comb_s[kRowsInLds ? 1 : NWV][QG][kCombRow];
     __shared__ float wts[QG][16], m_all[QG], den_all[QG];
     extern __shared__ __align__(16) float comb_d[]; // [NR][QG][kCombRow] when kRowsInLds
     float(*comb)[QG][kCombRow] = kRowsInLds ? reinterpret_cast<float(*)[QG][kCombRow]>(comb_d) : comb_s;
     pin_args(A);
-    const int kvh = blockIdx.x, sp = blockIdx.y;
+    const int kvh = blockIdx.x, sp = blockIdx.y, slice = DS > 1 ? blockIdx.z : 0;
     const int pos = A.dpos ? A.dpos[0] : A.pos;
     const int t0 = sp * A.ts;
     if (t0 > pos) return;
-    const int t1 = min(t0 + A.ts, pos + 1);
+    // The cached positions of this block; the new one, whose key and value are still to be written, is where the
+    // sums of one row of lanes start from, in the block whose range ends with it.
+    const int t1 = min(t0 + A.ts, pos);
+    const bool owns_new = pos < t0 + A.ts;
     const int n = t1 - t0;
     const int kv_dim = A.n_kv_heads * HS;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -108,20 +140,21 @@ __global__ __launch_bounds__(NWV * 64) void attn_decode_kernel(const AttnDecode 
     const float *__restrict__ vc = A.vcache;
     const uint32_t row_bytes = (uint32_t)kv_dim * 4u;
     const uint32_t lane_off = (uint32_t)(kvh * HS + ds * 8) * 4u;
-    const int t_last = t1 - 1;
+    const int t_last = max(t1 - 1, t0);
 
+    typedef float vec_v __attribute__((ext_vector_type(VE)));
+    const uint32_t v_off = (uint32_t)(kvh * HS + slice * VD + ds * VE) * 4u;
     struct Step {
-        float4 k0, k1, v0, v1;
+        float4 k0, k1;
+        vec_v v;
     };
-    // Unconditional loads: rows past the end re-read the last row, and the row
-    // of the new position is read although its values are replaced below.
+    // Unconditional loads: rows past the end re-read the last row.
     auto fetch = [&](int it, Step &d) {
         const int t = min(t0 + it * TSTEP + tl, t_last);
-        const uint32_t off = __umul24(t, row_bytes) + lane_off;
+        const uint32_t row = __umul24(t, row_bytes), off = row + lane_off;
         d.k0 = ld_at<float4>(kc, off);
         d.k1 = ld_at<float4>(kc, off + 16);
-        d.v0 = ld_at<float4>(vc, off);
-        d.v1 = ld_at<float4>(vc, off + 16);
+        d.v = ld_at<vec_v>(vc, row + v_off);
     };
     // The small loads that the staging below needs go out first: loads return in
     // order, so behind the first tile's loads they would wait for all of them.
@@ -161,14 +194,13 @@ __global__ __launch_bounds__(NWV * 64) void attn_decode_kernel(const AttnDecode 
     }
     // the new key, rotated, and the new value; the block whose range ends at pos
     // also writes them to the cache (:236-249)
-    const bool owns_new = (t1 == pos + 1);
     {
         const float first = nk_a * nc - nk_b * ns;
         const float second = nk_b * nc + first * ns;
         kvnew[0][hd] = first;
         kvnew[0][hd + HALF] = second;
         kvnew[1][tid & 127] = nv;
-        if (owns_new) {
+        if (owns_new && slice == 0) {
             if (tid < HALF) {
                 float *kw = A.kcache + (size_t)pos * kv_dim + kvh * HS;
                 kw[tid] = first;
@@ -192,16 +224,25 @@ __global__ __launch_bounds__(NWV * 64) void attn_decode_kernel(const AttnDecode 
             q[j][4] = b.x, q[j][5] = b.y, q[j][6] = b.z, q[j][7] = b.w;
         }
     }
-    float m[QG], l[QG], acc[QG][8];
-#pragma unroll
-    for (int j = 0; j < QG; j++) {
-        m[j] = kNoScore;
-        l[j] = 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; e++) acc[j][e] = 0.f;
-    }
     // log2(e) / sqrt(head_size): src/models.rs:154 divides the score by sqrt(head_size)
     const float scale = 1.44269504088896340736f / sqrtf((float)HS);
+    float m[QG], l[QG], acc[QG][VE];
+#pragma unroll
+    for (int j = 0; j < QG; j++) {
+        float s = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+            s = fmaf(kQInLds ? qs[j * HS + ds * 8 + e] : q[kQInLds ? 0 : j][e], kvnew[0][ds * 8 + e], s);
+        s += dpp_xchg<0xB1>(s);
+        s += dpp_xchg<0x4E>(s);
+        s += dpp_xchg<0x141>(s);
+        s += dpp_xchg<0x140>(s);
+        const bool mine = owns_new && tl == 0;
+        m[j] = mine ? s * scale : kNoScore;
+        l[j] = mine ? 1.f : 0.f;
+#pragma unroll
+        for (int e = 0; e < VE; e++) acc[j][e] = mine ? kvnew[1][slice * VD + ds * VE + e] : 0.f;
+    }
     const int n_it = (n + TSTEP - 1) / TSTEP;
     const int n_tiles = (n_it + PD - 1) / PD;
     for (int tile = 0; tile < n_tiles; tile++) {
@@ -215,7 +256,7 @@ __global__ __launch_bounds__(NWV * 64) void attn_decode_kernel(const AttnDecode 
         // all weights and weighted sums — so that the dependent chains of one step (dot product, four
         // cross-lane adds, exponential) interleave with those of the others: a block is often alone on its
         // CU, one wave per SIMD, and nothing else fills the gaps between dependent instructions.
-        float k[PD][8], v[PD][8];
+        float k[PD][8], v[PD][VE];
         float sc[PD][QG];
         bool valid[PD];
         float mt[QG];
@@ -225,19 +266,10 @@ __global__ __launch_bounds__(NWV * 64) void attn_decode_kernel(const AttnDecode 
             valid[u] = t < t1;
             const Step &d = pipe[u];
             const float kk[8] = {d.k0.x, d.k0.y, d.k0.z, d.k0.w, d.k1.x, d.k1.y, d.k1.z, d.k1.w};
-            const float vv[8] = {d.v0.x, d.v0.y, d.v0.z, d.v0.w, d.v1.x, d.v1.y, d.v1.z, d.v1.w};
 #pragma unroll
-            for (int e = 0; e < 8; e++) k[u][e] = kk[e], v[u][e] = vv[e];
-            if (__any(t == pos)) { // once per block: the row of the new position comes from LDS, not from the cache
-                const bool is_new = t == pos;
+            for (int e = 0; e < 8; e++) k[u][e] = kk[e];
 #pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    k[u][e] = is_new ? kvnew[0][ds * 8 + e] : k[u][e];
-                    v[u][e] = is_new ? kvnew[1][ds * 8 + e] : v[u][e];
-                }
-            }
-#pragma unroll
-            for (int e = 0; e < 8; e++) v[u][e] = valid[u] ? v[u][e] : 0.f; // a row past the end may hold anything, NaN included
+            for (int e = 0; e < VE; e++) v[u][e] = valid[u] ? d.v[e] : 0.f; // a row past the end may hold anything, NaN included
         }
 #pragma unroll
         for (int j = 0; j < QG; j++) {
@@ -276,7 +308,7 @@ __global__ __launch_bounds__(NWV * 64) void attn_decode_kernel(const AttnDecode 
                 const float c = exp2_fast(m[j] - m_new);
                 l[j] *= c;
 #pragma unroll
-                for (int e = 0; e < 8; e++) acc[j][e] *= c;
+                for (int e = 0; e < VE; e++) acc[j][e] *= c;
                 m[j] = m_new;
             }
         }
@@ -287,38 +319,39 @@ __global__ __launch_bounds__(NWV * 64) void attn_decode_kernel(const AttnDecode 
                 const float p = valid[u] ? exp2_fast(sc[u][j] - m[j]) : 0.f;
                 l[j] += p;
 #pragma unroll
-                for (int e = 0; e < 8; e++) acc[j][e] = fmaf(p, v[u][e], acc[j][e]);
+                for (int e = 0; e < VE; e++) acc[j][e] = fmaf(p, v[u][e], acc[j][e]);
             }
         }
     }
 
     if constexpr (!kRowsInLds) {
         // merge the 4 rows of the wave (lanes 16 and 32 apart hold the same dims)
-#pragma unroll
-        for (int step = 16; step <= 32; step *= 2) {
+        auto merge = [&](auto both) __attribute__((always_inline)) {
 #pragma unroll
             for (int j = 0; j < QG; j++) {
-                const float mo = __shfl_xor(m[j], step);
-                const float lo = __shfl_xor(l[j], step);
-                const float M = fmaxf(m[j], mo);
-                const float w1 = exp2_fast(m[j] - M), w2 = exp2_fast(mo - M);
-                l[j] = l[j] * w1 + lo * w2;
+                const Both mb = both(m[j]), lb = both(l[j]);
+                const float M = fmaxf(mb.lo, mb.hi);
+                const float w1 = exp2_fast(mb.lo - M), w2 = exp2_fast(mb.hi - M);
+                l[j] = lb.lo * w1 + lb.hi * w2;
 #pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    const float ao = __shfl_xor(acc[j][e], step);
-                    acc[j][e] = acc[j][e] * w1 + ao * w2;
+                for (int e = 0; e < VE; e++) {
+                    const Both a = both(acc[j][e]);
+                    acc[j][e] = a.lo * w1 + a.hi * w2;
                 }
                 m[j] = M;
             }
-        }
+        };
+        merge([](float v) { return both16(v); });
+        merge([](float v) { return both32(v); });
     }
     if (kRowsInLds || lane < 16) {
         const int slot = kRowsInLds ? wave * 4 + (lane >> 4) : wave;
 #pragma unroll
         for (int j = 0; j < QG; j++) {
-            *reinterpret_cast<float4 *>(&comb[slot][j][ds * 8]) = make_float4(acc[j][0], acc[j][1], acc[j][2], acc[j][3]);
-            *reinterpret_cast<float4 *>(&comb[slot][j][ds * 8 + 4]) =
-                make_float4(acc[j][4], acc[j][5], acc[j][6], acc[j][7]);
+            vec_v a;
+#pragma unroll
+            for (int e = 0; e < VE; e++) a[e] = acc[j][e];
+            *reinterpret_cast<vec_v *>(&comb[slot][j][ds * VE]) = a;
             if (ds == 0) {
                 comb[slot][j][HS] = m[j];
                 comb[slot][j][HS + 1] = l[j];
@@ -351,8 +384,8 @@ __global__ __launch_bounds__(NWV * 64) void attn_decode_kernel(const AttnDecode 
         __syncthreads();
     }
     // merge; one thread per (head, dim)
-    for (int idx = tid; idx < QG * HS; idx += NT) {
-        const int j = idx >> 7, d = idx & 127;
+    for (int idx = tid; idx < QG * VD; idx += NT) {
+        const int j = idx / VD, d = idx % VD, dv = slice * VD + d;
         float M, num = 0.f, den = 0.f;
         if constexpr (kRowsInLds) {
 #pragma unroll
@@ -372,12 +405,12 @@ __global__ __launch_bounds__(NWV * 64) void attn_decode_kernel(const AttnDecode 
         }
         const int h = kvh * QG + j;
         if (A.n_splits == 1) {
-            const int i = h * HS + d;
+            const int i = h * HS + dv;
             A.out[A.scatter ? A.scatter[i] : i] = num / den;
         } else {
             float *p = A.part + ((size_t)h * A.max_splits + sp) * (HS + 2);
-            p[d] = num;
-            if (d == 0) {
+            p[dv] = num;
+            if (dv == 0) {
                 p[HS] = M;
                 p[HS + 1] = den;
             }
@@ -1097,8 +1130,22 @@ __global__ __launch_bounds__(512) void attn_combine_kernel(const AttnDecode A) {
     }
 }
 
+template <int QG, int NWV, int DS>
+int attn_launch_sliced(const AttnDecode &a, hipStream_t st) {
+    hipLaunchKernelGGL((attn_decode_kernel<QG, NWV, DS>), dim3(a.n_kv_heads, 1, DS), dim3(NWV * 64), 0, st, a);
+    L2_HIP(hipGetLastError());
+    return L2_OK;
+}
+
 template <int QG>
 int attn_launch_qg(const AttnDecode &a, hipStream_t st) {
+    if constexpr (QG <= 4) {
+        if (a.n_splits == 1) { // slices of the head: as many as keep one block per CU
+            const bool wide = a.pos >= (QG <= 2 ? 64 : 128), eight = a.n_kv_heads * 8 <= cu_count();
+            if (eight) return wide ? attn_launch_sliced<QG, 8, 8>(a, st) : attn_launch_sliced<QG, 4, 8>(a, st);
+            return wide ? attn_launch_sliced<QG, 8, 4>(a, st) : attn_launch_sliced<QG, 4, 4>(a, st);
+        }
+    }
     if constexpr (QG >= 4) {
         static const bool valu = []() {
             const char *v = getenv("L2_ATTN_IMPL");
@@ -1113,9 +1160,9 @@ int attn_launch_qg(const AttnDecode &a, hipStream_t st) {
     constexpr size_t lds = QG >= 4 ? (size_t)16 * QG * kCombRow * sizeof(float) : 0; // the partial results of 16 rows
     if (lds > 48 * 1024) {
         static LdsLimit limit; // per instantiation
-        L2_TRY(limit.ensure(reinterpret_cast<const void *>(attn_decode_kernel<QG, 4>), lds));
+        L2_TRY(limit.ensure(reinterpret_cast<const void *>(attn_decode_kernel<QG, 4, 1>), lds));
     }
-    hipLaunchKernelGGL((attn_decode_kernel<QG, 4>), dim3(a.n_kv_heads, a.n_splits), dim3(256), lds, st, a);
+    hipLaunchKernelGGL((attn_decode_kernel<QG, 4, 1>), dim3(a.n_kv_heads, a.n_splits), dim3(256), lds, st, a);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }

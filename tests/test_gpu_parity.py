@@ -225,6 +225,28 @@ def test_decode_attention_long_context(ops, oracle, n_heads, n_kv, ctx):
     o.close()
 
 
+@pytest.mark.parametrize("n_heads,n_kv", [(2, 2), (4, 2), (8, 2), (8, 1), (33, 33)],
+                         ids=["mha", "gqa2", "gqa4", "gqa8", "33_kv_heads"])
+def test_decode_attention_tile_edges(ops, oracle, n_heads, n_kv):
+    """Decode steps at the edges of the attention's steps, tiles, block shapes and splits, first position included."""
+    dims = ck.Dims(dim=128 * n_heads, hidden_dim=512, n_layers=1, n_heads=n_heads, n_kv_heads=n_kv,
+                   vocab_size=300, seq_len=600, group_size=128)
+    img = ck.synth_weights_image(dims, seed=8)
+    m = ops.Model(img, dims)
+    o = oracle.Model(img, dims)
+    o.new_state()
+    m.fill_kv_synthetic(0, 590, seed=4)
+    ko, vo = o.kv_cache()
+    ko[0, :590], vo[0, :590] = m.read_kv(0, 0, 590)
+    for pos in (0, 1, 15, 16, 17, 63, 64, 65, 127, 128, 129, 255, 256, 257, 511, 512, 513, 577):
+        want = o.transformer([11], [pos])
+        assert nrel(m.forward([11], [pos]), want) < REL_FP32, pos
+    k, v = m.read_kv(0, 0, 590)
+    assert nrel(k, ko[0, :590]) < REL_FP32 and nrel(v, vo[0, :590]) < REL_FP32
+    m.close()
+    o.close()
+
+
 _VALU_ATTN_SNIPPET = r"""
 import sys, numpy as np
 sys.path.insert(0, sys.argv[1]); sys.path.insert(0, sys.argv[2])
