@@ -843,7 +843,7 @@ static int batch_planes(const l2_model *m, int B) {
     if (B < 2 || m->prefill_mode == L2_PREFILL_COLUMNS || m->d.dim > kGemmMaxDim || m->d.hidden_dim > kGemmMaxHidden) return 0;
     if (m->prefill_mode == L2_PREFILL_MFMA) return 1; // quantised models only
     if (!gemm_pays_layer(B, layer_weights(m))) return 0;
-    return m->d.group_size == 0 ? kDensePlanes : 3;
+    return 3;
 }
 
 // The same for the stand-alone operator.
@@ -1329,10 +1329,13 @@ extern "C" int l2_model_qmatvec(l2_model *m, int layer, int proj, const float *x
         hipStream_t st = m->stream;
         L2_HIP(hipMemcpyAsync(m->op_x, x_host, (size_t)B * q.in * 4, hipMemcpyHostToDevice, st));
         if (operator_planes(q, B, m->prefill_mode) && q.in == gemm_padded(q.in)) {
-            L2_TRY(operator_bufs(m->op_batch, q, B, kDensePlanes, st));
+            L2_TRY(operator_bufs(m->op_batch, q, B, 3, st));
+            GemmInput in{};
+            in.out[0] = m->op_batch.planes, in.x = m->op_x, in.n = 1;
+            L2_TRY(gemm_input_launch(in, q.in, B, 3, st));
             Q4Launch L = launch_of(q, B, 0.f);
             L.m[0] = mat_of(q, nullptr, nullptr, m->op_y);
-            L2_TRY(gemm_launch(L, XhList{{m->op_x, nullptr, nullptr}}, nullptr, m->op_batch.ws, m->op_batch.ws_floats, kDensePlanes, B, st));
+            L2_TRY(gemm_launch(L, XhList{{m->op_batch.planes, nullptr, nullptr}}, nullptr, m->op_batch.ws, m->op_batch.ws_floats, 3, B, st));
         } else {
             DenseArgs a{};
             a.y = m->op_y, a.w = q.dense, a.x = m->op_x, a.in = q.in, a.out = q.out, a.batch = B;

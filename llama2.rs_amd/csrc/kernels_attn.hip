@@ -1066,9 +1066,7 @@ void attn_prefill_mfma16_kernel(void *__restrict__ out, const float *__restrict_
                 const int i = (kvh * QG + j % QG) * HS + d;
                 const int dst = scatter ? scatter[i] : i;
                 const float v = nu / de;
-                if constexpr (NP == kDensePlanes) {
-                    reinterpret_cast<float *>(out)[(size_t)qi * dim + dst] = v;
-                } else if constexpr (NP == 1) {
+                if constexpr (NP == 1) {
                     reinterpret_cast<_Float16 *>(out)[(size_t)qi * dim + h16_slot(dst)] = (_Float16)v;
                 } else { // three bf16 numbers that add up to v exactly
                     uint16_t *o = reinterpret_cast<uint16_t *>(out) + (size_t)qi * NP * dim + b16_slot(dst);
@@ -1206,7 +1204,6 @@ static int prefill_qg(void *out, int planes, const float *q, const float *kc, co
     switch (planes) {
         case 0: hipLaunchKernelGGL(attn_prefill_kernel<QG>, dim3(n_kv_heads, (B * QG + 7) / 8), block, 0, st, (float *)out, q, kc, vc, pos, scatter, n_heads, n_kv_heads, B); break;
         case 1: L2_PREFILL_ATTN(1);
-        case kDensePlanes: L2_PREFILL_ATTN(kDensePlanes);
         case 3: L2_PREFILL_ATTN(3);
         default: return l2_fail(L2_ERR_ARG, "attention: %d planes", planes);
     }

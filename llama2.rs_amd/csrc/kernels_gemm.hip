@@ -26,10 +26,10 @@
 
 namespace {
 
-typedef float f16v __attribute__((ext_vector_type(16)));
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+typedef __bf16 b2 __attribute__((ext_vector_type(2)));
 typedef float v2f __attribute__((ext_vector_type(2)));
 
 union Frag {
@@ -69,10 +69,7 @@ struct Piece {
 template <int NP>
 __device__ __forceinline__ Piece<NP> make_piece(const float (&v)[8]) {
     Piece<NP> r;
-    if constexpr (NP == kDensePlanes) {
-        r.q[0] = __builtin_bit_cast(uint4, make_float4(v[0], v[1], v[2], v[3]));
-        r.q[1] = __builtin_bit_cast(uint4, make_float4(v[4], v[5], v[6], v[7]));
-    } else if constexpr (NP == 1) {
+    if constexpr (NP == 1) {
         Frag f;
         f.p[0] = h2{(_Float16)v[0], (_Float16)v[4]};
         f.p[1] = h2{(_Float16)v[1], (_Float16)v[5]};
@@ -98,12 +95,12 @@ __device__ __forceinline__ Piece<NP> make_piece(const float (&v)[8]) {
     return r;
 }
 
-// Plane p of token t: [t][p][in_p], in_p = the row padded to whole K steps (fp32: [t][in_p]).
+// Plane p of token t: [t][p][in_p], in_p = the row padded to whole K steps.
 template <int NP>
 __device__ __forceinline__ void store_piece(void *out, size_t t, int in_p, int j8, const Piece<NP> &r) {
     uint4 *dst = reinterpret_cast<uint4 *>(reinterpret_cast<uint16_t *>(out) + t * NP * in_p);
 #pragma unroll
-    for (int p = 0; p < NP; p++) dst[NP == kDensePlanes ? 2 * j8 + p : p * (in_p >> 3) + j8] = r.q[p];
+    for (int p = 0; p < NP; p++) dst[p * (in_p >> 3) + j8] = r.q[p];
 }
 
 // x[b][g_index[j]] * wn[g_index[j]] -> planes: the gather of src/gptq.rs:110-114 and the norm weight of
@@ -115,7 +112,10 @@ __global__ __launch_bounds__(256) void gemm_input_kernel(const GemmInput A, int 
     if (j8 * 8 >= in_p) return;
     const float *x = A.x + (size_t)b * n;
     float v[8];
-    if (j8 * 8 < n) {
+    if (j8 * 8 < n && !A.g_index[c]) { // no act-order: the model without quantisation
+        const float4_any a = reinterpret_cast<const float4_any *>(x)[2 * j8], b4 = reinterpret_cast<const float4_any *>(x)[2 * j8 + 1];
+        v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b4.x, v[5] = b4.y, v[6] = b4.z, v[7] = b4.w;
+    } else if (j8 * 8 < n) {
         const int4 g0 = reinterpret_cast<const int4 *>(A.g_index[c])[2 * j8], g1 = reinterpret_cast<const int4 *>(A.g_index[c])[2 * j8 + 1];
         const int g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
 #pragma unroll
@@ -452,145 +452,252 @@ __global__ __launch_bounds__(64 * NW, NT == 1 ? 3 : 2) void q4_tile_gemm_kernel(
 }
 
 // Linear::matvec<B> of the model without quantisation (src/model.rs:22-31) for a batch: fp32 weights, fp32 activations,
-// fp32 products and sums (v_mfma_f32_32x32x2_f32, 157 TFLOP/s on this chip; it is what bounds the kernel, the loads hide
-// behind it).  The matvec kernel once per column read the weights once per column: two layers of 7B's widths, 99 columns
-// 16 -> 1 ms.
+// on the bf16 matrix cores.  The activations are three bf16 planes as above; the weights become three on the way in, each
+// rounded to nearest, so that what a plane leaves over has either sign.  Of the nine products of a weight and an activation
+// the six down to 2^-16 of the first are taken; the other three are below 2^-24, of either sign and average out.  That is
+// 6 products at 2.5 PFLOP/s against one at the 157 TFLOP/s of v_mfma_f32_32x32x2_f32.
 //
-// A block is four waves of NB tiles of 32 rows x 32 columns, side by side over the rows.  Lane (r = l % 32, h = l / 32)
-// loads inputs 16 h .. 16 h + 15 of every 32 of its row, 16 bytes at a time; step e of float4 i multiplies inputs 4 i + e
-// and 16 + 4 i + e.  The activations' 32 inputs per column pass through LDS, double-buffered.
+// Sums: the six products of 32 inputs from zero, the smallest first, so that one addition of the matrix unit sees the whole
+// of them; every other 32 inputs enter negated, as above; 32 inputs to each other in runs and the runs to each other in fp32 as the vector ALU rounds
+// it, the slices of K in a tree.  Runs of sqrt(steps / 2) and more make the two chains about equally long.
 //
-// Sums.  The matrix unit rounds once per product, and the error of a sum of n terms, each added to all before it, grows
-// with n.  The matvec adds 64 lanes' shares in a tree, so that in / 64 products follow each other; to be no further from
-// the exact sum than that, the products of a K step (of a part of it where the matvec's own chains are short) are summed
-// from zero, the steps of a run are added to each other, and the runs; the slices of K follow in a tree (sum_slices_n).
-// Runs of sqrt(steps / 2) and more make the two upper chains about equally long.  Relative rms error against fp64, normal
-// inputs, matvec / this / one accumulator for the whole slice: 1024 inputs, 61 columns 1.00e-7 / 9.1e-8 / 2.1e-7; 4096,
-// 128 columns 1.59e-7 / 1.27e-7 / 4.1e-7; 11008, 512 columns 2.44e-7 / 1.44e-7 / 9.4e-7.
-// The sums take the registers of a second row tile (which would reuse every LDS read twice: the matrix unit is slow enough
-// in fp32 for one).  Prompts, two row tiles and one accumulator / this: two layers of 7B's widths, 100 tokens 0.95-0.99 /
-// 0.98 ms, 512 tokens 3.60 / 3.41; four layers of 1024 inputs, 33 tokens 0.29 / 0.31; one of 70B's widths, 64 tokens
-// 1.09-1.13 / 1.12-1.17.
-template <int NB, int FOLDS> // FOLDS: sums from zero per K step
-__global__ __launch_bounds__(256, FOLDS == 4 ? 2 : 3) void dense_gemm_kernel(const Q4Launch L, const XhList xl, int in_p,
-                                                            const float *__restrict__ ss, float *__restrict__ ws, int KS,
-                                                            int t_tiles, int partials) {
-    constexpr int TN = 32 * NB, RB = 128, kRow = 36; // floats per staged column: 32 + 4
-    __shared__ __align__(16) float xs[4608]; // [2][TN][kRow], and the four output tiles of the epilogue
-    static_assert(2 * TN * kRow <= 4608 && 4 * 32 * 36 <= 4608, "LDS");
-    const int n_blocks = gridDim.x, per_xcd = n_blocks >> 3, over = n_blocks & 7, xcd = blockIdx.x & 7;
-    const int work = xcd * per_xcd + min(xcd, over) + (blockIdx.x >> 3); // as in q4_tile_gemm_kernel
-    int rb = work / t_tiles, mi = 0;
-    const int t0 = (work - rb * t_tiles) * TN;
-    const int row_blocks = n_blocks / (t_tiles * KS), ks = rb / row_blocks;
-    rb -= ks * row_blocks;
+// Infinities and NaN: the planes of an infinity are not one (inf - inf), so a sum that comes out as neither number is done
+// again in fp32 from what the planes stand for (dense_again).
+//
+// A wave owns 16 rows x 16 NT tokens, a block 8 waves over the rows: a weight is read and split once for up to 128 tokens.
+// Lane (row r = l % 16, kg = l / 16) loads 8 consecutive weights of each 32 inputs (a row's cache line, in two loads), four
+// such pairs ahead, and splits 32 inputs ahead of the products; the activations of 64 inputs pass through LDS,
+// double-buffered.  What bounds it is issue: a step of 64 inputs and 112 tokens is 437 instructions per wave, 84 of them
+// products (1344 cycles), 88 the splitting, and two waves per SIMD take some 5500 cycles for it.
+//
+// Against products in v_mfma_f32_32x32x2_f32 (128 rows x 64 columns per block, every weight read for each): one layer of 7B's
+// widths, 33, 64, 100, 200, 512 columns 327 / 331 / 531 / 1039 / 1846 -> 272 / 305 / 413 / 751 / 1320 us; w1|w3 alone at 99 columns
+// 234 -> 165; 32 rows x 64 tokens per wave: 190.  Relative rms error against fp64, normal inputs, 33 to 300 columns of 1024 / 4096 /
+// 11008 inputs: 9.1e-8 / 1.3e-7 / 1.4e-7 -> 7.4e-8 / 0.94e-7 / 1.0e-7 (the matvec 1.0e-7 / 1.6e-7 / 2.4e-7); without the
+// negation 8.2e-8 / 1.2e-7 / 1.5e-7.
+constexpr int kDenseWaves = 8, kDenseRows = 16 * kDenseWaves;
+template <int NT>
+struct DenseLds {
+    static constexpr int kPlane = 16 * NT * kStepRow, kTile = 3 * kPlane, kSize = 2 * kTile;
+};
+
+// One output over the inputs k0..k1-1 in plain fp32.
+__device__ __forceinline__ float dense_again(const float *w, const uint16_t *x, int in_p, int k0, int k1) {
+    float s = 0.f;
+#pragma unroll 1
+    for (int k = k0; k < k1; k++) {
+        const uint16_t *q = x + b16_slot(k);
+        auto plane = [&](int p) { return __builtin_bit_cast(float, (uint32_t)q[(size_t)p * in_p] << 16); };
+        const float hi = plane(0);
+        s = fmaf(w[k], __builtin_isfinite(hi) ? hi + (plane(1) + plane(2)) : hi, s);
+    }
+    return s;
+}
+
+template <int NT>
+__device__ __forceinline__ void dense_tile(const Q4Launch &L, const XhList &xl, int in_p, const float *__restrict__ ss, float *__restrict__ ws,
+                                           int KS, int partials, int rb, int ks, int t0) {
+    using S = DenseLds<NT>;
+    constexpr int NP = 3, TN = 16 * NT, THREADS = 64 * kDenseWaves;
+    extern __shared__ __align__(16) char lds[];
+    int mi = 0;
     while (mi + 1 < L.n_mats && rb >= L.m[mi].row_blocks) {
         rb -= L.m[mi].row_blocks;
         mi++;
     }
     const void *__restrict__ const xh = xl.p[mi];
     const void *__restrict__ const w = L.m[mi].qweight;
-    asm volatile("" ::"s"(xh), "s"(w));
     const int n_out = L.m[mi].out, in = L.in, B = L.batch;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int r = lane & 31, h = lane >> 5;
-    const int n_unit = in / 32;
+    const int r = lane & 15, kg = lane >> 4;
+    const int obase = rb * kDenseRows + wave * 16;
+    const int n_unit = in_p / 64;
     const int it0 = (int)((long)n_unit * ks / KS), it1 = (int)((long)n_unit * (ks + 1) / KS);
-    const int obase = rb * RB + wave * 32;
-    const uint32_t wrow = ((uint32_t)min(obase + r, n_out - 1) * (uint32_t)in + 16 * h) * 4u;
-    uint32_t xoff[NB];
+
+    // activations: pieces of 16 bytes, 8 to a token's 64 inputs in a plane
+    constexpr int PIECES = NP * TN * 8, XP = (PIECES + THREADS - 1) / THREADS;
+    uint32_t xoff[XP], xput[XP];
 #pragma unroll
-    for (int p = 0; p < NB; p++) xoff[p] = ((uint32_t)min(t0 + p * 32 + (tid >> 3), B - 1) * (uint32_t)in_p + (tid & 7) * 4) * 4u;
-    struct WStage {
-        float4 w[4];
-    };
-    auto fetch_w = [&](int it, WStage &d) __attribute__((always_inline)) {
-        const uint32_t c = (uint32_t)min(it, it1 - 1) * 128u;
-#pragma unroll
-        for (int i = 0; i < 4; i++) d.w[i] = ld_at<float4>(w, wrow + c + 16u * i);
-    };
-    float4 xr[NB];
+    for (int i = 0; i < XP; i++) {
+        const int q = (tid + i * THREADS) % PIECES, t = (q >> 3) % TN, p = q / (8 * TN), j = q & 7; // some twice, if it does not divide
+        xoff[i] = ((uint32_t)min(t0 + t, B - 1) * NP + p) * (uint32_t)in_p * 2u + j * 16u;
+        xput[i] = (uint32_t)(p * S::kPlane + t * kStepRow + ((j ^ ((t >> 1) & 7)) << 4));
+    }
+    uint4 xr[XP];
     auto fetch_x = [&](int it) __attribute__((always_inline)) {
 #pragma unroll
-        for (int p = 0; p < NB; p++) xr[p] = ld_at<float4>(xh, xoff[p] + (uint32_t)min(it, it1 - 1) * 128u);
+        for (int i = 0; i < XP; i++) xr[i] = ld_at<uint4>(xh, xoff[i] + (uint32_t)min(it, it1 - 1) * 128u);
     };
-    auto store_x = [&](int buf) __attribute__((always_inline)) {
+    auto store_x = [&](uint32_t tile) __attribute__((always_inline)) {
 #pragma unroll
-        for (int p = 0; p < NB; p++) *reinterpret_cast<float4 *>(xs + (buf * TN + p * 32 + (tid >> 3)) * kRow + (tid & 7) * 4) = xr[p];
+        for (int i = 0; i < XP; i++) *reinterpret_cast<uint4 *>(lds + tile + xput[i]) = xr[i];
     };
-    f16v run[NB], acc[NB];
+    uint32_t xread[2];
 #pragma unroll
-    for (int nb = 0; nb < NB; nb++) run[nb] = acc[nb] = f16v{};
-    int run_steps = 2; // K steps per run
-    while (2 * run_steps * run_steps < it1 - it0) run_steps *= 2;
-    WStage wr[2];
-    fetch_x(it0);
-    fetch_w(it0, wr[0]);
-    store_x(0);
-    __syncthreads();
-    auto k_step = [&](const int it, const int u) __attribute__((always_inline)) {
-        fetch_x(it + 1);
-        fetch_w(it + 1, wr[u ^ 1]);
-        __builtin_amdgcn_sched_barrier(0); // requested before this step's arithmetic, not behind it
-        const float *xb = xs + u * TN * kRow;
-        f16v even[NB]; // of four sums, pairs are added first
-#pragma unroll
-        for (int f = 0; f < FOLDS; f++) {
-            constexpr int N = 4 / FOLDS;
-            f16v sum[NB];
-#pragma unroll
-            for (int i = f * N; i < (f + 1) * N; i++) {
-                float4 b[NB];
-#pragma unroll
-                for (int nb = 0; nb < NB; nb++) b[nb] = *reinterpret_cast<const float4 *>(xb + (nb * 32 + r) * kRow + 16 * h + 4 * i);
-#pragma unroll
-                for (int e = 0; e < 4; e++)
-#pragma unroll
-                    for (int nb = 0; nb < NB; nb++)
-                        sum[nb] = __builtin_amdgcn_mfma_f32_32x32x2f32((&wr[u].w[i].x)[e], (&b[nb].x)[e],
-                                                                       i == f * N && e == 0 ? f16v{} : sum[nb], 0, 0, 0);
-            }
-#pragma unroll
-            for (int nb = 0; nb < NB; nb++) {
-                if (FOLDS < 4) run[nb] += sum[nb];
-                else if (f & 1) run[nb] += even[nb] + sum[nb];
-                else even[nb] = sum[nb];
-            }
-        }
-        store_x(u ^ 1);
-        __syncthreads();
-    };
-    int it = it0;
-    for (int end = it0 + run_steps; it + 1 < it1; it += 2) {
-        k_step(it, 0);
-        k_step(it + 1, 1);
-        if (it + 2 == end) {
-            end += run_steps;
-#pragma unroll
-            for (int nb = 0; nb < NB; nb++) acc[nb] += run[nb], run[nb] = f16v{};
-        }
-    }
-    if (it < it1) k_step(it, 0);
-#pragma unroll
-    for (int nb = 0; nb < NB; nb++) acc[nb] += run[nb];
+    for (int k = 0; k < 2; k++) xread[k] = (uint32_t)r * kStepRow + (((4 * k + kg) ^ ((r >> 1) & 7)) << 4);
 
+    // weights: half h of the K steps is 32 inputs, 8 kg .. 8 kg + 7 the lane's.  Inputs beyond the row are zero in the
+    // activations; their weights are the row's last ones again.
+    struct Raw {
+        float4 v[2];
+    };
+    const uint32_t wrow = (uint32_t)min(obase + r, n_out - 1) * (uint32_t)in * 4u;
+    const int h_last = 2 * it1 - 1;
+    auto fetch_w = [&](int h, Raw &d) __attribute__((always_inline)) {
+        const uint32_t c = wrow + (uint32_t)min(min(h, h_last) * 32 + 8 * kg, in - 8) * 4u;
+#pragma unroll
+        for (int i = 0; i < 2; i++) d.v[i] = ld_at<float4>(w, c + 16u * i);
+    };
+    Raw raw[4];
+    Frag a[2][NP]; // [half][plane]
+    auto split = [&](const int from, const int half, const int i) __attribute__((always_inline)) { // a pair of weights, of four
+        constexpr int order[8] = {0, 2, 4, 6, 1, 3, 5, 7}; // the activations' slots
+        float x = (&raw[from].v[order[2 * i] >> 2].x)[order[2 * i] & 3], y = (&raw[from].v[order[2 * i + 1] >> 2].x)[order[2 * i + 1] & 3];
+        if (half == 1) x = -x, y = -y;
+#pragma unroll
+        for (int p = 0; p < NP; p++) {
+            const uint32_t b = __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{x, y}, b2));
+            a[half][p].u[i] = b;
+            if (p < NP - 1) x -= __builtin_bit_cast(float, b << 16), y -= __builtin_bit_cast(float, b & 0xFFFF0000u);
+        }
+    };
+
+    f4v top[NT], run[NT], sum[4]; // sums of the runs, of the current run; of 32 inputs
+#pragma unroll
+    for (int n = 0; n < NT; n++) top[n] = run[n] = f4v{0.f, 0.f, 0.f, 0.f};
+    // The products of a half step go by pairs of token tiles, whose chains do not wait for each other.
+    constexpr int PAIRS = (NT + 1) / 2;
+    Frag b[4][NP];
+    auto read_x = [&](const int pair, uint32_t tile) __attribute__((always_inline)) { // of the step's 2 PAIRS
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const int n = pair % PAIRS * 2 + u;
+            if (n < NT) {
+#pragma unroll
+                for (int p = 0; p < NP; p++)
+                    b[(pair & 1) * 2 + u][p].q = *reinterpret_cast<const uint4 *>(lds + xread[pair / PAIRS] + tile + p * S::kPlane + n * 16 * kStepRow);
+            }
+        }
+    };
+    auto fold = [&](const int pair) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const int n = pair % PAIRS * 2 + u;
+            if (n < NT) {
+                if (pair < PAIRS) run[n] += sum[(pair & 1) * 2 + u];
+                else run[n] -= sum[(pair & 1) * 2 + u];
+                asm volatile("" : "+v"(run[n])); // here, and not where the compiler would rather have it
+            }
+        }
+    };
+    int run_len = 1; // K steps per run
+    while (4 * run_len * run_len < it1 - it0) run_len *= 2;
+    int end = it0 + run_len;
+    uint32_t tile = 0;
+    auto step = [&](const int it, const int par) __attribute__((always_inline)) {
+        store_x(tile ^ S::kTile);
+        fetch_x(it + 2);
+        read_x(0, tile);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int g = 0; g < 2 * PAIRS; g++) {
+            const int k = g / PAIRS, next = (2 * par + k + 1) & 3; // the half whose weights are split meanwhile
+            if (g + 1 < 2 * PAIRS) read_x(g + 1, tile);
+            if (g > 0) fold(g - 1);
+            constexpr int pa[6] = {2, 1, 0, 1, 0, 0}, pb[6] = {0, 1, 2, 0, 1, 0};
+#pragma unroll
+            for (int q = 0; q < 6; q++)
+#pragma unroll
+                for (int u = 0; u < 2; u++) {
+                    const int at = (g & 1) * 2 + u;
+                    if (g % PAIRS * 2 + u < NT)
+                        sum[at] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[k][pa[q]].b, b[at][pb[q]].b, q == 0 ? f4v{} : sum[at], 0, 0, 0);
+                }
+#pragma unroll
+            for (int i = g % PAIRS * 4 / PAIRS; i < (g % PAIRS + 1) * 4 / PAIRS; i++) split(next, k ^ 1, i);
+            __builtin_amdgcn_sched_barrier(0);
+            if (g % PAIRS == PAIRS - 1) { // after the last use of what was there: a load hoisted above it costs copies that wait for it
+#pragma unroll
+                for (int p = 0; p < NP; p++) asm volatile("" : "+v"(a[k ^ 1][p].b));
+                fetch_w(2 * it + k + 5, raw[next]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        fold(2 * PAIRS - 1);
+        if (it + 1 == end) {
+            end += run_len;
+#pragma unroll
+            for (int n = 0; n < NT; n++) top[n] += run[n], run[n] = f4v{0.f, 0.f, 0.f, 0.f};
+        }
+        __syncthreads();
+        tile ^= S::kTile;
+    };
+    // the first requests, in the order of the loop, so that its waits are the steady state's
+    fetch_x(it0);
+    fetch_w(2 * it0, raw[0]);
+    fetch_w(2 * it0 + 1, raw[1]);
+    fetch_w(2 * it0 + 2, raw[2]);
+    store_x(0);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_x(it0 + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_w(2 * it0 + 3, raw[3]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 4; i++) split(0, 0, i);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_w(2 * it0 + 4, raw[0]);
+    __syncthreads();
+    int it = it0;
+    for (; it + 1 < it1; it += 2) step(it, 0), step(it + 1, 1);
+    if (it < it1) step(it, 0);
+#pragma unroll
+    for (int n = 0; n < NT; n++) top[n] += run[n];
+
+    // C layout: lane (column r = token, kg), register e -> row 4 kg + e
     size_t ws_base = 0;
     for (int i = 0; i < mi; i++) ws_base += (size_t)KS * B * L.m[i].out;
-    float *tile = xs + wave * 32 * 36;
-    const int tl = lane >> 3, oc = (lane & 7) * 4;
+    const int o = obase + 4 * kg;
 #pragma unroll
-    for (int nb = 0; nb < NB; nb++) {
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-            *reinterpret_cast<float4 *>(&tile[r * 36 + q * 8 + h * 4]) =
-                make_float4(acc[nb][4 * q], acc[nb][4 * q + 1], acc[nb][4 * q + 2], acc[nb][4 * q + 3]);
-#pragma unroll
-        for (int pass = 0; pass < 4; pass++) {
-            const int tt = pass * 8 + tl;
-            float4 v = *reinterpret_cast<const float4 *>(&tile[tt * 36 + oc]);
-            const int t = t0 + nb * 32 + tt, o = obase + oc;
-            if (t < B && o < n_out) finish4(L, mi, ss, ws + ws_base, KS, ks, partials, t, o, v);
+    for (int n = 0; n < NT; n++) {
+        const int t = t0 + n * 16 + r;
+        if (t >= B || o >= n_out) continue;
+        float4 v = make_float4(top[n][0], top[n][1], top[n][2], top[n][3]);
+        if (!__builtin_isfinite((v.x + v.y) + (v.z + v.w))) {
+            const uint16_t *xt = reinterpret_cast<const uint16_t *>(xh) + (size_t)t * NP * in_p;
+            const float *wo = reinterpret_cast<const float *>(w) + (size_t)o * in;
+            const int k0 = it0 * 64, k1 = min(it1 * 64, in);
+            v = make_float4(dense_again(wo, xt, in_p, k0, k1), dense_again(wo + in, xt, in_p, k0, k1),
+                            dense_again(wo + 2 * (size_t)in, xt, in_p, k0, k1), dense_again(wo + 3 * (size_t)in, xt, in_p, k0, k1));
         }
+        finish4(L, mi, ss, ws + ws_base, KS, ks, partials, t, o, v);
+    }
+}
+
+// NT: the tiles of tokens of a block at most; the last one has as many as it needs.
+template <int NT>
+__global__ __launch_bounds__(64 * kDenseWaves, 2) void dense_gemm_kernel(const Q4Launch L, const XhList xl, int in_p,
+                                                                         const float *__restrict__ ss, float *__restrict__ ws, int KS,
+                                                                         int t_tiles, int partials) {
+    const int work = xcd_item(blockIdx.x, gridDim.x); // as in q4_tile_gemm_kernel
+    int rb = work / t_tiles;
+    const int t0 = (work - rb * t_tiles) * 16 * NT, need = min(NT, (L.batch - t0 + 15) / 16);
+    const int row_blocks = gridDim.x / (t_tiles * KS), ks = rb / row_blocks;
+    rb -= ks * row_blocks;
+    switch (need) {
+#define DENSE_TILE(n) \
+    case n: \
+        if constexpr (n <= NT) dense_tile<n>(L, xl, in_p, ss, ws, KS, partials, rb, ks, t0); \
+        break
+        DENSE_TILE(1);
+        DENSE_TILE(2);
+        DENSE_TILE(3);
+        DENSE_TILE(4);
+        DENSE_TILE(5);
+        DENSE_TILE(6);
+        DENSE_TILE(7);
+        DENSE_TILE(8);
+#undef DENSE_TILE
     }
 }
 
@@ -825,36 +932,35 @@ int ready_group() {
 }
 
 template <int G>
-int launch_group(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, int partials, hipStream_t st) {
-    for (int i = 0; i < L.n_mats; i++) L.m[i].row_blocks = (L.m[i].out + s.rows - 1) / s.rows;
+int launch_group(const Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, int partials, hipStream_t st) {
     if (s.tokens == 64) return launch_tile<G, 4, 8>(L, xh, ss, ws, s.slices, partials, s.row_blocks, st);
     if (s.tokens == 32) return launch_tile<G, 2, 4>(L, xh, ss, ws, s.slices, partials, s.row_blocks, st);
     return launch_tile<G, 1, 4>(L, xh, ss, ws, s.slices, partials, s.row_blocks, st);
 }
 
+template <int NT>
+int launch_dense(const Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, int partials, hipStream_t st) {
+    static LdsLimit limit; // per instantiation
+    const size_t lds = DenseLds<NT>::kSize;
+    L2_TRY(limit.ensure(reinterpret_cast<const void *>(dense_gemm_kernel<NT>), lds));
+    const int t_tiles = (L.batch + 16 * NT - 1) / (16 * NT);
+    hipLaunchKernelGGL(dense_gemm_kernel<NT>, dim3(s.row_blocks * t_tiles * s.slices), dim3(64 * kDenseWaves), lds, st, L, xh, gemm_padded(L.in), ss, ws, s.slices, t_tiles, partials);
+    L2_HIP(hipGetLastError());
+    return L2_OK;
+}
+
 int launch_fp32(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, int partials, hipStream_t st) {
+    for (int i = 0; i < L.n_mats; i++) L.m[i].row_blocks = (L.m[i].out + s.rows - 1) / s.rows;
     switch (L.group_size) {
+        case 0:
+            if (s.tokens == 128) return launch_dense<8>(L, xh, ss, ws, s, partials, st);
+            if (s.tokens == 64) return launch_dense<4>(L, xh, ss, ws, s, partials, st);
+            return launch_dense<2>(L, xh, ss, ws, s, partials, st);
         case 32: return launch_group<32>(L, xh, ss, ws, s, partials, st);
         case 64: return launch_group<64>(L, xh, ss, ws, s, partials, st);
         case 128: return launch_group<128>(L, xh, ss, ws, s, partials, st);
     }
     return l2_fail(L2_ERR_ARG, "q4 gemm: group size %d", L.group_size);
-}
-
-int launch_dense(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, int partials, hipStream_t st) {
-    for (int i = 0; i < L.n_mats; i++) L.m[i].row_blocks = (L.m[i].out + s.rows - 1) / s.rows;
-    const int t_tiles = (L.batch + s.tokens - 1) / s.tokens, in_p = gemm_padded(L.in);
-    const dim3 grid(s.row_blocks * t_tiles * s.slices), block(256);
-    auto launch = [&](void (*kernel)(Q4Launch, XhList, int, const float *, float *, int, int, int)) {
-        hipLaunchKernelGGL(kernel, grid, block, 0, st, L, xh, in_p, ss, ws, s.slices, t_tiles, partials);
-    };
-    // products summed from zero: 32; 16 and 8 where the matvec's chains are so short that it would be nearer to the exact sum
-    // (1024 inputs: 16s 1.01e-7 in eight slices and 1.09e-7 in one against its 1.00e-7)
-    if (L.in >= 2560) launch(s.tokens == 64 ? dense_gemm_kernel<2, 1> : dense_gemm_kernel<1, 1>);
-    else if (L.in >= 2048) launch(s.tokens == 64 ? dense_gemm_kernel<2, 2> : dense_gemm_kernel<1, 2>);
-    else launch(s.tokens == 64 ? dense_gemm_kernel<2, 4> : dense_gemm_kernel<1, 4>);
-    L2_HIP(hipGetLastError());
-    return L2_OK;
 }
 
 } // namespace
@@ -869,38 +975,46 @@ GemmShape gemm_shape(const Q4Launch &L, int slice_batch, int planes) {
     if (planes == 1) return gemm_shape_f16(L, slice_batch);
     GemmShape s{};
     const int B = L.batch;
-    // inputs per slice, at least: 64 (fp32 weights), 256, and from 4096 inputs on 512 (4096 -> 4096, group 128, 32 columns, 16 slices
+    // inputs per slice, at least: 256, and from 4096 inputs on 512 (4096 -> 4096, group 128, 32 columns, 16 slices
     // 19.4 us, 8 17.0; 1024 inputs, 4 slices or 2, a three-layer prompt of 32: 140 or 153)
-    const int shortest = planes == kDensePlanes ? 64 : L.in >= 4096 && L.group_size > 32 ? 512 : 256;
+    const int shortest = L.in >= 4096 && L.group_size > 32 ? 512 : 256;
     auto slices = [&](int slots, int blocks, int most) { return std::max(1, std::min({slots / blocks, most, gemm_padded(L.in) / shortest})); };
     const int rows32 = row_blocks(L, 128), rows64 = row_blocks(L, 256), cus = cu_count();
-    if (planes == kDensePlanes) {
-        // as many K slices as keep the grid within one round of resident blocks, four per CU up to 32 columns, else three
-        s.slices = slice_batch <= 32 ? slices(4 * cus, rows32, kMaxGemmSlices) : slices(3 * cus, rows32 * ((slice_batch + 63) / 64), 8);
-        s.tokens = B <= 32 ? 32 : 64, s.rows = 128;
-    } else if (slice_batch <= 32) {
+    // The slices of K, of those that take `max_rounds` rounds of one block per CU at most, with the smallest cost: a block costs its
+    // share of K, the first and last microseconds (4.5 % of 4096 inputs) and, with several slices, its partial tile, written and
+    // read again (7.5 %).
+    auto cheapest = [&](int blocks, int most, int max_rounds) {
+        const float per = 4096.0f / L.in;
+        float best = 0.f;
+        int slices = 1;
+        for (int n = 1; n <= std::max(1, most) && (n == 1 || n * blocks <= max_rounds * cus); n++) {
+            const int rounds = (n * blocks + cus - 1) / cus;
+            const float cost = rounds * (1.0f / n + 0.045f * per) + (n > 1 ? 0.075f * per * n * blocks / cus : 0.f);
+            if (n == 1 || cost < best) best = cost, slices = n;
+        }
+        return slices;
+    };
+    if (L.group_size == 0) {
+        // Blocks of 128 columns, so that a weight is read and split once; of 64 where those would leave half the CUs without a
+        // block (four layers of 1024 inputs, 128 columns: 391 -> 350 us; 7B's widths keep 128: 64 columns at three quarters of
+        // the CUs 451 -> 478).  128 inputs per slice at least (1024 inputs, 100 columns 349 us with 256, 338).
+        s.slices = cheapest(rows32 * ((slice_batch + 127) / 128), std::min(kMaxGemmSlices, L.in / 128), 4);
+        s.tokens = B <= 32 ? 32 : B <= 64 || 2 * rows32 * ((B + 127) / 128) * s.slices <= cus ? 64 : 128;
+        s.rows = 128, s.row_blocks = rows32;
+        return s;
+    }
+    if (slice_batch <= 32) {
         // two blocks of 128 rows per CU (13824 -> 5120, 16 columns, 12 slices: 26 us; with three or four per CU 28)
         s.slices = slices(2 * cus, rows32, kMaxGemmSlices);
     } else {
-        // One block of 256 rows x 64 columns per CU.  A block costs its share of K, the first and last microseconds (4.5 % of
-        // 4096 inputs) and, with several slices, its partial tile, written and read again (7.5 %): the slices, of those that
-        // take two rounds of blocks at most (what the operator's fixed workspace holds), for which that sum is the smallest.
-        const int blocks = rows64 * ((slice_batch + 63) / 64), most = std::min(slice_batch <= 64 ? kMaxGemmSlices : 8, L.in / shortest);
-        const float per = 4096.0f / L.in;
-        float best = 0.f;
-        for (int n = 1; n <= std::max(1, most) && (n == 1 || n * blocks <= 2 * cus); n++) {
-            const int rounds = (n * blocks + cus - 1) / cus;
-            const float cost = rounds * (1.0f / n + 0.045f * per) + (n > 1 ? 0.075f * per * n * blocks / cus : 0.f);
-            if (n == 1 || cost < best) best = cost, s.slices = n;
-        }
+        // one block of 256 rows x 64 columns per CU; two rounds of blocks is what the operator's fixed workspace holds
+        s.slices = cheapest(rows64 * ((slice_batch + 63) / 64), std::min(slice_batch <= 64 ? kMaxGemmSlices : 8, L.in / shortest), 2);
     }
-    if (planes != kDensePlanes) {
-        // tiles of 32 columns and 128 rows too where wider blocks would leave half the CUs without one (six layers of 1024
-        // inputs, group 64, 64 columns: 404 -> 380 us)
-        const bool few = 2 * rows64 * ((B + 63) / 64) * s.slices <= cus;
-        s.tokens = B <= 16 ? 16 : B <= 32 || few ? 32 : 64;
-        s.rows = s.tokens == 64 ? 256 : 128;
-    }
+    // tiles of 32 columns and 128 rows too where wider blocks would leave half the CUs without one (six layers of 1024
+    // inputs, group 64, 64 columns: 404 -> 380 us)
+    const bool few = 2 * rows64 * ((B + 63) / 64) * s.slices <= cus;
+    s.tokens = B <= 16 ? 16 : B <= 32 || few ? 32 : 64;
+    s.rows = s.tokens == 64 ? 256 : 128;
     s.row_blocks = s.rows == 128 ? rows32 : rows64;
     return s;
 }
@@ -908,11 +1022,11 @@ GemmShape gemm_shape(const Q4Launch &L, int slice_batch, int planes) {
 int gemm_launch(Q4Launch &L, const XhList &xh, const float *ss, float *ws, size_t ws_floats, int planes, int slice_batch,
                 hipStream_t st, int *ks_out) {
     if (L.n_mats < 1 || L.n_mats > 3 || L.pair) return l2_fail(L2_ERR_ARG, "q4 gemm: n_mats=%d pair=%d", L.n_mats, L.pair);
-    if (L.in % 32 || (planes != kDensePlanes && L.in % L.group_size) || L.batch < 1) return l2_fail(L2_ERR_ARG, "q4 gemm: in=%d batch=%d", L.in, L.batch);
+    if (L.in % 32 || (L.group_size && L.in % L.group_size) || L.batch < 1) return l2_fail(L2_ERR_ARG, "q4 gemm: in=%d batch=%d", L.in, L.batch);
     if (L.e.kind == Q4_EPI_SCATTER_ONLY || L.e.n_scatter) return l2_fail(L2_ERR_ARG, "q4 gemm: no scatter epilogue");
     long rows = 0;
     for (int i = 0; i < L.n_mats; i++) {
-        if (L.m[i].out < 8 || L.m[i].out % 8 || (size_t)L.m[i].out * (planes == kDensePlanes ? L.in : L.in / 8) * 4 >= ((size_t)1 << 32))
+        if (L.m[i].out < 8 || L.m[i].out % 8 || (size_t)L.m[i].out * (L.group_size ? L.in / 8 : L.in) * 4 >= ((size_t)1 << 32))
             return l2_fail(L2_ERR_ARG, "q4 gemm: out=%d in=%d", L.m[i].out, L.in);
         rows += L.m[i].out;
     }
@@ -922,8 +1036,6 @@ int gemm_launch(Q4Launch &L, const XhList &xh, const float *ss, float *ws, size_
         return l2_fail(L2_ERR_ARG, "q4 gemm: %d slices of %d x %ld in a workspace of %zu", s.slices, L.batch, rows, ws_floats);
     if (planes == 1)
         L2_TRY(gemm_launch_f16(L, xh, ss, ws, s, partials, st));
-    else if (planes == kDensePlanes)
-        L2_TRY(launch_dense(L, xh, ss, ws, s, partials, st));
     else
         L2_TRY(launch_fp32(L, xh, ss, ws, s, partials, st));
     if (ks_out) {
@@ -982,7 +1094,7 @@ int gemm_residual_norm_launch(const ResNormPrep &A, int planes, hipStream_t st) 
     if (A.KS < 1 || A.KS > kMaxGemmSlices || A.out % 32 || A.out > kGemmMaxDim || A.n < 1 || A.n > 3)
         return l2_fail(L2_ERR_ARG, "residual epilogue: %d slices, %d outputs, %d consumers", A.KS, A.out, A.n);
     static_assert(kGemmMaxDim <= kTrips * 4096, "a thread keeps its part of the row in registers");
-    return planes == 1 ? residual_norm<1>(A, st) : planes == kDensePlanes ? residual_norm<kDensePlanes>(A, st) : residual_norm<3>(A, st);
+    return planes == 1 ? residual_norm<1>(A, st) : residual_norm<3>(A, st);
 }
 
 int gemm_rope_kv_launch(const RopeKvArgs &A, hipStream_t st) {
@@ -1013,5 +1125,5 @@ static int silu(const SiluArgs &A, hipStream_t st) {
 int gemm_silu_launch(const SiluArgs &A, int planes, hipStream_t st) {
     if (A.KS < 1 || A.KS > kMaxGemmSlices || A.n % 32 || A.n > kGemmMaxHidden)
         return l2_fail(L2_ERR_ARG, "silu gate: %d slices, n=%d", A.KS, A.n);
-    return planes == 1 ? silu<1>(A, st) : planes == kDensePlanes ? silu<kDensePlanes>(A, st) : silu<3>(A, st);
+    return planes == 1 ? silu<1>(A, st) : silu<3>(A, st);
 }

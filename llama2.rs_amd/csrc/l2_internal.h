@@ -181,9 +181,8 @@ bool q4_gathers_in_kernel(const Q4Launch &L);
 
 // ---- batches through the matrix cores (kernels_gemm.hip) -----------------------
 // `planes` is 1 (activations rounded to fp16) or 3 (fp32 activations as three exact bf16 planes).  The activations of
-// a GEMM are [B][planes][gemm_padded(in)] 16-bit values in the layer's g_index order, zero beyond `in`.  The model
-// without quantisation has fp32 activations as they are, [B][gemm_padded(in)] floats: as much room as two planes.
-constexpr int kDensePlanes = 2;
+// a GEMM are [B][planes][gemm_padded(in)] 16-bit values in the layer's g_index order, zero beyond `in`.  A launch with
+// group_size 0 has fp32 weights (the model without quantisation, always 3 planes).
 constexpr int kMaxGemmSlices = 16;
 constexpr int kGemmMaxDim = 16384, kGemmMaxHidden = 38912; // a row of floats in LDS
 __host__ __device__ inline int gemm_padded(int in) { return (in + 63) / 64 * 64; }

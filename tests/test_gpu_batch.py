@@ -109,6 +109,31 @@ def test_dense_batch_error(ops, dim, hidden):
     m.close()
 
 
+# tiles of tokens from one to eight and one more block, rows that do not fill a block; then infinities and NaN, which the
+# planes of a split number do not carry: a batch has them where its columns one by one have them.  Sums of K terms of either
+# association differ by K 2^-24 of the sum of magnitudes at most, which is below sqrt(K) 2 rms for these inputs
+@pytest.mark.parametrize("hidden", [2816, 1344])
+def test_dense_batch_tiles(ops, hidden):
+    from llama2_rs import _lib
+    import tests.test_oracle_loop as tol
+    dims = ck.Dims(dim=1024, hidden_dim=hidden, n_layers=1, n_heads=8, n_kv_heads=1, vocab_size=64, seq_len=32, group_size=0)
+    img = ops.synth_image(dims, 6)
+    m, rng = ops.Model(img, dims), np.random.default_rng(hidden)
+    for name, proj in (("w1", _lib.W1), ("w2", _lib.W2)):
+        W = tol._split_image(img, dims)[name][0].astype(np.float64)
+        for B in (16, 17, 33, 48, 64, 65, 81, 97, 112, 113, 128, 129, 177):
+            x = rng.standard_normal((B, W.shape[1])).astype(np.float32)
+            assert nrel(m.qmatvec(0, proj, x), x.astype(np.float64) @ W.T) < 1e-5, (name, B)
+        x = rng.standard_normal((100, W.shape[1])).astype(np.float32)
+        x[3, 5], x[40, 100], x[99, 7], x[99, 9], x[70, -1], x[50] = np.inf, -np.inf, np.inf, -np.inf, np.nan, 3e38
+        got, one = m.qmatvec(0, proj, x), np.stack([m.qmatvec(0, proj, v) for v in x])
+        for b in (3, 40, 70, 99):
+            np.testing.assert_array_equal(got[b], one[b])
+        fine = [b for b in range(100) if b not in (3, 40, 50, 70, 99)]
+        assert nrel(got[fine], x[fine].astype(np.float64) @ W.T) < 1e-5
+    m.close()
+
+
 # the same for quantised weights: several K slices and one, of one run of groups and of several (4128 and 4160 inputs, 512
 # columns: three and two; 8320: two), an odd number of K steps and half of one.  The rounding of the matrix unit must not
 # lean to one side either: the mean error of 512 columns' 4e6 values is below a thirtieth of their rms
