@@ -17,6 +17,7 @@
 #include <string.h>
 
 #include "l2_internal.h"
+#include "lanes.h"
 
 namespace {
 
@@ -40,22 +41,6 @@ __device__ __forceinline__ void pin_args(const AttnDecode &A) {
                  "s"(A.ts), "s"(A.n_splits), "s"(A.max_splits));
 }
 
-// A lane's value and that of the lane 32 (16) away, in the same order for both lanes: one instruction that swaps
-// halves (rows) of two registers, in the vector ALU, where a shuffle goes through the LDS pipe.
-struct Both {
-    float lo, hi;
-};
-__device__ __forceinline__ Both both32(float v) {
-    const uint32_t b = __builtin_bit_cast(uint32_t, v);
-    const auto r = __builtin_amdgcn_permlane32_swap(b, b, false, false);
-    return {__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1])};
-}
-__device__ __forceinline__ Both both16(float v) {
-    const uint32_t b = __builtin_bit_cast(uint32_t, v);
-    const auto r = __builtin_amdgcn_permlane16_swap(b, b, false, false);
-    return {__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1])};
-}
-
 constexpr float kNoScore = -1e30f; // "no timestep yet": finite, so that differences never give NaN
 
 __device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
@@ -65,9 +50,7 @@ __device__ __forceinline__ float wave_sum(float v) {
     v += dpp_xchg<0x4E>(v);
     v += dpp_xchg<0x141>(v);
     v += dpp_xchg<0x140>(v);
-    v += __shfl_xor(v, 16);
-    v += __shfl_xor(v, 32);
-    return v;
+    return lanes::rows_sum(v);
 }
 
 __device__ __forceinline__ float wave_max(float v) {
@@ -75,9 +58,7 @@ __device__ __forceinline__ float wave_max(float v) {
     v = fmaxf(v, dpp_xchg<0x4E>(v));
     v = fmaxf(v, dpp_xchg<0x141>(v));
     v = fmaxf(v, dpp_xchg<0x140>(v));
-    v = fmaxf(v, __shfl_xor(v, 16));
-    v = fmaxf(v, __shfl_xor(v, 32));
-    return v;
+    return lanes::rows_max(v);
 }
 
 // Floats per row of the LDS tiles in which rows of lanes, waves and splits meet: the 128 partial outputs, then
@@ -329,20 +310,20 @@ __global__ __launch_bounds__(NWV * 64) void attn_decode_kernel(const AttnDecode 
         auto merge = [&](auto both) __attribute__((always_inline)) {
 #pragma unroll
             for (int j = 0; j < QG; j++) {
-                const Both mb = both(m[j]), lb = both(l[j]);
+                const lanes::Both mb = both(m[j]), lb = both(l[j]);
                 const float M = fmaxf(mb.lo, mb.hi);
                 const float w1 = exp2_fast(mb.lo - M), w2 = exp2_fast(mb.hi - M);
                 l[j] = lb.lo * w1 + lb.hi * w2;
 #pragma unroll
                 for (int e = 0; e < VE; e++) {
-                    const Both a = both(acc[j][e]);
+                    const lanes::Both a = both(acc[j][e]);
                     acc[j][e] = a.lo * w1 + a.hi * w2;
                 }
                 m[j] = M;
             }
         };
-        merge([](float v) { return both16(v); });
-        merge([](float v) { return both32(v); });
+        merge([](float v) { return lanes::both16(v); });
+        merge([](float v) { return lanes::both32(v); });
     }
     if (kRowsInLds || lane < 16) {
         const int slot = kRowsInLds ? wave * 4 + (lane >> 4) : wave;
@@ -590,8 +571,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_mfma_kernel(const AttnDeco
             mx = fmaxf(mx, sc[r]);
         }
         if (__any(mx > m_run)) { // some head's maximum moves: agree on it among the head's four lanes, rescale
-            mx = fmaxf(mx, __shfl_xor(mx, 16));
-            mx = fmaxf(mx, __shfl_xor(mx, 32));
+            mx = lanes::rows_max(mx);
             const float m_new = fmaxf(m_run, mx);
             const float c = exp2_fast(m_run - m_new);
             l *= c;
@@ -633,8 +613,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_mfma_kernel(const AttnDeco
 
     // this wave's (m, l, O) -> LDS.  The head's four lanes hold disjoint d: lane (j, kb), accumulators 0..3,
     // register r are d = 16 kb + 4 r + 0..3, accumulators 4..7 the same 64 further on.
-    l += __shfl_xor(l, 16);
-    l += __shfl_xor(l, 32);
+    l = lanes::rows_sum(l);
     if (li < QG) {
 #pragma unroll
         for (int r = 0; r < 4; r++) {
@@ -988,8 +967,7 @@ void attn_prefill_mfma16_kernel(void *__restrict__ out, const float *__restrict_
                 mx = fmaxf(mx, sc[r]);
             }
             if (__any(mx > R.m)) { // some column's maximum moves: agree on it among the column's four lanes, rescale
-                mx = fmaxf(mx, __shfl_xor(mx, 16));
-                mx = fmaxf(mx, __shfl_xor(mx, 32));
+                mx = lanes::rows_max(mx);
                 const float m_new = fmaxf(R.m, mx);
                 const float c = exp2_fast(R.m - m_new);
                 R.l *= c;
@@ -1032,8 +1010,7 @@ void attn_prefill_mfma16_kernel(void *__restrict__ out, const float *__restrict_
         if (cs > 0) __syncthreads(); // the set before has been read
         // this wave's (m, l, O) -> LDS: lane (column j, kb), accumulators 0..3, register r are d = 16 kb + 4 r + 0..3,
         // accumulators 4..7 the same 64 further on
-        l += __shfl_xor(l, 16);
-        l += __shfl_xor(l, 32);
+        l = lanes::rows_sum(l);
 #pragma unroll
         for (int r = 0; r < 4; r++) {
             *reinterpret_cast<float4 *>(&comb[wave][li][16 * kb + 4 * r]) = make_float4(acc[0][r], acc[1][r], acc[2][r], acc[3][r]);

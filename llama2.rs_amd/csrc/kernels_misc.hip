@@ -11,6 +11,7 @@
 // which is that layer's x[g_index[j]] gather (src/gptq.rs:110-114) done once
 // at the source instead of once per consumer block.
 #include "l2_internal.h"
+#include "lanes.h"
 
 namespace {
 
@@ -25,9 +26,7 @@ __device__ __forceinline__ float wave_sum(float v) {
     v += dpp_xchg<0x4E>(v);
     v += dpp_xchg<0x141>(v);
     v += dpp_xchg<0x140>(v);
-    v += __shfl_xor(v, 16);
-    v += __shfl_xor(v, 32);
-    return v;
+    return lanes::rows_sum(v);
 }
 
 __device__ __forceinline__ float wave_max(float v) {
@@ -35,9 +34,7 @@ __device__ __forceinline__ float wave_max(float v) {
     v = fmaxf(v, dpp_xchg<0x4E>(v));
     v = fmaxf(v, dpp_xchg<0x141>(v));
     v = fmaxf(v, dpp_xchg<0x140>(v));
-    v = fmaxf(v, __shfl_xor(v, 16));
-    v = fmaxf(v, __shfl_xor(v, 32));
-    return v;
+    return lanes::rows_max(v);
 }
 
 // Block-wide sum / max for blocks of up to 1024 threads; `red` holds 16 floats.

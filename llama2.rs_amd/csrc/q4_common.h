@@ -2,6 +2,7 @@
 #pragma once
 
 #include "l2_internal.h"
+#include "lanes.h"
 
 namespace q4 {
 
@@ -19,9 +20,7 @@ __device__ __forceinline__ float wave_sum(float v) {
     v += dpp_xchg<0x4E>(v);  // quad_perm [2,3,0,1]
     v += dpp_xchg<0x141>(v); // row_half_mirror
     v += dpp_xchg<0x140>(v); // row_mirror
-    v += __shfl_xor(v, 16);
-    v += __shfl_xor(v, 32);
-    return v;
+    return lanes::rows_sum(v);
 }
 
 typedef float v2f __attribute__((ext_vector_type(2)));
