@@ -230,19 +230,19 @@ def test_decode_attention_long_context(ops, oracle, n_heads, n_kv, ctx):
 def test_decode_attention_tile_edges(ops, oracle, n_heads, n_kv):
     """Decode steps at the edges of the attention's steps, tiles, block shapes and splits, first position included."""
     dims = ck.Dims(dim=128 * n_heads, hidden_dim=512, n_layers=1, n_heads=n_heads, n_kv_heads=n_kv,
-                   vocab_size=300, seq_len=600, group_size=128)
+                   vocab_size=300, seq_len=2100, group_size=128)
     img = ck.synth_weights_image(dims, seed=8)
     m = ops.Model(img, dims)
     o = oracle.Model(img, dims)
     o.new_state()
-    m.fill_kv_synthetic(0, 590, seed=4)
+    m.fill_kv_synthetic(0, 2090, seed=4)
     ko, vo = o.kv_cache()
-    ko[0, :590], vo[0, :590] = m.read_kv(0, 0, 590)
-    for pos in (0, 1, 15, 16, 17, 63, 64, 65, 127, 128, 129, 255, 256, 257, 511, 512, 513, 577):
+    ko[0, :2090], vo[0, :2090] = m.read_kv(0, 0, 2090)
+    for pos in (0, 1, 15, 16, 17, 63, 64, 65, 127, 128, 129, 255, 256, 257, 511, 512, 513, 577, 1023, 1024, 2047, 2048):
         want = o.transformer([11], [pos])
         assert nrel(m.forward([11], [pos]), want) < REL_FP32, pos
-    k, v = m.read_kv(0, 0, 590)
-    assert nrel(k, ko[0, :590]) < REL_FP32 and nrel(v, vo[0, :590]) < REL_FP32
+    k, v = m.read_kv(0, 0, 2090)
+    assert nrel(k, ko[0, :2090]) < REL_FP32 and nrel(v, vo[0, :2090]) < REL_FP32
     m.close()
     o.close()
 
