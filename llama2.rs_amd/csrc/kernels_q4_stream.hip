@@ -675,20 +675,6 @@ static int plan_rows(const Q4Launch &L, int NW, int TR, size_t lds, bool pair, i
     return rpb;
 }
 
-// Wave-rows of arithmetic per CU for a candidate shape: what the choice between shapes minimises.
-static long plan_cost(const Q4Launch &L, int NWK, int S, int P, bool pair) {
-    const size_t lds = (size_t)NWK * 64 * (kChunkPad + 1) * sizeof(float) * (pair ? 2 : 1);
-    const int NW = NWK * S, TR = P * S;
-    int per_cu = 16 / NW;
-    if (pair) per_cu = 1; // w1|w3: one block per CU measured faster than two (7B: 13.1 -> 12.4 us, 722 -> 733 tok/s)
-    if (per_cu < 1) per_cu = 1;
-    const int by_lds = (int)((150 * 1024) / (lds + 4 * 1024));
-    if (per_cu > by_lds) per_cu = by_lds < 1 ? 1 : by_lds;
-    const int rpb = plan_rows(L, NW, TR, lds, pair, nullptr);
-    const long tiles = (rpb + TR - 1) / TR;
-    return (long)per_cu * NW * tiles * P;
-}
-
 template <int G, int NWK, int S, bool PAIR, int MODE, int P = (PAIR ? 2 : 4), bool GATHER = false>
 int launch_s(Q4Launch &L, hipStream_t stream) {
     constexpr int NW = NWK * S;
@@ -723,20 +709,21 @@ int launch_s(Q4Launch &L, hipStream_t stream) {
     return L2_OK;
 }
 
-// Rows in flight per stream (P) were measured per shape on whole decode steps.  Where the rows of a block are
-// few (4096 and 11008 inputs: 4 to 8 rows per stream), fewer loads primed in front of x let x arrive sooner,
-// and every instruction of the kernel waits for x: two rows at 4096 inputs (7B +1.2 %), three at 11008 (+0.9 %)
-// and at 13824 through the per-wave form (13B +0.7 %); priming all rows of the block is 15-20 % slower.
+// Rows in flight per stream (P) and streams per block (S) were measured per shape on whole decode steps.  Where the rows of a
+// block are few (4096 and 11008 inputs: 4 to 8 rows per stream), fewer loads primed in front of x let x arrive sooner,
+// and every instruction of the kernel waits for x: two rows at 4096 inputs (7B +1.2 %), three at 11008 (+0.9 %); priming all
+// rows of the block is 15-20 % slower.  Blocks have a whole number of waves per SIMD: with 12 waves instead of 15 at 5120 inputs
+// 13B's w1|w3 takes 17.3 us instead of 22.5 (9 waves 23.6, 6 waves 23.3) and wo 6.4 instead of 7.0.  16 waves with one pair of rows
+// in flight against 8 with two at 8192 inputs: 70B's w1|w3 43.9 -> 42.6 (12 waves with one or two pairs 46.8, 44.1).
+// 28672 -> 8192, two, three, four, five, six rows: 27.6 / 24.8 / 25.7 / 26.2 / 26.7 us; 13824 -> 5120, two rows or three: 11.0, 11.1.
 template <int G, int MODE>
 int launch_sg(Q4Launch &L, hipStream_t stream) {
     const int nwk = (L.in / 32 + 63) / 64;
     if constexpr (MODE == 2) { // only the shapes q4_stream_launch sends here
         if (!L.pair) switch (nwk) {
-            case 3:
-                if (plan_cost(L, 3, 5, 4, false) < plan_cost(L, 3, 4, 4, false)) return launch_s<G, 3, 5, false, MODE>(L, stream);
-                return launch_s<G, 3, 4, false, MODE>(L, stream);
-            case 7: return launch_s<G, 7, 2, false, MODE, 3>(L, stream);
-            case 9: case 10: case 11: case 12: case 13: case 14: return launch_s<G, 14, 1, false, MODE>(L, stream);
+            case 3: return launch_s<G, 3, 4, false, MODE>(L, stream);
+            case 7: return launch_s<G, 7, 2, false, MODE, 2>(L, stream);
+            case 9: case 10: case 11: case 12: case 13: case 14: return launch_s<G, 14, 1, false, MODE, 3>(L, stream);
         }
     } else if (MODE == 0 && !L.pair && L.n_mats == 1 && L.m[0].gidx) {
         if constexpr (MODE == 0) switch (nwk) { // the gathering form, where one staging batch covers the vector
@@ -749,9 +736,7 @@ int launch_sg(Q4Launch &L, hipStream_t stream) {
         switch (nwk) {
             case 1: return launch_s<G, 1, 4, false, MODE>(L, stream);
             case 2: return launch_s<G, 2, 4, false, MODE, 2>(L, stream);
-            case 3: // 5120: 20 rows per block are one tile of 5 streams, 60 or so are four tiles either way
-                if (plan_cost(L, 3, 5, 4, false) < plan_cost(L, 3, 4, 4, false)) return launch_s<G, 3, 5, false, MODE>(L, stream);
-                return launch_s<G, 3, 4, false, MODE>(L, stream);
+            case 3: return launch_s<G, 3, 4, false, MODE>(L, stream);
             case 4: return launch_s<G, 4, 4, false, MODE, 2>(L, stream); // 8192: rows of 4 KB; two in flight per stream measured faster than four (q|k|v 13.4 -> 12.2 us, wo 12.1 -> 10.9)
             case 5: case 6: return launch_s<G, 6, 2, false, MODE, 3>(L, stream);
             case 7: return launch_s<G, 7, 2, false, MODE, 5>(L, stream); // 13824 -> 5120: 20 rows per block in two tiles
@@ -762,8 +747,8 @@ int launch_sg(Q4Launch &L, hipStream_t stream) {
         switch (nwk) {
             case 1: return launch_s<G, 1, 4, true, MODE>(L, stream);
             case 2: return launch_s<G, 2, 4, true, MODE>(L, stream);
-            case 3: return launch_s<G, 3, 5, true, MODE>(L, stream);
-            case 4: return launch_s<G, 4, 2, true, MODE>(L, stream);
+            case 3: return launch_s<G, 3, 4, true, MODE>(L, stream);
+            case 4: return launch_s<G, 4, 4, true, MODE, 1>(L, stream);
         }
     }
     return l2_fail(L2_ERR_ARG, "q4 matvec (streaming): in=%d pair=%d has no kernel", L.in, L.pair);
