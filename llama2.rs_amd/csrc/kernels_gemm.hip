@@ -453,13 +453,15 @@ __global__ __launch_bounds__(64 * NW, NT == 1 ? 3 : 2) void q4_tile_gemm_kernel(
 
 // Linear::matvec<B> of the model without quantisation (src/model.rs:22-31) for a batch: fp32 weights, fp32 activations,
 // on the bf16 matrix cores.  The activations are three bf16 planes as above; the weights become three on the way in, each
-// rounded to nearest, so that what a plane leaves over has either sign.  Of the nine products of a weight and an activation
-// the six down to 2^-16 of the first are taken; the other three are below 2^-24, of either sign and average out.  That is
-// 6 products at 2.5 PFLOP/s against one at the 157 TFLOP/s of v_mfma_f32_32x32x2_f32.
+// rounded to nearest, so that what a plane leaves over has either sign.  All nine products of a weight and an activation are
+// taken, so a product is exact as long as both planes are: numbers below 2^-109 have bits below bf16's smallest, 2^-133, and
+// enter as multiples of that.  That is 9 products at 2.5 PFLOP/s against one at the 157 TFLOP/s of v_mfma_f32_32x32x2_f32.
 //
-// Sums: the six products of 32 inputs from zero, the smallest first, so that one addition of the matrix unit sees the whole
-// of them; every other 32 inputs enter negated, as above; 32 inputs to each other in runs and the runs to each other in fp32 as the vector ALU rounds
-// it, the slices of K in a tree.  Runs of sqrt(steps / 2) and more make the two chains about equally long.
+// Sums: the product of the first planes, 16 bits, is all but 2^-7 of a weight times its activation.  These products of 32 inputs
+// are summed from zero (one term alone: exactly) and the vector ALU adds them up, rounded to nearest; every other 32 inputs enter
+// negated, as above; in runs and the runs to each other, the slices of K in a tree.  Runs of sqrt(steps / 2) and more
+// make the two chains about equally long.  The other eight products go through the matrix unit from end to end: its rounding
+// is of sums that are 2^-7 of the output's.
 //
 // Infinities and NaN: the planes of an infinity are not one (inf - inf), so a sum that comes out as neither number is done
 // again in fp32 from what the planes stand for (dense_again).
@@ -467,19 +469,27 @@ __global__ __launch_bounds__(64 * NW, NT == 1 ? 3 : 2) void q4_tile_gemm_kernel(
 // A wave owns 16 rows x 16 NT tokens, a block 8 waves over the rows: a weight is read and split once for up to 128 tokens.
 // Lane (row r = l % 16, kg = l / 16) loads 8 consecutive weights of each 32 inputs (a row's cache line, in two loads), four
 // such pairs ahead, and splits 32 inputs ahead of the products; the activations of 64 inputs pass through LDS,
-// double-buffered.  What bounds it is issue: a step of 64 inputs and 112 tokens is 437 instructions per wave, 84 of them
-// products (1344 cycles), 88 the splitting, and two waves per SIMD take some 5500 cycles for it.
+// double-buffered; the sums of the runs wait in LDS, which takes up all of it (NT = 8).  What bounds it is the products
+// and what issues beside them, one behind the other: a step of 64 inputs and 112 tokens is 480 instructions per wave, 126 of
+// them products (2016 cycles), 96 the splitting, and two waves per SIMD take some 7000 cycles for it.
 //
 // Against products in v_mfma_f32_32x32x2_f32 (128 rows x 64 columns per block, every weight read for each): one layer of 7B's
-// widths, 33, 64, 100, 200, 512 columns 327 / 331 / 531 / 1039 / 1846 -> 272 / 305 / 413 / 751 / 1320 us; w1|w3 alone at 99 columns
-// 234 -> 165; 32 rows x 64 tokens per wave: 190.  Relative rms error against fp64, normal inputs, 33 to 300 columns of 1024 / 4096 /
-// 11008 inputs: 9.1e-8 / 1.3e-7 / 1.4e-7 -> 7.4e-8 / 0.94e-7 / 1.0e-7 (the matvec 1.0e-7 / 1.6e-7 / 2.4e-7); without the
-// negation 8.2e-8 / 1.2e-7 / 1.5e-7.
+// widths, 33, 64, 100, 200, 512 columns 332 / 347 / 557 / 1021 / 1818 -> 301 / 341 / 496 / 954 / 1652 us; w1|w3 alone at 99 columns
+// 234 -> 214.  Without the three smallest products, and all six in one chain: 285 / 305 / 416 / 773 / 1330 us; but a sum of one term
+// then errs by 3.9e-8 rms, 2.3e-7 at most, where fp32 errs by 2.5e-8 and 6.0e-8.
+//
+// Relative rms error against fp64, that product -> this one (the matvec), 100 columns of 1024 and of 4096 inputs: normal 9.1e-8 -> 6.9e-8
+// (9.9e-8), 12.7e-8 -> 8.1e-8 (16.0e-8); one term 2.5e-8 in all; four terms 4.6e-8 -> 4.3e-8 (4.7e-8), 4.7e-8 -> 4.4e-8 (4.6e-8);
+// one input 1e6 times the others 10.1e-8 -> 9.1e-8 (9.5e-8), 16.1e-8 -> 10.4e-8 (15.5e-8); all of one sign 3.4e-8 -> 3.8e-8 (3.4e-8),
+// 3.5e-8 -> 3.4e-8 (3.6e-8).  11008 inputs, normal: 14e-8 -> 9.3e-8 (24e-8).
 constexpr int kDenseWaves = 8, kDenseRows = 16 * kDenseWaves;
 template <int NT>
 struct DenseLds {
-    static constexpr int kPlane = 16 * NT * kStepRow, kTile = 3 * kPlane, kSize = 2 * kTile;
+    static constexpr int kPlane = 16 * NT * kStepRow, kTile = 3 * kPlane;
+    static constexpr int kTop = NT * 64 * (int)sizeof(f4v); // of a wave
+    static constexpr int kSize = 2 * kTile + kDenseWaves * kTop;
 };
+static_assert(DenseLds<8>::kSize <= 160 * 1024, "LDS of a compute unit");
 
 // One output over the inputs k0..k1-1 in plain fp32.
 __device__ __forceinline__ float dense_again(const float *w, const uint16_t *x, int in_p, int k0, int k1) {
@@ -549,22 +559,25 @@ __device__ __forceinline__ void dense_tile(const Q4Launch &L, const XhList &xl, 
         for (int i = 0; i < 2; i++) d.v[i] = ld_at<float4>(w, c + 16u * i);
     };
     Raw raw[4];
-    Frag a[2][NP]; // [half][plane]
+    Frag a[2][NP], minus; // [half][plane]; the first plane of half 1, negated
     auto split = [&](const int from, const int half, const int i) __attribute__((always_inline)) { // a pair of weights, of four
         constexpr int order[8] = {0, 2, 4, 6, 1, 3, 5, 7}; // the activations' slots
         float x = (&raw[from].v[order[2 * i] >> 2].x)[order[2 * i] & 3], y = (&raw[from].v[order[2 * i + 1] >> 2].x)[order[2 * i + 1] & 3];
-        if (half == 1) x = -x, y = -y;
 #pragma unroll
         for (int p = 0; p < NP; p++) {
             const uint32_t b = __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{x, y}, b2));
             a[half][p].u[i] = b;
+            if (p == 0 && half == 1) minus.u[i] = b ^ 0x80008000u;
             if (p < NP - 1) x -= __builtin_bit_cast(float, b << 16), y -= __builtin_bit_cast(float, b & 0xFFFF0000u);
         }
     };
 
-    f4v top[NT], run[NT], sum[4]; // sums of the runs, of the current run; of 32 inputs
+    // first x first: the products of 32 inputs, the sums of the current run and of the runs (this one in LDS, for want of
+    // registers); all others
+    f4v sum[4], run[NT], low[NT];
+    f4v *const top = reinterpret_cast<f4v *>(lds + 2 * S::kTile + wave * S::kTop) + lane;
 #pragma unroll
-    for (int n = 0; n < NT; n++) top[n] = run[n] = f4v{0.f, 0.f, 0.f, 0.f};
+    for (int n = 0; n < NT; n++) run[n] = low[n] = top[64 * n] = f4v{0.f, 0.f, 0.f, 0.f};
     // The products of a half step go by pairs of token tiles, whose chains do not wait for each other.
     constexpr int PAIRS = (NT + 1) / 2;
     Frag b[4][NP];
@@ -604,14 +617,15 @@ __device__ __forceinline__ void dense_tile(const Q4Launch &L, const XhList &xl, 
             const int k = g / PAIRS, next = (2 * par + k + 1) & 3; // the half whose weights are split meanwhile
             if (g + 1 < 2 * PAIRS) read_x(g + 1, tile);
             if (g > 0) fold(g - 1);
-            constexpr int pa[6] = {2, 1, 0, 1, 0, 0}, pb[6] = {0, 1, 2, 0, 1, 0};
+            constexpr int pa[8] = {2, 2, 1, 2, 1, 0, 1, 0}, pb[8] = {2, 1, 2, 0, 1, 2, 0, 1};
 #pragma unroll
-            for (int q = 0; q < 6; q++)
+            for (int q = 0; q < 9; q++)
 #pragma unroll
                 for (int u = 0; u < 2; u++) {
-                    const int at = (g & 1) * 2 + u;
-                    if (g % PAIRS * 2 + u < NT)
-                        sum[at] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[k][pa[q]].b, b[at][pb[q]].b, q == 0 ? f4v{} : sum[at], 0, 0, 0);
+                    const int at = (g & 1) * 2 + u, n = g % PAIRS * 2 + u;
+                    if (n >= NT) continue;
+                    if (q == 0) sum[at] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k ? minus.b : a[k][0].b, b[at][0].b, f4v{}, 0, 0, 0);
+                    else low[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[k][pa[q - 1]].b, b[at][pb[q - 1]].b, low[n], 0, 0, 0);
                 }
 #pragma unroll
             for (int i = g % PAIRS * 4 / PAIRS; i < (g % PAIRS + 1) * 4 / PAIRS; i++) split(next, k ^ 1, i);
@@ -619,15 +633,16 @@ __device__ __forceinline__ void dense_tile(const Q4Launch &L, const XhList &xl, 
             if (g % PAIRS == PAIRS - 1) { // after the last use of what was there: a load hoisted above it costs copies that wait for it
 #pragma unroll
                 for (int p = 0; p < NP; p++) asm volatile("" : "+v"(a[k ^ 1][p].b));
+                if (k == 0) asm volatile("" : "+v"(minus.b));
                 fetch_w(2 * it + k + 5, raw[next]);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
         fold(2 * PAIRS - 1);
-        if (it + 1 == end) {
+        if (it + 1 == end && end < it1) { // the last run stays in registers
             end += run_len;
 #pragma unroll
-            for (int n = 0; n < NT; n++) top[n] += run[n], run[n] = f4v{0.f, 0.f, 0.f, 0.f};
+            for (int n = 0; n < NT; n++) top[64 * n] += run[n], run[n] = f4v{0.f, 0.f, 0.f, 0.f};
         }
         __syncthreads();
         tile ^= S::kTile;
@@ -652,7 +667,7 @@ __device__ __forceinline__ void dense_tile(const Q4Launch &L, const XhList &xl, 
     for (; it + 1 < it1; it += 2) step(it, 0), step(it + 1, 1);
     if (it < it1) step(it, 0);
 #pragma unroll
-    for (int n = 0; n < NT; n++) top[n] += run[n];
+    for (int n = 0; n < NT; n++) run[n] = top[64 * n] + (run[n] + low[n]);
 
     // C layout: lane (column r = token, kg), register e -> row 4 kg + e
     size_t ws_base = 0;
@@ -662,7 +677,7 @@ __device__ __forceinline__ void dense_tile(const Q4Launch &L, const XhList &xl, 
     for (int n = 0; n < NT; n++) {
         const int t = t0 + n * 16 + r;
         if (t >= B || o >= n_out) continue;
-        float4 v = make_float4(top[n][0], top[n][1], top[n][2], top[n][3]);
+        float4 v = make_float4(run[n][0], run[n][1], run[n][2], run[n][3]);
         if (!__builtin_isfinite((v.x + v.y) + (v.z + v.w))) {
             const uint16_t *xt = reinterpret_cast<const uint16_t *>(xh) + (size_t)t * NP * in_p;
             const float *wo = reinterpret_cast<const float *>(w) + (size_t)o * in;

@@ -109,6 +109,36 @@ def test_dense_batch_error(ops, dim, hidden):
     m.close()
 
 
+# sums in which one or a few terms are all there is, where nothing averages out.  One term: its product is rounded once,
+# to 2^-24 of it; what is added before that is below 2^-7 of it, and its at most eight additions err by 2^-23 of that each.
+# A few terms, and one far above the others: no further from the exact sums than the columns, as above (N = 2.8e5 values)
+@pytest.mark.parametrize("dim,hidden", [(1024, 2816), (2048, 2816)])
+def test_dense_batch_few_terms(ops, dim, hidden):
+    from llama2_rs import _lib
+    import tests.test_oracle_loop as tol
+    dims = ck.Dims(dim=dim, hidden_dim=hidden, n_layers=1, n_heads=dim // 128, n_kv_heads=1, vocab_size=64, seq_len=32, group_size=0)
+    img = ops.synth_image(dims, 4)
+    m, rng, B = ops.Model(img, dims), np.random.default_rng(dim), 100
+    W = tol._split_image(img, dims)["w1"][0].astype(np.float64)
+    one, few, far = np.zeros((B, dim), np.float32), np.zeros((B, dim), np.float32), rng.standard_normal((B, dim)).astype(np.float32)
+    for b in range(B):
+        one[b, rng.integers(dim)] = rng.standard_normal()
+        few[b, rng.choice(dim, 4, replace=False)] = rng.standard_normal(4)
+    far[:, dim // 2] *= 1e6
+    want = one.astype(np.float64) @ W.T
+    err = np.abs(m.qmatvec(0, _lib.W1, one) - want)
+    assert np.all(err <= (2.0 ** -24 + 8 * 2.0 ** -30) * np.abs(want)), np.max(err / np.maximum(np.abs(want), 1e-30))
+    for x in (few, far):
+        want = x.astype(np.float64) @ W.T
+        assert rms_error(m.qmatvec(0, _lib.W1, x), want) < 1.02 * rms_error(np.stack([m.qmatvec(0, _lib.W1, v) for v in x]), want)
+    # numbers that bf16 planes do not hold whole: cut at 2^-133, beside the K 2^-24 of the magnitudes that any association stays within
+    for e in (-100, -112, -124):
+        x = (rng.standard_normal((B, dim)) * 2.0 ** e).astype(np.float32)
+        err = np.abs(m.qmatvec(0, _lib.W1, x) - x.astype(np.float64) @ W.T)
+        assert np.all(err <= 2.0 ** -133 * np.abs(W).sum(1) + dim * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(W).T) + dim * 2.0 ** -149)
+    m.close()
+
+
 # tiles of tokens from one to eight and one more block, rows that do not fill a block; then infinities and NaN, which the
 # planes of a split number do not carry: a batch has them where its columns one by one have them.  Sums of K terms of either
 # association differ by K 2^-24 of the sum of magnitudes at most, which is below sqrt(K) 2 rms for these inputs
