@@ -44,7 +44,9 @@ enum { L2_WQ = 0, L2_WK = 1, L2_WV = 2, L2_WO = 3, L2_W1 = 4, L2_W2 = 5, L2_W3 =
 enum {
     L2_PREFILL_FP32 = 0, /* fp32 throughout: a few columns are the bits of B=1; larger batches run on the
                           * matrix cores with every product exact and fp32 accumulation, so they differ
-                          * from B=1 by the rounding of the additions only (1e-6)                    */
+                          * from B=1 by the rounding of the additions only (1e-6).  Exact means: operands
+                          * enter as three bf16 numbers, which hold all 24 bits of a value from 2^-109 on
+                          * and smaller ones to 2^-133                                               */
     L2_PREFILL_MFMA = 1, /* dequant -> fp16 tiles -> MFMA, fp32 accumulate (tolerance 2e-3)    */
     L2_PREFILL_COLUMNS = 2 /* fp32 throughout, and every column of a projection is the bits of B=1
                             * whatever the batch, as L2_PREFILL_FP32 has for a few columns: the
