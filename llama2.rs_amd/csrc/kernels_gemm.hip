@@ -464,8 +464,11 @@ __global__ __launch_bounds__(64 * NW, NT == 1 ? 3 : 2) void q4_tile_gemm_kernel(
 // make the two chains about equally long.  The other eight products go through the matrix unit from end to end: its rounding
 // is of sums that are 2^-7 of the output's.
 //
-// Infinities and NaN: the planes of an infinity are not one (inf - inf), so a sum that comes out as neither number is done
-// again in fp32 from what the planes stand for (dense_again).
+// Infinities and NaN: the planes of an infinity are not one (inf - inf), and a plane can be rounded to one.  A tile of 16 x 16 with
+// a sum that is not finite is done again at the end with v_mfma_f32_16x16x4_f32, from the weights and what the planes stand for,
+// unless its token holds a NaN anyway (attention hands one to every token behind it).  7B's w1, 100 columns, 106 us: with a NaN
+// in one column 117, in all 187, with an infinity in one 181, in all 640 (one output at a time in the vector ALU: one column
+// 2150 us, all 34 ms).
 //
 // A wave owns 16 rows x 16 NT tokens, a block 8 waves over the rows: a weight is read and split once for up to 128 tokens.
 // Lane (row r = l % 16, kg = l / 16) loads 8 consecutive weights of each 32 inputs (a row's cache line, in two loads), four
@@ -492,17 +495,40 @@ struct DenseLds {
 };
 static_assert(DenseLds<8>::kSize <= 160 * 1024, "LDS of a compute unit");
 
-// One output over the inputs k0..k1-1 in plain fp32.
-__device__ __forceinline__ float dense_again(const float *w, const uint16_t *x, int in_p, int k0, int k1) {
-    float s = 0.f;
-#pragma unroll 1
-    for (int k = k0; k < k1; k++) {
-        const uint16_t *q = x + b16_slot(k);
-        auto plane = [&](int p) { return __builtin_bit_cast(float, (uint32_t)q[(size_t)p * in_p] << 16); };
-        const float hi = plane(0);
-        s = fmaf(w[k], __builtin_isfinite(hi) ? hi + (plane(1) + plane(2)) : hi, s);
+// A tile of 16 x 16 outputs over the inputs k0..k1-1 (whole 32) in fp32 products.  w, x: the lane's row and token, from its 8
+// inputs of the first 32 on.  Every lane of the wave takes part.
+__device__ __forceinline__ f4v dense_again(const float *w, const uint16_t *x, int in_p, int k0, int k1) {
+    f4v sum{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int k = k0; k < k1; k += 32) {
+        const float4 wv[2] = {*reinterpret_cast<const float4 *>(w + k), *reinterpret_cast<const float4 *>(w + k + 4)};
+        Frag q[3];
+#pragma unroll
+        for (int p = 0; p < 3; p++) q[p].q = *reinterpret_cast<const uint4 *>(x + (size_t)p * in_p + k);
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            auto plane = [&](int p) { return __builtin_bit_cast(float, b16_slot(j) & 1 ? q[p].u[b16_slot(j) >> 1] & 0xFFFF0000u : q[p].u[b16_slot(j) >> 1] << 16); };
+            const float hi = plane(0), v = __builtin_isfinite(hi) ? hi + (plane(1) + plane(2)) : hi;
+            sum = __builtin_amdgcn_mfma_f32_16x16x4f32((&wv[j >> 2].x)[j & 3], v, sum, 0, 0, 0);
+        }
     }
-    return s;
+    return sum;
+}
+
+// Whether this lane's token has a NaN among the same inputs: then so are its outputs.  Every lane of the wave takes part.
+__device__ __forceinline__ bool dense_nan(const uint16_t *x, int k0, int k1) {
+    uint32_t most = 0;
+#pragma unroll 8
+    for (int k = k0; k < k1; k += 32) {
+        Frag q;
+        q.q = *reinterpret_cast<const uint4 *>(x + k);
+#pragma unroll
+        for (int i = 0; i < 4; i++) most = max(most, max(q.u[i] & 0x7FFFu, q.u[i] >> 16 & 0x7FFFu));
+    }
+    uint64_t any = __ballot(most > 0x7F80u); // of the four lanes that share the token
+    any |= any >> 32;
+    any |= any >> 16;
+    return any >> (threadIdx.x & 15) & 1;
 }
 
 template <int NT>
@@ -674,19 +700,27 @@ __device__ __forceinline__ void dense_tile(const Q4Launch &L, const XhList &xl, 
     size_t ws_base = 0;
     for (int i = 0; i < mi; i++) ws_base += (size_t)KS * B * L.m[i].out;
     const int o = obase + 4 * kg;
+    uint32_t again = 0; // the tiles of which this lane's part is not finite
 #pragma unroll
     for (int n = 0; n < NT; n++) {
         const int t = t0 + n * 16 + r;
         if (t >= B || o >= n_out) continue;
-        float4 v = make_float4(run[n][0], run[n][1], run[n][2], run[n][3]);
-        if (!__builtin_isfinite((v.x + v.y) + (v.z + v.w))) {
-            const uint16_t *xt = reinterpret_cast<const uint16_t *>(xh) + (size_t)t * NP * in_p;
-            const float *wo = reinterpret_cast<const float *>(w) + (size_t)o * in;
-            const int k0 = it0 * 64, k1 = min(it1 * 64, in);
-            v = make_float4(dense_again(wo, xt, in_p, k0, k1), dense_again(wo + in, xt, in_p, k0, k1),
-                            dense_again(wo + 2 * (size_t)in, xt, in_p, k0, k1), dense_again(wo + 3 * (size_t)in, xt, in_p, k0, k1));
-        }
-        finish4(L, mi, ss, ws + ws_base, KS, ks, partials, t, o, v);
+        const f4v v = run[n];
+        if (__builtin_isfinite((v[0] + v[1]) + (v[2] + v[3]))) finish4(L, mi, ss, ws + ws_base, KS, ks, partials, t, o, make_float4(v[0], v[1], v[2], v[3]));
+        else again |= 1u << n;
+    }
+    if (!__any(again)) return;
+    const float *const w_lane = reinterpret_cast<const float *>(w) + (size_t)min(obase + r, n_out - 1) * in + 8 * kg;
+#pragma unroll 1
+    for (int n = 0; n < NT; n++) {
+        if (!__any(again >> n & 1)) continue;
+        const int t = t0 + n * 16 + r;
+        const uint16_t *const x_lane = reinterpret_cast<const uint16_t *>(xh) + (size_t)min(t, B - 1) * NP * in_p + 8 * kg;
+        const int k0 = it0 * 64, k1 = min(it1 * 64, in);
+        f4v v{NAN, NAN, NAN, NAN};
+        const bool nan = dense_nan(x_lane, k0, k1);
+        if (__any((again >> n & 1) && !nan)) v = dense_again(w_lane, x_lane, in_p, k0, k1);
+        if (again >> n & 1) finish4(L, mi, ss, ws + ws_base, KS, ks, partials, t, o, make_float4(v[0], v[1], v[2], v[3]));
     }
 }
 

@@ -164,6 +164,34 @@ def test_dense_batch_tiles(ops, hidden):
     m.close()
 
 
+# finite operands whose planes or sums are not: every association has an infinity where all terms of a sum have one sign and it is
+# above the range, and none where the terms' magnitudes add up to less than the range; a weight that a plane would round to
+# infinity; the largest number of all.  Rows beyond the first block, the last tile of tokens, one K slice and several
+@pytest.mark.parametrize("dim,hidden", [(1024, 2816), (2048, 1344)])
+def test_dense_batch_overflow(ops, dim, hidden):
+    from llama2_rs import _lib
+    import tests.test_oracle_loop as tol
+    dims = ck.Dims(dim=dim, hidden_dim=hidden, n_layers=1, n_heads=dim // 128, n_kv_heads=1, vocab_size=64, seq_len=32, group_size=0)
+    img, top = ops.synth_image(dims, 6), np.finfo(np.float32).max
+    at = 1 + 64 * dim + dim + 2 * dim * dim + 2 * 128 * dim + dim  # of w1: in front of it eps, embedding, norm, q, k, v, o, norm
+    w1 = img.view(np.float32)[at:at + hidden * dim].reshape(hidden, dim)
+    w1[300, 7], w1[hidden - 1, 8] = 3.4e38, -top
+    m, rng, W = ops.Model(img, dims), np.random.default_rng(dim), w1.astype(np.float64)
+    np.testing.assert_array_equal(W, tol._split_image(img, dims)["w1"][0])
+    for B in (33, 100, 300):
+        x = rng.standard_normal((B, dim)).astype(np.float32)
+        x[:, 7:9] = rng.uniform(0.1, 0.3, (B, 2))
+        x[5], x[5, 3] = 0, top
+        x[B - 1], x[9] = np.sign(w1[2]) * 3e38, -np.sign(w1[hidden - 2]) * 3e38
+        got = m.qmatvec(0, _lib.W1, x)
+        assert got[B - 1, 2] == np.inf and got[9, hidden - 2] == -np.inf
+        want, mag = x.astype(np.float64) @ W.T, np.abs(x).astype(np.float64) @ np.abs(W).T
+        held = mag < top  # of the rest of the two rows, associations differ
+        assert held[5].all() and np.all(held[[b for b in range(B) if b not in (9, B - 1)]])
+        assert np.all(np.abs(got[held] - want[held]) <= dim * 2.0 ** -24 * mag[held])
+    m.close()
+
+
 # the same for quantised weights: several K slices and one, of one run of groups and of several (4128 and 4160 inputs, 512
 # columns: three and two; 8320: two), an odd number of K steps and half of one.  The rounding of the matrix unit must not
 # lean to one side either: the mean error of 512 columns' 4e6 values is below a thirtieth of their rms
