@@ -20,13 +20,14 @@ __device__ __forceinline__ u4v buffer(const void *base, size_t bytes) {
 __device__ __forceinline__ uint32_t lds_offset(void *p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)p; }
 
 // From memory into LDS past the registers: lane l's piece (16 or 4 bytes) at `off` + `soff` bytes of the buffer goes to
-// lds + size * l.  `at` (0..4095) shifts both by the same constant, so callers have it taken off `off`; buffers therefore begin kBias
-// bytes early and offsets are that much larger.  vmcnt counts these loads in order with all others, and since the compiler does
+// lds + `at` + size * l.  `at` (0..4095) shifts the source too, so callers have it taken off `off`; buffers therefore begin kBias
+// bytes early and offsets are that much larger.  The destination goes through m0, set in the same statement: the compiler keeps
+// what it holds there itself out of the way.  vmcnt counts these loads in order with all others, and since the compiler does
 // not know of them, nothing else in a loop that waits for them by number may load from memory.
 constexpr int kBias = 4096;
-#define LDS_TO(lds) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" ::"s"(lds) : "memory")
-#define LDS_LOAD(n, at, buf, off, soff) \
-    asm volatile("buffer_load_dword" n " %0, %1, %2 offen offset:%3 lds" ::"v"(off), "s"(buf), "s"(soff), "n"(at) : "memory")
+#define LDS_LOAD(n, lds, at, buf, off, soff) \
+    asm volatile("s_mov_b32 m0, %4\n\ts_nop 0\n\tbuffer_load_dword" n " %0, %1, %2 offen offset:%3 lds" \
+                 ::"v"(off), "s"(buf), "s"(soff), "n"(at), "s"(lds) : "memory", "m0")
 
 __device__ __forceinline__ u4v biased_buffer(const void *base, size_t bytes) { return buffer(reinterpret_cast<const char *>(base) - kBias, bytes + kBias); }
 

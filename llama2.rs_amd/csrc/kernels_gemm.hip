@@ -225,21 +225,20 @@ __device__ __forceinline__ void q4_tile(const Q4Launch &L, const XhList &xl, int
     const uint32_t x_last = (uint32_t)(it1 - 1) * 128;
     uint32_t x_at = (uint32_t)it0 * 128, w_at = (uint32_t)it0 * 32; // what is requested next (requests past the slice's end are never read)
     auto fetch_x = [&](uint32_t tile, const int i) __attribute__((always_inline)) {
-        LDS_TO(lds0 + tile + xfirst * 1024);
-        LDS_LOAD("x4", i * 1024, xbuf, xoff[i], x_at);
+        LDS_LOAD("x4", lds0 + tile + xfirst * 1024, i * 1024, xbuf, xoff[i], x_at);
         if (i == XP - 1) x_at = min(x_at + 128, x_last);
     };
     constexpr int WL = 2 + 2 * S::kGroupLoads;
     auto fetch_w = [&](uint32_t unit, const int i) __attribute__((always_inline)) {
-        LDS_TO(lds0 + wave_at + unit);
+        const uint32_t to = lds0 + wave_at + unit;
         if (i < 2) {
-            LDS_LOAD("x4", i * 1024, wbuf, woff[i], w_at);
+            LDS_LOAD("x4", to, i * 1024, wbuf, woff[i], w_at);
         } else { // in % 64 = 32: the last step's second group is the first one again (its inputs are zero)
             const uint32_t g = min(w_at * 2 / G + lane_group + (i >= 4 ? 2 : 0), (uint32_t)groups - 1) * 4;
-            if (i == 2) LDS_LOAD("", S::kWeights, sbuf, soff + g, 0);
-            else if (i == 3) LDS_LOAD("", S::kWeights + S::kScales, zbuf, zoff + g, 0);
-            else if (i == 4) LDS_LOAD("", S::kWeights + 256, sbuf, soff - 256 + g, 0);
-            else LDS_LOAD("", S::kWeights + S::kScales + 256, zbuf, zoff - 256 + g, 0);
+            if (i == 2) LDS_LOAD("", to, S::kWeights, sbuf, soff + g, 0);
+            else if (i == 3) LDS_LOAD("", to, S::kWeights + S::kScales, zbuf, zoff + g, 0);
+            else if (i == 4) LDS_LOAD("", to, S::kWeights + 256, sbuf, soff - 256 + g, 0);
+            else LDS_LOAD("", to, S::kWeights + S::kScales + 256, zbuf, zoff - 256 + g, 0);
         }
         if (i == WL - 1) w_at += 64;
     };

@@ -144,18 +144,17 @@ __device__ __forceinline__ void q4_gemm_tile(const Q4Launch &L, const XhList &xh
     uint32_t x_at = (uint32_t)u0 * 256, w_at = (uint32_t)u0 * 64;                       // what is requested next
     constexpr int WL = 2 + 2 * S::kScaleLoads;
     auto fetch_x = [&](const int slot, const int i) __attribute__((always_inline)) { // piece i of XP
-        LDS_TO(lds0 + slot * kTile + xfirst * 1024);
-        LDS_LOAD("x4", i * 1024, xbuf, xoff[i], x_at);
+        LDS_LOAD("x4", lds0 + slot * kTile + xfirst * 1024, i * 1024, xbuf, xoff[i], x_at);
         if (i == XP - 1) x_at = min(x_at + 128, x_last);
     };
     auto fetch_w = [&](const uint32_t unit, const int i) __attribute__((always_inline)) { // piece i of WL
         const uint32_t s_at = G == 128 ? w_at >> 4 : G == 64 ? w_at >> 3 : w_at >> 2;
-        LDS_TO(lds0 + wave_at + unit);
-        if (i < 2) LDS_LOAD("x4", i * 1024, wbuf, woff[i], w_at);
-        else if (i == 2) LDS_LOAD("", S::kWeights, sbuf, soff, s_at);
-        else if (i == 3) LDS_LOAD("", S::kWeights + S::kScales, zbuf, zoff, s_at);
-        else if (i == 4) LDS_LOAD("", S::kWeights + 256, sbuf, soff - 256 + 8, s_at); // G = 32: the second step's groups
-        else LDS_LOAD("", S::kWeights + S::kScales + 256, zbuf, zoff - 256 + 8, s_at);
+        const uint32_t to = lds0 + wave_at + unit;
+        if (i < 2) LDS_LOAD("x4", to, i * 1024, wbuf, woff[i], w_at);
+        else if (i == 2) LDS_LOAD("", to, S::kWeights, sbuf, soff, s_at);
+        else if (i == 3) LDS_LOAD("", to, S::kWeights + S::kScales, zbuf, zoff, s_at);
+        else if (i == 4) LDS_LOAD("", to, S::kWeights + 256, sbuf, soff - 256 + 8, s_at); // G = 32: the second step's groups
+        else LDS_LOAD("", to, S::kWeights + S::kScales + 256, zbuf, zoff - 256 + 8, s_at);
         if (i == WL - 1) w_at = min(w_at + 64, w_last);
     };
 
