@@ -87,10 +87,7 @@ __global__ __launch_bounds__(NWV * 64) void attn_decode_kernel(const AttnDecode 
     constexpr int NT = NWV * 64, TSTEP = NWV * 4;
     constexpr int HS = 128, HALF = 64;
     constexpr int VD = HS / DS, VE = VD / 16; // head dimensions of the value that are this block's, and a lane's share
-#ifndef V_PD
-#define V_PD 4
-#endif
-    constexpr int PD = QG >= 8 ? 2 : NWV > 4 ? V_PD : 4; // steps in flight and per pass through the phases (4 at 8 heads: over 256 registers, one block per CU, slower)
+    constexpr int PD = QG >= 8 ? 2 : 4; // steps in flight and per pass through the phases (4 at 8 heads: over 256 registers, one block per CU, slower)
     __shared__ float qs[QG * HS];
     __shared__ float kvnew[2][HS];
     // With 4 or 8 query heads per kv head the four 16-lane rows of every wave hand their partial results
