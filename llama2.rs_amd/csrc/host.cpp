@@ -1328,7 +1328,7 @@ extern "C" int l2_model_qmatvec(l2_model *m, int layer, int proj, const float *x
     if (q.dense) { // Linear::matvec<B> (src/model.rs:22-31)
         hipStream_t st = m->stream;
         L2_HIP(hipMemcpyAsync(m->op_x, x_host, (size_t)B * q.in * 4, hipMemcpyHostToDevice, st));
-        if (operator_planes(q, B, m->prefill_mode) && q.in == gemm_padded(q.in)) {
+        if (operator_planes(q, B, m->prefill_mode)) {
             L2_TRY(operator_bufs(m->op_batch, q, B, 3, st));
             GemmInput in{};
             in.out[0] = m->op_batch.planes, in.x = m->op_x, in.n = 1;

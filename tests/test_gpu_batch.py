@@ -164,6 +164,27 @@ def test_dense_batch_tiles(ops, hidden):
     m.close()
 
 
+# rows that end with half a K step: the operator takes the matrix cores as the model does (its bits are not the columns'), and
+# what lies behind a row's end, the last weights times zero, adds nothing even where those are infinite
+def test_dense_operator_half_step(ops):
+    from llama2_rs import _lib
+    import tests.test_oracle_loop as tol
+    dims = ck.Dims(dim=1024, hidden_dim=2848, n_layers=1, n_heads=8, n_kv_heads=1, vocab_size=64, seq_len=32, group_size=0)
+    img = ops.synth_image(dims, 6)
+    at = 1 + 64 * 1024 + 1024 + 2 * 1024 * 1024 + 2 * 128 * 1024 + 1024 + 2848 * 1024  # of w2
+    w2 = img.view(np.float32)[at:at + 1024 * 2848].reshape(1024, 2848)
+    w2[77, -1] = np.inf
+    m, rng, W = ops.Model(img, dims), np.random.default_rng(9), w2.astype(np.float64)
+    np.testing.assert_array_equal(W, tol._split_image(img, dims)["w2"][0])
+    for B in (33, 100, 300):
+        x = np.abs(rng.standard_normal((B, 2848))).astype(np.float32) + 0.01
+        got, one = m.qmatvec(0, _lib.W2, x), np.stack([m.qmatvec(0, _lib.W2, v) for v in x])
+        fine = np.arange(1024) != 77
+        assert not np.array_equal(got[:, fine], one[:, fine]) and np.all(got[:, 77] == np.inf)
+        assert nrel(got[:, fine], x.astype(np.float64) @ W[fine].T) < 1e-5
+    m.close()
+
+
 # finite operands whose planes or sums are not: every association has an infinity where all terms of a sum have one sign and it is
 # above the range, and none where the terms' magnitudes add up to less than the range; a weight that a plane would round to
 # infinity; the largest number of all.  Rows beyond the first block, the last tile of tokens, one K slice and several
