@@ -104,8 +104,7 @@ __device__ __forceinline__ void store_piece(void *out, size_t t, int in_p, int j
     for (int p = 0; p < NP; p++) dst[p * (in_p >> 3) + j8] = r.q[p];
 }
 
-// x[b][g_index[j]] * wn[g_index[j]] -> planes: the gather of src/gptq.rs:110-114 and the norm weight of
-// src/models.rs:63-66 in one pass.  grid (pieces / 256, B, consumers).
+// x[b][g_index[j]] -> planes: the gather of src/gptq.rs:110-114.  grid (pieces / 256, B, consumers).
 template <int NP>
 __global__ __launch_bounds__(256) void gemm_input_kernel(const GemmInput A, int n, int in_p) {
     const int b = blockIdx.y, c = blockIdx.z;
@@ -121,10 +120,6 @@ __global__ __launch_bounds__(256) void gemm_input_kernel(const GemmInput A, int 
         const int g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
 #pragma unroll
         for (int e = 0; e < 8; e++) v[e] = x[g[e]];
-        if (A.wn) {
-#pragma unroll
-            for (int e = 0; e < 8; e++) v[e] *= A.wn[g[e]];
-        }
     } else {
 #pragma unroll
         for (int e = 0; e < 8; e++) v[e] = 0.f;

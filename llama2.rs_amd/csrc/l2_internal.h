@@ -209,9 +209,8 @@ int gemm_warm_up(int group_size);
 struct GemmInput {
     void *out[3];
     const int32_t *g_index[3];
-    const float *x;  // [B][n], natural order
-    const float *wn; // [n] norm weight in natural order, or null
-    int n;           // consumers (1..3)
+    const float *x; // [B][n], natural order
+    int n;          // consumers (1..3)
 };
 int gemm_input_launch(const GemmInput &A, int n, int B, int planes, hipStream_t st);
 
