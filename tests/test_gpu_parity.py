@@ -247,6 +247,25 @@ def test_decode_attention_tile_edges(ops, oracle, n_heads, n_kv):
     o.close()
 
 
+@pytest.mark.parametrize("n_heads,n_kv", [(1, 1), (4, 2), (15, 15), (16, 16)])
+def test_decode_attention_whole_or_split(ops, oracle, n_heads, n_kv):
+    """Both sides of where a context is first cut into splits: 384 timesteps with few kv heads, 512 with more."""
+    dims = ck.Dims(dim=128 * n_heads, hidden_dim=512, n_layers=1, n_heads=n_heads, n_kv_heads=n_kv,
+                   vocab_size=300, seq_len=600, group_size=128)
+    img = ck.synth_weights_image(dims, seed=9)
+    m = ops.Model(img, dims)
+    o = oracle.Model(img, dims)
+    o.new_state()
+    m.fill_kv_synthetic(0, 590, seed=5)
+    ko, vo = o.kv_cache()
+    ko[0, :590], vo[0, :590] = m.read_kv(0, 0, 590)
+    for pos in (319, 320, 382, 383, 384, 385, 447, 448, 510, 511, 512):
+        want = o.transformer([11], [pos])
+        assert nrel(m.forward([11], [pos]), want) < REL_FP32, pos
+    m.close()
+    o.close()
+
+
 _VALU_ATTN_SNIPPET = r"""
 import sys, numpy as np
 sys.path.insert(0, sys.argv[1]); sys.path.insert(0, sys.argv[2])
