@@ -192,8 +192,8 @@ def test_forward_logits_and_cache_vs_oracle(ops, oracle, dims, tmp_path):
     o.close()
 
 
-@pytest.mark.parametrize("n_heads,n_kv,ctx", [(2, 2, 300), (8, 2, 257), (8, 1, 1000), (4, 2, 4300)],
-                         ids=["mha_5splits", "gqa4_first_split", "gqa8_16splits", "gqa2_deep"])
+@pytest.mark.parametrize("n_heads,n_kv,ctx", [(2, 2, 300), (2, 2, 700), (8, 2, 257), (8, 1, 1000), (4, 2, 4300)],
+                         ids=["mha_whole", "mha_11splits", "gqa4_first_split", "gqa8_16splits", "gqa2_deep"])
 def test_decode_attention_long_context(ops, oracle, n_heads, n_kv, ctx):
     """Decode steps behind a long cache: the timesteps are cut across blocks and merged.  The cache rows
     are synthetic (written on the device, copied into the oracle's cache), so no long prompt is needed."""
