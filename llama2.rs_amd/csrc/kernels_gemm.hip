@@ -1040,8 +1040,8 @@ GemmShape gemm_shape(const Q4Launch &L, int slice_batch, int planes) {
     };
     if (L.group_size == 0) {
         // Blocks of 128 columns, so that a weight is read and split once; of 64 where those would leave half the CUs without a
-        // block (four layers of 1024 inputs, 128 columns: 391 -> 350 us; 7B's widths keep 128: 64 columns at three quarters of
-        // the CUs 451 -> 478).  128 inputs per slice at least (1024 inputs, 100 columns 349 us with 256, 338).
+        // block (four layers of 1024 inputs, 128 columns: 424 -> 363 us; 7B's widths keep 128: 64 columns at three quarters of
+        // the CUs 530 -> 585).  128 inputs per slice at least (1024 inputs, 100 columns 367 us with 256, 348; with 64 349).
         s.slices = cheapest(rows32 * ((slice_batch + 127) / 128), std::min(kMaxGemmSlices, L.in / 128), 4);
         s.tokens = B <= 32 ? 32 : B <= 64 || 2 * rows32 * ((B + 127) / 128) * s.slices <= cus ? 64 : 128;
         s.rows = 128, s.row_blocks = rows32;
