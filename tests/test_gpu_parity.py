@@ -393,6 +393,29 @@ def test_decode_steps_as_graphs(ops, oracle, dims):
     o.close()
 
 
+@pytest.mark.parametrize("n_heads,n_kv", [(1, 1), (4, 2), (16, 16)])
+def test_decode_graphs_behind_a_context(ops, oracle, n_heads, n_kv):
+    """Captured steps of the buckets from 256 and 512 on: cut for the bucket's last position, replayed at its first ones."""
+    dims = ck.Dims(dim=128 * n_heads, hidden_dim=512, n_layers=2, n_heads=n_heads, n_kv_heads=n_kv,
+                   vocab_size=300, seq_len=700, group_size=128)
+    img = ck.synth_weights_image(dims, seed=10)
+    m = ops.Model(img, dims)
+    o = oracle.Model(img, dims)
+    o.new_state()
+    m.fill_kv_synthetic(0, 690, seed=6)
+    ko, vo = o.kv_cache()
+    for l in range(2):
+        ko[l, :690], vo[l, :690] = m.read_kv(l, 0, 690)
+    m.set_step_graph(True)
+    for pos in (511, 256, 300, 383, 384, 385, 447, 448, 255, 640, 512, 513, 511):
+        tok = pos % 300
+        assert m.decode_greedy(tok, pos) == oracle.argmax(o.transformer([tok], [pos])), pos
+        k, v = m.read_kv(1, pos, 1)
+        assert nrel(k, ko[1, pos:pos + 1]) < REL_FP32 and nrel(v, vo[1, pos:pos + 1]) < REL_FP32
+    m.close()
+    o.close()
+
+
 def test_kv_snapshot_restore(ops):
     """read_kv / write_kv: a cache restored into a fresh state continues with the same tokens."""
     dims = TINY_GQA
