@@ -115,6 +115,8 @@ __global__ __launch_bounds__(256) void gemm_input_kernel(const GemmInput A, int 
     if (j8 * 8 < n && !A.g_index[c]) { // no act-order: the model without quantisation
         const float4_any a = reinterpret_cast<const float4_any *>(x)[2 * j8], b4 = reinterpret_cast<const float4_any *>(x)[2 * j8 + 1];
         v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b4.x, v[5] = b4.y, v[6] = b4.z, v[7] = b4.w;
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = __builtin_canonicalizef(v[e]); // a signalling NaN's first plane could be an infinity (dense_again)
     } else if (j8 * 8 < n) {
         const int4 g0 = reinterpret_cast<const int4 *>(A.g_index[c])[2 * j8], g1 = reinterpret_cast<const int4 *>(A.g_index[c])[2 * j8 + 1];
         const int g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};

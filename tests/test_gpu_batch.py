@@ -161,6 +161,8 @@ def test_dense_batch_tiles(ops, hidden):
             np.testing.assert_array_equal(got[b], one[b])
         fine = [b for b in range(100) if b not in (3, 40, 50, 70, 99)]
         assert nrel(got[fine], x[fine].astype(np.float64) @ W.T) < 1e-5
+        x.view(np.uint32)[20, 9] = 0x7F800001  # a NaN by its last bit, as only memory holds one: no arithmetic makes it
+        assert np.all(np.isnan(m.qmatvec(0, proj, x)[20])) and np.all(np.isnan(m.qmatvec(0, proj, x[20])))
     m.close()
 
 
