@@ -570,6 +570,10 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const Q4Launch L
             }
         }
     };
+    auto pin = [](float(&pr)[NM]) __attribute__((always_inline)) {
+        if constexpr (NM == 2) asm volatile("" : "+v"(pr[0]), "+v"(pr[NM - 1])::"memory");
+        else asm volatile("" : "+v"(pr[0])::"memory");
+    };
     // 64 partials -> 4 (one per 16-lane row) -> the tile's slot for this row
     auto row_fold = [&](int u, const float(&pr)[NM]) __attribute__((always_inline)) {
 #pragma unroll
@@ -618,8 +622,7 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const Q4Launch L
             // live registers of the other slots, and each copy waits on its load.
             // The empty statements pin the row's result before the loads and
             // the loads before what follows.
-            if constexpr (NM == 2) asm volatile("" : "+v"(pr[0]), "+v"(pr[NM - 1])::"memory");
-            else asm volatile("" : "+v"(pr[0])::"memory");
+            pin(pr);
             __builtin_amdgcn_sched_barrier(0);
             fetch(i + P, pipe[u]);
             __builtin_amdgcn_sched_barrier(0);
@@ -641,12 +644,19 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const Q4Launch L
             if (u < n_rem) {
                 float pr[NM];
                 row_dot(row0 + stream + (n_full * P + u) * S, pipe[u], pr);
+                pin(pr); // else the scale's multiplication joins the fold's first addition, here and not in the loop, and a row's bits depend on P
                 row_fold(u, pr);
             }
         }
         __syncthreads();
         if ((unsigned)r < (unsigned)TR && eo < row1) tile_finish(r);
     }
+}
+
+static long total_rows(const Q4Launch &L) {
+    long rows = 0;
+    for (int i = 0; i < (L.pair ? 1 : L.n_mats); i++) rows += L.m[i].out;
+    return rows;
 }
 
 // Rows per block for a block of NW waves and tiles of TR rows: a whole number of rounds over the CUs, as
@@ -658,9 +668,8 @@ static int plan_rows(const Q4Launch &L, int NW, int TR, size_t lds, bool pair, i
     if (per_cu < 1) per_cu = 1;
     const int by_lds = (int)((150 * 1024) / (lds + 4 * 1024));
     if (per_cu > by_lds) per_cu = by_lds < 1 ? 1 : by_lds;
-    long rows = 0;
     const int nm = pair ? 1 : L.n_mats;
-    for (int i = 0; i < nm; i++) rows += L.m[i].out;
+    const long rows = total_rows(L);
     const long slots = (long)cu_count() * per_cu;
     int rpb = (int)((rows + slots - 1) / slots);
     if (rpb < TR) rpb = TR;
@@ -716,9 +725,24 @@ int launch_s(Q4Launch &L, hipStream_t stream) {
 // 13B's w1|w3 takes 17.3 us instead of 22.5 (9 waves 23.6, 6 waves 23.3) and wo 6.4 instead of 7.0.  16 waves with one pair of rows
 // in flight against 8 with two at 8192 inputs: 70B's w1|w3 43.9 -> 42.6 (12 waves with one or two pairs 46.8, 44.1).
 // 28672 -> 8192, two, three, four, five, six rows: 27.6 / 24.8 / 25.7 / 26.2 / 26.7 us; 13824 -> 5120, two rows or three: 11.0, 11.1.
+//
+// Few rows: a tile of P rows per stream is the least a block takes, so with the shapes above 1024 rows are 64 to 128 blocks, and
+// a launch is as long as the serial work of one of them.  With one row in flight per stream (and, at up to 2048 inputs, eight
+// streams) every CU has a block and a stream a row or two.  Cadence of the operator, before -> with the shape for few rows, us:
+// 1024 inputs, 1024 rows 3.37 -> 3.24, 4096 rows 3.50, 3.68 (not taken); 4096 inputs, 1024 rows 3.45 -> 3.20, 1536 rows 3.55,
+// 4.05 (not taken); 8192 inputs, 1024 rows 4.26 -> 3.98, 1536 rows 4.35, 4.70 (not taken).  The small model (1024 inputs, 2816
+// hidden, three layers), per token 74.5 -> 69.5.
+// Row pairs at up to 2048 inputs: eight streams of two pairs, 2048 -> 2 x 8192 87.3 -> 83.2 us per token of three layers.
+//
+// The gathering form has more to stage (x and where each of its elements goes) and nothing behind the sums, so it gains from more
+// waves per block: 4096 inputs in one block of 16 waves per CU instead of two of 8, two rows in flight: 4096 rows 4.70 -> 4.35 us,
+// 11008 rows 7.43 -> 6.76, 2048 rows 3.65, 4.02 (not taken); as a projection of the model the same shape loses (7B 287 -> 289 us
+// per 8 layers).  5120 inputs: two rows in flight up to 8192 rows, three beyond, instead of four: 1024 rows 4.65 -> 3.76, 5120 rows
+// 5.79 -> 5.54, 13824 rows 10.05 -> 9.81.
 template <int G, int MODE>
 int launch_sg(Q4Launch &L, hipStream_t stream) {
     const int nwk = (L.in / 32 + 63) / 64;
+    const long rows = total_rows(L), cus = cu_count();
     if constexpr (MODE == 2) { // only the shapes q4_stream_launch sends here
         if (!L.pair) switch (nwk) {
             case 3: return launch_s<G, 3, 4, false, MODE>(L, stream);
@@ -727,15 +751,18 @@ int launch_sg(Q4Launch &L, hipStream_t stream) {
         }
     } else if (MODE == 0 && !L.pair && L.n_mats == 1 && L.m[0].gidx) {
         if constexpr (MODE == 0) switch (nwk) { // the gathering form, where one staging batch covers the vector
-            case 1: return launch_s<G, 1, 4, false, 0, 4, true>(L, stream);
-            case 2: return launch_s<G, 2, 4, false, 0, 2, true>(L, stream);
-            case 3: return launch_s<G, 3, 4, false, 0, 4, true>(L, stream);
-            case 4: return launch_s<G, 4, 4, false, 0, 2, true>(L, stream);
+            case 1: return rows <= 8 * cus ? launch_s<G, 1, 8, false, 0, 1, true>(L, stream) : launch_s<G, 1, 4, false, 0, 4, true>(L, stream);
+            case 2:
+                if (rows <= 4 * cus) return launch_s<G, 2, 4, false, 0, 1, true>(L, stream);
+                if (rows <= 8 * cus) return launch_s<G, 2, 4, false, 0, 2, true>(L, stream);
+                return launch_s<G, 2, 8, false, 0, 2, true>(L, stream);
+            case 3: return rows <= 32 * cus ? launch_s<G, 3, 4, false, 0, 2, true>(L, stream) : launch_s<G, 3, 4, false, 0, 3, true>(L, stream);
+            case 4: return rows <= 4 * cus ? launch_s<G, 4, 4, false, 0, 1, true>(L, stream) : launch_s<G, 4, 4, false, 0, 2, true>(L, stream);
         }
     } else if (!L.pair) {
         switch (nwk) {
-            case 1: return launch_s<G, 1, 4, false, MODE>(L, stream);
-            case 2: return launch_s<G, 2, 4, false, MODE, 2>(L, stream);
+            case 1: return rows <= 8 * cus ? launch_s<G, 1, 8, false, MODE, 1>(L, stream) : launch_s<G, 1, 4, false, MODE>(L, stream);
+            case 2: return rows <= 4 * cus ? launch_s<G, 2, 4, false, MODE, 1>(L, stream) : launch_s<G, 2, 4, false, MODE, 2>(L, stream);
             case 3: return launch_s<G, 3, 4, false, MODE>(L, stream);
             case 4: return launch_s<G, 4, 4, false, MODE, 2>(L, stream); // 8192: rows of 4 KB; two in flight per stream measured faster than four (q|k|v 13.4 -> 12.2 us, wo 12.1 -> 10.9)
             case 5: case 6: return launch_s<G, 6, 2, false, MODE, 3>(L, stream);
@@ -745,7 +772,7 @@ int launch_sg(Q4Launch &L, hipStream_t stream) {
         }
     } else {
         switch (nwk) {
-            case 1: return launch_s<G, 1, 4, true, MODE>(L, stream);
+            case 1: return launch_s<G, 1, 8, true, MODE, 2>(L, stream);
             case 2: return launch_s<G, 2, 4, true, MODE>(L, stream);
             case 3: return launch_s<G, 3, 4, true, MODE>(L, stream);
             case 4: return launch_s<G, 4, 4, true, MODE, 1>(L, stream);

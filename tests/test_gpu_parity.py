@@ -80,6 +80,25 @@ def test_qmatvec_staging_edges(ops, oracle, n_in, n_out):
     q.close()
 
 
+# Both sides of where the number of rows chooses another shape of block (4, 8 and 32 rows per compute unit of 256), with x in
+# its natural order (one column) and gathered in front (three); group 32 with its most scales per row among them.
+@pytest.mark.parametrize("n_in,G,rows", [(1024, 32, (8, 2048, 2056)), (2048, 128, (2048, 2056)), (4096, 128, (1024, 1032, 2048, 2056)),
+                                         (2112, 64, (1024, 1032, 2056)), (5120, 128, (1024, 8192, 8200)), (4160, 32, (8200,)),
+                                         (8192, 64, (1024, 1032)), (6208, 64, (1024, 1032))])
+def test_qmatvec_shapes_by_rows(ops, oracle, n_in, G, rows):
+    rng = np.random.default_rng(n_in)
+    for n_out in rows:
+        qw, qz, sc, gi = ck.synth_qlinear(rng, n_in, n_out, G, act_order=True)
+        x = rng.standard_normal((3, n_in)).astype(np.float32)
+        want = oracle.qmatvec(qw, qz, sc, gi, G, x)
+        q = ops.QLinear(qw, qz, sc, gi, G)
+        got = q.matvec(x)
+        assert nrel(got, want) < REL_FP32, n_out
+        for b in range(3):
+            np.testing.assert_array_equal(q.matvec(x[b]), got[b], err_msg=str(n_out))
+        q.close()
+
+
 _ALT_FORM_SNIPPET = r"""
 import sys, numpy as np
 sys.path.insert(0, sys.argv[1]); sys.path.insert(0, sys.argv[2])
