@@ -1032,6 +1032,13 @@ static int q4_one(const DevQLinear &q, const float *xg, float *y, int B, hipStre
     return q4_matvec_launch(L, st);
 }
 
+// Whether the matvec kernel can apply g_index itself.
+static bool takes_natural_order(const DevQLinear &q) {
+    Q4Launch L = launch_of(q, 1, 0.f);
+    L.m[0] = mat_of(q, nullptr, nullptr, nullptr);
+    return q4_gathers_in_kernel(L);
+}
+
 // QLinear::matvec<B> on x in its natural order (src/gptq.rs:94-176, the act-order gather of :99-122 included):
 // one launch where the kernel can apply g_index itself, else a gather into xg_scratch and the matvec.
 static int q4_one_natural(const DevQLinear &q, const float *x, float *xg_scratch, float *y, int B, hipStream_t st) {
@@ -1070,16 +1077,21 @@ static int scratch_ptr(FixedScratch *out);
 // each) are resident at once, two per CU.
 static constexpr size_t kOperatorWsFloats = (size_t)512 * 256 * 64;
 
-// The operator on a batch through the matrix cores: gather + split into planes, GEMM, sum of the K slices.
-static int gemm_operator(const DevQLinear &q, const float *x, int B, float *y, int planes, void *xh, float *ws,
-                         size_t ws_floats, hipStream_t st) {
-    GemmInput in{};
-    in.out[0] = xh, in.g_index[0] = q.g_index, in.x = x, in.n = 1;
-    L2_TRY(gemm_input_launch(in, q.in, B, planes, st));
+// The operator on a batch through the matrix cores, activations already in planes: GEMM, sum of the K slices.
+static int gemm_operator(const DevQLinear &q, int B, float *y, int planes, void *xh, float *ws, size_t ws_floats, hipStream_t st) {
     Q4Launch L = launch_of(q, B, 0.f);
     L.m[0] = mat_of(q, nullptr, nullptr, y);
     XhList X{{xh, nullptr, nullptr}};
     return gemm_launch(L, X, nullptr, ws, ws_floats, planes, B, st);
+}
+
+// ... with x in device memory: gather + split into planes first.
+static int gemm_operator_natural(const DevQLinear &q, const float *x, int B, float *y, int planes, void *xh, float *ws,
+                                 size_t ws_floats, hipStream_t st) {
+    GemmInput in{};
+    in.out[0] = xh, in.g_index[0] = q.g_index, in.x = x, in.n = 1;
+    L2_TRY(gemm_input_launch(in, q.in, B, planes, st));
+    return gemm_operator(q, B, y, planes, xh, ws, ws_floats, st);
 }
 
 static int operator_bufs(OperatorBufs &b, const DevQLinear &q, int B, int planes, hipStream_t st) {
@@ -1201,17 +1213,19 @@ static int qlinear_scratch(l2_qlinear *q, int B) {
     return L2_OK;
 }
 
-static constexpr size_t kCopyKernelBytes = 64 * 1024; // up to here a copy kernel is quicker than the copy engine
+// From here on x comes in two parts: 16 columns of 13824 inputs 84.9 us whole, 81.5 by halves, 82.5 as a quarter and the rest.
+static constexpr size_t kSplitBytes = 256 * 1024;
 
 static int operator_enqueue(const DevQLinear &q, const float *dx, float *dxg, float *y, const OperatorBufs &bufs, int planes,
                             int B, hipStream_t st) {
     if (!planes) return q4_one_natural(q, dx, dxg, y, B, st);
-    return gemm_operator(q, dx, B, y, planes, bufs.planes, bufs.ws, bufs.ws_floats, st);
+    return gemm_operator_natural(q, dx, B, y, planes, bufs.planes, bufs.ws, bufs.ws_floats, st);
 }
 
 // x (host, natural order) -> gather through g_index -> matvec -> y (host).  Through a slot of pinned memory where x and y
-// fit one: x is fetched from there and the last kernel writes y there.  One 4096x4096 matvec 28-40 -> 19.6 us (pageable
-// copies either way before).
+// fit one: kernels fetch x from there and the last one writes y there.  One 4096x4096 matvec 28-40 -> 19.6 us (pageable
+// copies either way before); against a DMA from the slot and a gather on the device, 16 columns of 13824x5120 89 -> 82 us, 61 of
+// 4096x4096 116 -> 107, one of 28672x1024 32.8 -> 26.8.
 static int matvec_host(const DevQLinear &q, float *dx, float *dxg, float *dy, OperatorBufs &bufs, int planes,
                        const float *x_host, int B, float *y_host, hipStream_t st) {
     if (planes) L2_TRY(operator_bufs(bufs, q, B, planes, st));
@@ -1226,12 +1240,20 @@ static int matvec_host(const DevQLinear &q, float *dx, float *dxg, float *dy, Op
     HostSlot slot;
     L2_TRY(host_slots.take(&slot));
     auto call = [&]() -> int {
-        memcpy(slot.x, x_host, xb);
-        if (xb <= kCopyKernelBytes)
-            L2_TRY(copy_launch(dx, slot.x, xb / 4, st));
-        else
-            L2_HIP(hipMemcpyAsync(dx, slot.x, xb, hipMemcpyHostToDevice, st));
-        return operator_enqueue(q, dx, dxg, slot.y, bufs, planes, B, st);
+        const bool natural = !planes && takes_natural_order(q); // the matvec kernel gathers
+        // a long x in two parts: the host brings the second one while the first crosses the bus
+        for (int b0 = 0, b1 = B > 1 && xb >= kSplitBytes ? B / 2 : B; b0 < B; b0 = b1, b1 = B) {
+            const size_t at = (size_t)b0 * q.in, n = (size_t)(b1 - b0) * q.in;
+            memcpy(slot.x + at, x_host + at, n * sizeof(float));
+            if (natural)
+                L2_TRY(copy_launch(dx + at, slot.x + at, n, st));
+            else
+                L2_TRY(host_input_launch(planes ? (char *)bufs.planes + (size_t)b0 * planes * gemm_padded(q.in) * 2 : (char *)(dxg + at),
+                                         slot.x + at, q.inv_index, q.in, b1 - b0, planes, st));
+        }
+        if (natural) return q4_one_natural(q, dx, dxg, slot.y, B, st);
+        if (!planes) return q4_one(q, dxg, slot.y, B, st);
+        return gemm_operator(q, B, slot.y, planes, bufs.planes, bufs.ws, bufs.ws_floats, st);
     };
     int rc = call();
     const hipError_t e = hipStreamSynchronize(st);
@@ -1294,7 +1316,7 @@ extern "C" int l2_qlinear_matvec_device(l2_qlinear *q, const float *x_dev, int B
     // Every element of the scratch that is read has been written before by the same call: nothing of the
     // previous call's contents is read, so nothing needs clearing.
     if (operator_planes(q->q, B, q->mode))
-        return gemm_operator(q->q, x_dev, B, y_dev, 3, fixed.planes, fixed.ws, kOperatorWsFloats, st);
+        return gemm_operator_natural(q->q, x_dev, B, y_dev, 3, fixed.planes, fixed.ws, kOperatorWsFloats, st);
     // One column: the kernel applies the permutation while it stages x (one launch where the host's launch rate is what
     // counts: 9.7 -> 6.6 us per call at 8192x1024).  Its blocks read all of x while others write y already, so where y lies
     // over x, x is gathered by a launch in front.  Several columns are gathered once, rather than by every block of every column.

@@ -129,6 +129,53 @@ __global__ __launch_bounds__(256) void gemm_input_kernel(const GemmInput A, int 
     store_piece<NP>(A.out[c], b, in_p, j8, make_piece<NP>(v));
 }
 
+// The same from x in pinned host memory, where every element should cross the bus once and in order: read in order, 16 bytes per
+// thread and load, and scattered to its places.  NP = 0: fp32, for the matvec kernels.  What bounds it is the bus (48 GB/s, 18 us
+// for the 0.9 MB of 16 columns of 13824 inputs; the scattered stores take a third of that, behind it), so it is launched for a part
+// of the columns while the host brings the next one.  A DMA engine reads at 65 GB/s, but a kernel behind a DMA starts 10 us late.
+// With a column per block, read into LDS and permuted there, one compute unit's reads are the bound: one column of 28672 inputs
+// 32.8 -> 39.3 us for the call.
+constexpr int kHostPieces = 2; // of 16 bytes per thread (four: 84 us for 16 columns of 13824x5120, two 82)
+template <int NP>
+__global__ __launch_bounds__(256) void host_input_kernel(void *__restrict__ out, const float *__restrict__ x,
+                                                         const int32_t *__restrict__ inv, int n, int in_p) {
+    const int b = blockIdx.y, i0 = blockIdx.x * kHostPieces * 256 + threadIdx.x, n4 = n >> 2;
+    const float4 *src = reinterpret_cast<const float4 *>(x + (size_t)b * n);
+    float4 v[kHostPieces];
+    int4 to[kHostPieces];
+#pragma unroll
+    for (int u = 0; u < kHostPieces; u++) {
+        const int i = min(i0 + u * 256, n4 - 1); // past the end: the last piece again
+        v[u] = src[i];
+        to[u] = reinterpret_cast<const int4 *>(inv)[i];
+    }
+#pragma unroll
+    for (int u = 0; u < kHostPieces; u++) {
+        const float e[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+        const int j[4] = {to[u].x, to[u].y, to[u].z, to[u].w};
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            if constexpr (NP == 0) {
+                reinterpret_cast<float *>(out)[(size_t)b * n + j[k]] = e[k];
+            } else if constexpr (NP == 1) {
+                reinterpret_cast<_Float16 *>(out)[(size_t)b * in_p + h16_slot(j[k])] = (_Float16)e[k];
+            } else {
+                uint16_t *o = reinterpret_cast<uint16_t *>(out) + (size_t)b * NP * in_p + b16_slot(j[k]);
+                float left = e[k];
+#pragma unroll
+                for (int p = 0; p < NP; p++) { // as make_piece cuts it
+                    const uint32_t bits = __builtin_bit_cast(uint32_t, left) & 0xFFFF0000u;
+                    o[(size_t)p * in_p] = (uint16_t)(bits >> 16);
+                    left -= __builtin_bit_cast(float, bits);
+                }
+            }
+        }
+    }
+    if (NP > 0 && n + i0 < in_p && i0 < 64) // the rest of the row's last K step
+#pragma unroll
+        for (int p = 0; p < NP; p++) reinterpret_cast<uint16_t *>(out)[((size_t)b * NP + p) * in_p + n + i0] = 0;
+}
+
 // ---- the GEMM ----------------------------------------------------------------------------------------------------
 
 // Four consecutive outputs of column t: a partial tile of this K slice, or the result through the launch's epilogue.
@@ -1112,6 +1159,19 @@ int gemm_input_launch(const GemmInput &A, int n, int B, int planes, hipStream_t 
         hipLaunchKernelGGL(gemm_input_kernel<1>, grid, dim3(256), 0, st, A, n, in_p);
     else
         hipLaunchKernelGGL(gemm_input_kernel<3>, grid, dim3(256), 0, st, A, n, in_p);
+    L2_HIP(hipGetLastError());
+    return L2_OK;
+}
+
+int host_input_launch(void *out, const float *x, const int32_t *inv, int n, int B, int planes, hipStream_t st) {
+    if (n % 32 || n < 32 || B < 1 || !inv) return l2_fail(L2_ERR_ARG, "host input: n=%d, %d columns", n, B);
+    const dim3 grid((n / 4 + kHostPieces * 256 - 1) / (kHostPieces * 256), B);
+    switch (planes) {
+        case 0: hipLaunchKernelGGL(host_input_kernel<0>, grid, dim3(256), 0, st, out, x, inv, n, n); break;
+        case 1: hipLaunchKernelGGL(host_input_kernel<1>, grid, dim3(256), 0, st, out, x, inv, n, gemm_padded(n)); break;
+        case 3: hipLaunchKernelGGL(host_input_kernel<3>, grid, dim3(256), 0, st, out, x, inv, n, gemm_padded(n)); break;
+        default: return l2_fail(L2_ERR_ARG, "host input: %d planes", planes);
+    }
     L2_HIP(hipGetLastError());
     return L2_OK;
 }

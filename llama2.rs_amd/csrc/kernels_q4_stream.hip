@@ -742,7 +742,7 @@ int launch_s(Q4Launch &L, hipStream_t stream) {
 template <int G, int MODE>
 int launch_sg(Q4Launch &L, hipStream_t stream) {
     const int nwk = (L.in / 32 + 63) / 64;
-    const long rows = total_rows(L), cus = cu_count();
+    const long rows = total_rows(L) * L.batch, cus = cu_count(); // every column has blocks of its own
     if constexpr (MODE == 2) { // only the shapes q4_stream_launch sends here
         if (!L.pair) switch (nwk) {
             case 3: return launch_s<G, 3, 4, false, MODE>(L, stream);

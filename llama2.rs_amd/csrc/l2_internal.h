@@ -213,6 +213,9 @@ struct GemmInput {
     int n;          // consumers (1..3)
 };
 int gemm_input_launch(const GemmInput &A, int n, int B, int planes, hipStream_t st);
+// x[B][n] in pinned host memory, brought into the order of `inv` (the inverse of g_index) in device memory: as `planes`, or as
+// fp32 (planes 0).
+int host_input_launch(void *out, const float *x, const int32_t *inv, int n, int B, int planes, hipStream_t st);
 
 struct ResNormPrep {
     const float *ws;   // partial tiles [KS][B][out] of one matrix, or null: the stream is already complete

@@ -60,6 +60,24 @@ def test_any_float_address(ops, n_in, n_out, G, batches):
     hip.close()
 
 
+# The operator on host arrays scatters x from pinned memory where the one on device memory gathers it: the same bits.  Rows that end
+# inside a thread's first or second piece and with half a K step (4128), in one part and in two (256 KiB), even and odd; long rows for
+# the matvec kernels (12320).
+@pytest.mark.parametrize("n_in,n_out,G,batches", [(4128, 4104, 32, (4, 15, 16, 17, 61)), (2048, 4104, 64, (31, 32, 33, 128)),
+                                                  (12320, 264, 32, (1, 2, 3)), (28672, 1024, 64, (1, 3, 9))])
+def test_host_input_is_the_device_input(ops, n_in, n_out, G, batches):
+    hip = _Hip()
+    rng = np.random.default_rng(n_in)
+    q = ops.QLinear(*ck.synth_qlinear(rng, n_in, n_out, G, act_order=True), G)
+    for B in batches:
+        x = (rng.standard_normal((B, n_in)) * 10.0 ** rng.integers(-6, 7, (B, n_in))).astype(np.float32)
+        px, py = hip.upload(x), hip.empty(4 * B * n_out)
+        q.matvec_device(px, B, py)
+        np.testing.assert_array_equal(q.matvec(x), hip.download(py, (B, n_out)), err_msg=str(B))
+    q.close()
+    hip.close()
+
+
 # what one column enqueues (captured, not run): one kernel where x and y are apart, a gather in front where they meet
 def test_one_launch_only_apart(ops):
     hip = _Hip()
