@@ -31,6 +31,14 @@ constexpr int kBias = 4096;
 
 __device__ __forceinline__ u4v biased_buffer(const void *base, size_t bytes) { return buffer(reinterpret_cast<const char *>(base) - kBias, bytes + kBias); }
 
+// By what the 16-byte pieces 0..7 of token t lie permuted (xor) in an activation tile of 128-byte rows.  A 16-byte LDS read takes
+// the lanes 0-3, 12-15, 20-23 and 24-27 of each half of a wave together, then the others: with token r = l % 16 and piece
+// 2 (l / 16 % 4) + s in the lanes, or piece l / 16 % 4 + 4 s, these sixteen then meet sixteen different places.
+__device__ __forceinline__ int piece_xor(int t) {
+    const int q = t >> 1;
+    return (q & 1) | (q >> 1 & 2) | ((q << 1 ^ q) & 4);
+}
+
 // Blocks are dealt round-robin over the 8 XCDs, each with an L2 of its own: a contiguous range of the n items for each.
 __device__ __forceinline__ int xcd_item(int b, int n) {
     const int per = n >> 3, over = n & 7, xcd = b & 7;

@@ -248,7 +248,7 @@ __device__ __forceinline__ void q4_tile(const Q4Launch &L, const XhList &xl, int
 #pragma unroll
     for (int i = 0; i < XP; i++) {
         const int p = (xfirst + i) / (2 * NT), t = (xfirst + i) % (2 * NT) * 8 + (lane >> 3);
-        xoff[i] = ((uint32_t)min(t0 + t, B - 1) * NP + p) * (uint32_t)in_p * 2u + (((lane & 7) ^ ((t >> 1) & 7)) << 4) + kBias - i * 1024;
+        xoff[i] = ((uint32_t)min(t0 + t, B - 1) * NP + p) * (uint32_t)in_p * 2u + (((lane & 7) ^ piece_xor(t)) << 4) + kBias - i * 1024;
     }
 #pragma unroll
     for (int i = 0; i < 2; i++) {
@@ -259,7 +259,7 @@ __device__ __forceinline__ void q4_tile(const Q4Launch &L, const XhList &xl, int
     const uint32_t soff = (uint32_t)(srow * groups) * 4u + kBias - S::kWeights, zoff = (uint32_t)((srow >> 3) * groups) * 4u + kBias - S::kWeights - S::kScales;
     uint32_t xr[2]; // where the lane reads a token's piece of MFMA k
 #pragma unroll
-    for (int k = 0; k < 2; k++) xr[k] = (uint32_t)r * kStepRow + (((G == 32 ? 4 * k + kg : 2 * kg + k) ^ ((r >> 1) & 7)) << 4);
+    for (int k = 0; k < 2; k++) xr[k] = (uint32_t)r * kStepRow + (((G == 32 ? 4 * k + kg : 2 * kg + k) ^ piece_xor(r)) << 4);
     // ... and its words of a unit's first step (the second's: ^ 32)
     const int wsw = (r >> 2) & 3;
     const uint32_t wr0 = wave_at + r * 64 + (G == 32 ? (wsw << 4) + kg * 4 : (((kg >> 1) ^ wsw) << 4) + (kg & 1) * 8);

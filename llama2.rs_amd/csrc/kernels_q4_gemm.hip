@@ -122,7 +122,7 @@ __device__ __forceinline__ void q4_gemm_tile(const Q4Launch &L, const XhList &xh
 #pragma unroll
     for (int i = 0; i < XP; i++) { // activations: 8 tokens of 128 bytes, a token's 16-byte pieces permuted by its number
         const int t = (xfirst + i) * 8 + (lane >> 3);
-        xoff[i] = (uint32_t)min(t0 + t, B - 1) * (uint32_t)in * 2u + (((lane & 7) ^ ((t >> 1) & 7)) << 4) + kBias - i * 1024;
+        xoff[i] = (uint32_t)min(t0 + t, B - 1) * (uint32_t)in * 2u + (((lane & 7) ^ piece_xor(t)) << 4) + kBias - i * 1024;
     }
 #pragma unroll
     for (int i = 0; i < 2; i++) { // weights: 16 rows of 64 bytes, permuted likewise
@@ -135,7 +135,7 @@ __device__ __forceinline__ void q4_gemm_tile(const Q4Launch &L, const XhList &xh
     // ... and where it reads them
     uint32_t xr[2]; // piece 2 kg + s of token r
 #pragma unroll
-    for (int s = 0; s < 2; s++) xr[s] = (uint32_t)r * kStepRow + (((2 * kg + s) ^ ((r >> 1) & 7)) << 4);
+    for (int s = 0; s < 2; s++) xr[s] = (uint32_t)r * kStepRow + (((2 * kg + s) ^ piece_xor(r)) << 4);
     const uint32_t wr = wave_at + r * 64 + (((kg >> 1) ^ ((r >> 2) & 3)) << 4) + (kg & 1) * 8; // of a unit's first step; the second's: ^ 32
     const uint32_t sr = wave_at + S::kWeights + kg * 16, zr = wave_at + S::kWeights + ((G == 32 ? (kg >> 1) * 32 : 0) + r) * 4;
     const int zsh = 4 * (r & 7); // obase is a multiple of 8
