@@ -570,10 +570,6 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const Q4Launch L
             }
         }
     };
-    auto pin = [](float(&pr)[NM]) __attribute__((always_inline)) {
-        if constexpr (NM == 2) asm volatile("" : "+v"(pr[0]), "+v"(pr[NM - 1])::"memory");
-        else asm volatile("" : "+v"(pr[0])::"memory");
-    };
     // 64 partials -> 4 (one per 16-lane row) -> the tile's slot for this row
     auto row_fold = [&](int u, const float(&pr)[NM]) __attribute__((always_inline)) {
 #pragma unroll
@@ -622,7 +618,8 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const Q4Launch L
             // live registers of the other slots, and each copy waits on its load.
             // The empty statements pin the row's result before the loads and
             // the loads before what follows.
-            pin(pr);
+            if constexpr (NM == 2) asm volatile("" : "+v"(pr[0]), "+v"(pr[NM - 1])::"memory");
+            else asm volatile("" : "+v"(pr[0])::"memory");
             __builtin_amdgcn_sched_barrier(0);
             fetch(i + P, pipe[u]);
             __builtin_amdgcn_sched_barrier(0);
@@ -644,7 +641,8 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const Q4Launch L
             if (u < n_rem) {
                 float pr[NM];
                 row_dot(row0 + stream + (n_full * P + u) * S, pipe[u], pr);
-                pin(pr); // else the scale's multiplication joins the fold's first addition, here and not in the loop, and a row's bits depend on P
+                // no pin: here the scale's multiplication joins the fold's first addition, so a row's last bit depends on whether it
+                // stands behind the loop, that is on the shape and on the rows of the block
                 row_fold(u, pr);
             }
         }
@@ -684,12 +682,21 @@ static int plan_rows(const Q4Launch &L, int NW, int TR, size_t lds, bool pair, i
     return rpb;
 }
 
+static size_t staging_lds(int NWK, bool pair) { return (size_t)NWK * 64 * (kChunkPad + 1) * sizeof(float) * (pair ? 2 : 1); }
+
+// Whether one matrix in blocks of S streams with P rows in flight has no rows behind the loop (whose last bit is another).
+static bool whole_tiles(const Q4Launch &L, int NWK, int S, int P) {
+    int blocks = 0;
+    const int rpb = plan_rows(L, NWK * S, P * S, staging_lds(NWK, false), false, &blocks), last = L.m[0].out - (blocks - 1) * rpb;
+    return (rpb + S - 1) / S % P == 0 && (last + S - 1) / S % P == 0;
+}
+
 template <int G, int NWK, int S, bool PAIR, int MODE, int P = (PAIR ? 2 : 4), bool GATHER = false>
 int launch_s(Q4Launch &L, hipStream_t stream) {
     constexpr int NW = NWK * S;
     constexpr int TR = P * S;
     const size_t lds = MODE == 2 ? (size_t)NW * 64 * kChunkPad * sizeof(float)
-                                 : (size_t)NWK * 64 * (kChunkPad + 1) * sizeof(float) * (PAIR ? 2 : 1);
+                                 : staging_lds(NWK, PAIR);
     if (lds + 8 * 1024 > 160 * 1024) return l2_fail(L2_ERR_ARG, "q4 matvec: in=%d needs %zu B of LDS", L.in, lds);
     int total = 0;
     const int rpb = plan_rows(L, NW, TR, lds, PAIR, &total);
@@ -738,7 +745,8 @@ int launch_s(Q4Launch &L, hipStream_t stream) {
 // waves per block: 4096 inputs in one block of 16 waves per CU instead of two of 8, two rows in flight: 4096 rows 4.70 -> 4.35 us,
 // 11008 rows 7.43 -> 6.76, 2048 rows 3.65, 4.02 (not taken); as a projection of the model the same shape loses (7B 287 -> 289 us
 // per 8 layers).  5120 inputs: two rows in flight up to 8192 rows, three beyond, instead of four: 1024 rows 4.65 -> 3.76, 5120 rows
-// 5.79 -> 5.54, 13824 rows 10.05 -> 9.81.
+// 5.79 -> 5.54, 13824 rows 10.05 -> 9.81.  These are taken where neither shape has rows behind the loop, so that one column of
+// the operator is, bit for bit, a column of several, which the form without the gathering takes in its own shape.
 template <int G, int MODE>
 int launch_sg(Q4Launch &L, hipStream_t stream) {
     const int nwk = (L.in / 32 + 63) / 64;
@@ -754,10 +762,13 @@ int launch_sg(Q4Launch &L, hipStream_t stream) {
             case 1: return rows <= 8 * cus ? launch_s<G, 1, 8, false, 0, 1, true>(L, stream) : launch_s<G, 1, 4, false, 0, 4, true>(L, stream);
             case 2:
                 if (rows <= 4 * cus) return launch_s<G, 2, 4, false, 0, 1, true>(L, stream);
-                if (rows <= 8 * cus) return launch_s<G, 2, 4, false, 0, 2, true>(L, stream);
-                return launch_s<G, 2, 8, false, 0, 2, true>(L, stream);
-            case 3: return rows <= 32 * cus ? launch_s<G, 3, 4, false, 0, 2, true>(L, stream) : launch_s<G, 3, 4, false, 0, 3, true>(L, stream);
-            case 4: return rows <= 4 * cus ? launch_s<G, 4, 4, false, 0, 1, true>(L, stream) : launch_s<G, 4, 4, false, 0, 2, true>(L, stream);
+                if (rows > 8 * cus && whole_tiles(L, 2, 4, 2) && whole_tiles(L, 2, 8, 2)) return launch_s<G, 2, 8, false, 0, 2, true>(L, stream);
+                return launch_s<G, 2, 4, false, 0, 2, true>(L, stream);
+            case 3:
+                if (rows <= 32 * cus && whole_tiles(L, 3, 4, 4) && whole_tiles(L, 3, 4, 2)) return launch_s<G, 3, 4, false, 0, 2, true>(L, stream);
+                if (rows > 32 * cus && whole_tiles(L, 3, 4, 4) && whole_tiles(L, 3, 4, 3)) return launch_s<G, 3, 4, false, 0, 3, true>(L, stream);
+                return launch_s<G, 3, 4, false, 0, 4, true>(L, stream);
+            case 4: return rows <= 4 * cus && whole_tiles(L, 4, 4, 2) ? launch_s<G, 4, 4, false, 0, 1, true>(L, stream) : launch_s<G, 4, 4, false, 0, 2, true>(L, stream);
         }
     } else if (!L.pair) {
         switch (nwk) {
