@@ -1836,8 +1836,13 @@ int l2_forward_weights(l2_model *m, l2_state *s, int32_t token, int32_t pos, flo
     return L2_OK;
 }
 
-// The lanes of l2_prefill_chunks: streams, events, buffers.
-static int ensure_prefill_pipeline(l2_model *m, int lanes, int B, int slice_batch, int planes) {
+// One pass over consecutive positions: whole chunks of the caller's that are cut into the same K slices.
+struct PrefillPass {
+    int first, n, slice_batch, planes;
+};
+// The lanes of l2_prefill_chunks: streams, events and buffers for `passes`, any of them on any lane.  (A longer chunk may be
+// cut into more slices than a shorter one, so no single pass stands for all.)
+static int ensure_prefill_pipeline(l2_model *m, int lanes, const std::vector<PrefillPass> &passes) {
     for (int i = 0; i + 1 < lanes; i++)
         if (!m->extra_stream[i]) L2_HIP(hipStreamCreate(&m->extra_stream[i])); // default priority, as the model's own
     if (!m->pf_join) L2_HIP(hipEventCreateWithFlags(&m->pf_join, hipEventDisableTiming));
@@ -1847,15 +1852,14 @@ static int ensure_prefill_pipeline(l2_model *m, int lanes, int B, int slice_batc
             L2_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
             m->pf_ev[i].push_back(e);
         }
-        if (planes) L2_TRY(ensure_lane(m, i, B, slice_batch, planes));
+        for (size_t p = 0; p < passes.size(); p++) {
+            const bool again = p > 0 && passes[p].n == passes[p - 1].n && passes[p].slice_batch == passes[p - 1].slice_batch;
+            if (passes[p].planes && !again) L2_TRY(ensure_lane(m, i, passes[p].n, passes[p].slice_batch, passes[p].planes));
+        }
     }
     return L2_OK;
 }
 
-// One pass over consecutive positions: whole chunks of the caller's that are cut into the same K slices.
-struct PrefillPass {
-    int first, n, slice_batch, planes;
-};
 static constexpr int kPassTokens = 512;
 
 // prefill<A> (src/inference.rs:16-40) for a whole prompt: tokens[i] at position pos0 + i, in chunks of `chunk`, no
@@ -1875,7 +1879,6 @@ static int prefill_chunks(l2_model *m, l2_state *s, const int32_t *tokens, int n
             return l2_fail(L2_ERR_RANGE, "token id %d outside 0..%d", tokens[i], m->d.vocab_size - 1);
     std::vector<PrefillPass> passes;
     int rest = 0; // most columns of a chunk that the matvec kernels take
-    int widest = 0, cut = 0, planes = 0;
     for (int c0 = 0; c0 < n; c0 += chunk) {
         const int B = std::min(chunk, n - c0), p = batch_planes(m, B);
         if (!p) rest = std::max(rest, B);
@@ -1889,10 +1892,8 @@ static int prefill_chunks(l2_model *m, l2_state *s, const int32_t *tokens, int n
         passes.push_back({c0, B, B, p});
     }
     const int lanes = passes.size() > 1 ? m->n_lanes : 1;
-    for (const PrefillPass &p : passes)
-        if (p.planes) widest = std::max(widest, p.n), cut = cut ? std::min(cut, p.slice_batch) : p.slice_batch, planes = p.planes;
     L2_TRY(ensure_batch(m, std::max(rest, 1)));
-    L2_TRY(ensure_prefill_pipeline(m, lanes, widest, cut, planes));
+    L2_TRY(ensure_prefill_pipeline(m, lanes, passes));
     L2_TRY(ensure_ids(m, n));
     L2_TRY(claim_host_ids(m));
     memcpy(m->hs.in, tokens, (size_t)n * 4);

@@ -400,3 +400,21 @@ def test_prompt_past_the_steps(ops):
     for a, b in zip(*rows):
         assert np.any(a[383]) and np.array_equal(a, b)
     m.close()
+
+
+# two passes of one prompt, the longer chunk cut into more slices of K than the shorter one (5120 inputs, 3 x 5120 rows: 256
+# columns in two, 143 in one): the buffers hold either
+def test_chunks_cut_into_more_slices_than_the_last(ops):
+    from llama2_rs import _lib
+    dims = ck.Dims(dim=5120, hidden_dim=384, n_layers=1, n_heads=40, n_kv_heads=40, vocab_size=64, seq_len=512, group_size=64)
+    m = ops.Model(ck.synth_weights_image(dims, seed=4), dims)
+    m.set_prefill_mode(_lib.PREFILL_MFMA)
+    toks = np.random.default_rng(1).integers(0, 64, size=399).astype(np.int32)
+    m.prefill_chunks(toks, 0, 256)
+    got = m.read_kv(0, 0, 399)
+    m.reset()
+    for a, b in ((0, 256), (256, 399)):
+        m.forward(toks[a:b], np.arange(a, b, dtype=np.int32))
+    for x, y in zip(got, m.read_kv(0, 0, 399)):
+        np.testing.assert_array_equal(x, y)
+    m.close()
