@@ -315,7 +315,7 @@ __device__ __forceinline__ void q4_gemm_tile(const Q4Launch &L, const XhList &xh
             if (KS > 1 || partials) { // partial tile of this K slice
                 float *at = ws + ws_base + ((size_t)ks * B + t) * n_out + o;
                 if (partials > 1) __builtin_nontemporal_store(f4v{v.x, v.y, v.z, v.w}, reinterpret_cast<f4v *>(at));
-                else *reinterpret_cast<float4 *>(at) = v;
+                else store_through(reinterpret_cast<float4 *>(at), v);
                 continue;
             }
             const float scale_t = ss ? ss[t] : 1.0f;
@@ -382,7 +382,8 @@ int launch_gemm(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const
     // 224 narrow tiles behind 64 left over (70B's, 776) they take 822 and whole tiles 804
     if (NB == 4 && s.slices == 1 && 2 * (tiles % cu_count()) + narrow * row_blocks <= cu_count()) whole = tiles / cu_count() * cu_count();
     // partial tiles past the caches where they would fill them: what a launch leaves dirty there is written back at its end
-    // (7B, 511 tokens: the four launches 13 us less per layer, their consumers 5 more; below 16 MB the other way round)
+    // (7B, 511 tokens: the four launches 13 us less per layer, their consumers 5 more; below 16 MB the other way round: there they
+    // go past the L2 but not past the memory-side cache, see store_through)
     size_t bytes = 0;
     for (int i = 0; i < L.n_mats; i++) bytes += (size_t)s.slices * L.batch * L.m[i].out * 4;
     if (partials && bytes > ((size_t)16 << 20)) partials = 2;

@@ -33,6 +33,19 @@ inline int cu_count() {
 // at any multiple of four, so a load or store through this is the same one instruction as through float4.
 typedef float float4_any __attribute__((ext_vector_type(4), aligned(4)));
 
+// 16 bytes (aligned) past the L2: what a launch leaves dirty there is written back at its end, with nothing else to do, and the
+// kernels of a batch write megabytes in their last microseconds.  Not for single columns: the store's own way is longer, and that
+// is what the end of a decode kernel waits for (7B token 2 to 3 % longer, 70B 5 %).  The s_nop: data of a store wider than 8 bytes
+// must not be overwritten by the very next instruction, which the compiler sees to for its own stores only.
+#if defined(__HIPCC__)
+template <class T>
+__device__ __forceinline__ void store_through(T *p, const T &v) {
+    static_assert(sizeof(T) == 16, "one instruction");
+    typedef uint32_t four __attribute__((ext_vector_type(4)));
+    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 0" ::"v"(p), "v"(__builtin_bit_cast(four, v)) : "memory");
+}
+#endif
+
 // ---- error plumbing -------------------------------------------------------
 int l2_fail(int code, const char *fmt, ...) __attribute__((format(printf, 2, 3)));
 
