@@ -379,8 +379,9 @@ int launch_gemm(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const
     const int tiles = row_blocks * t_full * s.slices;
     int whole = tiles;
     // halves where they and the narrow tiles fit one round: 7B's w1|w3, 511 tokens, 344 tiles on 256 CUs 123 -> 112 us; with
-    // 224 narrow tiles behind 64 left over (70B's, 776) they take 822 and whole tiles 804
-    if (NB == 4 && s.slices == 1 && 2 * (tiles % cu_count()) + narrow * row_blocks <= cu_count()) whole = tiles / cu_count() * cu_count();
+    // 224 narrow tiles behind 64 left over (70B's, 776) they take 822 and whole tiles 804.  With several slices too: four layers of
+    // 13B, group 64, 399 tokens 2192 -> 2135, six of 7B, group 32, 249 tokens 1656 -> 1610
+    if (NB == 4 && 2 * (tiles % cu_count()) + narrow * row_blocks * s.slices <= cu_count()) whole = tiles / cu_count() * cu_count();
     // partial tiles past the caches where they would fill them: what a launch leaves dirty there is written back at its end
     // (7B, 511 tokens: the four launches 13 us less per layer, their consumers 5 more; below 16 MB the other way round: there they
     // go past the L2 but not past the memory-side cache, see store_through)
