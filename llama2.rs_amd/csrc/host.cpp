@@ -289,6 +289,7 @@ struct l2_model {
                 *wcls = nullptr;
     std::vector<DevQLinear> q[7]; // indexed by L2_WQ..L2_W3, then layer
     int32_t *dinv = nullptr;      // all inverse permutations
+    float *dtiles = nullptr;      // scales and zero points of all projections in tiles of 32 rows
     float *rope_cos = nullptr, *rope_sin = nullptr; // [max_seq][head_size/2]
 
     float *dwn = nullptr;         // norm weights in consumer order: [L][5][dim] (q, k, v, w1, w3)
@@ -422,7 +423,7 @@ static void step_graph_drop(StepGraph &g);
 
 struct l2_qlinear {
     DevQLinear q;
-    void *bufs[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
+    void *bufs[6] = {}; // the five arrays, the group tiles
     hipStream_t stream = nullptr;
     float *x = nullptr, *xg = nullptr, *y = nullptr;
     int cap_B = 0;
@@ -521,6 +522,13 @@ static void invert_perm(const int32_t *g, int n, int32_t *inv, bool *ok) {
 }
 
 static constexpr size_t kImageShift = 124; // image offset 4 (first tensor) lands on a 128-byte boundary
+
+// q's group tiles in the memory at `tiles`; returns how much of it they take.
+static size_t make_group_tiles(DevQLinear &q, float *tiles) {
+    q.scales_t = tiles;
+    q.zeros_t = reinterpret_cast<const int32_t *>(tiles + (size_t)((q.out + 31) / 32) * q.groups * 32);
+    return group_tiles_floats(q.out, q.groups);
+}
 
 static int model_build(const char *weights, size_t nbytes, const l2_dims *dims, int max_seq, l2_model **out) {
     L2_TRY(check_dims(dims));
@@ -647,6 +655,15 @@ static int model_build(const char *weights, size_t nbytes, const l2_dims *dims, 
         M_TRY(dalloc(&m->dinv, inv_total));
         M_HIP(hipMemcpy(m->dinv, inv.data(), inv_total * 4, hipMemcpyHostToDevice));
         for (const Pending &p : pend) m->q[p.proj][p.layer].inv_index = m->dinv + p.inv_off;
+        size_t tiles = 0;
+        for (const Pending &p : pend) tiles += group_tiles_floats(m->q[p.proj][p.layer].out, m->q[p.proj][p.layer].groups);
+        M_TRY(dalloc(&m->dtiles, tiles));
+        tiles = 0;
+        for (const Pending &p : pend) tiles += make_group_tiles(m->q[p.proj][p.layer], m->dtiles + tiles);
+        for (const Pending &p : pend) {
+            const DevQLinear &q = m->q[p.proj][p.layer];
+            M_TRY(group_tiles_launch(q.scales, q.qzeros, q.out, q.groups, const_cast<float *>(q.scales_t), m->stream));
+        }
     }
 
     M_TRY(dalloc(&m->attn_part, (size_t)dims->n_heads * kMaxSplits * 130));
@@ -761,7 +778,7 @@ extern "C" void l2_model_close(l2_model *m) {
     if (m->stream) (void)hipStreamSynchronize(m->stream);
     for (hipStream_t es : m->extra_stream)
         if (es) (void)hipStreamSynchronize(es);
-    void *ptrs[] = {m->dimage, m->dinv, m->rope_cos, m->rope_sin, m->dwn, m->attn_part, m->x, m->xq, m->xk,
+    void *ptrs[] = {m->dimage, m->dinv, m->dtiles, m->rope_cos, m->rope_sin, m->dwn, m->attn_part, m->x, m->xq, m->xk,
                     m->xv, m->qv, m->kv, m->vv, m->attg, m->x1, m->x3, m->hg, m->hd, m->logits, m->dtok, m->dpos, m->dloop,
                     m->amax, m->dprompt, m->dout_ids, m->op_x, m->op_xg, m->op_y, m->op_batch.planes, m->op_batch.ws};
     for (void *p : ptrs) dfree(p);
@@ -1013,6 +1030,13 @@ static Q4Mat mat_of(const DevQLinear &q, const float *x, const float *wn, float 
     return M;
 }
 
+// The same for gemm_launch.
+static Q4Mat gemm_mat_of(const DevQLinear &q, float *y) {
+    Q4Mat M = mat_of(q, nullptr, nullptr, y);
+    M.qzeros = q.zeros_t, M.scales = q.scales_t;
+    return M;
+}
+
 static Q4Launch launch_of(const DevQLinear &q, int B, float eps) {
     Q4Launch L{};
     L.n_mats = 1;
@@ -1080,7 +1104,7 @@ static constexpr size_t kOperatorWsFloats = (size_t)512 * 256 * 64;
 // The operator on a batch through the matrix cores, activations already in planes: GEMM, sum of the K slices.
 static int gemm_operator(const DevQLinear &q, int B, float *y, int planes, void *xh, float *ws, size_t ws_floats, hipStream_t st) {
     Q4Launch L = launch_of(q, B, 0.f);
-    L.m[0] = mat_of(q, nullptr, nullptr, y);
+    L.m[0] = gemm_mat_of(q, y);
     XhList X{{xh, nullptr, nullptr}};
     return gemm_launch(L, X, nullptr, ws, ws_floats, planes, B, st);
 }
@@ -1169,7 +1193,14 @@ extern "C" int l2_qlinear_create(const int32_t *qweight, const int32_t *qzeros, 
     q->q.out = out;
     q->q.groups = groups;
     q->q.group_size = group_size;
-    const int rc = qlinear_warm_up(q);
+    float *tiles = nullptr;
+    int rc = dalloc(&tiles, group_tiles_floats(out, groups));
+    q->bufs[5] = tiles;
+    if (rc == L2_OK) {
+        make_group_tiles(q->q, tiles);
+        rc = group_tiles_launch(q->q.scales, q->q.qzeros, out, groups, tiles, q->stream);
+    }
+    if (rc == L2_OK) rc = qlinear_warm_up(q);
     if (rc != L2_OK) {
         l2_qlinear_free(q);
         return rc;
@@ -1356,7 +1387,7 @@ extern "C" int l2_model_qmatvec(l2_model *m, int layer, int proj, const float *x
             in.out[0] = m->op_batch.planes, in.x = m->op_x, in.n = 1;
             L2_TRY(gemm_input_launch(in, q.in, B, 3, st));
             Q4Launch L = launch_of(q, B, 0.f);
-            L.m[0] = mat_of(q, nullptr, nullptr, m->op_y);
+            L.m[0] = gemm_mat_of(q, m->op_y);
             L2_TRY(gemm_launch(L, XhList{{m->op_batch.planes, nullptr, nullptr}}, nullptr, m->op_batch.ws, m->op_batch.ws_floats, 3, B, st));
         } else {
             DenseArgs a{};
@@ -1710,9 +1741,9 @@ static int forward_enqueue_gemm(l2_model *m, l2_state *s, int B, int max_pos, co
         float *vc = s->vcache + (size_t)l * m->max_seq * kvd;
         {   // q, k, v: partial tiles; the kernel that adds them also applies the rms scale, RoPE and the cache write
             Q4Launch Q = launch_of(wq, B, m->rms_eps);
-            Q.m[0] = mat_of(wq, nullptr, nullptr, nullptr);
-            Q.m[1] = mat_of(wk, nullptr, nullptr, nullptr);
-            Q.m[2] = mat_of(wv, nullptr, nullptr, nullptr);
+            Q.m[0] = gemm_mat_of(wq, nullptr);
+            Q.m[1] = gemm_mat_of(wk, nullptr);
+            Q.m[2] = gemm_mat_of(wv, nullptr);
             Q.n_mats = 3;
             RopeKvArgs R{};
             L2_TRY(gemm(Q, dense ? XhList{{b.h[0], b.h[0], b.h[0]}} : XhList{{b.h[0], b.h[1], b.h[2]}}, nullptr, &R.KS));
@@ -1729,7 +1760,7 @@ static int forward_enqueue_gemm(l2_model *m, l2_state *s, int B, int max_pos, co
                                 max_pos, B, st));
         {   // wo: partial tiles, then residual + rms scale + the inputs of w1 and w3 in one kernel
             Q4Launch Q = launch_of(wo, B, 0.f);
-            Q.m[0] = mat_of(wo, nullptr, nullptr, nullptr);
+            Q.m[0] = gemm_mat_of(wo, nullptr);
             ResNormPrep R{};
             L2_TRY(gemm(Q, XhList{{b.h[0], nullptr, nullptr}}, nullptr, &R.KS));
             R.ws = b.ws, R.B = B, R.out = dim, R.res = b.x, R.x = b.x, R.ss = b.ss, R.eps = m->rms_eps;
@@ -1740,8 +1771,8 @@ static int forward_enqueue_gemm(l2_model *m, l2_state *s, int B, int max_pos, co
         }
         {   // w1 | w3, then the gate in w2's order
             Q4Launch Q = launch_of(w1, B, m->rms_eps);
-            Q.m[0] = mat_of(w1, nullptr, nullptr, nullptr);
-            Q.m[1] = mat_of(w3, nullptr, nullptr, nullptr);
+            Q.m[0] = gemm_mat_of(w1, nullptr);
+            Q.m[1] = gemm_mat_of(w3, nullptr);
             Q.n_mats = 2;
             SiluArgs S{};
             L2_TRY(gemm(Q, XhList{{b.h[0], dense ? b.h[0] : b.h[1], nullptr}}, nullptr, &S.KS));
@@ -1750,7 +1781,7 @@ static int forward_enqueue_gemm(l2_model *m, l2_state *s, int B, int max_pos, co
         }
         {   // w2; the kernel that adds its tiles hands the next layer its q, k and v inputs
             Q4Launch Q = launch_of(w2, B, 0.f);
-            Q.m[0] = mat_of(w2, nullptr, nullptr, b.x);
+            Q.m[0] = gemm_mat_of(w2, b.x);
             int ks = 0;
             if (l + 1 < L) {
                 L2_TRY(gemm(Q, XhList{{b.h[2], nullptr, nullptr}}, nullptr, &ks));

@@ -238,9 +238,10 @@ __device__ __forceinline__ void q4_tile(const Q4Launch &L, const XhList &xl, int
     const int n_unit = in_p / (64 * KPG);
     const int it0 = (int)((long)n_unit * ks / KS) * KPG, it1 = (int)((long)n_unit * (ks + 1) / KS) * KPG, n_it = it1 - it0;
 
+    const int row_tiles = (n_out + 31) >> 5; // of scales and zero points
     const uint32_t lds0 = lds_offset(lds), wave_at = 3 * S::kTile + wave * 3 * S::kUnit;
     const u4v xbuf = biased_buffer(xl.p[mi], (size_t)B * NP * in_p * 2), wbuf = biased_buffer(L.m[mi].qweight, (size_t)n_out * (in >> 1));
-    const u4v sbuf = biased_buffer(L.m[mi].scales, (size_t)n_out * groups * 4), zbuf = biased_buffer(L.m[mi].qzeros, (size_t)(n_out >> 3) * groups * 4);
+    const u4v sbuf = biased_buffer(L.m[mi].scales, (size_t)row_tiles * groups * 128), zbuf = biased_buffer(L.m[mi].qzeros, (size_t)row_tiles * groups * 16);
     constexpr int PIECES = NP * 2 * NT, XP = (PIECES + NW - 1) / NW; // 1 KB pieces of a tile: 8 tokens of a plane
     static_assert(XP <= 4, "the instruction's own offset has 12 bits");
     const int xfirst = min(wave * XP, PIECES - XP);
@@ -255,8 +256,9 @@ __device__ __forceinline__ void q4_tile(const Q4Launch &L, const XhList &xl, int
         const int row = i * 16 + (lane >> 2);
         woff[i] = (uint32_t)min(obase + row, n_out - 1) * (uint32_t)(in >> 1) + (((lane & 3) ^ ((row >> 2) & 3)) << 4) + kBias - i * 1024;
     }
-    const int srow = min(obase + (lane & 31), n_out - 1), lane_group = G == 128 ? 0 : lane >> 5;
-    const uint32_t soff = (uint32_t)(srow * groups) * 4u + kBias - S::kWeights, zoff = (uint32_t)((srow >> 3) * groups) * 4u + kBias - S::kWeights - S::kScales;
+    const int lane_group = G == 128 ? 0 : lane >> 5;
+    const uint32_t group0 = (uint32_t)(min(obase >> 5, row_tiles - 1) * groups);
+    const uint32_t soff = group0 * 128u + (lane & 31) * 4u + kBias - S::kWeights, zoff = group0 * 16u + (lane >> 3 & 3) * 4u + kBias - S::kWeights - S::kScales;
     uint32_t xr[2]; // where the lane reads a token's piece of MFMA k
 #pragma unroll
     for (int k = 0; k < 2; k++) xr[k] = (uint32_t)r * kStepRow + (((G == 32 ? 4 * k + kg : 2 * kg + k) ^ piece_xor(r)) << 4);
@@ -278,11 +280,11 @@ __device__ __forceinline__ void q4_tile(const Q4Launch &L, const XhList &xl, int
         if (i < 2) {
             LDS_LOAD("x4", to, i * 1024, wbuf, woff[i], w_at);
         } else { // in % 64 = 32: the last step's second group is the first one again (its inputs are zero)
-            const uint32_t g = min(w_at * 2 / G + lane_group + (i >= 4 ? 2 : 0), (uint32_t)groups - 1) * 4;
+            const uint32_t g = min(w_at * 2 / G + lane_group + (i >= 4 ? 2 : 0), (uint32_t)groups - 1) * 128, z = g >> 3;
             if (i == 2) LDS_LOAD("", to, S::kWeights, sbuf, soff + g, 0);
-            else if (i == 3) LDS_LOAD("", to, S::kWeights + S::kScales, zbuf, zoff + g, 0);
+            else if (i == 3) LDS_LOAD("", to, S::kWeights + S::kScales, zbuf, zoff + z, 0);
             else if (i == 4) LDS_LOAD("", to, S::kWeights + 256, sbuf, soff - 256 + g, 0);
-            else LDS_LOAD("", to, S::kWeights + S::kScales + 256, zbuf, zoff - 256 + g, 0);
+            else LDS_LOAD("", to, S::kWeights + S::kScales + 256, zbuf, zoff - 256 + z, 0);
         }
         if (i == WL - 1) w_at += 64;
     };
@@ -1000,6 +1002,21 @@ __global__ __launch_bounds__(1024, SL <= 2 ? 8 : 4) void gemm_silu_kernel(const 
     }
 }
 
+// A tile of 32 rows x 32 groups per block, turned through LDS.
+__global__ __launch_bounds__(256) void group_tiles_kernel(const float *scales, const int32_t *qzeros, int out, int groups, float *scales_t, int32_t *zeros_t) {
+    __shared__ float s[32][33];
+    const int tile = blockIdx.x, g0 = blockIdx.y * 32, lo = threadIdx.x & 31, hi = threadIdx.x >> 5;
+    for (int r = hi; r < 32; r += 8) {
+        const int row = tile * 32 + r;
+        s[r][lo] = row < out && g0 + lo < groups ? scales[(size_t)row * groups + g0 + lo] : 0.f;
+    }
+    __syncthreads();
+    for (int g = hi; g < 32; g += 8)
+        if (g0 + g < groups) scales_t[((size_t)tile * groups + g0 + g) * 32 + lo] = s[lo][g];
+    const int z = tile * 4 + hi; // a word of eight rows
+    if (hi < 4 && g0 + lo < groups) zeros_t[((size_t)tile * groups + g0 + lo) * 4 + hi] = z < out >> 3 ? qzeros[(size_t)z * groups + g0 + lo] : 0;
+}
+
 // ---- launchers ---------------------------------------------------------------------------------------------------
 
 template <int G, int NT, int NW>
@@ -1143,6 +1160,16 @@ int gemm_launch(Q4Launch &L, const XhList &xh, const float *ss, float *ws, size_
         hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)((rows + 1023) / 1024), L.batch), dim3(256), 0, st, L, ss, ws, s.slices);
         L2_HIP(hipGetLastError());
     }
+    return L2_OK;
+}
+
+size_t group_tiles_floats(int out, int groups) { return (size_t)((out + 31) / 32) * groups * 36; }
+
+int group_tiles_launch(const float *scales, const int32_t *qzeros, int out, int groups, float *tiles, hipStream_t st) {
+    const int row_tiles = (out + 31) / 32;
+    hipLaunchKernelGGL(group_tiles_kernel, dim3(row_tiles, (groups + 31) / 32), dim3(256), 0, st, scales, qzeros, out, groups, tiles,
+                       reinterpret_cast<int32_t *>(tiles + (size_t)row_tiles * groups * 32));
+    L2_HIP(hipGetLastError());
     return L2_OK;
 }
 

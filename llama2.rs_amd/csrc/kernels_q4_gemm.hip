@@ -115,8 +115,9 @@ __device__ __forceinline__ void q4_gemm_tile(const Q4Launch &L, const XhList &xh
     // than waves: the last ones fetch the same), as do the parts of a unit: one base each, the rest in the instructions.
     constexpr int XP = (NB * 4 + NW - 1) / NW;
     static_assert(XP <= 4, "the instruction's own offset has 12 bits");
+    const int row_tiles = (n_out + 31) >> 5; // of scales and zero points
     const u4v xbuf = biased_buffer(xh_list.p[mi], (size_t)B * in * 2), wbuf = biased_buffer(M.qweight, (size_t)n_out * (in >> 1));
-    const u4v sbuf = biased_buffer(M.scales, (size_t)n_out * groups * 4), zbuf = biased_buffer(M.qzeros, (size_t)(n_out >> 3) * groups * 4);
+    const u4v sbuf = biased_buffer(M.scales, (size_t)row_tiles * groups * 128), zbuf = biased_buffer(M.qzeros, (size_t)row_tiles * groups * 16);
     const int xfirst = min(wave * XP, NB * 4 - XP);
     uint32_t xoff[XP], woff[2], soff, zoff;
 #pragma unroll
@@ -129,9 +130,9 @@ __device__ __forceinline__ void q4_gemm_tile(const Q4Launch &L, const XhList &xh
         const int row = i * 16 + (lane >> 2);
         woff[i] = (uint32_t)min(obase + row, n_out - 1) * (uint32_t)(in >> 1) + (((lane & 3) ^ ((row >> 2) & 3)) << 4) + kBias - i * 1024;
     }
-    const int srow = min(obase + (lane & 31), n_out - 1), lane_group = G == 128 ? 0 : lane >> 5; // of two groups (G = 128: the same one again)
-    soff = ((uint32_t)(srow * groups) + lane_group) * 4u + kBias - S::kWeights;
-    zoff = ((uint32_t)((srow >> 3) * groups) + lane_group) * 4u + kBias - S::kWeights - S::kScales;
+    const uint32_t group0 = (uint32_t)(min(obase >> 5, row_tiles - 1) * groups) + (G == 128 ? 0 : lane >> 5); // two groups (G = 128: the same one again)
+    soff = group0 * 128u + (lane & 31) * 4u + kBias - S::kWeights;
+    zoff = group0 * 16u + (lane >> 3 & 3) * 4u + kBias - S::kWeights - S::kScales;
     // ... and where it reads them
     uint32_t xr[2]; // piece 2 kg + s of token r
 #pragma unroll
@@ -148,13 +149,13 @@ __device__ __forceinline__ void q4_gemm_tile(const Q4Launch &L, const XhList &xh
         if (i == XP - 1) x_at = min(x_at + 128, x_last);
     };
     auto fetch_w = [&](const uint32_t unit, const int i) __attribute__((always_inline)) { // piece i of WL
-        const uint32_t s_at = G == 128 ? w_at >> 4 : G == 64 ? w_at >> 3 : w_at >> 2;
+        const uint32_t s_at = w_at * (256 / G), z_at = s_at >> 3;
         const uint32_t to = lds0 + wave_at + unit;
         if (i < 2) LDS_LOAD("x4", to, i * 1024, wbuf, woff[i], w_at);
         else if (i == 2) LDS_LOAD("", to, S::kWeights, sbuf, soff, s_at);
-        else if (i == 3) LDS_LOAD("", to, S::kWeights + S::kScales, zbuf, zoff, s_at);
-        else if (i == 4) LDS_LOAD("", to, S::kWeights + 256, sbuf, soff - 256 + 8, s_at); // G = 32: the second step's groups
-        else LDS_LOAD("", to, S::kWeights + S::kScales + 256, zbuf, zoff - 256 + 8, s_at);
+        else if (i == 3) LDS_LOAD("", to, S::kWeights + S::kScales, zbuf, zoff, z_at);
+        else if (i == 4) LDS_LOAD("", to, S::kWeights + 256, sbuf, soff - 256 + 2 * 128, s_at); // G = 32: the second step's groups
+        else LDS_LOAD("", to, S::kWeights + S::kScales + 256, zbuf, zoff - 256 + 2 * 16, z_at);
         if (i == WL - 1) w_at = min(w_at + 64, w_last);
     };
 

@@ -61,6 +61,19 @@ def test_batch_tiles_vs_fp64(ops, n_in, n_out, G, batches):
     q.close()
 
 
+# scales and zero points in tiles of 32 rows x 32 groups: a last tile of 8 rows alone, of 24, behind a whole one, and of one group
+@pytest.mark.parametrize("n_in,n_out,G,B", [(28672, 8, 32, 300), (28672, 24, 64, 90), (28672, 40, 128, 60), (1056, 2056, 32, 32),
+                                            (4160, 520, 64, 33)])
+def test_batch_group_tiles_vs_fp64(ops, n_in, n_out, G, B):
+    rng = np.random.default_rng(n_out)
+    qw, qz, sc, gi = ck.synth_qlinear(rng, n_in, n_out, G, act_order=True)
+    x = rng.standard_normal((B, n_in)).astype(np.float32)
+    want = x.astype(np.float64) @ ck.dequant_bin(qw, qz, sc, gi, G).astype(np.float64).T
+    q = ops.QLinear(qw, qz, sc, gi, G)
+    assert nrel(q.matvec(x), want) < 1e-5
+    q.close()
+
+
 @pytest.mark.parametrize("kv,hidden,G,n", [(8, 2816, 32, 70), (4, 2848, 32, 64), (2, 2816, 64, 131), (1, 2816, 128, 97),
                                              (2, 2816, 0, 66), (8, 2848, 0, 135)])
 def test_fp32_prompt_vs_oracle(ops, oracle, kv, hidden, G, n):
