@@ -929,9 +929,11 @@ __global__ __launch_bounds__(1024, TRIPS <= 2 && TRIPS * SL <= 8 ? 8 : 4) void g
 
 // What follows the q|k|v projection of a chunk: add the partial tiles of the three matrices, apply the
 // token's rms scale, rotate q and k (src/models.rs:100-129: the second half of a head uses the first half's ROTATED
-// value), write q back and k and v into the cache rows of the tokens' positions (:236-249).  One block per token; a thread
-// takes four neighbouring pairs of a head, or four values of v.  Blocks of 512: at one slice the launch is bound by memory
-// (50 MB in 12.3 us for 511 tokens of 4096 + 2 x 4096; 14.6 with blocks of 256, eight to a token).
+// value), write q back and k and v into the cache rows of the tokens' positions (:236-249).  A thread takes four
+// neighbouring pairs of a head, or four values of v, and no more: what bounds it is latency with few tokens and memory with many
+// (50 MB at one slice and 511 tokens of 4096 + 2 x 4096), and blocks that loop over a token's row have one trip's loads in flight.
+// One block per token -> this: 4096 + 2 x 4096, 16, 64, 399, 899 tokens 6.4 / 6.8 / 8.0 / 17.4 -> 4.0 / 4.7 / 7.6 / 15.1 us, 8192 + 2 x
+// 1024, 64 and 776 tokens 7.4 / 14.0 -> 5.4 / 12.2.
 template <int SL>
 __global__ __launch_bounds__(512) void gemm_rope_kv_kernel(const RopeKvArgs A) {
     constexpr int HS = 128, HALF = 64;
@@ -946,27 +948,27 @@ __global__ __launch_bounds__(512) void gemm_rope_kv_kernel(const RopeKvArgs A) {
     const size_t sq = (size_t)A.B * dim, sk = (size_t)A.B * kv_dim;
     float *kc = A.kcache + (size_t)p * kv_dim, *vc = A.vcache + (size_t)p * kv_dim;
     const int nq = dim >> 3, nk = kv_dim >> 3, nv = kv_dim >> 2;
-    for (int idx = threadIdx.x; idx < nq + nk + nv; idx += 512) {
-        if (idx >= nq + nk) {
-            const int i = (idx - nq - nk) * 4;
-            const float4 v = sum_slices_n<SL>(wv + i, sk, A.KS);
-            store_through(reinterpret_cast<float4 *>(vc + i), make_float4(v.x * ss, v.y * ss, v.z * ss, v.w * ss));
-            continue;
-        }
-        const bool is_q = idx < nq;
-        const int j = is_q ? idx : idx - nq, i = (j & 15) * 4, at = (j >> 4) * HS + i;
-        const float4 c = *reinterpret_cast<const float4 *>(ct + i), s = *reinterpret_cast<const float4 *>(st + i);
-        const float *src = (is_q ? wq : wk) + at;
-        const size_t slice = is_q ? sq : sk;
-        float4 x = sum_slices_n<SL>(src, slice, A.KS), y = sum_slices_n<SL>(src + HALF, slice, A.KS);
-        x.x *= ss, x.y *= ss, x.z *= ss, x.w *= ss;
-        y.x *= ss, y.y *= ss, y.z *= ss, y.w *= ss;
-        const float4 f = make_float4(x.x * c.x - y.x * s.x, x.y * c.y - y.y * s.y, x.z * c.z - y.z * s.z, x.w * c.w - y.w * s.w);
-        float *dst = (is_q ? A.q + (size_t)b * dim : kc) + at;
-        store_through(reinterpret_cast<float4 *>(dst), f);
-        store_through(reinterpret_cast<float4 *>(dst + HALF),
-                      make_float4(y.x * c.x + f.x * s.x, y.y * c.y + f.y * s.y, y.z * c.z + f.z * s.z, y.w * c.w + f.w * s.w));
+    const int idx = blockIdx.y * 512 + threadIdx.x;
+    if (idx >= nq + nk + nv) return;
+    if (idx >= nq + nk) {
+        const int i = (idx - nq - nk) * 4;
+        const float4 v = sum_slices_n<SL>(wv + i, sk, A.KS);
+        store_through(reinterpret_cast<float4 *>(vc + i), make_float4(v.x * ss, v.y * ss, v.z * ss, v.w * ss));
+        return;
     }
+    const bool is_q = idx < nq;
+    const int j = is_q ? idx : idx - nq, i = (j & 15) * 4, at = (j >> 4) * HS + i;
+    const float4 c = *reinterpret_cast<const float4 *>(ct + i), s = *reinterpret_cast<const float4 *>(st + i);
+    const float *src = (is_q ? wq : wk) + at;
+    const size_t slice = is_q ? sq : sk;
+    float4 x = sum_slices_n<SL>(src, slice, A.KS), y = sum_slices_n<SL>(src + HALF, slice, A.KS);
+    x.x *= ss, x.y *= ss, x.z *= ss, x.w *= ss;
+    y.x *= ss, y.y *= ss, y.z *= ss, y.w *= ss;
+    const float4 f = make_float4(x.x * c.x - y.x * s.x, x.y * c.y - y.y * s.y, x.z * c.z - y.z * s.z, x.w * c.w - y.w * s.w);
+    float *dst = (is_q ? A.q + (size_t)b * dim : kc) + at;
+    store_through(reinterpret_cast<float4 *>(dst), f);
+    store_through(reinterpret_cast<float4 *>(dst + HALF),
+                  make_float4(y.x * c.x + f.x * s.x, y.y * c.y + f.y * s.y, y.z * c.z + f.z * s.z, y.w * c.w + f.w * s.w));
 }
 
 // The SiLU gate (src/models.rs:92-98) behind w1|w3 of a chunk: add the partial tiles of both, apply the token's rms
@@ -1237,7 +1239,7 @@ int gemm_residual_norm_launch(const ResNormPrep &A, int planes, hipStream_t st) 
 int gemm_rope_kv_launch(const RopeKvArgs &A, hipStream_t st) {
     if (A.KS < 1 || A.KS > kMaxGemmSlices || A.B < 1 || A.n_heads < A.n_kv_heads)
         return l2_fail(L2_ERR_ARG, "q|k|v epilogue: %d slices, %d tokens", A.KS, A.B);
-    const dim3 grid(A.B), block(512);
+    const dim3 grid(A.B, (A.n_heads * 16 + A.n_kv_heads * 48 + 511) / 512), block(512); // a thread per eight of q and k, four of v
     if (A.KS <= 2) hipLaunchKernelGGL(gemm_rope_kv_kernel<2>, grid, block, 0, st, A);
     else if (A.KS <= 8) hipLaunchKernelGGL(gemm_rope_kv_kernel<8>, grid, block, 0, st, A);
     else hipLaunchKernelGGL(gemm_rope_kv_kernel<kMaxGemmSlices>, grid, block, 0, st, A);
