@@ -908,6 +908,15 @@ void attn_prefill_mfma16_kernel(void *__restrict__ out, const float *__restrict_
     }
     fetch_k(wave);
     fetch_v(wave);
+    // Where this thread's outputs go, asked for here and not when they are there: output u of a set is of head j % QG (see the
+    // merge), which recurs.  7B, 16 / 64 / 128 tokens 6.6 / 7.8 / 9.7 -> 6.2 / 7.0 / 9.3 us, three planes and 64 tokens 10.1 -> 8.9.
+    constexpr int PER = NT / HS, HEADS = QG > PER ? QG / PER : 1;
+    int dst[HEADS];
+#pragma unroll
+    for (int u = 0; u < HEADS; u++) {
+        const int i = (kvh * QG + (tid / HS + u * PER) % QG) * HS + tid % HS;
+        dst[u] = scatter ? scatter[i] : i;
+    }
     __builtin_amdgcn_sched_barrier(0);
     int t_end = my_pos[0] + 1; // the block's tiles end with the last row any of its columns sees
 #pragma unroll
@@ -1037,13 +1046,12 @@ void attn_prefill_mfma16_kernel(void *__restrict__ out, const float *__restrict_
                 de = fmaf(e, comb[w][j][HS + 1], de);
             }
             if (qi < B) {
-                const int i = (kvh * QG + j % QG) * HS + d;
-                const int dst = scatter ? scatter[i] : i;
+                const int to = dst[u % HEADS];
                 const float v = nu / de;
                 if constexpr (NP == 1) {
-                    reinterpret_cast<_Float16 *>(out)[(size_t)qi * dim + h16_slot(dst)] = (_Float16)v;
+                    reinterpret_cast<_Float16 *>(out)[(size_t)qi * dim + h16_slot(to)] = (_Float16)v;
                 } else { // three bf16 numbers that add up to v exactly
-                    uint16_t *o = reinterpret_cast<uint16_t *>(out) + (size_t)qi * NP * dim + b16_slot(dst);
+                    uint16_t *o = reinterpret_cast<uint16_t *>(out) + (size_t)qi * NP * dim + b16_slot(to);
                     float left = v;
 #pragma unroll
                     for (int p = 0; p < NP; p++) {
