@@ -154,6 +154,15 @@ __global__ __launch_bounds__(NWV * 64) void attn_decode_kernel(const AttnDecode 
     const float nk_a = A.k_new[(size_t)kvh * HS + hd], nk_b = A.k_new[(size_t)kvh * HS + hd + HALF];
     const float nv = A.v_new[(size_t)kvh * HS + (tid & 127)];
     const float nc = ct[hd], ns = st[hd];
+    // Sliced, a thread has one output at most: where it goes is asked for here, not when it is there.
+    constexpr bool kOneOut = DS > 1 && QG * VD <= NT;
+    int out_i = 0;
+    if constexpr (kOneOut) {
+        const int o = tid % (QG * VD);
+        out_i = (kvh * QG + o / VD) * HS + slice * VD + o % VD;
+        const int32_t at = *((A.scatter ? A.scatter : reinterpret_cast<const int32_t *>(A.q)) + out_i);
+        out_i = A.scatter ? at : out_i;
+    }
     __builtin_amdgcn_sched_barrier(0);
 
     Step pipe[PD];
@@ -384,7 +393,7 @@ __global__ __launch_bounds__(NWV * 64) void attn_decode_kernel(const AttnDecode 
         const int h = kvh * QG + j;
         if (A.n_splits == 1) {
             const int i = h * HS + dv;
-            A.out[A.scatter ? A.scatter[i] : i] = num / den;
+            A.out[kOneOut ? out_i : A.scatter ? A.scatter[i] : i] = num / den;
         } else {
             float *p = A.part + ((size_t)h * A.max_splits + sp) * (HS + 2);
             p[dv] = num;

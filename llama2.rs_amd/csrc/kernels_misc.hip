@@ -68,6 +68,10 @@ __global__ void embed_kernel(float *x, const float *emb, const TokenSource src_,
     const int b = blockIdx.y;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     int32_t token = src_.token;
+    int32_t to[3] = {0, 0, 0}; // asked for before the token is known, and all at once
+#pragma unroll
+    for (int c = 0; c < 3; c++)
+        if (c < t.n && i < dim) to[c] = t.inv[c][i];
     if (src_.tokens)
         token = src_.tokens[b];
     else if (src_.prev) { // src/inference.rs:160-162, 185-189: the argmax of the step before is this step's token
@@ -78,7 +82,9 @@ __global__ void embed_kernel(float *x, const float *emb, const TokenSource src_,
     if (i < dim) {
         const float v = src[i];
         x[(size_t)b * dim + i] = v;
-        for (int c = 0; c < t.n; c++) t.out[c][(size_t)b * dim + t.inv[c][i]] = v;
+#pragma unroll
+        for (int c = 0; c < 3; c++)
+            if (c < t.n) t.out[c][(size_t)b * dim + to[c]] = v;
     }
     if (amax && b == 0 && i == 0) amax[0] = 0ull;
 }
