@@ -61,6 +61,18 @@ def test_batch_tiles_vs_fp64(ops, n_in, n_out, G, batches):
     q.close()
 
 
+# a last round of tiles in halves: 291 tiles of 256 rows x 64 columns, of the last ones the second half empty, of 17 columns, whole
+@pytest.mark.parametrize("B", [150, 177, 192])
+def test_batch_halves_vs_fp64(ops, B):
+    rng = np.random.default_rng(B)
+    qw, qz, sc, gi = ck.synth_qlinear(rng, 256, 24584, 64, act_order=True)
+    x = rng.standard_normal((B, 256)).astype(np.float32)
+    q = ops.QLinear(qw, qz, sc, gi, 64)
+    got = q.matvec(x)
+    assert nrel(got, x.astype(np.float64) @ ck.dequant_bin(qw, qz, sc, gi, 64).astype(np.float64).T) < 1e-5
+    q.close()
+
+
 # scales and zero points in tiles of 32 rows x 32 groups: a last tile of 8 rows alone, of 24, behind a whole one, and of one group
 @pytest.mark.parametrize("n_in,n_out,G,B", [(28672, 8, 32, 300), (28672, 24, 64, 90), (28672, 40, 128, 60), (1056, 2056, 32, 32),
                                             (4160, 520, 64, 33)])
