@@ -378,11 +378,14 @@ int launch_gemm(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const
     for (int i = 0; i < L.n_mats; i++) row_blocks += L.m[i].row_blocks = (L.m[i].out + 32 * NW - 1) / (32 * NW);
     const int rest = L.batch % TN, t_full = L.batch / TN + (rest > TN / 2), narrow = rest > 0 && rest <= TN / 2;
     const int tiles = row_blocks * t_full * s.slices;
-    int whole = tiles;
-    // halves where they and the narrow tiles fit one round: 7B's w1|w3, 511 tokens, 344 tiles on 256 CUs 123 -> 112 us; with
+    // Halves where they and the narrow tiles fit one round: 7B's w1|w3, 511 tokens, 344 tiles on 256 CUs 123 -> 112 us; with
     // 224 narrow tiles behind 64 left over (70B's, 776) they take 822 and whole tiles 804.  With several slices too: four layers of
-    // 13B, group 64, 399 tokens 2192 -> 2135, six of 7B, group 32, 249 tokens 1656 -> 1610
-    if (NB == 4 && 2 * (tiles % cu_count()) + narrow * row_blocks * s.slices <= cu_count()) whole = tiles / cu_count() * cu_count();
+    // 13B, group 64, 399 tokens 2192 -> 2135, six of 7B, group 32, 249 tokens 1656 -> 1610.  Of the blocks of four waves too, where
+    // some CUs have two and others one (two take twice as long as one): six layers of 7B, 64, 99, 128 tokens 918 / 1075 / 1120 ->
+    // 903 / 1047 / 1080, four of 13B, 128 1057 -> 1041; with more of them than two per CU whole tiles (70B, 179 1965 against 1978).
+    const int cus = cu_count(), left = tiles % cus;
+    const bool last_round = NB == 4 || (NB == 2 && tiles > cus && tiles < 2 * cus);
+    const int whole = last_round && 2 * left + narrow * row_blocks * s.slices <= cus ? tiles - left : tiles;
     // partial tiles past the caches where they would fill them: what a launch leaves dirty there is written back at its end
     // (7B, 511 tokens: the four launches 13 us less per layer, their consumers 5 more; below 16 MB the other way round: there they
     // go past the L2 but not past the memory-side cache, see store_through)
