@@ -833,31 +833,24 @@ __device__ __forceinline__ float4 sum_slices(const float *p, size_t slice, int K
     return sum_slices_n<kMaxGemmSlices>(p, slice, KS);
 }
 
-// Adds the partial tiles of a launch with several K slices and runs the epilogue (store or residual add); a thread owns
-// four consecutive outputs of one token.  grid: (ceil(sum_out / 1024), B); the matrices are laid end to end.
-__global__ __launch_bounds__(256) void gemm_reduce_kernel(const Q4Launch L, const float *__restrict__ ss,
-                                                          const float *__restrict__ ws, int KS) {
-    const int t = blockIdx.y, B = L.batch;
-    int o = (blockIdx.x * 256 + threadIdx.x) * 4, mi = 0;
-    size_t ws_base = 0;
-    while (mi + 1 < L.n_mats && o >= L.m[mi].out) {
-        o -= L.m[mi].out;
-        ws_base += (size_t)KS * B * L.m[mi].out;
-        mi++;
-    }
-    const Q4Mat &M = L.m[mi];
-    if (o >= M.out) return;
-    const size_t at = (size_t)t * M.out + o;
-    float4 v = sum_slices(ws + ws_base + at, (size_t)B * M.out, KS);
+// Adds the partial tiles of a launch of one matrix with several K slices and runs the epilogue (store or residual add); a thread
+// owns four consecutive outputs of one token.  grid: (ceil(out / 1024), B).  With a launch's description for several matrices as
+// its argument, read field by field, it was 0.4 to 0.9 us longer (8192x1024, 100 columns 20.8 -> 19.9 us for the call).
+__global__ __launch_bounds__(256) void gemm_reduce_kernel(float *y, const float *ws, const float *res, const float *ss, int out, int B, int KS) {
+    asm volatile("" ::"s"(y), "s"(ws), "s"(res), "s"(ss), "s"(out), "s"(B), "s"(KS)); // at once
+    const int t = blockIdx.y, o = (blockIdx.x * 256 + threadIdx.x) * 4;
+    if (o >= out) return;
+    const size_t at = (size_t)t * out + o;
+    float4 v = sum_slices(ws + at, (size_t)B * out, KS);
     if (ss) {
         const float sc = ss[t];
         v.x *= sc, v.y *= sc, v.z *= sc, v.w *= sc;
     }
-    if (L.e.kind == Q4_EPI_RESIDUAL) {
-        const float4 r = *reinterpret_cast<const float4 *>(L.e.res + at);
+    if (res) {
+        const float4 r = *reinterpret_cast<const float4 *>(res + at);
         v.x += r.x, v.y += r.y, v.z += r.z, v.w += r.w;
     }
-    *reinterpret_cast<float4_any *>(M.y + at) = float4_any{v.x, v.y, v.z, v.w};
+    *reinterpret_cast<float4_any *>(y + at) = float4_any{v.x, v.y, v.z, v.w};
 }
 
 // What follows a residual projection (wo, w2) of a chunk: add the partial tiles and the residual (src/models.rs:263-264,
@@ -1163,6 +1156,7 @@ int gemm_launch(Q4Launch &L, const XhList &xh, const float *ss, float *ws, size_
     }
     const GemmShape s = gemm_shape(L, slice_batch, planes);
     const bool partials = ks_out;
+    if (!partials && L.n_mats != 1) return l2_fail(L2_ERR_ARG, "q4 gemm: %d matrices without a consumer of their partial tiles", L.n_mats);
     if ((s.slices > 1 || partials) && (size_t)s.slices * L.batch * rows > ws_floats)
         return l2_fail(L2_ERR_ARG, "q4 gemm: %d slices of %d x %ld in a workspace of %zu", s.slices, L.batch, rows, ws_floats);
     if (planes == 1)
@@ -1173,8 +1167,9 @@ int gemm_launch(Q4Launch &L, const XhList &xh, const float *ss, float *ws, size_
         *ks_out = s.slices;
         return L2_OK;
     }
-    if (s.slices > 1 || partials) {
-        hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)((rows + 1023) / 1024), L.batch), dim3(256), 0, st, L, ss, ws, s.slices);
+    if (s.slices > 1) {
+        hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)((rows + 1023) / 1024), L.batch), dim3(256), 0, st, L.m[0].y, ws,
+                           L.e.kind == Q4_EPI_RESIDUAL ? L.e.res : nullptr, ss, L.m[0].out, L.batch, s.slices);
         L2_HIP(hipGetLastError());
     }
     return L2_OK;
