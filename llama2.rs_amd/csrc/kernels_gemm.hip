@@ -481,24 +481,23 @@ __device__ __forceinline__ void q4_tile(const Q4Launch &L, const XhList &xl, int
     }
 }
 
-// The first `whole` blocks take a tile each, the others half of one of the tiles that are left.  The last tile of tokens takes 16,
-// 32 or 48 where that is enough (48 against 64: six layers of 7B, 33 and 48 tokens 1114 / 1131 -> 1046 / 1066 us, 299 2743 -> 2685, three
-// of 70B, 44 1531 -> 1397; 13824x5120, 40 columns 36.4 -> 32.6).
+// The first `whole` blocks take the tiles of as many row blocks (and slices) as they are, the others tiles of `width` columns of the
+// row blocks that are left.  The last tile of tokens takes 16, 32 or 48 where that is enough (48 against 64: six layers of 7B, 33 and
+// 48 tokens 1114 / 1131 -> 1046 / 1066 us, 299 2743 -> 2685, three of 70B, 44 1531 -> 1397; 13824x5120, 40 columns 36.4 -> 32.6).
 template <int G, int NT, int NW>
 __global__ __launch_bounds__(64 * NW, NT == 1 ? 3 : 2) void q4_tile_gemm_kernel(const Q4Launch L, const XhList xl, int in_p,
                                                               const float *__restrict__ ss, float *__restrict__ ws, int KS,
-                                                              int t_tiles, int row_blocks, int whole, int partials) {
+                                                              int t_tiles, int row_blocks, int whole, int width, int partials) {
     // an XCD gets all token tiles of a row block one behind the other: what runs on it at one time shares weights and tiles
-    int work, half = -1;
+    int rb, t0, n;
     if (NT < 4 || (int)blockIdx.x < whole) {
-        work = xcd_item(blockIdx.x, whole);
+        const int work = xcd_item(blockIdx.x, whole);
+        rb = work / t_tiles, t0 = (work - rb * t_tiles) * 16 * NT, n = L.batch - t0;
     } else {
-        work = xcd_item(blockIdx.x - whole, gridDim.x - whole);
-        half = work & 1, work = whole + (work >> 1);
+        const int work = xcd_item(blockIdx.x - whole, gridDim.x - whole), per = (L.batch + width - 1) / width;
+        rb = work / per, t0 = (work - rb * per) * width, n = min(L.batch - t0, width);
+        rb += whole / t_tiles;
     }
-    int rb = work / t_tiles;
-    const int t0 = (work - rb * t_tiles) * 16 * NT + (half > 0 ? 8 * NT : 0), n = half < 0 ? L.batch - t0 : min(L.batch - t0, 8 * NT);
-    if (n <= 0) return; // the second half of a narrow tile
     const int ks = rb / row_blocks;
     rb -= ks * row_blocks;
     if (NT > 1 && n <= 16) q4_tile<G, 1, NW>(L, xl, in_p, ss, ws, KS, partials, rb, ks, t0);
@@ -1037,13 +1036,19 @@ template <int G, int NT, int NW>
 int launch_tile(const Q4Launch &L, const XhList &xh, const float *ss, float *ws, int KS, int partials, int total, hipStream_t st) {
     size_t lds = 0;
     L2_TRY((ready_tile<G, NT, NW>(&lds)));
-    const int t_tiles = (L.batch + 16 * NT - 1) / (16 * NT), tiles = total * t_tiles * KS, left = tiles % cu_count();
-    // One block per CU: the tiles of a last round that is less than half full go in halves, a half in some 0.7 of a tile's time.  Six
-    // layers of 7B, 169, 250, 439 tokens 2239 / 2470 / 3871 -> 2120 / 2357 / 3635 us, four of 13B, 149 1964 -> 1881.
-    const bool halves = NT == 4 && tiles > cu_count() && 2 * left <= cu_count();
-    const int whole = halves ? tiles - left : tiles;
-    hipLaunchKernelGGL((q4_tile_gemm_kernel<G, NT, NW>), dim3(whole + 2 * (tiles - whole)), dim3(64 * NW), lds, st, L, xh, gemm_padded(L.in), ss, ws, KS,
-                       t_tiles, total, whole, partials);
+    const int t_tiles = (L.batch + 16 * NT - 1) / (16 * NT), tiles = total * t_tiles * KS, cus = cu_count();
+    // One block per CU: the row blocks that whole rounds of tiles leave over go in tiles of 32 columns, or of 48, where that is one
+    // round of blocks, in some 0.7 or 0.85 of a whole one's time.  Six layers of 7B, 32: 169, 250, 439 tokens 2239 / 2470 / 3871 ->
+    // 2120 / 2357 / 3635 us, four of 13B, 149 1964 -> 1881; 48: 299 and 511 tokens of 7B 2668 / 3971 -> 2632 /
+    // 3934, 179 of 70B 3251 -> 3196; 4096x11008, group 32, 130 columns 68.3 -> 58.7.
+    int whole = tiles, width = 16 * NT, blocks = tiles;
+    if (NT == 4 && tiles > cus && tiles % cus) {
+        const int units = tiles / cus * cus / t_tiles, left = total * KS - units;
+        for (const int w : {48, 32})
+            if (left * ((L.batch + w - 1) / w) <= cus) whole = units * t_tiles, width = w, blocks = whole + left * ((L.batch + w - 1) / w);
+    }
+    hipLaunchKernelGGL((q4_tile_gemm_kernel<G, NT, NW>), dim3(blocks), dim3(64 * NW), lds, st, L, xh, gemm_padded(L.in), ss, ws, KS, t_tiles, total, whole,
+                       width, partials);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }

@@ -61,11 +61,12 @@ def test_batch_tiles_vs_fp64(ops, n_in, n_out, G, batches):
     q.close()
 
 
-# a last round of tiles in halves: 291 tiles of 256 rows x 64 columns, of the last ones the second half empty, of 17 columns, whole
-@pytest.mark.parametrize("B", [150, 177, 192])
-def test_batch_halves_vs_fp64(ops, B):
+# the row blocks of a last round in narrower tiles: 97 row blocks, 12 of them in tiles of 32 columns (their last of 22, 17 and 32), 86,
+# 35 of them in tiles of 48 (their last of 18 and 12)
+@pytest.mark.parametrize("n_out,B", [(24584, 150), (24584, 177), (24584, 192), (22008, 258), (22008, 300)])
+def test_batch_last_round_vs_fp64(ops, n_out, B):
     rng = np.random.default_rng(B)
-    qw, qz, sc, gi = ck.synth_qlinear(rng, 256, 24584, 64, act_order=True)
+    qw, qz, sc, gi = ck.synth_qlinear(rng, 256, n_out, 64, act_order=True)
     x = rng.standard_normal((B, 256)).astype(np.float32)
     q = ops.QLinear(qw, qz, sc, gi, 64)
     got = q.matvec(x)
