@@ -333,34 +333,30 @@ __device__ __forceinline__ void q4_gemm_tile(const Q4Launch &L, const XhList &xh
     }
 }
 
-// One block per work item.  The first `whole` items are tiles of 32 NB tokens, K slice by K slice; the tiles of a last,
-// partly filled round of blocks follow in two halves; then the last tokens of every row block, where they need no more than
-// half a tile.  A tile costs its width in steps of 32 and the dequantisation of its weights (128, 64, 32 tokens of 70B's w1:
-// 119, 75, 62 us).
+// One block per work item.  A unit is a row block and a slice of K.  The first `units` of them go in tiles of 32 NB tokens; those that
+// whole rounds of blocks leave over in tiles of `width`; then come the last tokens of the first ones, where they need no more than
+// half a tile.  A tile costs its width in steps of 32 and the dequantisation of its weights (128, 64, 32 tokens of 70B's w1: 119, 75,
+// 62 us).
 template <int G, int NB, int NW>
 __global__ __launch_bounds__(64 * NW, NB > 2 ? 2 : 1) void q4_gemm_kernel(const Q4Launch L, const XhList xh, const float *__restrict__ ss,
-                                                      float *__restrict__ ws, int KS, int partials, int row_blocks, int t_full, int whole) {
+                                                      float *__restrict__ ws, int KS, int partials, int row_blocks, int t_full, int units, int width) {
     constexpr int TN = 32 * NB, CHUNK = 8;
-    const int tiles = row_blocks * t_full;
-    int item, half = -1, ks, rb, tt;
-    if ((int)blockIdx.x < whole) {
-        item = xcd_item(blockIdx.x, whole);
+    const int whole = units * t_full, per = (L.batch + width - 1) / width, other = (row_blocks * KS - units) * per, b = blockIdx.x;
+    int unit, t0, n;
+    if (b < whole) { // 8 row blocks at a time, token tile by token tile: what runs on an XCD shares tiles and weights
+        int item = xcd_item(b, whole);
+        const int first = item / (row_blocks * t_full) * row_blocks, c = (item -= first * t_full) / (CHUNK * t_full);
+        const int of = min(CHUNK, min(row_blocks, units - first) - c * CHUNK), at = item - c * CHUNK * t_full, tt = at / of;
+        unit = first + c * CHUNK + at - tt * of, t0 = tt * TN, n = L.batch - t0;
+    } else if (b < whole + other) {
+        const int item = xcd_item(b - whole, other);
+        const int left = row_blocks * KS - units, c = item / (CHUNK * per), of = min(CHUNK, left - c * CHUNK);
+        const int at = item - c * CHUNK * per, tt = at / of;
+        unit = units + c * CHUNK + at - tt * of, t0 = tt * width, n = min(L.batch - t0, width);
     } else {
-        const int halves = 2 * (tiles * KS - whole);
-        item = xcd_item(blockIdx.x - whole, gridDim.x - whole);
-        if (item < halves) half = item & 1, item = whole + (item >> 1);
-        else item += tiles * KS - halves;
+        unit = xcd_item(b - whole - other, gridDim.x - whole - other), t0 = t_full * TN, n = L.batch - t0;
     }
-    if (item < tiles * KS) { // 8 row blocks at a time, token tile by token tile: what runs on an XCD shares tiles and weights
-        ks = item / tiles, item -= ks * tiles;
-        const int c = item / (CHUNK * t_full), n = min(CHUNK, row_blocks - c * CHUNK);
-        item -= c * CHUNK * t_full;
-        tt = item / n, rb = c * CHUNK + item - tt * n;
-    } else {
-        item -= tiles * KS;
-        ks = item / row_blocks, rb = item - ks * row_blocks, tt = t_full;
-    }
-    const int t0 = tt * TN + (half > 0 ? TN / 2 : 0), n = half < 0 ? L.batch - t0 : min(L.batch - t0, TN / 2);
+    const int ks = unit / row_blocks, rb = unit - ks * row_blocks;
     if (NB > 1 && n <= 32)
         q4_gemm_tile<G, 1, NW>(L, xh, ss, ws, KS, partials, rb, ks, t0);
     else if (NB > 2 && n <= 64)
@@ -377,27 +373,33 @@ int launch_gemm(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const
     int row_blocks = 0;
     for (int i = 0; i < L.n_mats; i++) row_blocks += L.m[i].row_blocks = (L.m[i].out + 32 * NW - 1) / (32 * NW);
     const int rest = L.batch % TN, t_full = L.batch / TN + (rest > TN / 2), narrow = rest > 0 && rest <= TN / 2;
-    const int tiles = row_blocks * t_full * s.slices;
-    // Halves where they and the narrow tiles fit one round: 7B's w1|w3, 511 tokens, 344 tiles on 256 CUs 123 -> 112 us; with
-    // 224 narrow tiles behind 64 left over (70B's, 776) they take 822 and whole tiles 804.  With several slices too: four layers of
-    // 13B, group 64, 399 tokens 2192 -> 2135, six of 7B, group 32, 249 tokens 1656 -> 1610.  Of the blocks of four waves too, where
-    // some CUs have two and others one (two take twice as long as one): six layers of 7B, 64, 99, 128 tokens 918 / 1075 / 1120 ->
-    // 903 / 1047 / 1080, four of 13B, 128 1057 -> 1041; with more of them than two per CU whole tiles (70B, 179 1965 against 1978).
-    const int cus = cu_count(), left = tiles % cus;
-    const bool last_round = NB == 4 || (NB == 2 && tiles > cus && tiles < 2 * cus);
-    const int whole = last_round && 2 * left + narrow * row_blocks * s.slices <= cus ? tiles - left : tiles;
+    // The units that whole rounds leave over go in narrower tiles where these, and what is left of the others' tokens, fit one round:
+    // 7B's w1|w3, 511 tokens, 344 tiles on 256 CUs 123 -> 112 us; with 224 narrow tiles behind 64 left over (70B's, 776) they take 822
+    // and whole tiles 804.  With several slices too: four layers of 13B, group 64, 399 tokens 2192 -> 2135, six of 7B, group 32, 249
+    // tokens 1656 -> 1610.  Of the blocks of four waves too, where some CUs have two and others one (two take twice as long as one):
+    // six layers of 7B, 64, 99, 128 tokens 918 / 1075 / 1120 -> 903 / 1047 / 1080, four of 13B, 128 1057 -> 1041; with more of them than
+    // two per CU whole tiles (70B, 179 1965 against 1978).  Tiles of 96 where those of 64 are more than a round, six layers of 7B: 287,
+    // 349, 599 tokens 1702 / 1889 / 2469 -> 1670 / 1835 / 2450; four of 13B, 199, 299 1311 / 1716 -> 1291 / 1687.  Where both fit those
+    // of 64: 349 of 7B 1835 against 1886.
+    const int all = row_blocks * s.slices, tiles = all * t_full, cus = cu_count();
+    int units = all, width = TN;
+    if ((NB == 4 || (NB == 2 && tiles > cus && tiles < 2 * cus)) && tiles % cus) {
+        const int first = tiles / cus * cus / t_full;
+        for (const int w : {TN / 4 * 3, TN / 2})
+            if ((w % 32 == 0) && (all - first) * ((L.batch + w - 1) / w) + narrow * first <= cus) units = first, width = w;
+    }
     // partial tiles past the caches where they would fill them: what a launch leaves dirty there is written back at its end
     // (7B, 511 tokens: the four launches 13 us less per layer, their consumers 5 more; below 16 MB the other way round: there they
     // go past the L2 but not past the memory-side cache, see store_through)
     size_t bytes = 0;
     for (int i = 0; i < L.n_mats; i++) bytes += (size_t)s.slices * L.batch * L.m[i].out * 4;
     if (partials && bytes > ((size_t)16 << 20)) partials = 2;
-    const dim3 grid(whole + 2 * (tiles - whole) + narrow * row_blocks * s.slices), block(64 * NW);
+    const dim3 grid(units * t_full + (all - units) * ((L.batch + width - 1) / width) + narrow * units), block(64 * NW);
     // the tiles, or the output staging tiles of the epilogue (32 x 36 floats per wave)
     const size_t lds = std::max(GemmLds<G, NW>::size(TN), (size_t)NW * 32 * 36 * sizeof(float));
     static LdsLimit limit(48 * 1024);
     L2_TRY(limit.ensure(reinterpret_cast<const void *>(q4_gemm_kernel<G, NB, NW>), lds));
-    hipLaunchKernelGGL((q4_gemm_kernel<G, NB, NW>), grid, block, lds, st, L, xh, ss, ws, s.slices, partials, row_blocks, t_full, whole);
+    hipLaunchKernelGGL((q4_gemm_kernel<G, NB, NW>), grid, block, lds, st, L, xh, ss, ws, s.slices, partials, row_blocks, t_full, units, width);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }

@@ -343,6 +343,24 @@ def test_fp16_operator_wide_blocks(ops, dim, hidden, G, batches):
     m.close()
 
 
+# the row blocks that whole rounds leave over, in tiles of 64 (300, 350 rows) and of 96 (520, 590): first and last tiles that are
+# not full, a last row block that is not full, whole tiles that end inside eight row blocks
+@pytest.mark.parametrize("B", [300, 350, 520, 590])
+def test_fp16_operator_last_round(ops, B):
+    from llama2_rs import _lib
+    dims = ck.Dims(dim=256, hidden_dim=21888, n_layers=1, n_heads=2, n_kv_heads=2, vocab_size=64, seq_len=1024, group_size=64)
+    m = ops.Model(ck.synth_weights_image(dims, seed=11), dims)
+    x = np.random.default_rng(B).standard_normal((B, 256)).astype(np.float16).astype(np.float32) # as above: only fp32 sums round
+    m.set_prefill_mode(_lib.PREFILL_FP32)
+    want = m.qmatvec(0, _lib.W1, x)
+    m.set_prefill_mode(_lib.PREFILL_MFMA)
+    got = m.qmatvec(0, _lib.W1, x)
+    m.close()
+    assert not np.array_equal(got, want)
+    for b in range(B):
+        assert nrel(got[b], want[b]) < 2e-5, b
+
+
 # prompt attention with two sets of columns per block (two blocks per compute unit and more), the last block with one
 # set, and grids of one to two blocks per unit, whose tiles go in pairs, against passes too short for either
 @pytest.mark.parametrize("n_heads,n_kv,n", [(32, 32, 505), (16, 2, 1021), (32, 32, 200), (32, 32, 250), (16, 16, 300)])
