@@ -17,8 +17,8 @@
 // inputs 0.45 to 0.74, inputs all of one sign, where the matvec is better than elsewhere, 0.39 to 1.06 (1024 inputs, group 128).
 //
 // Against the matvec kernels run once per column, which read and dequantise the weights for each of them: 4096x11008,
-// group 32, 61 columns 330 -> 35.0 us with everything around it.  Against the form before this one (activations and weights
-// through registers, 32x32x16 tiles, two blocks of four waves per CU): that call 40.3 us; 16 columns of 13824x5120 33.7 -> 26.3;
+// group 32, 61 columns 330 -> 30.2 us with everything around it.  Against the form before this one (activations and weights
+// through registers, 32x32x16 tiles, two blocks of four waves per CU): that call 40.3 us; 16 columns of 13824x5120 33.7 -> 22.6;
 // two layers of 7B, group 128, 16, 64, 299 columns 280 / 365 / 967 -> 222 / 328 / 930; 70B, group 64, 16 and 299 763 / 3593 ->
 // 544 / 3350.
 #include <algorithm>
@@ -212,7 +212,7 @@ struct TileLds {
 // (kernels_q4_gemm.hip, which explains the layout and the waits): tiles of 64 k two steps ahead, weights two units.  One
 // barrier per step; a step is 6 NT pairs of MFMAs, with the dequantisation of the next one's weights and the folds of finished
 // groups spread between them: some 230 instructions for 64 tokens, which the two waves of a SIMD issue at one per 4.9 cycles
-// (2546 cycles per step of 7B's w1|w3 at 299 tokens, 1536 of them MFMAs).  Eight waves and 64 tokens take 133 KB of LDS, one
+// (2546 cycles per step of 7B's w1|w3 at 299 tokens before the scales and zero points came in tiles, 1536 of them MFMAs).  Eight waves and 64 tokens take 133 KB of LDS, one
 // block per CU; four waves and 16 or 32 tokens, where weights are what is read, two or three.
 //
 // Lane (r = l % 16, kg = l / 16).  G >= 64: the lane's words of a step are 2 kg and 2 kg + 1, MFMA k takes one each.  G = 32: an

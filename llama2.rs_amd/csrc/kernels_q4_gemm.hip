@@ -14,11 +14,13 @@
 //
 // Memory.  Everything the K loop reads comes through LDS without touching a register (buffer_load ... lds): the activation
 // tiles [tokens][64 k], which the block shares, and, for each wave alone, the packed weights, scales and zero points of its
-// rows in units of 128 k.  Tiles are requested one unit ahead, weights two; the only waits are one vmcnt per kind and unit
+// rows in units of 128 k (the latter two out of tiles of 32 rows, 144 bytes in two cache lines instead of 36: 64 tokens on six
+// layers of 7B 986 -> 938 us).  Tiles are requested one unit ahead, weights two; the only waits are one vmcnt per kind and unit
 // and ONE block barrier per unit.  16-byte pieces of a token (a row of weights) lie in the tile permuted by its number, so
 // that the reads of 16 lanes meet 16 different banks; the lanes of the load permute their addresses accordingly.
 //
-// What bounds it, and what the layout of the loop answers (70B's w1|w3, 776 tokens: 928 -> 804 us; 7B's at 511: 116 -> 107):
+// What bounds it, and what the layout of the loop answers (70B's w1|w3, 776 tokens: 928 -> 804 us, 7B's at 511 116 -> 107,
+// before the scales and zero points came in tiles):
 //   - A SIMD issues an instruction every 4 to 5 cycles from its two waves, and one wave alone gets half of that.  So the
 //     vector work (dequantisation of the next step, fold of the group before) stands evenly between the MFMAs of both halves
 //     of a step, operands are read from LDS four pairs of MFMAs ahead, and a wave's priority falls with its progress since
