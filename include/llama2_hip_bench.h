@@ -79,6 +79,11 @@ int l2_model_q4_kernels(l2_model *m, char *out, size_t cap);
 int l2_q4_plan(int in, const int32_t *out, int n_mats, int group_size, int pair, int norm, char *kernel, size_t cap,
                int32_t *geometry);
 
+/* The same for `batch` columns of one matrix as l2_qlinear_matvec and l2_qlinear_matvec_device run them through the
+ * matvec kernels: natural != 0 with x in its natural order, permuted by the kernel (inputs that it cannot permute are
+ * refused), 0 with x permuted in front. */
+int l2_qlinear_plan(int in, int out, int group_size, int batch, int natural, char *kernel, size_t cap, int32_t *geometry);
+
 /* Plain device-to-device copy of nbytes, iters times: the box's achievable
  * copy bandwidth (bytes moved = 2*nbytes per iteration). */
 int l2_copy_bench(size_t nbytes, int iters, float *ms_total);

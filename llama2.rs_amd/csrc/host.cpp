@@ -2359,12 +2359,33 @@ extern "C" int l2_model_q4_kernels(l2_model *m, char *out, size_t cap) {
     return L2_OK;
 }
 
+// What the q4 launcher would do for L: nothing is launched, only null / non-null pointers matter.
+static int plan_of(Q4Launch &L, char *kernel, size_t cap, int32_t *geometry) {
+    kernel[0] = '\0';
+    g_q4_name = Q4NameHook{};
+    g_q4_name.buf = kernel;
+    g_q4_name.cap = (int)cap;
+    g_q4_name.armed = true;
+    const int rc = q4_matvec_launch(L, nullptr);
+    const bool answered = !g_q4_name.armed;
+    g_q4_name.armed = false;
+    L2_TRY(rc);
+    if (!answered) return l2_fail(L2_ERR_ARG, "the launcher did not name its kernel");
+    geometry[0] = g_q4_name.grid, geometry[1] = g_q4_name.block, geometry[2] = g_q4_name.rows_per_block;
+    geometry[3] = (int32_t)g_q4_name.lds;
+    // every row of every matrix belongs to exactly one block, and the blocks of all matrices fit the grid
+    long blocks = 0;
+    for (int i = 0; i < (L.pair ? 1 : L.n_mats); i++) blocks += (L.m[i].out + geometry[2] - 1) / geometry[2];
+    if (blocks != geometry[0]) return l2_fail(L2_ERR_ARG, "plan: %ld row blocks for a grid of %d", blocks, geometry[0]);
+    return L2_OK;
+}
+
 extern "C" int l2_q4_plan(int in, const int32_t *out, int n_mats, int group_size, int pair, int norm, char *kernel,
                           size_t cap, int32_t *geometry) {
     if (!out || !kernel || cap < 2 || !geometry || n_mats < 1 || n_mats > 3) return l2_fail(L2_ERR_ARG, "bad argument");
     if (group_size != 32 && group_size != 64 && group_size != 128) return l2_fail(L2_ERR_ARG, "group size %d", group_size);
     if (in <= 0 || in % 32 || in % group_size) return l2_fail(L2_ERR_ARG, "in=%d", in);
-    static const float dummy[4] = {0.f, 0.f, 0.f, 0.f}; // only null / non-null matters: nothing is launched
+    static const float dummy[4] = {0.f, 0.f, 0.f, 0.f};
     Q4Launch L{};
     L.n_mats = n_mats;
     L.in = in;
@@ -2380,23 +2401,21 @@ extern "C" int l2_q4_plan(int in, const int32_t *out, int n_mats, int group_size
         L.m[i].wn = norm ? dummy : nullptr;
         L.m[i].out = out[i];
     }
-    kernel[0] = '\0';
-    g_q4_name = Q4NameHook{};
-    g_q4_name.buf = kernel;
-    g_q4_name.cap = (int)cap;
-    g_q4_name.armed = true;
-    const int rc = q4_matvec_launch(L, nullptr);
-    const bool answered = !g_q4_name.armed;
-    g_q4_name.armed = false;
-    L2_TRY(rc);
-    if (!answered) return l2_fail(L2_ERR_ARG, "the launcher did not name its kernel");
-    geometry[0] = g_q4_name.grid, geometry[1] = g_q4_name.block, geometry[2] = g_q4_name.rows_per_block;
-    geometry[3] = (int32_t)g_q4_name.lds;
-    // every row of every matrix belongs to exactly one block, and the blocks of all matrices fit the grid
-    long blocks = 0;
-    for (int i = 0; i < (pair ? 1 : n_mats); i++) blocks += (out[i] + geometry[2] - 1) / geometry[2];
-    if (blocks != geometry[0]) return l2_fail(L2_ERR_ARG, "plan: %ld row blocks for a grid of %d", blocks, geometry[0]);
-    return L2_OK;
+    return plan_of(L, kernel, cap, geometry);
+}
+
+extern "C" int l2_qlinear_plan(int in, int out, int group_size, int batch, int natural, char *kernel, size_t cap, int32_t *geometry) {
+    if (!kernel || cap < 2 || !geometry || batch < 1 || batch > 4096) return l2_fail(L2_ERR_ARG, "bad argument");
+    L2_TRY(check_qlinear_shape(in, out, group_size));
+    static const float dummy[4] = {0.f, 0.f, 0.f, 0.f};
+    static const int32_t order[4] = {0, 0, 0, 0};
+    DevQLinear q;
+    q.in = in, q.out = out, q.group_size = group_size, q.groups = in / group_size;
+    Q4Launch L = launch_of(q, batch, 0.f);
+    L.m[0] = mat_of(q, dummy, nullptr, nullptr);
+    if (natural && !q4_gathers_in_kernel(L)) return l2_fail(L2_ERR_ARG, "in=%d: x is gathered in front", in);
+    L.m[0].gidx = natural ? order : nullptr;
+    return plan_of(L, kernel, cap, geometry);
 }
 
 extern "C" int l2_kernel_class_count(void) { return K_NCLASS; }

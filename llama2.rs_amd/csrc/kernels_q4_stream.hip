@@ -684,11 +684,14 @@ static int plan_rows(const Q4Launch &L, int NW, int TR, size_t lds, bool pair, i
 
 static size_t staging_lds(int NWK, bool pair) { return (size_t)NWK * 64 * (kChunkPad + 1) * sizeof(float) * (pair ? 2 : 1); }
 
-// Whether one matrix in blocks of S streams with P rows in flight has no rows behind the loop (whose last bit is another).
+// Whether a launch in blocks of S streams with P rows in flight has no rows behind the loop (whose last bit is another).
 static bool whole_tiles(const Q4Launch &L, int NWK, int S, int P) {
-    int blocks = 0;
-    const int rpb = plan_rows(L, NWK * S, P * S, staging_lds(NWK, false), false, &blocks), last = L.m[0].out - (blocks - 1) * rpb;
-    return (rpb + S - 1) / S % P == 0 && (last + S - 1) / S % P == 0;
+    const int rpb = plan_rows(L, NWK * S, P * S, staging_lds(NWK, false), false, nullptr);
+    for (int i = 0; i < L.n_mats; i++) {
+        const int out = L.m[i].out, last = out - (out - 1) / rpb * rpb;
+        if ((last + S - 1) / S % P || (out > rpb && (rpb + S - 1) / S % P)) return false;
+    }
+    return true;
 }
 
 template <int G, int NWK, int S, bool PAIR, int MODE, int P = (PAIR ? 2 : 4), bool GATHER = false>
@@ -745,8 +748,12 @@ int launch_s(Q4Launch &L, hipStream_t stream) {
 // waves per block: 4096 inputs in one block of 16 waves per CU instead of two of 8, two rows in flight: 4096 rows 4.70 -> 4.35 us,
 // 11008 rows 7.43 -> 6.76, 2048 rows 3.65, 4.02 (not taken); as a projection of the model the same shape loses (7B 287 -> 289 us
 // per 8 layers).  5120 inputs: two rows in flight up to 8192 rows, three beyond, instead of four: 1024 rows 4.65 -> 3.76, 5120 rows
-// 5.79 -> 5.54, 13824 rows 10.05 -> 9.81.  These are taken where neither shape has rows behind the loop, so that one column of
-// the operator is, bit for bit, a column of several, which the form without the gathering takes in its own shape.
+// 5.79 -> 5.54, 13824 rows 10.05 -> 9.81.
+//
+// The rows here are those of all columns, so one column may take another shape than several of the same matrix, and the form
+// without the gathering another than the one with it.  So that a column is the same bits all the same, the shapes of one matrix
+// differ only where none of them has rows behind its loop: that is asked, or holds wherever the rows are whole eights (4096 inputs up
+// to 1024 rows).  Up to 2048 inputs a matrix whose last block has eight rows (1032 of them) keeps four streams of four rows.
 template <int G, int MODE>
 int launch_sg(Q4Launch &L, hipStream_t stream) {
     const int nwk = (L.in / 32 + 63) / 64;
@@ -759,7 +766,7 @@ int launch_sg(Q4Launch &L, hipStream_t stream) {
         }
     } else if (MODE == 0 && !L.pair && L.n_mats == 1 && L.m[0].gidx) {
         if constexpr (MODE == 0) switch (nwk) { // the gathering form, where one staging batch covers the vector
-            case 1: return rows <= 8 * cus ? launch_s<G, 1, 8, false, 0, 1, true>(L, stream) : launch_s<G, 1, 4, false, 0, 4, true>(L, stream);
+            case 1: return rows <= 8 * cus && whole_tiles(L, 1, 4, 4) ? launch_s<G, 1, 8, false, 0, 1, true>(L, stream) : launch_s<G, 1, 4, false, 0, 4, true>(L, stream);
             case 2:
                 if (rows <= 4 * cus) return launch_s<G, 2, 4, false, 0, 1, true>(L, stream);
                 if (rows > 8 * cus && whole_tiles(L, 2, 4, 2) && whole_tiles(L, 2, 8, 2)) return launch_s<G, 2, 8, false, 0, 2, true>(L, stream);
@@ -772,7 +779,7 @@ int launch_sg(Q4Launch &L, hipStream_t stream) {
         }
     } else if (!L.pair) {
         switch (nwk) {
-            case 1: return rows <= 8 * cus ? launch_s<G, 1, 8, false, MODE, 1>(L, stream) : launch_s<G, 1, 4, false, MODE>(L, stream);
+            case 1: return rows <= 8 * cus && whole_tiles(L, 1, 4, 4) ? launch_s<G, 1, 8, false, MODE, 1>(L, stream) : launch_s<G, 1, 4, false, MODE>(L, stream);
             case 2: return rows <= 4 * cus ? launch_s<G, 2, 4, false, MODE, 1>(L, stream) : launch_s<G, 2, 4, false, MODE, 2>(L, stream);
             case 3: return launch_s<G, 3, 4, false, MODE>(L, stream);
             case 4: return launch_s<G, 4, 4, false, MODE, 2>(L, stream); // 8192: rows of 4 KB; two in flight per stream measured faster than four (q|k|v 13.4 -> 12.2 us, wo 12.1 -> 10.9)

@@ -80,8 +80,8 @@ def test_qmatvec_staging_edges(ops, oracle, n_in, n_out):
     q.close()
 
 
-# Both sides of where the number of rows chooses another shape of block (4, 8 and 32 rows per compute unit of 256), with x in
-# its natural order (one column) and gathered in front (three); group 32 with its most scales per row among them.
+# Both sides of where the number of rows chooses another shape of block (4, 8 and 32 rows per compute unit of 256), one column and
+# three; group 32 with its most scales per row among them.
 @pytest.mark.parametrize("n_in,G,rows", [(1024, 32, (8, 2048, 2056)), (2048, 128, (2048, 2056)), (4096, 128, (1024, 1032, 2048, 2056)),
                                          (2112, 64, (1024, 1032, 2056)), (5120, 128, (1024, 8192, 8200)), (4160, 32, (8200,)),
                                          (8192, 64, (1024, 1032)), (6208, 64, (1024, 1032))])
@@ -97,6 +97,32 @@ def test_qmatvec_shapes_by_rows(ops, oracle, n_in, G, rows):
         for b in range(3):
             np.testing.assert_array_equal(q.matvec(x[b]), got[b], err_msg=str(n_out))
         q.close()
+
+
+# A column of several is the bits of one alone, by the entry point on host arrays (up to 8192 inputs the kernel permutes x) and by
+# the one on device memory (several columns are permuted in front): where one column takes the shape for few rows and several do
+# not, with rows behind the loop of a last block of eight (1032, 2040, 696, 264 rows) and without.
+@pytest.mark.parametrize("n_in,G,n_out,batches", [(1024, 32, 1032, (2, 3, 8)), (1024, 64, 2040, (2, 3, 8)), (2048, 128, 696, (2, 3, 8)),
+                                                  (2048, 32, 264, (8,)), (1024, 128, 1024, (2, 3, 8)), (4096, 128, 520, (2, 3, 8)),
+                                                  (8192, 64, 1032, (2, 8))])
+def test_qmatvec_columns_are_the_bits_of_one(ops, n_in, G, n_out, batches):
+    from llama2_rs import _lib
+    from tests.test_zz_no_alloc import _Hip
+    hip = _Hip()
+    rng = np.random.default_rng(n_out)
+    qw, qz, sc, gi = ck.synth_qlinear(rng, n_in, n_out, G, act_order=True)
+    q = ops.QLinear(qw, qz, sc, gi, G)
+    q.set_mode(_lib.PREFILL_COLUMNS)
+    x = rng.standard_normal((8, n_in)).astype(np.float32)
+    one = np.stack([q.matvec(c) for c in x])
+    assert nrel(one, x.astype(np.float64) @ ck.dequant_bin(qw, qz, sc, gi, G).astype(np.float64).T) < 1e-5
+    px, py = hip.upload(x), hip.empty(4 * 8 * n_out)
+    for B in batches:
+        np.testing.assert_array_equal(q.matvec(x[:B]), one[:B], err_msg=f"host arrays, {B}")
+        q.matvec_device(px, B, py)
+        np.testing.assert_array_equal(hip.download(py, (B, n_out)), one[:B], err_msg=f"device memory, {B}")
+    q.close()
+    hip.close()
 
 
 _ALT_FORM_SNIPPET = r"""
