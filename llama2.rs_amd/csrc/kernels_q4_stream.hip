@@ -246,6 +246,12 @@ struct RowData {
     int32_t z;
 };
 
+// A chunk's sum from those of its fours, in the association the block-wide staging uses (the tree of its three cross-lane
+// adds), so that a form of the operator which takes the sum by itself gives the same bits.
+__device__ __forceinline__ float chunk_sum(const float (&s4)[8]) {
+    return ((s4[0] + s4[1]) + (s4[2] + s4[3])) + ((s4[7] + s4[6]) + (s4[5] + s4[4]));
+}
+
 // MODE 0: fp32 inner loop, x staged through LDS (rmsnorm prologue, several matrices, row pairs).
 // MODE 1: integer-dot inner loop, x staged and quantised in LDS.
 // MODE 2: fp32 inner loop, one matrix without rmsnorm: every wave loads its own slice of x (coalesced)
@@ -426,7 +432,7 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const Q4Launch L
             const float4 v = kslice * 512 + j4 < n4 ? xd[i] : make_float4(0.f, 0.f, 0.f, 0.f);
             *reinterpret_cast<float4 *>(&xw[(j4 >> 3) * kChunkPad + (j4 & 7) * 4]) = v;
         }
-        float t = 0.f;
+        float t = 0.f, s4[8];
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             const float4 v = *reinterpret_cast<const float4 *>(&xw[lane * kChunkPad + 4 * i]);
@@ -434,8 +440,11 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const Q4Launch L
             x[0][4 * i + 1] = v.y;
             x[0][4 * i + 2] = v.z;
             x[0][4 * i + 3] = v.w;
-            t += (v.x + v.y) + (v.z + v.w);
+            s4[i] = (v.x + v.y) + (v.z + v.w);
+            t += s4[i];
         }
+        // The operator by itself (nothing in its epilogue) runs these rows through the gathering form too: the same bits then
+        if (NWK == 3 && epi_kind == Q4_EPI_STORE) t = chunk_sum(s4);
         sx[0] = t;
         xdelta[0] = 0.f;
     } else {
@@ -514,13 +523,11 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const Q4Launch L
                         x[q][4 * i + 3] = v.w;
                     }
                     if constexpr (GATHER) {
-                        // the chunk's sum in the association the block-wide staging uses (fours, then the tree of
-                        // its three cross-lane adds), so that both forms of the operator give the same bits
                         float s4[8];
 #pragma unroll
                         for (int k = 0; k < 8; k++)
                             s4[k] = (x[q][4 * k] + x[q][4 * k + 1]) + (x[q][4 * k + 2] + x[q][4 * k + 3]);
-                        sx[q] = ((s4[0] + s4[1]) + (s4[2] + s4[3])) + ((s4[7] + s4[6]) + (s4[5] + s4[4]));
+                        sx[q] = chunk_sum(s4);
                     } else {
                         sx[q] = xs[NC * kChunkPad + c];
                     }

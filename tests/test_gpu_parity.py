@@ -104,6 +104,7 @@ def test_qmatvec_shapes_by_rows(ops, oracle, n_in, G, rows):
 # not, with rows behind the loop of a last block of eight (1032, 2040, 696, 264 rows) and without.
 @pytest.mark.parametrize("n_in,G,n_out,batches", [(1024, 32, 1032, (2, 3, 8)), (1024, 64, 2040, (2, 3, 8)), (2048, 128, 696, (2, 3, 8)),
                                                   (2048, 32, 264, (8,)), (1024, 128, 1024, (2, 3, 8)), (4096, 128, 520, (2, 3, 8)),
+                                                  (5120, 128, 8200, (2, 8)), (4160, 32, 1032, (3,)), (6112, 32, 520, (3, 8)),
                                                   (8192, 64, 1032, (2, 8))])
 def test_qmatvec_columns_are_the_bits_of_one(ops, n_in, G, n_out, batches):
     from llama2_rs import _lib
