@@ -35,14 +35,15 @@ typedef float float4_any __attribute__((ext_vector_type(4), aligned(4)));
 
 // 16 bytes (aligned) past the L2: what a launch leaves dirty there is written back at its end, with nothing else to do, and the
 // kernels of a batch write megabytes in their last microseconds.  Not for single columns: the store's own way is longer, and that
-// is what the end of a decode kernel waits for (7B token 2 to 3 % longer, 70B 5 %).  The s_nop: data of a store wider than 8 bytes
-// must not be overwritten by the very next instruction, which the compiler sees to for its own stores only.
+// is what the end of a decode kernel waits for (7B token 2 to 3 % longer, 70B 5 %).  A store that the compiler knows (sc1 is what it
+// makes of "agent"), and not a statement of assembly: data of such a store may come out of a matrix instruction, whose result is
+// not there for another 10 wait states, and must not be overwritten for two behind it, neither of which the hardware sees to.
 #if defined(__HIPCC__)
 template <class T>
 __device__ __forceinline__ void store_through(T *p, const T &v) {
     static_assert(sizeof(T) == 16, "one instruction");
     typedef uint32_t four __attribute__((ext_vector_type(4)));
-    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 0" ::"v"(p), "v"(__builtin_bit_cast(four, v)) : "memory");
+    __builtin_amdgcn_global_store_b128((__attribute__((address_space(1))) four *)p, __builtin_bit_cast(four, v), "agent");
 }
 #endif
 
