@@ -1705,7 +1705,7 @@ static int ensure_lane(l2_model *m, int lane, int B, int slice_batch, int planes
 // layer, so `before_attn[l]` (the event of the pass before) is waited for in front of the attention of layer l, behind
 // the kernel that writes this pass's own rows of layer l, and `after_kv[l]` is recorded right there (either may be null).
 static int forward_enqueue_gemm(l2_model *m, l2_state *s, int B, int max_pos, const int32_t *dtok, const int32_t *dpos,
-                                int planes, int slice_batch, int lane, const hipEvent_t *after_kv,
+                                int planes, int slice_batch, int lane, bool beside, const hipEvent_t *after_kv,
                                 const hipEvent_t *before_attn) {
     L2_TRY(check_position(m, max_pos));
     s->rows = std::max(s->rows, max_pos + 1);
@@ -1715,7 +1715,7 @@ static int forward_enqueue_gemm(l2_model *m, l2_state *s, int B, int max_pos, co
     const bool dense = d.group_size == 0;
     hipStream_t st = lane ? m->extra_stream[lane - 1] : m->stream;
     auto gemm = [&](Q4Launch &Q, const XhList &X, const float *ss, int *ks) {
-        return gemm_launch(Q, X, ss, b.ws, b.ws_floats, planes, slice_batch, st, ks);
+        return gemm_launch(Q, X, ss, b.ws, b.ws_floats, planes, slice_batch, st, ks, beside);
     };
     // rms scale of the stream in b.x and the inputs of layer l's q, k and v; ks partial tiles are added first
     auto attn_inputs = [&](int l, int ks) {
@@ -1805,7 +1805,7 @@ static int forward_batch(l2_model *m, l2_state *s, int B, int max_pos, const int
         return forward_enqueue(m, s, B, max_pos, in);
     }
     L2_TRY(ensure_lane(m, 0, B, B, planes));
-    return forward_enqueue_gemm(m, s, B, max_pos, dtok, dpos, planes, B, 0, nullptr, nullptr);
+    return forward_enqueue_gemm(m, s, B, max_pos, dtok, dpos, planes, B, 0, false, nullptr, nullptr);
 }
 
 static int check_tokens(const l2_model *m, const int32_t *tokens, const int32_t *pos, int B, int *max_pos) {
@@ -1946,13 +1946,14 @@ static int prefill_chunks(l2_model *m, l2_state *s, const int32_t *tokens, int n
         return L2_OK;
     };
     auto enqueue_all = [&]() -> int {
+        const bool beside = lanes > 1 && std::count_if(passes.begin(), passes.end(), [](const PrefillPass &p) { return p.planes != 0; }) > 1;
         int c = 0; // GEMM passes so far
         for (const PrefillPass &p : passes) {
             const int max_pos = pos0 + p.first + p.n - 1;
             if (p.planes) {
                 const int lane = c % lanes, before = (c + lanes - 1) % lanes;
                 L2_TRY(forward_enqueue_gemm(m, s, p.n, max_pos, dtok + p.first, dpos + p.first, p.planes, p.slice_batch,
-                                            lane, passes.size() > 1 ? m->pf_ev[lane].data() : nullptr, c > 0 ? m->pf_ev[before].data() : nullptr));
+                                            lane, beside, passes.size() > 1 ? m->pf_ev[lane].data() : nullptr, c > 0 ? m->pf_ev[before].data() : nullptr));
                 c++;
             } else {
                 // few columns: the matvec kernels on the model's stream, behind everything

@@ -1151,7 +1151,7 @@ GemmShape gemm_shape(const Q4Launch &L, int slice_batch, int planes) {
 }
 
 int gemm_launch(Q4Launch &L, const XhList &xh, const float *ss, float *ws, size_t ws_floats, int planes, int slice_batch,
-                hipStream_t st, int *ks_out) {
+                hipStream_t st, int *ks_out, bool beside) {
     if (L.n_mats < 1 || L.n_mats > 3 || L.pair) return l2_fail(L2_ERR_ARG, "q4 gemm: n_mats=%d pair=%d", L.n_mats, L.pair);
     if (L.in % 32 || (L.group_size && L.in % L.group_size) || L.batch < 1) return l2_fail(L2_ERR_ARG, "q4 gemm: in=%d batch=%d", L.in, L.batch);
     if (L.e.kind == Q4_EPI_SCATTER_ONLY || L.e.n_scatter) return l2_fail(L2_ERR_ARG, "q4 gemm: no scatter epilogue");
@@ -1167,7 +1167,7 @@ int gemm_launch(Q4Launch &L, const XhList &xh, const float *ss, float *ws, size_
     if ((s.slices > 1 || partials) && (size_t)s.slices * L.batch * rows > ws_floats)
         return l2_fail(L2_ERR_ARG, "q4 gemm: %d slices of %d x %ld in a workspace of %zu", s.slices, L.batch, rows, ws_floats);
     if (planes == 1)
-        L2_TRY(gemm_launch_f16(L, xh, ss, ws, s, partials, st));
+        L2_TRY(gemm_launch_f16(L, xh, ss, ws, s, partials, beside, st));
     else
         L2_TRY(launch_fp32(L, xh, ss, ws, s, partials, st));
     if (ks_out) {

@@ -370,7 +370,7 @@ __global__ __launch_bounds__(64 * NW, NB > 2 ? 2 : 1) void q4_gemm_kernel(const 
 }
 
 template <int G, int NB, int NW>
-int launch_gemm(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, int partials, hipStream_t st) {
+int launch_gemm(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, int partials, bool beside, hipStream_t st) {
     constexpr int TN = 32 * NB;
     int row_blocks = 0;
     for (int i = 0; i < L.n_mats; i++) row_blocks += L.m[i].row_blocks = (L.m[i].out + 32 * NW - 1) / (32 * NW);
@@ -382,13 +382,14 @@ int launch_gemm(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const
     // six layers of 7B, 64, 99, 128 tokens 918 / 1075 / 1120 -> 903 / 1047 / 1080, four of 13B, 128 1057 -> 1041; with more of them than
     // two per CU whole tiles (70B, 179 1965 against 1978).  Tiles of 96 where those of 64 are more than a round, six layers of 7B: 287,
     // 349, 599 tokens 1702 / 1889 / 2469 -> 1670 / 1835 / 2450; four of 13B, 199, 299 1311 / 1716 -> 1291 / 1687.  Where both fit those
-    // of 64: 349 of 7B 1835 against 1886.
+    // of 64: 349 of 7B 1835 against 1886.  None of 96 beside another pass, which has a use for the CUs that a round
+    // leaves: four layers of 13B, 300 and 399 tokens in chunks of 256 1359 / 1742 -> 1302 / 1713, six of 7B, 899 in chunks of 128 3891 -> 3812.
     const int all = row_blocks * s.slices, tiles = all * t_full, cus = cu_count();
     int units = all, width = TN;
     if ((NB == 4 || (NB == 2 && tiles > cus && tiles < 2 * cus)) && tiles % cus) {
         const int first = tiles / cus * cus / t_full;
         for (const int w : {TN / 4 * 3, TN / 2})
-            if ((w % 32 == 0) && (all - first) * ((L.batch + w - 1) / w) + narrow * first <= cus) units = first, width = w;
+            if (w % 32 == 0 && !(beside && w > TN / 2) && (all - first) * ((L.batch + w - 1) / w) + narrow * first <= cus) units = first, width = w;
     }
     // partial tiles past the caches where they would fill them: what a launch leaves dirty there is written back at its end
     // (7B, 511 tokens: the four launches 13 us less per layer, their consumers 5 more; below 16 MB the other way round: there they
@@ -407,11 +408,11 @@ int launch_gemm(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const
 }
 
 template <int G>
-int launch_gemm_g(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, int partials, hipStream_t st) {
+int launch_gemm_g(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, int partials, bool beside, hipStream_t st) {
     switch (s.tokens) {
-        case 32: return launch_gemm<G, 1, 4>(L, xh, ss, ws, s, partials, st);
-        case 64: return launch_gemm<G, 2, 4>(L, xh, ss, ws, s, partials, st);
-        case 128: return launch_gemm<G, 4, 8>(L, xh, ss, ws, s, partials, st);
+        case 32: return launch_gemm<G, 1, 4>(L, xh, ss, ws, s, partials, beside, st);
+        case 64: return launch_gemm<G, 2, 4>(L, xh, ss, ws, s, partials, beside, st);
+        case 128: return launch_gemm<G, 4, 8>(L, xh, ss, ws, s, partials, beside, st);
     }
     return l2_fail(L2_ERR_ARG, "q4 gemm: token tile");
 }
@@ -444,16 +445,16 @@ GemmShape gemm_shape_f16(const Q4Launch &L, int slice_batch) {
     return s;
 }
 
-int gemm_launch_f16(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, int partials, hipStream_t st) {
+int gemm_launch_f16(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, int partials, bool beside, hipStream_t st) {
     if (L.in % 128 != 0) return l2_fail(L2_ERR_ARG, "q4 gemm: in=%d must be a multiple of 128", L.in);
     if (L.group_size >= 64 && (L.in / L.group_size) % 2 != 0)
         return l2_fail(L2_ERR_ARG, "q4 gemm: in=%d is an odd number of groups of %d", L.in, L.group_size);
     for (int i = 0; i < L.n_mats; i++)
         if (L.m[i].out % 32 != 0) return l2_fail(L2_ERR_ARG, "q4 gemm: out=%d must be a multiple of 32", L.m[i].out);
     switch (L.group_size) {
-        case 32: return launch_gemm_g<32>(L, xh, ss, ws, s, partials, st);
-        case 64: return launch_gemm_g<64>(L, xh, ss, ws, s, partials, st);
-        case 128: return launch_gemm_g<128>(L, xh, ss, ws, s, partials, st);
+        case 32: return launch_gemm_g<32>(L, xh, ss, ws, s, partials, beside, st);
+        case 64: return launch_gemm_g<64>(L, xh, ss, ws, s, partials, beside, st);
+        case 128: return launch_gemm_g<128>(L, xh, ss, ws, s, partials, beside, st);
     }
     return l2_fail(L2_ERR_ARG, "q4 gemm: group size %d", L.group_size);
 }

@@ -225,10 +225,12 @@ GemmShape gemm_shape(const Q4Launch &L, int slice_batch, int planes);
 GemmShape gemm_shape_f16(const Q4Launch &L, int slice_batch);
 // Y = X W^T for L.batch columns; ss (per column, may be null) scales them.  Epilogues: store, residual add.  ws:
 // workspace for the K slices' partial tiles.  ks_out given: the kernel leaves its slices as partial tiles [KS][B][out]
-// in ws (also when there is one), no reduction is launched, and *ks_out says how many there are.
+// in ws (also when there is one), no reduction is launched, and *ks_out says how many there are.  beside: a launch on another
+// stream runs at the same time and takes the CUs that this one leaves.
 int gemm_launch(Q4Launch &L, const XhList &xh, const float *ss, float *ws, size_t ws_floats, int planes, int slice_batch,
-                hipStream_t st, int *ks_out = nullptr);
-int gemm_launch_f16(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, int partials, hipStream_t st);
+                hipStream_t st, int *ks_out = nullptr, bool beside = false);
+int gemm_launch_f16(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, int partials, bool beside,
+                    hipStream_t st);
 // What a first launch for this group size does besides enqueueing (for callers under graph capture).
 int gemm_warm_up(int group_size);
 
