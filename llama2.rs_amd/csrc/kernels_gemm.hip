@@ -180,10 +180,10 @@ __global__ __launch_bounds__(256) void host_input_kernel(void *__restrict__ out,
 
 // Four consecutive outputs of column t: a partial tile of this K slice, or the result through the launch's epilogue.
 __device__ __forceinline__ void finish4(const Q4Launch &L, int mi, const float *ss, float *ws, int KS, int ks, int partials,
-                                        int t, int o, float4 v) {
+                                        int t, int o, float4 v, int B) {
     const int n_out = L.m[mi].out;
     if (KS > 1 || partials) {
-        store_through(reinterpret_cast<float4 *>(ws + ((size_t)ks * L.batch + t) * n_out + o), v);
+        store_through(reinterpret_cast<float4 *>(ws + ((size_t)ks * B + t) * n_out + o), v);
         return;
     }
     const float sc = ss ? ss[t] : 1.0f;
@@ -219,7 +219,7 @@ struct TileLds {
 // MFMA must stay inside one group, so its words are kg and 4 + kg.
 template <int G, int NT, int NW>
 __device__ __forceinline__ void q4_tile(const Q4Launch &L, const XhList &xl, int in_p, const float *__restrict__ ss, float *__restrict__ ws,
-                                        int KS, int partials, int rb, int ks, int t0) {
+                                        int KS, int partials, int rb, int ks, int t0, int B) {
     using S = TileLds<G, NT, NW>;
     constexpr int NP = 3, TN = 16 * NT, RB = 32 * NW;
     constexpr int KPG = G >= 64 ? G / 64 : 1; // K steps per group
@@ -230,7 +230,7 @@ __device__ __forceinline__ void q4_tile(const Q4Launch &L, const XhList &xl, int
         rb -= L.m[mi].row_blocks;
         mi++;
     }
-    const int n_out = L.m[mi].out, groups = L.groups, B = L.batch, in = L.in;
+    const int n_out = L.m[mi].out, groups = L.groups, in = L.in;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, kg = lane >> 4;
     const int obase = rb * RB + wave * 32;
@@ -476,34 +476,36 @@ __device__ __forceinline__ void q4_tile(const Q4Launch &L, const XhList &xl, int
             const int tt = pass * 8 + tl;
             float4 v = *reinterpret_cast<const float4 *>(&tile_o[tt * kTRow + oc]);
             const int t = t0 + n0 * 16 + tt, o = obase + oc;
-            if (t < B && o < n_out) finish4(L, mi, ss, ws + ws_base, KS, ks, partials, t, o, v);
+            if (t < B && o < n_out) finish4(L, mi, ss, ws + ws_base, KS, ks, partials, t, o, v, B);
         }
     }
 }
 
-// The first `whole` blocks take the tiles of as many row blocks (and slices) as they are, the others tiles of `width` columns of the
-// row blocks that are left.  The last tile of tokens takes 16, 32 or 48 where that is enough (48 against 64: six layers of 7B, 33 and
-// 48 tokens 1114 / 1131 -> 1046 / 1066 us, 299 2743 -> 2685, three of 70B, 44 1531 -> 1397; 13824x5120, 40 columns 36.4 -> 32.6).
+// The first `whole` blocks take a tile each, row block (and slice) by row block, the others tiles of `width` columns of what is
+// left; these are 48, in whole row blocks, or 32, and then may begin within one.  The last tile of tokens takes 16, 32 or 48 where that
+// is enough (48 against 64: six layers of 7B, 33 and 48 tokens 1114 / 1131 -> 1046 / 1066 us, 299 2743 -> 2685, three of 70B, 44
+// 1531 -> 1397; 13824x5120, 40 columns 36.4 -> 32.6).
 template <int G, int NT, int NW>
 __global__ __launch_bounds__(64 * NW, NT == 1 ? 3 : 2) void q4_tile_gemm_kernel(const Q4Launch L, const XhList xl, int in_p,
                                                               const float *__restrict__ ss, float *__restrict__ ws, int KS,
                                                               int t_tiles, int row_blocks, int whole, int width, int partials) {
     // an XCD gets all token tiles of a row block one behind the other: what runs on it at one time shares weights and tiles
-    int rb, t0, n;
+    int rb, t0, n, B = L.batch;
+    asm volatile("" : "+s"(B)); // read once, and not in front of every store again (0.5 % of 13B's prompts)
     if (NT < 4 || (int)blockIdx.x < whole) {
         const int work = xcd_item(blockIdx.x, whole);
-        rb = work / t_tiles, t0 = (work - rb * t_tiles) * 16 * NT, n = L.batch - t0;
+        rb = work / t_tiles, t0 = (work - rb * t_tiles) * 16 * NT, n = B - t0;
     } else {
-        const int work = xcd_item(blockIdx.x - whole, gridDim.x - whole), per = (L.batch + width - 1) / width;
-        rb = work / per, t0 = (work - rb * per) * width, n = min(L.batch - t0, width);
-        rb += whole / t_tiles;
+        const int per = (B + width - 1) / width, begun = whole / t_tiles; // a tile of this row block is two of 32
+        const int work = xcd_item(blockIdx.x - whole, gridDim.x - whole) + begun * per + (whole - begun * t_tiles) * 2;
+        rb = work / per, t0 = (work - rb * per) * width, n = min(B - t0, width);
     }
     const int ks = rb / row_blocks;
     rb -= ks * row_blocks;
-    if (NT > 1 && n <= 16) q4_tile<G, 1, NW>(L, xl, in_p, ss, ws, KS, partials, rb, ks, t0);
-    else if (NT > 2 && n <= 32) q4_tile<G, NT < 2 ? NT : 2, NW>(L, xl, in_p, ss, ws, KS, partials, rb, ks, t0);
-    else if (NT > 3 && n <= 48) q4_tile<G, NT < 3 ? NT : 3, NW>(L, xl, in_p, ss, ws, KS, partials, rb, ks, t0);
-    else q4_tile<G, NT, NW>(L, xl, in_p, ss, ws, KS, partials, rb, ks, t0);
+    if (NT > 1 && n <= 16) q4_tile<G, 1, NW>(L, xl, in_p, ss, ws, KS, partials, rb, ks, t0, B);
+    else if (NT > 2 && n <= 32) q4_tile<G, NT < 2 ? NT : 2, NW>(L, xl, in_p, ss, ws, KS, partials, rb, ks, t0, B);
+    else if (NT > 3 && n <= 48) q4_tile<G, NT < 3 ? NT : 3, NW>(L, xl, in_p, ss, ws, KS, partials, rb, ks, t0, B);
+    else q4_tile<G, NT, NW>(L, xl, in_p, ss, ws, KS, partials, rb, ks, t0, B);
 }
 
 // Linear::matvec<B> of the model without quantisation (src/model.rs:22-31) for a batch: fp32 weights, fp32 activations,
@@ -760,7 +762,7 @@ __device__ __forceinline__ void dense_tile(const Q4Launch &L, const XhList &xl, 
         const int t = t0 + n * 16 + r;
         if (t >= B || o >= n_out) continue;
         const f4v v = run[n];
-        if (__builtin_isfinite((v[0] + v[1]) + (v[2] + v[3]))) finish4(L, mi, ss, ws + ws_base, KS, ks, partials, t, o, make_float4(v[0], v[1], v[2], v[3]));
+        if (__builtin_isfinite((v[0] + v[1]) + (v[2] + v[3]))) finish4(L, mi, ss, ws + ws_base, KS, ks, partials, t, o, make_float4(v[0], v[1], v[2], v[3]), B);
         else again |= 1u << n;
     }
     if (!__any(again)) return;
@@ -774,7 +776,7 @@ __device__ __forceinline__ void dense_tile(const Q4Launch &L, const XhList &xl, 
         f4v v{NAN, NAN, NAN, NAN};
         const bool nan = dense_nan(x_lane, k0, k1);
         if (__any((again >> n & 1) && !nan)) v = dense_again(w_lane, x_lane, in_p, k0, k1);
-        if (again >> n & 1) finish4(L, mi, ss, ws + ws_base, KS, ks, partials, t, o, make_float4(v[0], v[1], v[2], v[3]));
+        if (again >> n & 1) finish4(L, mi, ss, ws + ws_base, KS, ks, partials, t, o, make_float4(v[0], v[1], v[2], v[3]), B);
     }
 }
 
@@ -1037,15 +1039,19 @@ int launch_tile(const Q4Launch &L, const XhList &xh, const float *ss, float *ws,
     size_t lds = 0;
     L2_TRY((ready_tile<G, NT, NW>(&lds)));
     const int t_tiles = (L.batch + 16 * NT - 1) / (16 * NT), tiles = total * t_tiles * KS, cus = cu_count();
-    // One block per CU: the row blocks that whole rounds of tiles leave over go in tiles of 32 columns, or of 48, where that is one
-    // round of blocks, in some 0.7 or 0.85 of a whole one's time.  Six layers of 7B, 32: 169, 250, 439 tokens 2239 / 2470 / 3871 ->
+    // One block per CU: what whole rounds of tiles leave over goes in tiles of 32 columns, or of 48, where that is one round of
+    // blocks, in some 0.7 or 0.85 of a whole one's time.  Six layers of 7B, 32: 169, 250, 439 tokens 2239 / 2470 / 3871 ->
     // 2120 / 2357 / 3635 us, four of 13B, 149 1964 -> 1881; 48: 299 and 511 tokens of 7B 2668 / 3971 -> 2632 /
     // 3934, 179 of 70B 3251 -> 3196; 4096x11008, group 32, 130 columns 68.3 -> 58.7.
     int whole = tiles, width = 16 * NT, blocks = tiles;
     if (NT == 4 && tiles > cus && tiles % cus) {
-        const int units = tiles / cus * cus / t_tiles, left = total * KS - units;
-        for (const int w : {48, 32})
-            if (left * ((L.batch + w - 1) / w) <= cus) whole = units * t_tiles, width = w, blocks = whole + left * ((L.batch + w - 1) / w);
+        // Whole tiles for full rounds, to the tile where the narrower ones divide one (three layers of 70B, 750 tokens, where only then
+        // those of 32 fit: 10690 -> 10440).
+        const int rounds = tiles / cus * cus, begun = rounds / t_tiles;
+        for (const int w : {48, 32}) {
+            const int done = 16 * NT % w ? 0 : rounds % t_tiles, per = (L.batch + w - 1) / w, at = begun * per + done * (16 * NT / w);
+            if (total * KS * per - at <= cus) whole = begun * t_tiles + done, width = w, blocks = whole + total * KS * per - at;
+        }
     }
     hipLaunchKernelGGL((q4_tile_gemm_kernel<G, NT, NW>), dim3(blocks), dim3(64 * NW), lds, st, L, xh, gemm_padded(L.in), ss, ws, KS, t_tiles, total, whole,
                        width, partials);

@@ -335,26 +335,33 @@ __device__ __forceinline__ void q4_gemm_tile(const Q4Launch &L, const XhList &xh
     }
 }
 
-// One block per work item.  A unit is a row block and a slice of K.  The first `units` of them go in tiles of 32 NB tokens; those that
-// whole rounds of blocks leave over in tiles of `width`; then come the last tokens of the first ones, where they need no more than
-// half a tile.  A tile costs its width in steps of 32 and the dequantisation of its weights (128, 64, 32 tokens of 70B's w1: 119, 75,
-// 62 us).
+// One block per work item.  A unit is a row block and a slice of K.  The first `units` of them, and `extra` tiles of the next one, go in
+// tiles of 32 NB tokens; what whole rounds of blocks leave over goes in tiles of `width`; then come the last tokens of the first units,
+// where they need no more than half a tile.  A tile costs its width in steps of 32 and the dequantisation of its weights (128, 64,
+// 32 tokens of 70B's w1: 119, 75, 62 us).
 template <int G, int NB, int NW>
 __global__ __launch_bounds__(64 * NW, NB > 2 ? 2 : 1) void q4_gemm_kernel(const Q4Launch L, const XhList xh, const float *__restrict__ ss,
-                                                      float *__restrict__ ws, int KS, int partials, int row_blocks, int t_full, int units, int width) {
+                                                      float *__restrict__ ws, int KS, int partials, int row_blocks, int t_full, int units, int extra,
+                                                      int width) {
     constexpr int TN = 32 * NB, CHUNK = 8;
-    const int whole = units * t_full, per = (L.batch + width - 1) / width, other = (row_blocks * KS - units) * per, b = blockIdx.x;
+    const int b = blockIdx.x, whole = units * t_full + extra, per = (L.batch + width - 1) / width;
+    const int head = extra ? (L.batch - extra * TN + width - 1) / width : 0; // of the unit that has tiles of both kinds
+    const int begun = units + (extra > 0), left = row_blocks * KS - begun, other = head + left * per;
     int unit, t0, n;
     if (b < whole) { // 8 row blocks at a time, token tile by token tile: what runs on an XCD shares tiles and weights
         int item = xcd_item(b, whole);
+        const bool of_next = item >= units * t_full;
+        const int next_tile = item - units * t_full;
+        if (of_next) item = 0;
         const int first = item / (row_blocks * t_full) * row_blocks, c = (item -= first * t_full) / (CHUNK * t_full);
         const int of = min(CHUNK, min(row_blocks, units - first) - c * CHUNK), at = item - c * CHUNK * t_full, tt = at / of;
-        unit = first + c * CHUNK + at - tt * of, t0 = tt * TN, n = L.batch - t0;
+        unit = of_next ? units : first + c * CHUNK + at - tt * of, t0 = (of_next ? next_tile : tt) * TN, n = L.batch - t0;
     } else if (b < whole + other) {
-        const int item = xcd_item(b - whole, other);
-        const int left = row_blocks * KS - units, c = item / (CHUNK * per), of = min(CHUNK, left - c * CHUNK);
+        const int item = xcd_item(b - whole, other) - head, c = max(item, 0) / (CHUNK * per), of = min(CHUNK, max(left - c * CHUNK, 1));
         const int at = item - c * CHUNK * per, tt = at / of;
-        unit = units + c * CHUNK + at - tt * of, t0 = tt * width, n = min(L.batch - t0, width);
+        if (item < 0) unit = units, t0 = extra * TN + (item + head) * width;
+        else unit = begun + c * CHUNK + at - tt * of, t0 = tt * width;
+        n = min(L.batch - t0, width);
     } else {
         unit = xcd_item(b - whole - other, gridDim.x - whole - other), t0 = t_full * TN, n = L.batch - t0;
     }
@@ -375,7 +382,7 @@ int launch_gemm(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const
     int row_blocks = 0;
     for (int i = 0; i < L.n_mats; i++) row_blocks += L.m[i].row_blocks = (L.m[i].out + 32 * NW - 1) / (32 * NW);
     const int rest = L.batch % TN, t_full = L.batch / TN + (rest > TN / 2), narrow = rest > 0 && rest <= TN / 2;
-    // The units that whole rounds leave over go in narrower tiles where these, and what is left of the others' tokens, fit one round:
+    // What whole rounds of tiles leave over goes in narrower ones where these, and the last tokens of the other units, fit one round:
     // 7B's w1|w3, 511 tokens, 344 tiles on 256 CUs 123 -> 112 us; with 224 narrow tiles behind 64 left over (70B's, 776) they take 822
     // and whole tiles 804.  With several slices too: four layers of 13B, group 64, 399 tokens 2192 -> 2135, six of 7B, group 32, 249
     // tokens 1656 -> 1610.  Of the blocks of four waves too, where some CUs have two and others one (two take twice as long as one):
@@ -385,11 +392,16 @@ int launch_gemm(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const
     // of 64: 349 of 7B 1835 against 1886.  None of 96 beside another pass, which has a use for the CUs that a round
     // leaves: four layers of 13B, 300 and 399 tokens in chunks of 256 1359 / 1742 -> 1302 / 1713, six of 7B, 899 in chunks of 128 3891 -> 3812.
     const int all = row_blocks * s.slices, tiles = all * t_full, cus = cu_count();
-    int units = all, width = TN;
+    int units = all, extra = 0, width = TN, blocks = tiles + narrow * all;
     if ((NB == 4 || (NB == 2 && tiles > cus && tiles < 2 * cus)) && tiles % cus) {
-        const int first = tiles / cus * cus / t_full;
-        for (const int w : {TN / 4 * 3, TN / 2})
-            if (w % 32 == 0 && !(beside && w > TN / 2) && (all - first) * ((L.batch + w - 1) / w) + narrow * first <= cus) units = first, width = w;
+        // Whole tiles for full rounds: of these units, and `done` of the next one, without which those of 64 may not fit (three layers of
+        // 70B, 399 tokens in chunks of 128: 2785 -> 2735).  With four waves none of the next one: 70B, 176 tokens 1405, with them 1433.
+        const int rounds = tiles / cus * cus, begun = rounds / t_full, done = NB == 4 ? rounds % t_full : 0;
+        for (const int w : {TN / 4 * 3, TN / 2}) {
+            if (w % 32 || (beside && w > TN / 2)) continue;
+            const int n = (done ? (L.batch - done * TN + w - 1) / w : 0) + (all - begun - (done > 0)) * ((L.batch + w - 1) / w) + narrow * begun;
+            if (n <= cus) units = begun, extra = done, width = w, blocks = begun * t_full + done + n;
+        }
     }
     // partial tiles past the caches where they would fill them: what a launch leaves dirty there is written back at its end
     // (7B, 511 tokens: the four launches 13 us less per layer, their consumers 5 more; below 16 MB the other way round: there they
@@ -397,12 +409,12 @@ int launch_gemm(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const
     size_t bytes = 0;
     for (int i = 0; i < L.n_mats; i++) bytes += (size_t)s.slices * L.batch * L.m[i].out * 4;
     if (partials && bytes > ((size_t)16 << 20)) partials = 2;
-    const dim3 grid(units * t_full + (all - units) * ((L.batch + width - 1) / width) + narrow * units), block(64 * NW);
+    const dim3 grid(blocks), block(64 * NW);
     // the tiles, or the output staging tiles of the epilogue (32 x 36 floats per wave)
     const size_t lds = std::max(GemmLds<G, NW>::size(TN), (size_t)NW * 32 * 36 * sizeof(float));
     static LdsLimit limit(48 * 1024);
     L2_TRY(limit.ensure(reinterpret_cast<const void *>(q4_gemm_kernel<G, NB, NW>), lds));
-    hipLaunchKernelGGL((q4_gemm_kernel<G, NB, NW>), grid, block, lds, st, L, xh, ss, ws, s.slices, partials, row_blocks, t_full, units, width);
+    hipLaunchKernelGGL((q4_gemm_kernel<G, NB, NW>), grid, block, lds, st, L, xh, ss, ws, s.slices, partials, row_blocks, t_full, units, extra, width);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }

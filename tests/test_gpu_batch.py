@@ -74,6 +74,22 @@ def test_batch_last_round_vs_fp64(ops, n_out, B):
     q.close()
 
 
+# A column's bits are the same in tiles of every width: rows of weights that repeat every 256 (a block) and columns that repeat every
+# seven give the same outputs wherever they stand.  Row blocks with tiles of both widths (their narrow ones from column 64 or 128 on),
+# tiles of 32 and 48 columns, a last tile of every width, one round with nothing left over.
+@pytest.mark.parametrize("n_out,B", [(24584, 150), (24584, 177), (24584, 192), (22008, 258), (22008, 300), (16640, 250), (4104, 61)])
+def test_batch_bits_whatever_the_tile(ops, n_out, B):
+    rng = np.random.default_rng(B)
+    qw, qz, sc, gi = ck.synth_qlinear(rng, 256, 256, 64, act_order=True)
+    rep = -(-n_out // 256)
+    q = ops.QLinear(np.tile(qw, (rep, 1))[:n_out], np.tile(qz, (rep, 1))[:n_out // 8], np.tile(sc, (rep, 1))[:n_out], gi, 64)
+    x = rng.standard_normal((7, 256)).astype(np.float32)[np.arange(B) % 7]
+    got = q.matvec(x)
+    assert nrel(got[:7, :256], x[:7].astype(np.float64) @ ck.dequant_bin(qw, qz, sc, gi, 64).astype(np.float64).T) < 1e-5
+    np.testing.assert_array_equal(got, got[:7, :256][np.arange(B) % 7][:, np.arange(n_out) % 256])
+    q.close()
+
+
 # scales and zero points in tiles of 32 rows x 32 groups: a last tile of 8 rows alone, of 24, behind a whole one, and of one group
 @pytest.mark.parametrize("n_in,n_out,G,B", [(28672, 8, 32, 300), (28672, 24, 64, 90), (28672, 40, 128, 60), (1056, 2056, 32, 32),
                                             (4160, 520, 64, 33)])
@@ -359,6 +375,29 @@ def test_fp16_operator_last_round(ops, B):
     assert not np.array_equal(got, want)
     for b in range(B):
         assert nrel(got[b], want[b]) < 2e-5, b
+
+
+# as test_batch_bits_whatever_the_tile: tiles of 128 tokens with ones of 64 and 96 for what is left, row blocks that have both, with
+# and without last tokens of their own; blocks of 128 rows, tiles of 64 tokens with ones of 32
+@pytest.mark.parametrize("hidden,B", [(21888, 350), (21888, 590), (25472, 350), (25472, 424), (21888, 520), (15360, 180), (15360, 99)])
+def test_fp16_bits_whatever_the_tile(ops, hidden, B):
+    from llama2_rs import _lib
+    dims = ck.Dims(dim=256, hidden_dim=hidden, n_layers=1, n_heads=2, n_kv_heads=2, vocab_size=64, seq_len=1024, group_size=64)
+    img = ck.synth_weights_image(dims, seed=11)
+    rows, words = np.arange(hidden), img.view(np.int32)
+    at = 1 + 64 * 256 + 256 + 4 * (256 * 32 + 32 * 4 + 256 * 4 + 256) + 256  # w1 begins behind q, k, v, o and two norms
+    for n, per in ((hidden, 32), (hidden // 8, 4), (hidden, 4)):             # packed weights, zero points, scales
+        part = words[at:at + n * per].reshape(n, per)
+        part[:] = part[np.arange(n) % (256 * n // hidden)].copy()
+        at += n * per
+    m = ops.Model(img, dims)
+    m.set_prefill_mode(_lib.PREFILL_MFMA)
+    x = np.random.default_rng(B).standard_normal((7, 256)).astype(np.float32)[np.arange(B) % 7]
+    got = m.qmatvec(0, _lib.W1, x)
+    m.set_prefill_mode(_lib.PREFILL_FP32)
+    assert nrel(got[:7, :256], m.qmatvec(0, _lib.W1, x)[:7, :256]) < 2e-3
+    np.testing.assert_array_equal(got, got[:7, :256][np.arange(B) % 7][:, rows % 256])
+    m.close()
 
 
 # prompt attention with two sets of columns per block (two blocks per compute unit and more), the last block with one
