@@ -754,7 +754,8 @@ int launch_s(Q4Launch &L, hipStream_t stream) {
 // The gathering form has more to stage (x and where each of its elements goes) and nothing behind the sums, so it gains from more
 // waves per block: 4096 inputs in one block of 16 waves per CU instead of two of 8, two rows in flight: 4096 rows 4.70 -> 4.35 us,
 // 11008 rows 7.43 -> 6.76, 2048 rows 3.65, 4.02 (not taken); as a projection of the model the same shape loses (7B 287 -> 289 us
-// per 8 layers).  5120 inputs: two rows in flight up to 8192 rows, three beyond, instead of four: 1024 rows 4.65 -> 3.76, 5120 rows
+// per 8 layers); and several columns are more blocks than a CU holds at once, of which two of 8 waves overlap and one of 16 does not
+// (4096 rows, 8, 16, 48 columns on host arrays 44.4 / 72.4 / 175 us, with 16 waves 47.7 / 79.5 / 198).  5120 inputs: two rows in flight up to 8192 rows, three beyond, instead of four: 1024 rows 4.65 -> 3.76, 5120 rows
 // 5.79 -> 5.54, 13824 rows 10.05 -> 9.81.
 //
 // The rows here are those of all columns, so one column may take another shape than several of the same matrix, and the form
@@ -776,7 +777,7 @@ int launch_sg(Q4Launch &L, hipStream_t stream) {
             case 1: return rows <= 8 * cus && whole_tiles(L, 1, 4, 4) ? launch_s<G, 1, 8, false, 0, 1, true>(L, stream) : launch_s<G, 1, 4, false, 0, 4, true>(L, stream);
             case 2:
                 if (rows <= 4 * cus) return launch_s<G, 2, 4, false, 0, 1, true>(L, stream);
-                if (rows > 8 * cus && whole_tiles(L, 2, 4, 2) && whole_tiles(L, 2, 8, 2)) return launch_s<G, 2, 8, false, 0, 2, true>(L, stream);
+                if (L.batch <= 2 && rows > 8 * cus && whole_tiles(L, 2, 4, 2) && whole_tiles(L, 2, 8, 2)) return launch_s<G, 2, 8, false, 0, 2, true>(L, stream);
                 return launch_s<G, 2, 4, false, 0, 2, true>(L, stream);
             case 3:
                 if (rows <= 32 * cus && whole_tiles(L, 3, 4, 4) && whole_tiles(L, 3, 4, 2)) return launch_s<G, 3, 4, false, 0, 2, true>(L, stream);
