@@ -1244,8 +1244,10 @@ static int qlinear_scratch(l2_qlinear *q, int B) {
     return L2_OK;
 }
 
-// From here on x comes in two parts: 16 columns of 13824 inputs 84.9 us whole, 81.5 by halves, 82.5 as a quarter and the rest.
-static constexpr size_t kSplitBytes = 256 * 1024;
+// From here on x comes in two parts, whose second kernel costs 3 us: 384 KB (24 columns of 4096 inputs) 57.4 us whole, 58.5 by
+// halves, 512 KB 67.8 and 67.9, 768 KB 91.6 and 89.6, 884 KB (16 of 13824) 82.8 and 78.5; with the matvec that permutes x itself
+// 50.1 and 50.5, 62.3 and 61.2, 85.7 and 83.4 for 24, 32 and 48 of 4096.
+static constexpr size_t kSplitBytes = 512 * 1024;
 
 static int operator_enqueue(const DevQLinear &q, const float *dx, float *dxg, float *y, const OperatorBufs &bufs, int planes,
                             int B, hipStream_t st) {

@@ -317,7 +317,8 @@ int sample_weights_launch(float *w, unsigned long long *redo, const float *logit
                           const unsigned long long *amax, hipStream_t st);
 // *id = the index of the running maximum.
 int index_launch(const unsigned long long *amax, int32_t *id, hipStream_t st);
-// dst = src, n floats; for small pieces of pinned host memory.
+// dst = src, n floats; for pieces of pinned host memory up to a megabyte: quicker than the copy engine, behind which a kernel starts
+// late (the operator on host arrays, 4096x1024, 4, 16, 64 columns by themselves 22.7 / 38.4 / 104 us, with it 27.8 / 42.2 / 120).
 int copy_launch(float *dst, const float *src, size_t n, hipStream_t st);
 // k and v: the first n floats (a multiple of 4) of each of `layers` stretches of `stride` floats become zero.
 int clear_rows_launch(float *k, float *v, int layers, size_t stride, size_t n, hipStream_t st);
