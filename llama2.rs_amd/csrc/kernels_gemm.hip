@@ -212,7 +212,8 @@ struct TileLds {
 // (kernels_q4_gemm.hip, which explains the layout and the waits): tiles of 64 k two steps ahead, weights two units.  One
 // barrier per step; a step is 6 NT pairs of MFMAs, with the dequantisation of the next one's weights and the folds of finished
 // groups spread between them: some 230 instructions for 64 tokens, which the two waves of a SIMD issue at one per 4.9 cycles
-// (2546 cycles per step of 7B's w1|w3 at 299 tokens before the scales and zero points came in tiles, 1536 of them MFMAs).  Eight waves and 64 tokens take 133 KB of LDS, one
+// (2546 cycles per step of 7B's w1|w3 at 299 tokens before the scales and zero points came in tiles, 1536 of them MFMAs; what a
+// SIMD can issue is 1624, the rest are waits).  Eight waves and 64 tokens take 133 KB of LDS, one
 // block per CU; four waves and 16 or 32 tokens, where weights are what is read, two or three.
 //
 // Lane (r = l % 16, kg = l / 16).  G >= 64: the lane's words of a step are 2 kg and 2 kg + 1, MFMA k takes one each.  G = 32: an

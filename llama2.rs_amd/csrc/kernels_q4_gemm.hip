@@ -25,10 +25,10 @@
 //     vector work (dequantisation of the next step, fold of the group before) stands evenly between the MFMAs of both halves
 //     of a step, operands are read from LDS four pairs of MFMAs ahead, and a wave's priority falls with its progress since
 //     the last barrier: with equal priorities the older wave of a SIMD ran ahead and waited 30 % of the time at the barrier
-//     (1862 cycles per step of 64 k; 1650 now, 1024 of them MFMAs).
-//   - Power.  With 70B's shapes the clock falls to 1.8 - 1.9 GHz; all-zero activations run the same code at 2.23 GHz.  The
-//     16x16x32 form needs less than 32x32x16 for the same products (a loop of nothing else: 1974 against 1655 TFLOP/s), and
-//     blocks of 256 rows read every activation tile half as often as blocks of 128.
+//     (1862 cycles per step of 64 k; 1650 now, 1024 of them MFMAs; what a SIMD can issue is 1104, the rest are waits).
+//   - Power, a cost and not the bound.  With 70B's shapes the clock falls to 1.8 - 1.9 GHz; all-zero activations run the same
+//     code at 2.23 GHz.  The 16x16x32 form needs less than 32x32x16 for the same products (a loop of nothing else: 1974
+//     against 1655 TFLOP/s), and blocks of 256 rows read every activation tile half as often as blocks of 128.
 //
 // Dequant.  (w >> 4i) & 0x000F000F | 0x64006400 is the fp16 pair (1024+n_i,
 // 1024+n_{i+4}); subtracting 1024+z1 is exact.  The pairs come out as
