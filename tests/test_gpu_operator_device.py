@@ -61,9 +61,9 @@ def test_any_float_address(ops, n_in, n_out, G, batches):
 
 
 # The operator on host arrays scatters x from pinned memory where the one on device memory gathers it: the same bits.  Rows that end
-# inside a thread's first or second piece and with half a K step (4128), in one part and in two (256 KiB), even and odd; long rows for
+# inside a thread's first or second piece and with half a K step (4128), in one part and in two (512 KiB), even and odd; long rows for
 # the matvec kernels (12320).
-@pytest.mark.parametrize("n_in,n_out,G,batches", [(4128, 4104, 32, (4, 15, 16, 17, 61)), (2048, 4104, 64, (31, 32, 33, 128)),
+@pytest.mark.parametrize("n_in,n_out,G,batches", [(4128, 4104, 32, (4, 15, 16, 17, 31, 32, 61)), (2048, 4104, 64, (31, 32, 33, 63, 64, 65, 128)),
                                                   (12320, 264, 32, (1, 2, 3)), (28672, 1024, 64, (1, 3, 9))])
 def test_host_input_is_the_device_input(ops, n_in, n_out, G, batches):
     hip = _Hip()
@@ -74,6 +74,23 @@ def test_host_input_is_the_device_input(ops, n_in, n_out, G, batches):
         px, py = hip.upload(x), hip.empty(4 * B * n_out)
         q.matvec_device(px, B, py)
         np.testing.assert_array_equal(q.matvec(x), hip.download(py, (B, n_out)), err_msg=str(B))
+    q.close()
+    hip.close()
+
+
+# The same where the matvec kernel permutes x, which is then copied in one part and in two: every column by itself.
+@pytest.mark.parametrize("n_in,G,batches", [(2048, 64, (63, 64, 65)), (8192, 128, (15, 17))])
+def test_host_columns_are_the_device_columns(ops, n_in, G, batches):
+    from llama2_rs import _lib
+    hip = _Hip()
+    rng = np.random.default_rng(n_in)
+    q = ops.QLinear(*ck.synth_qlinear(rng, n_in, 264, G, act_order=True), G)
+    q.set_mode(_lib.PREFILL_COLUMNS)
+    for B in batches:
+        x = rng.standard_normal((B, n_in)).astype(np.float32)
+        px, py = hip.upload(x), hip.empty(4 * B * 264)
+        q.matvec_device(px, B, py)
+        np.testing.assert_array_equal(q.matvec(x), hip.download(py, (B, 264)), err_msg=str(B))
     q.close()
     hip.close()
 
