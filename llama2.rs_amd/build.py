@@ -24,7 +24,8 @@ COMMON = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function", f"--off
 SOURCES = {
     # file: extra flags
     "kernels_q4.hip": [],
-    "kernels_q4_stream.hip": [],
+    # the leading arguments of its kernels arrive in scalar registers
+    "kernels_q4_stream.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=14"],
     # MFMA accumulators in VGPRs: the per-group fold reads and writes them with plain FMAs
     "kernels_q4_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "kernels_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1", "-ffp-contract=off"],

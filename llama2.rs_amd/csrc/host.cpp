@@ -2335,6 +2335,7 @@ extern "C" int l2_model_q4_kernels(l2_model *m, char *out, size_t cap) {
     items[1].cls = "q4_wo";
     items[1].L = launch_of(wo, 1, 0.f);
     items[1].L.m[0] = mat_of(wo, some, nullptr, nullptr);
+    items[1].L.e.kind = Q4_EPI_RESIDUAL;
     items[2].cls = "q4_w13";
     items[2].L = launch_of(w1, 1, m->rms_eps);
     items[2].L.m[0] = mat_of(w1, some, some, nullptr);
@@ -2344,6 +2345,7 @@ extern "C" int l2_model_q4_kernels(l2_model *m, char *out, size_t cap) {
     items[3].cls = "q4_w2";
     items[3].L = launch_of(w2, 1, 0.f);
     items[3].L.m[0] = mat_of(w2, some, nullptr, nullptr);
+    items[3].L.e.kind = Q4_EPI_RESIDUAL;
     std::string all;
     for (auto &it : items) {
         char name[160] = "";

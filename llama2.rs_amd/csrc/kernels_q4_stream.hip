@@ -149,26 +149,29 @@ __device__ __forceinline__ T pin_s(T v) {
     return v;
 }
 
-// The operands of one matrix of a launch, in scalar registers.
+// The operands of one matrix of a launch.
 struct MatOps {
     const uint4 *qweight;
     const int32_t *qzeros;
     const float *scales;
-    const float *x;
-    const int32_t *gidx;
-    const float *wn;
     float *y;
     int out;
 };
 
-__device__ __forceinline__ MatOps mat_ops(const Q4Mat &M) {
+// What a launch passes besides the leading arguments (see q4_stream_kernel).
+struct StreamArgs {
+    MatOps m[3];
+    Q4Epi e;
+    int groups, rows_per_block;
+    float eps;
+};
+
+// A matrix's operands, in scalar registers.
+__device__ __forceinline__ MatOps mat_ops(const MatOps &M) {
     MatOps o;
     o.qweight = pin_s(M.qweight);
     o.qzeros = pin_s(M.qzeros);
     o.scales = pin_s(M.scales);
-    o.x = pin_s(M.x);
-    o.gidx = pin_s(M.gidx);
-    o.wn = pin_s(M.wn);
     o.y = pin_s(M.y);
     o.out = pin_s(M.out);
     return o;
@@ -252,21 +255,32 @@ __device__ __forceinline__ float chunk_sum(const float (&s4)[8]) {
     return ((s4[0] + s4[1]) + (s4[2] + s4[3])) + ((s4[7] + s4[6]) + (s4[5] + s4[4]));
 }
 
+// The leading arguments are what the loads of x need: x of the launch's matrices (blocks0 and blocks1 of the grid belong to the
+// first and second), the norm weights of the first, those of the others behind it, or null, and the inverse of g_index of the
+// gathering form.  The dispatch puts them into scalar registers (-amdgpu-kernarg-preload-count), so x is asked for while the
+// rest of the arguments, cold in the scalar cache, is still on its way.  In a chain of dependent kernels that is 0.15 us of each
+// (8 MB 3.57 -> 3.43 us, 46 MB 10.08 -> 9.92); 8 layers of 7B, a token 378.6 -> 373.3 us.
+//
 // MODE 0: fp32 inner loop, x staged through LDS (rmsnorm prologue, several matrices, row pairs).
 // MODE 1: integer-dot inner loop, x staged and quantised in LDS.
 // MODE 2: fp32 inner loop, one matrix without rmsnorm: every wave loads its own slice of x (coalesced)
 //         and turns it into the per-lane chunks through LDS of its own; no barrier before the first row.
+// MODE 3: MODE 0, a block doing the work of two of half its waves (see two_in_one).
 // GATHER (MODE 0, one matrix, no rmsnorm): x arrives in its natural order and the kernel applies the act-order
 //         permutation itself, x[g_index[j]] (src/gptq.rs:99-122), for a caller with no producer to do it: x and the
 //         inverse of g_index are requested together and every element is written straight to its place in the
 //         staged chunks (the scatter a producer's epilogue would have done); the chunk sums are taken by the lanes.
 template <int G, int NWK, int S, bool PAIR, int MODE, int P, bool GATHER = false>
-__global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const Q4Launch L) {
-    constexpr bool IDOT = MODE == 1, DIRECT = MODE == 2;
+__global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const float *x0, const float *x1, const float *x2, const float *wn0,
+                                                                const int32_t *gidx, const int in, const int blocks0, const int blocks1,
+                                                                const StreamArgs L) {
+    constexpr bool IDOT = MODE == 1, DIRECT = MODE == 2, TWO = MODE == 3;
     static_assert(!GATHER || (MODE == 0 && !PAIR), "the gathering form takes one matrix through the block-wide staging");
     static_assert(!(DIRECT && PAIR), "the direct form takes one matrix");
+    static_assert(!(TWO && PAIR), "two blocks in one: single rows");
     constexpr int NM = PAIR ? 2 : 1;
     constexpr int NW = NWK * S;
+    constexpr int NWX = TWO ? NW / 2 : NW; // the waves that stage x (the sum of squares has the order of so many)
     // P rows (row pairs) are in flight per stream
     constexpr int TR = P * S;       // rows per reduction tile
     constexpr int PW = NWK * 4;     // partials per row
@@ -275,12 +289,68 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const Q4Launch L
     __shared__ float red[NW];
     __shared__ float part[2][TR][NM][PW];
 
-    // Every scalar operand the prologue needs is asked for here, at once, and pinned in SGPRs: a kernel's
+    const int b = blockIdx.y;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    // the wave's number as a scalar: the row a wave works on, and with it the row's part of every address and
+    // the shift that extracts its zero point, are then scalar arithmetic, off the vector ALU
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kslice = wave % NWK;
+    const int stream = wave / NWK;
+    constexpr int NC = NWK * 64;                 // chunks the waves of a row cover
+    constexpr int xstride = NC * kChunkPad + NC; // floats of LDS per staged vector
+    constexpr int NX = (8 * NWK + NWX - 1) / NWX; // pieces of x per thread of the NWX waves that stage it
+    const bool stages = NWX == NW || wave < NWX;
+
+    // Which matrix the block's rows belong to.
+    int rb = blockIdx.x, mi = 0;
+    const float *x_of[2] = {x0, x1};
+    if constexpr (!PAIR) {
+        if (rb >= blocks0) {
+            rb -= blocks0;
+            mi = 1;
+            x_of[0] = x1;
+            if (rb >= blocks1) {
+                rb -= blocks1;
+                mi = 2;
+                x_of[0] = x2;
+            }
+        }
+    }
+    const bool has_wn = wn0 != nullptr;
+
+    // x first, then the first rows of the weights: loads return in order, and
+    // the staging of x (a cache hit) must not queue behind rows that come from HBM.
+    XRegs<NX> xr[DIRECT ? 1 : NM];
+    float4 xd[DIRECT ? 8 : 1];
+    int4 gi[GATHER ? NX : 1];
+    if constexpr (GATHER) {
+        const int n4 = in >> 2;
+        const int4 *g4 = reinterpret_cast<const int4 *>(gidx);
+#pragma unroll
+        for (int u = 0; u < NX; u++) {
+            const int j4 = u * (NW * 64) + tid;
+            gi[u] = j4 < n4 ? g4[j4] : make_int4(0, 0, 0, 0);
+        }
+    }
+    if constexpr (DIRECT) {
+        // this wave's 64 chunks of x, 1 KB per load instruction (whole cache lines); past the end the last
+        // 16 bytes are re-read and zeroed below
+        const float4 *x4 = reinterpret_cast<const float4 *>(x0 + (size_t)b * in);
+        const int n4 = in >> 2;
+#pragma unroll
+        for (int i = 0; i < 8; i++) xd[i] = x4[min(kslice * 512 + i * 64 + lane, n4 - 1)];
+    } else if (stages) {
+#pragma unroll
+        for (int q = 0; q < NM; q++)
+            x_issue<NWX, NX>(x_of[q] + (size_t)b * in, has_wn ? wn0 + (size_t)(mi + q) * in : nullptr, in, tid, xr[q]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+
+    // Every other scalar operand is asked for at once, and pinned in SGPRs: a kernel's
     // arguments are cold in the scalar cache, a load that misses takes some 0.3 us, and loads the compiler
     // places where their values are first used follow each other (the matrix of this block, then its
     // pointers, then the row geometry: three round trips in front of the first weight load).
-    const int in = pin_s(L.in);
-    const int n_mats = pin_s(L.n_mats);
     const int groups = pin_s(L.groups);
     const int rows_per_block = pin_s(L.rows_per_block);
     const float eps = pin_s(L.eps);
@@ -291,36 +361,18 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const Q4Launch L
     const int32_t *__restrict__ sc_idx[3] = {pin_s(L.e.sc_idx[0]), pin_s(L.e.sc_idx[1]), pin_s(L.e.sc_idx[2])};
     float *__restrict__ sc_out[3] = {pin_s(L.e.sc_out[0]), pin_s(L.e.sc_out[1]), pin_s(L.e.sc_out[2])};
     MatOps mat[NM];
-    int rb = blockIdx.x;
     if constexpr (PAIR) {
         mat[0] = mat_ops(L.m[0]);
         mat[1] = mat_ops(L.m[1]);
     } else {
         const MatOps m0 = mat_ops(L.m[0]), m1 = mat_ops(L.m[1]), m2 = mat_ops(L.m[2]);
-        const int rb0 = pin_s(L.m[0].row_blocks), rb1 = pin_s(L.m[1].row_blocks);
         mat[0] = m0;
-        if (n_mats > 1 && rb >= rb0) {
-            rb -= rb0;
+        if (mi > 0) {
             mat[0] = m1;
-            if (n_mats > 2 && rb >= rb1) {
-                rb -= rb1;
-                mat[0] = m2;
-            }
+            if (mi > 1) mat[0] = m2;
         }
     }
     const int C = in >> 5;
-    constexpr int NC = NWK * 64;                 // chunks the waves of a row cover
-    constexpr int xstride = NC * kChunkPad + NC; // floats of LDS per staged vector
-    constexpr int NX = (8 + S - 1) / S;          // pieces of x per thread
-
-    const int b = blockIdx.y;
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    // the wave's number as a scalar: the row a wave works on, and with it the row's part of every address and
-    // the shift that extracts its zero point, are then scalar arithmetic, off the vector ALU
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int kslice = wave % NWK;
-    const int stream = wave / NWK;
     const int n_out = mat[0].out;
     const int row0 = rb * rows_per_block;
     const int row1 = min(row0 + rows_per_block, n_out);
@@ -354,31 +406,7 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const Q4Launch L
         }
     };
 
-    // x first, then the first rows of the weights: loads return in order, and
-    // the staging of x (a cache hit) must not queue behind rows that come from HBM.
-    XRegs<NX> xr[DIRECT ? 1 : NM];
-    float4 xd[DIRECT ? 8 : 1];
-    int4 gi[GATHER ? NX : 1];
-    if constexpr (GATHER) {
-        const int n4 = in >> 2;
-        const int4 *g4 = reinterpret_cast<const int4 *>(mat[0].gidx);
-#pragma unroll
-        for (int u = 0; u < NX; u++) {
-            const int j4 = u * (NW * 64) + tid;
-            gi[u] = j4 < n4 ? g4[j4] : make_int4(0, 0, 0, 0);
-        }
-    }
-    if constexpr (DIRECT) {
-        // this wave's 64 chunks of x, 1 KB per load instruction (whole cache lines); past the end the last
-        // 16 bytes are re-read and zeroed below
-        const float4 *xp = reinterpret_cast<const float4 *>(mat[0].x + (size_t)b * in);
-        const int n4 = in >> 2;
-#pragma unroll
-        for (int i = 0; i < 8; i++) xd[i] = xp[min(kslice * 512 + i * 64 + lane, n4 - 1)];
-    } else {
-#pragma unroll
-        for (int q = 0; q < NM; q++)
-            x_issue<NW, NX>(mat[q].x + (size_t)b * in, mat[q].wn, in, tid, xr[q]);
+    if constexpr (!DIRECT) {
         // No wave of the block asks for weights before every wave has asked for its piece of x: a CU returns
         // loads in the order it received them, and a piece of x (a cache hit) requested behind another wave's
         // first rows (HBM) would hold up the staging of the whole block until those rows are in.
@@ -420,7 +448,7 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const Q4Launch L
     float sx[NM];     // fp32 form: sum of the chunk's x; integer form: sum of its q
     float xdelta[NM]; // integer form: the chunk's step
     float ss = 1.0f;
-    const bool norm = !DIRECT && mat[0].wn != nullptr;
+    const bool norm = !DIRECT && has_wn;
     if constexpr (DIRECT) {
         // Turned through a region of LDS of the wave's own, from "lane l holds floats 4l..4l+3 of every 256"
         // to "lane l holds its chunk's 32": no block barrier (a wave's LDS accesses execute in order).
@@ -450,37 +478,38 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const Q4Launch L
     } else {
         // stage x for the whole block, then take this lane's chunk into registers
         float ssq = 0.f;
+        if (stages) {
 #pragma unroll
-        for (int q = 0; q < NM; q++) {
-            const MatOps &M = mat[q];
-            float *xs = lds + q * xstride;
-            float p = 0.f;
-            if constexpr (GATHER) {
-                const int n4 = in >> 2;
+            for (int q = 0; q < NM; q++) {
+                float *xs = lds + q * xstride;
+                float p = 0.f;
+                if constexpr (GATHER) {
+                    const int n4 = in >> 2;
 #pragma unroll
-                for (int u = 0; u < NX; u++) {
-                    const int j4 = u * (NW * 64) + tid;
-                    if (j4 < n4) { // element 4 j4 + e of x is input gi[u].e of the sorted rows
-                        xs[(gi[u].x >> 5) * kChunkPad + (gi[u].x & 31)] = xr[q].v[u].x;
-                        xs[(gi[u].y >> 5) * kChunkPad + (gi[u].y & 31)] = xr[q].v[u].y;
-                        xs[(gi[u].z >> 5) * kChunkPad + (gi[u].z & 31)] = xr[q].v[u].z;
-                        xs[(gi[u].w >> 5) * kChunkPad + (gi[u].w & 31)] = xr[q].v[u].w;
+                    for (int u = 0; u < NX; u++) {
+                        const int j4 = u * (NW * 64) + tid;
+                        if (j4 < n4) { // element 4 j4 + e of x is input gi[u].e of the sorted rows
+                            xs[(gi[u].x >> 5) * kChunkPad + (gi[u].x & 31)] = xr[q].v[u].x;
+                            xs[(gi[u].y >> 5) * kChunkPad + (gi[u].y & 31)] = xr[q].v[u].y;
+                            xs[(gi[u].z >> 5) * kChunkPad + (gi[u].z & 31)] = xr[q].v[u].z;
+                            xs[(gi[u].w >> 5) * kChunkPad + (gi[u].w & 31)] = xr[q].v[u].w;
+                        }
                     }
+                } else {
+                    p = x_stage<NWK, NWX, NX>(norm, tid, xr[q], xs, xs + NC * kChunkPad);
                 }
-            } else {
-                p = x_stage<NWK, NW, NX>(M.wn != nullptr, tid, xr[q], xs, xs + NC * kChunkPad);
+                if (q == 0) ssq = p;
             }
-            if (q == 0) ssq = p;
-        }
-        if (norm) {
-            ssq = wave_sum(ssq);
-            if (lane == 0) red[wave] = ssq;
+            if (norm) {
+                ssq = wave_sum(ssq);
+                if (lane == 0) red[wave] = ssq;
+            }
         }
         __syncthreads();
         if (norm) { // rmsnorm scale, src/models.rs:55-60
             float t = 0.f;
 #pragma unroll
-            for (int i = 0; i < NW; i++) t += red[i];
+            for (int i = 0; i < NWX; i++) t += red[i];
             t /= (float)in;
             t += eps;
             ss = 1.0f / sqrtf(t);
@@ -549,6 +578,10 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const Q4Launch L
     const int n_full = n_steps / P;
     const int n_rem = n_steps - n_full * P;
     int buf = 0;
+    // A block that does the work of two: the rows of each half that would stand behind the loop of a block of their own.
+    const int row_half = row0 + rows_per_block / 2;
+    auto behind = [](int rows) { return (rows + S / 2 - 1) / (P * S / 2) * (P * S / 2); };
+    const int behind0 = TWO ? behind(min(rows_per_block / 2, n_rows)) : 0, behind1 = TWO ? behind(max(row1 - row_half, 0)) : 0;
     // The second half of the rows, and a wait for the first, which arrived while x was staged.  The compiler's wait
     // counts inside the loop are then those of the steady state alone: vmcnt leaves the P - 1 younger rows in
     // flight.  Otherwise the issue order of the prologue leaks into the loop's waits.
@@ -573,7 +606,14 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const Q4Launch L
             } else {
                 const float p = chunk_dot(d[q].w, x[q]);
                 // -(zn + 1) sx as one FMA on the converted nibble (the same real number, rounded once either way)
-                pr[q] = d[q].s * fmaf(p, 512.0f, fmaf((float)zn, nsx[q], nsx[q]));
+                const float f = fmaf(p, 512.0f, fmaf((float)zn, nsx[q], nsx[q]));
+                pr[q] = d[q].s * f;
+                if constexpr (TWO) { // with the first addition across lanes, rounded as in a block of half the rows
+                    asm volatile("" : "+v"(pr[q]));
+                    const float other = dpp_xchg<0xB1>(pr[q]);
+                    const int half = o >= row_half ? o - row_half : o - row0;
+                    pr[q] = half >= (o >= row_half ? behind1 : behind0) ? fmaf(d[q].s, f, other) : pr[q] + other;
+                }
             }
         }
     };
@@ -582,7 +622,7 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const Q4Launch L
 #pragma unroll
         for (int q = 0; q < NM; q++) {
             float v = pr[q];
-            v += dpp_xchg<0xB1>(v);
+            if constexpr (!TWO) v += dpp_xchg<0xB1>(v);
             v += dpp_xchg<0x4E>(v);
             v += dpp_xchg<0x141>(v);
             v += dpp_xchg<0x140>(v);
@@ -701,15 +741,32 @@ static bool whole_tiles(const Q4Launch &L, int NWK, int S, int P) {
     return true;
 }
 
+// Whether two blocks of eight waves (rows of two) run as one of sixteen.  A CU returns loads in the order it received them, so of two
+// blocks on a CU the second has its x behind the first rows of the other's weights: with time stamps in 7B's q|k|v the one had x
+// staged 1.2 us after the launch and was through at 5.2, the other at 2.3 and 6.4.  In one block all of x is asked for in front of all
+// weights: 8 layers of 7B, a token 378 -> 371 us, q|k|v 4.2 of them, wo 1.8.  So where CUs would get two of them; not for several
+// columns, which are more blocks than a CU holds at once.  A row is the same bits either way: the sum of squares is taken by eight
+// waves, and the rows that stand behind the loop in a block of eight waves keep that rounding.
+static bool two_in_one(const Q4Launch &L) {
+    if (L.batch != 1 || (!L.m[0].wn && L.e.kind != Q4_EPI_RESIDUAL)) return false;
+    int total = 0, halves = 0;
+    const int rpb = plan_rows(L, 8, 8, staging_lds(2, false), false, &total);
+    for (int i = 0; i < L.n_mats; i++) halves += (L.m[i].out + 2 * rpb - 1) / (2 * rpb);
+    return total > cu_count() && halves <= cu_count();
+}
+
 template <int G, int NWK, int S, bool PAIR, int MODE, int P = (PAIR ? 2 : 4), bool GATHER = false>
 int launch_s(Q4Launch &L, hipStream_t stream) {
     constexpr int NW = NWK * S;
     constexpr int TR = P * S;
+    constexpr bool TWO = MODE == 3;
     const size_t lds = MODE == 2 ? (size_t)NW * 64 * kChunkPad * sizeof(float)
                                  : staging_lds(NWK, PAIR);
     if (lds + 8 * 1024 > 160 * 1024) return l2_fail(L2_ERR_ARG, "q4 matvec: in=%d needs %zu B of LDS", L.in, lds);
     int total = 0;
-    const int rpb = plan_rows(L, NW, TR, lds, PAIR, &total);
+    const int rpb = TWO ? 2 * plan_rows(L, NW / 2, TR / 2, lds, PAIR, nullptr) : plan_rows(L, NW, TR, lds, PAIR, &total);
+    if (TWO)
+        for (int i = 0; i < L.n_mats; i++) total += (L.m[i].out + rpb - 1) / rpb;
     L.rows_per_block = rpb;
     for (int i = 0; i < L.n_mats; i++) L.m[i].row_blocks = (L.m[i].out + rpb - 1) / rpb;
     auto kern = q4_stream_kernel<G, NWK, S, PAIR, MODE, P, GATHER>;
@@ -724,12 +781,19 @@ int launch_s(Q4Launch &L, hipStream_t stream) {
         static LdsLimit limit; // per instantiation
         L2_TRY(limit.ensure(reinterpret_cast<const void *>(kern), lds));
     }
+    for (int i = 1; i < L.n_mats; i++) // the kernel finds them behind those of the first
+        if (L.m[i].wn != (L.m[0].wn ? L.m[0].wn + (size_t)i * L.in : nullptr)) return l2_fail(L2_ERR_ARG, "q4 matvec: norm weights apart");
     dim3 grid(total, L.batch), block(NW * 64);
+    StreamArgs a{};
+    for (int i = 0; i < L.n_mats; i++) a.m[i] = {L.m[i].qweight, L.m[i].qzeros, L.m[i].scales, L.m[i].y, L.m[i].out};
+    a.e = L.e, a.groups = L.groups, a.rows_per_block = rpb, a.eps = L.eps;
+    const Q4Mat *const m = L.m;
     if (g_q4_prof.armed) {
         g_q4_prof.armed = false;
-        hipExtLaunchKernelGGL(kern, grid, block, lds, stream, g_q4_prof.start, g_q4_prof.stop, 0, L);
+        hipExtLaunchKernelGGL(kern, grid, block, lds, stream, g_q4_prof.start, g_q4_prof.stop, 0, m[0].x, m[1].x, m[2].x, m[0].wn, m[0].gidx, L.in,
+                              m[0].row_blocks, m[1].row_blocks, a);
     } else {
-        hipLaunchKernelGGL(kern, grid, block, lds, stream, L);
+        hipLaunchKernelGGL(kern, grid, block, lds, stream, m[0].x, m[1].x, m[2].x, m[0].wn, m[0].gidx, L.in, m[0].row_blocks, m[1].row_blocks, a);
     }
     L2_HIP(hipGetLastError());
     return L2_OK;
@@ -788,7 +852,11 @@ int launch_sg(Q4Launch &L, hipStream_t stream) {
     } else if (!L.pair) {
         switch (nwk) {
             case 1: return rows <= 8 * cus && whole_tiles(L, 1, 4, 4) ? launch_s<G, 1, 8, false, MODE, 1>(L, stream) : launch_s<G, 1, 4, false, MODE>(L, stream);
-            case 2: return rows <= 4 * cus ? launch_s<G, 2, 4, false, MODE, 1>(L, stream) : launch_s<G, 2, 4, false, MODE, 2>(L, stream);
+            case 2:
+                if (rows <= 4 * cus) return launch_s<G, 2, 4, false, MODE, 1>(L, stream);
+                if constexpr (MODE == 0)
+                    if (two_in_one(L)) return launch_s<G, 2, 8, false, 3, 2>(L, stream);
+                return launch_s<G, 2, 4, false, MODE, 2>(L, stream);
             case 3: return launch_s<G, 3, 4, false, MODE>(L, stream);
             case 4: return launch_s<G, 4, 4, false, MODE, 2>(L, stream); // 8192: rows of 4 KB; two in flight per stream measured faster than four (q|k|v 13.4 -> 12.2 us, wo 12.1 -> 10.9)
             case 5: case 6: return launch_s<G, 6, 2, false, MODE, 3>(L, stream);

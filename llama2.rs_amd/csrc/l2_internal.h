@@ -134,7 +134,7 @@ struct Q4Mat {
     const float *x;  // input already in this layer's g_index order: [B][in] (in its natural order if gidx is set)
     const int32_t *gidx; // null, or the INVERSE of this layer's g_index: x is in its natural order and the kernel puts
                          // x[b][i] where input gidx[i] of the sorted rows is read (one matrix, no rmsnorm)
-    const float *wn; // rmsnorm weights in the same order, or null: x is used as it is
+    const float *wn; // rmsnorm weights in the same order, or null: x is used as it is (a launch's matrices have theirs one behind the other)
     float *y;        // [B][out]
     int out;
     int row_blocks;  // blocks of grid.x that belong to this matrix

@@ -126,6 +126,26 @@ def test_qmatvec_columns_are_the_bits_of_one(ops, n_in, G, n_out, batches):
     hip.close()
 
 
+# The blocks of a single step's launches may do the work of two of those that a batch's columns have (rows of two waves: 2049 to 4096
+# inputs): the same bits, with rows that stand behind the loop of the smaller block (q|k|v of 4096 and 3072, w2 of 4480) and without.
+# Keys and values of the second layer hold what all projections of the first one gave.
+@pytest.mark.parametrize("dim,hidden,heads,kv,G", [(4096, 2816, 32, 32, 128), (4096, 2816, 32, 8, 64), (3072, 4096, 24, 24, 32),
+                                                   (4480, 4096, 35, 35, 32)])
+def test_single_step_has_the_projection_bits_of_columns(ops, dim, hidden, heads, kv, G):
+    from llama2_rs import _lib
+    d = ck.Dims(dim=dim, hidden_dim=hidden, n_layers=2, n_heads=heads, n_kv_heads=kv, vocab_size=64, seq_len=16, group_size=G)
+    m = ops.Model(ops.synth_image(d, 5), d)
+    m.forward([3], [0])
+    one = [m.read_kv(layer, 0, 1) for layer in range(2)]
+    m.reset()
+    m.set_prefill_mode(_lib.PREFILL_COLUMNS)
+    m.forward([3, 9], [0, 1], want_logits=False)
+    for layer in range(2):
+        for name, a, b in zip("kv", one[layer], m.read_kv(layer, 0, 1)):
+            np.testing.assert_array_equal(a, b, err_msg=f"layer {layer}, {name}")
+    m.close()
+
+
 _ALT_FORM_SNIPPET = r"""
 import sys, numpy as np
 sys.path.insert(0, sys.argv[1]); sys.path.insert(0, sys.argv[2])
