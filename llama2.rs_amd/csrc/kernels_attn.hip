@@ -1124,7 +1124,7 @@ __global__ __launch_bounds__(512) void attn_combine_kernel(const AttnDecode A) {
 
 template <int QG, int NWV, int DS>
 int attn_launch_sliced(const AttnDecode &a, hipStream_t st) {
-    hipLaunchKernelGGL((attn_decode_kernel<QG, NWV, DS>), dim3(a.n_kv_heads, 1, DS), dim3(NWV * 64), 0, st, a);
+    l2_launch((attn_decode_kernel<QG, NWV, DS>), dim3(a.n_kv_heads, 1, DS), dim3(NWV * 64), 0, st, a);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }
@@ -1144,7 +1144,7 @@ int attn_launch_qg(const AttnDecode &a, hipStream_t st) {
             return v && !strcmp(v, "valu");
         }();
         if (!valu) {
-            hipLaunchKernelGGL((attn_decode_mfma_kernel<QG>), dim3(a.n_kv_heads, a.n_splits), dim3(256), 0, st, a);
+            l2_launch((attn_decode_mfma_kernel<QG>), dim3(a.n_kv_heads, a.n_splits), dim3(256), 0, st, a);
             L2_HIP(hipGetLastError());
             return L2_OK;
         }
@@ -1154,7 +1154,7 @@ int attn_launch_qg(const AttnDecode &a, hipStream_t st) {
         static LdsLimit limit; // per instantiation
         L2_TRY(limit.ensure(reinterpret_cast<const void *>(attn_decode_kernel<QG, 4, 1>), lds));
     }
-    hipLaunchKernelGGL((attn_decode_kernel<QG, 4, 1>), dim3(a.n_kv_heads, a.n_splits), dim3(256), lds, st, a);
+    l2_launch((attn_decode_kernel<QG, 4, 1>), dim3(a.n_kv_heads, a.n_splits), dim3(256), lds, st, a);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }
@@ -1177,7 +1177,7 @@ int attention_decode_launch(const AttnDecode &a, hipStream_t st) {
                              : a.n_splits <= 16 ? attn_combine_kernel<4>
                              : a.n_splits <= 32 ? attn_combine_kernel<8>
                                                 : attn_combine_kernel<16>;
-        hipLaunchKernelGGL(combine, dim3(a.n_heads), dim3(512), 0, st, a);
+        l2_launch(combine, dim3(a.n_heads), dim3(512), 0, st, a);
         L2_HIP(hipGetLastError());
     }
     return L2_OK;
@@ -1195,12 +1195,12 @@ static int prefill_qg(void *out, int planes, const float *q, const float *kc, co
     const int unit_rows = cus % n_kv_heads == 0 && rows > per_unit && rows <= 2 * per_unit ? per_unit : 0; // see column_tile
 #define L2_PREFILL_ATTN(NP)                                                                                              \
     if (two)                                                                                                             \
-        hipLaunchKernelGGL((attn_prefill_mfma16_kernel<QG, 4, NP, 2>), grid, block, 0, st, out, q, kc, vc, pos, scatter, n_heads, n_kv_heads, B, max_pos, unit_rows); \
+        l2_launch((attn_prefill_mfma16_kernel<QG, 4, NP, 2>), grid, block, 0, st, out, q, kc, vc, pos, scatter, n_heads, n_kv_heads, B, max_pos, unit_rows); \
     else                                                                                                                 \
-        hipLaunchKernelGGL((attn_prefill_mfma16_kernel<QG, 4, NP, 1>), grid, block, 0, st, out, q, kc, vc, pos, scatter, n_heads, n_kv_heads, B, max_pos, unit_rows); \
+        l2_launch((attn_prefill_mfma16_kernel<QG, 4, NP, 1>), grid, block, 0, st, out, q, kc, vc, pos, scatter, n_heads, n_kv_heads, B, max_pos, unit_rows); \
     break
     switch (planes) {
-        case 0: hipLaunchKernelGGL(attn_prefill_kernel<QG>, dim3(n_kv_heads, (B * QG + 7) / 8), block, 0, st, (float *)out, q, kc, vc, pos, scatter, n_heads, n_kv_heads, B); break;
+        case 0: l2_launch(attn_prefill_kernel<QG>, dim3(n_kv_heads, (B * QG + 7) / 8), block, 0, st, (float *)out, q, kc, vc, pos, scatter, n_heads, n_kv_heads, B); break;
         case 1: L2_PREFILL_ATTN(1);
         case 3: L2_PREFILL_ATTN(3);
         default: return l2_fail(L2_ERR_ARG, "attention: %d planes", planes);

@@ -1054,7 +1054,7 @@ int launch_tile(const Q4Launch &L, const XhList &xh, const float *ss, float *ws,
             if (total * KS * per - at <= cus) whole = begun * t_tiles + done, width = w, blocks = whole + total * KS * per - at;
         }
     }
-    hipLaunchKernelGGL((q4_tile_gemm_kernel<G, NT, NW>), dim3(blocks), dim3(64 * NW), lds, st, L, xh, gemm_padded(L.in), ss, ws, KS, t_tiles, total, whole,
+    l2_launch((q4_tile_gemm_kernel<G, NT, NW>), dim3(blocks), dim3(64 * NW), lds, st, L, xh, gemm_padded(L.in), ss, ws, KS, t_tiles, total, whole,
                        width, partials);
     L2_HIP(hipGetLastError());
     return L2_OK;
@@ -1082,7 +1082,7 @@ int launch_dense(const Q4Launch &L, const XhList &xh, const float *ss, float *ws
     const size_t lds = DenseLds<NT>::kSize;
     L2_TRY(limit.ensure(reinterpret_cast<const void *>(dense_gemm_kernel<NT>), lds));
     const int t_tiles = (L.batch + 16 * NT - 1) / (16 * NT);
-    hipLaunchKernelGGL(dense_gemm_kernel<NT>, dim3(s.row_blocks * t_tiles * s.slices), dim3(64 * kDenseWaves), lds, st, L, xh, gemm_padded(L.in), ss, ws, s.slices, t_tiles, partials);
+    l2_launch(dense_gemm_kernel<NT>, dim3(s.row_blocks * t_tiles * s.slices), dim3(64 * kDenseWaves), lds, st, L, xh, gemm_padded(L.in), ss, ws, s.slices, t_tiles, partials);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }
@@ -1182,7 +1182,7 @@ int gemm_launch(Q4Launch &L, const XhList &xh, const float *ss, float *ws, size_
         return L2_OK;
     }
     if (s.slices > 1) {
-        hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)((rows + 1023) / 1024), L.batch), dim3(256), 0, st, L.m[0].y, ws,
+        l2_launch(gemm_reduce_kernel, dim3((unsigned)((rows + 1023) / 1024), L.batch), dim3(256), 0, st, L.m[0].y, ws,
                            L.e.kind == Q4_EPI_RESIDUAL ? L.e.res : nullptr, ss, L.m[0].out, L.batch, s.slices);
         L2_HIP(hipGetLastError());
     }
@@ -1193,7 +1193,7 @@ size_t group_tiles_floats(int out, int groups) { return (size_t)((out + 31) / 32
 
 int group_tiles_launch(const float *scales, const int32_t *qzeros, int out, int groups, float *tiles, hipStream_t st) {
     const int row_tiles = (out + 31) / 32;
-    hipLaunchKernelGGL(group_tiles_kernel, dim3(row_tiles, (groups + 31) / 32), dim3(256), 0, st, scales, qzeros, out, groups, tiles,
+    l2_launch(group_tiles_kernel, dim3(row_tiles, (groups + 31) / 32), dim3(256), 0, st, scales, qzeros, out, groups, tiles,
                        reinterpret_cast<int32_t *>(tiles + (size_t)row_tiles * groups * 32));
     L2_HIP(hipGetLastError());
     return L2_OK;
@@ -1213,9 +1213,9 @@ int gemm_input_launch(const GemmInput &A, int n, int B, int planes, hipStream_t 
     const int in_p = gemm_padded(n);
     const dim3 grid((in_p / 8 + 255) / 256, B, A.n);
     if (planes == 1)
-        hipLaunchKernelGGL(gemm_input_kernel<1>, grid, dim3(256), 0, st, A, n, in_p);
+        l2_launch(gemm_input_kernel<1>, grid, dim3(256), 0, st, A, n, in_p);
     else
-        hipLaunchKernelGGL(gemm_input_kernel<3>, grid, dim3(256), 0, st, A, n, in_p);
+        l2_launch(gemm_input_kernel<3>, grid, dim3(256), 0, st, A, n, in_p);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }
@@ -1224,9 +1224,9 @@ int host_input_launch(void *out, const float *x, const int32_t *inv, int n, int 
     if (n % 32 || n < 32 || B < 1 || !inv) return l2_fail(L2_ERR_ARG, "host input: n=%d, %d columns", n, B);
     const dim3 grid((n / 4 + kHostPieces * 256 - 1) / (kHostPieces * 256), B);
     switch (planes) {
-        case 0: hipLaunchKernelGGL(host_input_kernel<0>, grid, dim3(256), 0, st, out, x, inv, n, n); break;
-        case 1: hipLaunchKernelGGL(host_input_kernel<1>, grid, dim3(256), 0, st, out, x, inv, n, gemm_padded(n)); break;
-        case 3: hipLaunchKernelGGL(host_input_kernel<3>, grid, dim3(256), 0, st, out, x, inv, n, gemm_padded(n)); break;
+        case 0: l2_launch(host_input_kernel<0>, grid, dim3(256), 0, st, out, x, inv, n, n); break;
+        case 1: l2_launch(host_input_kernel<1>, grid, dim3(256), 0, st, out, x, inv, n, gemm_padded(n)); break;
+        case 3: l2_launch(host_input_kernel<3>, grid, dim3(256), 0, st, out, x, inv, n, gemm_padded(n)); break;
         default: return l2_fail(L2_ERR_ARG, "host input: %d planes", planes);
     }
     L2_HIP(hipGetLastError());
@@ -1240,7 +1240,7 @@ static int residual_norm(const ResNormPrep &A, hipStream_t st) {
     const size_t lds = (size_t)rows * A.out * sizeof(float);
     static LdsLimit limit(48 * 1024);
     L2_TRY(limit.ensure(reinterpret_cast<const void *>(gemm_residual_norm_kernel<NP, TRIPS, SL>), lds));
-    hipLaunchKernelGGL((gemm_residual_norm_kernel<NP, TRIPS, SL>), dim3(A.B), dim3(1024), lds, st, A, rows);
+    l2_launch((gemm_residual_norm_kernel<NP, TRIPS, SL>), dim3(A.B), dim3(1024), lds, st, A, rows);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }
@@ -1264,10 +1264,10 @@ int gemm_rope_kv_launch(const RopeKvArgs &A, hipStream_t st) {
     if (A.KS < 1 || A.KS > kMaxGemmSlices || A.B < 1 || A.n_heads < A.n_kv_heads)
         return l2_fail(L2_ERR_ARG, "q|k|v epilogue: %d slices, %d tokens", A.KS, A.B);
     const dim3 grid(A.B, (A.n_heads * 16 + A.n_kv_heads * 48 + 511) / 512), block(512); // a thread per eight of q and k, four of v
-    if (A.KS <= 2) hipLaunchKernelGGL(gemm_rope_kv_kernel<2>, grid, block, 0, st, A);
-    else if (A.KS <= 4) hipLaunchKernelGGL(gemm_rope_kv_kernel<4>, grid, block, 0, st, A);
-    else if (A.KS <= 8) hipLaunchKernelGGL(gemm_rope_kv_kernel<8>, grid, block, 0, st, A);
-    else hipLaunchKernelGGL(gemm_rope_kv_kernel<kMaxGemmSlices>, grid, block, 0, st, A);
+    if (A.KS <= 2) l2_launch(gemm_rope_kv_kernel<2>, grid, block, 0, st, A);
+    else if (A.KS <= 4) l2_launch(gemm_rope_kv_kernel<4>, grid, block, 0, st, A);
+    else if (A.KS <= 8) l2_launch(gemm_rope_kv_kernel<8>, grid, block, 0, st, A);
+    else l2_launch(gemm_rope_kv_kernel<kMaxGemmSlices>, grid, block, 0, st, A);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }
@@ -1277,7 +1277,7 @@ static int silu(const SiluArgs &A, hipStream_t st) {
     const size_t lds = (size_t)A.n * sizeof(float);
     static LdsLimit limit(48 * 1024);
     L2_TRY(limit.ensure(reinterpret_cast<const void *>(gemm_silu_kernel<NP, SL>), lds));
-    hipLaunchKernelGGL((gemm_silu_kernel<NP, SL>), dim3(A.B), dim3(1024), lds, st, A);
+    l2_launch((gemm_silu_kernel<NP, SL>), dim3(A.B), dim3(1024), lds, st, A);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }

@@ -360,27 +360,27 @@ __global__ void fill_pattern_kernel(float *p, size_t n, uint64_t seed) {
 int embed_launch(float *x, const float *emb, const TokenSource &src, int dim, int B, const ScatterTargets &t,
                  unsigned long long *amax_key, hipStream_t st) {
     if (t.n < 0 || t.n > 3) return l2_fail(L2_ERR_ARG, "embed: %d targets", t.n);
-    hipLaunchKernelGGL(embed_kernel, dim3((dim + 255) / 256, B), dim3(256), 0, st, x, emb, src, dim, t, amax_key);
+    l2_launch(embed_kernel, dim3((dim + 255) / 256, B), dim3(256), 0, st, x, emb, src, dim, t, amax_key);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }
 
 int sample_weights_launch(float *w, unsigned long long *redo, const float *logits, int n, float temperature,
                           const unsigned long long *amax, hipStream_t st) {
-    hipLaunchKernelGGL(sample_weights_kernel, dim3((n + 255) / 256), dim3(256), 0, st, w, redo, logits, n, temperature, amax);
+    l2_launch(sample_weights_kernel, dim3((n + 255) / 256), dim3(256), 0, st, w, redo, logits, n, temperature, amax);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }
 
 int index_launch(const unsigned long long *amax, int32_t *id, hipStream_t st) {
-    hipLaunchKernelGGL(index_kernel, dim3(1), dim3(64), 0, st, amax, id);
+    l2_launch(index_kernel, dim3(1), dim3(64), 0, st, amax, id);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }
 
 int copy_launch(float *dst, const float *src, size_t n, hipStream_t st) {
     const int n4 = (int)(n / 4); // inputs are multiples of 32 floats
-    hipLaunchKernelGGL(copy_kernel, dim3((n4 + 63) / 64), dim3(64), 0, st, reinterpret_cast<float4 *>(dst), reinterpret_cast<const float4 *>(src), n4);
+    l2_launch(copy_kernel, dim3((n4 + 63) / 64), dim3(64), 0, st, reinterpret_cast<float4 *>(dst), reinterpret_cast<const float4 *>(src), n4);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }
@@ -388,14 +388,14 @@ int copy_launch(float *dst, const float *src, size_t n, hipStream_t st) {
 int clear_rows_launch(float *k, float *v, int layers, size_t stride, size_t n, hipStream_t st) {
     if (n == 0) return L2_OK;
     const size_t n4 = n / 4, per = (n4 + 255) / 256, most = (size_t)(8 * cu_count() / layers + 1);
-    hipLaunchKernelGGL(clear_rows_kernel, dim3((unsigned)(per < most ? per : most), layers, 2), dim3(256), 0, st,
+    l2_launch(clear_rows_kernel, dim3((unsigned)(per < most ? per : most), layers, 2), dim3(256), 0, st,
                        reinterpret_cast<float4 *>(k), reinterpret_cast<float4 *>(v), stride / 4, n4);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }
 
 int gather_launch(float *out, const float *x, const int32_t *g_index, int n, int B, hipStream_t st) {
-    hipLaunchKernelGGL(gather_kernel, dim3((n + 255) / 256, B), dim3(256), 0, st, out, x, g_index, n);
+    l2_launch(gather_kernel, dim3((n + 255) / 256, B), dim3(256), 0, st, out, x, g_index, n);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }
@@ -403,7 +403,7 @@ int gather_launch(float *out, const float *x, const int32_t *g_index, int n, int
 int rope_kv_launch(float *q, const float *k, const float *v, const int32_t *pos, const float *cos_t,
                    const float *sin_t, float *kcache_l, float *vcache_l, int n_heads, int n_kv_heads,
                    int head_size, int B, hipStream_t st) {
-    hipLaunchKernelGGL(rope_kv_kernel, dim3(B), dim3(1024), 0, st, q, k, v, pos, cos_t, sin_t, kcache_l,
+    l2_launch(rope_kv_kernel, dim3(B), dim3(1024), 0, st, q, k, v, pos, cos_t, sin_t, kcache_l,
                        vcache_l, n_heads, n_kv_heads, head_size);
     L2_HIP(hipGetLastError());
     return L2_OK;
@@ -437,7 +437,7 @@ int dense_launch(const DenseArgs &a0, hipStream_t st) {
         static LdsLimit limit;
         L2_TRY(limit.ensure(reinterpret_cast<const void *>(dense_matvec_kernel<32, 1>), lds));
     }
-    auto launch = [&](void (*kernel)(DenseArgs)) { hipLaunchKernelGGL(kernel, grid, block, lds, st, a); };
+    auto launch = [&](void (*kernel)(DenseArgs)) { l2_launch(kernel, grid, block, lds, st, a); };
     switch (KI) {
         case 4: launch(few ? dense_matvec_kernel<4, 2> : dense_matvec_kernel<4, 8>); break;
         case 8: launch(few ? dense_matvec_kernel<8, 1> : dense_matvec_kernel<8, 4>); break;
@@ -459,20 +459,20 @@ int dense_matvec_launch(float *y, const float *w, const float *x, const float *w
 int next_token_launch(const unsigned long long *amax_key, const int32_t *prompt, int n_prompt,
                       int32_t *dpos, int32_t *out_ids, int pos0, int32_t *tok, hipStream_t st,
                       const int32_t *loop_params) {
-    hipLaunchKernelGGL(next_token_kernel, dim3(1), dim3(64), 0, st, amax_key, prompt, n_prompt, dpos,
+    l2_launch(next_token_kernel, dim3(1), dim3(64), 0, st, amax_key, prompt, n_prompt, dpos,
                        out_ids, pos0, tok, loop_params);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }
 
 int set_i32_launch(int32_t *p, int32_t a, int32_t *q, int32_t b, hipStream_t st) {
-    hipLaunchKernelGGL(set_i32_kernel, dim3(1), dim3(64), 0, st, p, a, q, b);
+    l2_launch(set_i32_kernel, dim3(1), dim3(64), 0, st, p, a, q, b);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }
 
 int fill_pattern_launch(float *p, size_t n, uint64_t seed, hipStream_t st) {
-    hipLaunchKernelGGL(fill_pattern_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, p, n, seed);
+    l2_launch(fill_pattern_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, p, n, seed);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }

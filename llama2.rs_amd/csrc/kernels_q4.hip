@@ -237,7 +237,7 @@ int launch_t(Q4Launch &L, hipStream_t stream) {
         g_q4_prof.armed = false;
         hipExtLaunchKernelGGL(kern, grid, block, lds, stream, g_q4_prof.start, g_q4_prof.stop, 0, L);
     } else {
-        hipLaunchKernelGGL(kern, grid, block, lds, stream, L);
+        l2_launch(kern, grid, block, lds, stream, L);
     }
     L2_HIP(hipGetLastError());
     return L2_OK;

@@ -414,7 +414,7 @@ int launch_gemm(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const
     const size_t lds = std::max(GemmLds<G, NW>::size(TN), (size_t)NW * 32 * 36 * sizeof(float));
     static LdsLimit limit(48 * 1024);
     L2_TRY(limit.ensure(reinterpret_cast<const void *>(q4_gemm_kernel<G, NB, NW>), lds));
-    hipLaunchKernelGGL((q4_gemm_kernel<G, NB, NW>), grid, block, lds, st, L, xh, ss, ws, s.slices, partials, row_blocks, t_full, units, extra, width);
+    l2_launch((q4_gemm_kernel<G, NB, NW>), grid, block, lds, st, L, xh, ss, ws, s.slices, partials, row_blocks, t_full, units, extra, width);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }

@@ -793,7 +793,7 @@ int launch_s(Q4Launch &L, hipStream_t stream) {
         hipExtLaunchKernelGGL(kern, grid, block, lds, stream, g_q4_prof.start, g_q4_prof.stop, 0, m[0].x, m[1].x, m[2].x, m[0].wn, m[0].gidx, L.in,
                               m[0].row_blocks, m[1].row_blocks, a);
     } else {
-        hipLaunchKernelGGL(kern, grid, block, lds, stream, m[0].x, m[1].x, m[2].x, m[0].wn, m[0].gidx, L.in, m[0].row_blocks, m[1].row_blocks, a);
+        l2_launch(kern, grid, block, lds, stream, m[0].x, m[1].x, m[2].x, m[0].wn, m[0].gidx, L.in, m[0].row_blocks, m[1].row_blocks, a);
     }
     L2_HIP(hipGetLastError());
     return L2_OK;

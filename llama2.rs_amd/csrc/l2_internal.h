@@ -64,6 +64,17 @@ int l2_fail(int code, const char *fmt, ...) __attribute__((format(printf, 2, 3))
         if (rc_ != L2_OK) return rc_; \
     } while (0)
 
+// A launch, whose error the next hipGetLastError gives.  hipLaunchKernel by itself: `kernel<<<...>>>` and hipLaunchKernelGGL leave the
+// launch's shape with the runtime and fetch it back in a stub (a queued launch of nine arguments 2.65 us of the host, this 2.41).
+template <class... P, class... A>
+inline void l2_launch(void (*kernel)(P...), const dim3 &grid, const dim3 &block, size_t lds, hipStream_t stream, const A &...args) {
+    static_assert(sizeof...(P) == sizeof...(A), "one value per parameter");
+    [&](P... p) {
+        void *at[] = {const_cast<void *>(static_cast<const void *>(&p))...};
+        (void)hipLaunchKernel(reinterpret_cast<const void *>(kernel), grid, block, at, lds, stream);
+    }(args...);
+}
+
 // A kernel's dynamic-LDS limit (hipFuncAttributeMaxDynamicSharedMemorySize), raised when a launch needs more than it
 // was last raised to.  One of these per kernel (a function-local static at the launch site).  The attribute belongs to
 // the kernel as loaded on ONE device, so what was raised is kept per device; model handles on different host threads

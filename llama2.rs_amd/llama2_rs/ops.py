@@ -18,7 +18,15 @@ from . import checkpoint as ck
 
 
 def _p(a: np.ndarray):
-    return a.ctypes.data_as(C.c_void_p)
+    """The address of an array for a C call (which keeps the array meanwhile); data_as takes 2 us for that, its buffer 0.25."""
+    try:
+        return C.byref(C.c_char.from_buffer(a))
+    except (TypeError, ValueError, BufferError):  # read-only, empty, or with strides
+        return a.ctypes.data_as(C.c_void_p)
+
+
+def _address(a):
+    return a if type(a) is int else C.c_void_p(a)
 
 
 def _f32(a):
@@ -94,8 +102,9 @@ class QLinear:
         """The same operator on DEVICE pointers (addresses as integers), enqueued on `stream` (a hipStream_t
         as an integer, 0 = the default stream) without waiting and without allocating anything: for callers
         under graph capture or in a serving loop.  B * in is bounded by the library's fixed scratch."""
-        check(lib().l2_qlinear_matvec_device(self.h, C.c_void_p(x_dev), B, C.c_void_p(y_dev),
-                                             C.c_void_p(stream) if stream else None))
+        rc = lib().l2_qlinear_matvec_device(self.h, _address(x_dev), B, _address(y_dev), _address(stream) if stream else None)
+        if rc:
+            check(rc)
 
     def close(self):
         if self.h:
