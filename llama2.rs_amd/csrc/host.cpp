@@ -1417,20 +1417,22 @@ extern "C" int l2_model_classifier(l2_model *m, const float *x_host, float *y_ho
 // ---------------------------------------------------------------------------
 // transformer<B>
 
-// How the timesteps of a decode step are cut across blocks: not at all in a short context, where with one or
-// two query heads per kv head a head's dimensions are spread over blocks instead.  That takes 512 timesteps where the
-// slices of all heads are blocks for half the CUs (16 kv heads: 23.2 us per layer against 23.5 in splits at 380, 23.8 and
-// 23.7 at 500; 32: 28.5 and 29.2, 29.0 and 29.6; 7B at 400 393 us per token of 8 layers against 402, equal near 850; 13B at
-// 400 575 against 585, equal near 700), and 384 with fewer blocks, whose scan of all keys is the launch (1, 2, 4, 8 kv
-// heads, one query head each, at 380 19.7 / 20.5 / 20.8 / 21.3 against 20.0 / 20.3 / 20.9 / 21.4, at 500 20.3 / 21.3 / 21.9 /
-// 22.0 against 20.0 / 20.4 / 20.9 / 21.6; two query heads 21.0 / 21.5 / 21.9 / 23.0 and 21.1 / 21.4 / 22.0 / 23.1, 21.9 / 22.4 /
-// 23.1 / 23.7 and 21.1 / 21.4 / 22.0 / 23.1).  256 for more query heads: four, 2 kv heads, 3 layers 82.3 against 84.1 at 260,
-// 87.7 against 84.6 at 400.  Beyond that one block per CU where
+// How the timesteps of a decode step are cut across blocks: not at all in a short context, where each query head's dimensions
+// are spread over blocks instead, which every one scans all keys for; splits cost their merge, a launch of their own.  Whole
+// against in splits, us per layer:
+//   a query head per kv head, few of them: up to 640.  1, 4, 8, 16 heads at 510 20.2 / 22.2 / 21.9 / 23.3 and 22.9 / 21.9 / 23.3 / 24.2,
+//   at 800 23.7 / 23.8 / 23.4 / 24.9 and 22.8 / 21.7 / 23.3 / 24.5
+//   several to a kv head, whose blocks share its rows in an L2, and whose splits take longer (the matrix cores, or two chains): up
+//   to 896, 1024 from 32 query heads on.  8 heads of 2 kv heads at 800, 1000 22.8 / 23.6 and 23.6 / 23.4, of 1 23.1 / 23.7 and
+//   23.9 / 24.7; 32 of 4 29.9 / 30.4 and 31.9 / 31.8, of 16 30.5 / 31.2 and 31.5 / 32.2; 64 of 8 38.7 / 39.6 and 40.4 / 40.3
+//   32 heads of 32: 1024, while the rows that an XCD's blocks read fit its L2 (32 KB a timestep: at 800, 1000, 1250 31.8 / 33.7 / 37.8
+//   and 34.8 / 35.5 / 37.1); above 32 kv heads 768 (40 at 640, 800, 1000 36.6 / 39.6 / 44.4 and 38.6 / 39.7 / 41.3)
+// Beyond that one block per CU where
 // the context allows it, at least 64 timesteps each.  (Two per CU, the earlier rule, left some CUs with two blocks
 // and the launch as long as those: 70B behind 4096 positions 18.6 -> 16.5 us per layer, 13B behind 1000 positions
 // 16.7 -> 15.3, 7B unchanged; half a block per CU is slower everywhere.)
 static void attn_split_policy(int n_t, int n_heads, int n_kv_heads, int *ts_out, int *n_splits_out) {
-    const int whole = n_heads / n_kv_heads > 2 ? 256 : 16 * n_kv_heads >= cu_count() ? 512 : 384; // (eight slices per head)
+    const int whole = n_kv_heads > 32 ? 768 : n_heads >= 32 ? 1024 : n_heads > n_kv_heads ? 896 : 640;
     if (n_t <= whole) {
         *ts_out = whole;
         *n_splits_out = 1;

@@ -68,25 +68,28 @@ static_assert(kCombRow * sizeof(float) % 16 == 0, "rows of the merge tiles are w
 
 // Layout of a block: NWV waves x 4 rows of 16 lanes.  One row of lanes handles one timestep at a time, each lane 8
 // of the 128 head dimensions of the key; a block covers 4 NWV timesteps per step and PD steps per tile, all of a
-// tile's loads being issued before its arithmetic.  All QG query heads of the kv head share each K and V load
-// (grouped-query attention, src/models.rs:142-145).
+// tile's loads being issued before its arithmetic.
 //
-// A short context (n_splits == 1) is one block per kv head and slice of 128 / DS output dimensions: every slice
-// computes all scores, and reads and sums only its part of the values, so nothing has to be merged across blocks.  A
-// single block per kv head leaves most CUs idle and is bound by what one CU can fetch (some 100 GB/s) and by the
+// A short context (n_splits == 1, QG = 1) is one block per query head and slice of 128 / DS output dimensions: every
+// slice computes all scores, and reads and sums only its part of the values, so nothing has to be merged across blocks.  A
+// single block per head leaves most CUs idle and is bound by what one CU can fetch (some 110 GB/s, 0.5 us per 100
+// timesteps; asking for the next tile before this one's arithmetic changes nothing) and by the
 // merge of its rows; eight slices read 9/16 of the bytes each and merge an eighth.  7B (32 kv heads), per token of 32
 // layers, one block -> 8 slices: 1241 -> 1215 us at position 16, 1292 -> 1257 at 120; 13B (40 kv heads), 8 layers, 4
 // slices: 566 -> 561 at 190, where 8 (320 blocks) took 570.  4 waves up to one tile of timesteps (position 16: 1215 us
-// against 1227 with 8 waves), 8 beyond (190: 381 against 383 with 8 layers); four query heads have more to merge per
-// wave, there 4 waves are better up to two tiles (100: 76.4 against 77.2 us).  Four query heads through this kernel
-// instead of the matrix cores: 76.6 -> 72.7 us per token of 3 layers at 30, 88 -> 79 at 190; at eight the matrix cores
-// stay ahead (70B: 937 against 940-948 us at 60).
-// Longer contexts are cut into splits of timesteps (DS = 1, 4 waves) that attn_combine_kernel merges.
+// against 1227 with 8 waves), 8 beyond (190: 381 against 383 with 8 layers).  The query heads of one kv head (grouped-query
+// attention, src/models.rs:142-145) are blocks of their own too: they read the same rows out of the same XCD's L2 (blocks are dealt
+// over the XCDs by kv head), and a block has one chain of scores and sums instead of four or eight.  Whole layers, against a block for
+// all heads of the kv head (at 8 of them on the matrix cores), at 50, 100, 240 timesteps: 16 heads of 2 kv heads 22.8 / 24.1 / 27.4 ->
+// 21.9 / 22.6 / 22.9 us, 32 of 4 28.3 / 29.8 / 31.8 -> 25.7 / 25.7 / 26.8, 64 of 8 37.0 / 38.3 / 42.0 -> 35.4 / 35.8 / 36.7.
+// Longer contexts are cut into splits of timesteps (DS = 1, 4 waves) that attn_combine_kernel merges; there all QG query heads
+// of the kv head share each K and V load.
 template <int QG, int NWV, int DS>
 __global__ __launch_bounds__(NWV * 64) void attn_decode_kernel(const AttnDecode A) {
     constexpr int NT = NWV * 64, TSTEP = NWV * 4;
     constexpr int HS = 128, HALF = 64;
     constexpr int VD = HS / DS, VE = VD / 16; // head dimensions of the value that are this block's, and a lane's share
+    static_assert(DS == 1 || QG == 1, "sliced: one head per block");
     constexpr int PD = QG >= 8 ? 2 : 4; // steps in flight and per pass through the phases (4 at 8 heads: over 256 registers, one block per CU, slower)
     __shared__ float qs[QG * HS];
     __shared__ float kvnew[2][HS];
@@ -100,7 +103,9 @@ __global__ __launch_bounds__(NWV * 64) void attn_decode_kernel(const AttnDecode 
     extern __shared__ __align__(16) float comb_d[]; // [NR][QG][kCombRow] when kRowsInLds
     float(*comb)[QG][kCombRow] = kRowsInLds ? reinterpret_cast<float(*)[QG][kCombRow]>(comb_d) : comb_s;
     pin_args(A);
-    const int kvh = blockIdx.x, sp = blockIdx.y, slice = DS > 1 ? blockIdx.z : 0;
+    const int kvh = blockIdx.x, sp = DS > 1 ? 0 : blockIdx.y, slice = DS > 1 ? blockIdx.z : 0;
+    // the block's first query head; sliced, one of the 1, 2, 4 or 8 of the kv head
+    const int head = DS > 1 ? (kvh << (__builtin_ctz(A.n_heads) - __builtin_ctz(A.n_kv_heads))) + blockIdx.y : kvh * QG;
     const int pos = A.dpos ? A.dpos[0] : A.pos;
     const int t0 = sp * A.ts;
     if (t0 > pos) return;
@@ -146,7 +151,7 @@ __global__ __launch_bounds__(NWV * 64) void attn_decode_kernel(const AttnDecode 
     for (int r = 0; r < NQ; r++) {
         const int idx = (tid + r * NT) % (QG * HALF);
         const int j = idx >> 6, i = idx & 63;
-        const float *qh = A.q + (size_t)(kvh * QG + j) * HS;
+        const float *qh = A.q + (size_t)(head + j) * HS;
         qa[r] = qh[i], qb[r] = qh[i + HALF];
         qc[r] = ct[i], qsn[r] = st[i];
     }
@@ -155,11 +160,9 @@ __global__ __launch_bounds__(NWV * 64) void attn_decode_kernel(const AttnDecode 
     const float nv = A.v_new[(size_t)kvh * HS + (tid & 127)];
     const float nc = ct[hd], ns = st[hd];
     // Sliced, a thread has one output at most: where it goes is asked for here, not when it is there.
-    constexpr bool kOneOut = DS > 1 && QG * VD <= NT;
     int out_i = 0;
-    if constexpr (kOneOut) {
-        const int o = tid % (QG * VD);
-        out_i = (kvh * QG + o / VD) * HS + slice * VD + o % VD;
+    if constexpr (DS > 1) {
+        out_i = head * HS + slice * VD + tid % VD;
         const int32_t at = *((A.scatter ? A.scatter : reinterpret_cast<const int32_t *>(A.q)) + out_i);
         out_i = A.scatter ? at : out_i;
     }
@@ -187,7 +190,7 @@ __global__ __launch_bounds__(NWV * 64) void attn_decode_kernel(const AttnDecode 
         kvnew[0][hd] = first;
         kvnew[0][hd + HALF] = second;
         kvnew[1][tid & 127] = nv;
-        if (owns_new && slice == 0) {
+        if (owns_new && (DS == 1 || blockIdx.y + slice == 0)) {
             if (tid < HALF) {
                 float *kw = A.kcache + (size_t)pos * kv_dim + kvh * HS;
                 kw[tid] = first;
@@ -390,10 +393,9 @@ __global__ __launch_bounds__(NWV * 64) void attn_decode_kernel(const AttnDecode 
                 den = fmaf(e, comb[w][j][HS + 1], den);
             }
         }
-        const int h = kvh * QG + j;
-        if (A.n_splits == 1) {
-            const int i = h * HS + dv;
-            A.out[kOneOut ? out_i : A.scatter ? A.scatter[i] : i] = num / den;
+        const int h = head + j;
+        if constexpr (DS > 1) {
+            A.out[out_i] = num / den;
         } else {
             float *p = A.part + ((size_t)h * A.max_splits + sp) * (HS + 2);
             p[dv] = num;
@@ -478,13 +480,6 @@ __global__ __launch_bounds__(256, 2) void attn_decode_mfma_kernel(const AttnDeco
         const float *qh = A.q + (size_t)(kvh * QG + j) * HS;
         qa[r] = qh[i], qb[r] = qh[i + HALF];
         qc[r] = ct[i], qsn[r] = st[i];
-    }
-    // where this thread's outputs go when the step is not split: fetched now, used at the very end
-    int sdst[QG * HS / NT];
-#pragma unroll
-    for (int u = 0; u < QG * HS / NT; u++) {
-        const int i = kvh * QG * HS + tid + u * NT;
-        sdst[u] = (A.scatter && A.n_splits == 1) ? A.scatter[i] : i;
     }
     const int hd = tid & 63;
     const float nk_a = A.k_new[(size_t)kvh * HS + hd], nk_b = A.k_new[(size_t)kvh * HS + hd + HALF];
@@ -657,15 +652,11 @@ __global__ __launch_bounds__(256, 2) void attn_decode_mfma_kernel(const AttnDeco
         const int idx = tid + u * NT;
         const int j = idx >> 7, d = idx & 127;
         const int h = kvh * QG + j;
-        if (A.n_splits == 1) {
-            A.out[sdst[u]] = num[u] / den[u];
-        } else {
-            float *pp = A.part + ((size_t)h * A.max_splits + sp) * (HS + 2);
-            pp[d] = num[u];
-            if (d == 0) {
-                pp[HS] = Mx[u];
-                pp[HS + 1] = den[u];
-            }
+        float *pp = A.part + ((size_t)h * A.max_splits + sp) * (HS + 2);
+        pp[d] = num[u];
+        if (d == 0) {
+            pp[HS] = Mx[u];
+            pp[HS + 1] = den[u];
         }
     }
 }
@@ -1122,21 +1113,19 @@ __global__ __launch_bounds__(512) void attn_combine_kernel(const AttnDecode A) {
     }
 }
 
-template <int QG, int NWV, int DS>
+template <int NWV, int DS>
 int attn_launch_sliced(const AttnDecode &a, hipStream_t st) {
-    l2_launch((attn_decode_kernel<QG, NWV, DS>), dim3(a.n_kv_heads, 1, DS), dim3(NWV * 64), 0, st, a);
+    l2_launch((attn_decode_kernel<1, NWV, DS>), dim3(a.n_kv_heads, a.n_heads / a.n_kv_heads, DS), dim3(NWV * 64), 0, st, a);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }
 
 template <int QG>
 int attn_launch_qg(const AttnDecode &a, hipStream_t st) {
-    if constexpr (QG <= 4) {
-        if (a.n_splits == 1) { // slices of the head: as many as keep one block per CU
-            const bool wide = a.pos >= (QG <= 2 ? 64 : 128), eight = a.n_kv_heads * 8 <= cu_count();
-            if (eight) return wide ? attn_launch_sliced<QG, 8, 8>(a, st) : attn_launch_sliced<QG, 4, 8>(a, st);
-            return wide ? attn_launch_sliced<QG, 8, 4>(a, st) : attn_launch_sliced<QG, 4, 4>(a, st);
-        }
+    if (a.n_splits == 1) { // slices of the head: as many as keep one block per CU
+        const bool wide = a.pos >= 64, eight = a.n_heads * 8 <= cu_count();
+        if (eight) return wide ? attn_launch_sliced<8, 8>(a, st) : attn_launch_sliced<4, 8>(a, st);
+        return wide ? attn_launch_sliced<8, 4>(a, st) : attn_launch_sliced<4, 4>(a, st);
     }
     if constexpr (QG >= 4) {
         static const bool valu = []() {

@@ -332,6 +332,27 @@ def test_decode_attention_whole_or_split(ops, oracle, n_heads, n_kv):
     o.close()
 
 
+# A block per query head: several to a kv head, slices of 16 dimensions and of 32 (64 heads), both sides of where the context is cut
+@pytest.mark.parametrize("n_heads,n_kv,whole", [(2, 2, 640), (2, 1, 896), (8, 2, 896), (8, 1, 896), (32, 16, 1024), (64, 8, 1024), (33, 33, 768)])
+def test_decode_attention_block_per_head(ops, oracle, n_heads, n_kv, whole):
+    dims = ck.Dims(dim=128 * n_heads, hidden_dim=512, n_layers=1, n_heads=n_heads, n_kv_heads=n_kv,
+                   vocab_size=300, seq_len=1100, group_size=128)
+    img = ck.synth_weights_image(dims, seed=9)
+    m = ops.Model(img, dims)
+    o = oracle.Model(img, dims)
+    o.new_state()
+    m.fill_kv_synthetic(0, 1090, seed=5)
+    ko, vo = o.kv_cache()
+    ko[0, :1090], vo[0, :1090] = m.read_kv(0, 0, 1090)
+    for pos in (0, 31, 64, 128, 300, whole - 2, whole - 1, whole, whole + 1):
+        want = o.transformer([11], [pos])
+        assert nrel(m.forward([11], [pos]), want) < REL_FP32, pos
+    k, v = m.read_kv(0, 0, 1090)  # each new row written once, by one block of its kv head
+    assert nrel(k, ko[0, :1090]) < REL_FP32 and nrel(v, vo[0, :1090]) < REL_FP32
+    m.close()
+    o.close()
+
+
 _VALU_ATTN_SNIPPET = r"""
 import sys, numpy as np
 sys.path.insert(0, sys.argv[1]); sys.path.insert(0, sys.argv[2])
