@@ -8,8 +8,8 @@
 // layer's g_index order, multiplied by the norm weight where one applies, and
 // rounded to fp16 (kernels_gemm.hip).
 //
-// Tiling.  A wave owns 32 output rows and 32 NB tokens (its dequantised weights are reused for all of them); a block is 8 waves
-// side by side over the rows with NB = 4, one per CU, or 4 waves with NB <= 2, two or three per CU.  K may be cut into KS
+// Tiling.  A wave owns 32 output rows and 16 NT tokens (its dequantised weights are reused for all of them); a block is 8 waves
+// side by side over the rows with NT = 8 or 9, one per CU, or 4 waves with NT <= 4, two or three per CU.  K may be cut into KS
 // slices; each writes its fp32 partial tile to a workspace and the consumer (or gemm_reduce_kernel) adds them in a fixed order.
 //
 // Memory.  Everything the K loop reads comes through LDS without touching a register (buffer_load ... lds): the activation
@@ -26,9 +26,13 @@
 //     of a step, operands are read from LDS four pairs of MFMAs ahead, and a wave's priority falls with its progress since
 //     the last barrier: with equal priorities the older wave of a SIMD ran ahead and waited 30 % of the time at the barrier
 //     (1862 cycles per step of 64 k; 1650 now, 1024 of them MFMAs; what a SIMD can issue is 1104, the rest are waits).
-//   - Power, a cost and not the bound.  With 70B's shapes the clock falls to 1.8 - 1.9 GHz; all-zero activations run the same
-//     code at 2.23 GHz.  The 16x16x32 form needs less than 32x32x16 for the same products (a loop of nothing else: 1974
-//     against 1655 TFLOP/s), and blocks of 256 rows read every activation tile half as often as blocks of 128.
+//   - Power, and with many tokens that is the bound: a kernel that takes fewer cycles runs at a lower clock.  70B's w1|w3, 776 tokens,
+//     runs at 1.86 GHz, 7B's, 511, at 1.63, where nothing but MFMAs on the same data runs at 1.99 (1.8 PFLOP/s) and all-zero
+//     activations at 2.4.  With 32x32x16 MFMAs a step takes 1512 cycles instead of 1658, and the clock falls to 1.57 GHz: 70B's prompt
+//     14.11 -> 14.41 ms, 7B's 11.22 -> 11.55.  So what counts is the work per token: without the reads of activations from LDS the
+//     launch would take 24 % less, without the folds 15, without the dequantisation 13.  Hence tiles of 144 tokens, as many as the
+//     registers hold, where that makes fewer of them: 70B's 776 tokens 13.97 -> 13.18 ms, six layers of 7B, 280 tokens 1632 -> 1542 us,
+//     699 2911 -> 2714, four of 13B, 280, 899 1594 / 3616 -> 1471 / 3518, three of 70B, 419 3196 -> 3052.
 //
 // Dequant.  (w >> 4i) & 0x000F000F | 0x64006400 is the fp16 pair (1024+n_i,
 // 1024+n_{i+4}); subtracting 1024+z1 is exact.  The pairs come out as
@@ -88,12 +92,12 @@ struct GemmLds {
     static constexpr size_t size(int tokens) { return (size_t)4 * tokens * kStepRow + (size_t)NW * 3 * kUnit; }
 };
 
-// 32 NW rows rb * 32 NW.. of the matrices of a launch against the 32 NB tokens t0.., K slice ks of KS.
-template <int G, int NB, int NW>
+// 32 NW rows rb * 32 NW.. of the matrices of a launch against the 16 NT tokens t0.., K slice ks of KS.
+template <int G, int NT, int NW>
 __device__ __forceinline__ void q4_gemm_tile(const Q4Launch &L, const XhList &xh_list, const float *__restrict__ ss,
                                              float *__restrict__ ws, int KS, int partials, int rb, int ks, int t0) {
     using S = GemmLds<G, NW>;
-    constexpr int TN = 32 * NB, kTile = TN * kStepRow;
+    constexpr int TN = 16 * NT, kTile = TN * kStepRow;
     constexpr bool SA = G >= 64; // scale after the group's partial sum
     extern __shared__ __align__(16) char lds[];
     int mi = 0;
@@ -115,23 +119,22 @@ __device__ __forceinline__ void q4_gemm_tile(const Q4Launch &L, const XhList &xh
 
     // Where a lane's pieces come from.  A wave's 1 KB pieces of an activation tile follow each other in the LDS (fewer pieces
     // than waves: the last ones fetch the same), as do the parts of a unit: one base each, the rest in the instructions.
-    constexpr int XP = (NB * 4 + NW - 1) / NW;
+    constexpr int XP = (2 * NT + NW - 1) / NW;
     static_assert(XP <= 4, "the instruction's own offset has 12 bits");
     const int row_tiles = (n_out + 31) >> 5; // of scales and zero points
     const u4v xbuf = biased_buffer(xh_list.p[mi], (size_t)B * in * 2), wbuf = biased_buffer(M.qweight, (size_t)n_out * (in >> 1));
     const u4v sbuf = biased_buffer(M.scales, (size_t)row_tiles * groups * 128), zbuf = biased_buffer(M.qzeros, (size_t)row_tiles * groups * 16);
-    const int xfirst = min(wave * XP, NB * 4 - XP);
-    uint32_t xoff[XP], woff[2], soff, zoff;
+    const int xfirst = min(wave * XP, 2 * NT - XP);
+    uint32_t xoff[XP], woff, soff, zoff;
 #pragma unroll
     for (int i = 0; i < XP; i++) { // activations: 8 tokens of 128 bytes, a token's 16-byte pieces permuted by its number
         const int t = (xfirst + i) * 8 + (lane >> 3);
         xoff[i] = (uint32_t)min(t0 + t, B - 1) * (uint32_t)in * 2u + (((lane & 7) ^ piece_xor(t)) << 4) + kBias - i * 1024;
     }
-#pragma unroll
-    for (int i = 0; i < 2; i++) { // weights: 16 rows of 64 bytes, permuted likewise
-        const int row = i * 16 + (lane >> 2);
-        woff[i] = (uint32_t)min(obase + row, n_out - 1) * (uint32_t)(in >> 1) + (((lane & 3) ^ ((row >> 2) & 3)) << 4) + kBias - i * 1024;
-    }
+    // weights: 16 rows of 64 bytes, permuted likewise, and 16 more (n_out is whole 32s; a wave beyond takes the last ones again)
+    const int wrow = min(obase, n_out - 32);
+    woff = (uint32_t)(wrow + (lane >> 2)) * (uint32_t)(in >> 1) + (((lane & 3) ^ (lane >> 4)) << 4) + kBias;
+    const uint32_t w_half = (uint32_t)in * 8u - 1024;
     const uint32_t group0 = (uint32_t)(min(obase >> 5, row_tiles - 1) * groups) + (G == 128 ? 0 : lane >> 5); // two groups (G = 128: the same one again)
     soff = group0 * 128u + (lane & 31) * 4u + kBias - S::kWeights;
     zoff = group0 * 16u + (lane >> 3 & 3) * 4u + kBias - S::kWeights - S::kScales;
@@ -139,6 +142,9 @@ __device__ __forceinline__ void q4_gemm_tile(const Q4Launch &L, const XhList &xh
     uint32_t xr[2]; // piece 2 kg + s of token r
 #pragma unroll
     for (int s = 0; s < 2; s++) xr[s] = (uint32_t)r * kStepRow + (((2 * kg + s) ^ piece_xor(r)) << 4);
+    // the second two of four tiles of 144 tokens lie beyond what an LDS read can have as a constant
+    uint32_t xr_far[2] = {xr[0] + 2 * kTile, xr[1] + 2 * kTile};
+    if constexpr (NT > 8) asm volatile("" : "+v"(xr_far[0]), "+v"(xr_far[1]));
     const uint32_t wr = wave_at + r * 64 + (((kg >> 1) ^ ((r >> 2) & 3)) << 4) + (kg & 1) * 8; // of a unit's first step; the second's: ^ 32
     const uint32_t sr = wave_at + S::kWeights + kg * 16, zr = wave_at + S::kWeights + ((G == 32 ? (kg >> 1) * 32 : 0) + r) * 4;
     const int zsh = 4 * (r & 7); // obase is a multiple of 8
@@ -153,7 +159,7 @@ __device__ __forceinline__ void q4_gemm_tile(const Q4Launch &L, const XhList &xh
     auto fetch_w = [&](const uint32_t unit, const int i) __attribute__((always_inline)) { // piece i of WL
         const uint32_t s_at = w_at * (256 / G), z_at = s_at >> 3;
         const uint32_t to = lds0 + wave_at + unit;
-        if (i < 2) LDS_LOAD("x4", to, i * 1024, wbuf, woff[i], w_at);
+        if (i < 2) LDS_LOAD("x4", to, i * 1024, wbuf, woff, w_at + i * w_half);
         else if (i == 2) LDS_LOAD("", to, S::kWeights, sbuf, soff, s_at);
         else if (i == 3) LDS_LOAD("", to, S::kWeights + S::kScales, zbuf, zoff, z_at);
         else if (i == 4) LDS_LOAD("", to, S::kWeights + 256, sbuf, soff - 256 + 2 * 128, s_at); // G = 32: the second step's groups
@@ -161,8 +167,7 @@ __device__ __forceinline__ void q4_gemm_tile(const Q4Launch &L, const XhList &xh
         if (i == WL - 1) w_at = min(w_at + 64, w_last);
     };
 
-    constexpr int NT = 2 * NB; // tiles of 16 tokens
-    f4v acc[NT][2], accg[NT][2]; // running result, two tiles of 16 rows; partial sums of the current group (SA)
+    f4v acc[NT][2], accg[NT][2]; // running result of each tile of 16 tokens, two tiles of 16 rows; partial sums of the current group (SA)
 #pragma unroll
     for (int n = 0; n < NT; n++)
 #pragma unroll
@@ -183,9 +188,11 @@ __device__ __forceinline__ void q4_gemm_tile(const Q4Launch &L, const XhList &xh
     h8 bq[8];             // activations of eight pairs of MFMAs
     auto read_w = [&](const int par, uint32_t unit) __attribute__((always_inline)) {
         const int gi = G == 128 ? 0 : G == 64 ? par * 128 : par * 256; // of the step's group
+        uint32_t w_lds = wr;
+        if constexpr (NT > 8) asm volatile("" : "+v"(w_lds)); // one register, not two
 #pragma unroll
         for (int m = 0; m < 2; m++) {
-            wd[m] = *reinterpret_cast<const uint2 *>(lds + (wr ^ (par * 32)) + unit + m * 1024);
+            wd[m] = *reinterpret_cast<const uint2 *>(lds + (w_lds ^ (par * 32)) + unit + m * 1024);
             if (G != 128 || par == 0) zw[m] = *reinterpret_cast<const int *>(lds + zr + unit + S::kScales + gi + m * 64);
             if (!SA) sl[m] = *reinterpret_cast<const float *>(lds + zr + unit + gi + m * 64);
         }
@@ -204,14 +211,16 @@ __device__ __forceinline__ void q4_gemm_tile(const Q4Launch &L, const XhList &xh
         aq[to][m][k].p[i % 4] = dq[m].template pair<!SA>(w, i % 4, s16[m]);
     };
 
-    // A step of 64 k is 4 NB pairs of MFMAs (two tiles of 16 rows with one of 16 tokens, 32 k), the first half of the token
+    // A step of 64 k is 2 NT pairs of MFMAs (two tiles of 16 rows with one of 16 tokens, 32 k), the first half of the token
     // tiles', then the others'.  Between them stands, evenly spread, what the vector unit has to do: the fold of the OTHER
-    // tiles' finished group, the next step's weights.
-    constexpr int T = 4 * NB, H = T / 2, N0 = NT / 2, AHEAD = 4;
-    auto n_of = [](int t) { return t / H * N0 + t % H % N0; };
-    auto k_of = [](int t) { return t % H / N0; };
-    auto read_x = [&](const int par, const int t, const int tile) __attribute__((always_inline)) {
-        bq[(par * T + t) % 8] = *reinterpret_cast<const h8 *>(lds + xr[k_of(t)] + tile + n_of(t) * 16 * kStepRow);
+    // tiles' finished group, the next step's weights.  Activations are read, and their registers dealt out, by the pairs' number
+    // within the four steps of a round (2 NT is not a multiple of four where NT is odd).
+    constexpr int T = 2 * NT, N0 = NT / 2, N1 = NT - N0, H = 2 * N0, AHEAD = 4;
+    auto n_of = [](int t) { return t < H ? t % N0 : N0 + (t - H) % N1; };
+    auto k_of = [](int t) { return t < H ? t / N0 : (t - H) / N1; };
+    auto read_x = [&](const int u, const int t, const int tile) __attribute__((always_inline)) {
+        const bool far = NT > 8 && tile >= 2 * kTile;
+        bq[(u * T + t) % 8] = *reinterpret_cast<const h8 *>(lds + (far ? xr_far[k_of(t)] + tile - 2 * kTile : xr[k_of(t)] + tile) + n_of(t) * 16 * kStepRow);
     };
     uint32_t unit = 0, unit1 = S::kUnit, unit2 = 2 * S::kUnit; // this unit's place, the next one's and the one's after it
     // Step u of a round of four, which fixes the tiles' places.  Two steps (a unit) go between barriers; in the first of them
@@ -231,22 +240,27 @@ __device__ __forceinline__ void q4_gemm_tile(const Q4Launch &L, const XhList &xh
             }
             const int behind = (par * T + t + AHEAD) % (2 * T); // MFMA pairs since the barrier
             if (behind % (T / 2) == 0) asm volatile("s_setprio %0" ::"n"(3 - behind / (T / 2)));
-            if (t % 4 == 0) { // the next four pairs' activations, behind the arrival of these four's
+            if ((u * T + t) % 4 == 0) { // the next four pairs' activations, behind the arrival of these four's
                 __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0)
 #pragma unroll
-                for (int i = t + 4; i < t + 8; i++) read_x(i < T ? par : par ^ 1, i < T ? i : i - T, i < T ? tile : tile1);
+                for (int i = t + 4; i < t + 8; i++) read_x(i < T ? u : u + 1, i < T ? i : i - T, i < T ? tile : tile1);
             }
 #pragma unroll
             for (int m = 0; m < 2; m++) {
                 f4v &c = SA ? accg[n][m] : acc[n][m];
-                c = __builtin_amdgcn_mfma_f32_16x16x32_f16(aq[par][m][k].v, bq[(par * T + t) % 8], SA && first && k == 0 ? f4v{} : c, 0, 0, 0);
+                c = __builtin_amdgcn_mfma_f32_16x16x32_f16(aq[par][m][k].v, bq[(u * T + t) % 8], SA && first && k == 0 ? f4v{} : c, 0, 0, 0);
             }
-            if (SA && (t < H ? first : last)) fold((t < H ? N0 : 0) + t % H / 2, t % 2);
+            if (SA && (t < H ? first : last)) {
+                const int j = t < H ? t : t - H, slots = t < H ? H : T - H, folds = t < H ? 2 * N1 : 2 * N0;
+#pragma unroll
+                for (int f = j * folds / slots; f < (j + 1) * folds / slots; f++) fold((t < H ? N0 : 0) + f / 2, f % 2);
+            }
 #pragma unroll
             for (int i = t * 16 / T; i < (t + 1) * 16 / T; i++) dequant(par ^ 1, i);
             // the scales of the group that ends with this step, once the folds above no longer need the one before's
-            if (SA && last && t >= H - 2 && t < H)
-                sv[t % 2] = *reinterpret_cast<const f4v *>(lds + sr + unit + gi + t % 2 * 64);
+#pragma unroll
+            for (int m = 0; m < 2; m++)
+                if (SA && last && t == (N0 == N1 ? H - 2 + m : H - 1)) sv[m] = *reinterpret_cast<const f4v *>(lds + sr + unit + gi + m * 64);
             if (par == 0) {
                 // one request at a time: several in a row wait for the address unit
                 constexpr int NL = 2 * XP + WL;
@@ -302,13 +316,13 @@ __device__ __forceinline__ void q4_gemm_tile(const Q4Launch &L, const XhList &xh
     float *tile_o = reinterpret_cast<float *>(lds) + wave * 32 * kTRow; // 4.5 KB per wave
     const int tl = lane >> 3, oc = (lane & 7) * 4; // read-back map: token within a pass of 8, 4 rows
 #pragma unroll
-    for (int nb = 0; nb < NB; nb++) {
+    for (int nb = 0; nb < (NT + 1) / 2; nb++) {
 #pragma unroll
         for (int i = 0; i < 4; i++)
-            *reinterpret_cast<f4v *>(&tile_o[(i / 2 * 16 + r) * kTRow + i % 2 * 16 + kg * 4]) = acc[2 * nb + i / 2][i % 2];
+            if (2 * nb + i / 2 < NT) *reinterpret_cast<f4v *>(&tile_o[(i / 2 * 16 + r) * kTRow + i % 2 * 16 + kg * 4]) = acc[2 * nb + i / 2][i % 2];
         // the wave reads what the wave wrote: no block barrier, the LDS queue of a wave is in order
 #pragma unroll
-        for (int pass = 0; pass < 4; pass++) {
+        for (int pass = 0; pass < (2 * nb + 1 < NT ? 4 : 2); pass++) {
             const int tt = pass * 8 + tl;
             float4 v = *reinterpret_cast<const float4 *>(&tile_o[tt * kTRow + oc]);
             const int t = t0 + nb * 32 + tt;
@@ -339,11 +353,11 @@ __device__ __forceinline__ void q4_gemm_tile(const Q4Launch &L, const XhList &xh
 // tiles of 32 NB tokens; what whole rounds of blocks leave over goes in tiles of `width`; then come the last tokens of the first units,
 // where they need no more than half a tile.  A tile costs its width in steps of 32 and the dequantisation of its weights (128, 64,
 // 32 tokens of 70B's w1: 119, 75, 62 us).
-template <int G, int NB, int NW>
-__global__ __launch_bounds__(64 * NW, NB > 2 ? 2 : 1) void q4_gemm_kernel(const Q4Launch L, const XhList xh, const float *__restrict__ ss,
+template <int G, int NT, int NW>
+__global__ __launch_bounds__(64 * NW, NT > 4 ? 2 : 1) void q4_gemm_kernel(const Q4Launch L, const XhList xh, const float *__restrict__ ss,
                                                       float *__restrict__ ws, int KS, int partials, int row_blocks, int t_full, int units, int extra,
                                                       int width) {
-    constexpr int TN = 32 * NB, CHUNK = 8;
+    constexpr int TN = 16 * NT, CHUNK = 8;
     const int b = blockIdx.x, whole = units * t_full + extra, per = (L.batch + width - 1) / width;
     const int head = extra ? (L.batch - extra * TN + width - 1) / width : 0; // of the unit that has tiles of both kinds
     const int begun = units + (extra > 0), left = row_blocks * KS - begun, other = head + left * per;
@@ -366,55 +380,77 @@ __global__ __launch_bounds__(64 * NW, NB > 2 ? 2 : 1) void q4_gemm_kernel(const 
         unit = xcd_item(b - whole - other, gridDim.x - whole - other), t0 = t_full * TN, n = L.batch - t0;
     }
     const int ks = unit / row_blocks, rb = unit - ks * row_blocks;
-    if (NB > 1 && n <= 32)
-        q4_gemm_tile<G, 1, NW>(L, xh, ss, ws, KS, partials, rb, ks, t0);
-    else if (NB > 2 && n <= 64)
-        q4_gemm_tile<G, NB < 2 ? NB : 2, NW>(L, xh, ss, ws, KS, partials, rb, ks, t0);
-    else if (NB > 3 && n <= 96)
-        q4_gemm_tile<G, NB < 3 ? NB : 3, NW>(L, xh, ss, ws, KS, partials, rb, ks, t0);
+    if (NT > 2 && n <= 32)
+        q4_gemm_tile<G, 2, NW>(L, xh, ss, ws, KS, partials, rb, ks, t0);
+    else if (NT > 4 && n <= 64)
+        q4_gemm_tile<G, NT < 4 ? NT : 4, NW>(L, xh, ss, ws, KS, partials, rb, ks, t0);
+    else if (NT > 6 && n <= 96)
+        q4_gemm_tile<G, NT < 6 ? NT : 6, NW>(L, xh, ss, ws, KS, partials, rb, ks, t0);
+    else if (NT > 8 && n <= 128)
+        q4_gemm_tile<G, NT < 8 ? NT : 8, NW>(L, xh, ss, ws, KS, partials, rb, ks, t0);
     else
-        q4_gemm_tile<G, NB, NW>(L, xh, ss, ws, KS, partials, rb, ks, t0);
+        q4_gemm_tile<G, NT, NW>(L, xh, ss, ws, KS, partials, rb, ks, t0);
 }
 
-template <int G, int NB, int NW>
-int launch_gemm(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, int partials, bool beside, hipStream_t st) {
-    constexpr int TN = 32 * NB;
-    int row_blocks = 0;
-    for (int i = 0; i < L.n_mats; i++) row_blocks += L.m[i].row_blocks = (L.m[i].out + 32 * NW - 1) / (32 * NW);
-    const int rest = L.batch % TN, t_full = L.batch / TN + (rest > TN / 2), narrow = rest > 0 && rest <= TN / 2;
-    // What whole rounds of tiles leave over goes in narrower ones where these, and the last tokens of the other units, fit one round:
-    // 7B's w1|w3, 511 tokens, 344 tiles on 256 CUs 123 -> 112 us; with 224 narrow tiles behind 64 left over (70B's, 776) they take 822
-    // and whole tiles 804.  With several slices too: four layers of 13B, group 64, 399 tokens 2192 -> 2135, six of 7B, group 32, 249
-    // tokens 1656 -> 1610.  Of the blocks of four waves too, where some CUs have two and others one (two take twice as long as one):
-    // six layers of 7B, 64, 99, 128 tokens 918 / 1075 / 1120 -> 903 / 1047 / 1080, four of 13B, 128 1057 -> 1041; with more of them than
-    // two per CU whole tiles (70B, 179 1965 against 1978).  Tiles of 96 where those of 64 are more than a round, six layers of 7B: 287,
-    // 349, 599 tokens 1702 / 1889 / 2469 -> 1670 / 1835 / 2450; four of 13B, 199, 299 1311 / 1716 -> 1291 / 1687.  Where both fit those
-    // of 64: 349 of 7B 1835 against 1886.  None of 96 beside another pass, which has a use for the CUs that a round
-    // leaves: four layers of 13B, 300 and 399 tokens in chunks of 256 1359 / 1742 -> 1302 / 1713, six of 7B, 899 in chunks of 128 3891 -> 3812.
-    const int all = row_blocks * s.slices, tiles = all * t_full, cus = cu_count();
-    int units = all, extra = 0, width = TN, blocks = tiles + narrow * all;
-    if ((NB == 4 || (NB == 2 && tiles > cus && tiles < 2 * cus)) && tiles % cus) {
+// How the blocks of a launch are dealt out (q4_gemm_kernel), with what it takes: a tile of w tokens 43 + 0.594 w (of 70B's w1: 62,
+// 75 and 119 us for 32, 64 and 128).
+struct GemmPlan {
+    int t_full, units, extra, width, blocks;
+    float cost;
+};
+
+// What whole rounds of tiles leave over goes in narrower ones where these, and the last tokens of the other units, fit one round:
+// 7B's w1|w3, 511 tokens, 344 tiles on 256 CUs 123 -> 112 us; with 224 narrow tiles behind 64 left over (70B's, 776) they take 822
+// and whole tiles 804.  With several slices too: four layers of 13B, group 64, 399 tokens 2192 -> 2135, six of 7B, group 32, 249
+// tokens 1656 -> 1610.  Of the blocks of four waves too, where some CUs have two and others one (two take twice as long as one):
+// six layers of 7B, 64, 99, 128 tokens 918 / 1075 / 1120 -> 903 / 1047 / 1080, four of 13B, 128 1057 -> 1041; with more of them than
+// two per CU whole tiles (70B, 179 1965 against 1978).  Tiles of 96 where those of 64 are more than a round, six layers of 7B: 287,
+// 349, 599 tokens 1702 / 1889 / 2469 -> 1670 / 1835 / 2450; four of 13B, 199, 299 1311 / 1716 -> 1291 / 1687.  Where both fit those
+// of 64: 349 of 7B 1835 against 1886.  None of 96 beside another pass, which has a use for the CUs that a round
+// leaves: four layers of 13B, 300 and 399 tokens in chunks of 256 1359 / 1742 -> 1302 / 1713, six of 7B, 899 in chunks of 128 3891 -> 3812.
+static GemmPlan plan_tiles(int TN, int all, int B, bool beside) {
+    const int rest = B % TN, most = std::min(TN / 2, 64), t_full = B / TN + (rest > most), narrow = rest > 0 && rest <= most;
+    const int tiles = all * t_full, cus = cu_count();
+    auto tile_cost = [](int w) { return 43.f + 0.594f * w; };
+    // whole tiles, and the last tokens' where a round leaves room
+    const float whole = tile_cost(TN), last = tile_cost(most);
+    const int room = tiles % cus ? (cus - tiles % cus) * (int)(whole / last) : 0;
+    GemmPlan p{t_full, all, 0, TN, tiles + narrow * all,
+               (tiles + cus - 1) / cus * whole + (narrow * all > room ? (narrow * all - room + cus - 1) / cus * last : 0.f)};
+    if ((TN > 64 || (TN == 64 && tiles > cus && tiles < 2 * cus)) && tiles % cus) {
         // Whole tiles for full rounds: of these units, and `done` of the next one, without which those of 64 may not fit (three layers of
         // 70B, 399 tokens in chunks of 128: 2785 -> 2735).  With four waves none of the next one: 70B, 176 tokens 1405, with them 1433.
-        const int rounds = tiles / cus * cus, begun = rounds / t_full, done = NB == 4 ? rounds % t_full : 0;
-        for (const int w : {TN / 4 * 3, TN / 2}) {
-            if (w % 32 || (beside && w > TN / 2)) continue;
-            const int n = (done ? (L.batch - done * TN + w - 1) / w : 0) + (all - begun - (done > 0)) * ((L.batch + w - 1) / w) + narrow * begun;
-            if (n <= cus) units = begun, extra = done, width = w, blocks = begun * t_full + done + n;
+        const int rounds = tiles / cus * cus, begun = rounds / t_full, done = TN > 64 ? rounds % t_full : 0;
+        for (const int w : {96, most}) {
+            if (w >= TN || (beside && w > most)) continue;
+            const int n = (done ? (B - done * TN + w - 1) / w : 0) + (all - begun - (done > 0)) * ((B + w - 1) / w) + narrow * begun;
+            if (n <= cus) p = {t_full, begun, done, w, begun * t_full + done + n, tiles / cus * whole + tile_cost(w)};
         }
     }
+    return p;
+}
+
+template <int G, int NT, int NW>
+int launch_gemm(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, int partials, bool beside, hipStream_t st) {
+    constexpr int TN = 16 * NT;
+    int row_blocks = 0;
+    for (int i = 0; i < L.n_mats; i++) row_blocks += L.m[i].row_blocks = (L.m[i].out + 32 * NW - 1) / (32 * NW);
+    const GemmPlan p = plan_tiles(TN, row_blocks * s.slices, L.batch, beside);
+    // Tiles of 144 tokens where they take less (and not about the same: 7B, 899 tokens, a cost of 1.00, 3485 -> 3523 us for six layers).
+    if constexpr (NT == 8)
+        if (plan_tiles(144, row_blocks * s.slices, L.batch, beside).cost < 0.98f * p.cost) return launch_gemm<G, 9, NW>(L, xh, ss, ws, s, partials, beside, st);
     // partial tiles past the caches where they would fill them: what a launch leaves dirty there is written back at its end
     // (7B, 511 tokens: the four launches 13 us less per layer, their consumers 5 more; below 16 MB the other way round: there they
     // go past the L2 but not past the memory-side cache, see store_through)
     size_t bytes = 0;
     for (int i = 0; i < L.n_mats; i++) bytes += (size_t)s.slices * L.batch * L.m[i].out * 4;
     if (partials && bytes > ((size_t)16 << 20)) partials = 2;
-    const dim3 grid(blocks), block(64 * NW);
+    const dim3 grid(p.blocks), block(64 * NW);
     // the tiles, or the output staging tiles of the epilogue (32 x 36 floats per wave)
     const size_t lds = std::max(GemmLds<G, NW>::size(TN), (size_t)NW * 32 * 36 * sizeof(float));
     static LdsLimit limit(48 * 1024);
-    L2_TRY(limit.ensure(reinterpret_cast<const void *>(q4_gemm_kernel<G, NB, NW>), lds));
-    l2_launch((q4_gemm_kernel<G, NB, NW>), grid, block, lds, st, L, xh, ss, ws, s.slices, partials, row_blocks, t_full, units, extra, width);
+    L2_TRY(limit.ensure(reinterpret_cast<const void *>(q4_gemm_kernel<G, NT, NW>), lds));
+    l2_launch((q4_gemm_kernel<G, NT, NW>), grid, block, lds, st, L, xh, ss, ws, s.slices, partials, row_blocks, p.t_full, p.units, p.extra, p.width);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }
@@ -422,9 +458,9 @@ int launch_gemm(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const
 template <int G>
 int launch_gemm_g(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, int partials, bool beside, hipStream_t st) {
     switch (s.tokens) {
-        case 32: return launch_gemm<G, 1, 4>(L, xh, ss, ws, s, partials, beside, st);
-        case 64: return launch_gemm<G, 2, 4>(L, xh, ss, ws, s, partials, beside, st);
-        case 128: return launch_gemm<G, 4, 8>(L, xh, ss, ws, s, partials, beside, st);
+        case 32: return launch_gemm<G, 2, 4>(L, xh, ss, ws, s, partials, beside, st);
+        case 64: return launch_gemm<G, 4, 4>(L, xh, ss, ws, s, partials, beside, st);
+        case 128: return launch_gemm<G, 8, 8>(L, xh, ss, ws, s, partials, beside, st);
     }
     return l2_fail(L2_ERR_ARG, "q4 gemm: token tile");
 }

@@ -359,6 +359,26 @@ def test_fp16_operator_wide_blocks(ops, dim, hidden, G, batches):
     m.close()
 
 
+# tiles of 144 tokens: one unit of K, two, three, five and six, a last tile of 113, 129 and 144 tokens; the columns are the bits of tiles of 128
+@pytest.mark.parametrize("dim,hidden,G", [(128, 22016, 32), (128, 22016, 64), (256, 22016, 128), (384, 22272, 64), (640, 22016, 32), (768, 22016, 128)])
+def test_fp16_operator_tiles_of_144(ops, dim, hidden, G):
+    from llama2_rs import _lib
+    dims = ck.Dims(dim=dim, hidden_dim=hidden, n_layers=1, n_heads=dim // 128, n_kv_heads=dim // 128, vocab_size=64, seq_len=1024,
+                   group_size=G)
+    m = ops.Model(ck.synth_weights_image(dims, seed=13), dims)
+    x = np.random.default_rng(dim).standard_normal((288, dim)).astype(np.float16).astype(np.float32) # as above: only fp32 sums round
+    m.set_prefill_mode(_lib.PREFILL_FP32)
+    want = m.qmatvec(0, _lib.W1, x)
+    m.set_prefill_mode(_lib.PREFILL_MFMA)
+    of_128 = m.qmatvec(0, _lib.W1, x[:256])
+    for B in (257, 273, 288):
+        got = m.qmatvec(0, _lib.W1, x[:B])
+        assert np.array_equal(got[:256], of_128), B
+        for b in range(B):
+            assert nrel(got[b], want[b]) < (4e-3 if G == 32 else 2e-5), (B, b)
+    m.close()
+
+
 # the row blocks that whole rounds leave over, in tiles of 64 (300, 350 rows) and of 96 (520, 590): first and last tiles that are
 # not full, a last row block that is not full, whole tiles that end inside eight row blocks
 @pytest.mark.parametrize("B", [300, 350, 520, 590])
