@@ -380,16 +380,22 @@ __global__ __launch_bounds__(64 * NW, NT > 4 ? 2 : 1) void q4_gemm_kernel(const 
         unit = xcd_item(b - whole - other, gridDim.x - whole - other), t0 = t_full * TN, n = L.batch - t0;
     }
     const int ks = unit / row_blocks, rb = unit - ks * row_blocks;
-    if (NT > 2 && n <= 32)
-        q4_gemm_tile<G, 2, NW>(L, xh, ss, ws, KS, partials, rb, ks, t0);
-    else if (NT > 4 && n <= 64)
-        q4_gemm_tile<G, NT < 4 ? NT : 4, NW>(L, xh, ss, ws, KS, partials, rb, ks, t0);
-    else if (NT > 6 && n <= 96)
-        q4_gemm_tile<G, NT < 6 ? NT : 6, NW>(L, xh, ss, ws, KS, partials, rb, ks, t0);
-    else if (NT > 8 && n <= 128)
-        q4_gemm_tile<G, NT < 8 ? NT : 8, NW>(L, xh, ss, ws, KS, partials, rb, ks, t0);
-    else
-        q4_gemm_tile<G, NT, NW>(L, xh, ss, ws, KS, partials, rb, ks, t0);
+    switch (min((n + 15) >> 4, NT)) { // tiles of 16 tokens that it takes
+#define GEMM_TILE(t) \
+    case t: \
+        if constexpr (t <= NT) q4_gemm_tile<G, t, NW>(L, xh, ss, ws, KS, partials, rb, ks, t0); \
+        break
+        case 1:
+        GEMM_TILE(2);
+        GEMM_TILE(3);
+        GEMM_TILE(4);
+        GEMM_TILE(5);
+        GEMM_TILE(6);
+        GEMM_TILE(7);
+        GEMM_TILE(8);
+        GEMM_TILE(9);
+#undef GEMM_TILE
+    }
 }
 
 // How the blocks of a launch are dealt out (q4_gemm_kernel), with what it takes: a tile of w tokens 43 + 0.594 w (of 70B's w1: 62,
@@ -399,32 +405,32 @@ struct GemmPlan {
     float cost;
 };
 
-// What whole rounds of tiles leave over goes in narrower ones where these, and the last tokens of the other units, fit one round:
-// 7B's w1|w3, 511 tokens, 344 tiles on 256 CUs 123 -> 112 us; with 224 narrow tiles behind 64 left over (70B's, 776) they take 822
-// and whole tiles 804.  With several slices too: four layers of 13B, group 64, 399 tokens 2192 -> 2135, six of 7B, group 32, 249
+// What whole rounds of tiles leave over goes in narrower ones, the narrowest with which these, and the last tokens of the other units,
+// fit one round: 7B's w1|w3, 511 tokens, 344 tiles on 256 CUs 123 -> 112 us with 64; with 224 narrow tiles behind 64 left over (70B's, 776)
+// they took 822 and whole tiles 804.  With several slices too: four layers of 13B, group 64, 399 tokens 2192 -> 2135, six of 7B, group 32, 249
 // tokens 1656 -> 1610.  Of the blocks of four waves too, where some CUs have two and others one (two take twice as long as one):
 // six layers of 7B, 64, 99, 128 tokens 918 / 1075 / 1120 -> 903 / 1047 / 1080, four of 13B, 128 1057 -> 1041; with more of them than
-// two per CU whole tiles (70B, 179 1965 against 1978).  Tiles of 96 where those of 64 are more than a round, six layers of 7B: 287,
-// 349, 599 tokens 1702 / 1889 / 2469 -> 1670 / 1835 / 2450; four of 13B, 199, 299 1311 / 1716 -> 1291 / 1687.  Where both fit those
-// of 64: 349 of 7B 1835 against 1886.  None of 96 beside another pass, which has a use for the CUs that a round
+// two per CU whole tiles (70B, 179 1965 against 1978).  Of 32 to 112 tokens in steps of 16 against 96 and 64 alone: 70B's 776 13.47 ->
+// 13.28 ms; six layers of 7B, 199, 511, 776 1330 / 2180 / 3260 -> 1298 / 2163 / 3230; four of 13B, 199 1280 -> 1230; 350 1735, 1740.
+// None above 64 beside another pass, which has a use for the CUs that a round
 // leaves: four layers of 13B, 300 and 399 tokens in chunks of 256 1359 / 1742 -> 1302 / 1713, six of 7B, 899 in chunks of 128 3891 -> 3812.
 static GemmPlan plan_tiles(int TN, int all, int B, bool beside) {
     const int rest = B % TN, most = std::min(TN / 2, 64), t_full = B / TN + (rest > most), narrow = rest > 0 && rest <= most;
     const int tiles = all * t_full, cus = cu_count();
     auto tile_cost = [](int w) { return 43.f + 0.594f * w; };
     // whole tiles, and the last tokens' where a round leaves room
-    const float whole = tile_cost(TN), last = tile_cost(most);
-    const int room = tiles % cus ? (cus - tiles % cus) * (int)(whole / last) : 0;
+    const float whole = tile_cost(TN), last = narrow ? tile_cost(std::max((rest + 15) / 16 * 16, 32)) : 0.f;
+    const int room = narrow && tiles % cus ? (cus - tiles % cus) * (int)(whole / last) : 0;
     GemmPlan p{t_full, all, 0, TN, tiles + narrow * all,
                (tiles + cus - 1) / cus * whole + (narrow * all > room ? (narrow * all - room + cus - 1) / cus * last : 0.f)};
     if ((TN > 64 || (TN == 64 && tiles > cus && tiles < 2 * cus)) && tiles % cus) {
         // Whole tiles for full rounds: of these units, and `done` of the next one, without which those of 64 may not fit (three layers of
         // 70B, 399 tokens in chunks of 128: 2785 -> 2735).  With four waves none of the next one: 70B, 176 tokens 1405, with them 1433.
         const int rounds = tiles / cus * cus, begun = rounds / t_full, done = TN > 64 ? rounds % t_full : 0;
-        for (const int w : {96, most}) {
-            if (w >= TN || (beside && w > most)) continue;
+        for (int w = beside ? most : TN - 16; w >= 32; w -= 16) {
             const int n = (done ? (B - done * TN + w - 1) / w : 0) + (all - begun - (done > 0)) * ((B + w - 1) / w) + narrow * begun;
-            if (n <= cus) p = {t_full, begun, done, w, begun * t_full + done + n, tiles / cus * whole + tile_cost(w)};
+            const float cost = tiles / cus * whole + std::max(tile_cost(w), begun ? last : 0.f);
+            if (n <= cus && cost < p.cost) p = {t_full, begun, done, w, begun * t_full + done + n, cost};
         }
     }
     return p;

@@ -379,6 +379,29 @@ def test_fp16_operator_tiles_of_144(ops, dim, hidden, G):
     m.close()
 
 
+# tiles of an odd number of 16 tokens: 112 and 96 (200 columns), 80, 48, a last one of 33, 65, 97, 113, blocks of four waves too; the
+# columns are the bits of tiles of 32
+@pytest.mark.parametrize("dim,hidden,G,batches", [(256, 22016, 64, (200,)), (256, 20480, 128, (240, 193)), (384, 12800, 64, (230, 353)), (256, 12800, 32, (225,)),
+                                                  (512, 1024, 128, (33, 48, 65, 97, 113, 177))])
+def test_fp16_operator_odd_tiles(ops, dim, hidden, G, batches):
+    from llama2_rs import _lib
+    dims = ck.Dims(dim=dim, hidden_dim=hidden, n_layers=1, n_heads=dim // 128, n_kv_heads=dim // 128, vocab_size=64, seq_len=1024,
+                   group_size=G)
+    m = ops.Model(ck.synth_weights_image(dims, seed=15), dims)
+    x = np.random.default_rng(dim).standard_normal((max(batches), dim)).astype(np.float16).astype(np.float32) # as above: only fp32 sums round
+    m.set_prefill_mode(_lib.PREFILL_FP32)
+    want = m.qmatvec(0, _lib.W1, x)
+    m.set_prefill_mode(_lib.PREFILL_MFMA)
+    for B in batches:
+        got = m.qmatvec(0, _lib.W1, x[:B])
+        for b in range(B):
+            assert nrel(got[b], want[b]) < (4e-3 if G == 32 else 2e-5), (B, b)
+        if dim < 512:  # one slice of K whatever the batch
+            of_32 = np.concatenate([m.qmatvec(0, _lib.W1, x[b:b + 32]) for b in range(0, B // 32 * 32, 32)])
+            assert np.array_equal(got[:len(of_32)], of_32), B
+    m.close()
+
+
 # the row blocks that whole rounds leave over, in tiles of 64 (300, 350 rows) and of 96 (520, 590): first and last tiles that are
 # not full, a last row block that is not full, whole tiles that end inside eight row blocks
 @pytest.mark.parametrize("B", [300, 350, 520, 590])
