@@ -214,7 +214,7 @@ struct TileLds {
 // groups spread between them: some 230 instructions for 64 tokens, which the two waves of a SIMD issue at one per 4.9 cycles
 // (2546 cycles per step of 7B's w1|w3 at 299 tokens before the scales and zero points came in tiles, 1536 of them MFMAs; what a
 // SIMD can issue is 1624, the rest are waits).  Eight waves and 64 tokens take 133 KB of LDS, one
-// block per CU; four waves and 16 or 32 tokens, where weights are what is read, two or three.
+// block per CU, and 80 tokens (not with groups of 32) 154; four waves and 16 or 32 tokens, where weights are what is read, two or three.
 //
 // Lane (r = l % 16, kg = l / 16).  G >= 64: the lane's words of a step are 2 kg and 2 kg + 1, MFMA k takes one each.  G = 32: an
 // MFMA must stay inside one group, so its words are kg and 4 + kg.
@@ -483,8 +483,8 @@ __device__ __forceinline__ void q4_tile(const Q4Launch &L, const XhList &xl, int
 }
 
 // The first `whole` blocks take a tile each, row block (and slice) by row block, the others tiles of `width` columns of what is
-// left; these are 48, in whole row blocks, or 32, and then may begin within one.  The last tile of tokens takes 16, 32 or 48 where that
-// is enough (48 against 64: six layers of 7B, 33 and 48 tokens 1114 / 1131 -> 1046 / 1066 us, 299 2743 -> 2685, three of 70B, 44
+// left, which may begin within a row block where they divide a whole tile.  The last tile of tokens takes as many 16s as it needs (48
+// against 64: six layers of 7B, 33 and 48 tokens 1114 / 1131 -> 1046 / 1066 us, 299 2743 -> 2685, three of 70B, 44
 // 1531 -> 1397; 13824x5120, 40 columns 36.4 -> 32.6).
 template <int G, int NT, int NW>
 __global__ __launch_bounds__(64 * NW, NT == 1 ? 3 : 2) void q4_tile_gemm_kernel(const Q4Launch L, const XhList xl, int in_p,
@@ -497,16 +497,24 @@ __global__ __launch_bounds__(64 * NW, NT == 1 ? 3 : 2) void q4_tile_gemm_kernel(
         const int work = xcd_item(blockIdx.x, whole);
         rb = work / t_tiles, t0 = (work - rb * t_tiles) * 16 * NT, n = B - t0;
     } else {
-        const int per = (B + width - 1) / width, begun = whole / t_tiles; // a tile of this row block is two of 32
-        const int work = xcd_item(blockIdx.x - whole, gridDim.x - whole) + begun * per + (whole - begun * t_tiles) * 2;
+        const int per = (B + width - 1) / width, begun = whole / t_tiles;
+        const int work = xcd_item(blockIdx.x - whole, gridDim.x - whole) + begun * per + (whole - begun * t_tiles) * (16 * NT / width);
         rb = work / per, t0 = (work - rb * per) * width, n = min(B - t0, width);
     }
     const int ks = rb / row_blocks;
     rb -= ks * row_blocks;
-    if (NT > 1 && n <= 16) q4_tile<G, 1, NW>(L, xl, in_p, ss, ws, KS, partials, rb, ks, t0, B);
-    else if (NT > 2 && n <= 32) q4_tile<G, NT < 2 ? NT : 2, NW>(L, xl, in_p, ss, ws, KS, partials, rb, ks, t0, B);
-    else if (NT > 3 && n <= 48) q4_tile<G, NT < 3 ? NT : 3, NW>(L, xl, in_p, ss, ws, KS, partials, rb, ks, t0, B);
-    else q4_tile<G, NT, NW>(L, xl, in_p, ss, ws, KS, partials, rb, ks, t0, B);
+    switch (min((n + 15) >> 4, NT)) {
+#define Q4_TILE(t) \
+    case t: \
+        if constexpr (t <= NT) q4_tile<G, t, NW>(L, xl, in_p, ss, ws, KS, partials, rb, ks, t0, B); \
+        break
+        Q4_TILE(1);
+        Q4_TILE(2);
+        Q4_TILE(3);
+        Q4_TILE(4);
+        Q4_TILE(5);
+#undef Q4_TILE
+    }
 }
 
 // Linear::matvec<B> of the model without quantisation (src/model.rs:22-31) for a batch: fp32 weights, fp32 activations,
@@ -1035,27 +1043,45 @@ int ready_tile(size_t *lds) {
     return limit.ensure(reinterpret_cast<const void *>(q4_tile_gemm_kernel<G, NT, NW>), *lds);
 }
 
-template <int G, int NT, int NW>
-int launch_tile(const Q4Launch &L, const XhList &xh, const float *ss, float *ws, int KS, int partials, int total, hipStream_t st) {
-    size_t lds = 0;
-    L2_TRY((ready_tile<G, NT, NW>(&lds)));
-    const int t_tiles = (L.batch + 16 * NT - 1) / (16 * NT), tiles = total * t_tiles * KS, cus = cu_count();
-    // One block per CU: what whole rounds of tiles leave over goes in tiles of 32 columns, or of 48, where that is one round of
-    // blocks, in some 0.7 or 0.85 of a whole one's time.  Six layers of 7B, 32: 169, 250, 439 tokens 2239 / 2470 / 3871 ->
-    // 2120 / 2357 / 3635 us, four of 13B, 149 1964 -> 1881; 48: 299 and 511 tokens of 7B 2668 / 3971 -> 2632 /
-    // 3934, 179 of 70B 3251 -> 3196; 4096x11008, group 32, 130 columns 68.3 -> 58.7.
-    int whole = tiles, width = 16 * NT, blocks = tiles;
-    if (NT == 4 && tiles > cus && tiles % cus) {
+// How the blocks of a launch are dealt out (q4_tile_gemm_kernel), and what it takes in whole tiles of 64: a tile of w columns 0.4 + 0.15 w / 16.
+struct TilePlan {
+    int whole, width, blocks;
+    float cost;
+};
+
+// One block per CU: what whole rounds of tiles leave over goes in the narrowest tiles with which it is one round of
+// blocks.  Six layers of 7B, 32: 169, 250, 439 tokens 2239 / 2470 / 3871 ->
+// 2120 / 2357 / 3635 us, four of 13B, 149 1964 -> 1881; 48: 299 and 511 tokens of 7B 2668 / 3971 -> 2632 /
+// 3934, 179 of 70B 3251 -> 3196; 4096x11008, group 32, 130 columns 68.3 -> 58.7.  And where a last round is all there is, of any
+// whole 16s, and tiles of 80 where those take less (a weight is dequantised once per tile): six layers of 7B, 149, 639 tokens 1931 / 4997 ->
+// 1892 / 4905, four of 13B, 149, 399 in chunks of 256 1914 / 3501 -> 1729 / 3399, of 7B, group 32, 129 1391 -> 1341.
+static TilePlan plan_tiles(int TN, int blocks_per_tile, int B, bool narrower) {
+    auto cost = [](int w) { return 0.4f + 0.15f / 16 * w; };
+    const int t_tiles = (B + TN - 1) / TN, tiles = blocks_per_tile * t_tiles, cus = cu_count();
+    TilePlan p{tiles, TN, tiles, (tiles + cus - 1) / cus * cost(t_tiles > 1 ? TN : (B + 15) / 16 * 16)};
+    if (narrower && tiles % cus) {
         // Whole tiles for full rounds, to the tile where the narrower ones divide one (three layers of 70B, 750 tokens, where only then
         // those of 32 fit: 10690 -> 10440).
         const int rounds = tiles / cus * cus, begun = rounds / t_tiles;
-        for (const int w : {48, 32}) {
-            const int done = 16 * NT % w ? 0 : rounds % t_tiles, per = (L.batch + w - 1) / w, at = begun * per + done * (16 * NT / w);
-            if (total * KS * per - at <= cus) whole = begun * t_tiles + done, width = w, blocks = whole + total * KS * per - at;
+        for (int w = TN - 16; w >= 16; w -= 16) {
+            const int done = TN % w ? 0 : rounds % t_tiles, per = (B + w - 1) / w, at = begun * per + done * (TN / w), n = blocks_per_tile * per - at;
+            const float c = tiles / cus * cost(TN) + cost(w);
+            if (n <= cus && c < p.cost) p = {begun * t_tiles + done, w, begun * t_tiles + done + n, c};
         }
     }
-    l2_launch((q4_tile_gemm_kernel<G, NT, NW>), dim3(blocks), dim3(64 * NW), lds, st, L, xh, gemm_padded(L.in), ss, ws, KS, t_tiles, total, whole,
-                       width, partials);
+    return p;
+}
+
+template <int G, int NT, int NW>
+int launch_tile(const Q4Launch &L, const XhList &xh, const float *ss, float *ws, int KS, int partials, int total, hipStream_t st) {
+    const TilePlan p = plan_tiles(16 * NT, total * KS, L.batch, NW == 8);
+    if constexpr (NT == 4 && NW == 8 && G >= 64) // (groups of 32 have more scales, and no LDS for it)
+        if (plan_tiles(80, total * KS, L.batch, true).cost < 0.98f * p.cost) return launch_tile<G, 5, 8>(L, xh, ss, ws, KS, partials, total, st);
+    size_t lds = 0;
+    L2_TRY((ready_tile<G, NT, NW>(&lds)));
+    const int t_tiles = (L.batch + 16 * NT - 1) / (16 * NT);
+    l2_launch(q4_tile_gemm_kernel<G, NT, NW>, dim3(p.blocks), dim3(64 * NW), lds, st, L, xh, gemm_padded(L.in), ss, ws, KS, t_tiles, total, p.whole,
+              p.width, partials);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }
@@ -1066,6 +1092,7 @@ int ready_group() {
     L2_TRY((ready_tile<G, 1, 4>(&lds)));
     L2_TRY((ready_tile<G, 2, 4>(&lds)));
     L2_TRY((ready_tile<G, 4, 8>(&lds)));
+    if constexpr (G >= 64) L2_TRY((ready_tile<G, 5, 8>(&lds)));
     return L2_OK;
 }
 

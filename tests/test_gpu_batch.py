@@ -317,6 +317,26 @@ def test_columns_mode(ops):
         m.close()
 
 
+# tiles of 80 columns, and what rounds leave over in 16, 32 and 48: last tiles of 1, 49, 70 and 80, one, two and three units of K, half a
+# one; a column is the bits it has in a batch of 64
+@pytest.mark.parametrize("n_in,n_out,G,batches", [(128, 22016, 64, (150, 160)), (256, 22016, 128, (129, 150, 225)), (320, 22016, 64, (150,)),
+                                                  (384, 22016, 32, (130, 90)), (384, 12800, 128, (230,))])
+def test_batch_tiles_of_80(ops, n_in, n_out, G, batches):
+    rng = np.random.default_rng(n_in + G)
+    qw, qz, sc, gi = ck.synth_qlinear(rng, n_in, n_out, G, act_order=True)
+    W = ck.dequant_bin(qw, qz, sc, gi, G).astype(np.float64)
+    q = ops.QLinear(qw, qz, sc, gi, G)
+    x = rng.standard_normal((max(batches), n_in)).astype(np.float32)
+    want = x.astype(np.float64) @ W.T
+    of_64 = np.concatenate([q.matvec(x[b:b + 64]) for b in range(0, len(x), 64)])
+    for B in batches:
+        got = q.matvec(x[:B])
+        np.testing.assert_array_equal(got[:B // 64 * 64], of_64[:B // 64 * 64])
+        for b in range(B):
+            assert nrel(got[b], want[b]) < 1e-5, (B, b)
+    q.close()
+
+
 # fp16 prompts: the last tile of tokens in each of its widths, behind tiles of 128 tokens and of 64
 @pytest.mark.parametrize("G,batches", [(32, (65, 100)), (64, (65, 257, 300, 340, 370)), (128, (65, 272, 300, 340, 370))])
 def test_fp16_operator_last_tile(ops, G, batches):
