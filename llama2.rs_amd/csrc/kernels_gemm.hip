@@ -992,35 +992,61 @@ __global__ __launch_bounds__(512) void gemm_rope_kv_kernel(const RopeKvArgs A) {
 }
 
 // The SiLU gate (src/models.rs:92-98) behind w1|w3 of a chunk: add the partial tiles of both, apply the token's rms
-// scale, gate, and hand the row to w2 in its act-order (permuted in LDS).  One block per token; with few slices in 64
+// scale, gate, and hand the row to w2 in its act-order (permuted in LDS, as fp16 where that is what w2 reads: 28672 values in fp32
+// were all the LDS that one block per CU has).  One block per token, two trips' loads in flight; with few slices in 64
 // registers, two blocks per CU: 11008 values, 511 tokens 13.6 -> 11.4 us.
 template <int NP, int SL>
 __global__ __launch_bounds__(1024, SL <= 2 ? 8 : 4) void gemm_silu_kernel(const SiluArgs A) {
-    extern __shared__ __align__(16) float perm[]; // [n]
-    const int t = blockIdx.x, tid = threadIdx.x, n = A.n, in_p = gemm_padded(n);
+    typedef std::conditional_t<NP == 1, _Float16, float> In;
+    extern __shared__ __align__(16) char perm_lds[];
+    In *const perm = reinterpret_cast<In *>(perm_lds); // [n]
+    const int t = blockIdx.x, tid = threadIdx.x, n = A.n, in_p = gemm_padded(n), n4 = n >> 2;
     const size_t slice = (size_t)A.B * n, row = (size_t)t * n;
     const float ss = A.ss[t];
-    for (int i4 = tid; i4 < (n >> 2); i4 += 1024) {
-        const int4 id = A.inv ? *reinterpret_cast<const int4 *>(A.inv + 4 * i4) : make_int4(4 * i4, 4 * i4 + 1, 4 * i4 + 2, 4 * i4 + 3);
-        const float4 a = sum_slices_n<SL>(A.ws + row + 4 * i4, slice, A.KS);
-        const float4 c = sum_slices_n<SL>(A.ws + A.KS * slice + row + 4 * i4, slice, A.KS);
-        const float as[4] = {a.x, a.y, a.z, a.w}, cs[4] = {c.x, c.y, c.z, c.w};
-        const int ids[4] = {id.x, id.y, id.z, id.w};
+    constexpr int U = SL <= 2 ? 2 : 1;
+    for (int i0 = tid; i0 < n4; i0 += U * 1024) {
+        int4 id[U];
+        float4 a[U], c[U];
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            float s = as[e] * ss;
-            s = s * (1.0f / (1.0f + expf(-s)));
-            perm[ids[e]] = s * (cs[e] * ss);
+        for (int u = 0; u < U; u++) {
+            const int i4 = min(i0 + u * 1024, n4 - 1);
+            id[u] = A.inv ? *reinterpret_cast<const int4 *>(A.inv + 4 * i4) : make_int4(4 * i4, 4 * i4 + 1, 4 * i4 + 2, 4 * i4 + 3);
+            a[u] = sum_slices_n<SL>(A.ws + row + 4 * i4, slice, A.KS);
+            c[u] = sum_slices_n<SL>(A.ws + A.KS * slice + row + 4 * i4, slice, A.KS);
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (u > 0 && i0 + u * 1024 >= n4) break;
+            const float as[4] = {a[u].x, a[u].y, a[u].z, a[u].w}, cs[4] = {c[u].x, c[u].y, c[u].z, c[u].w};
+            const int ids[4] = {id[u].x, id[u].y, id[u].z, id[u].w};
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                float s = as[e] * ss;
+                s = s * (1.0f / (1.0f + expf(-s)));
+                s = s * (cs[e] * ss);
+                if constexpr (NP == 1) {
+                    asm("" : "+v"(s)); // rounded to fp32 first, as ever
+                    perm[h16_slot(ids[e])] = (_Float16)s;
+                } else {
+                    perm[ids[e]] = s;
+                }
+            }
         }
     }
     __syncthreads();
     for (int j8 = tid; j8 < (in_p >> 3); j8 += 1024) {
-        float e[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        if (8 * j8 < n) {
-            const float4 a = *reinterpret_cast<const float4 *>(&perm[8 * j8]), b = *reinterpret_cast<const float4 *>(&perm[8 * j8 + 4]);
-            e[0] = a.x, e[1] = a.y, e[2] = a.z, e[3] = a.w, e[4] = b.x, e[5] = b.y, e[6] = b.z, e[7] = b.w;
+        if constexpr (NP == 1) { // as the GEMM wants them already
+            Piece<NP> r{};
+            if (8 * j8 < n) r.q[0] = *reinterpret_cast<const uint4 *>(&perm[8 * j8]);
+            store_piece<NP>(A.out_h, t, in_p, j8, r);
+        } else {
+            float e[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            if (8 * j8 < n) {
+                const float4 a = *reinterpret_cast<const float4 *>(&perm[8 * j8]), b = *reinterpret_cast<const float4 *>(&perm[8 * j8 + 4]);
+                e[0] = a.x, e[1] = a.y, e[2] = a.z, e[3] = a.w, e[4] = b.x, e[5] = b.y, e[6] = b.z, e[7] = b.w;
+            }
+            store_piece<NP>(A.out_h, t, in_p, j8, make_piece<NP>(e));
         }
-        store_piece<NP>(A.out_h, t, in_p, j8, make_piece<NP>(e));
     }
 }
 
@@ -1278,7 +1304,7 @@ static int residual_norm(const ResNormPrep &A, hipStream_t st) {
 }
 template <int NP, int TRIPS>
 static int residual_norm(const ResNormPrep &A, hipStream_t st) {
-    return A.KS <= 2 ? residual_norm<NP, TRIPS, 2>(A, st) : A.KS <= 4 ? residual_norm<NP, TRIPS, 4>(A, st) : A.KS <= 8 ? residual_norm<NP, TRIPS, 8>(A, st) : residual_norm<NP, TRIPS, kMaxGemmSlices>(A, st);
+    return A.KS == 1 ? residual_norm<NP, TRIPS, 1>(A, st) : A.KS <= 2 ? residual_norm<NP, TRIPS, 2>(A, st) : A.KS <= 4 ? residual_norm<NP, TRIPS, 4>(A, st) : A.KS <= 8 ? residual_norm<NP, TRIPS, 8>(A, st) : residual_norm<NP, TRIPS, kMaxGemmSlices>(A, st);
 }
 template <int NP>
 static int residual_norm(const ResNormPrep &A, hipStream_t st) {
@@ -1296,7 +1322,8 @@ int gemm_rope_kv_launch(const RopeKvArgs &A, hipStream_t st) {
     if (A.KS < 1 || A.KS > kMaxGemmSlices || A.B < 1 || A.n_heads < A.n_kv_heads)
         return l2_fail(L2_ERR_ARG, "q|k|v epilogue: %d slices, %d tokens", A.KS, A.B);
     const dim3 grid(A.B, (A.n_heads * 16 + A.n_kv_heads * 48 + 511) / 512), block(512); // a thread per eight of q and k, four of v
-    if (A.KS <= 2) l2_launch(gemm_rope_kv_kernel<2>, grid, block, 0, st, A);
+    if (A.KS == 1) l2_launch(gemm_rope_kv_kernel<1>, grid, block, 0, st, A);
+    else if (A.KS <= 2) l2_launch(gemm_rope_kv_kernel<2>, grid, block, 0, st, A);
     else if (A.KS <= 4) l2_launch(gemm_rope_kv_kernel<4>, grid, block, 0, st, A);
     else if (A.KS <= 8) l2_launch(gemm_rope_kv_kernel<8>, grid, block, 0, st, A);
     else l2_launch(gemm_rope_kv_kernel<kMaxGemmSlices>, grid, block, 0, st, A);
@@ -1306,7 +1333,7 @@ int gemm_rope_kv_launch(const RopeKvArgs &A, hipStream_t st) {
 
 template <int NP, int SL>
 static int silu(const SiluArgs &A, hipStream_t st) {
-    const size_t lds = (size_t)A.n * sizeof(float);
+    const size_t lds = (size_t)A.n * (NP == 1 ? sizeof(_Float16) : sizeof(float));
     static LdsLimit limit(48 * 1024);
     L2_TRY(limit.ensure(reinterpret_cast<const void *>(gemm_silu_kernel<NP, SL>), lds));
     l2_launch((gemm_silu_kernel<NP, SL>), dim3(A.B), dim3(1024), lds, st, A);
@@ -1315,7 +1342,7 @@ static int silu(const SiluArgs &A, hipStream_t st) {
 }
 template <int NP>
 static int silu(const SiluArgs &A, hipStream_t st) {
-    return A.KS <= 2 ? silu<NP, 2>(A, st) : A.KS <= 4 ? silu<NP, 4>(A, st) : A.KS <= 8 ? silu<NP, 8>(A, st) : silu<NP, kMaxGemmSlices>(A, st);
+    return A.KS == 1 ? silu<NP, 1>(A, st) : A.KS <= 2 ? silu<NP, 2>(A, st) : A.KS <= 4 ? silu<NP, 4>(A, st) : A.KS <= 8 ? silu<NP, 8>(A, st) : silu<NP, kMaxGemmSlices>(A, st);
 }
 
 int gemm_silu_launch(const SiluArgs &A, int planes, hipStream_t st) {

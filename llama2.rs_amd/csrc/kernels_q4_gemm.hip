@@ -445,12 +445,13 @@ int launch_gemm(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const
     // Tiles of 144 tokens where they take less (and not about the same: 7B, 899 tokens, a cost of 1.00, 3485 -> 3523 us for six layers).
     if constexpr (NT == 8)
         if (plan_tiles(144, row_blocks * s.slices, L.batch, beside).cost < 0.98f * p.cost) return launch_gemm<G, 9, NW>(L, xh, ss, ws, s, partials, beside, st);
-    // partial tiles past the caches where they would fill them: what a launch leaves dirty there is written back at its end
-    // (7B, 511 tokens: the four launches 13 us less per layer, their consumers 5 more; below 16 MB the other way round: there they
-    // go past the L2 but not past the memory-side cache, see store_through)
+    // Partial tiles past the L2 (what a launch leaves dirty there is written back at its end, see store_through), and past the memory-side
+    // cache too where they would fill it: up to 100 MB their consumer finds them there.  Above 16, 64, 100 MB: 7B, 511 tokens 11270 /
+    // 11032 / 11038 us; six layers of 7B, 299, 699, 899 1700 / 2768 / 3570, 1666 / 2721 / 3537 and 1673 / 2720 / 3514; four of 13B, 249
+    // 1364 / 1351 / 1346; none past it: 899 tokens of 13B 3606 -> 3631, 70B's 776 (178 MB of w1|w3) 13.39 -> 13.43 ms.
     size_t bytes = 0;
     for (int i = 0; i < L.n_mats; i++) bytes += (size_t)s.slices * L.batch * L.m[i].out * 4;
-    if (partials && bytes > ((size_t)16 << 20)) partials = 2;
+    if (partials && bytes > ((size_t)100 << 20)) partials = 2;
     const dim3 grid(p.blocks), block(64 * NW);
     // the tiles, or the output staging tiles of the epilogue (32 x 36 floats per wave)
     const size_t lds = std::max(GemmLds<G, NW>::size(TN), (size_t)NW * 32 * 36 * sizeof(float));
