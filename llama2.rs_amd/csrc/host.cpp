@@ -1432,7 +1432,8 @@ extern "C" int l2_model_classifier(l2_model *m, const float *x_host, float *y_ho
 // and the launch as long as those: 70B behind 4096 positions 18.6 -> 16.5 us per layer, 13B behind 1000 positions
 // 16.7 -> 15.3, 7B unchanged; half a block per CU is slower everywhere.)
 static void attn_split_policy(int n_t, int n_heads, int n_kv_heads, int *ts_out, int *n_splits_out) {
-    const int whole = n_kv_heads > 32 ? 768 : n_heads >= 32 ? 1024 : n_heads > n_kv_heads ? 896 : 640;
+    int whole = n_kv_heads > 32 ? 768 : n_heads >= 32 ? 1024 : n_heads > n_kv_heads ? 896 : 640;
+    if (n_heads == 8 * n_kv_heads && n_t <= kFewTimesteps) whole = kFewTimesteps;
     if (n_t <= whole) {
         *ts_out = whole;
         *n_splits_out = 1;

@@ -481,6 +481,15 @@ __global__ __launch_bounds__(256, 2) void attn_decode_mfma_kernel(const AttnDeco
         qa[r] = qh[i], qb[r] = qh[i + HALF];
         qc[r] = ct[i], qsn[r] = st[i];
     }
+    // where this thread's outputs go when the step is not split: fetched now, used at the very end
+    int sdst[QG * HS / NT];
+    if constexpr (QG == 8) {
+#pragma unroll
+        for (int u = 0; u < QG * HS / NT; u++) {
+            const int i = kvh * QG * HS + tid + u * NT;
+            sdst[u] = (A.scatter && A.n_splits == 1) ? A.scatter[i] : i;
+        }
+    }
     const int hd = tid & 63;
     const float nk_a = A.k_new[(size_t)kvh * HS + hd], nk_b = A.k_new[(size_t)kvh * HS + hd + HALF];
     const float nv = A.v_new[(size_t)kvh * HS + (tid & 127)];
@@ -652,6 +661,10 @@ __global__ __launch_bounds__(256, 2) void attn_decode_mfma_kernel(const AttnDeco
         const int idx = tid + u * NT;
         const int j = idx >> 7, d = idx & 127;
         const int h = kvh * QG + j;
+        if (QG == 8 && A.n_splits == 1) {
+            A.out[sdst[u]] = num[u] / den[u];
+            continue;
+        }
         float *pp = A.part + ((size_t)h * A.max_splits + sp) * (HS + 2);
         pp[d] = num[u];
         if (d == 0) {
@@ -1122,16 +1135,19 @@ int attn_launch_sliced(const AttnDecode &a, hipStream_t st) {
 
 template <int QG>
 int attn_launch_qg(const AttnDecode &a, hipStream_t st) {
-    if (a.n_splits == 1) { // slices of the head: as many as keep one block per CU
+    static const bool valu = []() {
+        const char *v = getenv("L2_ATTN_IMPL");
+        return v && !strcmp(v, "valu");
+    }();
+    // With eight query heads per kv head the first 256 timesteps stay on the matrix cores: in other sums the texts that are sampled from
+    // a model are others (of 20 of 60 tokens from 70B's widths three were).  64 heads of 8, 50, 240 timesteps 37.0 / 42.0 us per layer, with blocks of one head
+    // 35.4 / 36.7.
+    if (a.n_splits == 1 && (QG < 8 || valu || a.ts > kFewTimesteps)) { // slices of the head: as many as keep one block per CU
         const bool wide = a.pos >= 64, eight = a.n_heads * 8 <= cu_count();
         if (eight) return wide ? attn_launch_sliced<8, 8>(a, st) : attn_launch_sliced<4, 8>(a, st);
         return wide ? attn_launch_sliced<8, 4>(a, st) : attn_launch_sliced<4, 4>(a, st);
     }
     if constexpr (QG >= 4) {
-        static const bool valu = []() {
-            const char *v = getenv("L2_ATTN_IMPL");
-            return v && !strcmp(v, "valu");
-        }();
         if (!valu) {
             l2_launch((attn_decode_mfma_kernel<QG>), dim3(a.n_kv_heads, a.n_splits), dim3(256), 0, st, a);
             L2_HIP(hipGetLastError());

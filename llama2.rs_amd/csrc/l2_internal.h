@@ -343,6 +343,8 @@ int attention_launch(void *out, int planes, const float *q, const float *kcache_
                      const int32_t *pos, const int32_t *scatter, int n_heads, int n_kv_heads,
                      int head_size, int max_pos, int B, hipStream_t st);
 
+// Up to so many timesteps eight query heads per kv head go together (attn_launch_qg).
+constexpr int kFewTimesteps = 256;
 // Decode attention (one query) with RoPE and the cache write folded in.
 struct AttnDecode {
     const float *q;      // [dim]    raw query of this step
