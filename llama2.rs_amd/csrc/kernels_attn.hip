@@ -80,8 +80,9 @@ static_assert(kCombRow * sizeof(float) % 16 == 0, "rows of the merge tiles are w
 // against 1227 with 8 waves), 8 beyond (190: 381 against 383 with 8 layers).  The query heads of one kv head (grouped-query
 // attention, src/models.rs:142-145) are blocks of their own too: they read the same rows out of the same XCD's L2 (blocks are dealt
 // over the XCDs by kv head), and a block has one chain of scores and sums instead of four or eight.  Whole layers, against a block for
-// all heads of the kv head (at 8 of them on the matrix cores), at 50, 100, 240 timesteps: 16 heads of 2 kv heads 22.8 / 24.1 / 27.4 ->
-// 21.9 / 22.6 / 22.9 us, 32 of 4 28.3 / 29.8 / 31.8 -> 25.7 / 25.7 / 26.8, 64 of 8 37.0 / 38.3 / 42.0 -> 35.4 / 35.8 / 36.7.
+// all heads of the kv head (in splits beyond 256), at 50, 100, 240 timesteps: 16 heads of 2 kv heads 22.8 / 24.1 / 27.4 ->
+// 21.9 / 22.6 / 22.9 us, 32 of 4 28.3 / 29.8 / 31.8 -> 25.7 / 25.7 / 26.8, 64 of 8 at 500, 800 40.5 / 42.1 -> 37.7 / 38.7 (not taken for
+// eight up to 256, see attn_launch_qg).
 // Longer contexts are cut into splits of timesteps (DS = 1, 4 waves) that attn_combine_kernel merges; there all QG query heads
 // of the kv head share each K and V load.
 template <int QG, int NWV, int DS>
