@@ -16,6 +16,8 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <type_traits>
+
 #include "l2_internal.h"
 #include "lanes.h"
 
@@ -956,7 +958,7 @@ void attn_prefill_mfma16_kernel(void *__restrict__ out, const float *__restrict_
 
     // A tile's scores, then its weighted sums.  K of the next tile is requested as soon as the scores have been taken and
     // V as soon as the sums have, so that each arrives behind the other's products.
-    for (int tile = wave; tile < n_tiles; tile += NWV) {
+    auto step = [&](int tile, auto last) __attribute__((always_inline)) {
         const int tb = tile * TK;
         float p[CS][4];
 #pragma unroll
@@ -1002,7 +1004,7 @@ void attn_prefill_mfma16_kernel(void *__restrict__ out, const float *__restrict_
                 R.l += p[cs][r];
             }
         }
-        if (tile + NWV < n_tiles) fetch_k(tile + NWV);
+        if (!last) fetch_k(tile + NWV);
 #pragma unroll
         for (int cs = 0; cs < CS; cs++) {
             v4f(&acc)[8] = run[cs].acc;
@@ -1020,8 +1022,13 @@ void attn_prefill_mfma16_kernel(void *__restrict__ out, const float *__restrict_
                 acc[7] = __builtin_amdgcn_mfma_f32_16x16x4f32(v1.w, pr, acc[7], 0, 0, 0);
             }
         }
-        if (tile + NWV < n_tiles) fetch_v(tile + NWV);
-    }
+        if (!last) fetch_v(tile + NWV);
+    };
+    // The last tile apart: with a branch around the loads of the next tile these are copied, and waited for, where the branch
+    // ends.  32 heads, 64 tokens behind 1500 rows 40.1 -> 36.3 us, 511 tokens 30.5 -> 29.6; 64 heads on 8 kv heads, 777 108.9 -> 105.5.
+    int tile = wave;
+    for (; tile + NWV < n_tiles; tile += NWV) step(tile, std::false_type());
+    if (tile < n_tiles) step(tile, std::true_type());
 
 #pragma unroll
     for (int cs = 0; cs < CS; cs++) {
