@@ -873,13 +873,13 @@ __device__ __forceinline__ int column_tile(int y, int n, int unit_rows) {
 // tokens 8.6, 7.9.  (v_mfma_f32_16x16x4_f32 at its peak: 63 us for the first of these.)  (A form on 32 columns and tiles of 32 rows,
 // v_mfma_f32_32x32x2_f32 with K and V turned through LDS, had half the blocks and took 16 to 31 us per chunk of a
 // 512-token prompt where this one takes 11 to 19.)
-template <int QG, int NWV, int NP, int CS>
+template <int QG, int NWV, int CS>
 __global__ __launch_bounds__(NWV * 64, NWV == 4 ? 2 : 1)
 void attn_prefill_mfma16_kernel(void *__restrict__ out, const float *__restrict__ q, const float *__restrict__ kc,
                                 const float *__restrict__ vc, const int32_t *__restrict__ pos,
                                 const int32_t *__restrict__ scatter, int n_heads, int n_kv_heads, int B, int max_pos,
                                 int unit_rows) {
-    constexpr int NT = NWV * 64, TK = 16, HS = 128, HALF = 64, NC = 16, QPT = NC / QG;
+    constexpr int NP = 3, NT = NWV * 64, TK = 16, HS = 128, HALF = 64, NC = 16, QPT = NC / QG;
     __shared__ __align__(16) float comb[NWV][NC][kCombRow];
     __shared__ float4 qs[CS > 1 ? CS : 1][CS > 1 ? 8 : 1][64]; // several sets: their B operands
     const int kvh = blockIdx.x, ct = column_tile(blockIdx.y, gridDim.y, unit_rows) * CS;
@@ -1069,19 +1069,294 @@ void attn_prefill_mfma16_kernel(void *__restrict__ out, const float *__restrict_
             if (qi < B) {
                 const int to = dst[u % HEADS];
                 const float v = nu / de;
-                if constexpr (NP == 1) {
-                    reinterpret_cast<_Float16 *>(out)[(size_t)qi * dim + h16_slot(to)] = (_Float16)v;
-                } else { // three bf16 numbers that add up to v exactly
-                    uint16_t *o = reinterpret_cast<uint16_t *>(out) + (size_t)qi * NP * dim + b16_slot(to);
-                    float left = v;
+                // three bf16 numbers that add up to v exactly
+                uint16_t *o = reinterpret_cast<uint16_t *>(out) + (size_t)qi * NP * dim + b16_slot(to);
+                float left = v;
 #pragma unroll
-                    for (int p = 0; p < NP; p++) {
-                        const uint32_t bits = __builtin_bit_cast(uint32_t, left) & 0xFFFF0000u;
-                        o[(size_t)p * dim] = (uint16_t)(bits >> 16);
-                        left -= __builtin_bit_cast(float, bits);
-                    }
+                for (int p = 0; p < NP; p++) {
+                    const uint32_t bits = __builtin_bit_cast(uint32_t, left) & 0xFFFF0000u;
+                    o[(size_t)p * dim] = (uint16_t)(bits >> 16);
+                    left -= __builtin_bit_cast(float, bits);
                 }
             }
+        }
+    }
+}
+
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+
+// Two fp32 numbers as three pairs of bf16 numbers each, cut after the first, second and third byte of the significand: exact.
+// What a cut leaves is one v_dot2_f32_bf16 of the pair that was cut off with (-1, 0) or (0, -1).
+struct Cut {
+    uint32_t p[3];
+    __device__ __forceinline__ Cut(float x, float y, uint32_t minus_lo, uint32_t minus_hi) {
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            p[k] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, y), __builtin_bit_cast(uint32_t, x), 0x07060302u);
+            if (k == 2) break;
+            x = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(b2, p[k]), __builtin_bit_cast(b2, minus_lo), x, false);
+            y = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(b2, p[k]), __builtin_bit_cast(b2, minus_hi), y, false);
+        }
+    }
+};
+struct Plane {
+    uint32_t u[4];
+    __device__ __forceinline__ b8 b() const { return __builtin_bit_cast(b8, *this); }
+};
+
+// The same for the fp16 mode (L2_PREFILL_MFMA), on v_mfma_f32_16x16x32_bf16 with every fp32 number cut into three bf16 numbers
+// (sixteen times the rate of v_mfma_f32_16x16x4_f32): six products, down to 2^-16 of the first; the three left out are below an
+// fp32 rounding.  Relative rms error against fp64, 33 to 777 queries over up to 2040 rows, of that of the fp32 form: normal inputs
+// 0.49 to 0.77, sharper scores on values of one sign 0.63 to 1.04 (32 rows).  Blocks, columns and tiles are the fp32 form's, and a column's
+// result depends on neither the other columns nor the number of sets: a pass gives the bits of the same tokens in several.
+//   - Scores contract over 32 dimensions: a lane holds 16 m + 4 kb .. + 3 of two m, of K as of Q.
+//   - The sums contract over the 16 rows of a tile, so one instruction takes two products: half its contraction is one plane of
+//     V times one of the weights, half another.
+//   - K, V and the weights are cut by the wave that uses them, 7 vector instructions a pair of numbers (4 of them the dot
+//     products of Cut; with masks and subtractions 11), Q once per block.
+// What bounds it is the issue of vector instructions, most of them the cutting (half of a SIMD's cycles; the matrix unit's 28 %).
+// Against the fp32 form, per launch: 32 heads, 16, 64, 128, 299, 511 tokens 5.5, 6.2, 8.0, 19.3, 29.6 -> 4.7, 5.2, 6.8, 15.6, 24.2 us;
+// 128 tokens behind 384 17.2 -> 15.0, 64 behind 1500 36.3 -> 33.8; 64 heads on 8 kv heads, 128, 777 tokens 10.7, 105.5 -> 9.4, 79.8.
+// Tiles of 32 rows, a product per instruction: 16, 128 and 777 of these tokens 6.0, 7.5 and 86.0; rescaling whenever a maximum
+// moves: 511 and 777 tokens 26.0 and 83.7.
+template <int QG, int CS>
+__global__ __launch_bounds__(256, 2)
+void attn_prefill_cut_kernel(void *__restrict__ out, const float *__restrict__ q, const float *__restrict__ kc,
+                             const float *__restrict__ vc, const int32_t *__restrict__ pos,
+                             const int32_t *__restrict__ scatter, int n_heads, int n_kv_heads, int B, int max_pos,
+                             int unit_rows) {
+    constexpr int NWV = 4, TK = 16, HS = 128, NC = 16, QPT = NC / QG;
+    __shared__ __align__(16) float comb[NWV][NC][kCombRow];
+    __shared__ float2 ml[CS][NWV][NC];
+    __shared__ uint4 qs[CS][4][3][64]; // the columns' B operands: [set][32 dimensions][plane][lane]
+    const int kvh = blockIdx.x, ct = column_tile(blockIdx.y, gridDim.y, unit_rows) * CS;
+    const int dim = n_heads * HS, kv_dim = n_kv_heads * HS;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 15, kb = lane >> 4;
+    const uint32_t row_bytes = (uint32_t)kv_dim * 4u;
+    const uint32_t k_lane = (uint32_t)(kvh * HS + 4 * kb) * 4u; // + 64 m bytes
+    const uint32_t v_lane = (uint32_t)(kvh * HS + 4 * li) * 4u; // + 256 bytes for the second half of d
+    uint32_t minus_lo = 0x0000BF80u, minus_hi = 0xBF800000u; // (-1, 0) and (0, -1) as bf16, in registers
+    asm volatile("" : "+s"(minus_lo), "+s"(minus_hi));
+    // 32 dimensions of a row: four pairs of a, the next four of b
+    auto cut8 = [&](const float4 a, const float4 b, Plane(&c)[3]) __attribute__((always_inline)) {
+        const Cut w[4] = {{a.x, a.y, minus_lo, minus_hi}, {a.z, a.w, minus_lo, minus_hi}, {b.x, b.y, minus_lo, minus_hi}, {b.z, b.w, minus_lo, minus_hi}};
+#pragma unroll
+        for (int k = 0; k < 3; k++) c[k] = Plane{{w[0].p[k], w[1].p[k], w[2].p[k], w[3].p[k]}};
+    };
+
+    // Unconditional loads: rows past the last one written re-read it (masked below).
+    float4 x[8]; // x[m]: K[t = li][16 m + 4 kb ..]
+    float4 v[8]; // v[2 r + half]: V[t = 4 kb + r][64 half + 4 li ..]
+    auto fetch_k = [&](int tile) __attribute__((always_inline)) {
+        const uint32_t ko = __umul24(min(tile * TK + li, max_pos), row_bytes) + k_lane;
+#pragma unroll
+        for (int m = 0; m < 8; m++) x[m] = ld_at<float4>(kc, ko + 64u * m);
+    };
+    auto fetch_v = [&](int tile) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const uint32_t vo = __umul24(min(tile * TK + 4 * kb + r, max_pos), row_bytes) + v_lane;
+            v[2 * r] = ld_at<float4>(vc, vo);
+            v[2 * r + 1] = ld_at<float4>(vc, vo + 256u);
+        }
+    };
+    int my_pos[CS];
+    float4 qa[CS], qb[CS];
+#pragma unroll
+    for (int cs = 0; cs < CS; cs++) {
+        const int my_qi = (ct + cs) * QPT + li / QG;
+        my_pos[cs] = my_qi < B ? pos[my_qi] : -1;
+        // wave w cuts dimensions 32 w .. 32 w + 31
+        const float *qrow = q + (size_t)min(my_qi, B - 1) * dim + (size_t)(kvh * QG + li % QG) * HS + 32 * wave + 4 * kb;
+        qa[cs] = *reinterpret_cast<const float4 *>(qrow), qb[cs] = *reinterpret_cast<const float4 *>(qrow + 16);
+    }
+    fetch_k(wave);
+    fetch_v(wave);
+    constexpr int PER = NWV * 64 / HS, HEADS = QG > PER ? QG / PER : 1;
+    int dst[HEADS]; // where this thread's outputs go (as in the kernel above)
+#pragma unroll
+    for (int u = 0; u < HEADS; u++) {
+        const int i = (kvh * QG + (tid / HS + u * PER) % QG) * HS + tid % HS;
+        dst[u] = scatter ? scatter[i] : i;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int cs = 0; cs < CS; cs++) {
+        Plane c[3];
+        cut8(qa[cs], qb[cs], c);
+#pragma unroll
+        for (int k = 0; k < 3; k++) qs[cs][wave][k][lane] = make_uint4(c[k].u[0], c[k].u[1], c[k].u[2], c[k].u[3]);
+    }
+    int t_end = my_pos[0] + 1; // the block's tiles end with the last row any of its columns sees
+#pragma unroll
+    for (int cs = 1; cs < CS; cs++) t_end = max(t_end, my_pos[cs] + 1);
+#pragma unroll
+    for (int off = 8; off > 0; off >>= 1) t_end = max(t_end, __shfl_xor(t_end, off));
+    t_end = __builtin_amdgcn_readfirstlane(t_end);
+    const int n_tiles = (t_end + TK - 1) / TK;
+
+    float run_m[CS], run_l[CS];
+    v4f acc[CS][8];
+#pragma unroll
+    for (int cs = 0; cs < CS; cs++) {
+        run_m[cs] = kNoScore, run_l[cs] = 0.f;
+#pragma unroll
+        for (int c = 0; c < 8; c++) acc[cs][c] = v4f{0.f, 0.f, 0.f, 0.f};
+    }
+    const float scale = 1.44269504088896340736f / sqrtf((float)HS); // log2(e) / sqrt(head_size), src/models.rs:154
+    float sign = 1.f;
+    __syncthreads();
+
+    // What is cut next goes between the products of what was cut before; K and V of the next tile are asked for when the last of
+    // this one's has been cut.
+    auto step = [&](int tile, auto last) __attribute__((always_inline)) {
+        // Scores: K's planes times Q's, what is below the first planes' product summed apart.
+        v4f s[CS], lo[CS];
+        {
+            Plane kp[2][3], q0[2][CS];
+            auto ask = [&](int cs, int i, int k) __attribute__((always_inline)) {
+                const uint4 u = qs[cs][i][k][lane];
+                return Plane{{u.x, u.y, u.z, u.w}};
+            };
+            cut8(x[0], x[1], kp[0]);
+#pragma unroll
+            for (int cs = 0; cs < CS; cs++) q0[0][cs] = ask(cs, 0, 0), s[cs] = lo[cs] = v4f{0.f, 0.f, 0.f, 0.f};
+            if (CS > 1) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const Plane(&c)[3] = kp[i % 2];
+                Plane q1[CS], q2[CS];
+#pragma unroll
+                for (int cs = 0; cs < CS; cs++) q1[cs] = ask(cs, i, 1);
+#pragma unroll
+                for (int cs = 0; cs < CS; cs++) q2[cs] = ask(cs, i, 2);
+                if (i < 3) {
+#pragma unroll
+                    for (int cs = 0; cs < CS; cs++) q0[(i + 1) % 2][cs] = ask(cs, i + 1, 0);
+                    cut8(x[2 * i + 2], x[2 * i + 3], kp[(i + 1) % 2]);
+                }
+#define L2_SCORES(D, KP, Q) _Pragma("unroll") for (int cs = 0; cs < CS; cs++) D[cs] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c[KP].b(), Q[cs].b(), D[cs], 0, 0, 0)
+                L2_SCORES(lo, 2, q0[i % 2]);
+                L2_SCORES(s, 0, q0[i % 2]);
+                L2_SCORES(lo, 1, q0[i % 2]);
+                L2_SCORES(lo, 1, q1);
+                L2_SCORES(lo, 0, q1);
+                L2_SCORES(lo, 0, q2);
+#undef L2_SCORES
+                if (CS > 1 || i == 3) __builtin_amdgcn_sched_barrier(0);
+                if (i == 2 && !last) fetch_k(tile + NWV);
+            }
+        }
+        // Weights, their planes as the sums take them: (0, 2), (1, 1) and (0, 0)
+        Plane pc[CS][3];
+#pragma unroll
+        for (int cs = 0; cs < CS; cs++) {
+            float sc[4], mx = kNoScore;
+            const int see = my_pos[cs] - tile * TK - 4 * kb; // causal: this column's query sees rows 0..pos
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                sc[r] = r <= see ? (s[cs][r] + lo[cs][r]) * scale : kNoScore;
+                mx = fmaxf(mx, sc[r]);
+            }
+            // A maximum moves only by more than 8, for the column that it is of: weights of up to 2^8 lose nothing in fp32, and what
+            // was summed is seldom rescaled.
+            if (__any(mx > run_m[cs] + 8.f)) {
+                mx = lanes::rows_max(mx); // the column's four lanes agree
+                const float m_new = mx > run_m[cs] + 8.f ? mx : run_m[cs];
+                const float c = exp2_fast(run_m[cs] - m_new);
+                run_l[cs] *= c;
+#pragma unroll
+                for (int cc = 0; cc < 8; cc++) acc[cs][cc] *= c;
+                run_m[cs] = m_new;
+            }
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const float p = r <= see ? exp2_fast(sc[r] - run_m[cs]) : 0.f;
+                run_l[cs] += p;
+                sc[r] = p * sign;
+            }
+            const Cut a(sc[0], sc[1], minus_lo, minus_hi), b(sc[2], sc[3], minus_lo, minus_hi);
+            pc[cs][0] = Plane{{a.p[0], b.p[0], a.p[2], b.p[2]}};
+            pc[cs][1] = Plane{{a.p[1], b.p[1], a.p[1], b.p[1]}};
+            pc[cs][2] = Plane{{a.p[0], b.p[0], a.p[0], b.p[0]}};
+        }
+        // V's planes times the weights', two products of 16 rows in one of 32: (2 0, 0 2), (1 1, 0 1), (1 0, 0 0).  Summed for the
+        // tile and added with the rounding of the vector unit: the matrix unit's sums come out too small on average, so
+        // every other tile's are taken negated.
+        {
+            Plane w[2][2]; // (2, 0) and (1, 0)
+            v4f t[2][CS];
+            auto cut = [&](int i) __attribute__((always_inline)) {
+                const int h = i / 4, e = i % 4;
+                const float4 r[4] = {v[h], v[2 + h], v[4 + h], v[6 + h]};
+                const Cut a(reinterpret_cast<const float *>(&r[0])[e], reinterpret_cast<const float *>(&r[1])[e], minus_lo, minus_hi);
+                const Cut b(reinterpret_cast<const float *>(&r[2])[e], reinterpret_cast<const float *>(&r[3])[e], minus_lo, minus_hi);
+                w[i % 2][0] = Plane{{a.p[2], b.p[2], a.p[0], b.p[0]}};
+                w[i % 2][1] = Plane{{a.p[1], b.p[1], a.p[0], b.p[0]}};
+            };
+            auto add = [&](int i) __attribute__((always_inline)) {
+#pragma unroll
+                for (int cs = 0; cs < CS; cs++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) acc[cs][i][r] = fmaf(t[i % 2][cs][r], sign, acc[cs][i][r]);
+            };
+            cut(0);
+            if (CS > 1) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const Plane(&c)[2] = w[i % 2];
+                if (i > 0) add(i - 1);
+                if (i < 7) cut(i + 1);
+#pragma unroll
+                for (int cs = 0; cs < CS; cs++) t[i % 2][cs] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c[0].b(), pc[cs][0].b(), v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+                for (int cs = 0; cs < CS; cs++) t[i % 2][cs] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c[1].b(), pc[cs][1].b(), t[i % 2][cs], 0, 0, 0);
+#pragma unroll
+                for (int cs = 0; cs < CS; cs++) t[i % 2][cs] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c[1].b(), pc[cs][2].b(), t[i % 2][cs], 0, 0, 0);
+                if (CS > 1 || i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+                if (i == 6 && !last) fetch_v(tile + NWV);
+            }
+            add(7);
+        }
+        sign = -sign;
+    };
+    // The last tile apart: with a branch around the loads for the next one they are waited for at once.
+    int tile = wave;
+    for (; tile + NWV < n_tiles; tile += NWV) step(tile, std::false_type());
+    if (tile < n_tiles) step(tile, std::true_type());
+
+    // The waves agree on each column's maximum and sum, each scales its O by its share, and these add up in LDS.
+#pragma unroll
+    for (int cs = 0; cs < CS; cs++) {
+        const float l = lanes::rows_sum(run_l[cs]);
+        if (kb == 0) ml[cs][wave][li] = make_float2(run_m[cs], l);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int cs = 0; cs < CS; cs++) {
+        float M = kNoScore, den = 0.f;
+#pragma unroll
+        for (int w = 0; w < NWV; w++) M = fmaxf(M, ml[cs][w][li].x);
+#pragma unroll
+        for (int w = 0; w < NWV; w++) den = fmaf(exp2_fast(ml[cs][w][li].x - M), ml[cs][w][li].y, den);
+        const float share = exp2_fast(run_m[cs] - M) / den;
+        if (cs > 0) __syncthreads(); // the set before has been read
+#pragma unroll
+        for (int c = 0; c < 8; c++) acc[cs][c] *= share;
+#pragma unroll
+        for (int r = 0; r < 4; r++) // register r of accumulators 0..3 is d = 16 kb + 4 r + 0..3, of 4..7 the same 64 further on
+#pragma unroll
+            for (int half = 0; half < 2; half++)
+                *reinterpret_cast<float4 *>(&comb[wave][li][64 * half + 16 * kb + 4 * r]) =
+                    make_float4(acc[cs][4 * half][r], acc[cs][4 * half + 1][r], acc[cs][4 * half + 2][r], acc[cs][4 * half + 3][r]);
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < NC * HS / (NWV * 64); u++) {
+            const int j = tid / HS + u * PER, d = tid % HS, qi = (ct + cs) * QPT + j / QG;
+            const float v = (comb[0][j][d] + comb[1][j][d]) + (comb[2][j][d] + comb[3][j][d]);
+            if (qi < B) reinterpret_cast<_Float16 *>(out)[(size_t)qi * dim + h16_slot(dst[u % HEADS])] = (_Float16)v;
         }
     }
 }
@@ -1200,22 +1475,28 @@ template <int QG>
 static int prefill_qg(void *out, int planes, const float *q, const float *kc, const float *vc, const int32_t *pos,
                       const int32_t *scatter, int n_heads, int n_kv_heads, int max_pos, int B, hipStream_t st) {
     // 16 columns (queries x heads of the group) per block, or 32 where that still leaves two blocks per CU: with fewer
-    // the longer blocks cost more than the shared tiles save (32 heads, 299 tokens: 18.6 us with 16, 19.7 with 32)
+    // the longer blocks cost more than the shared tiles save (32 heads, 299 tokens: 18.6 us with 16, 19.7 with 32).  In the fp16
+    // mode, which cuts a tile once for all its columns, from one block per CU on: 32 heads, 200 tokens (224 blocks of 32 columns) 10.2
+    // with 16 and 12.1 with 32, 64 on 8 kv heads, 128 (256) 9.4 and 9.5, 40 heads, 200 (280) 13.9 and 13.8, 32 heads, 299 (320)
+    // 17.5 and 15.6, 64 on 8, 777 106.8 and 79.8.
     const int sets = (B * QG + 15) / 16;
-    const bool two = (long)n_kv_heads * ((sets + 1) / 2) >= 2 * cu_count();
+    const long pairs = (long)n_kv_heads * ((sets + 1) / 2);
+    const bool two = planes == 1 ? pairs > cu_count() : pairs >= 2 * cu_count();
     const dim3 block(256), grid(n_kv_heads, two ? (sets + 1) / 2 : sets);
     const int cus = cu_count(), per_unit = cus / n_kv_heads, rows = (int)grid.y;
     const int unit_rows = cus % n_kv_heads == 0 && rows > per_unit && rows <= 2 * per_unit ? per_unit : 0; // see column_tile
-#define L2_PREFILL_ATTN(NP)                                                                                              \
-    if (two)                                                                                                             \
-        l2_launch((attn_prefill_mfma16_kernel<QG, 4, NP, 2>), grid, block, 0, st, out, q, kc, vc, pos, scatter, n_heads, n_kv_heads, B, max_pos, unit_rows); \
-    else                                                                                                                 \
-        l2_launch((attn_prefill_mfma16_kernel<QG, 4, NP, 1>), grid, block, 0, st, out, q, kc, vc, pos, scatter, n_heads, n_kv_heads, B, max_pos, unit_rows); \
-    break
+#define L2_PREFILL_ATTN(...)                                                                                             \
+    l2_launch((__VA_ARGS__), grid, block, 0, st, out, q, kc, vc, pos, scatter, n_heads, n_kv_heads, B, max_pos, unit_rows)
     switch (planes) {
         case 0: l2_launch(attn_prefill_kernel<QG>, dim3(n_kv_heads, (B * QG + 7) / 8), block, 0, st, (float *)out, q, kc, vc, pos, scatter, n_heads, n_kv_heads, B); break;
-        case 1: L2_PREFILL_ATTN(1);
-        case 3: L2_PREFILL_ATTN(3);
+        case 1:
+            if (two) L2_PREFILL_ATTN(attn_prefill_cut_kernel<QG, 2>);
+            else L2_PREFILL_ATTN(attn_prefill_cut_kernel<QG, 1>);
+            break;
+        case 3:
+            if (two) L2_PREFILL_ATTN(attn_prefill_mfma16_kernel<QG, 4, 2>);
+            else L2_PREFILL_ATTN(attn_prefill_mfma16_kernel<QG, 4, 1>);
+            break;
         default: return l2_fail(L2_ERR_ARG, "attention: %d planes", planes);
     }
 #undef L2_PREFILL_ATTN

@@ -481,6 +481,31 @@ def test_prompt_attention_two_sets(ops, n_heads, n_kv, n):
     m.close()
 
 
+# the fp16 mode's attention (three bf16 numbers for each fp32 one): blocks of one set of 16 columns and of two, one to eight query
+# heads per kv head, tiles of 16 rows and sets that end anywhere, an odd number of sets, rows of an earlier pass in front, against
+# the fp32 mode.  Rows of the second layer: five inputs of products rounded to fp16 on the way, 2^-11 / sqrt(3) each, sqrt(5) of it
+@pytest.mark.parametrize("n_heads,n_kv,at,n", [(2, 2, 0, 17), (4, 2, 5, 40), (8, 2, 61, 100), (8, 1, 300, 33), (32, 32, 0, 289), (32, 32, 61, 300),
+                                               (16, 8, 0, 701), (32, 8, 3, 260), (64, 8, 33, 255)])
+def test_fp16_prompt_attention(ops, n_heads, n_kv, at, n):
+    from llama2_rs import _lib
+    dims = ck.Dims(dim=128 * n_heads, hidden_dim=256, n_layers=2, n_heads=n_heads, n_kv_heads=n_kv, vocab_size=64,
+                   seq_len=1056, group_size=64)
+    m = ops.Model(ck.synth_weights_image(dims, seed=9), dims)
+    toks = np.random.default_rng(n).integers(0, 64, size=at + n).astype(np.int32)
+    rows = []
+    for mode in (_lib.PREFILL_MFMA, _lib.PREFILL_FP32):
+        m.reset()
+        m.set_prefill_mode(mode)
+        if at:
+            m.prefill_chunks(toks[:at], 0, at)
+        m.prefill_chunks(toks[at:], at, n)
+        rows.append(m.read_kv(1, at, n))
+    for got, want in zip(*rows):
+        e = np.sqrt(np.mean((got - want).astype(np.float64) ** 2, axis=(1, 2)) / np.mean(want.astype(np.float64) ** 2, axis=(1, 2)))
+        assert e.max() < 6.4e-4
+    m.close()
+
+
 # the kernels between the products of a chunk: rows of one, two and four trips of the block (and a consumer's order per
 # LDS row, or in turns), few K slices and many, in each kind of plane, against single tokens.  fp16 inputs carry 2^-11 each:
 # through the five products in front of the second layer's cache rows some 1e-3, and 4.5 times that at the furthest of
