@@ -519,19 +519,17 @@ __global__ __launch_bounds__(64 * NW, NT == 1 ? 3 : 2) void q4_tile_gemm_kernel(
 
 // Linear::matvec<B> of the model without quantisation (src/model.rs:22-31) for a batch: fp32 weights, fp32 activations,
 // on the bf16 matrix cores.  The activations are three bf16 planes as above; the weights become three on the way in, each
-// rounded to nearest, so that what a plane leaves over has either sign.  Eight of the nine products of a weight and an activation are
-// taken, all but that of the third planes: it is 2^-34 of the whole at most (2^-18 of the weight, 2^-16 of the activation), a
-// thousandth of what fp32 rounds off, and the launch is bound by the power of its products (1332 -> 1287 us for two layers
-// of 7B's widths, 100 tokens with the logits).  Relative rms error against fp64 with nine and with eight, 100 columns of 1024, 2816, 4096
-// and 11008 inputs: normal 6.938 7.674 8.891 9.318e-8 and the same to a digit more; one term 2.526 2.534 2.528 2.531e-8 in both; four
-// terms, one sign, one input 1e6 times the others: one differs by 9e-5 of itself (downwards), the others by less than 3e-5, up as often as
-// down; the largest errors are the same.  Numbers below 2^-109 have bits below bf16's smallest, 2^-133, and
-// enter as multiples of that.  That is 8 products at 2.5 PFLOP/s against one at the 157 TFLOP/s of v_mfma_f32_32x32x2_f32.
+// rounded to nearest, so that what a plane leaves over has either sign.  All nine products of a weight and an activation are
+// taken, so a product is exact as long as both planes are: numbers below 2^-109 have bits below bf16's smallest, 2^-133, and
+// enter as multiples of that.  That is 9 products at 2.5 PFLOP/s against one at the 157 TFLOP/s of v_mfma_f32_32x32x2_f32.  (The
+// product of the third planes is up to 2^-32 of the whole, 2^-17 of the weight times 2^-15 of the activation.  Without it two layers
+// of 7B's widths, 100 tokens with the logits, take 1287 us instead of 1332, but a term is then exact no more, which shows where
+// larger ones cancel.)
 //
 // Sums: the product of the first planes, 16 bits, is all but 2^-7 of a weight times its activation.  These products of 32 inputs
 // are summed from zero (one term alone: exactly) and the vector ALU adds them up, rounded to nearest; every other 32 inputs enter
 // negated, as above; in runs and the runs to each other, the slices of K in a tree.  Runs of sqrt(steps / 2) and more
-// make the two chains about equally long.  The other seven products go through the matrix unit from end to end: its rounding
+// make the two chains about equally long.  The other eight products go through the matrix unit from end to end: its rounding
 // is of sums that are 2^-7 of the output's.
 //
 // Infinities and NaN: the planes of an infinity are not one (inf - inf), and a plane can be rounded to one.  A tile of 16 x 16 with
@@ -544,8 +542,8 @@ __global__ __launch_bounds__(64 * NW, NT == 1 ? 3 : 2) void q4_tile_gemm_kernel(
 // Lane (row r = l % 16, kg = l / 16) loads 8 consecutive weights of each 32 inputs (a row's cache line, in two loads), four
 // such pairs ahead, and splits 32 inputs ahead of the products; the activations of 64 inputs pass through LDS,
 // double-buffered; the sums of the runs wait in LDS, which takes up all of it (NT = 8).  What bounds it is the products
-// and what issues beside them, one behind the other: a step of 64 inputs and 112 tokens is 466 instructions per wave, 112 of
-// them products (1792 cycles), 96 the splitting, and two waves per SIMD took some 7000 cycles for it with 126.
+// and what issues beside them, one behind the other: a step of 64 inputs and 112 tokens is 480 instructions per wave, 126 of
+// them products (2016 cycles), 96 the splitting, and two waves per SIMD take some 7000 cycles for it.
 //
 // Against products in v_mfma_f32_32x32x2_f32 (128 rows x 64 columns per block, every weight read for each): one layer of 7B's
 // widths, 33, 64, 100, 200, 512 columns 332 / 347 / 557 / 1021 / 1818 -> 301 / 341 / 496 / 954 / 1652 us; w1|w3 alone at 99 columns
@@ -714,9 +712,9 @@ __device__ __forceinline__ void dense_tile(const Q4Launch &L, const XhList &xl, 
             const int k = g / PAIRS, next = (2 * par + k + 1) & 3; // the half whose weights are split meanwhile
             if (g + 1 < 2 * PAIRS) read_x(g + 1, tile);
             if (g > 0) fold(g - 1);
-            constexpr int pa[7] = {2, 1, 2, 1, 0, 1, 0}, pb[7] = {1, 2, 0, 1, 2, 0, 1};
+            constexpr int pa[8] = {2, 2, 1, 2, 1, 0, 1, 0}, pb[8] = {2, 1, 2, 0, 1, 2, 0, 1};
 #pragma unroll
-            for (int q = 0; q < 8; q++)
+            for (int q = 0; q < 9; q++)
 #pragma unroll
                 for (int u = 0; u < 2; u++) {
                     const int at = (g & 1) * 2 + u, n = g % PAIRS * 2 + u;

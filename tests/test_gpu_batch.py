@@ -181,6 +181,40 @@ def test_dense_batch_few_terms(ops, dim, hidden):
     m.close()
 
 
+# Every product of a weight and an activation is taken, that of their third planes (up to 2^-32 of the whole) included: pairs of terms
+# of which all cancels but the third plane of the weight, up to 2^-17, times the activation.  The matrix unit drops bits of what it
+# adds up, the last of them below 2^-32 of the pair's first plane products, and only downwards: a result above the exact one by more
+# than the rounding of what is left, 2^-17 2^-24, lacks a negative product
+@pytest.mark.parametrize("dim,hidden", [(1024, 2816), (2048, 1344)])
+def test_dense_products_are_exact(ops, dim, hidden):
+    from llama2_rs import _lib
+    import tests.test_oracle_loop as tol
+    dims = ck.Dims(dim=dim, hidden_dim=hidden, n_layers=1, n_heads=dim // 128, n_kv_heads=1, vocab_size=64, seq_len=32, group_size=0)
+    img, rng = ops.synth_image(dims, 4), np.random.default_rng(hidden)
+    at = 1 + 64 * dim + dim + 2 * dim * dim + 2 * 128 * dim + dim  # of w1: in front of it eps, embedding, norm, q, k, v, o, norm
+    w1 = img.view(np.float32)[at:at + hidden * dim].reshape(hidden, dim)
+
+    def nearest(v):  # bf16
+        b = v.view(np.uint32)
+        return ((b + 0x7FFF + (b >> 16 & 1)) & np.uint32(0xFFFF0000)).view(np.float32)
+
+    w = rng.uniform(1, 2, (hidden, dim // 2)).astype(np.float32)
+    w[nearest(w - (w - nearest(w) - nearest(w - nearest(w)))) != nearest(w)] = 1.25  # without the third plane the first is another
+    third = w - nearest(w) - nearest(w - nearest(w))
+    w1[:, 0::2], w1[:, 1::2] = w, third - w
+    m = ops.Model(img, dims)
+    np.testing.assert_array_equal(tol._split_image(img, dims)["w1"][0], w1)
+    for B in (33, 100, 300):
+        x, pair = np.zeros((B, dim), np.float32), rng.integers(0, dim // 2, B)
+        size = 2.0 ** rng.integers(-20, 20, B)
+        of = (size * rng.uniform(1, 2, B) * rng.choice([-1, 1], B)).astype(np.float32)
+        x[np.arange(B), 2 * pair] = x[np.arange(B), 2 * pair + 1] = of
+        want = of[:, None].astype(np.float64) * third[:, pair].T
+        err = (m.qmatvec(0, _lib.W1, x) - want) / size[:, None]
+        assert err.max() <= 2.0 ** -39 and err.min() >= -2.0 ** -29, (B, np.log2(np.abs([err.max(), err.min()])))
+    m.close()
+
+
 # tiles of tokens from one to eight and one more block, rows that do not fill a block; then infinities and NaN, which the
 # planes of a split number do not carry: a batch has them where its columns one by one have them.  Sums of K terms of either
 # association differ by K 2^-24 of the sum of magnitudes at most, which is below sqrt(K) 2 rms for these inputs
