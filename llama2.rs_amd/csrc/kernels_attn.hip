@@ -873,15 +873,15 @@ __device__ __forceinline__ int column_tile(int y, int n, int unit_rows) {
 // tokens 8.6, 7.9.  (v_mfma_f32_16x16x4_f32 at its peak: 63 us for the first of these.)  (A form on 32 columns and tiles of 32 rows,
 // v_mfma_f32_32x32x2_f32 with K and V turned through LDS, had half the blocks and took 16 to 31 us per chunk of a
 // 512-token prompt where this one takes 11 to 19.)
-template <int QG, int NWV, int CS>
-__global__ __launch_bounds__(NWV * 64, NWV == 4 ? 2 : 1)
-void attn_prefill_mfma16_kernel(void *__restrict__ out, const float *__restrict__ q, const float *__restrict__ kc,
-                                const float *__restrict__ vc, const int32_t *__restrict__ pos,
-                                const int32_t *__restrict__ scatter, int n_heads, int n_kv_heads, int B, int max_pos,
-                                int unit_rows) {
-    constexpr int NP = 3, NT = NWV * 64, TK = 16, HS = 128, HALF = 64, NC = 16, QPT = NC / QG;
-    __shared__ __align__(16) float comb[NWV][NC][kCombRow];
-    __shared__ float4 qs[CS > 1 ? CS : 1][CS > 1 ? 8 : 1][64]; // several sets: their B operands
+//
+// `keep`: which of a thread's outputs of each set are stored (comb and qs are LDS, qs of several sets only).
+constexpr int kSetOutputs = 16 * 128 / 256; // of a thread, of a set of 16 columns in a block of 256
+template <int QG, int NWV, int NP, int CS>
+__device__ __forceinline__ void prefill_fp32(void *__restrict__ out, const float *__restrict__ q, const float *__restrict__ kc,
+                                             const float *__restrict__ vc, const int32_t *__restrict__ pos,
+                                             const int32_t *__restrict__ scatter, int n_heads, int n_kv_heads, int B, int max_pos,
+                                             int unit_rows, float (*comb)[16][kCombRow], float4 (*qs)[8][64], const uint32_t (&keep)[CS]) {
+    constexpr int NT = NWV * 64, TK = 16, HS = 128, HALF = 64, NC = 16, QPT = NC / QG;
     const int kvh = blockIdx.x, ct = column_tile(blockIdx.y, gridDim.y, unit_rows) * CS;
     const int dim = n_heads * HS, kv_dim = n_kv_heads * HS;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1066,21 +1066,40 @@ void attn_prefill_mfma16_kernel(void *__restrict__ out, const float *__restrict_
                 nu = fmaf(e, comb[w][j][d], nu);
                 de = fmaf(e, comb[w][j][HS + 1], de);
             }
-            if (qi < B) {
+            if (qi < B && (keep[cs] >> u & 1)) {
                 const int to = dst[u % HEADS];
                 const float v = nu / de;
-                // three bf16 numbers that add up to v exactly
-                uint16_t *o = reinterpret_cast<uint16_t *>(out) + (size_t)qi * NP * dim + b16_slot(to);
-                float left = v;
+                if constexpr (NP == 1) {
+                    reinterpret_cast<_Float16 *>(out)[(size_t)qi * dim + h16_slot(to)] = (_Float16)v;
+                } else { // three bf16 numbers that add up to v exactly
+                    uint16_t *o = reinterpret_cast<uint16_t *>(out) + (size_t)qi * NP * dim + b16_slot(to);
+                    float left = v;
 #pragma unroll
-                for (int p = 0; p < NP; p++) {
-                    const uint32_t bits = __builtin_bit_cast(uint32_t, left) & 0xFFFF0000u;
-                    o[(size_t)p * dim] = (uint16_t)(bits >> 16);
-                    left -= __builtin_bit_cast(float, bits);
+                    for (int p = 0; p < NP; p++) {
+                        const uint32_t bits = __builtin_bit_cast(uint32_t, left) & 0xFFFF0000u;
+                        o[(size_t)p * dim] = (uint16_t)(bits >> 16);
+                        left -= __builtin_bit_cast(float, bits);
+                    }
                 }
             }
         }
     }
+}
+
+template <int QG, int CS>
+__global__ __launch_bounds__(256, 2)
+void attn_prefill_mfma16_kernel(void *__restrict__ out, const float *__restrict__ q, const float *__restrict__ kc,
+                                const float *__restrict__ vc, const int32_t *__restrict__ pos,
+                                const int32_t *__restrict__ scatter, int n_heads, int n_kv_heads, int B, int max_pos,
+                                int unit_rows) {
+    __shared__ __align__(16) float comb[4][16][kCombRow];
+    __shared__ float4 qs[CS > 1 ? CS : 1][CS > 1 ? 8 : 1][64]; // several sets: their B operands
+    constexpr uint32_t all = (1u << kSetOutputs) - 1;
+    uint32_t keep[CS];
+#pragma unroll
+    for (int cs = 0; cs < CS; cs++) keep[cs] = all;
+    prefill_fp32<QG, 4, 3, CS>(out, q, kc, vc, pos, scatter, n_heads, n_kv_heads, B, max_pos, unit_rows, comb,
+                               reinterpret_cast<float4(*)[8][64]>(qs), keep);
 }
 
 typedef __bf16 b8 __attribute__((ext_vector_type(8)));
@@ -1130,6 +1149,7 @@ void attn_prefill_cut_kernel(void *__restrict__ out, const float *__restrict__ q
     __shared__ __align__(16) float comb[NWV][NC][kCombRow];
     __shared__ float2 ml[CS][NWV][NC];
     __shared__ uint4 qs[CS][4][3][64]; // the columns' B operands: [set][32 dimensions][plane][lane]
+    __shared__ int again;
     const int kvh = blockIdx.x, ct = column_tile(blockIdx.y, gridDim.y, unit_rows) * CS;
     const int dim = n_heads * HS, kv_dim = n_kv_heads * HS;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1189,6 +1209,7 @@ void attn_prefill_cut_kernel(void *__restrict__ out, const float *__restrict__ q
 #pragma unroll
         for (int k = 0; k < 3; k++) qs[cs][wave][k][lane] = make_uint4(c[k].u[0], c[k].u[1], c[k].u[2], c[k].u[3]);
     }
+    if (tid == 0) again = 0;
     int t_end = my_pos[0] + 1; // the block's tiles end with the last row any of its columns sees
 #pragma unroll
     for (int cs = 1; cs < CS; cs++) t_end = max(t_end, my_pos[cs] + 1);
@@ -1328,6 +1349,8 @@ void attn_prefill_cut_kernel(void *__restrict__ out, const float *__restrict__ q
     if (tile < n_tiles) step(tile, std::true_type());
 
     // The waves agree on each column's maximum and sum, each scales its O by its share, and these add up in LDS.
+    static_assert(NC * HS / (NWV * 64) == kSetOutputs && sizeof(qs) >= CS * 8 * 64 * sizeof(float4), "what prefill_fp32 takes over");
+    uint32_t redo[CS] = {}; // this thread's outputs that are not finite
 #pragma unroll
     for (int cs = 0; cs < CS; cs++) {
         const float l = lanes::rows_sum(run_l[cs]);
@@ -1356,9 +1379,19 @@ void attn_prefill_cut_kernel(void *__restrict__ out, const float *__restrict__ q
         for (int u = 0; u < NC * HS / (NWV * 64); u++) {
             const int j = tid / HS + u * PER, d = tid % HS, qi = (ct + cs) * QPT + j / QG;
             const float v = (comb[0][j][d] + comb[1][j][d]) + (comb[2][j][d] + comb[3][j][d]);
-            if (qi < B) reinterpret_cast<_Float16 *>(out)[(size_t)qi * dim + h16_slot(dst[u % HEADS])] = (_Float16)v;
+            if (qi < B) {
+                reinterpret_cast<_Float16 *>(out)[(size_t)qi * dim + h16_slot(dst[u % HEADS])] = (_Float16)v;
+                if (!__builtin_isfinite(v)) redo[cs] |= 1u << u;
+            }
         }
+        if (redo[cs]) again = 1;
     }
+    // The planes of an infinity are not one (inf - inf), and one infinite term hides what the others add up to: outputs that are not
+    // finite are taken from the fp32 form.
+    __syncthreads();
+    if (again)
+        prefill_fp32<QG, NWV, 1, CS>(out, q, kc, vc, pos, scatter, n_heads, n_kv_heads, B, max_pos, unit_rows, comb,
+                                     reinterpret_cast<float4(*)[8][64]>(qs), redo);
 }
 
 // Merge the splits of one q head: out = sum_s 2^(m_s - M) o_s / sum_s 2^(m_s - M) l_s.
@@ -1494,8 +1527,8 @@ static int prefill_qg(void *out, int planes, const float *q, const float *kc, co
             else L2_PREFILL_ATTN(attn_prefill_cut_kernel<QG, 1>);
             break;
         case 3:
-            if (two) L2_PREFILL_ATTN(attn_prefill_mfma16_kernel<QG, 4, 2>);
-            else L2_PREFILL_ATTN(attn_prefill_mfma16_kernel<QG, 4, 1>);
+            if (two) L2_PREFILL_ATTN(attn_prefill_mfma16_kernel<QG, 2>);
+            else L2_PREFILL_ATTN(attn_prefill_mfma16_kernel<QG, 1>);
             break;
         default: return l2_fail(L2_ERR_ARG, "attention: %d planes", planes);
     }

@@ -540,6 +540,35 @@ def test_fp16_prompt_attention(ops, n_heads, n_kv, at, n):
     m.close()
 
 
+# ... and what its planes do not hold: an infinity among the keys, which takes a row's weight to zero or makes the output a NaN, as the
+# query's sign has it, and a value near the largest number on the row without weight.  One set of columns and two, both in the
+# same places as in the fp32 mode, the other outputs as above
+@pytest.mark.parametrize("n_heads,n_kv,at,n", [(4, 4, 40, 40), (8, 4, 5, 100), (32, 32, 61, 300)])
+def test_fp16_prompt_attention_not_finite(ops, n_heads, n_kv, at, n):
+    from llama2_rs import _lib
+    dims = ck.Dims(dim=128 * n_heads, hidden_dim=256, n_layers=2, n_heads=n_heads, n_kv_heads=n_kv, vocab_size=64,
+                   seq_len=400, group_size=64)
+    m = ops.Model(ck.synth_weights_image(dims, seed=9), dims)
+    toks = np.random.default_rng(n).integers(0, 64, size=at + n).astype(np.int32)
+    rows = []
+    for mode in (_lib.PREFILL_MFMA, _lib.PREFILL_FP32):
+        m.reset()
+        m.set_prefill_mode(mode)
+        m.prefill_chunks(toks[:at], 0, at)
+        k, v = m.read_kv(0, 0, at)
+        k[3, 0, 70], v[3, 0] = -np.inf, 3.4e38
+        m.write_kv(0, 0, k, v)
+        m.prefill_chunks(toks[at:], at, n)
+        rows.append(m.read_kv(1, at, n))
+    for got, want in zip(*rows):
+        fine = np.isfinite(want).all(axis=(1, 2))
+        np.testing.assert_array_equal(np.isfinite(got).all(axis=(1, 2)), fine)
+        assert n / 8 < fine.sum() < n
+        e = np.sqrt(np.mean((got - want)[fine].astype(np.float64) ** 2, axis=(1, 2)) / np.mean(want[fine].astype(np.float64) ** 2, axis=(1, 2)))
+        assert e.max() < 6.4e-4
+    m.close()
+
+
 # the kernels between the products of a chunk: rows of one, two and four trips of the block (and a consumer's order per
 # LDS row, or in turns), few K slices and many, in each kind of plane, against single tokens.  fp16 inputs carry 2^-11 each:
 # through the five products in front of the second layer's cache rows some 1e-3, and 4.5 times that at the furthest of
