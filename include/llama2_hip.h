@@ -47,7 +47,9 @@ enum {
                           * from B=1 by the rounding of the additions only (1e-6).  Exact means: operands
                           * enter as three bf16 numbers, which hold all 24 bits of a value from 2^-109 on
                           * and smaller ones to 2^-133                                               */
-    L2_PREFILL_MFMA = 1, /* dequant -> fp16 tiles -> MFMA, fp32 accumulate (tolerance 2e-3)    */
+    L2_PREFILL_MFMA = 1, /* projections: dequant -> fp16 tiles -> MFMA, fp32 accumulate (tolerance 2e-3).
+                          * Attention: its fp32 operands as three bf16 numbers, products to within
+                          * 2^-24, fp32 accumulate                                                */
     L2_PREFILL_COLUMNS = 2 /* fp32 throughout, and every column of a projection is the bits of B=1
                             * whatever the batch, as L2_PREFILL_FP32 has for a few columns: the
                             * weights are read once per column                                  */

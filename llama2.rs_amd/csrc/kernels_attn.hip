@@ -1104,15 +1104,16 @@ void attn_prefill_mfma16_kernel(void *__restrict__ out, const float *__restrict_
 
 typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+typedef float v2f __attribute__((ext_vector_type(2)));
 
-// Two fp32 numbers as three pairs of bf16 numbers each, cut after the first, second and third byte of the significand: exact.
-// What a cut leaves is one v_dot2_f32_bf16 of the pair that was cut off with (-1, 0) or (0, -1).
+// Two fp32 numbers as three pairs of bf16 numbers each, whose sum they are: each rounded to nearest (one instruction for the pair),
+// so that what it leaves has either sign.  What is left is one v_dot2_f32_bf16 of the pair with (-1, 0) or (0, -1).
 struct Cut {
     uint32_t p[3];
     __device__ __forceinline__ Cut(float x, float y, uint32_t minus_lo, uint32_t minus_hi) {
 #pragma unroll
         for (int k = 0; k < 3; k++) {
-            p[k] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, y), __builtin_bit_cast(uint32_t, x), 0x07060302u);
+            p[k] = __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{x, y}, b2));
             if (k == 2) break;
             x = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(b2, p[k]), __builtin_bit_cast(b2, minus_lo), x, false);
             y = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(b2, p[k]), __builtin_bit_cast(b2, minus_hi), y, false);
@@ -1124,17 +1125,20 @@ struct Plane {
     __device__ __forceinline__ b8 b() const { return __builtin_bit_cast(b8, *this); }
 };
 
-// The same for the fp16 mode (L2_PREFILL_MFMA), on v_mfma_f32_16x16x32_bf16 with every fp32 number cut into three bf16 numbers
-// (sixteen times the rate of v_mfma_f32_16x16x4_f32): six products, down to 2^-16 of the first; the three left out are below an
-// fp32 rounding.  Relative rms error against fp64, 33 to 777 queries over up to 2040 rows, of that of the fp32 form: normal inputs
-// 0.49 to 0.77, sharper scores on values of one sign 0.63 to 1.04 (32 rows).  Blocks, columns and tiles are the fp32 form's, and a column's
+// The same for the fp16 mode (L2_PREFILL_MFMA), on v_mfma_f32_16x16x32_bf16 with every fp32 number as three bf16 numbers
+// (sixteen times the rate of v_mfma_f32_16x16x4_f32): six products, down to the first by the third.  The second number is 2^-8 of
+// the first at most and the third 2^-17, so the three products left out are 2^-24 of the whole at most, as an fp32 rounding is; of either
+// sign, 2^-27.5 rms (2^-25.2).  (Cut off instead of rounded they are 2^-21.2 and all of one sign, 2^-24.7 on average.)  Relative rms
+// error against fp64, 33 to 777 queries over 33 to 2040 rows, of that of the fp32 form: normal inputs 0.46 to 0.68, values of one sign
+// 0.44 to 0.84, scores four times as sharp 0.52 to 0.70, nearly equal weights 0.35 to 0.93.  A number below 2^-102
+// is held to 2^-126 at worst.  Blocks, columns and tiles are the fp32 form's, and a column's
 // result depends on neither the other columns nor the number of sets: a pass gives the bits of the same tokens in several.
 //   - Scores contract over 32 dimensions: a lane holds 16 m + 4 kb .. + 3 of two m, of K as of Q.
 //   - The sums contract over the 16 rows of a tile, so one instruction takes two products: half its contraction is one plane of
 //     V times one of the weights, half another.
-//   - K, V and the weights are cut by the wave that uses them, 7 vector instructions a pair of numbers (4 of them the dot
+//   - K, V and the weights are split by the wave that uses them, 7 vector instructions a pair of numbers (4 of them the dot
 //     products of Cut; with masks and subtractions 11), Q once per block.
-// What bounds it is the issue of vector instructions, most of them the cutting (half of a SIMD's cycles; the matrix unit's 28 %).
+// What bounds it is the issue of vector instructions, most of them the splitting (half of a SIMD's cycles; the matrix unit's 28 %).
 // Against the fp32 form, per launch: 32 heads, 16, 64, 128, 299, 511 tokens 5.5, 6.2, 8.0, 19.3, 29.6 -> 4.7, 5.2, 6.8, 15.6, 24.2 us;
 // 128 tokens behind 384 17.2 -> 15.0, 64 behind 1500 36.3 -> 33.8; 64 heads on 8 kv heads, 128, 777 tokens 10.7, 105.5 -> 9.4, 79.8.
 // Tiles of 32 rows, a product per instruction: 16, 128 and 777 of these tokens 6.0, 7.5 and 86.0; rescaling whenever a maximum

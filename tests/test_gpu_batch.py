@@ -540,6 +540,115 @@ def test_fp16_prompt_attention(ops, n_heads, n_kv, at, n):
     m.close()
 
 
+def _planes(v):
+    """Three bf16 numbers for each fp32 one, rounded to nearest, in fp64."""
+    v, out = v.astype(np.float32), []
+    for _ in range(3):
+        b = v.view(np.uint32)
+        out.append(((b + 0x7FFF + (b >> 16 & 1)) & np.uint32(0xFFFF0000)).view(np.float32))
+        v = v - out[-1]
+    return [p.astype(np.float64) for p in out]
+
+
+def _see_through_image(d, rng, qk):
+    """Two layers that show attention of the first one in the values of the second: wk is wq (so that a key row is the query), wo and the
+    second layer's wv are one, w2 is zero."""
+    parts = []
+
+    def put(a, dtype=np.float32):
+        parts.append(np.ascontiguousarray(a, dtype).view(np.uint8).reshape(-1))
+
+    def linear(n, scale):  # n: whole numbers -8..7 [out][in]
+        g = n.shape[1] // d.group_size
+        put(ck.pack_nibbles(n + 8, axis=1), np.int32), put(ck.pack_nibbles(np.full((n.shape[0], g), 7), axis=0), np.int32)
+        put(np.full((n.shape[0], g), scale)), put(np.arange(n.shape[1]), np.int32)
+
+    q, one, none = rng.integers(-8, 8, (d.dim, d.dim)), np.eye(d.dim, dtype=np.int64), np.zeros((d.dim, d.dim), np.int64)
+    emb = rng.normal(0, 0.02, (d.vocab_size, d.dim)).astype(np.float32)
+    put([1e-5]), put(emb), put(np.ones((2, d.dim)))
+    for n in (q, q, q, q, none, one, one, none):  # wq, wk, wv and wo of both layers
+        linear(n, qk if n is q else 1)
+    put(np.ones((2, d.dim)))
+    for n_out, n_in in ((d.hidden_dim, d.dim), (d.dim, d.hidden_dim), (d.hidden_dim, d.dim)):
+        for _ in range(2):
+            linear(np.zeros((n_out, n_in), np.int64), 1)
+    put(np.ones(d.dim)), put(np.zeros((2, d.seq_len, 64))), put(emb)
+    img = np.concatenate(parts)
+    assert img.nbytes == ck.weights_bytes(d)
+    return img, emb
+
+
+# ... and its precision, where it shows behind outputs rounded to fp16: one query, its keys and values made so that much cancels.
+#   scores: products of 2e4 rms that add up to what the query has with itself and two more or less.  A partial sum of 2e4 sqrt(128) /
+#     sqrt(128) log2(e) = 2.9e4 is rounded to 2^-10, some ten of them: ln 2 sqrt(10) 2^-10 = 2e-3 of a weight; twice that
+#   sums: values of 2.4e4 sqrt(100) that add up to one: weights are right to some 2^-23, so 24000 2^-22.5 = 4e-3; five times that
+#   bias: scores of 2^18 of products of one sign, keys with all bits of the low planes set in turns with keys without them, whose
+#     values are 1 and -1.  A product that lacks 2^-24 of itself on one side takes ln 2 2^-7 = 5e-3 of the weight; the mean of 512 outputs
+#     errs by less than 1e-3 if it does not (numbers that were cut instead of rounded: 3e-3 to 9e-3)
+# Without any one of the six products an output would be off by more than twice the bound.
+@pytest.mark.parametrize("kind,seed", [("scores", 0), ("scores", 1), ("sums", 0), ("sums", 1), ("bias", 0), ("bias", 1), ("bias", 2)])
+def test_fp16_prompt_attention_precision(ops, kind, seed):
+    from llama2_rs import _lib
+    H, at, n, unit, rng = 4, 100, 16, np.log2(np.e) / np.sqrt(128), np.random.default_rng(seed)
+    q_rms, bound = {"scores": (8, 4e-3), "sums": (0.1, 2e-2), "bias": (8, 1e-3)}[kind]
+    d = ck.Dims(dim=128 * H, hidden_dim=256, n_layers=2, n_heads=H, n_kv_heads=H, vocab_size=64, seq_len=128, group_size=64)
+    img, emb = _see_through_image(d, rng, q_rms / (4.6 * np.sqrt(d.dim)))
+    m = ops.Model(img, d)
+    m.set_prefill_mode(_lib.PREFILL_MFMA)
+    toks = rng.integers(0, 64, n).astype(np.int32)
+    m.prefill_chunks(toks, at, n)
+    k_own, v_own = (a[0] for a in m.read_kv(0, at, 1))
+    q = k_own.astype(np.float64)
+    own = (q * q).sum(-1) * unit
+    score = (2.0 ** 18 if kind == "bias" else own) + rng.uniform(-2, 2, (at, H))
+    k = rng.standard_normal((at, H, 128)) * (20000 / q_rms if kind == "scores" else 1)
+    if kind == "bias":
+        bits = (np.sign(q) * 16000 / np.abs(q) * rng.uniform(0.5, 2, k.shape)).astype(np.float32).view(np.uint32)
+        bits[0::2] |= 0x7FFF
+        bits[1::2] &= 0xFFFF0000
+        k = bits.view(np.float32).astype(np.float64)
+        least = np.argmin(np.abs(q), axis=-1)  # takes what is missing from the score
+        k[:, np.arange(H), least] += (score / unit - (k * q).sum(-1)) / q[np.arange(H), least]
+    else:
+        k += q * ((score / unit - (k * q).sum(-1)) / (q * q).sum(-1))[..., None]
+    k = k.astype(np.float32)
+    s = np.concatenate([(k.astype(np.float64) * q).sum(-1) * unit, own[None]])
+    p = np.exp2(s - s.max(0))
+    w = p / p.sum(0)
+    v = rng.standard_normal((at, H, 128))
+    if kind == "sums":
+        v *= 24000 * np.sqrt(at)
+        for h, j in enumerate(np.argmax(w[:at], axis=0)):
+            v[j, h] -= (w[:at, h] @ v[:, h] - rng.standard_normal(128)) / w[j, h]
+    if kind == "bias":
+        v = np.where(np.arange(at) % 2, -1, 1)[:, None, None] + 0.02 * v
+    v = v.astype(np.float32)
+
+    def output(w):
+        return np.sum(w[:at, :, None] * v.astype(np.float64), axis=0) + w[at][:, None] * v_own
+
+    out = output(w)
+    if kind == "scores":  # without one product of planes
+        kp, qp = _planes(k), _planes(k_own)
+        for i, j in ((0, 0), (0, 1), (1, 0), (1, 1), (0, 2), (2, 0)):
+            less = s.copy()
+            less[:at] -= (kp[i] * qp[j]).sum(-1) * unit
+            less = np.exp2(less - less.max(0))
+            assert np.linalg.norm(output(less / less.sum(0)) - out) > 2 * bound * np.linalg.norm(out), (i, j)
+    if kind == "sums":
+        vp, pp = _planes(v), _planes(p[:at].astype(np.float32))
+        for i, j in ((0, 0), (0, 1), (1, 0), (1, 1), (0, 2), (2, 0)):
+            assert np.linalg.norm(np.sum(pp[j][..., None] * vp[i], axis=0) / p.sum(0)[:, None]) > 2 * bound * np.linalg.norm(out), (i, j)
+    m.write_kv(0, 0, k, v)
+    m.prefill_chunks(toks, at, n)
+    np.testing.assert_array_equal(m.read_kv(0, at, 1)[0][0], k_own)
+    x = emb[toks[0]].astype(np.float64) + out.reshape(-1)
+    rms = np.sqrt(np.mean(x * x) + 1e-5)
+    err = m.read_kv(1, at, 1)[1].reshape(-1) * rms - x
+    m.close()
+    assert (abs(err.mean()) if kind == "bias" else np.linalg.norm(err) / np.linalg.norm(x)) < bound
+
+
 # ... and what its planes do not hold: an infinity among the keys, which takes a row's weight to zero or makes the output a NaN, as the
 # query's sign has it, and a value near the largest number on the row without weight.  One set of columns and two, both in the
 # same places as in the fp32 mode, the other outputs as above
