@@ -29,6 +29,8 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <type_traits>
+
 #include "q4_common.h"
 
 namespace {
@@ -254,6 +256,22 @@ struct RowData {
 __device__ __forceinline__ float chunk_sum(const float (&s4)[8]) {
     return ((s4[0] + s4[1]) + (s4[2] + s4[3])) + ((s4[7] + s4[6]) + (s4[5] + s4[4]));
 }
+
+// A lane's share of a row's dot product: scale times sum.  What a row's first addition across lanes rounds is written out here, since
+// it is the row's last bit and every form of a launch must give the same: a row of the loop rounds the product, then the sum;
+// one of those that stand behind the loop, the remainder of a block's rows, rounds once.
+struct Share {
+    float scale, sum;
+    __device__ __forceinline__ float product() const {
+#pragma clang fp contract(off)
+        return scale * sum;
+    }
+    __device__ __forceinline__ float two_lanes(bool behind) const {
+#pragma clang fp contract(off)
+        const float other = dpp_xchg<0xB1>(scale * sum);
+        return behind ? fmaf(scale, sum, other) : scale * sum + other;
+    }
+};
 
 // The leading arguments are what the loads of x need: x of the launch's matrices (blocks0 and blocks1 of the grid belong to the
 // first and second), the norm weights of the first, those of the others behind it, or null, and the inverse of g_index of the
@@ -582,6 +600,7 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const float *x0,
     const int row_half = row0 + rows_per_block / 2;
     auto behind = [](int rows) { return (rows + S / 2 - 1) / (P * S / 2) * (P * S / 2); };
     const int behind0 = TWO ? behind(min(rows_per_block / 2, n_rows)) : 0, behind1 = TWO ? behind(max(row1 - row_half, 0)) : 0;
+    auto is_behind = [&](int o) { return o >= row_half ? o - row_half >= behind1 : o - row0 >= behind0; };
     // The second half of the rows, and a wait for the first, which arrived while x was staged.  The compiler's wait
     // counts inside the loop are then those of the steady state alone: vmcnt leaves the P - 1 younger rows in
     // flight.  Otherwise the issue order of the prologue leaks into the loop's waits.
@@ -595,34 +614,23 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const float *x0,
     epi_fetch();
     float *__restrict__ const yout = mat[0].y;
 
-    // one row (row pair) of this stream: dequantised dot product of the lane's chunk -> pr
-    auto row_dot = [&](int o, const RowData(&d)[NM], float(&pr)[NM]) __attribute__((always_inline)) {
+    // one row (row pair) of this stream: the lane's share of its dot product, a scale times the sum of the chunk
+    auto row_dot = [&](int o, const RowData(&d)[NM], Share(&p)[NM]) __attribute__((always_inline)) {
 #pragma unroll
         for (int q = 0; q < NM; q++) {
             const int zn = (int)(((uint32_t)d[q].z >> (4 * (o & 7))) & 15u);
-            if constexpr (IDOT) {
-                const float f = chunk_idot(d[q].w, xp[q]);
-                pr[q] = (d[q].s * xdelta[q]) * fmaf(-(float)(zn - 7), sx[q], f);
-            } else {
-                const float p = chunk_dot(d[q].w, x[q]);
-                // -(zn + 1) sx as one FMA on the converted nibble (the same real number, rounded once either way)
-                const float f = fmaf(p, 512.0f, fmaf((float)zn, nsx[q], nsx[q]));
-                pr[q] = d[q].s * f;
-                if constexpr (TWO) { // with the first addition across lanes, rounded as in a block of half the rows
-                    asm volatile("" : "+v"(pr[q]));
-                    const float other = dpp_xchg<0xB1>(pr[q]);
-                    const int half = o >= row_half ? o - row_half : o - row0;
-                    pr[q] = half >= (o >= row_half ? behind1 : behind0) ? fmaf(d[q].s, f, other) : pr[q] + other;
-                }
-            }
+            if constexpr (IDOT)
+                p[q] = {d[q].s * xdelta[q], fmaf(-(float)(zn - 7), sx[q], chunk_idot(d[q].w, xp[q]))};
+            else // -(zn + 1) sx as one FMA on the converted nibble (the same real number, rounded once either way)
+                p[q] = {d[q].s, fmaf(chunk_dot(d[q].w, x[q]), 512.0f, fmaf((float)zn, nsx[q], nsx[q]))};
         }
     };
-    // 64 partials -> 4 (one per 16-lane row) -> the tile's slot for this row
-    auto row_fold = [&](int u, const float(&pr)[NM]) __attribute__((always_inline)) {
+    // 64 partials -> 4 (one per 16-lane row) -> the tile's slot for this row; two_lanes: the first addition has been done
+    auto row_fold = [&](int u, const float(&pr)[NM], auto two_lanes) __attribute__((always_inline)) {
 #pragma unroll
         for (int q = 0; q < NM; q++) {
             float v = pr[q];
-            if constexpr (!TWO) v += dpp_xchg<0xB1>(v);
+            if (!two_lanes) v += dpp_xchg<0xB1>(v);
             v += dpp_xchg<0x4E>(v);
             v += dpp_xchg<0x141>(v);
             v += dpp_xchg<0x140>(v);
@@ -657,9 +665,12 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const float *x0,
     for (int tile = 0; tile < n_full; tile++) {
 #pragma unroll
         for (int u = 0; u < P; u++) {
-            const int i = tile * P + u;
+            const int i = tile * P + u, o = row0 + stream + i * S;
+            Share p[NM];
+            row_dot(o, pipe[u], p);
             float pr[NM];
-            row_dot(row0 + stream + i * S, pipe[u], pr);
+#pragma unroll
+            for (int q = 0; q < NM; q++) pr[q] = TWO ? p[q].two_lanes(is_behind(o)) : p[q].product();
             // Refill this slot with row i + P, after its last use and not before:
             // a load hoisted above the row's arithmetic makes the compiler copy
             // live registers of the other slots, and each copy waits on its load.
@@ -670,7 +681,7 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const float *x0,
             __builtin_amdgcn_sched_barrier(0);
             fetch(i + P, pipe[u]);
             __builtin_amdgcn_sched_barrier(0);
-            row_fold(u, pr);
+            row_fold(u, pr, std::bool_constant<TWO>());
         }
         __syncthreads();
         if ((unsigned)r < (unsigned)TR && eo < row1) tile_finish(r);
@@ -686,11 +697,13 @@ __global__ __launch_bounds__(NWK *S * 64) void q4_stream_kernel(const float *x0,
 #pragma unroll
         for (int u = 0; u < P - 1; u++) {
             if (u < n_rem) {
+                const int o = row0 + stream + (n_full * P + u) * S;
+                Share p[NM];
+                row_dot(o, pipe[u], p);
                 float pr[NM];
-                row_dot(row0 + stream + (n_full * P + u) * S, pipe[u], pr);
-                // no pin: here the scale's multiplication joins the fold's first addition, so a row's last bit depends on whether it
-                // stands behind the loop, that is on the shape and on the rows of the block
-                row_fold(u, pr);
+#pragma unroll
+                for (int q = 0; q < NM; q++) pr[q] = p[q].two_lanes(!TWO || is_behind(o));
+                row_fold(u, pr, std::true_type());
             }
         }
         __syncthreads();
