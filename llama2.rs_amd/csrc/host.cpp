@@ -1419,20 +1419,25 @@ extern "C" int l2_model_classifier(l2_model *m, const float *x_host, float *y_ho
 
 // How the timesteps of a decode step are cut across blocks: not at all in a short context, where each query head's dimensions
 // are spread over blocks instead, which every one scans all keys for; splits cost their merge, a launch of their own.  Whole
-// against in splits, us per layer:
-//   a query head per kv head, few of them: up to 640.  1, 4, 8, 16 heads at 510 20.2 / 22.2 / 21.9 / 23.3 and 22.9 / 21.9 / 23.3 / 24.2,
-//   at 800 23.7 / 23.8 / 23.4 / 24.9 and 22.8 / 21.7 / 23.3 / 24.5
-//   several to a kv head, whose blocks share its rows in an L2, and whose splits take longer (the matrix cores, or two chains): up
-//   to 896, 1024 from 32 query heads on.  8 heads of 2 kv heads at 800, 1000 22.8 / 23.6 and 23.6 / 23.4, of 1 23.1 / 23.7 and
-//   23.9 / 24.7; 32 of 4 29.9 / 30.4 and 31.9 / 31.8, of 16 30.5 / 31.2 and 31.5 / 32.2; 64 of 8 38.7 / 39.6 and 40.4 / 40.3
-//   32 heads of 32: 1024, while the rows that an XCD's blocks read fit its L2 (32 KB a timestep: at 800, 1000, 1250 31.8 / 33.7 / 37.8
-//   and 34.8 / 35.5 / 37.1); above 32 kv heads 768 (40 at 640, 800, 1000 36.6 / 39.6 / 44.4 and 38.6 / 39.7 / 41.3)
+// against in splits, us per layer, the median of three processes (whose launches differ by a us, and with them the splits' cost),
+// models of 32 layers (64 heads: 12, 64 of 8: 24) and the presets, so that a layer's rows come from memory as a user's do:
+//   one or two query heads per kv head: up to 640.  7B at 500, 620, 800, 1010 40.8 / 41.9 / 43.9 / 45.9 and 41.1 / 41.8 / 42.3 / 42.7; 24
+//   heads 33.5 / 35.0 / 37.4 / 39.4 and 34.9 / 35.2 / 36.4 / 36.5, 16 26.0 / 28.2 / 30.8 / 32.5 and 29.4 / 29.9 / 30.6 / 31.0, 8 21.0 /
+//   21.9 / 22.9 / 26.2 and 21.8 / 22.8 / 20.6 / 21.7, 4 21.5 / 22.2 / 23.5 / 24.4 and 22.4 / 23.5 / 23.1 / 23.1; 32 of 16 37.5 / 39.2 / 41.7 /
+//   43.2 and 39.3 / 39.9 / 40.6 / 40.4, 16 of 8 24.0 / 24.6 / 26.4 / 29.0 and 24.9 / 24.5 / 24.8 / 25.5
+//   above 32 kv heads, whose heads are four slices each: 512.  13B at 440, 500, 620, 800 57.0 / 57.4 / 58.7 / 61.7 and 57.0 / 56.9 / 57.0 /
+//   58.3; 64 heads 100.0 / 101.2 / 102.8 / 105.6 and 101.3 / 102.8 / 104.0 / 104.7
+//   four or eight, whose splits take longer (the matrix cores): 768 from 32 heads on.  70B at 620, 740, 800, 1010 98.7 / 98.4 / 99.5 / 100.4
+//   and 99.3 / 99.3 / 99.1 / 99.3; 32 of 8 39.9 / 40.8 / 41.6 / 44.6 and 41.8 / 42.2 / 42.2 / 42.4; 1024 where these have at most 4 kv heads,
+//   32 of 4 35.4 / 36.1 / 36.6 / 37.5 and 38.5 / 38.7 / 38.8 / 39.0.  Fewer heads: 896.  8 of 2 at 740, 860, 1010 22.0 / 22.8 / 23.4 and
+//   22.5 / 22.5 / 22.6, in 3 layers, as long as their launches, 25.5 / 26.8 / 26.8 and 26.4 / 27.2 / 27.0; 8 of 1 22.4 / 23.1 / 23.7 and 22.7 /
+//   22.7 / 23.0, 16 of 4 25.3 / 26.0 / 26.5 and 25.9 / 25.8 / 25.9
 // Beyond that one block per CU where
 // the context allows it, at least 64 timesteps each.  (Two per CU, the earlier rule, left some CUs with two blocks
 // and the launch as long as those: 70B behind 4096 positions 18.6 -> 16.5 us per layer, 13B behind 1000 positions
 // 16.7 -> 15.3, 7B unchanged; half a block per CU is slower everywhere.)
 static void attn_split_policy(int n_t, int n_heads, int n_kv_heads, int *ts_out, int *n_splits_out) {
-    int whole = n_kv_heads > 32 ? 768 : n_heads >= 32 ? 1024 : n_heads > n_kv_heads ? 896 : 640;
+    int whole = n_heads <= 2 * n_kv_heads ? (n_kv_heads > 32 ? 512 : 640) : n_heads < 32 ? 896 : n_kv_heads <= 4 ? 1024 : 768;
     if (n_heads == 8 * n_kv_heads && n_t <= kFewTimesteps) whole = kFewTimesteps;
     if (n_t <= whole) {
         *ts_out = whole;

@@ -333,7 +333,9 @@ def test_decode_attention_whole_or_split(ops, oracle, n_heads, n_kv):
 
 
 # A block per query head: several to a kv head, slices of 16 dimensions and of 32 (64 heads), both sides of where the context is cut
-@pytest.mark.parametrize("n_heads,n_kv,whole", [(2, 2, 640), (2, 1, 896), (8, 2, 896), (8, 1, 896), (32, 16, 1024), (64, 8, 1024), (33, 33, 768)])
+# (among them), and around other lengths
+@pytest.mark.parametrize("n_heads,n_kv,whole", [(2, 2, 640), (2, 1, 896), (8, 2, 896), (8, 1, 896), (32, 16, 1024), (64, 8, 1024), (33, 33, 768),
+                                                (2, 1, 640), (32, 16, 640), (64, 8, 768), (33, 33, 512), (32, 4, 1024)])
 def test_decode_attention_block_per_head(ops, oracle, n_heads, n_kv, whole):
     dims = ck.Dims(dim=128 * n_heads, hidden_dim=512, n_layers=1, n_heads=n_heads, n_kv_heads=n_kv,
                    vocab_size=300, seq_len=1100, group_size=128)
