@@ -84,6 +84,13 @@ int l2_q4_plan(int in, const int32_t *out, int n_mats, int group_size, int pair,
  * refused), 0 with x permuted in front. */
 int l2_qlinear_plan(int in, int out, int group_size, int batch, int natural, char *kernel, size_t cap, int32_t *geometry);
 
+/* The tiles that a batch's GEMM takes, for n_mats (1..3) matrices of `in` inputs and out[i] outputs and `batch` columns in one
+ * pass, without a device and without launching: mode L2_PREFILL_FP32 or L2_PREFILL_MFMA.  plan[8] receives {rows of a block,
+ * columns of its tile, slices of the inputs, blocks, how many of them take whole tiles, the width of the tiles of what whole
+ * rounds of blocks leave over, the last columns where they have a narrower tile of their own (MFMA; else 0), whether a
+ * row block has tiles of both kinds}. */
+int l2_gemm_plan(int in, const int32_t *out, int n_mats, int group_size, int batch, int mode, int32_t *plan);
+
 /* Plain device-to-device copy of nbytes, iters times: the box's achievable
  * copy bandwidth (bytes moved = 2*nbytes per iteration). */
 int l2_copy_bench(size_t nbytes, int iters, float *ms_total);

@@ -821,6 +821,10 @@ extern "C" int l2_model_set_step_graph(l2_model *m, int on) {
     return L2_OK;
 }
 
+static bool q4_gemm_supports(int in, int out, int g) {
+    return in % 128 == 0 && out % 32 == 0 && in % g == 0 && (g < 64 || (in / g) % 2 == 0);
+}
+
 extern "C" int l2_model_set_prefill_mode(l2_model *m, int mode) {
     if (!m) return l2_fail(L2_ERR_ARG, "null model");
     if (mode != L2_PREFILL_FP32 && mode != L2_PREFILL_MFMA && mode != L2_PREFILL_COLUMNS) return l2_fail(L2_ERR_ARG, "prefill mode %d", mode);
@@ -829,9 +833,6 @@ extern "C" int l2_model_set_prefill_mode(l2_model *m, int mode) {
     const int G = m->d.group_size;
     if (mode == L2_PREFILL_MFMA && m->head_size != 128)
         return l2_fail(L2_ERR_ARG, "the MFMA prefill path is built for heads of 128 (this model: %d)", m->head_size);
-    auto q4_gemm_supports = [](int in, int out, int g) {
-        return in % 128 == 0 && out % 32 == 0 && in % g == 0 && (g < 64 || (in / g) % 2 == 0);
-    };
     if (mode == L2_PREFILL_MFMA && !(q4_gemm_supports(m->d.dim, m->d.dim, G) && q4_gemm_supports(m->d.hidden_dim, m->kv_dim, G) &&
                                      q4_gemm_supports(m->d.dim, m->d.hidden_dim, G)))
         return l2_fail(L2_ERR_ARG, "the MFMA prefill path needs dim and hidden_dim to be multiples of 128 (of 2 groups for "
@@ -2429,6 +2430,25 @@ extern "C" int l2_qlinear_plan(int in, int out, int group_size, int batch, int n
     if (natural && !q4_gathers_in_kernel(L)) return l2_fail(L2_ERR_ARG, "in=%d: x is gathered in front", in);
     L.m[0].gidx = natural ? order : nullptr;
     return plan_of(L, kernel, cap, geometry);
+}
+
+extern "C" int l2_gemm_plan(int in, const int32_t *out, int n_mats, int group_size, int batch, int mode, int32_t *plan) {
+    if (!out || !plan || n_mats < 1 || n_mats > 3 || batch < 1) return l2_fail(L2_ERR_ARG, "bad argument");
+    if (mode != L2_PREFILL_FP32 && mode != L2_PREFILL_MFMA) return l2_fail(L2_ERR_ARG, "mode %d", mode);
+    Q4Launch L{};
+    L.n_mats = n_mats, L.in = in, L.batch = batch, L.group_size = group_size;
+    if (group_size) L2_TRY(check_qlinear_shape(in, 8, group_size));
+    else if (in < 32 || in % 32) return l2_fail(L2_ERR_ARG, "in=%d", in);
+    L.groups = group_size ? in / group_size : 0;
+    for (int i = 0; i < n_mats; i++) {
+        if (out[i] <= 0 || out[i] % 8) return l2_fail(L2_ERR_ARG, "out[%d]=%d", i, out[i]);
+        L.m[i].out = out[i];
+    }
+    if (mode == L2_PREFILL_MFMA && (!group_size || !q4_gemm_supports(in, 32, group_size))) return l2_fail(L2_ERR_ARG, "in=%d, groups of %d: not in fp16", in, group_size);
+    const GemmTiles t = gemm_tiles(L, batch, mode == L2_PREFILL_MFMA ? 1 : 3, false);
+    const int32_t all[8] = {t.rows, t.tokens, t.slices, t.blocks, t.whole, t.width, t.last, t.both};
+    memcpy(plan, all, sizeof all);
+    return L2_OK;
 }
 
 extern "C" int l2_kernel_class_count(void) { return K_NCLASS; }

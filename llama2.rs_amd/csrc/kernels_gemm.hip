@@ -1074,7 +1074,7 @@ int ready_tile(size_t *lds) {
 
 // How the blocks of a launch are dealt out (q4_tile_gemm_kernel), and what it takes in whole tiles of 64: a tile of w columns 0.4 + 0.15 w / 16.
 struct TilePlan {
-    int whole, width, blocks;
+    int tokens, whole, width, blocks;
     float cost;
 };
 
@@ -1087,7 +1087,7 @@ struct TilePlan {
 static TilePlan plan_tiles(int TN, int blocks_per_tile, int B, bool narrower) {
     auto cost = [](int w) { return 0.4f + 0.15f / 16 * w; };
     const int t_tiles = (B + TN - 1) / TN, tiles = blocks_per_tile * t_tiles, cus = cu_count();
-    TilePlan p{tiles, TN, tiles, (tiles + cus - 1) / cus * cost(t_tiles > 1 ? TN : (B + 15) / 16 * 16)};
+    TilePlan p{TN, tiles, TN, tiles, (tiles + cus - 1) / cus * cost(t_tiles > 1 ? TN : (B + 15) / 16 * 16)};
     if (narrower && tiles % cus) {
         // Whole tiles for full rounds, to the tile where the narrower ones divide one (three layers of 70B, 750 tokens, where only then
         // those of 32 fit: 10690 -> 10440).
@@ -1095,22 +1095,27 @@ static TilePlan plan_tiles(int TN, int blocks_per_tile, int B, bool narrower) {
         for (int w = TN - 16; w >= 16; w -= 16) {
             const int done = TN % w ? 0 : rounds % t_tiles, per = (B + w - 1) / w, at = begun * per + done * (TN / w), n = blocks_per_tile * per - at;
             const float c = tiles / cus * cost(TN) + cost(w);
-            if (n <= cus && c < p.cost) p = {begun * t_tiles + done, w, begun * t_tiles + done + n, c};
+            if (n <= cus && c < p.cost) p = {TN, begun * t_tiles + done, w, begun * t_tiles + done + n, c};
         }
     }
     return p;
 }
 
+static TilePlan plan_launch(const GemmShape &s, int group_size, int B) {
+    const int all = s.row_blocks * s.slices;
+    const TilePlan p = plan_tiles(s.tokens, all, B, s.tokens == 64);
+    if (s.tokens < 64 || group_size < 64) return p; // (groups of 32 have more scales, and no LDS for 80)
+    const TilePlan wide = plan_tiles(80, all, B, true);
+    return wide.cost < 0.98f * p.cost ? wide : p;
+}
+
 template <int G, int NT, int NW>
-int launch_tile(const Q4Launch &L, const XhList &xh, const float *ss, float *ws, int KS, int partials, int total, hipStream_t st) {
-    const TilePlan p = plan_tiles(16 * NT, total * KS, L.batch, NW == 8);
-    if constexpr (NT == 4 && NW == 8 && G >= 64) // (groups of 32 have more scales, and no LDS for it)
-        if (plan_tiles(80, total * KS, L.batch, true).cost < 0.98f * p.cost) return launch_tile<G, 5, 8>(L, xh, ss, ws, KS, partials, total, st);
+int launch_tile(const Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, const TilePlan &p, int partials, hipStream_t st) {
     size_t lds = 0;
     L2_TRY((ready_tile<G, NT, NW>(&lds)));
     const int t_tiles = (L.batch + 16 * NT - 1) / (16 * NT);
-    l2_launch(q4_tile_gemm_kernel<G, NT, NW>, dim3(p.blocks), dim3(64 * NW), lds, st, L, xh, gemm_padded(L.in), ss, ws, KS, t_tiles, total, p.whole,
-              p.width, partials);
+    l2_launch(q4_tile_gemm_kernel<G, NT, NW>, dim3(p.blocks), dim3(64 * NW), lds, st, L, xh, gemm_padded(L.in), ss, ws, s.slices, t_tiles, s.row_blocks,
+              p.whole, p.width, partials);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }
@@ -1127,9 +1132,12 @@ int ready_group() {
 
 template <int G>
 int launch_group(const Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, int partials, hipStream_t st) {
-    if (s.tokens == 64) return launch_tile<G, 4, 8>(L, xh, ss, ws, s.slices, partials, s.row_blocks, st);
-    if (s.tokens == 32) return launch_tile<G, 2, 4>(L, xh, ss, ws, s.slices, partials, s.row_blocks, st);
-    return launch_tile<G, 1, 4>(L, xh, ss, ws, s.slices, partials, s.row_blocks, st);
+    const TilePlan p = plan_launch(s, G, L.batch);
+    if constexpr (G >= 64)
+        if (p.tokens == 80) return launch_tile<G, 5, 8>(L, xh, ss, ws, s, p, partials, st);
+    if (p.tokens == 64) return launch_tile<G, 4, 8>(L, xh, ss, ws, s, p, partials, st);
+    if (p.tokens == 32) return launch_tile<G, 2, 4>(L, xh, ss, ws, s, p, partials, st);
+    return launch_tile<G, 1, 4>(L, xh, ss, ws, s, p, partials, st);
 }
 
 template <int NT>
@@ -1211,6 +1219,13 @@ GemmShape gemm_shape(const Q4Launch &L, int slice_batch, int planes) {
     s.rows = s.tokens == 64 ? 256 : 128;
     s.row_blocks = s.rows == 128 ? rows32 : rows64;
     return s;
+}
+
+GemmTiles gemm_tiles(const Q4Launch &L, int slice_batch, int planes, bool beside) {
+    const GemmShape s = gemm_shape(L, slice_batch, planes);
+    if (planes == 1) return gemm_tiles_f16(s, L.batch, beside);
+    const TilePlan p = L.group_size ? plan_launch(s, L.group_size, L.batch) : plan_tiles(s.tokens, s.row_blocks * s.slices, L.batch, false);
+    return {s.rows, p.tokens, s.slices, p.blocks, p.whole, p.width, 0, p.whole % ((L.batch + p.tokens - 1) / p.tokens) > 0};
 }
 
 int gemm_launch(Q4Launch &L, const XhList &xh, const float *ss, float *ws, size_t ws_floats, int planes, int slice_batch,

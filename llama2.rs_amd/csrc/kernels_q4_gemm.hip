@@ -350,9 +350,9 @@ __device__ __forceinline__ void q4_gemm_tile(const Q4Launch &L, const XhList &xh
 }
 
 // One block per work item.  A unit is a row block and a slice of K.  The first `units` of them, and `extra` tiles of the next one, go in
-// tiles of 32 NB tokens; what whole rounds of blocks leave over goes in tiles of `width`; then come the last tokens of the first units,
-// where they need no more than half a tile.  A tile costs its width in steps of 32 and the dequantisation of its weights (128, 64,
-// 32 tokens of 70B's w1: 119, 75, 62 us).
+// tiles of 16 NT tokens; what whole rounds of blocks leave over goes in tiles of `width`; then come the last tokens of the first units,
+// where they are no more than half a tile and 64.  A tile takes as many 16s as it needs, two at least, and costs those and the
+// dequantisation of its weights (128, 64, 32 tokens of 70B's w1: 119, 75, 62 us).
 template <int G, int NT, int NW>
 __global__ __launch_bounds__(64 * NW, NT > 4 ? 2 : 1) void q4_gemm_kernel(const Q4Launch L, const XhList xh, const float *__restrict__ ss,
                                                       float *__restrict__ ws, int KS, int partials, int row_blocks, int t_full, int units, int extra,
@@ -401,7 +401,7 @@ __global__ __launch_bounds__(64 * NW, NT > 4 ? 2 : 1) void q4_gemm_kernel(const 
 // How the blocks of a launch are dealt out (q4_gemm_kernel), with what it takes: a tile of w tokens 43 + 0.594 w (of 70B's w1: 62,
 // 75 and 119 us for 32, 64 and 128).
 struct GemmPlan {
-    int t_full, units, extra, width, blocks;
+    int tokens, t_full, units, extra, width, blocks;
     float cost;
 };
 
@@ -421,7 +421,7 @@ static GemmPlan plan_tiles(int TN, int all, int B, bool beside) {
     // whole tiles, and the last tokens' where a round leaves room
     const float whole = tile_cost(TN), last = narrow ? tile_cost(std::max((rest + 15) / 16 * 16, 32)) : 0.f;
     const int room = narrow && tiles % cus ? (cus - tiles % cus) * (int)(whole / last) : 0;
-    GemmPlan p{t_full, all, 0, TN, tiles + narrow * all,
+    GemmPlan p{TN, t_full, all, 0, TN, tiles + narrow * all,
                (tiles + cus - 1) / cus * whole + (narrow * all > room ? (narrow * all - room + cus - 1) / cus * last : 0.f)};
     if ((TN > 64 || (TN == 64 && tiles > cus && tiles < 2 * cus)) && tiles % cus) {
         // Whole tiles for full rounds: of these units, and `done` of the next one, without which those of 64 may not fit (three layers of
@@ -430,21 +430,25 @@ static GemmPlan plan_tiles(int TN, int all, int B, bool beside) {
         for (int w = beside ? most : TN - 16; w >= 32; w -= 16) {
             const int n = (done ? (B - done * TN + w - 1) / w : 0) + (all - begun - (done > 0)) * ((B + w - 1) / w) + narrow * begun;
             const float cost = tiles / cus * whole + std::max(tile_cost(w), begun ? last : 0.f);
-            if (n <= cus && cost < p.cost) p = {t_full, begun, done, w, begun * t_full + done + n, cost};
+            if (n <= cus && cost < p.cost) p = {TN, t_full, begun, done, w, begun * t_full + done + n, cost};
         }
     }
     return p;
 }
 
-template <int G, int NT, int NW>
-int launch_gemm(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, int partials, bool beside, hipStream_t st) {
-    constexpr int TN = 16 * NT;
-    int row_blocks = 0;
-    for (int i = 0; i < L.n_mats; i++) row_blocks += L.m[i].row_blocks = (L.m[i].out + 32 * NW - 1) / (32 * NW);
-    const GemmPlan p = plan_tiles(TN, row_blocks * s.slices, L.batch, beside);
+static GemmPlan plan_launch(const GemmShape &s, int B, bool beside) {
+    const int all = s.row_blocks * s.slices;
+    const GemmPlan p = plan_tiles(s.tokens, all, B, beside);
+    if (s.tokens < 128) return p;
     // Tiles of 144 tokens where they take less (and not about the same: 7B, 899 tokens, a cost of 1.00, 3485 -> 3523 us for six layers).
-    if constexpr (NT == 8)
-        if (plan_tiles(144, row_blocks * s.slices, L.batch, beside).cost < 0.98f * p.cost) return launch_gemm<G, 9, NW>(L, xh, ss, ws, s, partials, beside, st);
+    const GemmPlan wide = plan_tiles(144, all, B, beside);
+    return wide.cost < 0.98f * p.cost ? wide : p;
+}
+
+template <int G, int NT, int NW>
+int launch_gemm(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, const GemmPlan &p, int partials, hipStream_t st) {
+    constexpr int TN = 16 * NT;
+    for (int i = 0; i < L.n_mats; i++) L.m[i].row_blocks = (L.m[i].out + 32 * NW - 1) / (32 * NW);
     // Partial tiles past the L2 (what a launch leaves dirty there is written back at its end, see store_through), and past the memory-side
     // cache too where they would fill it: up to 100 MB their consumer finds them there.  Above 16, 64, 100 MB: 7B, 511 tokens 11270 /
     // 11032 / 11038 us; six layers of 7B, 299, 699, 899 1700 / 2768 / 3570, 1666 / 2721 / 3537 and 1673 / 2720 / 3514; four of 13B, 249
@@ -457,17 +461,19 @@ int launch_gemm(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const
     const size_t lds = std::max(GemmLds<G, NW>::size(TN), (size_t)NW * 32 * 36 * sizeof(float));
     static LdsLimit limit(48 * 1024);
     L2_TRY(limit.ensure(reinterpret_cast<const void *>(q4_gemm_kernel<G, NT, NW>), lds));
-    l2_launch((q4_gemm_kernel<G, NT, NW>), grid, block, lds, st, L, xh, ss, ws, s.slices, partials, row_blocks, p.t_full, p.units, p.extra, p.width);
+    l2_launch((q4_gemm_kernel<G, NT, NW>), grid, block, lds, st, L, xh, ss, ws, s.slices, partials, s.row_blocks, p.t_full, p.units, p.extra, p.width);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }
 
 template <int G>
 int launch_gemm_g(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, int partials, bool beside, hipStream_t st) {
-    switch (s.tokens) {
-        case 32: return launch_gemm<G, 2, 4>(L, xh, ss, ws, s, partials, beside, st);
-        case 64: return launch_gemm<G, 4, 4>(L, xh, ss, ws, s, partials, beside, st);
-        case 128: return launch_gemm<G, 8, 8>(L, xh, ss, ws, s, partials, beside, st);
+    const GemmPlan p = plan_launch(s, L.batch, beside);
+    switch (p.tokens) {
+        case 32: return launch_gemm<G, 2, 4>(L, xh, ss, ws, s, p, partials, st);
+        case 64: return launch_gemm<G, 4, 4>(L, xh, ss, ws, s, p, partials, st);
+        case 128: return launch_gemm<G, 8, 8>(L, xh, ss, ws, s, p, partials, st);
+        case 144: return launch_gemm<G, 9, 8>(L, xh, ss, ws, s, p, partials, st);
     }
     return l2_fail(L2_ERR_ARG, "q4 gemm: token tile");
 }
@@ -498,6 +504,11 @@ GemmShape gemm_shape_f16(const Q4Launch &L, int slice_batch) {
         else s.tokens = 64;
     }
     return s;
+}
+
+GemmTiles gemm_tiles_f16(const GemmShape &s, int B, bool beside) {
+    const GemmPlan p = plan_launch(s, B, beside);
+    return {s.rows, p.tokens, s.slices, p.blocks, p.units * p.t_full + p.extra, p.width, B > p.t_full * p.tokens ? B - p.t_full * p.tokens : 0, p.extra > 0};
 }
 
 int gemm_launch_f16(Q4Launch &L, const XhList &xh, const float *ss, float *ws, const GemmShape &s, int partials, bool beside, hipStream_t st) {

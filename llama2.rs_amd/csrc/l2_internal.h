@@ -234,6 +234,14 @@ struct GemmShape {
 };
 GemmShape gemm_shape(const Q4Launch &L, int slice_batch, int planes);
 GemmShape gemm_shape_f16(const Q4Launch &L, int slice_batch);
+// The tiles that a launch of this shape takes, for tests: rows and tokens of a block, slices of K, blocks, how many of them take whole
+// tiles, the width of the tiles of what whole rounds leave over, the tokens behind the whole tiles of a row block where they have a
+// narrower one of their own (fp16), whether a row block has whole tiles and others.
+struct GemmTiles {
+    int rows, tokens, slices, blocks, whole, width, last, both;
+};
+GemmTiles gemm_tiles(const Q4Launch &L, int slice_batch, int planes, bool beside);
+GemmTiles gemm_tiles_f16(const GemmShape &s, int B, bool beside);
 // Y = X W^T for L.batch columns; ss (per column, may be null) scales them.  Epilogues: store, residual add.  ws:
 // workspace for the K slices' partial tiles.  ks_out given: the kernel leaves its slices as partial tiles [KS][B][out]
 // in ws (also when there is one), no reduction is launched, and *ks_out says how many there are.  beside: a launch on another

@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 from llama2_rs import checkpoint as ck
+from tests import test_gemm_plan as shapes  # which tiles the shapes of the GEMMs' tests take
 
 pytestmark = pytest.mark.gpu
 
@@ -61,9 +62,9 @@ def test_batch_tiles_vs_fp64(ops, n_in, n_out, G, batches):
     q.close()
 
 
-# the row blocks of a last round in narrower tiles: 97 row blocks, 12 of them in tiles of 32 columns (their last of 22, 17 and 32), 86,
-# 35 of them in tiles of 48 (their last of 18 and 12)
-@pytest.mark.parametrize("n_out,B", [(24584, 150), (24584, 177), (24584, 192), (22008, 258), (22008, 300)])
+# what whole rounds of tiles of 64 and of 80 columns leave over, in tiles of every narrower width, in row blocks of their own and behind whole
+# tiles, last tiles that are not full
+@pytest.mark.parametrize("n_out,B", [s for s in shapes.FP32_TILES if s not in ((16640, 250), (4104, 61))])
 def test_batch_last_round_vs_fp64(ops, n_out, B):
     rng = np.random.default_rng(B)
     qw, qz, sc, gi = ck.synth_qlinear(rng, 256, n_out, 64, act_order=True)
@@ -75,9 +76,9 @@ def test_batch_last_round_vs_fp64(ops, n_out, B):
 
 
 # A column's bits are the same in tiles of every width: rows of weights that repeat every 256 (a block) and columns that repeat every
-# seven give the same outputs wherever they stand.  Row blocks with tiles of both widths (their narrow ones from column 64 or 128 on),
-# tiles of 32 and 48 columns, a last tile of every width, one round with nothing left over.
-@pytest.mark.parametrize("n_out,B", [(24584, 150), (24584, 177), (24584, 192), (22008, 258), (22008, 300), (16640, 250), (4104, 61)])
+# seven give the same outputs wherever they stand.  Row blocks with tiles of both widths, tiles of 16 to 80 columns, one round with
+# nothing left over.
+@pytest.mark.parametrize("n_out,B", list(shapes.FP32_TILES))
 def test_batch_bits_whatever_the_tile(ops, n_out, B):
     rng = np.random.default_rng(B)
     qw, qz, sc, gi = ck.synth_qlinear(rng, 256, 256, 64, act_order=True)
@@ -351,10 +352,9 @@ def test_columns_mode(ops):
         m.close()
 
 
-# tiles of 80 columns, and what rounds leave over in 16, 32 and 48: last tiles of 1, 49, 70 and 80, one, two and three units of K, half a
-# one; a column is the bits it has in a batch of 64
-@pytest.mark.parametrize("n_in,n_out,G,batches", [(128, 22016, 64, (150, 160)), (256, 22016, 128, (129, 150, 225)), (320, 22016, 64, (150,)),
-                                                  (384, 22016, 32, (130, 90)), (384, 12800, 128, (230,))])
+# tiles of 80 columns, alone and with what rounds leave over in 16, and of 64 with 16, 32 and 48: last tiles of 1, 49, 70 and 80, one, two and
+# three units of K, half a one; a column is the bits it has in a batch of 64
+@pytest.mark.parametrize("n_in,n_out,G,batches", [(*s, tuple(by_columns)) for s, by_columns in shapes.FP32_OF_80.items()])
 def test_batch_tiles_of_80(ops, n_in, n_out, G, batches):
     rng = np.random.default_rng(n_in + G)
     qw, qz, sc, gi = ck.synth_qlinear(rng, n_in, n_out, G, act_order=True)
@@ -413,8 +413,9 @@ def test_fp16_operator_wide_blocks(ops, dim, hidden, G, batches):
     m.close()
 
 
-# tiles of 144 tokens: one unit of K, two, three, five and six, a last tile of 113, 129 and 144 tokens; the columns are the bits of tiles of 128
-@pytest.mark.parametrize("dim,hidden,G", [(128, 22016, 32), (128, 22016, 64), (256, 22016, 128), (384, 22272, 64), (640, 22016, 32), (768, 22016, 128)])
+# tiles of 144 tokens and nothing else: one unit of K, two, three, five and six, a last tile of 113, 129 and 144 tokens; the columns are the
+# bits of tiles of 128.  (Narrower ones beside and behind them: test_fp16_bits_whatever_the_tile.)
+@pytest.mark.parametrize("dim,hidden,G", shapes.FP16_OF_144)
 def test_fp16_operator_tiles_of_144(ops, dim, hidden, G):
     from llama2_rs import _lib
     dims = ck.Dims(dim=dim, hidden_dim=hidden, n_layers=1, n_heads=dim // 128, n_kv_heads=dim // 128, vocab_size=64, seq_len=1024,
@@ -433,10 +434,9 @@ def test_fp16_operator_tiles_of_144(ops, dim, hidden, G):
     m.close()
 
 
-# tiles of an odd number of 16 tokens: 112 and 96 (200 columns), 80, 48, a last one of 33, 65, 97, 113, blocks of four waves too; the
+# tiles of an odd number of 16 tokens: of 112 with a last one of 88 (200 columns), 80, 48, a last one of 33, blocks of four waves too; the
 # columns are the bits of tiles of 32
-@pytest.mark.parametrize("dim,hidden,G,batches", [(256, 22016, 64, (200,)), (256, 20480, 128, (240, 193)), (384, 12800, 64, (230, 353)), (256, 12800, 32, (225,)),
-                                                  (512, 1024, 128, (33, 48, 65, 97, 113, 177))])
+@pytest.mark.parametrize("dim,hidden,G,batches", [(*s, tuple(by_columns)) for s, by_columns in shapes.FP16_ODD.items()])
 def test_fp16_operator_odd_tiles(ops, dim, hidden, G, batches):
     from llama2_rs import _lib
     dims = ck.Dims(dim=dim, hidden_dim=hidden, n_layers=1, n_heads=dim // 128, n_kv_heads=dim // 128, vocab_size=64, seq_len=1024,
@@ -456,8 +456,8 @@ def test_fp16_operator_odd_tiles(ops, dim, hidden, G, batches):
     m.close()
 
 
-# the row blocks that whole rounds leave over, in tiles of 64 (300, 350 rows) and of 96 (520, 590): first and last tiles that are
-# not full, a last row block that is not full, whole tiles that end inside eight row blocks
+# what whole rounds leave over of tiles of 144 columns, a narrow last one (300) and 48 (520), and of 128, 32 behind whole tiles of a row block
+# (350) and 96 (590): first and last tiles that are not full, a last row block that is not full, whole tiles that end inside eight row blocks
 @pytest.mark.parametrize("B", [300, 350, 520, 590])
 def test_fp16_operator_last_round(ops, B):
     from llama2_rs import _lib
@@ -474,9 +474,9 @@ def test_fp16_operator_last_round(ops, B):
         assert nrel(got[b], want[b]) < 2e-5, b
 
 
-# as test_batch_bits_whatever_the_tile: tiles of 128 tokens with ones of 64 and 96 for what is left, row blocks that have both, with
-# and without last tokens of their own; blocks of 128 rows, tiles of 64 tokens with ones of 32
-@pytest.mark.parametrize("hidden,B", [(21888, 350), (21888, 590), (25472, 350), (25472, 424), (21888, 520), (15360, 180), (15360, 99)])
+# as test_batch_bits_whatever_the_tile: tiles of 128 and of 144 tokens with narrower ones of 32 to 128 for what is left, row blocks that have
+# both, with and without last tokens of their own; blocks of 128 rows, tiles of 64 tokens with ones of 32
+@pytest.mark.parametrize("hidden,B", list(shapes.FP16_TILES))
 def test_fp16_bits_whatever_the_tile(ops, hidden, B):
     from llama2_rs import _lib
     dims = ck.Dims(dim=256, hidden_dim=hidden, n_layers=1, n_heads=2, n_kv_heads=2, vocab_size=64, seq_len=1024, group_size=64)
