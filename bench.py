@@ -25,6 +25,7 @@ Prints ONE JSON line.
 from __future__ import annotations
 
 import argparse
+import hashlib
 import json
 import os
 import re
@@ -68,39 +69,59 @@ def token_bytes(d, pos: int) -> int:
     return d.n_layers * per_layer + cb["classifier"] + d.dim * 4 + d.dim * 4 + kv
 
 
-def measured_traffic(model: str, kernels: dict):
-    """Mean HBM bytes per q4 launch of a layer from the committed rocprofv3 counter summary
-    profiles/q4_matvec_<model>_decode_hbm_counters.txt (FETCH_SIZE + WRITE_SIZE per dispatch, already scaled
-    to bytes there), matched by kernel name against the kernels this build launches.  Returns
-    (bytes or None, note): None with the reason when the summary is missing or names another build's kernels."""
-    path = os.path.join(ROOT, "profiles", f"q4_matvec_{model}_decode_hbm_counters.txt")
+Q4_SOURCES = ["kernels_q4.hip", "kernels_q4_stream.hip", "q4_common.h", "lanes.h"]
+
+
+def q4_sources_digest() -> str:
+    """What the q4 matvec kernels are compiled from, comments and spacing aside: a counter summary that does not carry it was
+    taken with other kernels, whatever their names."""
+    h = hashlib.sha256()
+    for name in Q4_SOURCES:
+        with open(os.path.join(ROOT, "llama2.rs_amd", "csrc", name)) as f:
+            code = re.sub(r"/\*.*?\*/|//[^\n]*", " ", f.read(), flags=re.S)
+        h.update(" ".join(code.split()).encode())
+    return h.hexdigest()[:16]
+
+
+def counter_summary(name: str):
+    """(table, note) of a committed rocprofv3 counter summary, profiles/<name>: {"FETCH_SIZE": {kernel: bytes}, "WRITE_SIZE": {...}} with
+    the kernels' names without their parameters, as the library gives them, or None with the reason when there is none or it was
+    taken with other kernels."""
+    path, note = os.path.join(ROOT, "profiles", name), f"profiles/{name}"
     if not os.path.exists(path):
-        return None, f"no counter summary profiles/{os.path.basename(path)}"
-    table = counter_table(path)
-    total = 0
-    for cls in Q4_CLASSES:
-        name = kernels.get(cls, "?") + "(Q4Launch)"
-        for section in ("FETCH_SIZE", "WRITE_SIZE"):
-            if name not in table[section]:
-                return None, (f"profiles/{os.path.basename(path)} holds no {section} reading for {name} ({cls}): "
-                              "it was taken with other kernels, take it again")
-            total += table[section][name]
-    return round(total / len(Q4_CLASSES)), f"profiles/{os.path.basename(path)}"
-
-
-def counter_table(path: str) -> dict:
-    """{"FETCH_SIZE": {kernel: bytes}, "WRITE_SIZE": {...}} of a committed counter summary."""
-    table = {"FETCH_SIZE": {}, "WRITE_SIZE": {}}
-    section = None
-    for line in open(path):
+        return None, f"no counter summary {note}"
+    with open(path) as f:
+        lines = f.read().splitlines()
+    if f"sources of the q4 kernels: {q4_sources_digest()}" not in lines:
+        return None, f"{note} was taken with other kernels than this build's, take it again"
+    table, section = {"FETCH_SIZE": {}, "WRITE_SIZE": {}}, None
+    for line in lines:
         m = re.match(r"^(FETCH_SIZE|WRITE_SIZE):", line)
         if m:
             section = m.group(1)
             continue
-        m = re.match(r"^\s+(\d+)\s+([\d.]+)\s+(\d+)\s+(\S.*)$", line)
+        m = re.match(r"^\s+\d+\s+[\d.]+\s+(\d+)\s+([\w:]+(?:<[^()]*>)?)", line)
         if m and section:
-            table[section][m.group(4).strip()] = int(m.group(3))
-    return table
+            table[section][m.group(2)] = int(m.group(1))
+    return table, note
+
+
+def measured_traffic(model: str, kernels: dict):
+    """Mean HBM bytes per q4 launch of a layer from the committed rocprofv3 counter summary
+    profiles/q4_matvec_<model>_decode_hbm_counters.txt (FETCH_SIZE + WRITE_SIZE per dispatch, already scaled
+    to bytes there), matched by kernel name against the kernels this build launches.  Returns
+    (bytes or None, note): None with the reason when the summary is missing or is of another build's kernels."""
+    table, note = counter_summary(f"q4_matvec_{model}_decode_hbm_counters.txt")
+    if table is None:
+        return None, note
+    total = 0
+    for cls in Q4_CLASSES:
+        name = kernels.get(cls, "?")
+        for section in ("FETCH_SIZE", "WRITE_SIZE"):
+            if name not in table[section]:
+                return None, f"{note} holds no {section} reading for {name} ({cls}): take it again"
+            total += table[section][name]
+    return round(total / len(Q4_CLASSES)), note
 
 
 def matvec_run(np, ops, n_inst: int, iters: int, reps: int, cpu: bool) -> dict:
@@ -136,15 +157,12 @@ def matvec_run(np, ops, n_inst: int, iters: int, reps: int, cpu: bool) -> dict:
     n_disp = min(iters, 1024)
     us_disp = ops.qlinear_bench_dispatch(qs, n_disp) / n_disp * 1e3               # us per dispatch, its own events
     kernel = ops.qlinear_kernel(qs[0])
-    traffic, note = None, "no counter summary profiles/q4_matvec_cfg0_hbm_counters.txt"
-    path = os.path.join(ROOT, "profiles", "q4_matvec_cfg0_hbm_counters.txt")
-    if os.path.exists(path):
-        t = counter_table(path)
-        name = kernel + "(Q4Launch)"
-        if name in t["FETCH_SIZE"] and name in t["WRITE_SIZE"]:
-            traffic, note = t["FETCH_SIZE"][name] + t["WRITE_SIZE"][name], "profiles/q4_matvec_cfg0_hbm_counters.txt"
-        else:
-            note = f"profiles/q4_matvec_cfg0_hbm_counters.txt holds no reading for {name}: take it again"
+    traffic = None
+    table, note = counter_summary("q4_matvec_cfg0_hbm_counters.txt")
+    if table is not None and kernel in table["FETCH_SIZE"] and kernel in table["WRITE_SIZE"]:
+        traffic = table["FETCH_SIZE"][kernel] + table["WRITE_SIZE"][kernel]
+    elif table is not None:
+        note += f" holds no reading for {kernel}: take it again"
     gbs = nbytes / us_cad / 1e3   # HIP events around the timed region on the launch stream, divided by its launches
     out = {
         "workload": (f"standalone GPTQ 4-bit act-order matvec (x in natural order -> y), in {n_in}, out {n_out}, group {G}, batch 1; {n_inst} distinct "
