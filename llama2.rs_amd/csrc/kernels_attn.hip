@@ -80,8 +80,8 @@ static_assert(kCombRow * sizeof(float) % 16 == 0, "rows of the merge tiles are w
 // layers, one block -> 8 slices: 1241 -> 1215 us at position 16, 1292 -> 1257 at 120; 13B (40 kv heads), 8 layers, 4
 // slices: 566 -> 561 at 190, where 8 (320 blocks) took 570.  4 waves up to one tile of timesteps (position 16: 1215 us
 // against 1227 with 8 waves), 8 beyond (190: 381 against 383 with 8 layers).  The query heads of one kv head (grouped-query
-// attention, src/models.rs:142-145) are blocks of their own too: they read the same rows out of the same XCD's L2 (blocks are dealt
-// over the XCDs by kv head), and a block has one chain of scores and sums instead of four or eight.  Whole layers, against a block for
+// attention, src/models.rs:142-145) are blocks of their own too: they read the same rows, out of one XCD's L2 where 8 divides the number
+// of kv heads (blocks are dealt over the XCDs in turn, kv head by kv head; with 2 kv heads on four XCDs each), and a block has one chain of scores and sums instead of four or eight.  Whole layers, against a block for
 // all heads of the kv head (in splits beyond 256), at 50, 100, 240 timesteps: 16 heads of 2 kv heads 22.8 / 24.1 / 27.4 ->
 // 21.9 / 22.6 / 22.9 us, 32 of 4 28.3 / 29.8 / 31.8 -> 25.7 / 25.7 / 26.8, 64 of 8 at 500, 800 40.5 / 42.1 -> 37.7 / 38.7 (not taken for
 // eight up to 256, see attn_launch_qg).
@@ -1459,9 +1459,10 @@ int attn_launch_qg(const AttnDecode &a, hipStream_t st) {
         const char *v = getenv("L2_ATTN_IMPL");
         return v && !strcmp(v, "valu");
     }();
-    // With eight query heads per kv head the first 256 timesteps stay on the matrix cores: in other sums the texts that are sampled from
-    // a model are others (of 20 of 60 tokens from 70B's widths three were).  64 heads of 8, 50, 240 timesteps 37.0 / 42.0 us per layer, with blocks of one head
-    // 35.4 / 36.7.
+    // With eight query heads per kv head the first 256 timesteps stay on the matrix cores, although blocks of one head are faster (64 heads
+    // of 8, 50 and 240 timesteps 37.0 / 42.0 us per layer, with blocks of one head 35.4 / 36.7): in other sums the texts that are sampled
+    // from a model are others (of 20 of 60 tokens from 70B's widths three were), and short contexts are where texts are sampled.  It is
+    // that and no rule of reproducibility: the form changes with the length, and with a captured step by the bucket's end.
     if (a.n_splits == 1 && (QG < 8 || valu || a.ts > kFewTimesteps)) { // slices of the head: as many as keep one block per CU
         const bool wide = a.pos >= 64, eight = a.n_heads * 8 <= cu_count();
         if (eight) return wide ? attn_launch_sliced<8, 8>(a, st) : attn_launch_sliced<4, 8>(a, st);
