@@ -26,9 +26,10 @@
 //     of a step, operands are read from LDS four pairs of MFMAs ahead, and a wave's priority falls with its progress since
 //     the last barrier: with equal priorities the older wave of a SIMD ran ahead and waited 30 % of the time at the barrier
 //     (1862 cycles per step of 64 k; 1650 now, 1024 of them MFMAs; what a SIMD can issue is 1104, the rest are waits).
-//   - Power, and with many tokens that is the bound: a kernel that takes fewer cycles runs at a lower clock.  70B's w1|w3, 776 tokens,
-//     runs at 1.86 GHz, 7B's, 511, at 1.63, where nothing but MFMAs on the same data runs at 1.99 (1.8 PFLOP/s) and all-zero
-//     activations at 2.4.  With 32x32x16 MFMAs a step takes 1512 cycles instead of 1658, and the clock falls to 1.57 GHz: 70B's prompt
+//   - Power, and with many tokens that is the bound: a kernel that takes fewer cycles runs at a lower clock.  By cycle stamps in the
+//     kernel, launches back to back, 70B's w1|w3, 776 tokens, runs at 1.86 GHz, 7B's, 511, at 1.63 (by counters of a profiled pass,
+//     with gaps between the launches, 1.83 and 1.97), all-zero activations at 2.4; nothing but MFMAs gives 1.8 PFLOP/s on such data
+//     and 2.4 on zeros.  With 32x32x16 MFMAs a step takes 1512 cycles instead of 1658, and the clock falls to 1.57 GHz: 70B's prompt
 //     14.11 -> 14.41 ms, 7B's 11.22 -> 11.55.  So what counts is the work per token: without the reads of activations from LDS the
 //     launch would take 24 % less, without the folds 15, without the dequantisation 13.  Hence tiles of 144 tokens, as many as the
 //     registers hold, where that makes fewer of them: 70B's 776 tokens 13.97 -> 13.18 ms, six layers of 7B, 280 tokens 1632 -> 1542 us,
