@@ -91,6 +91,22 @@ int l2_qlinear_plan(int in, int out, int group_size, int batch, int natural, cha
  * row block has tiles of both kinds}. */
 int l2_gemm_plan(int in, const int32_t *out, int n_mats, int group_size, int batch, int mode, int32_t *plan);
 
+/* The B = 1 steps of l2_forward, l2_decode_greedy, l2_generate_greedy and l2_generate go through one launch for all layers (the
+ * token kernel) where a query head's blocks take the context whole; the results are the bits of the layers' own launches.
+ * on = 0: the layers' own launches always (so does the environment variable L2_TOKEN_LAUNCHES, read when a model is built).  For tests:
+ * the kernel is launched with `missing` of its blocks left out, so that the others wait in vain, and gives up a wait after `looks` looks (a
+ * multiple of 64 in effect, at most 131072, the default); the call then does its steps again with the layers' own launches. */
+int l2_model_set_token_kernel(l2_model *m, int on, int missing, int looks);
+/* Whether steps may take the token kernel (no more after three calls whose waits were given up), and how many calls had such waits. */
+int l2_model_token_kernel(const l2_model *m, int *on, int *gave_up);
+
+/* How the token kernel deals the rows of a model of these dimensions over its blocks and waves, without a device: info[4] receives {whether
+ * it takes such a model, blocks, waves per block, dynamic LDS bytes}; walks (or null), room for `cap` numbers, receives 16 for every
+ * phase (q|k|v, wo, w1|w3, w2), block and wave: {projection (q, k, v, wo, w1, w3, w2), first row, stride, last row of the block, steps, the
+ * block's first row, its rows, where the wave's partial sums begin, its chunk of 2048 inputs, chunks of 32 inputs, groups, a bit per step
+ * that is rounded as rows behind a launch's loop are, whether one of these is looped, 0, 0, 0}. */
+int l2_token_plan(const l2_dims *d, int32_t *walks, size_t cap, int32_t *info);
+
 /* Plain device-to-device copy of nbytes, iters times: the box's achievable
  * copy bandwidth (bytes moved = 2*nbytes per iteration). */
 int l2_copy_bench(size_t nbytes, int iters, float *ms_total);

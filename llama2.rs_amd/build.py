@@ -26,6 +26,7 @@ SOURCES = {
     "kernels_q4.hip": [],
     # the leading arguments of its kernels arrive in scalar registers
     "kernels_q4_stream.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=14"],
+    "kernels_token.hip": [],
     # MFMA accumulators in VGPRs: the per-group fold reads and writes them with plain FMAs
     "kernels_q4_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "kernels_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1", "-ffp-contract=off"],

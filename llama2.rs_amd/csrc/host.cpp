@@ -319,6 +319,7 @@ struct l2_model {
         float *logits = nullptr;               // [vocab]: logits, or the sampler's weights
         unsigned long long *redo = nullptr;    // one bit per vocabulary entry
         int32_t *ids = nullptr, *in = nullptr; // [max_seq] out; [2 * max(max_seq, 4096)] in
+        volatile int *gave_up = nullptr;       // TokArgs::failed_host
         bool reading = false; // a copy from `in` may still be on its way: no call has waited since
     } hs;
     static constexpr int kMaxLanes = 4; // the process has four hardware queues
@@ -343,6 +344,23 @@ struct l2_model {
     float *op_x = nullptr, *op_xg = nullptr, *op_y = nullptr;
     size_t op_cap = 0;
     OperatorBufs op_batch;
+    // All layers of a decode step in one launch (kernels_token.hip).
+    struct TokenKernel {
+        bool on = false;
+        bool skip = false;      // this call's steps are done again with the layers' own launches
+        int gave_up = 0;        // calls that had to be
+        int missing = 0;        // l2_model_set_token_kernel
+        TokModel *model = nullptr; // in device memory
+        uint16_t *slots = nullptr;
+        TokWalk *walks = nullptr;
+        float *handed = nullptr; // two sets, used in turn: a step's kernel empties the other
+        size_t set_floats = 0;
+        int set = 0, grid = 0;
+        size_t lds = 0;
+        bool eight = false;
+        int *failed = nullptr;
+    } tok;
+    int device = 0;
     // per-launch event timing, on only inside l2_decode_profile
     struct ProfRec { int cls; hipEvent_t e0, e1; };
     bool prof_on = false;
@@ -404,6 +422,30 @@ static int timed_launch(l2_model *m, int cls, F &&launch) {
         else                                                                 \
             L2_TRY(call);                                                    \
     } while (0)
+
+// Blocks of a token kernel wait for one another, so all of them have to find room on the device, which two such kernels at once might not
+// (each would hold compute units that the other's blocks wait for).  So one model at a time has them in flight; the steps of
+// others go out as launches of their own meanwhile, which only ever wait for kernels that end.
+struct TokenDevice {
+    static constexpr int kMaxDevices = 64;
+    std::mutex mu;
+    const l2_model *owner[kMaxDevices] = {};
+    // Whether m may launch one now; it is then the owner until it has left().
+    bool claim(const l2_model *m) {
+        if (m->device < 0 || m->device >= kMaxDevices) return false;
+        std::lock_guard<std::mutex> lock(mu);
+        if (owner[m->device] && owner[m->device] != m) return false;
+        owner[m->device] = m;
+        return true;
+    }
+    // The caller has waited for everything on m's stream.
+    void left(const l2_model *m) {
+        if (m->device < 0 || m->device >= kMaxDevices) return;
+        std::lock_guard<std::mutex> lock(mu);
+        if (owner[m->device] == m) owner[m->device] = nullptr;
+    }
+};
+static TokenDevice token_device;
 
 struct StepGraph {
     hipGraph_t graph = nullptr;
@@ -529,6 +571,8 @@ static size_t make_group_tiles(DevQLinear &q, float *tiles) {
     q.zeros_t = reinterpret_cast<const int32_t *>(tiles + (size_t)((q.out + 31) / 32) * q.groups * 32);
     return group_tiles_floats(q.out, q.groups);
 }
+
+static int token_kernel_setup(l2_model *m);
 
 static int model_build(const char *weights, size_t nbytes, const l2_dims *dims, int max_seq, l2_model **out) {
     L2_TRY(check_dims(dims));
@@ -708,7 +752,7 @@ static int model_build(const char *weights, size_t nbytes, const l2_dims *dims, 
     {
         const size_t redo = ((size_t)dims->vocab_size * 4 + 255) / 256 * 256,
                      ids = redo + ((size_t)dims->vocab_size / 64 + 32) / 32 * 256,
-                     in = ids + ((size_t)max_seq * 4 + 255) / 256 * 256, end = in + (size_t)std::max(max_seq, 4096) * 8;
+                     in = ids + ((size_t)max_seq * 4 + 255) / 256 * 256, flag = in + (size_t)std::max(max_seq, 4096) * 8, end = flag + 256;
         void *p = nullptr;
         M_HIP(hipHostMalloc(&p, end, hipHostMallocCoherent));
         m->hs.base = (char *)p;
@@ -716,7 +760,11 @@ static int model_build(const char *weights, size_t nbytes, const l2_dims *dims, 
         m->hs.redo = (unsigned long long *)(m->hs.base + redo);
         m->hs.ids = (int32_t *)(m->hs.base + ids);
         m->hs.in = (int32_t *)(m->hs.base + in);
+        m->hs.gave_up = (volatile int *)(m->hs.base + flag);
+        *m->hs.gave_up = 0;
     }
+    M_HIP(hipGetDevice(&m->device));
+    M_TRY(token_kernel_setup(m));
     M_HIP(hipDeviceSynchronize());
 #undef M_HIP
 #undef M_TRY
@@ -780,8 +828,10 @@ extern "C" void l2_model_close(l2_model *m) {
         if (es) (void)hipStreamSynchronize(es);
     void *ptrs[] = {m->dimage, m->dinv, m->dtiles, m->rope_cos, m->rope_sin, m->dwn, m->attn_part, m->x, m->xq, m->xk,
                     m->xv, m->qv, m->kv, m->vv, m->attg, m->x1, m->x3, m->hg, m->hd, m->logits, m->dtok, m->dpos, m->dloop,
-                    m->amax, m->dprompt, m->dout_ids, m->op_x, m->op_xg, m->op_y, m->op_batch.planes, m->op_batch.ws};
+                    m->amax, m->dprompt, m->dout_ids, m->op_x, m->op_xg, m->op_y, m->op_batch.planes, m->op_batch.ws,
+                    m->tok.handed, m->tok.failed, m->tok.model, m->tok.slots, m->tok.walks};
     for (void *p : ptrs) dfree(p);
+    token_device.left(m);
     for (auto &a : m->lane) {
         void *bufs[] = {a.x, a.q, a.ss, a.ws, a.h[0], a.h[1], a.h[2]};
         for (void *p : bufs) dfree(p);
@@ -1467,6 +1517,7 @@ struct ForwardIn {
     const int32_t *dpos = nullptr;
     float *logits = nullptr;             // B == 1: where the logits go, or null
     unsigned long long *amax = nullptr;  // and their running maximum
+    bool whole = false;                  // B == 1: the caller asks token_gave_up behind its wait, so the token kernel may be taken
 };
 static int forward_enqueue_dense(l2_model *m, l2_state *s, int B, int max_pos, const ForwardIn &in);
 
@@ -1485,6 +1536,7 @@ static int wait_host(l2_model *m, const unsigned long long *amax, int32_t *id) {
     if (amax) L2_TRY(index_launch(amax, id, m->stream));
     L2_HIP(hipStreamSynchronize(m->stream));
     m->hs.reading = false;
+    token_device.left(m);
     return L2_OK;
 }
 
@@ -1496,6 +1548,191 @@ static int claim_host_ids(l2_model *m) {
     return L2_OK;
 }
 
+// How the token kernel deals a model's rows over its blocks and waves.
+struct TokenPlan {
+    TokPhase phase[4] = {};
+    std::vector<TokWalk> walks; // [4][grid][kTokenWaves]
+    int grid = 0, part_at = 0;  // part_at: TokModel::part_at
+    size_t lds = 0;
+    bool eight = false;         // slices of a head: eight or four, as many as keep one block per CU
+};
+// The launches of a layer's four kinds of matvec, for their plans alone.
+static void layer_launches(const l2_dims &d, Q4Launch (&L)[4]) {
+    static const float some[4] = {0.f, 0.f, 0.f, 0.f}; // pointers count as null or not
+    const auto one = [&](Q4Launch &l, std::initializer_list<int> outs, int in, bool norm) {
+        DevQLinear q;
+        q.in = in, q.group_size = d.group_size, q.groups = in / d.group_size;
+        l = launch_of(q, 1, 0.f);
+        l.n_mats = 0;
+        for (int out : outs) {
+            q.out = out;
+            l.m[l.n_mats++] = mat_of(q, some, norm ? some : nullptr, nullptr);
+        }
+    };
+    for (auto &l : L) l = Q4Launch{};
+    const int kvd = d.dim / d.n_heads * d.n_kv_heads;
+    one(L[TOK_QKV], {d.dim, kvd, kvd}, d.dim, true);
+    one(L[TOK_WO], {d.dim}, d.dim, false);
+    one(L[TOK_W13], {d.hidden_dim, d.hidden_dim}, d.dim, true);
+    one(L[TOK_W2], {d.dim}, d.hidden_dim, false);
+    L[TOK_W13].pair = 1, L[TOK_W13].e.kind = Q4_EPI_SCATTER_ONLY;
+    L[TOK_WO].e.kind = L[TOK_W2].e.kind = Q4_EPI_RESIDUAL;
+}
+
+// *ok: whether decode steps of such a model can go through the token kernel.
+static int token_plan(const l2_dims &d, TokenPlan &t, bool *ok) {
+    *ok = false;
+    if (d.group_size == 0) return L2_OK;
+    const int grid = t.grid = cu_count(), qg = d.n_heads / d.n_kv_heads;
+    t.eight = d.n_heads * 8 <= grid;
+    if (d.dim / d.n_heads != 128 || d.n_heads * (t.eight ? 8 : 4) > grid || (qg != 1 && qg != 2 && qg != 4 && qg != 8)) return L2_OK;
+    Q4Launch L[4];
+    layer_launches(d, L);
+    t.walks.assign((size_t)4 * grid * kTokenWaves, TokWalk{});
+    int part = 0;
+    for (int p = 0; p < 4; p++) {
+        char name[160];
+        g_q4_name = Q4NameHook{};
+        g_q4_name.buf = name, g_q4_name.cap = (int)sizeof name, g_q4_name.armed = true;
+        const int rc = q4_matvec_launch(L[p], nullptr);
+        const bool answered = !g_q4_name.armed;
+        g_q4_name.armed = false;
+        L2_TRY(rc);
+        const RowPlan plan = g_q4_name.rows;
+        if (!answered || plan.unit < 1) return L2_OK; // not the streaming fp32 form, whose sums the kernel repeats
+        const bool norm = p == TOK_QKV || p == TOK_W13;
+        const int in = L[p].in, C = in / 32, nwk = (C + 63) / 64, halves = p == TOK_W13 ? 2 : 1, n_mats = p == TOK_QKV ? 3 : 1;
+        TokPhase &f = t.phase[p];
+        f.n4 = in / 4, f.nwk = nwk, f.nwx = plan.nwx, f.direct = plan.direct, f.vec_floats = nwk * 64 * 36;
+        f.gshift = L[p].group_size == 128 ? 2 : L[p].group_size == 64 ? 1 : 0;
+        if (nwk > kTokenWaves || (norm && (nwk > 4 || f.nwx > kTokenWaves || f.nwx % 4 || nwk * 512 > 2 * f.nwx * 64))) return L2_OK;
+        // every block gets the same number of rows; q, k and v round up separately
+        long rows = 0;
+        for (int i = 0; i < n_mats; i++) {
+            rows += L[p].m[i].out;
+            const uint64_t bytes = (uint64_t)L[p].m[i].out * (in / 2 + L[p].groups * 4 + L[p].groups / 2 + 1);
+            if (bytes >= (uint64_t)1 << 31) return L2_OK; // a matrix's arrays are one buffer with 32-bit offsets
+        }
+        int rpb = (int)((rows + grid - 1) / grid);
+        const auto blocks = [&](int i) { return (L[p].m[i].out + rpb - 1) / rpb; };
+        if (n_mats == 3)
+            while (blocks(0) + blocks(1) + blocks(2) > grid) rpb++;
+        // wo: by the waves that do not attend, whose rows come in while the others do, unless these would be many (7B 224 -> 215 us)
+        int wave0 = 0, streams = kTokenWaves / nwk / halves;
+        if (p == TOK_WO && nwk <= 8 && rpb <= 8 / nwk * (kTokenRows + 1)) wave0 = 8, streams = 8 / nwk;
+        // A wave with more rows than that reads for so long that there is nothing to gain (70B's w1|w3, 56 pairs a wave: two layers behind 280
+        // positions, with the classifier, 337.6 us as launches and 338.6 so; 13B's 27: 243 and 231).
+        if (rpb > kTokenWaves * 64 || rpb > 32 * streams) return L2_OK;
+        const auto whole = [&](int n) { return (n + plan.streams - 1) / plan.tile * plan.tile; };
+        for (int b = 0; b < grid; b++) {
+            int rb = b, mi = 0;
+            while (mi + 1 < n_mats && rb >= blocks(mi)) rb -= blocks(mi), mi++;
+            const int out = L[p].m[mi].out;
+            for (int w = 0; w < kTokenWaves; w++) {
+                TokWalk &k = t.walks[((size_t)p * grid + b) * kTokenWaves + w];
+                int s = w < wave0 ? streams * halves : (w - wave0) / nwk;
+                k.kslice = w < wave0 ? 0 : (w - wave0) % nwk;
+                k.r0 = rb * rpb, k.n = std::max(0, std::min(rpb, out - k.r0));
+                k.mat = p == TOK_QKV ? mi : p == TOK_WO ? 3 : p == TOK_W13 ? 4 : 6;
+                if (halves == 2 && s >= streams) s -= streams, k.mat = 5, k.part_row = k.n; // the second half of the waves has w3
+                k.first = k.r0 + s, k.stride = streams, k.last = std::max(k.r0 + k.n - 1, 0);
+                k.steps = s < streams && k.n > s ? (k.n - s + streams - 1) / streams : 0;
+                k.C = C, k.groups = L[p].groups;
+                for (int i = 0; i < k.steps; i++) {
+                    const int o = k.first + i * k.stride, u = o / plan.unit, n = std::min(plan.unit, out - u * plan.unit);
+                    if (o - u * plan.unit < whole(n)) continue;
+                    k.behind |= 1u << i;
+                    if (i < (k.steps - 1) / kTokenRows * kTokenRows) k.behind_early = 1;
+                }
+            }
+        }
+        part = std::max(part, rpb * nwk * 4 * halves);
+    }
+    t.part_at = std::max(3 * t.phase[TOK_QKV].vec_floats, t.phase[TOK_W2].vec_floats);
+    t.lds = ((size_t)t.part_at + part) * 4;
+    *ok = t.lds + 8 * 1024 <= 160 * 1024;
+    return L2_OK;
+}
+
+// Every place that a step hands values on through becomes absent.
+static int token_kernel_clear(l2_model *m) {
+    L2_HIP(hipMemsetAsync(m->tok.handed, 0xFF, 2 * m->tok.set_floats * 4, m->stream));
+    L2_HIP(hipMemsetAsync(m->tok.failed, 0, 4, m->stream));
+    return L2_OK;
+}
+
+static constexpr int kTokenLooks = 1 << 17; // some 0.1 s
+
+static int token_kernel_setup(l2_model *m) {
+    const l2_dims &d = m->d;
+    l2_model::TokenKernel &t = m->tok;
+    if (getenv("L2_Q4_IMPL") || getenv("L2_ATTN_IMPL") || getenv("L2_TOKEN_LAUNCHES")) return L2_OK; // other forms of the launches
+    TokenPlan plan;
+    bool ok = false;
+    L2_TRY(token_plan(d, plan, &ok));
+    if (!ok) return L2_OK;
+    t.grid = plan.grid, t.lds = plan.lds, t.eight = plan.eight;
+    TokModel a{};
+    memcpy(a.phase, plan.phase, sizeof a.phase);
+    a.part_at = plan.part_at;
+    a.n_layers = d.n_layers, a.dim = d.dim, a.kv_dim = m->kv_dim, a.n_heads = d.n_heads, a.n_kv_heads = d.n_kv_heads;
+    a.at_qkv = d.dim, a.at_att = a.at_qkv + d.dim + 2 * m->kv_dim, a.at_xm = a.at_att + d.dim, a.at_hg = a.at_xm + d.dim;
+    a.layer_floats = a.at_hg + d.hidden_dim;
+    a.cache_layer = (size_t)m->max_seq * m->kv_dim;
+    a.eps = m->rms_eps;
+    a.limit = kTokenLooks;
+    t.set_floats = (size_t)d.n_layers * a.layer_floats;
+    size_t n_orders = 0;
+    for (const auto &proj : m->q)
+        for (const DevQLinear &q : proj) n_orders += (size_t)q.in;
+    L2_TRY(dalloc(&t.slots, n_orders));
+    L2_TRY(token_slots_launch(t.slots, m->dinv, n_orders, m->stream));
+    L2_TRY(dalloc(&t.walks, plan.walks.size()));
+    L2_HIP(hipMemcpy(t.walks, plan.walks.data(), plan.walks.size() * sizeof(TokWalk), hipMemcpyHostToDevice));
+    L2_TRY(dalloc(&t.handed, 2 * t.set_floats));
+    L2_TRY(dalloc(&t.failed, (size_t)1));
+    L2_TRY(dalloc(&t.model, (size_t)1));
+    const auto at = [](const void *p) { return (uint64_t)(uintptr_t)p; };
+    a.walks = at(t.walks), a.rms_att = at(m->rms_att), a.rms_ffn = at(m->rms_ffn);
+    a.cos_t = at(m->rope_cos), a.sin_t = at(m->rope_sin);
+    a.failed = at(t.failed), a.failed_host = at(const_cast<int *>(m->hs.gave_up));
+    // The layers' arrays stand at equal distances in the image and among the orders; the kernel counts on it.
+    const int order[7] = {L2_WQ, L2_WK, L2_WV, L2_WO, L2_W1, L2_W3, L2_W2}, consumer[7] = {L2_WQ, L2_WK, L2_WV, L2_W1, L2_W3, L2_W2, L2_WO};
+    for (int i = 0; i < 7; i++) {
+        const DevQLinear &q = m->q[order[i]][0];
+        TokMat &w = a.m[i];
+        w.qweight = at(q.qweight);
+        w.scales_at = (uint32_t)(at(q.scales) - w.qweight), w.zeros_at = (uint32_t)(at(q.qzeros) - w.qweight);
+        w.stride = d.n_layers > 1 ? at(m->q[order[i]][1].qweight) - w.qweight : 0;
+        const int32_t *const first = m->q[consumer[i]][0].inv_index;
+        a.slots[i] = at(t.slots + (first - m->dinv));
+        for (int l = 0; l < d.n_layers; l++) {
+            const DevQLinear &k = m->q[order[i]][l], &o = m->q[consumer[i]][l];
+            const uint64_t base = w.qweight + l * w.stride;
+            if (at(k.qweight) != base || at(k.scales) != base + w.scales_at || at(k.qzeros) != base + w.zeros_at ||
+                o.inv_index != first + (size_t)l * o.in)
+                return l2_fail(L2_ERR_FORMAT, "internal: layers at unequal distances");
+        }
+    }
+    L2_HIP(hipMemcpy(t.model, &a, sizeof a, hipMemcpyHostToDevice));
+    L2_TRY(token_kernel_clear(m));
+    t.on = true;
+    return L2_OK;
+}
+
+// Behind a wait for the stream: whether a token kernel gave up waiting (its blocks did not all find room on the device, which other
+// processes share), so that the call's steps have to be done again.
+static int token_gave_up(l2_model *m, bool *again) {
+    *again = false;
+    if (!m->tok.on || !*m->hs.gave_up) return L2_OK;
+    L2_TRY(token_kernel_clear(m));
+    L2_HIP(hipStreamSynchronize(m->stream));
+    *m->hs.gave_up = 0;
+    if (++m->tok.gave_up >= 3) m->tok.on = false;
+    *again = true;
+    return L2_OK;
+}
+
 static int forward_enqueue(l2_model *m, l2_state *s, int B, int max_pos, const ForwardIn &in) {
     L2_TRY(check_position(m, max_pos));
     s->rows = std::max(s->rows, max_pos + 1);
@@ -1503,6 +1740,24 @@ static int forward_enqueue(l2_model *m, l2_state *s, int B, int max_pos, const F
     const l2_dims &d = m->d;
     const int dim = d.dim, hid = d.hidden_dim, kvd = m->kv_dim, L = d.n_layers;
     hipStream_t st = m->stream;
+    bool whole = in.whole && m->tok.on && !m->tok.skip && !m->capturing && !m->prof_on;
+    if (whole) { // contexts that one query head's blocks take whole, see attn_launch_qg
+        int ts = 0, n_splits = 0;
+        attn_split_policy(max_pos + 1, d.n_heads, d.n_kv_heads, &ts, &n_splits);
+        whole = n_splits == 1 && (d.n_heads < 8 * d.n_kv_heads || ts > kFewTimesteps) && token_device.claim(m);
+    }
+    if (whole) {
+        l2_model::TokenKernel &t = m->tok;
+        float *const handed = t.handed + (t.set ? t.set_floats : 0), *const clear = t.handed + (t.set ? 0 : t.set_floats);
+        const TokArgs a{t.model, handed, clear, m->x, s->kcache, s->vcache, max_pos};
+        ScatterTargets to{};
+        L2_TRY(embed_launch(m->x, m->tok_emb, in.src, dim, 1, to, in.amax, st));
+        L2_TRY(token_layers_launch(a, t.grid - t.missing, t.lds, t.eight, st));
+        t.set ^= 1;
+        if (in.logits)
+            L2_TRY(dense_matvec_launch(in.logits, m->wcls, m->x, m->rms_final, m->rms_eps, dim, d.vocab_size, in.amax, st));
+        return L2_OK;
+    }
     {   // :189-191
         ScatterTargets t{};
         t.n = 3;
@@ -1850,10 +2105,14 @@ extern "C" int l2_forward(l2_model *m, l2_state *s, const int32_t *tokens, const
         return wait_host(m, nullptr, nullptr);
     }
     ForwardIn in;
-    in.src.token = tokens[0];
+    in.src.token = tokens[0], in.whole = true;
     in.logits = logits_host ? m->hs.logits : m->logits, in.amax = m->amax;
-    L2_TRY(forward_enqueue(m, s, 1, max_pos, in));
-    L2_TRY(wait_host(m, nullptr, nullptr));
+    for (bool again = true; again;) {
+        L2_TRY(forward_enqueue(m, s, 1, max_pos, in));
+        L2_TRY(wait_host(m, nullptr, nullptr));
+        L2_TRY(token_gave_up(m, &again));
+        m->tok.skip = again;
+    }
     if (logits_host) memcpy(logits_host, m->hs.logits, (size_t)m->d.vocab_size * 4);
     return L2_OK;
 }
@@ -1864,15 +2123,20 @@ int l2_forward_weights(l2_model *m, l2_state *s, int32_t token, int32_t pos, flo
     L2_TRY(check_tokens(m, &token, &pos, 1, &max_pos));
     L2_TRY(ensure_batch(m, 1));
     ForwardIn in;
-    in.src.token = token, in.logits = m->logits, in.amax = m->amax;
-    L2_TRY(forward_enqueue(m, s, 1, pos, in));
-    L2_TRY(sample_weights_launch(m->hs.logits, m->hs.redo, m->logits, m->d.vocab_size, temperature, m->amax, m->stream));
-    if (more) { // an event is all that a step inside a call has to wait for (7B: 24 us less than for the stream)
-        if (!m->step_done) L2_HIP(hipEventCreateWithFlags(&m->step_done, hipEventDisableTiming));
-        L2_HIP(hipEventRecord(m->step_done, m->stream));
-        L2_HIP(hipEventSynchronize(m->step_done));
-    } else {
-        L2_TRY(wait_host(m, nullptr, nullptr));
+    in.src.token = token, in.logits = m->logits, in.amax = m->amax, in.whole = true;
+    for (bool again = true; again;) {
+        L2_TRY(forward_enqueue(m, s, 1, pos, in));
+        L2_TRY(sample_weights_launch(m->hs.logits, m->hs.redo, m->logits, m->d.vocab_size, temperature, m->amax, m->stream));
+        if (more) { // an event is all that a step inside a call has to wait for (7B: 24 us less than for the stream)
+            if (!m->step_done) L2_HIP(hipEventCreateWithFlags(&m->step_done, hipEventDisableTiming));
+            L2_HIP(hipEventRecord(m->step_done, m->stream));
+            L2_HIP(hipEventSynchronize(m->step_done));
+            token_device.left(m);
+        } else {
+            L2_TRY(wait_host(m, nullptr, nullptr));
+        }
+        L2_TRY(token_gave_up(m, &again));
+        m->tok.skip = again;
     }
     *out = {m->hs.logits, m->hs.redo};
     return L2_OK;
@@ -1998,6 +2262,7 @@ extern "C" int l2_prefill_chunks(l2_model *m, l2_state *s, const int32_t *tokens
 
 static int steps_enqueue(l2_model *m, l2_state *s, int32_t first, int pos0, int n, const int32_t *prompt, int n_prompt);
 static int steps_collect(l2_model *m, int pos0, int n, const int32_t *prompt, int n_prompt, int32_t *ids);
+static int steps_run(l2_model *m, l2_state *s, int32_t first, int pos0, int n, const int32_t *prompt, int n_prompt, int32_t *ids);
 
 extern "C" int l2_decode_greedy(l2_model *m, l2_state *s, int32_t token, int32_t pos, int32_t *next) {
     if (!m || !s || !next) return l2_fail(L2_ERR_ARG, "null argument");
@@ -2005,8 +2270,7 @@ extern "C" int l2_decode_greedy(l2_model *m, l2_state *s, int32_t token, int32_t
     int max_pos = 0;
     L2_TRY(check_tokens(m, &token, &pos, 1, &max_pos));
     L2_TRY(ensure_batch(m, 1));
-    L2_TRY(steps_enqueue(m, s, token, pos, 1, nullptr, 0));
-    return steps_collect(m, pos, 1, nullptr, 0, next);
+    return steps_run(m, s, token, pos, 1, nullptr, 0, next);
 }
 
 static int ensure_loop_buffers(l2_model *m, int n_prompt, int n_out) {
@@ -2115,9 +2379,10 @@ static int steps_enqueue(l2_model *m, l2_state *s, int32_t first, int pos0, int 
     // 2.1 or 3.2 ms, 4.0 or 4.5 ms in all; 167 steps 14.0 or 14.5).  Asked about in between, the loop takes 4.04 and 14.1 ms in
     // every process.  That pays where a launch is too short to hide the enqueueing (an ask costs the GPU 5 us); not shortly
     // before the end, where the wait would meet it.
-    const int ask_steps = layer_weights(m) < kAskWeights ? std::max(1, kAskLaunches / (5 * m->d.n_layers + 2)) : n;
+    const int launches = m->tok.on && !m->tok.skip ? 3 : 5 * m->d.n_layers + 2;
+    const int ask_steps = layer_weights(m) < kAskWeights ? std::max(1, kAskLaunches / launches) : n;
     ForwardIn in;
-    in.src.token = first, in.logits = m->logits;
+    in.src.token = first, in.logits = m->logits, in.whole = true;
     for (int i = 0; i < n; i++) {
         const int pos = pos0 + i;
         in.amax = m->amax + (i & 1);
@@ -2144,6 +2409,16 @@ static int steps_collect(l2_model *m, int pos0, int n, const int32_t *prompt, in
         for (int i = 0; i < n && pos0 + i < n_prompt; i++) m->hs.ids[i] = prompt[pos0 + i];
     }
     if (ids) memcpy(ids, m->hs.ids, (size_t)n * 4);
+    return L2_OK;
+}
+
+static int steps_run(l2_model *m, l2_state *s, int32_t first, int pos0, int n, const int32_t *prompt, int n_prompt, int32_t *ids) {
+    for (bool again = true; again;) {
+        L2_TRY(steps_enqueue(m, s, first, pos0, n, prompt, n_prompt));
+        L2_TRY(steps_collect(m, pos0, n, prompt, n_prompt, ids));
+        L2_TRY(token_gave_up(m, &again));
+        m->tok.skip = again;
+    }
     return L2_OK;
 }
 
@@ -2192,8 +2467,7 @@ extern "C" int l2_generate_greedy(l2_model *m, l2_state *s, const int32_t *promp
     const int32_t first = pos == 0 ? 1 : prompt[pos - 1]; // :128-132
     const int n = std::max(steps - pos, 0); // :141
     if (n > 0 && pos + n > m->max_seq) return l2_fail(L2_ERR_RANGE, "position %d outside 0..%d", pos + n - 1, m->max_seq - 1);
-    L2_TRY(steps_enqueue(m, s, first, pos, n, prompt, n_prompt));
-    L2_TRY(steps_collect(m, pos, n, prompt, n_prompt, out_ids));
+    L2_TRY(steps_run(m, s, first, pos, n, prompt, n_prompt, out_ids));
     const auto t1 = std::chrono::steady_clock::now(); // :192
     *n_out = n;
     if (ms) *ms = std::chrono::duration<double, std::milli>(t1 - t0).count();
@@ -2313,14 +2587,19 @@ extern "C" int l2_decode_bench(l2_model *m, l2_state *s, int32_t token, int32_t 
     L2_HIP(hipEventCreate(&e0));
     L2_HIP(hipEventCreate(&e1));
     L2_HIP(hipStreamSynchronize(m->stream));
-    L2_HIP(hipEventRecord(e0, m->stream));
-    L2_TRY(steps_enqueue(m, s, token, pos, n_tokens, nullptr, 0));
-    L2_HIP(hipEventRecord(e1, m->stream));
-    L2_HIP(hipEventSynchronize(e1));
-    L2_HIP(hipEventElapsedTime(ms_total, e0, e1));
+    for (bool again = true; again;) {
+        L2_HIP(hipEventRecord(e0, m->stream));
+        L2_TRY(steps_enqueue(m, s, token, pos, n_tokens, nullptr, 0));
+        L2_HIP(hipEventRecord(e1, m->stream));
+        L2_HIP(hipEventSynchronize(e1));
+        L2_HIP(hipEventElapsedTime(ms_total, e0, e1));
+        L2_TRY(steps_collect(m, pos, n_tokens, nullptr, 0, out_ids));
+        L2_TRY(token_gave_up(m, &again));
+        m->tok.skip = again;
+    }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    return steps_collect(m, pos, n_tokens, nullptr, 0, out_ids);
+    return L2_OK;
 }
 
 // Which kernel each q4 launch class of this model's decode step runs: "class=kernel;..." with the kernel's
@@ -2448,6 +2727,36 @@ extern "C" int l2_gemm_plan(int in, const int32_t *out, int n_mats, int group_si
     const GemmTiles t = gemm_tiles(L, batch, mode == L2_PREFILL_MFMA ? 1 : 3, false);
     const int32_t all[8] = {t.rows, t.tokens, t.slices, t.blocks, t.whole, t.width, t.last, t.both};
     memcpy(plan, all, sizeof all);
+    return L2_OK;
+}
+
+extern "C" int l2_model_set_token_kernel(l2_model *m, int on, int missing, int looks) {
+    if (!m || missing < 0 || looks < 1 || looks > kTokenLooks) return l2_fail(L2_ERR_ARG, "bad argument");
+    if (!m->tok.model) return on ? l2_fail(L2_ERR_ARG, "this model has no token kernel") : L2_OK;
+    if (missing >= m->tok.grid) return l2_fail(L2_ERR_ARG, "missing %d of %d blocks", missing, m->tok.grid);
+    L2_HIP(hipStreamSynchronize(m->stream));
+    L2_HIP(hipMemcpy((char *)m->tok.model + offsetof(TokModel, limit), &looks, sizeof looks, hipMemcpyHostToDevice));
+    m->tok.on = on != 0, m->tok.missing = missing, m->tok.gave_up = 0;
+    return L2_OK;
+}
+
+extern "C" int l2_model_token_kernel(const l2_model *m, int *on, int *gave_up) {
+    if (!m || !on || !gave_up) return l2_fail(L2_ERR_ARG, "null argument");
+    *on = m->tok.on, *gave_up = m->tok.gave_up;
+    return L2_OK;
+}
+
+extern "C" int l2_token_plan(const l2_dims *d, int32_t *walks, size_t cap, int32_t *info) {
+    if (!d || !info) return l2_fail(L2_ERR_ARG, "null argument");
+    L2_TRY(check_dims(d));
+    TokenPlan t;
+    bool ok = false;
+    L2_TRY(token_plan(*d, t, &ok));
+    info[0] = ok, info[1] = t.grid, info[2] = kTokenWaves, info[3] = (int32_t)t.lds;
+    if (!ok || !walks) return L2_OK;
+    const size_t n = t.walks.size() * (sizeof(TokWalk) / 4);
+    if (cap < n) return l2_fail(L2_ERR_ARG, "room for %zu numbers, %zu needed", cap, n);
+    memcpy(walks, t.walks.data(), n * 4);
     return L2_OK;
 }
 

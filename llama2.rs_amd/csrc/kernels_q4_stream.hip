@@ -788,6 +788,7 @@ int launch_s(Q4Launch &L, hipStream_t stream) {
         snprintf(g_q4_name.buf, (size_t)g_q4_name.cap, "q4_stream_kernel<%d, %d, %d, %s, %d, %d, %s>", G, NWK, S,
                  PAIR ? "true" : "false", MODE, P, GATHER ? "true" : "false");
         g_q4_name.grid = total, g_q4_name.block = NW * 64, g_q4_name.rows_per_block = rpb, g_q4_name.lds = lds;
+        if (MODE != 1) g_q4_name.rows = {TWO ? rpb / 2 : rpb, TWO ? TR / 2 : TR, TWO ? S / 2 : S, TWO ? NW / 2 : NW, MODE == 2};
         return L2_OK;
     }
     if (lds > 48 * 1024) {

@@ -186,6 +186,14 @@ struct Q4ProfHook {
 };
 extern thread_local Q4ProfHook g_q4_prof;
 
+// How the streaming launch takes its rows: `unit` rows stand behind one another, tiles of `tile` of them, `streams` at once; a row of
+// a unit that is not in a whole tile stands behind the loop.  nwx: waves that the sum of squares of x is taken by; direct: the
+// chunk sums of x are taken by the lanes, one four behind the other.  unit 0: another kernel's.
+struct RowPlan {
+    int unit, tile, streams, nwx;
+    bool direct;
+};
+
 // When armed, the next q4 launch is not launched: the launcher writes the name of the kernel it would run
 // (as a profiler prints it, template arguments included) into buf and disarms the hook.
 struct Q4NameHook {
@@ -194,6 +202,7 @@ struct Q4NameHook {
     bool armed = false;
     int grid = 0, block = 0, rows_per_block = 0; // what the launch would have been
     size_t lds = 0;
+    RowPlan rows{};
 };
 extern thread_local Q4NameHook g_q4_name;
 
@@ -372,6 +381,59 @@ struct AttnDecode {
 };
 int attention_decode_launch(const AttnDecode &a, hipStream_t st);
 
+// ---- all layers of a decode step in one launch (kernels_token.hip) ---------------------------
+
+constexpr int kTokenWaves = 16; // of a block
+constexpr int kTokenRows = 3;   // rows of a wave in flight
+enum { TOK_QKV = 0, TOK_WO = 1, TOK_W13 = 2, TOK_W2 = 3 };
+
+// A projection: its arrays in the first layer, and how far apart those of two layers are (addresses: bytes).
+struct TokMat {
+    uint64_t qweight;
+    uint32_t scales_at, zeros_at; // from qweight
+    uint64_t stride;
+};
+// What is the same for a phase of every layer and wave.
+struct TokPhase {
+    int n4, nwk, gshift;  // inputs / 4, waves per row, log2(chunks of 32 inputs per group)
+    int nwx, vec_floats;  // rmsnorm: waves that the sum of squares is taken by; floats of LDS per staged vector
+    int direct;           // chunk sums of x one four behind the other
+};
+// What a wave does in a phase, the same in every layer: rows first, first + stride, ... (`steps` of them, none beyond `last`) of
+// projection `mat`, the chunks 64 kslice to 64 kslice + 63 of each; bit i of `behind`: step i is a row that stands behind the loop of the launch
+// that does this by itself, where its last bit is another.  The block's rows are n from r0 on, this wave's partial sums stand from row part_row on.
+struct TokWalk {
+    int mat, first, stride, last, steps, r0, n, part_row, kslice, C, groups;
+    uint32_t behind;
+    int32_t behind_early;  // whether one of them is among the looped steps, before the last kTokenRows or fewer
+    int32_t pad[3];
+};
+static_assert(sizeof(TokWalk) == 64, "one scalar load");
+struct TokModel { // in device memory
+    TokPhase phase[4];
+    TokMat m[7];               // q, k, v, wo, w1, w3, w2
+    uint64_t walks;            // [4][blocks][kTokenWaves]
+    uint64_t slots[7];         // of q, k, v, w1, w3, w2, wo: [layers][inputs], 16 bits: where an input stands in LDS (token_slots_launch)
+    uint64_t rms_att, rms_ffn; // [layers][dim]
+    uint64_t cos_t, sin_t;
+    uint64_t failed, failed_host; // set where a wait has been given up, in device and in pinned memory
+    uint64_t cache_layer;      // floats of one layer's K
+    int n_layers, dim, kv_dim, n_heads, n_kv_heads;
+    int layer_floats, at_qkv, at_att, at_xm, at_hg; // places in a layer's stretch; the layer's input stands at its start
+    int part_at;               // floats of LDS in front of the partial sums
+    int limit;                 // looks after which a wait is given up
+    float eps;
+};
+struct TokArgs {
+    const TokModel *model;
+    float *handed;             // [layers][layer_floats]: what blocks hand on in this step, every float absent (all ones) before
+    float *clear;              // the same for the next step
+    float *x;                  // [dim] the residual stream, in and out
+    float *kcache, *vcache;    // [layers][max_seq][kv_dim]
+    int pos;
+};
+int token_slots_launch(uint16_t *out, const int32_t *inv, size_t n, hipStream_t st);
+int token_layers_launch(const TokArgs &a, int grid, size_t lds, bool eight, hipStream_t st);
 // logits = wcls (rmsnorm(x, wn)); folds (value, index) into amax_key when set.
 // wn == nullptr: plain Linear::matvec of x.
 int dense_matvec_launch(float *y, const float *w, const float *x, const float *wn, float eps, int in, int out,

@@ -1,0 +1,131 @@
+"""The token kernel (all layers of a decode step in one launch) against the layers' own launches: the same bits."""
+import ctypes
+import os
+import sys
+import threading
+
+import numpy as np
+import pytest
+
+sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "llama2.rs_amd"))
+from llama2_rs import _lib, ops  # noqa: E402
+from llama2_rs.checkpoint import Dims  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+
+def model(dim, hid, heads, kv, group, layers=2, seed=3, max_seq=1100):
+    d = Dims(dim=dim, hidden_dim=hid, n_layers=layers, n_heads=heads, n_kv_heads=kv, vocab_size=700, seq_len=64, group_size=group)
+    return ops.Model(ops.synth_image(d, seed), d, max_seq=max_seq)
+
+
+def token_kernel(m, on, missing=0, looks=1 << 17):
+    _lib.check(_lib.lib().l2_model_set_token_kernel(m.h, on, missing, looks))
+
+
+def state_of(m):
+    on, gave_up = ctypes.c_int(), ctypes.c_int()
+    _lib.check(_lib.lib().l2_model_token_kernel(m.h, ctypes.byref(on), ctypes.byref(gave_up)))
+    return on.value, gave_up.value
+
+
+def bits(a):
+    return np.ascontiguousarray(a).view(np.uint32)
+
+
+# inputs of one to four waves per row and a part of one, hidden rows of one to fourteen, both associations of the chunk sums, rows behind
+# the launches' loops, 1 to 8 query heads per kv head, slices of 16 and of 32 outputs
+SHAPES = [(512, 768, 4, 2, 32), (1024, 2816, 8, 2, 64), (1152, 32, 9, 9, 32), (1536, 4480, 12, 12, 128), (2048, 13824, 16, 4, 128),
+          (3072, 8192, 24, 3, 64), (4096, 11008, 32, 32, 128), (5120, 5120, 40, 40, 64), (8192, 1024, 64, 8, 32), (2048, 28672, 16, 16, 64)]
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_logits_and_cache_rows_are_those_of_the_launches(shape):
+    m = model(*shape)
+    rng = np.random.default_rng(7)
+    for start, n in ((0, 4), (62, 4), (127, 3), (255, 3), (509, 3), (638, 3), (766, 3), (1023, 2)):
+        tokens = rng.integers(0, 700, n)
+        got = {}
+        for on in (1, 0):
+            token_kernel(m, on)
+            m.reset()
+            if start:
+                m.fill_kv_synthetic(0, start, seed=start)
+            logits = [m.forward([int(t)], [start + i]).copy() for i, t in enumerate(tokens)]
+            got[on] = (logits, [m.read_kv(l, start, n) for l in range(2)])
+        assert state_of(m)[1] == 0
+        for a, b in zip(got[1][0], got[0][0]):
+            assert np.isfinite(b).all() and np.array_equal(bits(a), bits(b)), (shape, start)
+        for (ka, va), (kb, vb) in zip(got[1][1], got[0][1]):
+            assert np.array_equal(bits(ka), bits(kb)) and np.array_equal(bits(va), bits(vb)), (shape, start)
+    m.close()
+
+
+def test_a_loop_of_steps_and_a_value_that_looks_absent():
+    """Greedy tokens over the loop, one call per token, and a step whose residual stream is the NaN that means "absent"."""
+    m = model(1024, 2816, 8, 2, 64)
+    prompt = np.array([5, 17, 99], np.int32)
+    ids = {}
+    for on in (1, 0):
+        token_kernel(m, on)
+        ids[on] = m.generate_greedy(prompt, 120)[0]
+        m.reset()
+        t, one = 5, []
+        for p in range(20):
+            t = m.decode_greedy(t, p)
+            one.append(t)
+        ids[on] = np.concatenate([ids[on], one])
+    assert np.array_equal(ids[1], ids[0])
+    m.close()
+    d = Dims(dim=512, hidden_dim=768, n_layers=2, n_heads=4, n_kv_heads=2, vocab_size=260, seq_len=64, group_size=32)
+    img = ops.synth_image(d, 1)
+    img[4:].view(np.uint32)[:512] = 0xFFFFFFFF  # the first token's embedding
+    m = ops.Model(img, d)
+    assert np.isnan(m.forward([0], [0])).all() and state_of(m) == (1, 0)
+    m.reset()
+    a = m.forward([3], [0]).copy()
+    token_kernel(m, 0)
+    m.reset()
+    assert np.array_equal(bits(a), bits(m.forward([3], [0])))
+    m.close()
+
+
+def test_waits_that_are_given_up():
+    """A block is left out, so that the others wait in vain: they leave after 64 looks, and the call does its steps again."""
+    m = model(1024, 2816, 8, 2, 64)
+    prompt = np.array([5, 17, 99], np.int32)
+    token_kernel(m, 0)
+    want = m.generate_greedy(prompt, 24)[0]
+    m.reset()
+    logits = m.forward([9], [0]).copy()
+    token_kernel(m, 1, missing=1, looks=64)
+    assert np.array_equal(m.generate_greedy(prompt, 24)[0], want) and state_of(m) == (1, 1)
+    m.reset()
+    assert np.array_equal(bits(m.forward([9], [0])), bits(logits)) and state_of(m) == (1, 2)
+    token_kernel(m, 1)  # and with all blocks the kernel is right again
+    assert np.array_equal(m.generate_greedy(prompt, 24)[0], want) and state_of(m) == (1, 0)
+    token_kernel(m, 1, missing=1, looks=64)
+    for i in range(4):  # not asked any more after three calls
+        assert np.array_equal(m.generate_greedy(prompt, 8)[0], want[:6]) and state_of(m) == (int(i < 2), min(i + 1, 3))
+    m.close()
+
+
+def test_models_on_threads():
+    """Two models decode side by side: one of them at a time has token kernels in flight, and both get their own results."""
+    ms = [model(1024, 2816, 8, 2, 64, seed=s) for s in (3, 4)]
+    prompt = np.array([5, 17, 99], np.int32)
+    want = [m.generate_greedy(prompt, 60)[0] for m in ms]
+    bad = []
+
+    def run(i):
+        for _ in range(15):
+            if not np.array_equal(ms[i].generate_greedy(prompt, 60)[0], want[i]):
+                bad.append(i)
+    threads = [threading.Thread(target=run, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad and [state_of(m) for m in ms] == [(1, 0), (1, 0)]
+    for m in ms:
+        m.close()
