@@ -1749,9 +1749,7 @@ static int forward_enqueue(l2_model *m, l2_state *s, int B, int max_pos, const F
     if (whole) {
         l2_model::TokenKernel &t = m->tok;
         float *const handed = t.handed + (t.set ? t.set_floats : 0), *const clear = t.handed + (t.set ? 0 : t.set_floats);
-        const TokArgs a{t.model, handed, clear, m->x, s->kcache, s->vcache, max_pos};
-        ScatterTargets to{};
-        L2_TRY(embed_launch(m->x, m->tok_emb, in.src, dim, 1, to, in.amax, st));
+        const TokArgs a{t.model, handed, clear, m->tok_emb, in.src, in.amax, m->x, s->kcache, s->vcache, max_pos};
         L2_TRY(token_layers_launch(a, t.grid - t.missing, t.lds, t.eight, st));
         t.set ^= 1;
         if (in.logits)
@@ -2379,7 +2377,7 @@ static int steps_enqueue(l2_model *m, l2_state *s, int32_t first, int pos0, int 
     // 2.1 or 3.2 ms, 4.0 or 4.5 ms in all; 167 steps 14.0 or 14.5).  Asked about in between, the loop takes 4.04 and 14.1 ms in
     // every process.  That pays where a launch is too short to hide the enqueueing (an ask costs the GPU 5 us); not shortly
     // before the end, where the wait would meet it.
-    const int launches = m->tok.on && !m->tok.skip ? 3 : 5 * m->d.n_layers + 2;
+    const int launches = m->tok.on && !m->tok.skip ? 2 : 5 * m->d.n_layers + 2;
     const int ask_steps = layer_weights(m) < kAskWeights ? std::max(1, kAskLaunches / launches) : n;
     ForwardIn in;
     in.src.token = first, in.logits = m->logits, in.whole = true;

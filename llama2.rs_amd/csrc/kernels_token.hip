@@ -186,12 +186,23 @@ __global__ __launch_bounds__(kThreads) void token_layers_kernel(const TokArgs S)
     Arrays arrays = arrays_of(A, walk.mat, 0);
     places_of<TOK_QKV>(A, 0, walk.mat, tid, places);
     ask(walk, arrays, at_of(walk, TOK_QKV), pipe);
+    // The step's token (as embed_kernel takes it), whose row of the table is the first layer's input.
+    int token = S.src.token;
+    if (S.src.tokens) token = S.src.tokens[0];
+    else if (S.src.prev) token = (int)(S.src.prev[0] & 0xFFFFFFFFull);
+    token = __builtin_amdgcn_readfirstlane(token);
+    const Floats row0 = (Floats)S.emb + (size_t)token * A->dim;
+    if (blockIdx.x == 0 && tid == 0) {
+        if (S.src.prev) S.src.record[0] = token;
+        if (S.amax) S.amax[0] = 0ull;
+    }
+
     // The last threads finish the block's rows, one each; the residual stream of wo's and w2's rows stays in a register of theirs.
     float res = 0.f;
     {
         const TokWalk k = walk_of(TOK_WO);
         const int fin = tid - (kThreads - (k.n + 63) / 64 * 64);
-        if (fin >= 0 && fin < k.n) res = ((Floats)S.x)[k.r0 + fin];
+        if (fin >= 0 && fin < k.n) res = row0[k.r0 + fin];
     }
 
     const auto phase = [&](auto which, const int l) __attribute__((always_inline)) {
@@ -223,7 +234,7 @@ __global__ __launch_bounds__(kThreads) void token_layers_kernel(const TokArgs S)
         // its own (with the order applied there, 32 blocks write into every cache line that all look at, some 4 us each time).
         float *const raw = lds + 2 * vec_floats;
         if constexpr (kNorm) {
-            const Floats xp = first ? (Floats)S.x : kPair ? E + A->at_xm : E;
+            const Floats xp = first ? row0 : kPair ? E + A->at_xm : E;
             u32x4 v[2];
             for (int looks = 0;;) {
                 bool ok = true;

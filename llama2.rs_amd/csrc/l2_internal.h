@@ -428,7 +428,10 @@ struct TokArgs {
     const TokModel *model;
     float *handed;             // [layers][layer_floats]: what blocks hand on in this step, every float absent (all ones) before
     float *clear;              // the same for the next step
-    float *x;                  // [dim] the residual stream, in and out
+    const float *emb;          // the embedding table: the step starts from its token's row
+    TokenSource src;
+    unsigned long long *amax;  // null, or a running maximum to clear
+    float *x;                  // [dim] the residual stream behind the last layer
     float *kcache, *vcache;    // [layers][max_seq][kv_dim]
     int pos;
 };
