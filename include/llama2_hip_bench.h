@@ -104,7 +104,8 @@ int l2_model_token_kernel(const l2_model *m, int *on, int *gave_up);
  * it takes such a model, blocks, waves per block, dynamic LDS bytes}; walks (or null), room for `cap` numbers, receives 16 for every
  * phase (q|k|v, wo, w1|w3, w2), block and wave: {projection (q, k, v, wo, w1, w3, w2), first row, stride, last row of the block, steps, the
  * block's first row, its rows, where the wave's partial sums begin, its chunk of 2048 inputs, chunks of 32 inputs, groups, a bit per step
- * that is rounded as rows behind a launch's loop are, whether one of these is looped, 0, 0, 0}. */
+ * that is rounded as rows behind a launch's loop are, whether one of these is looped, whether the wave asks for its rows behind
+ * attention, 0, 0}. */
 int l2_token_plan(const l2_dims *d, int32_t *walks, size_t cap, int32_t *info);
 
 /* Plain device-to-device copy of nbytes, iters times: the box's achievable

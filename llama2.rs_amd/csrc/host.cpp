@@ -1617,9 +1617,10 @@ static int token_plan(const l2_dims &d, TokenPlan &t, bool *ok) {
         const auto blocks = [&](int i) { return (L[p].m[i].out + rpb - 1) / rpb; };
         if (n_mats == 3)
             while (blocks(0) + blocks(1) + blocks(2) > grid) rpb++;
-        // wo: by the waves that do not attend, whose rows come in while the others do, unless these would be many (7B 224 -> 215 us)
-        int wave0 = 0, streams = kTokenWaves / nwk / halves;
-        if (p == TOK_WO && nwk <= 8 && rpb <= 8 / nwk * (kTokenRows + 1)) wave0 = 8, streams = 8 / nwk;
+        // wo, where a wave has few rows: those that do not attend have theirs there when attention is, and take more (`early` of a stream)
+        const bool uneven = p == TOK_WO && nwk <= 8 && rpb <= 8 / nwk * (kTokenRows + 1);
+        const int streams = uneven ? 8 / nwk : kTokenWaves / nwk / halves;
+        const int early = uneven ? std::min((rpb + streams - 1) / streams, (rpb + 2 * streams - 1) / (2 * streams) + 1) : 0;
         // A wave with more rows than that reads for so long that there is nothing to gain (70B's w1|w3, 56 pairs a wave: two layers behind 280
         // positions, with the classifier, 337.6 us as launches and 338.6 so; 13B's 27: 243 and 231).
         if (rpb > kTokenWaves * 64 || rpb > 32 * streams) return L2_OK;
@@ -1630,13 +1631,17 @@ static int token_plan(const l2_dims &d, TokenPlan &t, bool *ok) {
             const int out = L[p].m[mi].out;
             for (int w = 0; w < kTokenWaves; w++) {
                 TokWalk &k = t.walks[((size_t)p * grid + b) * kTokenWaves + w];
-                int s = w < wave0 ? streams * halves : (w - wave0) / nwk;
-                k.kslice = w < wave0 ? 0 : (w - wave0) % nwk;
+                const int v = uneven ? w & 7 : w;
+                int s = v / nwk;
+                k.kslice = v % nwk;
                 k.r0 = rb * rpb, k.n = std::max(0, std::min(rpb, out - k.r0));
                 k.mat = p == TOK_QKV ? mi : p == TOK_WO ? 3 : p == TOK_W13 ? 4 : 6;
                 if (halves == 2 && s >= streams) s -= streams, k.mat = 5, k.part_row = k.n; // the second half of the waves has w3
-                k.first = k.r0 + s, k.stride = streams, k.last = std::max(k.r0 + k.n - 1, 0);
-                k.steps = s < streams && k.n > s ? (k.n - s + streams - 1) / streams : 0;
+                // the rows that the wave's half has: all, or for wo the first and the rest
+                const int from = uneven && w < 8 ? std::min(early * streams, k.n) : 0, to = uneven && w >= 8 ? std::min(early * streams, k.n) : k.n;
+                k.first = k.r0 + from + s, k.stride = streams, k.last = std::max(k.r0 + k.n - 1, 0);
+                k.steps = s < streams && to - from > s ? (to - from - s + streams - 1) / streams : 0;
+                k.late = uneven && w < 8 && k.steps > 0;
                 k.C = C, k.groups = L[p].groups;
                 for (int i = 0; i < k.steps; i++) {
                     const int o = k.first + i * k.stride, u = o / plan.unit, n = std::min(plan.unit, out - u * plan.unit);

@@ -177,7 +177,7 @@ __global__ __launch_bounds__(kThreads) void token_layers_kernel(const TokArgs S)
     // What this wave does in a phase.
     const auto walk_of = [&](int ph) __attribute__((always_inline)) {
         const WalkPtr p = (WalkPtr)(uintptr_t)A->walks + (ph * gridDim.x + blockIdx.x) * kWaves + wave;
-        return TokWalk{p->mat, p->first, p->stride, p->last, p->steps, p->r0, p->n, p->part_row, p->kslice, p->C, p->groups, p->behind, p->behind_early, {}};
+        return TokWalk{p->mat, p->first, p->stride, p->last, p->steps, p->r0, p->n, p->part_row, p->kslice, p->C, p->groups, p->behind, p->behind_early, p->late, {}};
     };
     const auto at_of = [&](const TokWalk &k, int ph) __attribute__((always_inline)) { return lane_at(k, A->phase[ph].gshift, lane); };
     RowData pipe[kRows];
@@ -216,7 +216,7 @@ __global__ __launch_bounds__(kThreads) void token_layers_kernel(const TokArgs S)
         const TokWalk k = walk, next = walk_of(NEXT);
         const Arrays arr = arrays, next_arr = arrays_of(A, next.mat, PH == TOK_W2 && !last ? l + 1 : l);
         const LaneAt next_at = at_of(next, NEXT);
-        const int next_steps = last ? 0 : next.steps;
+        const int next_steps = last || (PH == TOK_QKV && next.late) ? 0 : next.steps;
         const Floats E = (Floats)S.handed + (size_t)l * A->layer_floats;
         float *const part = lds + A->part_at;
         const int dim = A->dim, n4 = q->n4, nwk = q->nwk, PW = nwk * 4, nwx = q->nwx, vec_floats = q->vec_floats;
@@ -477,6 +477,7 @@ __global__ __launch_bounds__(kThreads) void token_layers_kernel(const TokArgs S)
             };
             places_of<TOK_WO>(A, l, 0, tid, places);
             if (wave >= NWV) { // nothing to do but to meet the others
+                if (walk.late) ask(walk, arrays, at_of(walk, TOK_WO), pipe);
                 __syncthreads();
                 __syncthreads();
                 return;
@@ -583,6 +584,7 @@ __global__ __launch_bounds__(kThreads) void token_layers_kernel(const TokArgs S)
                 };
                 merge([](float v) { return lanes::both16(v); });
                 merge([](float v) { return lanes::both32(v); });
+                if (walk.late) ask(walk, arrays, at_of(walk, TOK_WO), pipe);
                 if (lane < 16) {
 #pragma unroll
                     for (int e = 0; e < VE; e++) comb[wave][ds * VE + e] = acc[e];
@@ -610,6 +612,7 @@ __global__ __launch_bounds__(kThreads) void token_layers_kernel(const TokArgs S)
                 attend(std::integral_constant<int, 4>());
         } else {
             places_of<TOK_WO>(A, l, 0, tid, places);
+            if (walk.late) ask(walk, arrays, at_of(walk, TOK_WO), pipe);
         }
         if (wave >= 8) { // the same layer's places of the next step are made empty
             const Global<u32x4> clear = (Global<u32x4>)((Floats)S.clear + (size_t)l * A->layer_floats);

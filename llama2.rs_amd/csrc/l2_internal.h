@@ -406,7 +406,8 @@ struct TokWalk {
     int mat, first, stride, last, steps, r0, n, part_row, kslice, C, groups;
     uint32_t behind;
     int32_t behind_early;  // whether one of them is among the looped steps, before the last kTokenRows or fewer
-    int32_t pad[3];
+    int32_t late;          // wo: the wave attends, and asks for its first rows behind that
+    int32_t pad[2];
 };
 static_assert(sizeof(TokWalk) == 64, "one scalar load");
 struct TokModel { // in device memory
