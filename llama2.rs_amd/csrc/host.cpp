@@ -4,6 +4,7 @@
 // (src/inference.rs:16-193), driving the HIP kernels.  Nothing here computes on
 // the CPU except the one-time RoPE angle table and the synthetic-image
 // generator.
+#include <emmintrin.h>
 #include <map>
 #include <fcntl.h>
 #include <math.h>
@@ -550,6 +551,41 @@ static struct HostSlots {
             (void)hipHostFree(s.base);
     }
 } host_slots;
+
+// Device memory that the host writes itself, over the bus (fine-grained; where all of the device's memory is mapped for the host): x of a
+// call on host arrays goes there, and the kernel that needs it reads it on the device.  Before, x went to pinned memory, and a kernel of its
+// own brought it over, or read it from there while it was cut into planes: 4096x4096, one column, 20.3 -> 17.9 us; 13824x5120, 16
+// columns 76.7 -> 67.  The host writes 46 GB/s this way (64 KB 1.7 -> 5.5 us, 885 KB 8.8 -> 19.1), the kernels read the bus at some 32.
+// At most kKept pieces of a device, for as long as the process runs (memory that others may have cached is not given back to be used as
+// something else); a call that finds none free takes the way through pinned memory.
+static struct HostWindows {
+    static constexpr int kKept = 4, kMaxDevices = 64;
+    std::mutex mu;
+    float *idle[kMaxDevices][kKept] = {};
+    int n_idle[kMaxDevices] = {}, made[kMaxDevices] = {};
+
+    float *take(int device) {
+        if (device < 0 || device >= kMaxDevices) return nullptr;
+        std::lock_guard<std::mutex> lock(mu);
+        if (n_idle[device] > 0) return idle[device][--n_idle[device]];
+        if (made[device] >= kKept) return nullptr;
+        int mapped = 0;
+        void *p = nullptr;
+        if (hipDeviceGetAttribute(&mapped, hipDeviceAttributeIsLargeBar, device) != hipSuccess || !mapped ||
+            hipExtMallocWithFlags(&p, HostSlot::kBytes, hipDeviceMallocFinegrained) != hipSuccess) {
+            (void)hipGetLastError();
+            made[device] = kKept; // not here
+            return nullptr;
+        }
+        made[device]++;
+        return (float *)p;
+    }
+    void give(int device, float *p) {
+        if (!p) return;
+        std::lock_guard<std::mutex> lock(mu);
+        idle[device][n_idle[device]++] = p;
+    }
+} host_windows;
 
 static void invert_perm(const int32_t *g, int n, int32_t *inv, bool *ok) {
     std::fill(inv, inv + n, -1);
@@ -1298,7 +1334,7 @@ static int qlinear_scratch(l2_qlinear *q, int B) {
 // From here on x comes in two parts, whose second kernel costs 3 us: 384 KB (24 columns of 4096 inputs) 57.4 us whole, 58.5 by
 // halves, 512 KB 67.8 and 67.9, 768 KB 91.6 and 89.6, 884 KB (16 of 13824) 82.8 and 78.5; with the matvec that permutes x itself
 // 50.1 and 50.5, 62.3 and 61.2, 85.7 and 83.4 for 24, 32 and 48 of 4096.
-static constexpr size_t kSplitBytes = 512 * 1024;
+static constexpr size_t kSplitBytes = 512 * 1024, kWindowBytes = 160 * 1024;
 
 static int operator_enqueue(const DevQLinear &q, const float *dx, float *dxg, float *y, const OperatorBufs &bufs, int planes,
                             int B, hipStream_t st) {
@@ -1323,19 +1359,26 @@ static int matvec_host(const DevQLinear &q, float *dx, float *dxg, float *dy, Op
     }
     HostSlot slot;
     L2_TRY(host_slots.take(&slot));
+    int device = 0;
+    const bool natural = !planes && takes_natural_order(q); // the matvec kernel gathers
+    // A shorter x that a kernel permutes anyway is as quick through pinned memory (13824 and 28672 inputs, one column: 27.6 and 27.0 us, in
+    // device memory 28.3 and 27.3; 13824, three columns 49.7 and 49.5).
+    const bool direct = natural || xb >= kWindowBytes;
+    float *const window = direct && hipGetDevice(&device) == hipSuccess ? host_windows.take(device) : nullptr;
+    float *const x = window ? window : slot.x;
     auto call = [&]() -> int {
-        const bool natural = !planes && takes_natural_order(q); // the matvec kernel gathers
         // a long x in two parts: the host brings the second one while the first crosses the bus
         for (int b0 = 0, b1 = B > 1 && xb >= kSplitBytes ? B / 2 : B; b0 < B; b0 = b1, b1 = B) {
             const size_t at = (size_t)b0 * q.in, n = (size_t)(b1 - b0) * q.in;
-            memcpy(slot.x + at, x_host + at, n * sizeof(float));
-            if (natural)
-                L2_TRY(copy_launch(dx + at, slot.x + at, n, st));
-            else
+            memcpy(x + at, x_host + at, n * sizeof(float));
+            if (window) _mm_sfence(); // written through before the launch is
+            if (!natural)
                 L2_TRY(host_input_launch(planes ? (char *)bufs.planes + (size_t)b0 * planes * gemm_padded(q.in) * 2 : (char *)(dxg + at),
-                                         slot.x + at, q.inv_index, q.in, b1 - b0, planes, st));
+                                         x + at, q.inv_index, q.in, b1 - b0, planes, st));
+            else if (!window)
+                L2_TRY(copy_launch(dx + at, x + at, n, st));
         }
-        if (natural) return q4_one_natural(q, dx, dxg, slot.y, B, st);
+        if (natural) return q4_one_natural(q, window ? window : dx, dxg, slot.y, B, st);
         if (!planes) return q4_one(q, dxg, slot.y, B, st);
         return gemm_operator(q, B, slot.y, planes, bufs.planes, bufs.ws, bufs.ws_floats, st);
     };
@@ -1344,6 +1387,7 @@ static int matvec_host(const DevQLinear &q, float *dx, float *dxg, float *dy, Op
     if (rc == L2_OK && e != hipSuccess) rc = l2_fail(L2_ERR_HIP, "matvec: %s", hipGetErrorString(e));
     if (rc == L2_OK) memcpy(y_host, slot.y, yb);
     host_slots.give(slot);
+    host_windows.give(device, window);
     return rc;
 }
 
