@@ -87,8 +87,9 @@ int l2_qlinear_plan(int in, int out, int group_size, int batch, int natural, cha
 /* The tiles that a batch's GEMM takes, for n_mats (1..3) matrices of `in` inputs and out[i] outputs and `batch` columns in one
  * pass, without a device and without launching: mode L2_PREFILL_FP32 or L2_PREFILL_MFMA.  plan[8] receives {rows of a block,
  * columns of its tile, slices of the inputs, blocks, how many of them take whole tiles, the width of the tiles of what whole
- * rounds of blocks leave over, the last columns where they have a narrower tile of their own (MFMA; else 0), whether a
- * row block has tiles of both kinds}. */
+ * rounds of blocks leave over, the last columns where they have a narrower tile of their own (MFMA) or, with
+ * fp32 weights, the K steps of 64 inputs of a last slice that is shorter than the others, else 0, whether a row block has
+ * tiles of both kinds}. */
 int l2_gemm_plan(int in, const int32_t *out, int n_mats, int group_size, int batch, int mode, int32_t *plan);
 
 /* The B = 1 steps of l2_forward, l2_decode_greedy, l2_generate_greedy and l2_generate go through one launch for all layers (the

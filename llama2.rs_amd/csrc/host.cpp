@@ -1962,7 +1962,8 @@ static Q4Launch layer_launch(const l2_model *m, int i, int B) {
 static bool cut_alike(const l2_model *m, int a, int b, int planes) {
     for (int i = 0; i < 4 && a != b; i++) {
         const Q4Launch L = layer_launch(m, i, a);
-        if (gemm_shape(L, a, planes).slices != gemm_shape(L, b, planes).slices) return false;
+        const GemmShape p = gemm_shape(L, a, planes), q = gemm_shape(L, b, planes);
+        if (p.slices != q.slices || p.last != q.last) return false;
     }
     return true;
 }

@@ -541,7 +541,8 @@ __global__ __launch_bounds__(64 * NW, NT == 1 ? 3 : 2) void q4_tile_gemm_kernel(
 // A wave owns 16 rows x 16 NT tokens, a block 8 waves over the rows: a weight is read and split once for up to 128 tokens.
 // Lane (row r = l % 16, kg = l / 16) loads 8 consecutive weights of each 32 inputs (a row's cache line, in two loads), four
 // such pairs ahead, and splits 32 inputs ahead of the products; the activations of 64 inputs pass through LDS,
-// double-buffered; the sums of the runs wait in LDS, which takes up all of it (NT = 8).  What bounds it is the products
+// double-buffered; the sums of the runs wait in LDS, which takes up all of it (NT = 8), so a compute unit has one block, and a launch
+// of 172 leaves a third of them idle unless K is cut for it (gemm_shape).  What bounds it is the products
 // and what issues beside them, one behind the other: a step of 64 inputs and 112 tokens is 480 instructions per wave, 126 of
 // them products (2016 cycles), 96 the splitting, and two waves per SIMD take some 7000 cycles for it.
 //
@@ -601,7 +602,7 @@ __device__ __forceinline__ bool dense_nan(const uint16_t *x, int k0, int k1) {
 
 template <int NT>
 __device__ __forceinline__ void dense_tile(const Q4Launch &L, const XhList &xl, int in_p, const float *__restrict__ ss, float *__restrict__ ws,
-                                           int KS, int partials, int rb, int ks, int t0) {
+                                           int KS, int last, int partials, int rb, int ks, int t0) {
     using S = DenseLds<NT>;
     constexpr int NP = 3, TN = 16 * NT, THREADS = 64 * kDenseWaves;
     extern __shared__ __align__(16) char lds[];
@@ -617,7 +618,8 @@ __device__ __forceinline__ void dense_tile(const Q4Launch &L, const XhList &xl, 
     const int r = lane & 15, kg = lane >> 4;
     const int obase = rb * kDenseRows + wave * 16;
     const int n_unit = in_p / 64;
-    const int it0 = (int)((long)n_unit * ks / KS), it1 = (int)((long)n_unit * (ks + 1) / KS);
+    const int before = n_unit - last, equal = last ? KS - 1 : KS;
+    const int it0 = ks < equal ? before * ks / equal : before, it1 = ks < equal ? before * (ks + 1) / equal : n_unit;
 
     // activations: pieces of 16 bytes, 8 to a token's 64 inputs in a plane
     constexpr int PIECES = NP * TN * 8, XP = (PIECES + THREADS - 1) / THREADS;
@@ -792,20 +794,22 @@ __device__ __forceinline__ void dense_tile(const Q4Launch &L, const XhList &xl, 
     }
 }
 
-// NT: the tiles of tokens of a block at most; the last one has as many as it needs.
+// NT: the tiles of tokens of a block at most; the last one has as many as it needs.  The slices of K are equal, or the last one
+// is `last` K steps: its blocks come behind all others.
 template <int NT>
 __global__ __launch_bounds__(64 * kDenseWaves, 2) void dense_gemm_kernel(const Q4Launch L, const XhList xl, int in_p,
                                                                          const float *__restrict__ ss, float *__restrict__ ws, int KS,
-                                                                         int t_tiles, int partials) {
-    const int work = xcd_item(blockIdx.x, gridDim.x); // as in q4_tile_gemm_kernel
+                                                                         int t_tiles, int last, int partials) {
+    const int row_blocks = gridDim.x / (t_tiles * KS), front = last ? gridDim.x - row_blocks * t_tiles : gridDim.x;
+    const int b = blockIdx.x;
+    const int work = b < front ? xcd_item(b, front) : front + xcd_item(b - front, gridDim.x - front); // as in q4_tile_gemm_kernel
     int rb = work / t_tiles;
-    const int t0 = (work - rb * t_tiles) * 16 * NT, need = min(NT, (L.batch - t0 + 15) / 16);
-    const int row_blocks = gridDim.x / (t_tiles * KS), ks = rb / row_blocks;
+    const int t0 = (work - rb * t_tiles) * 16 * NT, need = min(NT, (L.batch - t0 + 15) / 16), ks = rb / row_blocks;
     rb -= ks * row_blocks;
     switch (need) {
 #define DENSE_TILE(n) \
     case n: \
-        if constexpr (n <= NT) dense_tile<n>(L, xl, in_p, ss, ws, KS, partials, rb, ks, t0); \
+        if constexpr (n <= NT) dense_tile<n>(L, xl, in_p, ss, ws, KS, last, partials, rb, ks, t0); \
         break
         DENSE_TILE(1);
         DENSE_TILE(2);
@@ -1146,7 +1150,8 @@ int launch_dense(const Q4Launch &L, const XhList &xh, const float *ss, float *ws
     const size_t lds = DenseLds<NT>::kSize;
     L2_TRY(limit.ensure(reinterpret_cast<const void *>(dense_gemm_kernel<NT>), lds));
     const int t_tiles = (L.batch + 16 * NT - 1) / (16 * NT);
-    l2_launch(dense_gemm_kernel<NT>, dim3(s.row_blocks * t_tiles * s.slices), dim3(64 * kDenseWaves), lds, st, L, xh, gemm_padded(L.in), ss, ws, s.slices, t_tiles, partials);
+    l2_launch(dense_gemm_kernel<NT>, dim3(s.row_blocks * t_tiles * s.slices), dim3(64 * kDenseWaves), lds, st, L, xh, gemm_padded(L.in), ss, ws, s.slices, t_tiles, s.last,
+              partials);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }
@@ -1185,7 +1190,7 @@ GemmShape gemm_shape(const Q4Launch &L, int slice_batch, int planes) {
     // The slices of K, of those that take `max_rounds` rounds of one block per CU at most, with the smallest cost: a block costs its
     // share of K, the first and last microseconds (4.5 % of 4096 inputs) and, with several slices, its partial tile, written and
     // read again (7.5 %).
-    auto cheapest = [&](int blocks, int most, int max_rounds) {
+    auto cheapest = [&](int blocks, int most, int max_rounds, float *its = nullptr) {
         const float per = 4096.0f / L.in;
         float best = 0.f;
         int slices = 1;
@@ -1194,13 +1199,30 @@ GemmShape gemm_shape(const Q4Launch &L, int slice_batch, int planes) {
             const float cost = rounds * (1.0f / n + 0.045f * per) + (n > 1 ? 0.075f * per * n * blocks / cus : 0.f);
             if (n == 1 || cost < best) best = cost, slices = n;
         }
+        if (its) *its = best;
         return slices;
     };
     if (L.group_size == 0) {
         // Blocks of 128 columns, so that a weight is read and split once; of 64 where those would leave half the CUs without a
         // block (four layers of 1024 inputs, 128 columns: 424 -> 363 us; 7B's widths keep 128: 64 columns at three quarters of
         // the CUs 530 -> 585).  128 inputs per slice at least (1024 inputs, 100 columns 367 us with 256, 348; with 64 349).
-        s.slices = cheapest(rows32 * ((slice_batch + 127) / 128), std::min(kMaxGemmSlices, L.in / 128), 4);
+        const int blocks = rows32 * ((slice_batch + 127) / 128), n_unit = gemm_padded(L.in) / 64;
+        float best = 0.f;
+        s.slices = cheapest(blocks, std::min(kMaxGemmSlices, L.in / 128), 4, &best);
+        // Or n equal slices and one of `last` steps of 64 inputs, of which the CUs that the last round of the others leaves take `each` in
+        // their time, 2.9 steps (the 4.5 % above) to begin and end each: w1|w3 of 7B's widths, 172 row blocks, is one block per CU and
+        // two thirds of the CUs in whole rows, 50 steps and three times 14 with it.  Two layers, 100 columns, with the logits 1341 -> 1286 us
+        // (short slices of 12, 16, 18, 20 steps 1311 / 1316 / 1339 / 1365; four equal ones 1329); q|k|v in 26 + 26 + 12 steps for 32 + 32 another 10
+        // (3 x 16 + 16 67 more, five equal ones 11 more).
+        const float per = 4096.0f / L.in;
+        for (int n = 1; n + 1 < kMaxGemmSlices && n * blocks <= 4 * cus; n++) {
+            const int rounds = (n * blocks + cus - 1) / cus, idle = rounds * cus - n * blocks;
+            if (!idle) continue;
+            const int each = (blocks + idle - 1) / idle, last = (int)((n_unit - 2.9f * n * (each - 1)) / (n * each + 1));
+            if (last < 2) continue;
+            const float cost = rounds * ((float)(n_unit - last) / (n * n_unit) + 0.045f * per) + 0.075f * per * (n + 1) * blocks / cus;
+            if (cost < 0.97f * best) best = cost, s.slices = n + 1, s.last = last;
+        }
         s.tokens = B <= 32 ? 32 : B <= 64 || 2 * rows32 * ((B + 127) / 128) * s.slices <= cus ? 64 : 128;
         s.rows = 128, s.row_blocks = rows32;
         return s;
@@ -1225,7 +1247,7 @@ GemmTiles gemm_tiles(const Q4Launch &L, int slice_batch, int planes, bool beside
     const GemmShape s = gemm_shape(L, slice_batch, planes);
     if (planes == 1) return gemm_tiles_f16(s, L.batch, beside);
     const TilePlan p = L.group_size ? plan_launch(s, L.group_size, L.batch) : plan_tiles(s.tokens, s.row_blocks * s.slices, L.batch, false);
-    return {s.rows, p.tokens, s.slices, p.blocks, p.whole, p.width, 0, p.whole % ((L.batch + p.tokens - 1) / p.tokens) > 0};
+    return {s.rows, p.tokens, s.slices, p.blocks, p.whole, p.width, s.last, p.whole % ((L.batch + p.tokens - 1) / p.tokens) > 0};
 }
 
 int gemm_launch(Q4Launch &L, const XhList &xh, const float *ss, float *ws, size_t ws_floats, int planes, int slice_batch,

@@ -236,16 +236,17 @@ int group_tiles_launch(const float *scales, const int32_t *qzeros, int out, int 
 struct XhList {
     const void *p[3]; // activations per matrix of the launch
 };
-// How a launch is cut.  The results depend on `slices` alone, and that on slice_batch, the number of columns the
-// caller's chunk has: a pass over several chunks then gives what the chunks one by one would have given.
+// How a launch is cut.  The results depend on `slices` and `last` alone, and these on slice_batch, the number of columns the
+// caller's chunk has: a pass over several chunks then gives what the chunks one by one would have given.  last (fp32 weights): the
+// K steps of 64 inputs of the last slice, which is shorter than the others; 0, and all are equal.
 struct GemmShape {
-    int rows, tokens, row_blocks, slices;
+    int rows, tokens, row_blocks, slices, last;
 };
 GemmShape gemm_shape(const Q4Launch &L, int slice_batch, int planes);
 GemmShape gemm_shape_f16(const Q4Launch &L, int slice_batch);
 // The tiles that a launch of this shape takes, for tests: rows and tokens of a block, slices of K, blocks, how many of them take whole
 // tiles, the width of the tiles of what whole rounds leave over, the tokens behind the whole tiles of a row block where they have a
-// narrower one of their own (fp16), whether a row block has whole tiles and others.
+// narrower one of their own (fp16; with fp32 weights GemmShape's `last`), whether a row block has whole tiles and others.
 struct GemmTiles {
     int rows, tokens, slices, blocks, whole, width, last, both;
 };
