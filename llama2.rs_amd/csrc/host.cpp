@@ -1488,7 +1488,7 @@ extern "C" int l2_model_qmatvec(l2_model *m, int layer, int proj, const float *x
             L2_TRY(gemm_launch(L, XhList{{m->op_batch.planes, nullptr, nullptr}}, nullptr, m->op_batch.ws, m->op_batch.ws_floats, 3, B, st));
         } else {
             DenseArgs a{};
-            a.y = m->op_y, a.w = q.dense, a.x = m->op_x, a.in = q.in, a.out = q.out, a.batch = B;
+            a.m[0] = {q.dense, m->op_y, q.out}, a.n_mats = 1, a.x = m->op_x, a.in = q.in, a.batch = B;
             L2_TRY(dense_launch(a, st));
         }
         L2_HIP(hipMemcpyAsync(y_host, m->op_y, (size_t)B * q.out * 4, hipMemcpyDeviceToHost, st));
@@ -1901,18 +1901,21 @@ static int forward_enqueue_dense(l2_model *m, l2_state *s, int B, int max_pos, c
         ScatterTargets t{};
         LAUNCH(K_EMBED, embed_launch(m->x, m->tok_emb, in.src, dim, B, t, in.amax, st));
     }
-    auto dense = [&](const DevQLinear &w, const float *x, const float *wn, float *y, const float *res,
-                     const float *gate) {
+    auto dense = [&](const DevQLinear &w, const float *x, float *y, const float *res) {
         DenseArgs a{};
-        a.y = y, a.w = w.dense, a.x = x, a.wn = wn, a.eps = m->rms_eps, a.in = w.in, a.out = w.out, a.batch = B;
-        a.res = res, a.gate = gate;
+        a.m[0] = {w.dense, y, w.out}, a.n_mats = 1, a.x = x, a.in = w.in, a.batch = B, a.res = res;
+        return dense_launch(a, st);
+    };
+    auto normed = [&](std::initializer_list<DenseMat> mats, const float *wn, bool gated) {
+        DenseArgs a{};
+        for (const DenseMat &w : mats) a.m[a.n_mats++] = w;
+        a.x = m->x, a.wn = wn, a.eps = m->rms_eps, a.in = dim, a.batch = B, a.gated = gated;
         return dense_launch(a, st);
     };
     for (int l = 0; l < L; l++) {
         const float *att_n = m->rms_att + (size_t)l * dim, *ffn_n = m->rms_ffn + (size_t)l * dim;
-        LAUNCH(K_Q4_QKV, dense(m->q[L2_WQ][l], m->x, att_n, m->qv, nullptr, nullptr)); // :217-226
-        L2_TRY(dense(m->q[L2_WK][l], m->x, att_n, m->kv, nullptr, nullptr));
-        L2_TRY(dense(m->q[L2_WV][l], m->x, att_n, m->vv, nullptr, nullptr));
+        const float *const wq = m->q[L2_WQ][l].dense, *const wk = m->q[L2_WK][l].dense, *const wv = m->q[L2_WV][l].dense;
+        LAUNCH(K_Q4_QKV, normed({{wq, m->qv, dim}, {wk, m->kv, kvd}, {wv, m->vv, kvd}}, att_n, false)); // :217-226
         float *kc = s->kcache + (size_t)l * m->max_seq * kvd;
         float *vc = s->vcache + (size_t)l * m->max_seq * kvd;
         if (B == 1) {
@@ -1936,11 +1939,9 @@ static int forward_enqueue_dense(l2_model *m, l2_state *s, int B, int max_pos, c
             LAUNCH(K_ATTENTION, attention_launch(m->attg, 0, m->qv, kc, vc, in.dpos, nullptr, d.n_heads,
                                                  d.n_kv_heads, m->head_size, max_pos, B, st));
         }
-        LAUNCH(K_Q4_WO, dense(m->q[L2_WO][l], m->attg, nullptr, m->x, m->x, nullptr));       // :260-264
-        LAUNCH(K_Q4_W13, dense(m->q[L2_W1][l], m->x, ffn_n, m->hd, nullptr, nullptr));        // :266-271
-        L2_TRY(dense(m->q[L2_W3][l], m->x, ffn_n, m->hg, nullptr, m->hd));                    // :272-276
-        LAUNCH(K_Q4_W2, dense(m->q[L2_W2][l], m->hg, nullptr, m->x, m->x, nullptr));          // :279-285
-        (void)hid;
+        LAUNCH(K_Q4_WO, dense(m->q[L2_WO][l], m->attg, m->x, m->x));                                                        // :260-264
+        LAUNCH(K_Q4_W13, normed({{m->q[L2_W1][l].dense, m->hd, hid}, {m->q[L2_W3][l].dense, m->hg, hid}}, ffn_n, true)); // :266-276
+        LAUNCH(K_Q4_W2, dense(m->q[L2_W2][l], m->hg, m->x, m->x));                                                          // :279-285
     }
     if (in.logits)
         LAUNCH(K_CLASSIFIER, dense_matvec_launch(in.logits, m->wcls, m->x, m->rms_final, m->rms_eps, dim,

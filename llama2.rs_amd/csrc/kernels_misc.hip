@@ -161,38 +161,56 @@ __device__ __forceinline__ unsigned long long amax_key(float v, int idx) {
 // the end re-read the row's last 16 bytes against a zero of x, rows past the
 // end re-read the last row.  Inputs longer than 32 * 64 float4 take several
 // such passes over a row (R = 1) into the same accumulator.
+//
+// kRowsOf: q, k and v in one launch, their rows one behind the other.  kGate: w1 and w3 in one launch, the rows of a tile one of w1 and
+// one of w3 in turn, so that the gate needs nothing that another wave has.  A launch of 67 MB spends some 3 us of 14 before its first and
+// behind its last bytes: a token behind two layers of 7B's widths and a prompt of 99, with that prompt, 1251 -> 1183 us.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-template <int KI, int R> // float4 per lane, row and pass; rows
+enum { kOneMat, kRowsOf, kGate };
+template <int KI, int R, int MATS = kOneMat> // float4 per lane, row and pass; rows
 __global__ __launch_bounds__(256) void dense_matvec_kernel(const DenseArgs A) {
     extern __shared__ float xs[]; // n_pass * KI * 64 float4, zero beyond in
     __shared__ float red[16];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6); // uniform: row addresses stay scalar
-    const int in = A.in, out = A.out;
+    const int in = A.in, out = A.rows;
     const int n4 = in >> 2;
     const int n_pass = A.n_pass;
     const int padded = n_pass * KI * 64;
     const size_t bcol = blockIdx.y;
     const float *__restrict__ x = A.x + bcol * in;
     const float *__restrict__ wn = A.wn;
-    const float4 *__restrict__ w4 = reinterpret_cast<const float4 *>(A.w);
     const float4 *__restrict__ xs4 = reinterpret_cast<const float4 *>(xs);
 
     const int waves_total = gridDim.x * 4;
     const int o_first = (blockIdx.x * 4 + wave) * R;
     float4 wv[R][KI];
+    // Row o of the launch: its matrix, and its row there.
+    auto mat_of = [&](int &o) __attribute__((always_inline)) {
+        int mi = 0;
+        if constexpr (MATS == kGate) {
+            mi = o & 1, o >>= 1;
+        } else if constexpr (MATS == kRowsOf) {
+            const int o1 = o - A.m[0].out, o2 = o1 - A.m[1].out;
+            mi = o1 < 0 ? 0 : o2 < 0 ? 1 : 2;
+            o = o1 < 0 ? o : o2 < 0 ? o1 : o2;
+        }
+        return mi;
+    };
     auto load_tile = [&](int o, int pass) {
 #pragma unroll
         for (int k = 0; k < R; k++) {
-            // 32-bit byte offsets from the one base (the launcher checks that the matrix stays below 4 GiB)
-            const uint32_t row = (uint32_t)min(o + k, out - 1) * ((uint32_t)n4 << 4);
+            // 32-bit byte offsets from the matrix (the launcher checks that it stays below 4 GiB)
+            int in_mat = min(o + k, out - 1);
+            const int mi = mat_of(in_mat);
+            const char *__restrict__ const w = reinterpret_cast<const char *>(mi == 0 ? A.m[0].w : mi == 1 ? A.m[1].w : A.m[2].w);
+            const uint32_t row = (uint32_t)in_mat * ((uint32_t)n4 << 4);
 #pragma unroll
             for (int i = 0; i < KI; i++) {
                 const uint32_t col = (uint32_t)min((pass * KI + i) * 64 + lane, n4 - 1) << 4;
                 // read once per token: non-temporal, so that the rows do not displace what is re-read
-                wv[k][i] = __builtin_bit_cast(float4, __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(
-                                                          reinterpret_cast<const char *>(w4) + (row + col))));
+                wv[k][i] = __builtin_bit_cast(float4, __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(w + (row + col))));
             }
         }
     };
@@ -229,7 +247,7 @@ __global__ __launch_bounds__(256) void dense_matvec_kernel(const DenseArgs A) {
     __syncthreads();
 
     unsigned long long key = 0ull;
-    float *__restrict__ y = A.y + bcol * out;
+    float *__restrict__ y = A.m[0].y + bcol * out;
     const float *__restrict__ res = A.res ? A.res + bcol * out : nullptr;
     const float *__restrict__ gate = A.gate ? A.gate + bcol * out : nullptr;
     for (int o = o_first; o < out; o += waves_total * R) {
@@ -263,7 +281,20 @@ __global__ __launch_bounds__(256) void dense_matvec_kernel(const DenseArgs A) {
 #pragma unroll
         for (int k = 0; k < R; k++) {
             float v = wave_sum(a[k]) * ss;
-            if (lane == 0 && o + k < out) {
+            if constexpr (MATS == kGate) {
+                static_assert(R % 2 == 0 || MATS != kGate, "w1 and w3 in turn");
+                a[k] = v;
+                if (k % 2 && lane == 0 && o + k < out) {
+                    const float g = a[k - (k % 2)];
+                    A.m[1].y[bcol * (out >> 1) + ((o + k) >> 1)] = (g * (1.0f / (1.0f + expf(-g)))) * v;
+                }
+            } else if constexpr (MATS == kRowsOf) {
+                int in_mat = o + k;
+                const int mi = mat_of(in_mat);
+                float *const to = mi == 0 ? A.m[0].y : mi == 1 ? A.m[1].y : A.m[2].y;
+                const int n = mi == 0 ? A.m[0].out : mi == 1 ? A.m[1].out : A.m[2].out;
+                if (lane == 0 && o + k < out) to[bcol * n + in_mat] = v;
+            } else if (lane == 0 && o + k < out) {
                 if (gate) v = (gv[k] * (1.0f / (1.0f + expf(-gv[k])))) * v;
                 if (res) v = rv[k] + v;
                 y[o + k] = v;
@@ -409,42 +440,62 @@ int rope_kv_launch(float *q, const float *k, const float *v, const int32_t *pos,
     return L2_OK;
 }
 
+template <int KI, int R>
+static auto dense_form(const DenseArgs &a) -> void (*)(DenseArgs) {
+    if constexpr (R % 2 == 0)
+        if (a.gated) return dense_matvec_kernel<KI, R, kGate>;
+    return a.n_mats > 1 ? dense_matvec_kernel<KI, R, kRowsOf> : dense_matvec_kernel<KI, R>;
+}
+
 int dense_launch(const DenseArgs &a0, hipStream_t st) {
     DenseArgs a = a0;
-    if (a.in < 4 || a.in % 4 || a.in > 32768 || a.out < 1 || a.batch < 1 ||
-        (size_t)a.in * a.out * 4 >= ((size_t)1 << 32))
-        return l2_fail(L2_ERR_ARG, "dense matvec: in=%d out=%d batch=%d", a.in, a.out, a.batch);
+    if (a.n_mats < 1 || a.n_mats > 3 || (a.n_mats > 1 && (a.amax || a.res || a.gate)) || (a.gated && (a.n_mats != 2 || a.m[0].out != a.m[1].out)))
+        return l2_fail(L2_ERR_ARG, "dense matvec: %d matrices", a.n_mats);
+    a.rows = 0;
+    for (int i = 0; i < a.n_mats; i++) {
+        if (a.in < 4 || a.in % 4 || a.in > 32768 || a.m[i].out < 1 || a.batch < 1 || (size_t)a.in * a.m[i].out * 4 >= ((size_t)1 << 32))
+            return l2_fail(L2_ERR_ARG, "dense matvec: in=%d out=%d batch=%d", a.in, a.m[i].out, a.batch);
+        a.rows += a.m[i].out;
+    }
     if (a.amax && a.batch != 1) return l2_fail(L2_ERR_ARG, "dense matvec: the running maximum takes one column");
     const int ki = (a.in / 4 + 63) / 64; // float4 per lane and row
     const int KI = ki <= 4 ? 4 : ki <= 8 ? 8 : ki <= 16 ? 16 : ki <= 20 ? 20 : 32;
     int R = 32 / KI >= 1 ? 32 / KI : 1;
     // One column of few rows: fewer rows per wave where whole tiles would leave compute units without a block
     // (2000 rows of 1024: 63 blocks 9.9 us, 250 blocks 6.6).
-    const bool few = KI <= 16 && a.batch == 1 && (a.out + 4 * R - 1) / (4 * R) < cu_count();
+    const bool few = KI <= 16 && a.batch == 1 && (a.rows + 4 * R - 1) / (4 * R) < cu_count();
     if (few) R = KI == 4 ? 2 : 1;
+    if (a.gated && R % 2) { // a wave has one row: w1, then w3 with the gate in front
+        DenseArgs b = a0;
+        b.gated = false, b.n_mats = 1;
+        L2_TRY(dense_launch(b, st));
+        b.m[0] = a0.m[1], b.gate = a0.m[0].y;
+        return dense_launch(b, st);
+    }
     a.n_pass = (ki + KI - 1) / KI;
     // One column (the classifier of a decode step): one block per CU -- 7B 93 -> 85 us, 13B 112 -> 103, 70B 172 ->
     // 161 (7B now 81.5) against three per CU, which the registers would allow and which stays the rule for several columns.
     // Fewer when the rows run out.
     const int per_cu = a.batch == 1 ? 1 : 3;
     int blocks = (per_cu * cu_count() + a.batch - 1) / a.batch;
-    const int need = (a.out + 4 * R - 1) / (4 * R);
+    const int need = (a.rows + 4 * R - 1) / (4 * R);
     if (blocks > need) blocks = need;
     const size_t lds = (size_t)a.n_pass * KI * 64 * 16;
     dim3 grid(blocks, a.batch), block(256);
-    if (lds > 48 * 1024) { // only rows of more than one pass, which run with KI = 32
-        if (KI != 32) return l2_fail(L2_ERR_ARG, "dense matvec: in=%d out=%d needs %zu B of LDS with %d loads per pass", a.in, a.out, lds, KI);
-        static LdsLimit limit;
-        L2_TRY(limit.ensure(reinterpret_cast<const void *>(dense_matvec_kernel<32, 1>), lds));
-    }
-    auto launch = [&](void (*kernel)(DenseArgs)) { l2_launch(kernel, grid, block, lds, st, a); };
+    void (*kernel)(DenseArgs) = nullptr;
     switch (KI) {
-        case 4: launch(few ? dense_matvec_kernel<4, 2> : dense_matvec_kernel<4, 8>); break;
-        case 8: launch(few ? dense_matvec_kernel<8, 1> : dense_matvec_kernel<8, 4>); break;
-        case 16: launch(few ? dense_matvec_kernel<16, 1> : dense_matvec_kernel<16, 2>); break;
-        case 20: launch(dense_matvec_kernel<20, 1>); break;
-        default: launch(dense_matvec_kernel<32, 1>); break;
+        case 4: kernel = few ? dense_form<4, 2>(a) : dense_form<4, 8>(a); break;
+        case 8: kernel = few ? dense_form<8, 1>(a) : dense_form<8, 4>(a); break;
+        case 16: kernel = few ? dense_form<16, 1>(a) : dense_form<16, 2>(a); break;
+        case 20: kernel = dense_form<20, 1>(a); break;
+        default: kernel = dense_form<32, 1>(a); break;
     }
+    if (lds > 48 * 1024) { // only rows of more than one pass, which run with KI = 32
+        if (KI != 32) return l2_fail(L2_ERR_ARG, "dense matvec: in=%d needs %zu B of LDS with %d loads per pass", a.in, lds, KI);
+        static LdsLimit limit[2];
+        L2_TRY(limit[a.n_mats > 1].ensure(reinterpret_cast<const void *>(kernel), lds));
+    }
+    l2_launch(kernel, grid, block, lds, st, a);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }
@@ -452,7 +503,7 @@ int dense_launch(const DenseArgs &a0, hipStream_t st) {
 int dense_matvec_launch(float *y, const float *w, const float *x, const float *wn, float eps, int in, int out,
                         unsigned long long *amax_key, hipStream_t st) {
     DenseArgs a{};
-    a.y = y, a.w = w, a.x = x, a.wn = wn, a.eps = eps, a.in = in, a.out = out, a.amax = amax_key, a.batch = 1;
+    a.m[0] = {w, y, out}, a.n_mats = 1, a.x = x, a.wn = wn, a.eps = eps, a.in = in, a.amax = amax_key, a.batch = 1;
     return dense_launch(a, st);
 }
 

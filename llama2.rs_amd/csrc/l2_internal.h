@@ -444,17 +444,23 @@ int token_layers_launch(const TokArgs &a, int grid, size_t lds, bool eight, hipS
 int dense_matvec_launch(float *y, const float *w, const float *x, const float *wn, float eps, int in, int out,
                         unsigned long long *amax_key, hipStream_t st);
 // The general form: y[b] = epilogue(w (rmsnorm?)(x[b])) for `batch` columns (see dense_matvec_kernel).
+struct DenseMat {
+    const float *w; // [out][in]
+    float *y;       // [batch][out]
+    int out;
+};
 struct DenseArgs {
-    float *y;            // [batch][out]
-    const float *w;      // [out][in]
+    DenseMat m[3];
+    int n_mats;          // 1..3, one behind the other
+    bool gated;          // of two with as many rows: m[1].y = silu(m[0] x) * (m[1] x), and m[0].y is scratch of the same size
     const float *x;      // [batch][in]
     const float *wn;     // [in] or null: rmsnorm weight applied to x, with eps
     float eps;
-    int in, out, batch;
-    unsigned long long *amax; // null, or the running (value, index) maximum (batch == 1)
-    const float *res;    // null, or [batch][out] added to the result (may alias y)
-    const float *gate;   // null, or [batch][out]: result = silu(gate) * result
-    int n_pass;          // set by the launcher
+    int in, batch;
+    unsigned long long *amax; // null, or the running (value, index) maximum (one matrix, batch == 1)
+    const float *res;    // null, or [batch][out] added to the result (may alias y; one matrix)
+    const float *gate;   // null, or [batch][out]: result = silu(gate) * result (one matrix)
+    int n_pass, rows;    // set by the launcher: the matrices' rows
 };
 int dense_launch(const DenseArgs &a, hipStream_t st);
 // pos = dpos[0]; next = pos < n_prompt ? prompt[pos] : index(amax_key);

@@ -79,3 +79,26 @@ def test_short_slice_by_chunks():
         kv.append(m.forward([5], [150]))
         m.close()
     np.testing.assert_array_equal(kv[0], kv[1])
+
+
+# q|k|v in one launch and w1|w3 in one with the gate: each number of loads per lane, with as many rows per wave as it has and with fewer
+# (then w1 and w3 are two launches where that is one), rows that do not fill the last wave; one column and three
+@pytest.mark.gpu
+@pytest.mark.parametrize("dim,hidden", [(1024, 96), (1024, 4128), (2048, 1056), (2048, 2080), (4096, 96), (4096, 1056), (5120, 96)])
+def test_projections_in_one_launch(oracle, dim, hidden):
+    from llama2_rs import ops
+    dims = ck.Dims(dim=dim, hidden_dim=hidden, n_layers=1, n_heads=dim // 128, n_kv_heads=dim // 1024, vocab_size=72, seq_len=32,
+                   group_size=0)
+    img = ck.synth_weights_image(dims, seed=5)
+    m, o = ops.Model(img, dims), oracle.Model(img, dims)
+    o.new_state()
+    for pos, t in enumerate((1, 60)):
+        want, got = o.transformer([t], [pos]), m.forward([t], [pos])
+        assert nrel(got, want) < 1e-4, pos
+    m.forward([7, 8, 9], [2, 3, 4])
+    o.transformer([7, 8, 9], [2, 3, 4])
+    for a, b in zip(m.read_kv(0, 0, 5), o.kv_cache()):
+        assert nrel(a, b[0, :5]) < 1e-4
+    assert nrel(m.forward([3], [5]), o.transformer([3], [5])) < 1e-4
+    m.close()
+    o.close()
