@@ -69,7 +69,7 @@ def token_bytes(d, pos: int) -> int:
     return d.n_layers * per_layer + cb["classifier"] + d.dim * 4 + d.dim * 4 + kv
 
 
-Q4_SOURCES = ["kernels_q4.hip", "kernels_q4_stream.hip", "q4_common.h", "lanes.h"]
+Q4_SOURCES = ["kernels_q4.hip", "kernels_q4_stream.hip", "kernels_token.hip", "q4_common.h", "lanes.h"]
 
 
 def q4_sources_digest() -> str:
@@ -122,6 +122,17 @@ def measured_traffic(model: str, kernels: dict):
                 return None, f"{note} holds no {section} reading for {name} ({cls}): take it again"
             total += table[section][name]
     return round(total / len(Q4_CLASSES)), note
+
+
+def token_traffic(model: str):
+    """The same for the launch that takes all layers of a step: (bytes or None, note)."""
+    table, note = counter_summary(f"q4_matvec_{model}_decode_hbm_counters.txt")
+    if table is None:
+        return None, note
+    read, written = ([v for k, v in table[s].items() if k.startswith("token_layers_kernel")] for s in ("FETCH_SIZE", "WRITE_SIZE"))
+    if len(read) != 1 or len(written) != 1:
+        return None, f"{note} holds no reading for token_layers_kernel: take it again"
+    return read[0] + written[0], note
 
 
 def matvec_run(np, ops, n_inst: int, iters: int, reps: int, cpu: bool) -> dict:
@@ -209,7 +220,7 @@ class Loaded:
         d = ops.preset(name, group or (64 if name == "70B" else 128))
         if layers:
             d = ck.Dims(d.dim, d.hidden_dim, layers, d.n_heads, d.n_kv_heads, d.vocab_size, d.seq_len, d.group_size)
-        self.d = d
+        self.d, self.all_layers = d, not layers
         self.max_seq = max(d.seq_len, max_seq)
         t0 = time.time()
         self.img = ops.synth_image(d, seed)
@@ -227,7 +238,7 @@ class Loaded:
 
 def decode_run(np, M: Loaded, W: int, K: int, pos0: int, cpu: bool, cpu_tokens: int) -> dict:
     """W prompt positions forced through the B=1 loop (untimed), then K greedy steps timed; the q4 roofline from
-    per-dispatch events of further steps; optionally the CPU restatement on a bounded sample of the same run."""
+    those steps' events where all layers are one launch, else from per-dispatch events of further steps; optionally the CPU restatement on a bounded sample of the same run."""
     m, d = M.m, M.d
     rng = np.random.default_rng(M.seed)
     prompt = rng.integers(0, d.vocab_size, size=W).astype(np.int32)
@@ -238,9 +249,11 @@ def decode_run(np, M: Loaded, W: int, K: int, pos0: int, cpu: bool, cpu_tokens: 
     for i in range(W):
         m.decode_greedy(tok, pos0 + i)
         tok = int(prompt[i])
+    in_one = m.token_steps()
     t0 = time.perf_counter()
     ids, ms_events = m.decode_bench(tok, pos0 + W, K)
     wall_ms = (time.perf_counter() - t0) * 1e3
+    in_one = m.token_steps() - in_one  # timed steps whose layers were one launch
     tok_s = K / (wall_ms * 1e-3)
 
     n_prof = min(8, K)
@@ -267,6 +280,18 @@ def decode_run(np, M: Loaded, W: int, K: int, pos0: int, cpu: bool, cpu_tokens: 
                     "kernel": "q4 matvec: the four q4 launches of a layer (q|k|v, wo, w1|w3, w2), durations from "
                               "the dispatches' own start/stop events",
                     "per_launch": kern}
+    if roofline and in_one >= K and "classifier" in kern:
+        # The timed steps' layers were one launch: its time is the step's without the classifier's launch.  The layers' own launches
+        # (what the class times are of) stand beside it.
+        us = ms_events / K * 1e3 - kern["classifier"]["us"]
+        bytes_ = sum(cb[c] for c in Q4_CLASSES) * d.n_layers
+        traffic, note = token_traffic(M.name) if M.all_layers else (None, "the counter summary is of all layers")
+        roofline = {"bound": "hbm", "achieved": round(bytes_ / us / 1e3, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                    "frac": round(bytes_ / us / 1e3 / HBM_PEAK_GBS, 4), "traffic": traffic, "traffic_source": note,
+                    "algorithmic_bytes_per_launch": bytes_, "us_per_launch": round(us, 1),
+                    "kernel": "token_layers_kernel: all layers of a step in one launch, with attention and the exchanges between its phases; "
+                              "the timed step's events without the classifier's launch; bytes are the q4 weights, scales and zero points",
+                    "layers_own_launches": roofline}
     mid = pos0 + W + K // 2
     out = {
         "workload": (f"{M.label}; batch-1 greedy decode of {K} tokens after a {W}-token random prompt"

@@ -100,6 +100,8 @@ int l2_gemm_plan(int in, const int32_t *out, int n_mats, int group_size, int bat
 int l2_model_set_token_kernel(l2_model *m, int on, int missing, int looks);
 /* Whether steps may take the token kernel (no more after three calls whose waits were given up), and how many calls had such waits. */
 int l2_model_token_kernel(const l2_model *m, int *on, int *gave_up);
+/* How many steps have been launched through it so far. */
+int l2_model_token_steps(const l2_model *m, uint64_t *steps);
 
 /* How the token kernel deals the rows of a model of these dimensions over its blocks and waves, without a device: info[4] receives {whether
  * it takes such a model, blocks, waves per block, dynamic LDS bytes}; walks (or null), room for `cap` numbers, receives 16 for every

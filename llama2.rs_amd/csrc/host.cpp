@@ -350,6 +350,7 @@ struct l2_model {
         bool on = false;
         bool skip = false;      // this call's steps are done again with the layers' own launches
         int gave_up = 0;        // calls that had to be
+        uint64_t steps = 0;     // launched so far
         int missing = 0;        // l2_model_set_token_kernel
         TokModel *model = nullptr; // in device memory
         uint16_t *slots = nullptr;
@@ -1800,7 +1801,7 @@ static int forward_enqueue(l2_model *m, l2_state *s, int B, int max_pos, const F
         float *const handed = t.handed + (t.set ? t.set_floats : 0), *const clear = t.handed + (t.set ? 0 : t.set_floats);
         const TokArgs a{t.model, handed, clear, m->tok_emb, in.src, in.amax, m->x, s->kcache, s->vcache, max_pos};
         L2_TRY(token_layers_launch(a, t.grid - t.missing, t.lds, t.eight, st));
-        t.set ^= 1;
+        t.set ^= 1, t.steps++;
         if (in.logits)
             L2_TRY(dense_matvec_launch(in.logits, m->wcls, m->x, m->rms_final, m->rms_eps, dim, d.vocab_size, in.amax, st));
         return L2_OK;
@@ -2792,6 +2793,12 @@ extern "C" int l2_model_set_token_kernel(l2_model *m, int on, int missing, int l
 extern "C" int l2_model_token_kernel(const l2_model *m, int *on, int *gave_up) {
     if (!m || !on || !gave_up) return l2_fail(L2_ERR_ARG, "null argument");
     *on = m->tok.on, *gave_up = m->tok.gave_up;
+    return L2_OK;
+}
+
+extern "C" int l2_model_token_steps(const l2_model *m, uint64_t *steps) {
+    if (!m || !steps) return l2_fail(L2_ERR_ARG, "null argument");
+    *steps = m->tok.steps;
     return L2_OK;
 }
 

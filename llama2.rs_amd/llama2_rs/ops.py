@@ -253,6 +253,12 @@ class Model:
         check(lib().l2_model_q4_kernels(self.h, buf, 1024))
         return dict(item.split("=", 1) for item in buf.value.decode().split(";") if item)
 
+    def token_steps(self) -> int:
+        """Steps that went through one launch for all layers so far."""
+        n = C.c_uint64()
+        check(lib().l2_model_token_steps(self.h, C.byref(n)))
+        return n.value
+
     def read_kv(self, layer: int, pos0: int, npos: int):
         d = self.dims
         k = np.empty((npos, d.n_kv_heads, d.head_size), np.float32)
