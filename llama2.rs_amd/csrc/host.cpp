@@ -555,8 +555,8 @@ static struct HostSlots {
 
 // Device memory that the host writes itself, over the bus (fine-grained; where all of the device's memory is mapped for the host): x of a
 // call on host arrays goes there, and the kernel that needs it reads it on the device.  Before, x went to pinned memory, and a kernel of its
-// own brought it over, or read it from there while it was cut into planes: 4096x4096, one column, 20.3 -> 17.9 us; 13824x5120, 16
-// columns 76.7 -> 67.  The host writes 46 GB/s this way (64 KB 1.7 -> 5.5 us, 885 KB 8.8 -> 19.1), the kernels read the bus at some 32.
+// own brought it over, or read it from there while it was cut into planes: 4096x4096, one column, 19.9 -> 17.7 us; 13824x5120, 16
+// columns 76.6 -> 70.7.  The host writes 46 GB/s this way (64 KB 1.7 -> 5.5 us, 885 KB 8.8 -> 19.1), the kernels read the bus at some 32.
 // At most kKept pieces of a device, for as long as the process runs (memory that others may have cached is not given back to be used as
 // something else); a call that finds none free takes the way through pinned memory.
 static struct HostWindows {

@@ -5,9 +5,12 @@
 // residual stream behind w2.  A dependent launch spends some 3.5 us before its first FMA (the end of the one before it, arguments, x,
 // staging); here a vector is in the other blocks' LDS 1.5 to 2.5 us after the last block has stored its part, and the weights of the
 // next phase are on their way meanwhile.  Whole steps (kernel and classifier), the layers' own launches -> this, at position 30: three layers of 1024
-// inputs 67.7 -> 54.5 us, four of 7B 218.5 -> 211.6, three of 13B 242.6 -> 230.9; 7B's 96 tokens 103.5 -> 95.5 ms, which is more, since the
-// host's launches are not the kernels' length either.  What bounds it: the exchanges, some 2 us each, and inside a phase memory (w1|w3
-// of 7B run at 5.9 TB/s); blocks finish a phase 0.5 to 1.3 us apart, and all wait for the last.
+// inputs 67.7 -> 51.2 us, four of 7B 219.7 -> 206.6, three of 13B 243 -> 227.9; 7B's 96 tokens 103.5 -> 95 ms, which is more, since the
+// host's launches are not the kernels' length either.  What bounds it: a layer of 7B is 30 us, 18.5 of them in the rows of its four
+// phases (w1|w3 at 5.9 TB/s, wo 3 us for 9 MB) and 11.5 between them: the exchanges, attention, and the 0.5 to 1.5 us by which blocks finish
+// apart, all waiting for the last.  Rows that wait less (more of them asked for before x or as soon as it is there, wo's in front of
+// attention's sums) take longer, because x, or q, is then behind them; so do keys and values brought into LDS before q is there:
+// what attention takes behind 300 positions (3 us a layer more than behind 30) is what one compute unit can fetch.
 //
 // The exchange.  A place is "absent" (all ones, which as a float is one of the NaNs) until its value is stored; a consumer loads, at
 // agent scope, until no place of its piece is absent.  The value is its own flag, every place is 4 bytes and stored once, so no order among
