@@ -1214,8 +1214,10 @@ GemmShape gemm_shape(const Q4Launch &L, int slice_batch, int planes) {
         // two thirds of the CUs in whole rows, 50 steps and three times 14 with it.  Two layers, 100 columns, with the logits 1341 -> 1286 us
         // (short slices of 12, 16, 18, 20 steps 1311 / 1316 / 1339 / 1365; four equal ones 1329); q|k|v in 26 + 26 + 12 steps for 32 + 32 another 10
         // (3 x 16 + 16 67 more, five equal ones 11 more).
+        // Not for fewer slices than the equal ones, whose sums are shorter (2048 -> 17248, two for three: an error of 8.1e-8 for 7.8e-8; 4096 -> 22016, two
+        // for one: 9.4e-8 for 9.9e-8, 4096 -> 11008, three for two: 8.8e-8 for 8.9e-8).
         const float per = 4096.0f / L.in;
-        for (int n = 1; n + 1 < kMaxGemmSlices && n * blocks <= 4 * cus; n++) {
+        for (int n = s.slices; n + 1 < kMaxGemmSlices && n * blocks <= 4 * cus; n++) {
             const int rounds = (n * blocks + cus - 1) / cus, idle = rounds * cus - n * blocks;
             if (!idle) continue;
             const int each = (blocks + idle - 1) / idle, last = (int)((n_unit - 2.9f * n * (each - 1)) / (n * each + 1));
