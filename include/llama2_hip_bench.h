@@ -110,6 +110,10 @@ int l2_model_token_steps(const l2_model *m, uint64_t *steps);
  * that is rounded as rows behind a launch's loop are, whether one of these is looped, whether the wave asks for its rows behind
  * attention, 0, 0}. */
 int l2_token_plan(const l2_dims *d, int32_t *walks, size_t cap, int32_t *info);
+/* What the blocks of a launch with `missing` of them left out write, by the same rule as the kernel finds it, without a device: *blocks
+ * receives those that do not leave at once; rows, room for `cap` numbers, receives 4 for every phase, such block and wave: {projection,
+ * the block's first row, its rows, the bytes of LDS that these reach up to}. */
+int l2_token_rows(const l2_dims *d, int missing, int32_t *rows, size_t cap, int32_t *blocks);
 
 /* Plain device-to-device copy of nbytes, iters times: the box's achievable
  * copy bandwidth (bytes moved = 2*nbytes per iteration). */

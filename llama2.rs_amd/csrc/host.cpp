@@ -1675,7 +1675,7 @@ static int token_plan(const l2_dims &d, TokenPlan &t, bool *ok) {
             while (mi + 1 < n_mats && rb >= blocks(mi)) rb -= blocks(mi), mi++;
             const int out = L[p].m[mi].out;
             for (int w = 0; w < kTokenWaves; w++) {
-                TokWalk &k = t.walks[((size_t)p * grid + b) * kTokenWaves + w];
+                TokWalk &k = t.walks[token_walk_at(grid, p, b, w)];
                 const int v = uneven ? w & 7 : w;
                 int s = v / nwk;
                 k.kslice = v % nwk;
@@ -1799,8 +1799,9 @@ static int forward_enqueue(l2_model *m, l2_state *s, int B, int max_pos, const F
     if (whole) {
         l2_model::TokenKernel &t = m->tok;
         float *const handed = t.handed + (t.set ? t.set_floats : 0), *const clear = t.handed + (t.set ? 0 : t.set_floats);
-        const TokArgs a{t.model, handed, clear, m->tok_emb, in.src, in.amax, m->x, s->kcache, s->vcache, max_pos};
-        L2_TRY(token_layers_launch(a, t.grid - t.missing, t.lds, t.eight, st));
+        const TokGrid grid = token_grid(t.grid, t.missing);
+        const TokArgs a{t.model, handed, clear, m->tok_emb, in.src, in.amax, m->x, s->kcache, s->vcache, max_pos, grid.left_out};
+        L2_TRY(token_layers_launch(a, grid.blocks, t.lds, t.eight, st));
         t.set ^= 1, t.steps++;
         if (in.logits)
             L2_TRY(dense_matvec_launch(in.logits, m->wcls, m->x, m->rms_final, m->rms_eps, dim, d.vocab_size, in.amax, st));
@@ -2813,6 +2814,25 @@ extern "C" int l2_token_plan(const l2_dims *d, int32_t *walks, size_t cap, int32
     const size_t n = t.walks.size() * (sizeof(TokWalk) / 4);
     if (cap < n) return l2_fail(L2_ERR_ARG, "room for %zu numbers, %zu needed", cap, n);
     memcpy(walks, t.walks.data(), n * 4);
+    return L2_OK;
+}
+
+extern "C" int l2_token_rows(const l2_dims *d, int missing, int32_t *rows, size_t cap, int32_t *blocks) {
+    if (!d || !rows || !blocks) return l2_fail(L2_ERR_ARG, "null argument");
+    L2_TRY(check_dims(d));
+    TokenPlan t;
+    bool ok = false;
+    L2_TRY(token_plan(*d, t, &ok));
+    if (!ok || missing < 0 || missing >= t.grid) return l2_fail(L2_ERR_ARG, "missing %d of %d blocks", missing, ok ? t.grid : 0);
+    const TokGrid grid = token_grid(t.grid, missing);
+    const int n = *blocks = grid.blocks - grid.left_out;
+    if (cap < (size_t)4 * n * kTokenWaves * 4) return l2_fail(L2_ERR_ARG, "room for %zu numbers", cap);
+    for (int p = 0; p < 4; p++)
+        for (int b = 0; b < n; b++)
+            for (int w = 0; w < kTokenWaves; w++, rows += 4) {
+                const TokWalk &k = t.walks[token_walk_at(grid.blocks, p, b, w)];
+                rows[0] = k.mat, rows[1] = k.r0, rows[2] = k.n, rows[3] = (k.part_row + k.n) * t.phase[p].nwk * 16 + t.part_at * 4;
+            }
     return L2_OK;
 }
 
