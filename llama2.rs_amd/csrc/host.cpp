@@ -4,7 +4,6 @@
 // (src/inference.rs:16-193), driving the HIP kernels.  Nothing here computes on
 // the CPU except the one-time RoPE angle table and the synthetic-image
 // generator.
-#include <emmintrin.h>
 #include <map>
 #include <fcntl.h>
 #include <math.h>
@@ -21,6 +20,7 @@
 #include <numeric>
 #include <thread>
 
+#include "host_window.h"
 #include "l2_internal.h"
 
 // ---------------------------------------------------------------------------
@@ -553,38 +553,47 @@ static struct HostSlots {
     }
 } host_slots;
 
-// Device memory that the host writes itself, over the bus (fine-grained; where all of the device's memory is mapped for the host): x of a
+// Device memory that the host writes itself, over the bus (fine-grained; where all of the device's memory is mapped for the host, and with it
+// the register that says when the writes are there, see window_written): x of a
 // call on host arrays goes there, and the kernel that needs it reads it on the device.  Before, x went to pinned memory, and a kernel of its
-// own brought it over, or read it from there while it was cut into planes: 4096x4096, one column, 19.9 -> 17.7 us; 13824x5120, 16
-// columns 76.6 -> 70.7.  The host writes 46 GB/s this way (64 KB 1.7 -> 5.5 us, 885 KB 8.8 -> 19.1), the kernels read the bus at some 32.
+// own brought it over, or read it from there while it was cut into planes: 4096x4096, one column, 20.4 -> 19.0 us; 13824x5120, 16
+// columns 76.4 -> 72.3.  The host writes 45 GB/s this way (with the flush 16 KB 1.6 us, 64 KB 2.7, 864 KB 20.7), the kernels read the bus at some 32.
 // At most kKept pieces of a device, for as long as the process runs (memory that others may have cached is not given back to be used as
 // something else); a call that finds none free takes the way through pinned memory.
+struct HostWindow {
+    float *x = nullptr;
+    volatile uint32_t *flush = nullptr;
+};
 static struct HostWindows {
     static constexpr int kKept = 4, kMaxDevices = 64;
     std::mutex mu;
     float *idle[kMaxDevices][kKept] = {};
+    volatile uint32_t *flush[kMaxDevices] = {};
     int n_idle[kMaxDevices] = {}, made[kMaxDevices] = {};
 
-    float *take(int device) {
-        if (device < 0 || device >= kMaxDevices) return nullptr;
+    HostWindow take(int device) {
+        if (device < 0 || device >= kMaxDevices) return {};
         std::lock_guard<std::mutex> lock(mu);
-        if (n_idle[device] > 0) return idle[device][--n_idle[device]];
-        if (made[device] >= kKept) return nullptr;
+        if (n_idle[device] > 0) return {idle[device][--n_idle[device]], flush[device]};
+        if (made[device] >= kKept) return {};
         int mapped = 0;
+        uint64_t address = 0; // the attribute is one, and is stored as such
         void *p = nullptr;
         if (hipDeviceGetAttribute(&mapped, hipDeviceAttributeIsLargeBar, device) != hipSuccess || !mapped ||
+            hipDeviceGetAttribute(reinterpret_cast<int *>(&address), hipDeviceAttributeHdpMemFlushCntl, device) != hipSuccess || !address ||
             hipExtMallocWithFlags(&p, HostSlot::kBytes, hipDeviceMallocFinegrained) != hipSuccess) {
             (void)hipGetLastError();
             made[device] = kKept; // not here
-            return nullptr;
+            return {};
         }
+        flush[device] = reinterpret_cast<volatile uint32_t *>((uintptr_t)address);
         made[device]++;
-        return (float *)p;
+        return {(float *)p, flush[device]};
     }
-    void give(int device, float *p) {
-        if (!p) return;
+    void give(int device, const HostWindow &w) {
+        if (!w.x) return;
         std::lock_guard<std::mutex> lock(mu);
-        idle[device][n_idle[device]++] = p;
+        idle[device][n_idle[device]++] = w.x;
     }
 } host_windows;
 
@@ -1365,21 +1374,21 @@ static int matvec_host(const DevQLinear &q, float *dx, float *dxg, float *dy, Op
     // A shorter x that a kernel permutes anyway is as quick through pinned memory (13824 and 28672 inputs, one column: 27.6 and 27.0 us, in
     // device memory 28.3 and 27.3; 13824, three columns 49.7 and 49.5).
     const bool direct = natural || xb >= kWindowBytes;
-    float *const window = direct && hipGetDevice(&device) == hipSuccess ? host_windows.take(device) : nullptr;
-    float *const x = window ? window : slot.x;
+    const HostWindow window = direct && hipGetDevice(&device) == hipSuccess ? host_windows.take(device) : HostWindow{};
+    float *const x = window.x ? window.x : slot.x;
     auto call = [&]() -> int {
         // a long x in two parts: the host brings the second one while the first crosses the bus
         for (int b0 = 0, b1 = B > 1 && xb >= kSplitBytes ? B / 2 : B; b0 < B; b0 = b1, b1 = B) {
             const size_t at = (size_t)b0 * q.in, n = (size_t)(b1 - b0) * q.in;
             memcpy(x + at, x_host + at, n * sizeof(float));
-            if (window) _mm_sfence(); // written through before the launch is
+            if (window.x) window_written(window.flush);
             if (!natural)
                 L2_TRY(host_input_launch(planes ? (char *)bufs.planes + (size_t)b0 * planes * gemm_padded(q.in) * 2 : (char *)(dxg + at),
                                          x + at, q.inv_index, q.in, b1 - b0, planes, st));
-            else if (!window)
+            else if (!window.x)
                 L2_TRY(copy_launch(dx + at, x + at, n, st));
         }
-        if (natural) return q4_one_natural(q, window ? window : dx, dxg, slot.y, B, st);
+        if (natural) return q4_one_natural(q, window.x ? window.x : dx, dxg, slot.y, B, st);
         if (!planes) return q4_one(q, dxg, slot.y, B, st);
         return gemm_operator(q, B, slot.y, planes, bufs.planes, bufs.ws, bufs.ws_floats, st);
     };
