@@ -557,7 +557,7 @@ static struct HostSlots {
 // the register that says when the writes are there, see window_written): x of a
 // call on host arrays goes there, and the kernel that needs it reads it on the device.  Before, x went to pinned memory, and a kernel of its
 // own brought it over, or read it from there while it was cut into planes: 4096x4096, one column, 20.4 -> 19.0 us; 13824x5120, 16
-// columns 76.4 -> 72.3.  The host writes 45 GB/s this way (with the flush 16 KB 1.6 us, 64 KB 2.7, 864 KB 20.7), the kernels read the bus at some 32.
+// columns 76.4 -> 70.2.  The host writes 45 GB/s this way (with the flush 16 KB 1.6 us, 64 KB 2.7, 864 KB 20.7), the kernels read the bus at some 32.
 // At most kKept pieces of a device, for as long as the process runs (memory that others may have cached is not given back to be used as
 // something else); a call that finds none free takes the way through pinned memory.
 struct HostWindow {
@@ -1341,10 +1341,16 @@ static int qlinear_scratch(l2_qlinear *q, int B) {
     return L2_OK;
 }
 
-// From here on x comes in two parts, whose second kernel costs 3 us: 384 KB (24 columns of 4096 inputs) 57.4 us whole, 58.5 by
+// From here on x in pinned memory comes in two parts, whose second kernel costs 3 us: 384 KB (24 columns of 4096 inputs) 57.4 us whole, 58.5 by
 // halves, 512 KB 67.8 and 67.9, 768 KB 91.6 and 89.6, 884 KB (16 of 13824) 82.8 and 78.5; with the matvec that permutes x itself
 // 50.1 and 50.5, 62.3 and 61.2, 85.7 and 83.4 for 24, 32 and 48 of 4096.
-static constexpr size_t kSplitBytes = 512 * 1024, kWindowBytes = 160 * 1024;
+static constexpr size_t kSplitBytes = 512 * 1024;
+// From here on an x that a kernel permutes is written into device memory, in one part.  In device memory, in pinned memory: 13824 inputs, 1, 3,
+// 4, 6, 8, 10, 16 columns (54 to 864 KB) 28.7 and 27.1 us, 49.6 and 47.9, 42.9 and 41.7, 47.8 and 47.2, 52.0 and 53.5, 56.7 and 60.0, 70.3 and 76.0; 4096, 10, 20,
+// 24, 32, 61 columns (160 to 976 KB) 37.4 and 34.9, 48.1 and 48.7, 52.7 and 54.4, 62.5 and 65.8, 97.1 and 102; 8192, 10, 12, 16 columns (320 to 512 KB) 36.3 and
+// 35.8, 38.2 and 38.4, 41.9 and 45.0.  By halves it takes longer (13824, 16 columns 72.5; 4096, 61 columns 100): the host's writes take the time, and
+// each part waits for its own.
+static constexpr size_t kWindowBytes = 384 * 1024;
 
 static int operator_enqueue(const DevQLinear &q, const float *dx, float *dxg, float *y, const OperatorBufs &bufs, int planes,
                             int B, hipStream_t st) {
@@ -1352,10 +1358,10 @@ static int operator_enqueue(const DevQLinear &q, const float *dx, float *dxg, fl
     return gemm_operator_natural(q, dx, B, y, planes, bufs.planes, bufs.ws, bufs.ws_floats, st);
 }
 
-// x (host, natural order) -> gather through g_index -> matvec -> y (host).  Through a slot of pinned memory where x and y
-// fit one: kernels fetch x from there and the last one writes y there.  One 4096x4096 matvec 28-40 -> 19.6 us (pageable
-// copies either way before); against a DMA from the slot and a gather on the device, 16 columns of 13824x5120 89 -> 82 us, 61 of
-// 4096x4096 116 -> 107, one of 28672x1024 32.8 -> 26.8.
+// x (host, natural order) -> gather through g_index -> matvec -> y (host).  Where x and y fit a slot of pinned memory, the last kernel
+// writes y there, and x is in device memory (HostWindows) or in the slot, from where kernels fetch it.  In the slot, one 4096x4096 matvec
+// 28-40 -> 19.6 us (pageable copies either way before); against a DMA from the slot and a gather on the device, 16 columns of 13824x5120
+// 89 -> 82 us, 61 of 4096x4096 116 -> 107, one of 28672x1024 32.8 -> 26.8.
 static int matvec_host(const DevQLinear &q, float *dx, float *dxg, float *dy, OperatorBufs &bufs, int planes,
                        const float *x_host, int B, float *y_host, hipStream_t st) {
     if (planes) L2_TRY(operator_bufs(bufs, q, B, planes, st));
@@ -1371,14 +1377,12 @@ static int matvec_host(const DevQLinear &q, float *dx, float *dxg, float *dy, Op
     L2_TRY(host_slots.take(&slot));
     int device = 0;
     const bool natural = !planes && takes_natural_order(q); // the matvec kernel gathers
-    // A shorter x that a kernel permutes anyway is as quick through pinned memory (13824 and 28672 inputs, one column: 27.6 and 27.0 us, in
-    // device memory 28.3 and 27.3; 13824, three columns 49.7 and 49.5).
     const bool direct = natural || xb >= kWindowBytes;
     const HostWindow window = direct && hipGetDevice(&device) == hipSuccess ? host_windows.take(device) : HostWindow{};
     float *const x = window.x ? window.x : slot.x;
     auto call = [&]() -> int {
-        // a long x in two parts: the host brings the second one while the first crosses the bus
-        for (int b0 = 0, b1 = B > 1 && xb >= kSplitBytes ? B / 2 : B; b0 < B; b0 = b1, b1 = B) {
+        // a long x in pinned memory in two parts: the host brings the second one while the first crosses the bus
+        for (int b0 = 0, b1 = B > 1 && xb >= kSplitBytes && !window.x ? B / 2 : B; b0 < B; b0 = b1, b1 = B) {
             const size_t at = (size_t)b0 * q.in, n = (size_t)(b1 - b0) * q.in;
             memcpy(x + at, x_host + at, n * sizeof(float));
             if (window.x) window_written(window.flush);
