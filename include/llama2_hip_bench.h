@@ -48,6 +48,12 @@ int l2_qlinear_bench(l2_qlinear **qs, int n, int iters, float *ms_total);
  * iters dispatch durations, without the gaps between dispatches. */
 int l2_qlinear_bench_dispatch(l2_qlinear **qs, int n, int iters, float *ms_sum);
 
+/* For tests.  How many calls of this process had x written into device memory by the host (l2_qlinear_matvec and l2_model_qmatvec with
+ * host arrays: one column and up to a few that the matvec kernel permutes itself, and longer batches).  And: q counts as a handle of
+ * `device` from now on, where such calls have x in that device's memory, or, while it is not the calling thread's current device, in pinned memory. */
+int l2_host_windows_taken(uint64_t *n);
+int l2_qlinear_set_device(l2_qlinear *q, int device);
+
 /* The kernel a B=1 matvec of q runs, named as a profiler prints it.  Launches nothing. */
 int l2_qlinear_kernel(l2_qlinear *q, char *out, size_t cap);
 

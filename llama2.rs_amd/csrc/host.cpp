@@ -471,6 +471,7 @@ struct l2_qlinear {
     hipStream_t stream = nullptr;
     float *x = nullptr, *xg = nullptr, *y = nullptr;
     int cap_B = 0;
+    int device = 0; // that was current when the handle was made
     int mode = L2_PREFILL_FP32;
     OperatorBufs batch;
 };
@@ -570,11 +571,15 @@ static struct HostWindows {
     float *idle[kMaxDevices][kKept] = {};
     volatile uint32_t *flush[kMaxDevices] = {};
     int n_idle[kMaxDevices] = {}, made[kMaxDevices] = {};
+    uint64_t taken = 0;
 
+    // One for a handle of `device`, if that is the calling thread's current device too: another device's memory is not for its kernels
+    // (pinned memory is every device's).
     HostWindow take(int device) {
-        if (device < 0 || device >= kMaxDevices) return {};
+        int current = -1;
+        if (device < 0 || device >= kMaxDevices || hipGetDevice(&current) != hipSuccess || current != device) return {};
         std::lock_guard<std::mutex> lock(mu);
-        if (n_idle[device] > 0) return {idle[device][--n_idle[device]], flush[device]};
+        if (n_idle[device] > 0) return taken++, HostWindow{idle[device][--n_idle[device]], flush[device]};
         if (made[device] >= kKept) return {};
         int mapped = 0;
         uint64_t address = 0; // the attribute is one, and is stored as such
@@ -587,7 +592,7 @@ static struct HostWindows {
             return {};
         }
         flush[device] = reinterpret_cast<volatile uint32_t *>((uintptr_t)address);
-        made[device]++;
+        made[device]++, taken++;
         return {(float *)p, flush[device]};
     }
     void give(int device, const HostWindow &w) {
@@ -1290,6 +1295,10 @@ extern "C" int l2_qlinear_create(const int32_t *qweight, const int32_t *qzeros, 
     q->q.out = out;
     q->q.groups = groups;
     q->q.group_size = group_size;
+    if (hipGetDevice(&q->device) != hipSuccess) {
+        l2_qlinear_free(q);
+        return l2_fail(L2_ERR_HIP, "hipGetDevice failed");
+    }
     float *tiles = nullptr;
     int rc = dalloc(&tiles, group_tiles_floats(out, groups));
     q->bufs[5] = tiles;
@@ -1362,7 +1371,7 @@ static int operator_enqueue(const DevQLinear &q, const float *dx, float *dxg, fl
 // writes y there, and x is in device memory (HostWindows) or in the slot, from where kernels fetch it.  In the slot, one 4096x4096 matvec
 // 28-40 -> 19.6 us (pageable copies either way before); against a DMA from the slot and a gather on the device, 16 columns of 13824x5120
 // 89 -> 82 us, 61 of 4096x4096 116 -> 107, one of 28672x1024 32.8 -> 26.8.
-static int matvec_host(const DevQLinear &q, float *dx, float *dxg, float *dy, OperatorBufs &bufs, int planes,
+static int matvec_host(const DevQLinear &q, int device, float *dx, float *dxg, float *dy, OperatorBufs &bufs, int planes,
                        const float *x_host, int B, float *y_host, hipStream_t st) {
     if (planes) L2_TRY(operator_bufs(bufs, q, B, planes, st));
     const size_t xb = (size_t)B * q.in * 4, yb = (size_t)B * q.out * 4;
@@ -1375,10 +1384,9 @@ static int matvec_host(const DevQLinear &q, float *dx, float *dxg, float *dy, Op
     }
     HostSlot slot;
     L2_TRY(host_slots.take(&slot));
-    int device = 0;
     const bool natural = !planes && takes_natural_order(q); // the matvec kernel gathers
     const bool direct = natural || xb >= kWindowBytes;
-    const HostWindow window = direct && hipGetDevice(&device) == hipSuccess ? host_windows.take(device) : HostWindow{};
+    const HostWindow window = direct ? host_windows.take(device) : HostWindow{};
     float *const x = window.x ? window.x : slot.x;
     auto call = [&]() -> int {
         // a long x in pinned memory in two parts: the host brings the second one while the first crosses the bus
@@ -1409,7 +1417,7 @@ extern "C" int l2_qlinear_matvec(l2_qlinear *q, const float *x_host, int B, floa
     if (!q || !x_host || !y_host) return l2_fail(L2_ERR_ARG, "null argument");
     if (B < 1 || B > 4096) return l2_fail(L2_ERR_RANGE, "batch %d (1..4096)", B);
     L2_TRY(qlinear_scratch(q, B));
-    return matvec_host(q->q, q->x, q->xg, q->y, q->batch, operator_planes(q->q, B, q->mode), x_host, B, y_host, q->stream);
+    return matvec_host(q->q, q->device, q->x, q->xg, q->y, q->batch, operator_planes(q->q, B, q->mode), x_host, B, y_host, q->stream);
 }
 
 // ---- the same operator for callers that cannot allocate ---------------------------------------------
@@ -1510,7 +1518,7 @@ extern "C" int l2_model_qmatvec(l2_model *m, int layer, int proj, const float *x
         return L2_OK;
     }
     const int planes = m->prefill_mode == L2_PREFILL_MFMA ? batch_planes(m, B) : operator_planes(q, B, m->prefill_mode);
-    return matvec_host(q, m->op_x, m->op_xg, m->op_y, m->op_batch, planes, x_host, B, y_host, m->stream);
+    return matvec_host(q, m->device, m->op_x, m->op_xg, m->op_y, m->op_batch, planes, x_host, B, y_host, m->stream);
 }
 
 extern "C" int l2_model_classifier(l2_model *m, const float *x_host, float *y_host) {
@@ -2540,6 +2548,19 @@ extern "C" int l2_generate_greedy(l2_model *m, l2_state *s, const int32_t *promp
 
 // ---------------------------------------------------------------------------
 // measurement hooks
+
+extern "C" int l2_qlinear_set_device(l2_qlinear *q, int device) {
+    if (!q || device < 0) return l2_fail(L2_ERR_ARG, "bad argument");
+    q->device = device;
+    return L2_OK;
+}
+
+extern "C" int l2_host_windows_taken(uint64_t *n) {
+    if (!n) return l2_fail(L2_ERR_ARG, "null argument");
+    std::lock_guard<std::mutex> lock(host_windows.mu);
+    *n = host_windows.taken;
+    return L2_OK;
+}
 
 extern "C" int l2_qlinear_bench(l2_qlinear **qs, int n, int iters, float *ms_total) {
     if (!qs || n < 1 || iters < 1 || !ms_total) return l2_fail(L2_ERR_ARG, "bad argument");

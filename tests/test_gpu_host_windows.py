@@ -1,5 +1,6 @@
 """The operator on host arrays, whose x the host writes into device memory: the bits of the operator on device memory, also where more
 calls run at once than there are windows, and with x changing from call to call."""
+import ctypes
 import os
 import sys
 import threading
@@ -8,7 +9,7 @@ import numpy as np
 import pytest
 
 sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "llama2.rs_amd"))
-from llama2_rs import ops  # noqa: E402
+from llama2_rs import _lib, ops  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 
@@ -52,3 +53,28 @@ def test_host_arrays_give_the_bits_of_device_arrays(n_in, n_out, group, batch):
     assert not bad
     for q in ops_:
         q.close()
+
+
+def windows_taken():
+    n = ctypes.c_uint64()
+    _lib.check(_lib.lib().l2_host_windows_taken(ctypes.byref(n)))
+    return n.value
+
+
+def test_windows_are_of_the_handle_s_device():
+    """A handle of another device than the calling thread's current one has its x in pinned memory, which all devices read."""
+    rng = np.random.default_rng(5)
+    for n_in, batch in ((4096, 1), (4096, 2), (8192, 32)):
+        q = operator(rng, n_in, 256, 64)
+        x = rng.standard_normal((batch, n_in)).astype(np.float32)
+        n = windows_taken()
+        want = q.matvec(x)
+        assert windows_taken() == n + 1
+        _lib.check(_lib.lib().l2_qlinear_set_device(q.h, 1))
+        assert np.array_equal(q.matvec(x).view(np.uint32), want.view(np.uint32)) and windows_taken() == n + 1
+        q.close()
+    q = operator(rng, 13824, 256, 128)  # permuted in front, and below the line
+    n = windows_taken()
+    q.matvec(rng.standard_normal((3, 13824)).astype(np.float32))
+    assert windows_taken() == n
+    q.close()
