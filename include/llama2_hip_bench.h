@@ -108,6 +108,8 @@ int l2_model_set_token_kernel(l2_model *m, int on, int missing, int looks);
 int l2_model_token_kernel(const l2_model *m, int *on, int *gave_up);
 /* How many steps have been launched through it so far. */
 int l2_model_token_steps(const l2_model *m, uint64_t *steps);
+/* How many times loops of steps have asked the runtime about the stream so far, which a small model's do every 128 launches or fewer. */
+int l2_model_asked(const l2_model *m, uint64_t *asked);
 
 /* How the token kernel deals the rows of a model of these dimensions over its blocks and waves, without a device: info[4] receives {whether
  * it takes such a model, blocks, waves per block, dynamic LDS bytes}; walks (or null), room for `cap` numbers, receives 16 for every

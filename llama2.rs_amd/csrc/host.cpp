@@ -362,6 +362,7 @@ struct l2_model {
         bool eight = false;
         int *failed = nullptr;
     } tok;
+    uint64_t asked = 0; // times that a loop of steps has asked the runtime about the stream (kAskLaunches)
     int device = 0;
     // per-launch event timing, on only inside l2_decode_profile
     struct ProfRec { int cls; hipEvent_t e0, e1; };
@@ -2423,7 +2424,7 @@ static int step_bucket(const l2_model *m, int pos) {
 // each one's next token being prompt[pos] while that is inside the prompt, else the argmax.
 //
 // Launched: the embedding kernel of a step takes the step before's argmax itself and records it (in pinned host memory),
-// so a step is its layers' launches, one in front and the classifier.  Forced tokens travel as kernel arguments.
+// so a step is its layers' launches, one in front and the classifier, or the token kernel and the classifier.  Forced tokens travel as kernel arguments.
 // As graphs: see step_graph_get.
 static constexpr int kAskLaunches = 128;
 static constexpr double kAskWeights = 5e7; // a layer of 7B has 2e8 and takes 40 us
@@ -2451,15 +2452,22 @@ static int steps_enqueue(l2_model *m, l2_state *s, int32_t first, int pos0, int 
     // 2.1 or 3.2 ms, 4.0 or 4.5 ms in all; 167 steps 14.0 or 14.5).  Asked about in between, the loop takes 4.04 and 14.1 ms in
     // every process.  That pays where a launch is too short to hide the enqueueing (an ask costs the GPU 5 us); not shortly
     // before the end, where the wait would meet it.
-    const int launches = m->tok.on && !m->tok.skip ? 2 : 5 * m->d.n_layers + 2;
-    const int ask_steps = layer_weights(m) < kAskWeights ? std::max(1, kAskLaunches / launches) : n;
+    const bool asks = layer_weights(m) < kAskWeights;
+    int since = 0; // launches since it was asked
     ForwardIn in;
     in.src.token = first, in.logits = m->logits, in.whole = true;
     for (int i = 0; i < n; i++) {
         const int pos = pos0 + i;
         in.amax = m->amax + (i & 1);
+        const uint64_t in_one = m->tok.steps;
         L2_TRY(forward_enqueue(m, s, 1, pos, in));
-        if ((i + 1) % ask_steps == 0 && i + ask_steps < n && hipStreamQuery(m->stream) == hipErrorNotReady) (void)hipGetLastError();
+        // by the route that this step has taken: the next one's may be another
+        const int launches = m->tok.steps != in_one ? 2 : 5 * m->d.n_layers + 2, ask_steps = std::max(1, kAskLaunches / launches);
+        since += launches;
+        if (asks && since >= ask_steps * launches && i + ask_steps < n) {
+            if (hipStreamQuery(m->stream) == hipErrorNotReady) (void)hipGetLastError();
+            since = 0, m->asked++;
+        }
         in.src = TokenSource{};
         if (pos < n_prompt)
             in.src.token = prompt[pos];
@@ -2834,6 +2842,12 @@ extern "C" int l2_model_token_kernel(const l2_model *m, int *on, int *gave_up) {
 extern "C" int l2_model_token_steps(const l2_model *m, uint64_t *steps) {
     if (!m || !steps) return l2_fail(L2_ERR_ARG, "null argument");
     *steps = m->tok.steps;
+    return L2_OK;
+}
+
+extern "C" int l2_model_asked(const l2_model *m, uint64_t *asked) {
+    if (!m || !asked) return l2_fail(L2_ERR_ARG, "null argument");
+    *asked = m->asked;
     return L2_OK;
 }
 

@@ -110,6 +110,22 @@ def test_waits_that_are_given_up():
     m.close()
 
 
+def test_loops_ask_about_the_stream_by_the_launches_that_they_make():
+    """A step is two launches or 17: 64 or 7 of them between two asks, also behind contexts that the token kernel does not take."""
+    def asked(m):
+        n = ctypes.c_uint64()
+        _lib.check(_lib.lib().l2_model_asked(m.h, ctypes.byref(n)))
+        return n.value
+    m = model(1024, 2816, 8, 2, 64, layers=3, max_seq=1400)
+    m.fill_kv_synthetic(0, 1000, seed=1)
+    for on, pos, want, in_one in ((1, 40, 1, 160), (0, 40, 21, 0), (1, 1000, 21, 0), (1, 816, 11, 80)):  # attention takes up to 896 whole
+        token_kernel(m, on)
+        before, steps = asked(m), m.token_steps()
+        m.decode_bench(5, pos, 160)
+        assert (asked(m) - before, m.token_steps() - steps) == (want, in_one), pos
+    m.close()
+
+
 def test_models_on_threads():
     """Two models decode side by side: one of them at a time has token kernels in flight, and both get their own results."""
     ms = [model(1024, 2816, 8, 2, 64, seed=s) for s in (3, 4)]
