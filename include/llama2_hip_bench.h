@@ -101,7 +101,7 @@ int l2_gemm_plan(int in, const int32_t *out, int n_mats, int group_size, int bat
 /* The B = 1 steps of l2_forward, l2_decode_greedy, l2_generate_greedy and l2_generate go through one launch for all layers (the
  * token kernel) where a query head's blocks take the context whole; the results are the bits of the layers' own launches.
  * on = 0: the layers' own launches always (so does the environment variable L2_TOKEN_LAUNCHES, read when a model is built).  For tests:
- * the kernel is launched with `missing` of its blocks left out, so that the others wait in vain, and gives up a wait after `looks` looks (a
+ * the last `missing` of the kernel's blocks have no rows, so that the others wait in vain for what they would hand on, and it gives up a wait after `looks` looks (a
  * multiple of 64 in effect, at most 131072, the default); the call then does its steps again with the layers' own launches. */
 int l2_model_set_token_kernel(l2_model *m, int on, int missing, int looks);
 /* Whether steps may take the token kernel (no more after three calls whose waits were given up), and how many calls had such waits. */
@@ -118,10 +118,9 @@ int l2_model_asked(const l2_model *m, uint64_t *asked);
  * that is rounded as rows behind a launch's loop are, whether one of these is looped, whether the wave asks for its rows behind
  * attention, 0, 0}. */
 int l2_token_plan(const l2_dims *d, int32_t *walks, size_t cap, int32_t *info);
-/* What the blocks of a launch with `missing` of them left out write, by the same rule as the kernel finds it, without a device: *blocks
- * receives those that do not leave at once; rows, room for `cap` numbers, receives 4 for every phase, such block and wave: {projection,
- * the block's first row, its rows, the bytes of LDS that these reach up to}. */
-int l2_token_rows(const l2_dims *d, int missing, int32_t *rows, size_t cap, int32_t *blocks);
+/* What the blocks write when the last `missing` of them are left out (l2_model_set_token_kernel), without a device: rows, room for `cap`
+ * numbers, receives 4 for every phase, block and wave: {steps, the block's first row, its rows, the bytes of LDS that these reach up to}. */
+int l2_token_rows(const l2_dims *d, int missing, int32_t *rows, size_t cap);
 
 /* Plain device-to-device copy of nbytes, iters times: the box's achievable
  * copy bandwidth (bytes moved = 2*nbytes per iteration). */

@@ -1622,6 +1622,17 @@ struct TokenPlan {
     int grid = 0, part_at = 0;  // part_at: TokModel::part_at
     size_t lds = 0;
     bool eight = false;         // slices of a head: eight or four, as many as keep one block per CU
+
+    // The last blocks have no rows, and hand nothing on that others wait for: tests of waits that are given up.  They are launched like the
+    // others, for the kernel reads the table by its grid.
+    void leave_out(int blocks) {
+        for (int p = 0; p < 4; p++)
+            for (int b = grid - blocks; b < grid; b++)
+                for (int w = 0; w < kTokenWaves; w++) {
+                    TokWalk &k = walks[((size_t)p * grid + b) * kTokenWaves + w];
+                    k.steps = k.n = k.part_row = k.late = k.behind_early = 0, k.behind = 0;
+                }
+    }
 };
 // The launches of a layer's four kinds of matvec, for their plans alone.
 static void layer_launches(const l2_dims &d, Q4Launch (&L)[4]) {
@@ -1697,7 +1708,7 @@ static int token_plan(const l2_dims &d, TokenPlan &t, bool *ok) {
             while (mi + 1 < n_mats && rb >= blocks(mi)) rb -= blocks(mi), mi++;
             const int out = L[p].m[mi].out;
             for (int w = 0; w < kTokenWaves; w++) {
-                TokWalk &k = t.walks[token_walk_at(grid, p, b, w)];
+                TokWalk &k = t.walks[((size_t)p * grid + b) * kTokenWaves + w];
                 const int v = uneven ? w & 7 : w;
                 int s = v / nwk;
                 k.kslice = v % nwk;
@@ -1821,9 +1832,8 @@ static int forward_enqueue(l2_model *m, l2_state *s, int B, int max_pos, const F
     if (whole) {
         l2_model::TokenKernel &t = m->tok;
         float *const handed = t.handed + (t.set ? t.set_floats : 0), *const clear = t.handed + (t.set ? 0 : t.set_floats);
-        const TokGrid grid = token_grid(t.grid, t.missing);
-        const TokArgs a{t.model, handed, clear, m->tok_emb, in.src, in.amax, m->x, s->kcache, s->vcache, max_pos, grid.left_out};
-        L2_TRY(token_layers_launch(a, grid.blocks, t.lds, t.eight, st));
+        const TokArgs a{t.model, handed, clear, m->tok_emb, in.src, in.amax, m->x, s->kcache, s->vcache, max_pos};
+        L2_TRY(token_layers_launch(a, t.grid, t.lds, t.eight, st));
         t.set ^= 1, t.steps++;
         if (in.logits)
             L2_TRY(dense_matvec_launch(in.logits, m->wcls, m->x, m->rms_final, m->rms_eps, dim, d.vocab_size, in.amax, st));
@@ -2829,6 +2839,13 @@ extern "C" int l2_model_set_token_kernel(l2_model *m, int on, int missing, int l
     if (missing >= m->tok.grid) return l2_fail(L2_ERR_ARG, "missing %d of %d blocks", missing, m->tok.grid);
     L2_HIP(hipStreamSynchronize(m->stream));
     L2_HIP(hipMemcpy((char *)m->tok.model + offsetof(TokModel, limit), &looks, sizeof looks, hipMemcpyHostToDevice));
+    if (missing != m->tok.missing) {
+        TokenPlan plan;
+        bool ok = false;
+        L2_TRY(token_plan(m->d, plan, &ok));
+        plan.leave_out(missing);
+        L2_HIP(hipMemcpy(m->tok.walks, plan.walks.data(), plan.walks.size() * sizeof(TokWalk), hipMemcpyHostToDevice));
+    }
     m->tok.on = on != 0, m->tok.missing = missing, m->tok.gave_up = 0;
     return L2_OK;
 }
@@ -2865,22 +2882,19 @@ extern "C" int l2_token_plan(const l2_dims *d, int32_t *walks, size_t cap, int32
     return L2_OK;
 }
 
-extern "C" int l2_token_rows(const l2_dims *d, int missing, int32_t *rows, size_t cap, int32_t *blocks) {
-    if (!d || !rows || !blocks) return l2_fail(L2_ERR_ARG, "null argument");
+extern "C" int l2_token_rows(const l2_dims *d, int missing, int32_t *rows, size_t cap) {
+    if (!d || !rows) return l2_fail(L2_ERR_ARG, "null argument");
     L2_TRY(check_dims(d));
     TokenPlan t;
     bool ok = false;
     L2_TRY(token_plan(*d, t, &ok));
     if (!ok || missing < 0 || missing >= t.grid) return l2_fail(L2_ERR_ARG, "missing %d of %d blocks", missing, ok ? t.grid : 0);
-    const TokGrid grid = token_grid(t.grid, missing);
-    const int n = *blocks = grid.blocks - grid.left_out;
-    if (cap < (size_t)4 * n * kTokenWaves * 4) return l2_fail(L2_ERR_ARG, "room for %zu numbers", cap);
-    for (int p = 0; p < 4; p++)
-        for (int b = 0; b < n; b++)
-            for (int w = 0; w < kTokenWaves; w++, rows += 4) {
-                const TokWalk &k = t.walks[token_walk_at(grid.blocks, p, b, w)];
-                rows[0] = k.mat, rows[1] = k.r0, rows[2] = k.n, rows[3] = (k.part_row + k.n) * t.phase[p].nwk * 16 + t.part_at * 4;
-            }
+    if (cap < t.walks.size() * 4) return l2_fail(L2_ERR_ARG, "room for %zu numbers", cap);
+    t.leave_out(missing);
+    for (size_t i = 0; i < t.walks.size(); i++, rows += 4) {
+        const TokWalk &k = t.walks[i];
+        rows[0] = k.steps, rows[1] = k.r0, rows[2] = k.n, rows[3] = (t.part_at + (k.part_row + k.n) * t.phase[i / (t.walks.size() / 4)].nwk * 4) * 4;
+    }
     return L2_OK;
 }
 

@@ -162,7 +162,6 @@ __global__ __launch_bounds__(kThreads) void token_layers_kernel(const TokArgs S)
     __shared__ __align__(16) float comb[8][HS + 4];
     int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    if ((int)blockIdx.x >= (int)gridDim.x - S.left_out) return;
     uint64_t args = (uint64_t)(uintptr_t)S.model;
     ArgsPtr A = (ArgsPtr)(uintptr_t)args;
     const int n_layers = A->n_layers;
@@ -180,7 +179,7 @@ __global__ __launch_bounds__(kThreads) void token_layers_kernel(const TokArgs S)
 
     // What this wave does in a phase.
     const auto walk_of = [&](int ph) __attribute__((always_inline)) {
-        const WalkPtr p = (WalkPtr)(uintptr_t)A->walks + token_walk_at(gridDim.x, ph, blockIdx.x, wave);
+        const WalkPtr p = (WalkPtr)(uintptr_t)A->walks + (ph * gridDim.x + blockIdx.x) * kWaves + wave;
         return TokWalk{p->mat, p->first, p->stride, p->last, p->steps, p->r0, p->n, p->part_row, p->kslice, p->C, p->groups, p->behind, p->behind_early, p->late, {}};
     };
     const auto at_of = [&](const TokWalk &k, int ph) __attribute__((always_inline)) { return lane_at(k, A->phase[ph].gshift, lane); };
@@ -648,11 +647,11 @@ int token_slots_launch(uint16_t *out, const int32_t *inv, size_t n, hipStream_t 
     return L2_OK;
 }
 
-int token_layers_launch(const TokArgs &a, int blocks, size_t lds, bool eight, hipStream_t st) {
+int token_layers_launch(const TokArgs &a, int grid, size_t lds, bool eight, hipStream_t st) {
     const auto kernel = eight ? token_layers_kernel<8> : token_layers_kernel<4>;
     static LdsLimit limit[2];
     L2_TRY(limit[eight].ensure(reinterpret_cast<const void *>(kernel), lds));
-    l2_launch(kernel, dim3(blocks), dim3(kThreads), lds, st, a);
+    l2_launch(kernel, dim3(grid), dim3(kThreads), lds, st, a);
     L2_HIP(hipGetLastError());
     return L2_OK;
 }

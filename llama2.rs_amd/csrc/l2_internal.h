@@ -411,16 +411,6 @@ struct TokWalk {
     int32_t pad[2];
 };
 static_assert(sizeof(TokWalk) == 64, "one scalar load");
-// Where the walk of a wave stands, in a table of `blocks` blocks per phase.
-__host__ __device__ constexpr int token_walk_at(int blocks, int phase, int block, int wave) {
-    return (phase * blocks + block) * kTokenWaves + wave;
-}
-// A launch has all blocks of the plan, for its grid is what the table is read by; the last `left_out` return at once (which is for
-// tests of waits that are given up).
-struct TokGrid {
-    int blocks, left_out;
-};
-constexpr TokGrid token_grid(int planned, int missing) { return {planned, missing}; }
 struct TokModel { // in device memory
     TokPhase phase[4];
     TokMat m[7];               // q, k, v, wo, w1, w3, w2
@@ -446,10 +436,9 @@ struct TokArgs {
     float *x;                  // [dim] the residual stream behind the last layer
     float *kcache, *vcache;    // [layers][max_seq][kv_dim]
     int pos;
-    int left_out;              // TokGrid
 };
 int token_slots_launch(uint16_t *out, const int32_t *inv, size_t n, hipStream_t st);
-int token_layers_launch(const TokArgs &a, int blocks, size_t lds, bool eight, hipStream_t st);
+int token_layers_launch(const TokArgs &a, int grid, size_t lds, bool eight, hipStream_t st);
 // logits = wcls (rmsnorm(x, wn)); folds (value, index) into amax_key when set.
 // wn == nullptr: plain Linear::matvec of x.
 int dense_matvec_launch(float *y, const float *w, const float *x, const float *wn, float eps, int in, int out,

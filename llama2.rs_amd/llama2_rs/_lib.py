@@ -103,7 +103,7 @@ SIGNATURES = {
     "l2_token_plan": (_I, [C.POINTER(Dims), _VP, _SZ, _VP]),
     "l2_host_windows_taken": (_I, [C.POINTER(C.c_uint64)]),
     "l2_qlinear_set_device": (_I, [_VP, _I]),
-    "l2_token_rows": (_I, [C.POINTER(Dims), _I, _VP, _SZ, C.POINTER(_I)]),
+    "l2_token_rows": (_I, [C.POINTER(Dims), _I, _VP, _SZ]),
     "l2_copy_bench": (_I, [_SZ, _I, C.POINTER(C.c_float)]),
 }
 

@@ -88,18 +88,21 @@ def test_models_that_it_does_not_take():
 
 @pytest.mark.parametrize("shape", [(512, 768, 4, 2, 32), (1024, 2816, 8, 2, 64), (2048, 28672, 16, 16, 64), (4096, 11008, 32, 32, 128)])
 def test_a_launch_with_blocks_left_out_stays_within_its_buffers(shape):
-    """The blocks that stay have their own rows in every phase, and no others: nothing is written behind a vector or behind the LDS."""
+    """The kernel reads the plan by its grid, so all blocks are launched: those that stay have their own rows in every phase, the others none,
+    and nothing is written behind a vector or behind the LDS."""
     dim, hid, heads, kv, _ = shape
     d = dims(*shape)
     info, w = plan(d)
     out = np.array([dim, dim // heads * kv, dim // heads * kv, dim, hid, hid, dim])
     for missing in (0, 1, 5, int(info[1]) - 1):
-        rows, blocks = np.zeros(4 * 1024 * 16 * 4, np.int32), ctypes.c_int()
-        _lib.check(_lib.lib().l2_token_rows(ctypes.byref(ops.to_cdims(d)), missing, rows.ctypes.data, rows.size, ctypes.byref(blocks)))
-        assert blocks.value == info[1] - missing
-        r = rows[:4 * blocks.value * 16 * 4].reshape(4, blocks.value, 16, 4)
-        assert (r[..., :3] == w[:, :blocks.value][..., [0, 5, 6]]).all()
+        rows = np.zeros(4 * info[1] * 16 * 4, np.int32)
+        _lib.check(_lib.lib().l2_token_rows(ctypes.byref(ops.to_cdims(d)), missing, rows.ctypes.data, rows.size))
+        r, stay = rows.reshape(4, info[1], 16, 4), info[1] - missing
+        assert (r[:, :stay, :, :3] == w[:, :stay][..., [4, 5, 6]]).all() and (r[:, stay:, :, [0, 2]] == 0).all()
         assert (r[..., 1] >= 0).all() and (r[..., 2] >= 0).all()
-        reach = r[..., 1] + r[..., 2]
-        assert (reach[r[..., 2] > 0] <= out[r[..., 0]][r[..., 2] > 0]).all()
+        reach, here = r[..., 1] + r[..., 2], r[..., 2] > 0
+        assert (reach[here] <= out[w[..., 0]][here]).all()
         assert (r[..., 3] <= info[3]).all()
+    # all blocks of the plan, whatever is left out
+    source = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "llama2.rs_amd", "csrc", "host.cpp")
+    assert re.findall(r"token_layers_launch\(([^)]*)\)", open(source).read()) == ["a, t.grid, t.lds, t.eight, st"]
