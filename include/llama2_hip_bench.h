@@ -104,7 +104,10 @@ int l2_gemm_plan(int in, const int32_t *out, int n_mats, int group_size, int bat
  * the last `missing` of the kernel's blocks have no rows, so that the others wait in vain for what they would hand on, and it gives up a wait after `looks` looks (a
  * multiple of 64 in effect, at most 131072, the default); the call then does its steps again with the layers' own launches. */
 int l2_model_set_token_kernel(l2_model *m, int on, int missing, int looks);
-/* Whether steps may take the token kernel (no more after three calls whose waits were given up), and how many calls had such waits. */
+/* The last two for themselves, without a fresh start, and: the fail_in-th next step that takes the token kernel returns an error behind its
+ * launch (0: none does). */
+int l2_model_token_trouble(l2_model *m, int missing, int looks, int fail_in);
+/* Whether steps may take the token kernel (no more after three such calls in a row whose waits were given up), and how many calls had such waits. */
 int l2_model_token_kernel(const l2_model *m, int *on, int *gave_up);
 /* How many steps have been launched through it so far. */
 int l2_model_token_steps(const l2_model *m, uint64_t *steps);

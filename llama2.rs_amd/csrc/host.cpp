@@ -350,8 +350,9 @@ struct l2_model {
         bool on = false;
         bool skip = false;      // this call's steps are done again with the layers' own launches
         int gave_up = 0;        // calls that had to be
+        int in_a_row = 0;       // the last ones, with no call between whose token kernels came through
         uint64_t steps = 0;     // launched so far
-        int missing = 0;        // l2_model_set_token_kernel
+        int missing = 0, fail_in = 0; // l2_model_token_trouble
         TokModel *model = nullptr; // in device memory
         uint16_t *slots = nullptr;
         TokWalk *walks = nullptr;
@@ -1811,9 +1812,33 @@ static int token_gave_up(l2_model *m, bool *again) {
     L2_TRY(token_kernel_clear(m));
     L2_HIP(hipStreamSynchronize(m->stream));
     *m->hs.gave_up = 0;
-    if (++m->tok.gave_up >= 3) m->tok.on = false;
+    m->tok.gave_up++;
+    // The device is others' to stay, then; a call now and then that had to wait too long does not count for ever.
+    if (++m->tok.in_a_row >= 3) m->tok.on = false;
     *again = true;
     return L2_OK;
+}
+
+// Steps of a call: steps() enqueues them and waits.  Where a token kernel gave up they are done once more, with the layers' own launches.
+// Whatever comes back, nothing of the call is on the stream then and nothing of it is left for the next one.
+template <class F>
+static int token_tries(l2_model *m, F &&steps) {
+    bool again = false;
+    int rc = L2_OK;
+    do {
+        const uint64_t before = m->tok.steps;
+        rc = steps();
+        if (rc != L2_OK) { // some of them may be on their way
+            if (m->tok.steps != before && hipStreamSynchronize(m->stream) == hipSuccess) (void)token_gave_up(m, &again);
+            token_device.left(m);
+            break;
+        }
+        rc = token_gave_up(m, &again);
+        if (rc == L2_OK && !again && m->tok.steps != before) m->tok.in_a_row = 0;
+        m->tok.skip = again;
+    } while (rc == L2_OK && again);
+    m->tok.skip = false;
+    return rc;
 }
 
 static int forward_enqueue(l2_model *m, l2_state *s, int B, int max_pos, const ForwardIn &in) {
@@ -1835,6 +1860,7 @@ static int forward_enqueue(l2_model *m, l2_state *s, int B, int max_pos, const F
         const TokArgs a{t.model, handed, clear, m->tok_emb, in.src, in.amax, m->x, s->kcache, s->vcache, max_pos};
         L2_TRY(token_layers_launch(a, t.grid, t.lds, t.eight, st));
         t.set ^= 1, t.steps++;
+        if (t.fail_in > 0 && --t.fail_in == 0) return l2_fail(L2_ERR_HIP, "a step that a test has fail");
         if (in.logits)
             L2_TRY(dense_matvec_launch(in.logits, m->wcls, m->x, m->rms_final, m->rms_eps, dim, d.vocab_size, in.amax, st));
         return L2_OK;
@@ -2190,12 +2216,10 @@ extern "C" int l2_forward(l2_model *m, l2_state *s, const int32_t *tokens, const
     ForwardIn in;
     in.src.token = tokens[0], in.whole = true;
     in.logits = logits_host ? m->hs.logits : m->logits, in.amax = m->amax;
-    for (bool again = true; again;) {
+    L2_TRY(token_tries(m, [&]() -> int {
         L2_TRY(forward_enqueue(m, s, 1, max_pos, in));
-        L2_TRY(wait_host(m, nullptr, nullptr));
-        L2_TRY(token_gave_up(m, &again));
-        m->tok.skip = again;
-    }
+        return wait_host(m, nullptr, nullptr);
+    }));
     if (logits_host) memcpy(logits_host, m->hs.logits, (size_t)m->d.vocab_size * 4);
     return L2_OK;
 }
@@ -2207,20 +2231,17 @@ int l2_forward_weights(l2_model *m, l2_state *s, int32_t token, int32_t pos, flo
     L2_TRY(ensure_batch(m, 1));
     ForwardIn in;
     in.src.token = token, in.logits = m->logits, in.amax = m->amax, in.whole = true;
-    for (bool again = true; again;) {
+    L2_TRY(token_tries(m, [&]() -> int {
         L2_TRY(forward_enqueue(m, s, 1, pos, in));
         L2_TRY(sample_weights_launch(m->hs.logits, m->hs.redo, m->logits, m->d.vocab_size, temperature, m->amax, m->stream));
-        if (more) { // an event is all that a step inside a call has to wait for (7B: 24 us less than for the stream)
-            if (!m->step_done) L2_HIP(hipEventCreateWithFlags(&m->step_done, hipEventDisableTiming));
-            L2_HIP(hipEventRecord(m->step_done, m->stream));
-            L2_HIP(hipEventSynchronize(m->step_done));
-            token_device.left(m);
-        } else {
-            L2_TRY(wait_host(m, nullptr, nullptr));
-        }
-        L2_TRY(token_gave_up(m, &again));
-        m->tok.skip = again;
-    }
+        if (!more) return wait_host(m, nullptr, nullptr);
+        // an event is all that a step inside a call has to wait for (7B: 24 us less than for the stream)
+        if (!m->step_done) L2_HIP(hipEventCreateWithFlags(&m->step_done, hipEventDisableTiming));
+        L2_HIP(hipEventRecord(m->step_done, m->stream));
+        L2_HIP(hipEventSynchronize(m->step_done));
+        token_device.left(m);
+        return L2_OK;
+    }));
     *out = {m->hs.logits, m->hs.redo};
     return L2_OK;
 }
@@ -2503,13 +2524,10 @@ static int steps_collect(l2_model *m, int pos0, int n, const int32_t *prompt, in
 }
 
 static int steps_run(l2_model *m, l2_state *s, int32_t first, int pos0, int n, const int32_t *prompt, int n_prompt, int32_t *ids) {
-    for (bool again = true; again;) {
+    return token_tries(m, [&]() -> int {
         L2_TRY(steps_enqueue(m, s, first, pos0, n, prompt, n_prompt));
-        L2_TRY(steps_collect(m, pos0, n, prompt, n_prompt, ids));
-        L2_TRY(token_gave_up(m, &again));
-        m->tok.skip = again;
-    }
-    return L2_OK;
+        return steps_collect(m, pos0, n, prompt, n_prompt, ids);
+    });
 }
 
 // Position at which prefill<64>, <32>, ... <2> (src/inference.rs:78-127) leave off for a prompt of n_prompt
@@ -2690,19 +2708,17 @@ extern "C" int l2_decode_bench(l2_model *m, l2_state *s, int32_t token, int32_t 
     L2_HIP(hipEventCreate(&e0));
     L2_HIP(hipEventCreate(&e1));
     L2_HIP(hipStreamSynchronize(m->stream));
-    for (bool again = true; again;) {
+    const int rc = token_tries(m, [&]() -> int {
         L2_HIP(hipEventRecord(e0, m->stream));
         L2_TRY(steps_enqueue(m, s, token, pos, n_tokens, nullptr, 0));
         L2_HIP(hipEventRecord(e1, m->stream));
         L2_HIP(hipEventSynchronize(e1));
         L2_HIP(hipEventElapsedTime(ms_total, e0, e1));
-        L2_TRY(steps_collect(m, pos, n_tokens, nullptr, 0, out_ids));
-        L2_TRY(token_gave_up(m, &again));
-        m->tok.skip = again;
-    }
+        return steps_collect(m, pos, n_tokens, nullptr, 0, out_ids);
+    });
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    return L2_OK;
+    return rc;
 }
 
 // Which kernel each q4 launch class of this model's decode step runs: "class=kernel;..." with the kernel's
@@ -2833,9 +2849,9 @@ extern "C" int l2_gemm_plan(int in, const int32_t *out, int n_mats, int group_si
     return L2_OK;
 }
 
-extern "C" int l2_model_set_token_kernel(l2_model *m, int on, int missing, int looks) {
-    if (!m || missing < 0 || looks < 1 || looks > kTokenLooks) return l2_fail(L2_ERR_ARG, "bad argument");
-    if (!m->tok.model) return on ? l2_fail(L2_ERR_ARG, "this model has no token kernel") : L2_OK;
+extern "C" int l2_model_token_trouble(l2_model *m, int missing, int looks, int fail_in) {
+    if (!m || missing < 0 || looks < 1 || looks > kTokenLooks || fail_in < 0) return l2_fail(L2_ERR_ARG, "bad argument");
+    if (!m->tok.model) return l2_fail(L2_ERR_ARG, "this model has no token kernel");
     if (missing >= m->tok.grid) return l2_fail(L2_ERR_ARG, "missing %d of %d blocks", missing, m->tok.grid);
     L2_HIP(hipStreamSynchronize(m->stream));
     L2_HIP(hipMemcpy((char *)m->tok.model + offsetof(TokModel, limit), &looks, sizeof looks, hipMemcpyHostToDevice));
@@ -2846,7 +2862,15 @@ extern "C" int l2_model_set_token_kernel(l2_model *m, int on, int missing, int l
         plan.leave_out(missing);
         L2_HIP(hipMemcpy(m->tok.walks, plan.walks.data(), plan.walks.size() * sizeof(TokWalk), hipMemcpyHostToDevice));
     }
-    m->tok.on = on != 0, m->tok.missing = missing, m->tok.gave_up = 0;
+    m->tok.missing = missing, m->tok.fail_in = fail_in;
+    return L2_OK;
+}
+
+extern "C" int l2_model_set_token_kernel(l2_model *m, int on, int missing, int looks) {
+    if (!m || missing < 0 || looks < 1 || looks > kTokenLooks) return l2_fail(L2_ERR_ARG, "bad argument");
+    if (!m->tok.model) return on ? l2_fail(L2_ERR_ARG, "this model has no token kernel") : L2_OK;
+    L2_TRY(l2_model_token_trouble(m, missing, looks, 0));
+    m->tok.on = on != 0, m->tok.gave_up = m->tok.in_a_row = 0;
     return L2_OK;
 }
 

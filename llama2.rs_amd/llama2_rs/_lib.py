@@ -99,6 +99,7 @@ SIGNATURES = {
     "l2_model_set_token_kernel": (_I, [_VP, _I, _I, _I]),
     "l2_model_token_kernel": (_I, [_VP, C.POINTER(_I), C.POINTER(_I)]),
     "l2_model_token_steps": (_I, [_VP, C.POINTER(C.c_uint64)]),
+    "l2_model_token_trouble": (_I, [_VP, _I, _I, _I]),
     "l2_model_asked": (_I, [_VP, C.POINTER(C.c_uint64)]),
     "l2_token_plan": (_I, [C.POINTER(Dims), _VP, _SZ, _VP]),
     "l2_host_windows_taken": (_I, [C.POINTER(C.c_uint64)]),

@@ -126,6 +126,41 @@ def test_loops_ask_about_the_stream_by_the_launches_that_they_make():
     m.close()
 
 
+def test_a_call_that_comes_through_ends_the_row_of_those_that_did_not():
+    m = model(1024, 2816, 8, 2, 64)
+    want = m.forward([9], [0]).copy()
+    for gave_up in (0, 2, 4):
+        for missing, calls in ((1, 2), (0, 1)):
+            _lib.check(_lib.lib().l2_model_token_trouble(m.h, missing, 64 if missing else 1 << 17, 0))
+            for _ in range(calls):
+                steps = m.token_steps()
+                m.reset()
+                assert np.array_equal(bits(m.forward([9], [0])), bits(want)) and m.token_steps() == steps + 1
+        assert state_of(m) == (1, gave_up + 2)
+    m.close()
+
+
+def test_an_error_leaves_nothing_behind():
+    """Behind a step that failed: another model gets the device, and the calls that follow, of either, give what they always give."""
+    a, b = (model(1024, 2816, 8, 2, 64, seed=s) for s in (3, 4))
+    prompt = np.array([5, 17, 99], np.int32)
+    want = [m.generate_greedy(prompt, 24)[0] for m in (a, b)]
+    calls = [lambda: a.forward([9], [0]), lambda: a.generate_greedy(prompt, 24), lambda: a.decode_greedy(9, 0), lambda: a.decode_bench(9, 0, 12)]
+    for i, call in enumerate(calls):
+        for missing in (0, 1):  # 1: the step before the one that fails has given up a wait meanwhile
+            _lib.check(_lib.lib().l2_model_token_trouble(a.h, missing, 64, 1 if i in (0, 2) else 2))
+            with pytest.raises(_lib.L2Error):
+                call()
+            _lib.check(_lib.lib().l2_model_token_trouble(a.h, 0, 1 << 17, 0))
+            for m, ids in ((b, want[1]), (a, want[0])):
+                steps = m.token_steps()
+                m.reset()
+                assert np.array_equal(m.generate_greedy(prompt, 24)[0], ids) and m.token_steps() > steps, (i, missing)
+    assert state_of(a)[0] == 1 and state_of(b) == (1, 0)
+    for m in (a, b):
+        m.close()
+
+
 def test_models_on_threads():
     """Two models decode side by side: one of them at a time has token kernels in flight, and both get their own results."""
     ms = [model(1024, 2816, 8, 2, 64, seed=s) for s in (3, 4)]
