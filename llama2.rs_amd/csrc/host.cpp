@@ -330,7 +330,7 @@ struct l2_model {
     int32_t *pf_ids = nullptr; // ids, then positions, of a batch or prompt
     int cap_pf = 0;
     std::vector<hipEvent_t> pf_ev[kMaxLanes];
-    hipEvent_t pf_join = nullptr, step_done = nullptr;
+    hipEvent_t pf_join = nullptr, step_done = nullptr, ahead[2] = {}; // ahead: steps_ahead
     int32_t *dprompt = nullptr, *dout_ids = nullptr;
     int cap_prompt = 0, cap_out = 0;
     // The decode step as a HIP graph (one per bucket of positions, kept in the state).  Off by default: a
@@ -365,6 +365,7 @@ struct l2_model {
     } tok;
     uint64_t asked = 0; // times that a loop of steps has asked the runtime about the stream (kAskLaunches)
     int device = 0;
+    WorkMark work;
     // per-launch event timing, on only inside l2_decode_profile
     struct ProfRec { int cls; hipEvent_t e0, e1; };
     bool prof_on = false;
@@ -427,29 +428,57 @@ static int timed_launch(l2_model *m, int cls, F &&launch) {
             L2_TRY(call);                                                    \
     } while (0)
 
-// Blocks of a token kernel wait for one another, so all of them have to find room on the device, which two such kernels at once might not
-// (each would hold compute units that the other's blocks wait for).  So one model at a time has them in flight; the steps of
-// others go out as launches of their own meanwhile, which only ever wait for kernels that end.
-struct TokenDevice {
+// The calls that are at work on a device.  Blocks of a token kernel wait for one another, so all of them have to find room, which two such
+// kernels at once might not; and while one runs it leaves room for kernels of up to 32 registers alone, others get their next launch at the end
+// of a step (1 ms at 7B).  So a step takes it only while no other call of this process is at work on the device; else it goes out as launches of its own, which
+// those of others come between.  Side by side, ms a call, before there were token kernels / with one model at a time in them, whatever others do /
+// so: two models of eight layers of 7B, 100 tokens each, 59 and 59 / 34 and 383 / 60 and 60; a prompt of 256 tokens beside such a loop 1.8 / 9.8 / 1.8; 40
+// tokens of a small fp32 model beside it 5.4 / 23 / 3.7.
+// Calls that overlap do so again as a rule: steps stay with launches for kShared behind.
+struct DeviceCalls {
     static constexpr int kMaxDevices = 64;
+    static constexpr std::chrono::milliseconds kShared{10};
+    typedef std::chrono::steady_clock Clock;
     std::mutex mu;
-    const l2_model *owner[kMaxDevices] = {};
-    // Whether m may launch one now; it is then the owner until it has left().
-    bool claim(const l2_model *m) {
-        if (m->device < 0 || m->device >= kMaxDevices) return false;
+    struct {
+        int calls = 0;
+        Clock::time_point shared_until;
+    } dev[kMaxDevices];
+    std::atomic<int> claims{0}; // calls that have steps in token kernels
+
+    void enter(int device) {
         std::lock_guard<std::mutex> lock(mu);
-        if (owner[m->device] && owner[m->device] != m) return false;
-        owner[m->device] = m;
-        return true;
+        if (dev[device].calls++ > 0) dev[device].shared_until = Clock::now() + kShared;
     }
-    // The caller has waited for everything on m's stream.
-    void left(const l2_model *m) {
-        if (m->device < 0 || m->device >= kMaxDevices) return;
+    void leave(int device) {
         std::lock_guard<std::mutex> lock(mu);
-        if (owner[m->device] == m) owner[m->device] = nullptr;
+        if (--dev[device].calls > 0) dev[device].shared_until = Clock::now() + kShared;
+    }
+    // Work that is enqueued and not waited for, on a stream of the caller's.
+    void pass_by(int device) {
+        if (claims.load(std::memory_order_relaxed) == 0 || device < 0 || device >= kMaxDevices) return;
+        std::lock_guard<std::mutex> lock(mu);
+        dev[device].shared_until = Clock::now() + kShared;
+    }
+    // Whether the one call that asks may take a token kernel.
+    bool alone(int device) {
+        if (device < 0 || device >= kMaxDevices) return false;
+        std::lock_guard<std::mutex> lock(mu);
+        return dev[device].calls == 1 && Clock::now() >= dev[device].shared_until;
     }
 };
-static TokenDevice token_device;
+static DeviceCalls device_calls;
+
+AtWork::AtWork(int device, WorkMark *mark) : device(device), mark(mark) {
+    if (device >= 0 && device < DeviceCalls::kMaxDevices && mark->depth++ == 0) device_calls.enter(device);
+}
+// Token kernels of the call have been waited for.
+AtWork::~AtWork() {
+    if (device < 0 || device >= DeviceCalls::kMaxDevices || --mark->depth > 0) return;
+    if (mark->claims) device_calls.claims--, mark->claims = false;
+    device_calls.leave(device);
+}
+AtWork::AtWork(l2_model *m) : AtWork(m->device, &m->work) {}
 
 struct StepGraph {
     hipGraph_t graph = nullptr;
@@ -474,6 +503,7 @@ struct l2_qlinear {
     float *x = nullptr, *xg = nullptr, *y = nullptr;
     int cap_B = 0;
     int device = 0; // that was current when the handle was made
+    WorkMark work;
     int mode = L2_PREFILL_FP32;
     OperatorBufs batch;
 };
@@ -641,6 +671,10 @@ static int model_build(const char *weights, size_t nbytes, const l2_dims *dims, 
                            layer_bytes);
     }
     L2_TRY(require_device());
+    int device = 0;
+    L2_HIP(hipGetDevice(&device));
+    WorkMark mark;
+    const AtWork at_work(device, &mark);
 
     l2_model *m = new l2_model();
     host_slots.add_user();
@@ -816,7 +850,7 @@ static int model_build(const char *weights, size_t nbytes, const l2_dims *dims, 
         m->hs.gave_up = (volatile int *)(m->hs.base + flag);
         *m->hs.gave_up = 0;
     }
-    M_HIP(hipGetDevice(&m->device));
+    m->device = device;
     M_TRY(token_kernel_setup(m));
     M_HIP(hipDeviceSynchronize());
 #undef M_HIP
@@ -884,7 +918,6 @@ extern "C" void l2_model_close(l2_model *m) {
                     m->amax, m->dprompt, m->dout_ids, m->op_x, m->op_xg, m->op_y, m->op_batch.planes, m->op_batch.ws,
                     m->tok.handed, m->tok.failed, m->tok.model, m->tok.slots, m->tok.walks};
     for (void *p : ptrs) dfree(p);
-    token_device.left(m);
     for (auto &a : m->lane) {
         void *bufs[] = {a.x, a.q, a.ss, a.ws, a.h[0], a.h[1], a.h[2]};
         for (void *p : bufs) dfree(p);
@@ -894,6 +927,8 @@ extern "C" void l2_model_close(l2_model *m) {
         for (hipEvent_t e : v) (void)hipEventDestroy(e);
     if (m->pf_join) (void)hipEventDestroy(m->pf_join);
     if (m->step_done) (void)hipEventDestroy(m->step_done);
+    for (hipEvent_t e : m->ahead)
+        if (e) (void)hipEventDestroy(e);
     if (m->hs.base) (void)hipHostFree(m->hs.base);
     for (hipStream_t es : m->extra_stream)
         if (es) (void)hipStreamDestroy(es);
@@ -1072,6 +1107,7 @@ static int state_clear(l2_state *s) {
 
 extern "C" int l2_state_reset(l2_state *s) {
     if (!s) return l2_fail(L2_ERR_ARG, "null state");
+    const AtWork at_work(s->m);
     L2_TRY(state_clear(s));
     L2_HIP(hipStreamSynchronize(s->m->stream));
     return L2_OK;
@@ -1079,6 +1115,7 @@ extern "C" int l2_state_reset(l2_state *s) {
 
 extern "C" int l2_state_read_kv(l2_state *s, int layer, int pos0, int npos, float *k_host, float *v_host) {
     if (!s || !k_host || !v_host) return l2_fail(L2_ERR_ARG, "null argument");
+    const AtWork at_work(s->m);
     const l2_model *m = s->m;
     if (layer < 0 || layer >= m->d.n_layers || pos0 < 0 || npos < 0 || pos0 + npos > m->max_seq)
         return l2_fail(L2_ERR_RANGE, "read_kv: layer %d, positions [%d,%d)", layer, pos0, pos0 + npos);
@@ -1092,6 +1129,7 @@ extern "C" int l2_state_read_kv(l2_state *s, int layer, int pos0, int npos, floa
 extern "C" int l2_state_write_kv(l2_state *s, int layer, int pos0, int npos, const float *k_host,
                                  const float *v_host) {
     if (!s || !k_host || !v_host) return l2_fail(L2_ERR_ARG, "null argument");
+    const AtWork at_work(s->m);
     const l2_model *m = s->m;
     if (layer < 0 || layer >= m->d.n_layers || pos0 < 0 || npos < 0 || pos0 + npos > m->max_seq)
         return l2_fail(L2_ERR_RANGE, "write_kv: layer %d, positions [%d,%d)", layer, pos0, pos0 + npos);
@@ -1105,6 +1143,7 @@ extern "C" int l2_state_write_kv(l2_state *s, int layer, int pos0, int npos, con
 
 extern "C" int l2_state_fill_synthetic(l2_state *s, int pos0, int npos, uint64_t seed) {
     if (!s) return l2_fail(L2_ERR_ARG, "null state");
+    const AtWork at_work(s->m);
     const l2_model *m = s->m;
     if (pos0 < 0 || npos < 0 || pos0 + npos > m->max_seq)
         return l2_fail(L2_ERR_RANGE, "fill: positions [%d,%d)", pos0, pos0 + npos);
@@ -1266,6 +1305,10 @@ extern "C" int l2_qlinear_create(const int32_t *qweight, const int32_t *qzeros, 
     if (!qweight || !qzeros || !scales || !g_index || !ql) return l2_fail(L2_ERR_ARG, "null argument");
     L2_TRY(check_qlinear_shape(in, out, group_size));
     L2_TRY(require_device());
+    int device = 0;
+    L2_HIP(hipGetDevice(&device));
+    WorkMark mark;
+    const AtWork at_work(device, &mark);
     const int groups = (int)div_up(in, group_size);
     std::vector<int32_t> inv(in);
     bool ok = true;
@@ -1297,10 +1340,7 @@ extern "C" int l2_qlinear_create(const int32_t *qweight, const int32_t *qzeros, 
     q->q.out = out;
     q->q.groups = groups;
     q->q.group_size = group_size;
-    if (hipGetDevice(&q->device) != hipSuccess) {
-        l2_qlinear_free(q);
-        return l2_fail(L2_ERR_HIP, "hipGetDevice failed");
-    }
+    q->device = device;
     float *tiles = nullptr;
     int rc = dalloc(&tiles, group_tiles_floats(out, groups));
     q->bufs[5] = tiles;
@@ -1418,6 +1458,7 @@ static int matvec_host(const DevQLinear &q, int device, float *dx, float *dxg, f
 extern "C" int l2_qlinear_matvec(l2_qlinear *q, const float *x_host, int B, float *y_host) {
     if (!q || !x_host || !y_host) return l2_fail(L2_ERR_ARG, "null argument");
     if (B < 1 || B > 4096) return l2_fail(L2_ERR_RANGE, "batch %d (1..4096)", B);
+    const AtWork at_work(q->device, &q->work);
     L2_TRY(qlinear_scratch(q, B));
     return matvec_host(q->q, q->device, q->x, q->xg, q->y, q->batch, operator_planes(q->q, B, q->mode), x_host, B, y_host, q->stream);
 }
@@ -1462,6 +1503,7 @@ extern "C" int l2_qlinear_matvec_device(l2_qlinear *q, const float *x_dev, int B
         return l2_fail(L2_ERR_RANGE, "B * in = %zu floats exceed the fixed scratch of %zu (no allocation is made here: "
                                      "use a smaller batch, or l2_qlinear_matvec)",
                        (size_t)B * (size_t)q->q.in, kScratchFloats);
+    device_calls.pass_by(q->device);
     FixedScratch fixed{};
     L2_TRY(scratch_ptr(&fixed));
     hipStream_t st = (hipStream_t)hip_stream;
@@ -1497,6 +1539,7 @@ extern "C" int l2_model_qmatvec(l2_model *m, int layer, int proj, const float *x
     if (proj < 0 || proj > 6 || layer < 0 || layer >= m->d.n_layers)
         return l2_fail(L2_ERR_RANGE, "projection %d, layer %d", proj, layer);
     if (B < 1 || B > 4096) return l2_fail(L2_ERR_RANGE, "batch %d (1..4096)", B);
+    const AtWork at_work(m);
     const DevQLinear &q = m->q[proj][layer];
     L2_TRY(op_scratch(m, (size_t)B * std::max(std::max(q.in, q.out), m->d.vocab_size)));
     if (q.dense) { // Linear::matvec<B> (src/model.rs:22-31)
@@ -1525,6 +1568,7 @@ extern "C" int l2_model_qmatvec(l2_model *m, int layer, int proj, const float *x
 
 extern "C" int l2_model_classifier(l2_model *m, const float *x_host, float *y_host) {
     if (!m || !x_host || !y_host) return l2_fail(L2_ERR_ARG, "null argument");
+    const AtWork at_work(m);
     L2_TRY(op_scratch(m, (size_t)std::max(m->d.dim, m->d.vocab_size)));
     L2_HIP(hipMemcpyAsync(m->op_x, x_host, (size_t)m->d.dim * 4, hipMemcpyHostToDevice, m->stream));
     L2_TRY(dense_matvec_launch(m->op_y, m->wcls, m->op_x, nullptr, 0.f, m->d.dim, m->d.vocab_size, nullptr, m->stream));
@@ -1604,7 +1648,6 @@ static int wait_host(l2_model *m, const unsigned long long *amax, int32_t *id) {
     if (amax) L2_TRY(index_launch(amax, id, m->stream));
     L2_HIP(hipStreamSynchronize(m->stream));
     m->hs.reading = false;
-    token_device.left(m);
     return L2_OK;
 }
 
@@ -1830,7 +1873,6 @@ static int token_tries(l2_model *m, F &&steps) {
         rc = steps();
         if (rc != L2_OK) { // some of them may be on their way
             if (m->tok.steps != before && hipStreamSynchronize(m->stream) == hipSuccess) (void)token_gave_up(m, &again);
-            token_device.left(m);
             break;
         }
         rc = token_gave_up(m, &again);
@@ -1852,9 +1894,10 @@ static int forward_enqueue(l2_model *m, l2_state *s, int B, int max_pos, const F
     if (whole) { // contexts that one query head's blocks take whole, see attn_launch_qg
         int ts = 0, n_splits = 0;
         attn_split_policy(max_pos + 1, d.n_heads, d.n_kv_heads, &ts, &n_splits);
-        whole = n_splits == 1 && (d.n_heads < 8 * d.n_kv_heads || ts > kFewTimesteps) && token_device.claim(m);
+        whole = n_splits == 1 && (d.n_heads < 8 * d.n_kv_heads || ts > kFewTimesteps) && device_calls.alone(m->device);
     }
     if (whole) {
+        if (!m->work.claims) device_calls.claims++, m->work.claims = true;
         l2_model::TokenKernel &t = m->tok;
         float *const handed = t.handed + (t.set ? t.set_floats : 0), *const clear = t.handed + (t.set ? 0 : t.set_floats);
         const TokArgs a{t.model, handed, clear, m->tok_emb, in.src, in.amax, m->x, s->kcache, s->vcache, max_pos};
@@ -2201,6 +2244,7 @@ extern "C" int l2_forward(l2_model *m, l2_state *s, const int32_t *tokens, const
     if (!m || !s || !tokens || !pos) return l2_fail(L2_ERR_ARG, "null argument");
     if (s->m != m) return l2_fail(L2_ERR_ARG, "state belongs to another model");
     if (B < 1 || B > 4096) return l2_fail(L2_ERR_RANGE, "batch %d (1..4096)", B);
+    const AtWork at_work(m);
     int max_pos = 0;
     L2_TRY(check_tokens(m, tokens, pos, B, &max_pos));
     L2_TRY(ensure_batch(m, B));
@@ -2226,6 +2270,7 @@ extern "C" int l2_forward(l2_model *m, l2_state *s, const int32_t *tokens, const
 
 int l2_forward_weights(l2_model *m, l2_state *s, int32_t token, int32_t pos, float temperature, bool more, SampleWeights *out) {
     if (s->m != m) return l2_fail(L2_ERR_ARG, "state belongs to another model");
+    const AtWork at_work(m);
     int max_pos = 0;
     L2_TRY(check_tokens(m, &token, &pos, 1, &max_pos));
     L2_TRY(ensure_batch(m, 1));
@@ -2239,7 +2284,6 @@ int l2_forward_weights(l2_model *m, l2_state *s, int32_t token, int32_t pos, flo
         if (!m->step_done) L2_HIP(hipEventCreateWithFlags(&m->step_done, hipEventDisableTiming));
         L2_HIP(hipEventRecord(m->step_done, m->stream));
         L2_HIP(hipEventSynchronize(m->step_done));
-        token_device.left(m);
         return L2_OK;
     }));
     *out = {m->hs.logits, m->hs.redo};
@@ -2281,6 +2325,7 @@ static constexpr int kPassTokens = 512;
 static int prefill_chunks(l2_model *m, l2_state *s, const int32_t *tokens, int n, int pos0, int chunk, bool wait) {
     if (!m || !s || !tokens) return l2_fail(L2_ERR_ARG, "null argument");
     if (s->m != m) return l2_fail(L2_ERR_ARG, "state belongs to another model");
+    const AtWork at_work(m);
     if (n < 1 || chunk < 1 || chunk > 4096) return l2_fail(L2_ERR_RANGE, "%d tokens in chunks of %d (1..4096)", n, chunk);
     if (pos0 < 0 || (long)pos0 + n > m->max_seq)
         return l2_fail(L2_ERR_RANGE, "positions %d..%ld outside 0..%d", pos0, (long)pos0 + n - 1, m->max_seq - 1);
@@ -2371,6 +2416,7 @@ static int steps_run(l2_model *m, l2_state *s, int32_t first, int pos0, int n, c
 extern "C" int l2_decode_greedy(l2_model *m, l2_state *s, int32_t token, int32_t pos, int32_t *next) {
     if (!m || !s || !next) return l2_fail(L2_ERR_ARG, "null argument");
     if (s->m != m) return l2_fail(L2_ERR_ARG, "state belongs to another model");
+    const AtWork at_work(m);
     int max_pos = 0;
     L2_TRY(check_tokens(m, &token, &pos, 1, &max_pos));
     L2_TRY(ensure_batch(m, 1));
@@ -2459,6 +2505,13 @@ static int step_bucket(const l2_model *m, int pos) {
 // As graphs: see step_graph_get.
 static constexpr int kAskLaunches = 128;
 static constexpr double kAskWeights = 5e7; // a layer of 7B has 2e8 and takes 40 us
+// Steps in token kernels leave little room for other calls' kernels (DeviceCalls), which may come at any time, so a loop has no more of them
+// enqueued than 2 * steps_ahead, some 2 * kAheadUs; an event that is waited for every 4 ms costs some 1 us of each ms (7B 1053 -> 1054 us a step).
+static constexpr double kAheadUs = 4000;
+static int steps_ahead(const l2_model *m) {
+    const double us = m->d.n_layers * (layer_weights(m) * 0.53 / 4.2e6 + 12) + (double)m->d.vocab_size * m->d.dim * 4 / 5e6;
+    return std::max(2, (int)(kAheadUs / us));
+}
 static int steps_enqueue(l2_model *m, l2_state *s, int32_t first, int pos0, int n, const int32_t *prompt, int n_prompt) {
     if (m->use_graph && !m->prof_on) {
         L2_TRY(ensure_loop_buffers(m, std::max(n_prompt, 1), std::max(n, 1)));
@@ -2485,6 +2538,8 @@ static int steps_enqueue(l2_model *m, l2_state *s, int32_t first, int pos0, int 
     // before the end, where the wait would meet it.
     const bool asks = layer_weights(m) < kAskWeights;
     int since = 0; // launches since it was asked
+    const int ahead = steps_ahead(m);
+    int in_ones = 0, records = 0;
     ForwardIn in;
     in.src.token = first, in.logits = m->logits, in.whole = true;
     for (int i = 0; i < n; i++) {
@@ -2498,6 +2553,12 @@ static int steps_enqueue(l2_model *m, l2_state *s, int32_t first, int pos0, int 
         if (asks && since >= ask_steps * launches && i + ask_steps < n) {
             if (hipStreamQuery(m->stream) == hipErrorNotReady) (void)hipGetLastError();
             since = 0, m->asked++;
+        }
+        if (m->tok.steps != in_one && ++in_ones % ahead == 0 && i + 1 < n) {
+            for (hipEvent_t &e : m->ahead)
+                if (!e) L2_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+            L2_HIP(hipEventRecord(m->ahead[records & 1], m->stream));
+            if (records++ > 0) L2_HIP(hipEventSynchronize(m->ahead[records & 1]));
         }
         in.src = TokenSource{};
         if (pos < n_prompt)
@@ -2556,6 +2617,7 @@ extern "C" int l2_generate_greedy(l2_model *m, l2_state *s, const int32_t *promp
     if (s->m != m) return l2_fail(L2_ERR_ARG, "state belongs to another model");
     if (n_prompt < 0 || steps < 0) return l2_fail(L2_ERR_ARG, "negative count");
     if (steps > m->max_seq) return l2_fail(L2_ERR_RANGE, "steps %d exceeds the cache length %d", steps, m->max_seq);
+    const AtWork at_work(m);
     // The ladder runs whatever `steps` is: a prompt it would carry past the cache is refused before any launch
     // (the reference panics there on its fixed [SEQ_LEN] arrays).
     if (use_prefill && l2_prefill_ladder_end(n_prompt) > m->max_seq)
@@ -2695,6 +2757,7 @@ extern "C" int l2_decode_bench(l2_model *m, l2_state *s, int32_t token, int32_t 
     if (s->m != m) return l2_fail(L2_ERR_ARG, "state belongs to another model");
     if (pos < 0 || pos + n_tokens > m->max_seq) return l2_fail(L2_ERR_RANGE, "positions [%d,%d) exceed the cache", pos, pos + n_tokens);
     if (token < 0 || token >= m->d.vocab_size) return l2_fail(L2_ERR_RANGE, "token %d", token);
+    const AtWork at_work(m);
     L2_TRY(ensure_batch(m, 1));
     if (m->use_graph) { // capture (if need be) outside the timed region
         L2_TRY(ensure_loop_buffers(m, 1, n_tokens));
@@ -2932,6 +2995,7 @@ extern "C" int l2_decode_profile(l2_model *m, l2_state *s, int32_t token, int32_
     if (s->m != m) return l2_fail(L2_ERR_ARG, "state belongs to another model");
     if (pos < 0 || pos + n_tokens > m->max_seq) return l2_fail(L2_ERR_RANGE, "positions [%d,%d) exceed the cache", pos, pos + n_tokens);
     if (token < 0 || token >= m->d.vocab_size) return l2_fail(L2_ERR_RANGE, "token %d", token);
+    const AtWork at_work(m);
     L2_TRY(ensure_batch(m, 1));
     L2_HIP(hipStreamSynchronize(m->stream));
     m->prof.clear();

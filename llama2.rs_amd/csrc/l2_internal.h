@@ -382,6 +382,21 @@ struct AttnDecode {
 };
 int attention_decode_launch(const AttnDecode &a, hipStream_t st);
 
+// A call is at work on its handle's device for its time, for which it keeps one of these (host.cpp: DeviceCalls).  Calls that others make
+// count once.
+struct WorkMark {
+    int depth = 0;
+    bool claims = false; // steps of the call are in token kernels
+};
+struct AtWork {
+    int device;
+    WorkMark *mark;
+    explicit AtWork(l2_model *m);
+    AtWork(int device, WorkMark *mark);
+    ~AtWork();
+    AtWork(const AtWork &) = delete;
+};
+
 // ---- all layers of a decode step in one launch (kernels_token.hip) ---------------------------
 
 constexpr int kTokenWaves = 16; // of a block

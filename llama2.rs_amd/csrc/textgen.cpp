@@ -306,6 +306,7 @@ extern "C" int l2_generate(l2_model *m, l2_state *s, const l2_tokenizer *t, cons
                            int *n_tokens, int64_t *ms) {
     if (!m || !s || !t || !prompt || !n_tokens || !ms || steps < 0) return l2_fail(L2_ERR_ARG, "l2_generate: bad argument");
     if (temperature != 0.0f && !rng) return l2_fail(L2_ERR_ARG, "l2_generate: sampling needs a Random");
+    const AtWork at_work(m);
     l2_dims d;
     L2_TRY(l2_model_dims(m, &d));
     if ((int)t->vocab.size() < d.vocab_size) return l2_fail(L2_ERR_ARG, "tokenizer has %zu entries, the model %d", t->vocab.size(), d.vocab_size);

@@ -3,6 +3,7 @@ import ctypes
 import os
 import sys
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -159,6 +160,53 @@ def test_an_error_leaves_nothing_behind():
     assert state_of(a)[0] == 1 and state_of(b) == (1, 0)
     for m in (a, b):
         m.close()
+
+
+def test_steps_beside_other_calls_go_layer_by_layer():
+    """While another call is at work on the device, and for a while behind, a model's steps go out as launches that the other's come between; a
+    loop that has the device to itself when it starts has only some ms of steps in token kernels ahead when another call comes."""
+    a, b = model(1024, 2816, 8, 2, 64, layers=3, seed=3), model(1024, 2816, 8, 2, 64, layers=3, seed=4)
+    q = ops.QLinear(*[np.zeros(s, t) for s, t in (((256, 128), np.int32), ((32, 16), np.int32), ((256, 16), np.float32))], np.arange(1024), 64)
+    prompt, tokens, x = np.array([5, 17, 99], np.int32), np.arange(64, dtype=np.int32), np.zeros(1024, np.float32)
+    want = a.generate_greedy(prompt, 800)[0]
+
+    def steps_of(f):
+        n = a.token_steps()
+        f()
+        return a.token_steps() - n
+
+    def beside(other, f, delay=0.0):
+        """f() while another thread calls other() again and again, from `delay` seconds behind its start on."""
+        stop, started = threading.Event(), threading.Event()
+
+        def run():
+            started.set()
+            stop.wait(delay)
+            while not stop.is_set():
+                other()
+        t = threading.Thread(target=run)
+        t.start()
+        started.wait()
+        try:
+            return f()
+        finally:
+            stop.set()
+            t.join()
+
+    def check(steps):
+        assert np.array_equal(a.generate_greedy(prompt, steps)[0], want[:steps - 2])
+    assert steps_of(lambda: check(60)) == 58
+    for other in (lambda: b.prefill_chunks(tokens, 0, 64), lambda: b.generate_greedy(prompt, 40), lambda: b.decode_greedy(3, 5), lambda: q.matvec(x)):
+        def f():
+            check(60)  # the first of these may find the device free
+            return steps_of(lambda: [check(60) for _ in range(8)])
+        assert beside(other, f) < 58, "of 464"
+        time.sleep(0.05)
+        assert steps_of(lambda: check(60)) == 58
+    assert 20 < beside(lambda: b.prefill_chunks(tokens, 0, 64), lambda: steps_of(lambda: check(800)), delay=0.01) < 600
+    q.close()
+    a.close()
+    b.close()
 
 
 def test_models_on_threads():
