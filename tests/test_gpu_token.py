@@ -40,6 +40,14 @@ SHAPES = [(512, 768, 4, 2, 32), (1024, 2816, 8, 2, 64), (1152, 32, 9, 9, 32), (1
           (3072, 8192, 24, 3, 64), (4096, 11008, 32, 32, 128), (5120, 5120, 40, 40, 64), (8192, 1024, 64, 8, 32), (2048, 28672, 16, 16, 64)]
 
 
+def takes(shape, timesteps):
+    """Whether a step over so many timesteps goes through the token kernel: where attention takes a context whole, but not on the matrix cores."""
+    _, _, heads, kv, _ = shape
+    if heads == 8 * kv and timesteps <= 256:
+        return False
+    return timesteps <= ((512 if kv > 32 else 640) if heads <= 2 * kv else 896 if heads < 32 else 1024 if kv <= 4 else 768)
+
+
 @pytest.mark.parametrize("shape", SHAPES)
 def test_logits_and_cache_rows_are_those_of_the_launches(shape):
     m = model(*shape)
@@ -52,7 +60,9 @@ def test_logits_and_cache_rows_are_those_of_the_launches(shape):
             m.reset()
             if start:
                 m.fill_kv_synthetic(0, start, seed=start)
+            before = m.token_steps()
             logits = [m.forward([int(t)], [start + i]).copy() for i, t in enumerate(tokens)]
+            assert m.token_steps() - before == on * sum(takes(shape, start + i + 1) for i in range(n)), (shape, start)
             got[on] = (logits, [m.read_kv(l, start, n) for l in range(2)])
         assert state_of(m)[1] == 0
         for a, b in zip(got[1][0], got[0][0]):
@@ -69,7 +79,9 @@ def test_a_loop_of_steps_and_a_value_that_looks_absent():
     ids = {}
     for on in (1, 0):
         token_kernel(m, on)
+        before = m.token_steps()
         ids[on] = m.generate_greedy(prompt, 120)[0]
+        assert m.token_steps() - before == on * 118  # two positions are the ladder's
         m.reset()
         t, one = 5, []
         for p in range(20):
@@ -210,21 +222,29 @@ def test_steps_beside_other_calls_go_layer_by_layer():
 
 
 def test_models_on_threads():
-    """Two models decode side by side: one of them at a time has token kernels in flight, and both get their own results."""
+    """Two models decode on threads, side by side and one at a time as it comes, through the token kernel and as launches: both get their own results."""
     ms = [model(1024, 2816, 8, 2, 64, seed=s) for s in (3, 4)]
     prompt = np.array([5, 17, 99], np.int32)
-    want = [m.generate_greedy(prompt, 60)[0] for m in ms]
+    want = []
+    for m in ms:
+        token_kernel(m, 0)
+        want.append(m.generate_greedy(prompt, 60)[0])
+        token_kernel(m, 1)
+    assert [m.token_steps() for m in ms] == [0, 0]
     bad = []
 
-    def run(i):
-        for _ in range(15):
+    def run(i, pauses):
+        for pause in pauses:
             if not np.array_equal(ms[i].generate_greedy(prompt, 60)[0], want[i]):
                 bad.append(i)
-    threads = [threading.Thread(target=run, args=(i,)) for i in range(2)]
+            time.sleep(pause)
+    rng = np.random.default_rng(0)
+    threads = [threading.Thread(target=run, args=(i, [0.0] * 15 + list(rng.uniform(0, 0.03, 25)))) for i in range(2)]
     for t in threads:
         t.start()
     for t in threads:
         t.join()
     assert not bad and [state_of(m) for m in ms] == [(1, 0), (1, 0)]
+    assert all(0 < m.token_steps() < 40 * 58 for m in ms), [m.token_steps() for m in ms]
     for m in ms:
         m.close()
