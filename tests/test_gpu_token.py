@@ -40,14 +40,6 @@ SHAPES = [(512, 768, 4, 2, 32), (1024, 2816, 8, 2, 64), (1152, 32, 9, 9, 32), (1
           (3072, 8192, 24, 3, 64), (4096, 11008, 32, 32, 128), (5120, 5120, 40, 40, 64), (8192, 1024, 64, 8, 32), (2048, 28672, 16, 16, 64)]
 
 
-def takes(shape, timesteps):
-    """Whether a step over so many timesteps goes through the token kernel: where attention takes a context whole, but not on the matrix cores."""
-    _, _, heads, kv, _ = shape
-    if heads == 8 * kv and timesteps <= 256:
-        return False
-    return timesteps <= ((512 if kv > 32 else 640) if heads <= 2 * kv else 896 if heads < 32 else 1024 if kv <= 4 else 768)
-
-
 @pytest.mark.parametrize("shape", SHAPES)
 def test_logits_and_cache_rows_are_those_of_the_launches(shape):
     m = model(*shape)
@@ -60,9 +52,7 @@ def test_logits_and_cache_rows_are_those_of_the_launches(shape):
             m.reset()
             if start:
                 m.fill_kv_synthetic(0, start, seed=start)
-            before = m.token_steps()
             logits = [m.forward([int(t)], [start + i]).copy() for i, t in enumerate(tokens)]
-            assert m.token_steps() - before == on * sum(takes(shape, start + i + 1) for i in range(n)), (shape, start)
             got[on] = (logits, [m.read_kv(l, start, n) for l in range(2)])
         assert state_of(m)[1] == 0
         for a, b in zip(got[1][0], got[0][0]):
@@ -79,9 +69,7 @@ def test_a_loop_of_steps_and_a_value_that_looks_absent():
     ids = {}
     for on in (1, 0):
         token_kernel(m, on)
-        before = m.token_steps()
         ids[on] = m.generate_greedy(prompt, 120)[0]
-        assert m.token_steps() - before == on * 118  # two positions are the ladder's
         m.reset()
         t, one = 5, []
         for p in range(20):
@@ -120,6 +108,58 @@ def test_waits_that_are_given_up():
     token_kernel(m, 1, missing=1, looks=64)
     for i in range(4):  # not asked any more after three calls
         assert np.array_equal(m.generate_greedy(prompt, 8)[0], want[:6]) and state_of(m) == (int(i < 2), min(i + 1, 3))
+    m.close()
+
+
+def test_models_on_threads():
+    """Two models decode side by side: one of them at a time has token kernels in flight, and both get their own results."""
+    ms = [model(1024, 2816, 8, 2, 64, seed=s) for s in (3, 4)]
+    prompt = np.array([5, 17, 99], np.int32)
+    want = [m.generate_greedy(prompt, 60)[0] for m in ms]
+    bad = []
+
+    def run(i):
+        for _ in range(15):
+            if not np.array_equal(ms[i].generate_greedy(prompt, 60)[0], want[i]):
+                bad.append(i)
+    threads = [threading.Thread(target=run, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad and [state_of(m) for m in ms] == [(1, 0), (1, 0)]
+    for m in ms:
+        m.close()
+
+
+# ---- the route that steps take
+
+
+def takes(shape, timesteps):
+    """Whether a step over so many timesteps goes through the token kernel: where attention takes a context whole, but not on the matrix cores."""
+    _, _, heads, kv, _ = shape
+    if heads == 8 * kv and timesteps <= 256:
+        return False
+    return timesteps <= ((512 if kv > 32 else 640) if heads <= 2 * kv else 896 if heads < 32 else 1024 if kv <= 4 else 768)
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_the_steps_that_are_compared_take_the_kernel(shape):
+    """Steps at the starts of the comparison above, and a loop of them: in one launch where attention takes the context whole, none with the kernel off."""
+    m = model(*shape)
+    for on in (1, 0):
+        token_kernel(m, on)
+        for start, n in ((0, 4), (62, 4), (127, 3), (255, 3), (509, 3), (638, 3), (766, 3), (1023, 2)):
+            m.reset()
+            if start:
+                m.fill_kv_synthetic(0, start, seed=start)
+            before = m.token_steps()
+            for i in range(n):
+                m.forward([5 + i], [start + i])
+            assert m.token_steps() - before == on * sum(takes(shape, start + i + 1) for i in range(n)), start
+        before = m.token_steps()
+        m.generate_greedy(np.array([5, 17, 99], np.int32), 120)
+        assert m.token_steps() - before == on * sum(takes(shape, p + 1) for p in range(2, 120))  # two positions are the ladder's
     m.close()
 
 
@@ -221,7 +261,7 @@ def test_steps_beside_other_calls_go_layer_by_layer():
     b.close()
 
 
-def test_models_on_threads():
+def test_models_on_threads_take_both_routes():
     """Two models decode on threads, side by side and one at a time as it comes, through the token kernel and as launches: both get their own results."""
     ms = [model(1024, 2816, 8, 2, 64, seed=s) for s in (3, 4)]
     prompt = np.array([5, 17, 99], np.int32)
