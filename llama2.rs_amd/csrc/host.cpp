@@ -1599,6 +1599,13 @@ extern "C" int l2_model_classifier(l2_model *m, const float *x_host, float *y_ho
 // the context allows it, at least 64 timesteps each.  (Two per CU, the earlier rule, left some CUs with two blocks
 // and the launch as long as those: 70B behind 4096 positions 18.6 -> 16.5 us per layer, 13B behind 1000 positions
 // 16.7 -> 15.3, 7B unchanged; half a block per CU is slower everywhere.)
+// The limits are where launches cross, on both sides of which a step was launches.  Where a model has the token kernel they are also where its
+// steps go from one launch to five per layer, and one launch is the shorter by more than the splits give, right up to them: us a step as launches and
+// in one, at 30, 300, 500 positions and shortly before the limit, then behind it: 8 layers of 7B 276 / 298 / 309 / 312 and 248 / 266 / 277 / 280, then
+// 317; 6 of 13B 291 / 308 / - / 315 and 260 / 274 / - / 280, then 322; 6 of 2048 inputs, 16 heads on 4, 129 / 142 / 149 / 160 and 104 / 115 / 122 / 132,
+// then 159; 6 of 4096, 32 on 8, 200 / 215 / 222 / 229 and 180 / 192 / 200 / 206, then 230; 3 of 1024, 8 on 2, 55 / 61 / 63 / 68 and 50 / 54 / 56 / 60, then 70.
+// So one launch would still be the shorter some way behind them; how far has not been measured.  The limits move for both routes together, or a
+// call that is done again as launches would give other bits.
 static void attn_split_policy(int n_t, int n_heads, int n_kv_heads, int *ts_out, int *n_splits_out) {
     int whole = n_heads <= 2 * n_kv_heads ? (n_kv_heads > 32 ? 512 : 640) : n_heads < 32 ? 896 : n_kv_heads <= 4 ? 1024 : 768;
     if (n_heads == 8 * n_kv_heads && n_t <= kFewTimesteps) whole = kFewTimesteps;
@@ -1619,7 +1626,8 @@ static void attn_split_policy(int n_t, int n_heads, int n_kv_heads, int *ts_out,
 // max_pos).  max_pos is the largest position among them (sizes the attention
 // scratch).  With want_logits the classifier and the running argmax follow.
 //
-// Five launches per layer when B == 1: q|k|v with the attention rmsnorm in
+// When B == 1 all layers are one launch where the token kernel can be taken
+// (`whole`, below), else five per layer: q|k|v with the attention rmsnorm in
 // front; attention with RoPE and the cache write folded in; wo with the
 // residual add behind; w1|w3 with the ffn rmsnorm in front and the SiLU gate
 // behind; w2 with the residual add behind.  Every producer writes its result
@@ -1743,8 +1751,9 @@ static int token_plan(const l2_dims &d, TokenPlan &t, bool *ok) {
         const bool uneven = p == TOK_WO && nwk <= 8 && rpb <= 8 / nwk * (kTokenRows + 1);
         const int streams = uneven ? 8 / nwk : kTokenWaves / nwk / halves;
         const int early = uneven ? std::min((rpb + streams - 1) / streams, (rpb + 2 * streams - 1) / (2 * streams) + 1) : 0;
-        // A wave with more rows than that reads for so long that there is nothing to gain (70B's w1|w3, 56 pairs a wave: two layers behind 280
-        // positions, with the classifier, 337.6 us as launches and 338.6 so; 13B's 27: 243 and 231).
+        // A wave's rows that are rounded as behind a loop are a mask of 32 bits.  The more rows a wave has, the less there is to gain: two layers behind
+        // 280 positions, as launches and in one, with 27, 28 and 32 pairs of w1|w3 a wave (5120 inputs, 13824 hidden; 8192, 14336; 8192, 16384) 110.8 and 101.7
+        // us, 137.1 and 133.0, 146.4 and 143.8; with 56 (70B, with the classifier) 337.6 and 338.6.
         if (rpb > kTokenWaves * 64 || rpb > 32 * streams) return L2_OK;
         const auto whole = [&](int n) { return (n + plan.streams - 1) / plan.tile * plan.tile; };
         for (int b = 0; b < grid; b++) {

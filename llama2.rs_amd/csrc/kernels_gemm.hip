@@ -129,13 +129,14 @@ __global__ __launch_bounds__(256) void gemm_input_kernel(const GemmInput A, int 
     store_piece<NP>(A.out[c], b, in_p, j8, make_piece<NP>(v));
 }
 
-// The same from x in pinned host memory, where every element should cross the bus once and in order: read in order, 16 bytes per
-// thread and load, and scattered to its places.  NP = 0: fp32, for the matvec kernels.  What bounds it is the bus (48 GB/s, 18 us
-// for the 0.9 MB of 16 columns of 13824 inputs; the scattered stores take a third of that, behind it), so it is launched for a part
-// of the columns while the host brings the next one.  A DMA engine reads at 65 GB/s, but a kernel behind a DMA starts 10 us late.
+// The same from x as the host has left it, in pinned memory or, from kWindowBytes (host.cpp) on, in device memory: read in order, 16 bytes per
+// thread and load, and scattered to its places, so that every element crosses the bus once where it has to.  NP = 0: fp32, for the
+// matvec kernels.  From device memory 6.8 us for the 0.9 MB of 16 columns of 13824 inputs.  From pinned memory what bounds it is the bus (48 GB/s, 18 us
+// for the same; the scattered stores take a third of that, behind it), so a long x is launched for in two parts, one while the host
+// brings the other.  A DMA engine reads at 65 GB/s, but a kernel behind a DMA starts 10 us late.
 // With a column per block, read into LDS and permuted there, one compute unit's reads are the bound: one column of 28672 inputs
-// 32.8 -> 39.3 us for the call.
-constexpr int kHostPieces = 2; // of 16 bytes per thread (four: 84 us for 16 columns of 13824x5120, two 82)
+// 32.8 -> 39.3 us for the call, from pinned memory.
+constexpr int kHostPieces = 2; // of 16 bytes per thread (four: 84 us for 16 columns of 13824x5120 from pinned memory, two 82)
 template <int NP>
 __global__ __launch_bounds__(256) void host_input_kernel(void *__restrict__ out, const float *__restrict__ x,
                                                          const int32_t *__restrict__ inv, int n, int in_p) {
@@ -1216,6 +1217,9 @@ GemmShape gemm_shape(const Q4Launch &L, int slice_batch, int planes) {
         // (3 x 16 + 16 67 more, five equal ones 11 more).
         // Not for fewer slices than the equal ones, whose sums are shorter (2048 -> 17248, two for three: an error of 8.1e-8 for 7.8e-8; 4096 -> 22016, two
         // for one: 9.4e-8 for 9.9e-8, 4096 -> 11008, three for two: 8.8e-8 for 8.9e-8).
+        // The 2.9 and the 0.97 are of that shape.  Whole layers of other widths, 17 to 800 columns, equal slices -> with it where it is taken: 2048 inputs
+        // 5632 hidden, 17, 64, 400, 800 107 / 129 / 420 / 706 -> 101 / 122 / 407 / 687 us; 3072, 8192, 400 852 -> 821; 5120, 13824, 800 3696 -> 3695; 8192, 14336, 17, 64,
+        // 130, 400, 800 518 / 626 / 1584 / 3185 / 5850 -> 511 / 620 / 1556 / 3134 / 5702.
         const float per = 4096.0f / L.in;
         for (int n = s.slices; n + 1 < kMaxGemmSlices && n * blocks <= 4 * cus; n++) {
             const int rounds = (n * blocks + cus - 1) / cus, idle = rounds * cus - n * blocks;
