@@ -503,7 +503,6 @@ struct l2_qlinear {
     float *x = nullptr, *xg = nullptr, *y = nullptr;
     int cap_B = 0;
     int device = 0; // that was current when the handle was made
-    WorkMark work;
     int mode = L2_PREFILL_FP32;
     OperatorBufs batch;
 };
@@ -589,7 +588,7 @@ static struct HostSlots {
 // Device memory that the host writes itself, over the bus (fine-grained; where all of the device's memory is mapped for the host, and with it
 // the register that says when the writes are there, see window_written): x of a
 // call on host arrays goes there, and the kernel that needs it reads it on the device.  Before, x went to pinned memory, and a kernel of its
-// own brought it over, or read it from there while it was cut into planes: 4096x4096, one column, 20.4 -> 19.0 us; 13824x5120, 16
+// own brought it over, or read it from there while it was cut into planes: 4096x4096, one column, 20.4 -> 19.3 us; 13824x5120, 16
 // columns 76.4 -> 70.2.  The host writes 45 GB/s this way (with the flush 16 KB 1.6 us, 64 KB 2.7, 864 KB 20.7), the kernels read the bus at some 32.
 // At most kKept pieces of a device, for as long as the process runs (memory that others may have cached is not given back to be used as
 // something else); a call that finds none free takes the way through pinned memory.
@@ -1458,7 +1457,8 @@ static int matvec_host(const DevQLinear &q, int device, float *dx, float *dxg, f
 extern "C" int l2_qlinear_matvec(l2_qlinear *q, const float *x_host, int B, float *y_host) {
     if (!q || !x_host || !y_host) return l2_fail(L2_ERR_ARG, "null argument");
     if (B < 1 || B > 4096) return l2_fail(L2_ERR_RANGE, "batch %d (1..4096)", B);
-    const AtWork at_work(q->device, &q->work);
+    WorkMark mark; // of the call, not the handle: none is inside another here
+    const AtWork at_work(q->device, &mark);
     L2_TRY(qlinear_scratch(q, B));
     return matvec_host(q->q, q->device, q->x, q->xg, q->y, q->batch, operator_planes(q->q, B, q->mode), x_host, B, y_host, q->stream);
 }
@@ -1872,7 +1872,7 @@ static int token_gave_up(l2_model *m, bool *again) {
 }
 
 // Steps of a call: steps() enqueues them and waits.  Where a token kernel gave up they are done once more, with the layers' own launches.
-// Whatever comes back, nothing of the call is on the stream then and nothing of it is left for the next one.
+// Whatever comes back, no token kernel of the call is on the stream then and nothing of the call is left for the next one.
 template <class F>
 static int token_tries(l2_model *m, F &&steps) {
     bool again = false;
